@@ -1,0 +1,286 @@
+// The host path from a torch tensor to a launch: allocation of the result and of the workspace, the current stream
+// and the call of the C ABI, in one native call per layer.
+//
+// What bounds a decode-sized call is the host: a [4096 x 4096] product at one row is 3.8 us of GPU time, and the same
+// steps taken in Python (module attributes, torch.empty, torch.cuda.device, current_stream, five ctypes calls) were
+// 17 us of the 21 us a LowBitLinear call took.  The module is plain CPython (METH_FASTCALL, no argument parsing by
+// keyword).  It holds no state but the addresses of the C ABI functions, which the ctypes binding hands over
+// (`bind`), so that both always run the same library.
+//
+// Functions whose name says "or None" answer None for anything but the plain case (a tensor on another device, a
+// dtype they do not know, a weight of another size): the Python code behind them then takes its own way and words
+// the error.
+#include <torch/csrc/autograd/python_variable.h>
+#include <torch/csrc/Exceptions.h>
+#include <ATen/ATen.h>
+#include <c10/core/DeviceGuard.h>
+#include <c10/core/GradMode.h>
+#include <c10/hip/HIPStream.h>
+
+#include "../../include/lowbit_abi.h"
+
+namespace {
+
+using at::Tensor;
+
+struct Api {
+    decltype(&lowbit_last_error) last_error = nullptr;
+    decltype(&lowbit_blob_bytes) blob_bytes = nullptr;
+    decltype(&lowbit_tileable) tileable = nullptr;
+    decltype(&lowbit_workspace_bytes_for) workspace_bytes_for = nullptr;
+    decltype(&lowbit_forward) forward = nullptr;
+    decltype(&lowbit_forward_ws) forward_ws = nullptr;
+    decltype(&lowbit_forward_f32_workspace_bytes) forward_f32_workspace_bytes = nullptr;
+    decltype(&lowbit_forward_f32) forward_f32 = nullptr;
+    decltype(&lowbit_mlp_forward) mlp_forward = nullptr;
+    decltype(&lowbit_dequantize_rows) dequantize_rows = nullptr;
+} api;
+
+constexpr size_t WORKSPACE_CAP = (size_t)256 << 20;      // most that a product borrows for split-K partial sums
+
+struct Failed : std::runtime_error {
+    using std::runtime_error::runtime_error;
+};
+
+void check(int rc, const char *what) {
+    if (rc != 0) throw Failed(std::string(what) + " failed (" + std::to_string(rc) + "): " + api.last_error());
+}
+
+int dtype_code(at::ScalarType t) {
+    switch (t) {
+    case at::kHalf: return LOWBIT_DT_F16;
+    case at::kBFloat16: return LOWBIT_DT_BF16;
+    case at::kFloat: return LOWBIT_DT_F32;
+    default: return -1;
+    }
+}
+
+void *current_stream(const Tensor &t) { return (void *)c10::hip::getCurrentHIPStream(t.device().index()).stream(); }
+
+Tensor bytes_like(const Tensor &t, size_t n) { return at::empty({(int64_t)n}, t.options().dtype(at::kByte)); }
+
+// a tensor of this module's calls: strided, on the GPU
+bool on_gpu(const Tensor &t) { return t.device().is_cuda() && t.layout() == at::kStrided; }
+
+// w holds the packed [N, K] weight of this format on x's device
+bool is_blob(const Tensor &w, const Tensor &x, int qtype, int64_t N, int64_t K) {
+    if (w.device() != x.device() || w.layout() != at::kStrided || !w.is_contiguous()) return false;
+    const at::ScalarType st = w.scalar_type();
+    if (st != at::kByte && !(st == at::kBFloat16 && qtype == LOWBIT_QT_NF4)) return false;
+    return (size_t)w.nbytes() == api.blob_bytes(qtype, N * K) && w.nbytes() > 0;
+}
+
+// y = x * dequant(w)^T (+ bias), in x's dtype; x contiguous [.., K] with M rows, not empty
+Tensor product(const Tensor &x, const Tensor &w, const Tensor &bias, int qtype, int layout, int64_t M, int64_t N, int64_t K,
+               at::IntArrayRef shape) {
+    c10::DeviceGuard guard(x.device());
+    Tensor y = at::empty(shape, x.options());
+    void *st = current_stream(x);
+    const int dt = dtype_code(x.scalar_type());
+    // workspaces come from torch's caching allocator: ordered with the stream, no allocation in the steady state
+    if (dt == LOWBIT_DT_F32) {
+        const size_t bytes = api.forward_f32_workspace_bytes(M, N, K);
+        Tensor ws = bytes_like(x, bytes);
+        check(api.forward_f32((const float *)x.const_data_ptr(), w.const_data_ptr(), (float *)y.data_ptr(), qtype, layout, M, N, K,
+                              ws.data_ptr(), bytes, st), "lowbit_forward_f32");
+    } else if (const size_t bytes = M <= 16 ? 0 : api.workspace_bytes_for(qtype, layout, M, N, K, WORKSPACE_CAP)) {
+        Tensor ws = bytes_like(x, bytes);
+        check(api.forward_ws(x.const_data_ptr(), w.const_data_ptr(), y.data_ptr(), qtype, layout, dt, M, N, K, ws.data_ptr(), bytes,
+                             st), "lowbit_forward_ws");
+    } else {
+        check(api.forward(x.const_data_ptr(), w.const_data_ptr(), y.data_ptr(), qtype, layout, dt, M, N, K, st), "lowbit_forward");
+    }
+    if (bias.defined()) y.add_(bias);
+    return y;
+}
+
+// Whether a small batch of float32 rows stays float32 (use_batch_forward of low_bit_linear.py)
+bool batch_stays_f32(int qtype, int64_t M, int64_t N, int64_t K) {
+    if (M <= 1 || K % 128) return false;
+    if (qtype != LOWBIT_QT_SYM_INT4 && qtype != LOWBIT_QT_ASYM_INT4 && qtype != LOWBIT_QT_FP8_E4M3) return false;
+    return M <= 48 || (M <= 64 && K % 256 == 0 && N % 64 == 0);
+}
+
+int device_layout(int qtype, int64_t N, int64_t K) {
+    return api.tileable(qtype, N, K) ? LOWBIT_LAYOUT_TILED : LOWBIT_LAYOUT_GGML;
+}
+
+at::DimVector with_last(const Tensor &x, int64_t last) {
+    at::DimVector shape(x.sizes().begin(), x.sizes().end());
+    shape.back() = last;
+    return shape;
+}
+
+// LowBitLinear at inference on a GPU-resident weight; an undefined tensor when this is not the plain case
+Tensor linear(const Tensor &x_in, const Tensor &w, const Tensor &bias, int qtype, int64_t N, bool conver_to_half) {
+    if (!on_gpu(x_in) || x_in.dim() < 1 || x_in.numel() == 0 || dtype_code(x_in.scalar_type()) < 0) return {};
+    const int64_t K = x_in.size(-1), M = x_in.numel() / K;
+    if (!is_blob(w, x_in, qtype, N, K)) return {};
+    if (bias.defined() && (bias.scalar_type() != x_in.scalar_type() || bias.device() != x_in.device() || bias.numel() != N ||
+                           (bias.requires_grad() && c10::GradMode::is_enabled()))) return {};
+    const Tensor x = x_in.is_contiguous() ? x_in : x_in.contiguous();
+    const int layout = device_layout(qtype, N, K);
+    const auto shape = with_last(x, N);
+    if (x.scalar_type() == at::kFloat && conver_to_half && M > 1 && !batch_stays_f32(qtype, M, N, K)) {
+        Tensor y = product(x.to(at::kHalf), w, Tensor(), qtype, layout, M, N, K, shape).to(at::kFloat);
+        if (bias.defined()) y.add_(bias);
+        return y;
+    }
+    return product(x, w, bias, qtype, layout, M, N, K, shape);
+}
+
+// act(x Wg^T) * (x Wu^T) for 16-bit x and tiled weights; an undefined tensor when this is not the plain case
+Tensor gated(const Tensor &x_in, const Tensor &wg, const Tensor &wu, int qtype, int64_t N, int act) {
+    if (!on_gpu(x_in) || x_in.dim() < 1 || x_in.numel() == 0) return {};
+    const int dt = dtype_code(x_in.scalar_type());
+    if (dt != LOWBIT_DT_F16 && dt != LOWBIT_DT_BF16) return {};
+    const int64_t K = x_in.size(-1), M = x_in.numel() / K;
+    if (!is_blob(wg, x_in, qtype, N, K) || !is_blob(wu, x_in, qtype, N, K) || !api.tileable(qtype, N, K)) return {};
+    const Tensor x = x_in.is_contiguous() ? x_in : x_in.contiguous();
+    c10::DeviceGuard guard(x.device());
+    Tensor y = at::empty(with_last(x, N), x.options());
+    check(api.mlp_forward(x.const_data_ptr(), wg.const_data_ptr(), wu.const_data_ptr(), y.data_ptr(), qtype, dt, M, N, K, act,
+                          current_stream(x)), "lowbit_mlp_forward");
+    return y;
+}
+
+// rows ids[i] of the dequantized [N, K] table, in `dtype`; an undefined tensor when this is not the plain case
+Tensor embedding(const Tensor &ids_in, const Tensor &w, int qtype, int64_t N, int64_t K, at::ScalarType dtype) {
+    if (!on_gpu(ids_in) || ids_in.numel() == 0 || ids_in.scalar_type() != at::kLong || !is_blob(w, ids_in, qtype, N, K)) return {};
+    const int dt = dtype_code(dtype);
+    if (dt < 0) return {};
+    const Tensor ids = ids_in.contiguous();
+    c10::DeviceGuard guard(ids.device());
+    at::DimVector shape(ids.sizes().begin(), ids.sizes().end());
+    shape.push_back(K);
+    Tensor y = at::empty(shape, ids.options().dtype(dtype));
+    check(api.dequantize_rows(w.const_data_ptr(), ids.const_data_ptr<int64_t>(), ids.numel(), y.data_ptr(), qtype, N, K,
+                              device_layout(qtype, N, K), dt, current_stream(ids)), "lowbit_dequantize_rows");
+    return y;
+}
+
+// ------------------------------------------------------------------ CPython side
+
+// Arguments by position.  A tensor argument is a torch.Tensor or a Parameter (subclass): anything else, and a value
+// of the wrong kind, raises TypeError.
+struct Args {
+    PyObject *const *a;
+    Py_ssize_t n;
+    const Tensor &tensor(Py_ssize_t i) const {
+        if (!THPVariable_Check(a[i])) throw std::invalid_argument("a tensor is expected");
+        return THPVariable_Unpack(a[i]);
+    }
+    Tensor optional(Py_ssize_t i) const { return a[i] == Py_None ? Tensor() : tensor(i); }
+    int64_t integer(Py_ssize_t i) const {
+        const long long v = PyLong_AsLongLong(a[i]);
+        if (v == -1 && PyErr_Occurred()) { PyErr_Clear(); throw std::invalid_argument("an integer is expected"); }
+        return v;
+    }
+    bool truth(Py_ssize_t i) const { return PyObject_IsTrue(a[i]) == 1; }
+};
+
+// Runs fn (returning a Tensor) without the GIL and wraps the result, None for an undefined one.
+template <typename Fn> PyObject *answer(const char *name, Py_ssize_t got, Py_ssize_t want, Fn &&fn) {
+    HANDLE_TH_ERRORS
+    if (got != want) {
+        PyErr_Format(PyExc_TypeError, "%s takes %zd arguments (%zd given)", name, want, got);
+        return nullptr;
+    }
+    try {
+        Tensor y = fn();
+        if (!y.defined()) Py_RETURN_NONE;
+        return THPVariable_Wrap(std::move(y));
+    } catch (const std::invalid_argument &e) {
+        PyErr_Format(PyExc_TypeError, "%s: %s", name, e.what());
+    } catch (const Failed &e) {
+        PyErr_SetString(PyExc_RuntimeError, e.what());
+    }
+    return nullptr;
+    END_HANDLE_TH_ERRORS
+}
+
+struct NoGil {
+    PyThreadState *state = PyEval_SaveThread();
+    ~NoGil() { PyEval_RestoreThread(state); }
+};
+
+PyObject *py_bind(PyObject *, PyObject *const *args, Py_ssize_t n) {
+    if (n != 1 || !PyDict_Check(args[0])) {
+        PyErr_SetString(PyExc_TypeError, "bind takes a dict of function addresses");
+        return nullptr;
+    }
+#define BIND(name)                                                                                 \
+    do {                                                                                           \
+        PyObject *v = PyDict_GetItemString(args[0], "lowbit_" #name);                              \
+        void *p = v ? PyLong_AsVoidPtr(v) : nullptr;                                               \
+        if (!p) {                                                                                  \
+            if (!PyErr_Occurred()) PyErr_SetString(PyExc_KeyError, "lowbit_" #name);               \
+            return nullptr;                                                                        \
+        }                                                                                          \
+        api.name = (decltype(api.name))p;                                                          \
+    } while (0)
+    BIND(last_error); BIND(blob_bytes); BIND(tileable); BIND(workspace_bytes_for); BIND(forward); BIND(forward_ws);
+    BIND(forward_f32_workspace_bytes); BIND(forward_f32); BIND(mlp_forward); BIND(dequantize_rows);
+#undef BIND
+    Py_RETURN_NONE;
+}
+
+// product(x [M, K] contiguous, w, qtype, layout, N) -> [M, N] in x's dtype; the caller has checked the arguments
+PyObject *py_product(PyObject *, PyObject *const *args, Py_ssize_t n) {
+    return answer("product", n, 5, [&] {
+        const Args a{args, n};
+        const Tensor &x = a.tensor(0), &w = a.tensor(1);
+        const int qtype = (int)a.integer(2), layout = (int)a.integer(3);
+        const int64_t N = a.integer(4), M = x.size(0), K = x.size(1);
+        NoGil free;
+        return product(x, w, Tensor(), qtype, layout, M, N, K, {M, N});
+    });
+}
+
+// linear(x, weight, bias or None, qtype, out_len, conver_to_half) -> y or None
+PyObject *py_linear(PyObject *, PyObject *const *args, Py_ssize_t n) {
+    return answer("linear", n, 6, [&] {
+        const Args a{args, n};
+        const Tensor &x = a.tensor(0), &w = a.tensor(1);
+        const Tensor bias = a.optional(2);
+        const int qtype = (int)a.integer(3);
+        const int64_t N = a.integer(4);
+        const bool half = a.truth(5);
+        NoGil free;
+        return linear(x, w, bias, qtype, N, half);
+    });
+}
+
+// gated(x, w_gate, w_up, qtype, out_len, act) -> y or None
+PyObject *py_gated(PyObject *, PyObject *const *args, Py_ssize_t n) {
+    return answer("gated", n, 6, [&] {
+        const Args a{args, n};
+        const Tensor &x = a.tensor(0), &wg = a.tensor(1), &wu = a.tensor(2);
+        const int qtype = (int)a.integer(3), act = (int)a.integer(5);
+        const int64_t N = a.integer(4);
+        NoGil free;
+        return gated(x, wg, wu, qtype, N, act);
+    });
+}
+
+// embedding(ids, weight, qtype, num_embeddings, embedding_dim, tensor of the result's dtype) -> rows or None
+PyObject *py_embedding(PyObject *, PyObject *const *args, Py_ssize_t n) {
+    return answer("embedding", n, 6, [&] {
+        const Args a{args, n};
+        const Tensor &ids = a.tensor(0), &w = a.tensor(1);
+        const int qtype = (int)a.integer(2);
+        const int64_t N = a.integer(3), K = a.integer(4);
+        const at::ScalarType dtype = a.tensor(5).scalar_type();
+        NoGil free;
+        return embedding(ids, w, qtype, N, K, dtype);
+    });
+}
+
+#define METHOD(name) {#name, (PyCFunction)(void (*)(void))py_##name, METH_FASTCALL, nullptr}
+PyMethodDef methods[] = {METHOD(bind), METHOD(product), METHOD(linear), METHOD(gated), METHOD(embedding),
+                         {nullptr, nullptr, 0, nullptr}};
+PyModuleDef module = {PyModuleDef_HEAD_INIT, "lowbit_torch", "native host path of the low-bit layers", -1, methods};
+
+}  // namespace
+
+PyMODINIT_FUNC PyInit_lowbit_torch(void) { return PyModule_Create(&module); }

@@ -11,6 +11,7 @@ from typing import Optional
 import torch
 from torch import Tensor
 
+from ipex_llm.transformers.native_ops import ops
 from ipex_llm.utils.common import invalidInputError
 
 
@@ -31,6 +32,12 @@ class LowBitEmbedding(torch.nn.Embedding):
 
     def forward(self, x: Tensor):
         from ipex_llm.transformers.low_bit_linear import dequantize_rows
+        table = self.qweight
+        if table.quantized and table._shape is not None:
+            # one native call: the rows come out in the model's dtype (None: not the plain case, the steps below)
+            rows = ops.embedding(x, table, table.qtype, self.num_embeddings, self.embedding_dim, self.weight)
+            if rows is not None:
+                return rows
         invalidInputError(x.device.type == "cuda", "`LowBitEmbedding` only supports GPU now.")
         invalidInputError(self.qweight.quantized and self.qweight.device == x.device,
                           "move the module to the GPU first: the table is quantized on the way")

@@ -24,6 +24,7 @@ from torch import nn
 
 import ipex_llm.ggml.model.llama.llama_cpp as ggml
 from ipex_llm.ggml.quantize import ggml_tensor_qtype
+from ipex_llm.transformers.native_ops import ops
 from ipex_llm.utils.common import invalidInputError
 
 TORCH_LINEAR_THRESHOLD = int(os.getenv("BIGDL_LLM_LINEAR_THRESHOLD", "512"))
@@ -42,7 +43,6 @@ FP16 = ggml_tensor_qtype["fp16"]
 BF16 = ggml_tensor_qtype["bf16"]
 
 _ACCEL = "cuda"   # device.type of an MI355X under PyTorch-ROCm
-_WORKSPACE_CAP = 256 << 20   # most that forward_new borrows for split-K partial sums
 _DT = {torch.float16: ggml.DT_F16, torch.bfloat16: ggml.DT_BF16, torch.float32: ggml.DT_F32}
 
 
@@ -246,32 +246,10 @@ def forward_new(x: torch.Tensor, w: torch.Tensor, qtype: int, output_size: int, 
     invalidInputError(w.numel() == ggml.lowbit_blob_bytes(qtype, output_size * k),
                       f"weight blob has {w.numel()} bytes, expected "
                       f"{ggml.lowbit_blob_bytes(qtype, output_size * k)} for [{output_size}, {k}]")
-    if keep_fp32 and x.dtype == torch.float32:
-        xc = x.contiguous()
-        y = torch.empty((m, output_size), dtype=torch.float32, device=x.device)
-        if m and output_size:
-            with torch.cuda.device(x.device):
-                ws_bytes = ggml.lowbit_forward_f32_workspace_bytes(m, output_size, k)
-                ws = torch.empty(ws_bytes, dtype=torch.uint8, device=x.device)
-                ggml.lowbit_forward_f32(xc.data_ptr(), w.data_ptr(), y.data_ptr(), qtype, layout, m, output_size, k,
-                                        ws.data_ptr(), ws_bytes, _stream())
-        return y
-    xc = x if x.dtype != torch.float32 else x.half()
-    xc = xc.contiguous()
-    y = torch.empty((m, output_size), dtype=xc.dtype, device=x.device)
-    if m and output_size:
-        with torch.cuda.device(x.device):
-            # workspace for the fp32 partial tiles of the batch-size kernel and of the GEMM when it
-            # splits K; taken from torch's caching allocator, so steady-state calls do not allocate
-            # (the library is told the budget and says what the plan it makes within it needs)
-            ws_bytes = ggml.lowbit_workspace_bytes_for(qtype, layout, m, output_size, k, _WORKSPACE_CAP)
-            if ws_bytes:
-                ws = torch.empty(ws_bytes, dtype=torch.uint8, device=x.device)
-                ggml.lowbit_forward_ws(xc.data_ptr(), w.data_ptr(), y.data_ptr(), qtype, layout, _DT[xc.dtype],
-                                       m, output_size, k, ws.data_ptr(), ws_bytes, _stream())
-            else:
-                ggml.lowbit_forward(xc.data_ptr(), w.data_ptr(), y.data_ptr(), qtype, layout, _DT[xc.dtype],
-                                    m, output_size, k, _stream())
+    xc = (x if x.dtype != torch.float32 or keep_fp32 else x.half()).contiguous()
+    if not m or not output_size:
+        return torch.empty((m, output_size), dtype=x.dtype, device=x.device)
+    y = ops.product(xc, w, qtype, layout, output_size)
     return y if y.dtype == x.dtype else y.to(x.dtype)
 
 
@@ -576,6 +554,15 @@ class LowBitLinear(nn.Linear):
             self.device = "mi355x" if self.weight.data.device.type == _ACCEL else "cpu"
             # 288 GB of HBM: the cache flush around lm_head is opt-in only
             self.low_memory_mode = self.low_memory_mode and os.environ.get("IPEX_LLM_LOW_MEM", None) == "1"
+        if not (self.training or self.act_order or self.low_memory_mode) and self.mp_group is None:
+            # inference on a GPU-resident weight: one native call (None: not the plain case, the steps below)
+            params = self._parameters
+            weight = params["weight"]
+            if weight.quantized and weight._shape is not None and weight.qtype == self.qtype:
+                y = ops.linear(reshape_lm_head_input(x) if self.optimize_lm_head else x, weight, params["bias"], self.qtype,
+                               self.out_len, self.conver_to_half)
+                if y is not None:
+                    return y
         is_training = self.training and not torch.is_inference_mode_enabled()
         if is_training and self.compute_dtype is not None and x.device.type == _ACCEL:
             x = x.to(self.compute_dtype)

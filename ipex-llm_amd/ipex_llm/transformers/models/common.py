@@ -6,6 +6,7 @@ from typing import List
 import torch
 
 import ipex_llm.ggml.model.llama.llama_cpp as ggml
+from ipex_llm.transformers.native_ops import ops
 
 
 def merge_linear(linears: List[torch.nn.Linear]) -> torch.nn.Linear:
@@ -139,6 +140,15 @@ def fuse_mlp_base(module: torch.nn.Module, act: int, x: torch.Tensor):
     from ipex_llm.transformers.models.utils import mlp_fusion_check
     gate, up = module.gate_proj, module.up_proj
     qtype = getattr(gate, "qtype", None)
+    if type(gate) is LowBitLinear and type(up) is LowBitLinear and not module.training and not x.requires_grad:
+        g, u = gate._parameters, up._parameters
+        wg, wu = g["weight"], u["weight"]
+        if (g["bias"] is None and u["bias"] is None and wg.quantized and wu.quantized and wg._shape is not None
+                and wu._shape is not None and up.qtype == qtype and up.out_len == gate.out_len):
+            # one native call (None: not the plain case, the steps below)
+            h = ops.gated(x, wg, wu, qtype, gate.out_len, act)
+            if h is not None:
+                return module.down_proj(h)
     fusable = (isinstance(gate, LowBitLinear) and isinstance(up, LowBitLinear)
                and gate.bias is None and up.bias is None
                and gate.weight.quantized and up.weight.quantized
