@@ -22,20 +22,18 @@ int launch_quantize(const float *src, void *dst, int qtype, int64_t N, int64_t K
 int launch_relayout(const void *src, void *dst, int qtype, int64_t N, int64_t K, int src_layout, hipStream_t st);
 int launch_dequantize(const void *w, void *out, int qtype, int64_t N, int64_t K, int layout, int out_dtype,
                       hipStream_t st);
-int launch_gemv(const void *x, const void *w, void *y, int qtype, int layout, int act_dtype, int M, int N, int K,
+int launch_gemv(const void *x, const void *w, const void *bias, void *y, int qtype, int layout, int act_dtype, int M, int N, int K,
                 int waves, hipStream_t st);
 size_t ring_workspace_bytes(int M, int N, int K, int wgs);
 double ring_time_us(int M, int N, int K, int qtype, bool have_ws);
-int launch_gemm_ring(const void *x, const void *w, void *y, int qtype, int act_dtype, int M, int N, int K,
+int launch_gemm_ring(const void *x, const void *w, const void *bias, void *y, int qtype, int act_dtype, int M, int N, int K,
                      void *workspace, size_t workspace_bytes, int wgs, hipStream_t st);
-int launch_gemm(const void *x, const void *w, void *y, int qtype, int layout, int act_dtype, int M, int N, int K,
+int launch_gemm(const void *x, const void *w, const void *bias, void *y, int qtype, int layout, int act_dtype, int M, int N, int K,
                 void *workspace, size_t workspace_bytes, int want_splits, hipStream_t st);
-int launch_gemm_narrow(const void *x, const void *w, void *y, int qtype, int act_dtype, int M, int N, int K, hipStream_t st);
+int launch_gemm_narrow(const void *x, const void *w, const void *bias, void *y, int qtype, int act_dtype, int M, int N, int K, hipStream_t st);
 double narrow_time_us(int M, int N, int K, int qtype);
 int gemm_splits(int M, int N, int K, size_t ws_bytes, int qtype);
 double gemm_time_us(int M, int N, int K, int splits, int qtype);
-int launch_gemv_bf16_f32out(const void *x, const void *w, void *y, int qtype, int layout, int M, int N, int K,
-                            hipStream_t st);
 int launch_grouped_gemm(const void *x, const void *const *w, const void *const *w_up, void *y, const int32_t *offsets,
                         int n_groups, int total_rows, int qtype, int act_dtype, int N, int K, int act, void *workspace,
                         size_t workspace_bytes, hipStream_t st);
@@ -167,7 +165,7 @@ int lowbit_gemv(const void *x, const void *w, void *y, int qtype, int layout, in
     if (int rc = check_mm("lowbit_gemv", x, w, y, qtype, layout, act_dtype, M, N, K)) return rc;
     if (M * N == 0) return 0;
     if (K == 0) return fail(LOWBIT_ESHAPE, "lowbit_gemv: K == 0");
-    return check_launch(launch_gemv(x, w, y, qtype, layout, act_dtype, (int)M, (int)N, (int)K, waves,
+    return check_launch(launch_gemv(x, w, nullptr, y, qtype, layout, act_dtype, (int)M, (int)N, (int)K, waves,
                                     (hipStream_t)stream), "lowbit_gemv");
 }
 
@@ -180,7 +178,7 @@ int lowbit_gemm_ring(const void *x, const void *w, void *y, int qtype, int layou
     if (((uintptr_t)y) & 7) return fail(LOWBIT_EARG, "%s: y must be 8-byte aligned", what);
     if (wgs < 0 || wgs > 65535) return fail(LOWBIT_EARG, "%s: wgs must be 0 (automatic) .. 65535", what);
     if (workspace && !aligned16(workspace)) return fail(LOWBIT_EARG, "%s: workspace must be 16-byte aligned", what);
-    return check_launch(launch_gemm_ring(x, w, y, qtype, act_dtype, (int)M, (int)N, (int)K, workspace,
+    return check_launch(launch_gemm_ring(x, w, nullptr, y, qtype, act_dtype, (int)M, (int)N, (int)K, workspace,
                                          workspace ? workspace_bytes : 0, wgs, (hipStream_t)stream), what);
 }
 
@@ -204,7 +202,7 @@ static int gemm_entry(const char *what, const void *x, const void *w, void *y, i
             return fail(LOWBIT_ESHAPE, "%s: %d splits need the tiled layout and at least as many 128-column steps", what,
                         splits);
     }
-    return check_launch(launch_gemm(x, w, y, qtype, layout, act_dtype, (int)M, (int)N, (int)K, workspace,
+    return check_launch(launch_gemm(x, w, nullptr, y, qtype, layout, act_dtype, (int)M, (int)N, (int)K, workspace,
                                     workspace ? workspace_bytes : 0, splits, (hipStream_t)stream), what);
 }
 
@@ -227,7 +225,7 @@ int lowbit_gemm_narrow(const void *x, const void *w, void *y, int qtype, int lay
     if (K == 0) return fail(LOWBIT_ESHAPE, "%s: K == 0", what);
     if (layout != LOWBIT_LAYOUT_TILED) return fail(LOWBIT_ESHAPE, "%s: needs the tiled layout", what);
     if (((uintptr_t)y) & 7) return fail(LOWBIT_EARG, "%s: y must be 8-byte aligned", what);
-    return check_launch(launch_gemm_narrow(x, w, y, qtype, act_dtype, (int)M, (int)N, (int)K, (hipStream_t)stream), what);
+    return check_launch(launch_gemm_narrow(x, w, nullptr, y, qtype, act_dtype, (int)M, (int)N, (int)K, (hipStream_t)stream), what);
 }
 
 // Row counts up to which lowbit_forward_ws considers the ring kernel (its estimate is fitted up to there): the
@@ -333,52 +331,57 @@ extern "C" int lowbit_forward_plan(int qtype, int layout, int64_t M, int64_t N, 
     return plan_forward(qtype, layout, M, N, K, have_workspace != 0, have_workspace ? workspace_bytes : 0, true, nullptr);
 }
 
-static int forward_any(const void *x, const void *w, void *y, int qtype, int layout, int act_dtype, int64_t M,
-                       int64_t N, int64_t K, void *workspace, size_t workspace_bytes, void *stream) {
-    int splits = 1;
-    switch (plan_forward(qtype, layout, M, N, K, workspace != nullptr, workspace_bytes, !(((uintptr_t)y) & 7), &splits)) {
-    case PLAN_GEMV: return lowbit_gemv(x, w, y, qtype, layout, act_dtype, M, N, K, 0, stream);
-    case PLAN_RING: return lowbit_gemm_ring(x, w, y, qtype, layout, act_dtype, M, N, K, workspace, workspace_bytes, 0, stream);
-    case PLAN_GEMM_SPLIT:
-        return lowbit_gemm_ws(x, w, y, qtype, layout, act_dtype, M, N, K, workspace, workspace_bytes, splits, stream);
-    case PLAN_GEMM_NARROW: return lowbit_gemm_narrow(x, w, y, qtype, layout, act_dtype, M, N, K, stream);
-    default: return lowbit_gemm(x, w, y, qtype, layout, act_dtype, M, N, K, stream);
+static int forward_any(const char *what, const void *x, const void *w, const void *bias, void *y, int qtype, int layout,
+                       int act_dtype, int64_t M, int64_t N, int64_t K, void *workspace, size_t workspace_bytes, void *stream) {
+    if (int rc = check_mm(what, x, w, y, qtype, layout, act_dtype, M, N, K)) return rc;
+    if (M * N == 0) return 0;
+    if (K == 0) return fail(LOWBIT_ESHAPE, "%s: K == 0", what);
+    if (workspace && !aligned16(workspace)) return fail(LOWBIT_EARG, "%s: workspace must be 16-byte aligned", what);
+    if (((uintptr_t)bias) & 1) return fail(LOWBIT_EARG, "%s: misaligned bias", what);
+    if (!workspace) workspace_bytes = 0;
+    const int m = (int)M, n = (int)N, k = (int)K;
+    hipStream_t st = (hipStream_t)stream;
+    int splits = 1, rc = 0;
+    switch (plan_forward(qtype, layout, M, N, K, workspace != nullptr, workspace_bytes, !(((uintptr_t)y | (uintptr_t)bias) & 7), &splits)) {
+    case PLAN_GEMV: rc = launch_gemv(x, w, bias, y, qtype, layout, act_dtype, m, n, k, 0, st); break;
+    case PLAN_RING: rc = launch_gemm_ring(x, w, bias, y, qtype, act_dtype, m, n, k, workspace, workspace_bytes, 0, st); break;
+    case PLAN_GEMM_SPLIT: rc = launch_gemm(x, w, bias, y, qtype, layout, act_dtype, m, n, k, workspace, workspace_bytes, splits, st); break;
+    case PLAN_GEMM_NARROW: rc = launch_gemm_narrow(x, w, bias, y, qtype, act_dtype, m, n, k, st); break;
+    default: rc = launch_gemm(x, w, bias, y, qtype, layout, act_dtype, m, n, k, nullptr, 0, 0, st); break;
     }
+    return check_launch(rc, what);
 }
 
 int lowbit_forward(const void *x, const void *w, void *y, int qtype, int layout, int act_dtype, int64_t M, int64_t N,
                    int64_t K, void *stream) {
-    return forward_any(x, w, y, qtype, layout, act_dtype, M, N, K, nullptr, 0, stream);
+    return forward_any("lowbit_forward", x, w, nullptr, y, qtype, layout, act_dtype, M, N, K, nullptr, 0, stream);
 }
 
 int lowbit_forward_ws(const void *x, const void *w, void *y, int qtype, int layout, int act_dtype, int64_t M, int64_t N,
                       int64_t K, void *workspace, size_t workspace_bytes, void *stream) {
-    if (workspace && !aligned16(workspace))
-        return fail(LOWBIT_EARG, "lowbit_forward_ws: workspace must be 16-byte aligned");
-    return forward_any(x, w, y, qtype, layout, act_dtype, M, N, K, workspace, workspace ? workspace_bytes : 0, stream);
+    return forward_any("lowbit_forward_ws", x, w, nullptr, y, qtype, layout, act_dtype, M, N, K, workspace, workspace_bytes, stream);
 }
 
-// ---- lowbit_forward_f32: fp32 activations in, fp32 out
-//
-// The MFMA operands are 16-bit, so x is split into two bf16 planes, hi = bf16(x) and lo = bf16(x - hi)
-// (16 mantissa bits together, fp32's exponent range: no overflow whatever the magnitude of x), the product
-// runs on the 2M rows with fp32 output and the two halves are added.
-__global__ __launch_bounds__(256) void split_bf16_kernel(const float *__restrict__ x, __bf16 *__restrict__ hi,
-                                                         __bf16 *__restrict__ lo, int64_t n) {
-    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (i >= n) return;
-    const float v = x[i];
-    const __bf16 h = (__bf16)v;                              // round to nearest even
-    const float r = v - (float)h;                            // exact: both share the leading bits
-    hi[i] = h;
-    lo[i] = (r == r && (r - r) == 0.0f) ? (__bf16)r : (__bf16)0.0f;   // inf / nan stay in the hi plane only
-}
-__global__ __launch_bounds__(256) void add_f32_kernel(const float *__restrict__ a, const float *__restrict__ b,
-                                                      float *__restrict__ y, int64_t n) {
-    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (i < n) y[i] = a[i] + b[i];
+// ---- fp32 activations: the streaming kernel's F32 form for every M
+static int forward_f32(const char *what, const float *x, const void *w, const float *bias, float *y, int qtype, int layout,
+                       int64_t M, int64_t N, int64_t K, void *stream) {
+    if (int rc = check_weight_shape(what, qtype, N, K, layout)) return rc;
+    if (M < 0 || M > 0x3fffffff) return fail(LOWBIT_EARG, "%s: bad M", what);
+    if (M * N * K == 0) return 0;
+    if (!x || !w || !y || !aligned16(x) || !aligned16(w) || (((uintptr_t)y | (uintptr_t)bias) & 3))
+        return fail(LOWBIT_EARG, "%s: null or misaligned pointer (x, w: 16 bytes)", what);
+    if (K % 8) return fail(LOWBIT_ESHAPE, "%s: K must be a multiple of 8", what);
+    return check_launch(launch_gemv(x, w, bias, y, qtype, layout, LOWBIT_DT_F32, (int)M, (int)N, (int)K, 0, (hipStream_t)stream), what);
 }
 
+int lowbit_linear(const void *x, const void *w, const void *bias, void *y, int qtype, int layout, int dtype, int64_t M,
+                  int64_t N, int64_t K, void *workspace, size_t workspace_bytes, void *stream) {
+    if (dtype == LOWBIT_DT_F32)
+        return forward_f32("lowbit_linear", (const float *)x, w, (const float *)bias, (float *)y, qtype, layout, M, N, K, stream);
+    return forward_any("lowbit_linear", x, w, bias, y, qtype, layout, dtype, M, N, K, workspace, workspace_bytes, stream);
+}
+
+// ---- lowbit_forward_f32.  The workspace is part of the interface; the kernel keeps x's two planes in LDS and needs none.
 static size_t f32_plane_bytes(int64_t M, int64_t K) { return ((size_t)(2 * M * K * 2) + 255) & ~(size_t)255; }
 
 extern "C" size_t lowbit_forward_f32_workspace_bytes(int64_t M, int64_t N, int64_t K) {
@@ -389,24 +392,10 @@ extern "C" size_t lowbit_forward_f32_workspace_bytes(int64_t M, int64_t N, int64
 extern "C" int lowbit_forward_f32(const float *x, const void *w, float *y, int qtype, int layout, int64_t M, int64_t N,
                                   int64_t K, void *workspace, size_t workspace_bytes, void *stream) {
     const char *what = "lowbit_forward_f32";
-    if (int rc = check_weight_shape(what, qtype, N, K, layout)) return rc;
-    if (M < 0 || M > 0x3fffffff) return fail(LOWBIT_EARG, "%s: bad M", what);
-    if (M * N * K == 0) return 0;
-    if (!x || !w || !y || !aligned16(x) || !aligned16(w) || (((uintptr_t)y) & 3))
-        return fail(LOWBIT_EARG, "%s: null or misaligned pointer (x, w: 16 bytes)", what);
-    if (K % 8) return fail(LOWBIT_ESHAPE, "%s: K must be a multiple of 8", what);
     const size_t need = lowbit_forward_f32_workspace_bytes(M, N, K);
-    if (!workspace || !aligned16(workspace) || workspace_bytes < need)
+    if (need && (!workspace || !aligned16(workspace) || workspace_bytes < need))
         return fail(LOWBIT_ESIZE, "%s: needs %zu bytes of 16-byte aligned workspace", what, need);
-    hipStream_t st = (hipStream_t)stream;
-    __bf16 *planes = (__bf16 *)workspace;
-    float *y2 = (float *)((uint8_t *)workspace + f32_plane_bytes(M, K));
-    const int64_t nx = M * K, ny = M * N;
-    hipLaunchKernelGGL(split_bf16_kernel, dim3((unsigned)((nx + 255) / 256)), dim3(256), 0, st, x, planes, planes + nx, nx);
-    if (int rc = check_launch(launch_gemv_bf16_f32out(planes, w, y2, qtype, layout, (int)(2 * M), (int)N, (int)K, st), what))
-        return rc;
-    hipLaunchKernelGGL(add_f32_kernel, dim3((unsigned)((ny + 255) / 256)), dim3(256), 0, st, y2, y2 + ny, y, ny);
-    return check_hip(hipGetLastError(), what);
+    return forward_f32(what, x, w, nullptr, y, qtype, layout, M, N, K, stream);
 }
 
 // ---- lowbit_forward_noalloc: lowbit_forward_ws over a workspace that is part of the library's image.
@@ -453,10 +442,10 @@ int lowbit_forward_noalloc(const void *x, const void *w, void *y, int qtype, int
         return fail(LOWBIT_ESIZE, "%s: [%lld x %lld] at M = %lld wants %zu bytes of workspace, the built-in scratch holds "
                     "%zu; use lowbit_forward_ws with a caller-owned workspace", what, (long long)N, (long long)K,
                     (long long)M, need, NOALLOC_SCRATCH_BYTES);
-    if (!need) return forward_any(x, w, y, qtype, layout, act_dtype, M, N, K, nullptr, 0, stream);
+    if (!need) return forward_any(what, x, w, nullptr, y, qtype, layout, act_dtype, M, N, K, nullptr, 0, stream);
     void *ws = scratch_of_current_device(what);
     if (!ws) return LOWBIT_EHIP;
-    return forward_any(x, w, y, qtype, layout, act_dtype, M, N, K, ws, need, stream);
+    return forward_any(what, x, w, nullptr, y, qtype, layout, act_dtype, M, N, K, ws, need, stream);
 }
 
 int lowbit_dequantize_rows(const void *w, const int64_t *rows, int64_t n_rows, void *dst, int qtype, int64_t N,

@@ -18,14 +18,14 @@
 
 namespace lowbit {
 
-int launch_gemv(const void *x, const void *w, void *y, int qtype, int layout, int act_dtype, int M, int N, int K,
+int launch_gemv(const void *x, const void *w, const void *bias, void *y, int qtype, int layout, int act_dtype, int M, int N, int K,
                 int waves, hipStream_t st);
 
 // Sums the fp32 partial tiles of the splits (stored in the GEMM's register layout: split, tile, wave,
 // register group, lane) and writes y, rounded once.  One thread per group of 4 consecutive n.
 template <typename AT>
-__global__ __launch_bounds__(256) void splitk_reduce_kernel(const float *__restrict__ ws, AT *__restrict__ y, int M,
-                                                            int N, int splits) {
+__global__ __launch_bounds__(256) void splitk_reduce_kernel(const float *__restrict__ ws, AT *__restrict__ y,
+                                                            const AT *__restrict__ bias, int M, int N, int splits) {
     const int tiles_n = (N + GN - 1) / GN;
     const int64_t n_tiles_all = (int64_t)((M + GM - 1) / GM) * tiles_n;
     const int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x;       // (tile, wave, group, lane)
@@ -44,7 +44,7 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float *__restr
     typedef AT at4 __attribute__((ext_vector_type(4)));
     at4 o;
 #pragma unroll
-    for (int k = 0; k < 4; k++) o[k] = to_at<AT>(a[k]);
+    for (int k = 0; k < 4; k++) o[k] = to_at<AT>(bias ? a[k] + (float)bias[n + k] : a[k]);
     *(at4 *)(y + (int64_t)m * N + n) = o;
 }
 
@@ -147,7 +147,7 @@ static int band_rows(int tiles_m) {
 }
 
 template <int QT, typename AT>
-static int launch_gemm_t(const void *x, const void *w, void *y, int M, int N, int K, float *ws, int splits,
+static int launch_gemm_t(const void *x, const void *w, const void *bias, void *y, int M, int N, int K, float *ws, int splits,
                          hipStream_t st) {
     if (splits <= 1) ws = nullptr;
     const int G = K / TILE_COLS;
@@ -160,6 +160,8 @@ static int launch_gemm_t(const void *x, const void *w, void *y, int M, int N, in
     }();
     // tall form on the left columns, 128-row form on the rest (both in the same stream, the second starts when
     // the tall tiles, which all take the same time, are done)
+    GroupArgs ga{};
+    ga.bias = bias;
     const int tall = ws ? 0 : tall_columns(M, N, K, n_cus, QT == QT_SYM_INT8 || QT == QT_NF4);
     if (tall > 0) {
         const int tiles_m = M / GM_TALL;
@@ -169,10 +171,10 @@ static int launch_gemm_t(const void *x, const void *w, void *y, int M, int N, in
         // with four waves, which read each x operand from LDS once per two MFMAs.
         if constexpr (QT == QT_NF4)
             hipLaunchKernelGGL((gemm_mfma_kernel<QT, AT, true, MB32_TALL, false, false, 8>), dim3(grid), dim3(512), 0, st,
-                               (const AT *)x, (const uint8_t *)w, (AT *)y, M, N, K, band_rows(tiles_m), GroupArgs{}, G, (float *)nullptr, 0, tall);
+                               (const AT *)x, (const uint8_t *)w, (AT *)y, M, N, K, band_rows(tiles_m), ga, G, (float *)nullptr, 0, tall);
         else
             hipLaunchKernelGGL((gemm_mfma_kernel<QT, AT, true, MB32_TALL>), dim3(grid), dim3(256), 0, st,
-                               (const AT *)x, (const uint8_t *)w, (AT *)y, M, N, K, band_rows(tiles_m), GroupArgs{}, G, (float *)nullptr, 0, tall);
+                               (const AT *)x, (const uint8_t *)w, (AT *)y, M, N, K, band_rows(tiles_m), ga, G, (float *)nullptr, 0, tall);
         if (tall == tiles_n_all) return 0;
     }
     const int tn0 = tall, tiles_n = tiles_n_all - tall;
@@ -182,7 +184,6 @@ static int launch_gemm_t(const void *x, const void *w, void *y, int M, int N, in
     const int ny = ws ? (G + k_steps - 1) / k_steps : 1;             // splits that actually hold steps
     const bool fits24 = M < (1 << 24) && K < (1 << 23);              // 24-bit row offsets
     const bool dma = fits24 && (QT != QT_NF4 || tiles_m * tiles_n * ny > 256);
-    GroupArgs ga{};
     ga.split_tail = (dma && !ws) ? split_tail_tiles(M, (int64_t)tiles_m * tiles_n, n_cus) : 0;
     dim3 grid(8 * (unsigned)(((int64_t)tiles_m * tiles_n + 7) / 8 + ga.split_tail), ny);
     // Two forms of the kernel.  The DMA form (x straight into LDS, one K step of prefetch, 128 vector registers)
@@ -194,11 +195,11 @@ static int launch_gemm_t(const void *x, const void *w, void *y, int M, int N, in
                            (AT *)y, M, N, K, band_m, ga, k_steps, ws, tn0, tiles_n);
     else
         hipLaunchKernelGGL((gemm_mfma_kernel<QT, AT, false, MB32>), grid, dim3(256), 0, st, (const AT *)x, (const uint8_t *)w,
-                           (AT *)y, M, N, K, band_m, GroupArgs{}, k_steps, ws, tn0, tiles_n);
+                           (AT *)y, M, N, K, band_m, ga, k_steps, ws, tn0, tiles_n);
     if (ws) {
         const int64_t threads = (int64_t)tiles_m * tiles_n * (GM * GN / 4);
         hipLaunchKernelGGL((splitk_reduce_kernel<AT>), dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, st, ws,
-                           (AT *)y, M, N, ny);
+                           (AT *)y, (const AT *)bias, M, N, ny);
     }
     return 0;
 }
@@ -226,12 +227,13 @@ double narrow_time_us(int M, int N, int K, int qtype) {
 
 // The narrow form of the 128-row DMA kernel: tiles of 128 x 128, or 64 x 128 (narrow_halves).
 template <int QT, typename AT>
-static int launch_gemm_narrow_t(const void *x, const void *w, void *y, int M, int N, int K, hipStream_t st) {
+static int launch_gemm_narrow_t(const void *x, const void *w, const void *bias, void *y, int M, int N, int K, hipStream_t st) {
     if (M >= (1 << 24) || K >= (1 << 23)) return -3;                 // 24-bit row offsets
     const int G = K / TILE_COLS;
     const int tiles_n = (N + GN / 2 - 1) / (GN / 2), tiles_m = (M + GM - 1) / GM;
     const bool halves = narrow_halves(M, N);
     GroupArgs ga{};
+    ga.bias = bias;
     ga.split_tail = halves ? (int)(((int64_t)tiles_m * tiles_n) / 8) + 1 : 0;
     dim3 grid(8 * (unsigned)(((int64_t)tiles_m * tiles_n + 7) / 8 + ga.split_tail), 1);
     hipLaunchKernelGGL((gemm_mfma_kernel<QT, AT, true, MB32, false, false, 4, true>), grid, dim3(256), 0, st, (const AT *)x,
@@ -240,48 +242,48 @@ static int launch_gemm_narrow_t(const void *x, const void *w, void *y, int M, in
 }
 
 template <int QT>
-static int launch_gemm_narrow_q(const void *x, const void *w, void *y, int dt, int M, int N, int K, hipStream_t st) {
-    if (dt == DT_F16) return launch_gemm_narrow_t<QT, _Float16>(x, w, y, M, N, K, st);
-    if (dt == DT_BF16) return launch_gemm_narrow_t<QT, __bf16>(x, w, y, M, N, K, st);
+static int launch_gemm_narrow_q(const void *x, const void *w, const void *bias, void *y, int dt, int M, int N, int K, hipStream_t st) {
+    if (dt == DT_F16) return launch_gemm_narrow_t<QT, _Float16>(x, w, bias, y, M, N, K, st);
+    if (dt == DT_BF16) return launch_gemm_narrow_t<QT, __bf16>(x, w, bias, y, M, N, K, st);
     return -4;
 }
 
-int launch_gemm_narrow(const void *x, const void *w, void *y, int qtype, int act_dtype, int M, int N, int K, hipStream_t st) {
+int launch_gemm_narrow(const void *x, const void *w, const void *bias, void *y, int qtype, int act_dtype, int M, int N, int K, hipStream_t st) {
     if (M == 0 || N == 0) return 0;
     switch (qtype) {
-    case QT_SYM_INT4: return launch_gemm_narrow_q<QT_SYM_INT4>(x, w, y, act_dtype, M, N, K, st);
-    case QT_ASYM_INT4: return launch_gemm_narrow_q<QT_ASYM_INT4>(x, w, y, act_dtype, M, N, K, st);
-    case QT_SYM_INT8: return launch_gemm_narrow_q<QT_SYM_INT8>(x, w, y, act_dtype, M, N, K, st);
-    case QT_NF4: return launch_gemm_narrow_q<QT_NF4>(x, w, y, act_dtype, M, N, K, st);
-    case QT_FP8_E4M3: return launch_gemm_narrow_q<QT_FP8_E4M3>(x, w, y, act_dtype, M, N, K, st);
+    case QT_SYM_INT4: return launch_gemm_narrow_q<QT_SYM_INT4>(x, w, bias, y, act_dtype, M, N, K, st);
+    case QT_ASYM_INT4: return launch_gemm_narrow_q<QT_ASYM_INT4>(x, w, bias, y, act_dtype, M, N, K, st);
+    case QT_SYM_INT8: return launch_gemm_narrow_q<QT_SYM_INT8>(x, w, bias, y, act_dtype, M, N, K, st);
+    case QT_NF4: return launch_gemm_narrow_q<QT_NF4>(x, w, bias, y, act_dtype, M, N, K, st);
+    case QT_FP8_E4M3: return launch_gemm_narrow_q<QT_FP8_E4M3>(x, w, bias, y, act_dtype, M, N, K, st);
     default: return -2;
     }
 }
 
 template <int QT>
-static int launch_gemm_q(const void *x, const void *w, void *y, int dt, int M, int N, int K, float *ws, int splits,
+static int launch_gemm_q(const void *x, const void *w, const void *bias, void *y, int dt, int M, int N, int K, float *ws, int splits,
                          hipStream_t st) {
-    if (dt == DT_F16) return launch_gemm_t<QT, _Float16>(x, w, y, M, N, K, ws, splits, st);
-    if (dt == DT_BF16) return launch_gemm_t<QT, __bf16>(x, w, y, M, N, K, ws, splits, st);
+    if (dt == DT_F16) return launch_gemm_t<QT, _Float16>(x, w, bias, y, M, N, K, ws, splits, st);
+    if (dt == DT_BF16) return launch_gemm_t<QT, __bf16>(x, w, bias, y, M, N, K, ws, splits, st);
     return -4;
 }
 
 // splits: 0 = chosen here from the workspace size, otherwise as given (the caller has checked that it fits)
-int launch_gemm(const void *x, const void *w, void *y, int qtype, int layout, int act_dtype, int M, int N, int K,
+int launch_gemm(const void *x, const void *w, const void *bias, void *y, int qtype, int layout, int act_dtype, int M, int N, int K,
                 void *workspace, size_t workspace_bytes, int want_splits, hipStream_t st) {
     if (M == 0 || N == 0) return 0;
     // the MFMA GEMM reads the tiled layout and stores 8-byte groups of y (N % 4 == 0 is implied
     // by N % 16 == 0); anything else goes through the streaming kernel in 16-row slices
     if (layout != LAYOUT_TILED || (N % TILE_ROWS) || (K % TILE_COLS) || (((uintptr_t)y) & 7))
-        return launch_gemv(x, w, y, qtype, layout, act_dtype, M, N, K, 0, st);
+        return launch_gemv(x, w, bias, y, qtype, layout, act_dtype, M, N, K, 0, st);
     float *ws = (float *)workspace;
     const int splits = !ws ? 1 : want_splits > 0 ? want_splits : gemm_splits(M, N, K, workspace_bytes, qtype);
     switch (qtype) {
-    case QT_SYM_INT4: return launch_gemm_q<QT_SYM_INT4>(x, w, y, act_dtype, M, N, K, ws, splits, st);
-    case QT_ASYM_INT4: return launch_gemm_q<QT_ASYM_INT4>(x, w, y, act_dtype, M, N, K, ws, splits, st);
-    case QT_SYM_INT8: return launch_gemm_q<QT_SYM_INT8>(x, w, y, act_dtype, M, N, K, ws, splits, st);
-    case QT_NF4: return launch_gemm_q<QT_NF4>(x, w, y, act_dtype, M, N, K, ws, splits, st);
-    case QT_FP8_E4M3: return launch_gemm_q<QT_FP8_E4M3>(x, w, y, act_dtype, M, N, K, ws, splits, st);
+    case QT_SYM_INT4: return launch_gemm_q<QT_SYM_INT4>(x, w, bias, y, act_dtype, M, N, K, ws, splits, st);
+    case QT_ASYM_INT4: return launch_gemm_q<QT_ASYM_INT4>(x, w, bias, y, act_dtype, M, N, K, ws, splits, st);
+    case QT_SYM_INT8: return launch_gemm_q<QT_SYM_INT8>(x, w, bias, y, act_dtype, M, N, K, ws, splits, st);
+    case QT_NF4: return launch_gemm_q<QT_NF4>(x, w, bias, y, act_dtype, M, N, K, ws, splits, st);
+    case QT_FP8_E4M3: return launch_gemm_q<QT_FP8_E4M3>(x, w, bias, y, act_dtype, M, N, K, ws, splits, st);
     default: return -2;
     }
 }

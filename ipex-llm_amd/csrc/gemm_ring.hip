@@ -62,8 +62,8 @@ __host__ __device__ inline int ring_owner(int u, int q, int r) {
 // MB = 32-row blocks of x per workgroup, RNB = 32-row weight blocks per wave, S = ring stages
 template <int QT, typename AT, int MB, int RNB, int S>
 __global__ __launch_bounds__(64 * RING_WAVES, 1) void gemm_ring_kernel(const AT *__restrict__ x, const uint8_t *__restrict__ w,
-                                                                  AT *__restrict__ y, int M, int N, int K, int seg_slots,
-                                                                  int run_q, int run_r, float *__restrict__ ws) {
+                                                                  AT *__restrict__ y, const AT *__restrict__ bias, int M, int N, int K,
+                                                                  int seg_slots, int run_q, int run_r, float *__restrict__ ws) {
     using F = Fmt<QT>;
     using V8 = typename Vec8<AT>::type;
     constexpr int WAVES = RING_WAVES, NT = 2 * RNB * WAVES, RN = 16 * NT;   // tiles and weight rows per workgroup
@@ -204,15 +204,30 @@ __global__ __launch_bounds__(64 * RING_WAVES, 1) void gemm_ring_kernel(const AT 
     };
 
     f32x16 acc[MB][RNB];
-    auto clear_acc = [&]() {
+    // A segment starts from zero, the one that begins the walk along K from the bias: the sums start with it whether
+    // or not the tile is cut, and neither the stores nor the reduction have to know of it.
+    auto clear_acc = [&](int tile, bool first) {
+        const bool biased = bias != nullptr && first;
+#pragma unroll
+        for (int nb = 0; nb < RNB; nb++)
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+                typedef AT at4 __attribute__((ext_vector_type(4)));
+                at4 b = {};
+                if (biased) {
+                    const int n = (tile / tiles_m) * RN + wave * (32 * RNB) + nb * 32 + q * 8 + kg * 4;
+                    b = *(const at4 *)(bias + (n < N ? n : N - 4));
+                }
+#pragma unroll
+                for (int mb = 0; mb < MB; mb++)
+#pragma unroll
+                    for (int i = 0; i < 4; i++) acc[mb][nb][q * 4 + i] = (float)b[i];
+            }
 #pragma unroll
         for (int mb = 0; mb < MB; mb++)
 #pragma unroll
-            for (int nb = 0; nb < RNB; nb++)
-#pragma unroll
-                for (int i = 0; i < 16; i++) acc[mb][nb][i] = 0.0f;
+            for (int nb = 0; nb < RNB; nb++) asm volatile("" : "+a"(acc[mb][nb]));     // written here, not ahead of the first MFMA
     };
-    clear_acc();
 
     const DqCtx ctx = {lut, dq_magic<QT, AT>()};
     auto dequant_pair = [&](const WRegs &t, int ks, int nb, int p) -> uint32_t {
@@ -373,7 +388,7 @@ __global__ __launch_bounds__(64 * RING_WAVES, 1) void gemm_ring_kernel(const AT 
     for (int i = 0; i < n_units;) {
         const int seg_len = n_units - i < G - c_kt ? n_units - i : G - c_kt;
         const int seg_end = i + seg_len;
-        clear_acc();
+        clear_acc(c_tile, c_kt == 0);
         for (; i < seg_end; i++) {
             const int issued = n_units < i + S - 1 ? n_units : i + S - 1;
             wait_for(issued - i - 1);
@@ -500,7 +515,7 @@ size_t ring_workspace_bytes(int M, int N, int K, int wgs) {
 }
 
 template <int QT, typename AT, int MB, int RNB>
-static int launch_ring_m(const void *x, const void *w, void *y, int M, int N, int K, float *ws, const RingPlan &p,
+static int launch_ring_m(const void *x, const void *w, const void *bias, void *y, int M, int N, int K, float *ws, const RingPlan &p,
                          hipStream_t st) {
     constexpr int S = ring_stages<QT>(MB);
     constexpr int LDS = S * ring_stage_bytes<QT>(MB, RNB) + 64;
@@ -513,7 +528,7 @@ static int launch_ring_m(const void *x, const void *w, void *y, int M, int N, in
     const int64_t U = (int64_t)p.tiles * (K / TILE_COLS);
     if (U >= (int64_t)1 << 31) return -3;
     const int run_q = (int)(U / p.B), run_r = (int)(U % p.B);
-    hipLaunchKernelGGL(kern, dim3(p.B), dim3(64 * RING_WAVES), LDS, st, (const AT *)x, (const uint8_t *)w, (AT *)y, M, N, K,
+    hipLaunchKernelGGL(kern, dim3(p.B), dim3(64 * RING_WAVES), LDS, st, (const AT *)x, (const uint8_t *)w, (AT *)y, (const AT *)bias, M, N, K,
                        p.seg_slots, run_q, run_r, ws);
     if (p.ws_bytes) {
         constexpr int per_tile = (32 * MB) * (32 * RNB * RING_WAVES) / 4;     // threads: a multiple of 256
@@ -524,24 +539,24 @@ static int launch_ring_m(const void *x, const void *w, void *y, int M, int N, in
 }
 
 template <int QT, typename AT>
-static int launch_ring_t(const void *x, const void *w, void *y, int M, int N, int K, float *ws, const RingPlan &p,
+static int launch_ring_t(const void *x, const void *w, const void *bias, void *y, int M, int N, int K, float *ws, const RingPlan &p,
                          hipStream_t st) {
-    if (p.mb == 1) return launch_ring_m<QT, AT, 1, ring_rnb<QT>(1)>(x, w, y, M, N, K, ws, p, st);
-    if (p.mb == 2) return launch_ring_m<QT, AT, 2, ring_rnb<QT>(2)>(x, w, y, M, N, K, ws, p, st);
-    return launch_ring_m<QT, AT, 4, ring_rnb<QT>(4)>(x, w, y, M, N, K, ws, p, st);
+    if (p.mb == 1) return launch_ring_m<QT, AT, 1, ring_rnb<QT>(1)>(x, w, bias, y, M, N, K, ws, p, st);
+    if (p.mb == 2) return launch_ring_m<QT, AT, 2, ring_rnb<QT>(2)>(x, w, bias, y, M, N, K, ws, p, st);
+    return launch_ring_m<QT, AT, 4, ring_rnb<QT>(4)>(x, w, bias, y, M, N, K, ws, p, st);
 }
 
 template <int QT>
-static int launch_ring_q(const void *x, const void *w, void *y, int dt, int M, int N, int K, float *ws, const RingPlan &p,
+static int launch_ring_q(const void *x, const void *w, const void *bias, void *y, int dt, int M, int N, int K, float *ws, const RingPlan &p,
                          hipStream_t st) {
-    if (dt == DT_F16) return launch_ring_t<QT, _Float16>(x, w, y, M, N, K, ws, p, st);
-    if (dt == DT_BF16) return launch_ring_t<QT, __bf16>(x, w, y, M, N, K, ws, p, st);
+    if (dt == DT_F16) return launch_ring_t<QT, _Float16>(x, w, bias, y, M, N, K, ws, p, st);
+    if (dt == DT_BF16) return launch_ring_t<QT, __bf16>(x, w, bias, y, M, N, K, ws, p, st);
     return -4;
 }
 
 // Tiled layout only; the caller has checked the shape and the alignment of y (8 bytes).  A workspace
 // smaller than ring_workspace_bytes() for the same `wgs` is not used: the tiles are then not cut.
-int launch_gemm_ring(const void *x, const void *w, void *y, int qtype, int act_dtype, int M, int N, int K,
+int launch_gemm_ring(const void *x, const void *w, const void *bias, void *y, int qtype, int act_dtype, int M, int N, int K,
                      void *workspace, size_t workspace_bytes, int wgs, hipStream_t st) {
     if (M == 0 || N == 0) return 0;
     const int rnb = ring_rnb_of(qtype, M <= 32 ? 1 : M <= 64 ? 2 : 4);
@@ -549,11 +564,11 @@ int launch_gemm_ring(const void *x, const void *w, void *y, int qtype, int act_d
     if (p.ws_bytes > workspace_bytes) p = ring_plan(M, N, K, rnb, wgs, false);
     float *ws = (float *)workspace;
     switch (qtype) {
-    case QT_SYM_INT4: return launch_ring_q<QT_SYM_INT4>(x, w, y, act_dtype, M, N, K, ws, p, st);
-    case QT_ASYM_INT4: return launch_ring_q<QT_ASYM_INT4>(x, w, y, act_dtype, M, N, K, ws, p, st);
-    case QT_SYM_INT8: return launch_ring_q<QT_SYM_INT8>(x, w, y, act_dtype, M, N, K, ws, p, st);
-    case QT_NF4: return launch_ring_q<QT_NF4>(x, w, y, act_dtype, M, N, K, ws, p, st);
-    case QT_FP8_E4M3: return launch_ring_q<QT_FP8_E4M3>(x, w, y, act_dtype, M, N, K, ws, p, st);
+    case QT_SYM_INT4: return launch_ring_q<QT_SYM_INT4>(x, w, bias, y, act_dtype, M, N, K, ws, p, st);
+    case QT_ASYM_INT4: return launch_ring_q<QT_ASYM_INT4>(x, w, bias, y, act_dtype, M, N, K, ws, p, st);
+    case QT_SYM_INT8: return launch_ring_q<QT_SYM_INT8>(x, w, bias, y, act_dtype, M, N, K, ws, p, st);
+    case QT_NF4: return launch_ring_q<QT_NF4>(x, w, bias, y, act_dtype, M, N, K, ws, p, st);
+    case QT_FP8_E4M3: return launch_ring_q<QT_FP8_E4M3>(x, w, bias, y, act_dtype, M, N, K, ws, p, st);
     default: return -2;
     }
 }

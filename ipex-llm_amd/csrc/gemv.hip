@@ -12,8 +12,12 @@
 //   and the block scale is applied to the fp32 MFMA result.  M <= 16 costs the
 //   same weight traffic as M = 1.  Algorithmic bytes per launch:
 //   N*K*TS/QK (weights) + M*K*2 (x) + M*N*2 (y).
-// gemv_generic_kernel: any layout / any shape fallback, one wave per row.
+// The same kernel serves weights in the row-major (ggml) layout, whatever their shape (ROWS, lowbit_rows.h), and
+// float32 activations (F32).
 #include "lowbit_mfma.h"
+#include "lowbit_rows.h"
+
+#include <type_traits>
 
 namespace lowbit {
 
@@ -187,6 +191,20 @@ template <typename AT> __device__ inline typename Vec8<AT>::type ones8() {
     return r;
 }
 
+// Eight floats -> their bf16 values and those of what the rounding dropped.  inf / nan stay in the first plane only.
+__device__ inline void split_f32(const u32x4 &a, const u32x4 &b, u32x4 &hi, u32x4 &lo) {
+    bf16x8 h, l;
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+        const float v = __builtin_bit_cast(float, i < 4 ? a[i] : b[i - 4]);
+        h[i] = (__bf16)v;                                   // round to nearest even
+        const float r = v - (float)h[i];                    // exact: both share the leading bits
+        l[i] = (r - r) == 0.0f ? (__bf16)r : (__bf16)0.0f;
+    }
+    hi = __builtin_bit_cast(u32x4, h);
+    lo = __builtin_bit_cast(u32x4, l);
+}
+
 // ------------------------------------------------------------ MFMA GEMV
 
 constexpr int GEMV_MAX_WAVES = 16;
@@ -217,13 +235,23 @@ constexpr int GEMV_LDS_X_BUDGET = 64 * 1024;
 //             tile g of the K walk belongs to slot g / ge and is scaled by route_w[slot]:
 //             y = sum_j route_w[j] * (x_j Wd[e_j]^T).
 //
-// F32OUT: y is float [M, N] instead of AT (the fp32 path of lowbit_forward_f32: x arrives as two bf16 planes,
-// the sums must not be rounded to 8 bits on the way out).
-template <int QT, typename AT, int MT, int U, int XN, bool DUAL, int MOE, int R, bool F32OUT>
+// F32 (lowbit_forward_f32): x, bias and y are float.  The MFMA operands are 16-bit, so AT is bf16 and each value of x
+// becomes two on its way into LDS, hi = bf16(x) and lo = bf16(x - hi): 16 mantissa bits and fp32's exponent range.  Both
+// go through the MFMA into the same fp32 accumulator.  (Splitting x in a kernel of its own, running its 2M rows as rows
+// of a 16-bit product and adding the halves in a third kernel was 15.6 us of GPU time at 12 rows on [4096 x 4096] in
+// sym_int4, two passes over the weights; this way it is one pass of 10.1 us.)
+//
+// ROWS: the weight is in the row-major layout and of any shape: N rows of which the last workgroup's may be fewer than
+// 16, K any multiple of the block.  Loads and operand order as lowbit_rows.h says; everything else is the tiled
+// kernel.  A row of a tile is 72 .. 136 contiguous bytes instead of a 1 KiB tile; a workgroup's waves take
+// neighbouring columns, so lines are shared within the workgroup only.  (One wave per weight row and a scalar decode
+// per weight, four rows of x a pass, took 74 us per pass for [32003 x 4096] in asym_int4; at eight rows two passes, 29 us now.)
+template <int QT, typename AT, int MT, int U, int XN, bool DUAL, int MOE, int R, bool F32, bool ROWS>
 __global__ __launch_bounds__(1024) void gemv_mfma_kernel(const AT *__restrict__ x, const uint8_t *__restrict__ w,
-                                                         const uint8_t *__restrict__ w2, AT *__restrict__ y, int M,
-                                                         int N, int K, int act, const int32_t *__restrict__ ids,
-                                                         const float *__restrict__ route_w, int ge, int n_exp) {
+                                                         const uint8_t *__restrict__ w2, AT *__restrict__ y,
+                                                         const AT *__restrict__ bias, int M, int N, int K, int act,
+                                                         const int32_t *__restrict__ ids, const float *__restrict__ route_w,
+                                                         int ge, int n_exp) {
     using F = Fmt<QT>;
     using V8 = typename Vec8<AT>::type;
     constexpr bool IS4 = (F::BITS == 4);
@@ -231,7 +259,8 @@ __global__ __launch_bounds__(1024) void gemv_mfma_kernel(const AT *__restrict__ 
     constexpr float OFFSET = code_offset<QT, AT>();
     constexpr bool NEED_S = ASYM || OFFSET != 0.0f;
     constexpr int SLICE = U * TILE_COLS;                    // columns of x per wave and round
-    constexpr bool ZERO_X = XN == 1;                        // how tiles past K are silenced (see the x loads)
+    constexpr bool ZERO_X = XN == 1 || ROWS;                // how tiles past K are silenced (see the x loads)
+    constexpr int XREGION = XN * 512 * (F32 ? 2 : 1);       // elements of AT in a wave's part of LDS
 
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
     // tile rows walked side by side with one copy of x: the same row of two weights (DUAL) or R
@@ -239,13 +268,14 @@ __global__ __launch_bounds__(1024) void gemv_mfma_kernel(const AT *__restrict__ 
     // M = 16 a workgroup otherwise pulls 3.5 bytes of x out of L2 per byte of weight)
     constexpr int NW = DUAL ? 2 : R;
     static_assert(!(DUAL && R != 1) && XN * 1024 >= NW * MT * 256, "bad GEMV shape parameters");
+    static_assert(!ROWS || (!DUAL && MOE == 0), "row-major weights: the plain product only");
     // nf4 code book in the activation type (byte planes in registers).  With fp32 output a second table holds what
     // the rounding to AT dropped, and a second MFMA per sub-block adds it: the weights then carry 16 mantissa bits
     // like x does.
     const Nf4Planes lut_planes = (QT == QT_NF4) ? nf4_planes<AT, false>() : Nf4Planes{};
-    const Nf4Planes lut_lo_planes = (QT == QT_NF4 && F32OUT) ? nf4_planes<AT, true>() : Nf4Planes{};
+    const Nf4Planes lut_lo_planes = (QT == QT_NF4 && F32) ? nf4_planes<AT, true>() : Nf4Planes{};
     const void *const lut = &lut_planes, *const lut_lo = &lut_lo_planes;
-    constexpr bool NF4_IN_LDS = QT == QT_NF4 && MT == 1 && !F32OUT;     // (see Unpack<QT_NF4>)
+    constexpr bool NF4_IN_LDS = QT == QT_NF4 && MT == 1 && !F32;     // (see Unpack<QT_NF4>)
     __shared__ AT lut_lds[16];
     if constexpr (NF4_IN_LDS) {
         if (threadIdx.x < 16) lut_lds[threadIdx.x] = to_at<AT>(NF4_CODEBOOK[threadIdx.x]);
@@ -253,7 +283,7 @@ __global__ __launch_bounds__(1024) void gemv_mfma_kernel(const AT *__restrict__ 
     }
 
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, W = blockDim.x >> 6;
-    const int G = K / TILE_COLS;
+    const int G = ROWS ? (K + TILE_COLS - 1) / TILE_COLS : K / TILE_COLS;
     const int r = lane & 15, c = lane >> 4;
     // A rows: row r carries batch index (r/4)*MT + r%4 when r%4 < MT, so that the C registers
     // i < MT of lane group g hold batch indices g*MT + i and nothing else has to be scaled.
@@ -262,7 +292,15 @@ __global__ __launch_bounds__(1024) void gemv_mfma_kernel(const AT *__restrict__ 
     int m_of_r = (r >> 2) * MT + ((r & 3) < MT ? (r & 3) : MT - 1);
     m_of_r = m_of_r < M ? m_of_r : M - 1;
     gbytes wrow = nullptr, wrow2 = nullptr;
-    if constexpr (MOE == 0) {
+    gbytes wr[ROWS ? R : 1];                                // ROWS: this lane's row of each tile row
+    const int blocks = K / F::QK;
+    if constexpr (ROWS) {
+#pragma unroll
+        for (int wi = 0; wi < R; wi++) {
+            const int64_t n = ((int64_t)blockIdx.x * R + wi) * TILE_ROWS + r;
+            wr[wi] = (gbytes)w + (n < N ? n : N - 1) * (int64_t)blocks * F::TS;
+        }
+    } else if constexpr (MOE == 0) {
         wrow = (gbytes)w + (int64_t)blockIdx.x * R * G * F::TILE_BYTES;
         if constexpr (DUAL) wrow2 = (gbytes)w2 + (int64_t)blockIdx.x * G * F::TILE_BYTES;
     } else if constexpr (MOE == 1) {
@@ -279,7 +317,7 @@ __global__ __launch_bounds__(1024) void gemv_mfma_kernel(const AT *__restrict__ 
         return (gbytes)((const uint8_t *const *)w)[min(max(ids[slot], 0), n_exp - 1)] +
                ((int64_t)blockIdx.x * ge + (g - slot * ge)) * F::TILE_BYTES;
     };
-    AT *xs = (AT *)smem + (int64_t)wave * (XN * 512);       // [XN*64/(SLICE/8)][SLICE], private to this wave
+    AT *xs = (AT *)smem + (int64_t)wave * XREGION;          // [XN*64/(SLICE/8)][SLICE], private to this wave
     const AT *xa = xs + m_of_r * SLICE + 8 * c;
 
     float acc[NW * MT];
@@ -301,7 +339,7 @@ __global__ __launch_bounds__(1024) void gemv_mfma_kernel(const AT *__restrict__ 
         // then every weight tile of the round.  Loads return in order, so the LDS copy of x
         // waits for the x loads only and each tile is consumed as soon as it lands while the
         // later ones are still in flight.  XN = 16-byte chunks of x per lane (>= M*U/4).
-        u32x4 xv[XN];
+        u32x4 xv[F32 ? 2 * XN : XN];
 #pragma unroll
         for (int i = 0; i < XN; i++) {
             const int idx = i * 64 + lane;
@@ -316,33 +354,50 @@ __global__ __launch_bounds__(1024) void gemv_mfma_kernel(const AT *__restrict__ 
             // those shapes zero the scales (below).
             const bool past = col >= K;
             col = past ? K - 8 : col;
-            xv[i] = *(const u32x4 *)(x + (int64_t)m * K + col);
-            if constexpr (ZERO_X) xv[i] = past ? u32x4{0u, 0u, 0u, 0u} : xv[i];
-        }
-        __builtin_amdgcn_sched_barrier(0);                  // keep the x loads ahead of the weight loads
-        TileRegs<QT> tr[NW * U];
-        float rw[U];
-#pragma unroll
-        for (int t = 0; t < U; t++) {
-            const int g = gw + t < G ? gw + t : G - 1;
-            rw[t] = 1.0f;
-            if constexpr (MOE == 2) load_tile<QT, true>(moe_tile(g, rw[t]), lane, r, tr[t]);
-            else load_tile<QT, true>(wrow + (int64_t)g * F::TILE_BYTES, lane, r, tr[t]);
-        }
-        if constexpr (DUAL) {
-#pragma unroll
-            for (int t = 0; t < U; t++) {
-                const int g = gw + t;
-                load_tile<QT, true>(wrow2 + (int64_t)(g < G ? g : G - 1) * F::TILE_BYTES, lane, r, tr[U + t]);
+            if constexpr (F32) {
+                const u32x4 *xp = (const u32x4 *)((const float *)x + (int64_t)m * K + col);
+                xv[2 * i] = xp[0];
+                xv[2 * i + 1] = xp[1];
+                if constexpr (ZERO_X) {
+                    xv[2 * i] = past ? u32x4{0u, 0u, 0u, 0u} : xv[2 * i];
+                    xv[2 * i + 1] = past ? u32x4{0u, 0u, 0u, 0u} : xv[2 * i + 1];
+                }
+            } else {
+                xv[i] = *(const u32x4 *)(x + (int64_t)m * K + col);
+                if constexpr (ZERO_X) xv[i] = past ? u32x4{0u, 0u, 0u, 0u} : xv[i];
             }
         }
+        __builtin_amdgcn_sched_barrier(0);                  // keep the x loads ahead of the weight loads
+        typename std::conditional<ROWS, RowRegs<QT>, TileRegs<QT>>::type tr[NW * U];
+        float rw[U];
+        if constexpr (ROWS) {
 #pragma unroll
-        for (int wi = 1; wi < R; wi++)
+            for (int wi = 0; wi < R; wi++)
+#pragma unroll
+                for (int t = 0; t < U; t++) load_rows<QT>(wr[wi], gw + t < G ? gw + t : G - 1, c, blocks, tr[wi * U + t]);
+        } else {
 #pragma unroll
             for (int t = 0; t < U; t++) {
                 const int g = gw + t < G ? gw + t : G - 1;
-                load_tile<QT, true>(wrow + ((int64_t)wi * G + g) * F::TILE_BYTES, lane, r, tr[wi * U + t]);
+                rw[t] = 1.0f;
+                if constexpr (MOE == 2) load_tile<QT, true>(moe_tile(g, rw[t]), lane, r, tr[t]);
+                else load_tile<QT, true>(wrow + (int64_t)g * F::TILE_BYTES, lane, r, tr[t]);
             }
+            if constexpr (DUAL) {
+#pragma unroll
+                for (int t = 0; t < U; t++) {
+                    const int g = gw + t;
+                    load_tile<QT, true>(wrow2 + (int64_t)(g < G ? g : G - 1) * F::TILE_BYTES, lane, r, tr[U + t]);
+                }
+            }
+#pragma unroll
+            for (int wi = 1; wi < R; wi++)
+#pragma unroll
+                for (int t = 0; t < U; t++) {
+                    const int g = gw + t < G ? gw + t : G - 1;
+                    load_tile<QT, true>(wrow + ((int64_t)wi * G + g) * F::TILE_BYTES, lane, r, tr[wi * U + t]);
+                }
+        }
 
         __builtin_amdgcn_sched_barrier(0);
         // The LDS region is private to the wave and LDS operations of a wave execute in order:
@@ -350,7 +405,21 @@ __global__ __launch_bounds__(1024) void gemv_mfma_kernel(const AT *__restrict__ 
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
         __builtin_amdgcn_wave_barrier();
 #pragma unroll
-        for (int i = 0; i < XN; i++) *(u32x4 *)(xs + (i * 64 + lane) * 8) = xv[i];
+        for (int i = 0; i < XN; i++) {
+            const int at = i * 64 + lane;
+            auto put = [&](AT *plane, const u32x4 &v) __attribute__((always_inline)) {
+                if constexpr (ROWS) store_x_rows<QT>((uint8_t *)(plane + at / (SLICE / 8) * SLICE), at % (SLICE / 8), v);
+                else *(u32x4 *)(plane + at * 8) = v;
+            };
+            if constexpr (F32) {
+                u32x4 hi, lo;
+                split_f32(xv[2 * i], xv[2 * i + 1], hi, lo);
+                put(xs, hi);
+                put(xs + XN * 512, lo);
+            } else {
+                put(xs, xv[i]);
+            }
+        }
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
         __builtin_amdgcn_wave_barrier();
 
@@ -358,11 +427,17 @@ __global__ __launch_bounds__(1024) void gemv_mfma_kernel(const AT *__restrict__ 
         for (int wi = 0; wi < NW; wi++)
 #pragma unroll
             for (int t = 0; t < U; t++) {
-                const TileRegs<QT> &tl = tr[wi * U + t];
+                auto &tl = tr[wi * U + t];
+                uint32_t hb[4];
+                if constexpr (ROWS) arrange_rows<QT>(tl, hb);
                 const bool live = ZERO_X || gw + t < G;
-                V8 a[4];
+                V8 a[4], al[4];
 #pragma unroll
                 for (int j = 0; j < 4; j++) a[j] = *(const V8 *)(xa + (t * 4 + j) * 32);
+                if constexpr (F32) {
+#pragma unroll
+                    for (int j = 0; j < 4; j++) al[j] = *(const V8 *)(xa + XN * 512 + (t * 4 + j) * 32);
+                }
 #pragma unroll
                 for (int j = 0; j < 4; j++) {
                     V8 b;
@@ -371,7 +446,8 @@ __global__ __launch_bounds__(1024) void gemv_mfma_kernel(const AT *__restrict__ 
                     else if (j < 2) b = Unpack8<QT, AT>::run(tl.q0[2 * j], tl.q0[2 * j + 1]);
                     else b = Unpack8<QT, AT>::run(tl.q1[2 * (j - 2)], tl.q1[2 * (j - 2) + 1]);
                     float d, mn;
-                    tile_scale<QT>(tl, j, d, mn);
+                    if constexpr (ROWS) hdr_to_scale<QT>(hb[j], d, mn);
+                    else tile_scale<QT>(tl, j, d, mn);
                     if constexpr (MOE == 2) {
                         d *= rw[t];
                         mn *= rw[t];
@@ -381,9 +457,14 @@ __global__ __launch_bounds__(1024) void gemv_mfma_kernel(const AT *__restrict__ 
                         mn = live ? mn : 0.0f;
                     }
                     f32x4 p = mfma16(a[j], b, zero4);
-                    if constexpr (QT == QT_NF4 && F32OUT) p = mfma16(a[j], Unpack<QT, AT>::run(tl.q0[j], lut_lo, magic), p);
+                    if constexpr (F32) p = mfma16(al[j], b, p);
+                    if constexpr (QT == QT_NF4 && F32) {
+                        const V8 bl = Unpack<QT, AT>::run(tl.q0[j], lut_lo, magic);
+                        p = mfma16(al[j], bl, mfma16(a[j], bl, p));
+                    }
                     if constexpr (NEED_S) {
-                        const f32x4 s = mfma16(a[j], ones, zero4);
+                        f32x4 s = mfma16(a[j], ones, zero4);
+                        if constexpr (F32) s = mfma16(al[j], ones, s);
                         const float e = mn - OFFSET * d;
 #pragma unroll
                         for (int i = 0; i < MT; i++)
@@ -401,7 +482,7 @@ __global__ __launch_bounds__(1024) void gemv_mfma_kernel(const AT *__restrict__ 
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     __builtin_amdgcn_wave_barrier();
     float *red = (float *)smem;
-    constexpr int RS = XN * 256;                            // floats per wave region
+    constexpr int RS = XREGION / 2;                         // floats per wave region
 #pragma unroll
     for (int i = 0; i < NW * MT; i++) red[wave * RS + i * 64 + lane] = acc[i];
     __syncthreads();
@@ -418,156 +499,113 @@ __global__ __launch_bounds__(1024) void gemv_mfma_kernel(const AT *__restrict__ 
                 s = gate_act(s, act) * u;
             }
             const int m = grp * MT + i;
-            const int64_t at = (int64_t)m * N + ((int64_t)blockIdx.x * R + wave) * 16 + col;
-            if constexpr (F32OUT) {
-                if (m < M) ((float *)y)[at] = s;
+            const int64_t n = ((int64_t)blockIdx.x * R + wave) * 16 + col;
+            if (m >= M || (ROWS && n >= N)) continue;
+            if constexpr (F32) {
+                ((float *)y)[(int64_t)m * N + n] = bias ? s + ((const float *)bias)[n] : s;
             } else {
-                if (m < M) y[at] = to_at<AT>(s);
+                if constexpr (!DUAL && MOE == 0) s += bias ? (float)bias[n] : 0.0f;
+                y[(int64_t)m * N + n] = to_at<AT>(s);
             }
-        }
-    }
-}
-
-// --------------------------------------------------------- generic GEMV
-
-template <int QT, int LAYOUT, typename AT, int MC, bool F32OUT>
-__global__ __launch_bounds__(256) void gemv_generic_kernel(const AT *__restrict__ x, const uint8_t *__restrict__ w,
-                                                           AT *__restrict__ y, int m0, int M, int N, int K) {
-    const int lane = threadIdx.x & 63;
-    const int64_t n = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (n >= N) return;
-    float acc[MC];
-#pragma unroll
-    for (int i = 0; i < MC; i++) acc[i] = 0.0f;
-    const int sbpr = K / 32;
-    for (int sb = lane; sb < sbpr; sb += 64) {
-        SubBlock s;
-        if constexpr (LAYOUT == LAYOUT_GGML) ggml_load_sub<QT>(w, n, K, sb, s);
-        else tiled_load_sub<QT>(w, n, K, sb, s);
-        float wv[32];
-#pragma unroll
-        for (int i = 0; i < 32; i++) wv[i] = decode<QT>(s.code[i], s.d, s.m);
-#pragma unroll
-        for (int mi = 0; mi < MC; mi++) {
-            if (m0 + mi < M) {
-                const AT *xp = x + (int64_t)(m0 + mi) * K + sb * 32;
-                float a = 0.0f;
-#pragma unroll
-                for (int i = 0; i < 32; i++) a = fmaf((float)xp[i], wv[i], a);
-                acc[mi] += a;
-            }
-        }
-    }
-#pragma unroll
-    for (int mi = 0; mi < MC; mi++) {
-        float v = acc[mi];
-        for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-        if (lane == 0 && m0 + mi < M) {
-            if constexpr (F32OUT) ((float *)y)[(int64_t)(m0 + mi) * N + n] = v;
-            else y[(int64_t)(m0 + mi) * N + n] = to_at<AT>(v);
         }
     }
 }
 
 // -------------------------------------------------------------- launch
 
-template <int QT, typename AT, int MT, int U, int XN, bool DUAL = false, int MOE = 0, int R = 1, bool F32OUT = false>
-static void launch_mfma(const AT *x, const uint8_t *w, AT *y, int M, int N, int K, int waves, hipStream_t st,
-                        const uint8_t *w2 = nullptr, int act = 0, const int32_t *ids = nullptr,
-                        const float *route_w = nullptr, int ge = 0, int slots = 1, int n_exp = 1) {
-    const int G = K / TILE_COLS;
+struct GemvExtra {                                          // what the fused forms take besides
+    const uint8_t *w2 = nullptr;
+    int act = 0;
+    const int32_t *ids = nullptr;
+    const float *route_w = nullptr;
+    int ge = 0, slots = 1, n_exp = 1;
+};
+
+template <int QT, typename AT, int MT, int U, int XN, bool DUAL = false, int MOE = 0, int R = 1, bool F32 = false, bool ROWS = false>
+static void launch_mfma(const AT *x, const uint8_t *w, const AT *bias, AT *y, int M, int N, int K, int waves, hipStream_t st,
+                        const GemvExtra &e = {}) {
+    constexpr int XBYTES = XN * 1024 * (F32 ? 2 : 1);       // of x in LDS per wave
+    const int G = (K + TILE_COLS - 1) / TILE_COLS;
     // waves: enough that one round covers K, within the block size limit and the LDS budget for x
     int wv = (G + U - 1) / U;
-    const int lds_cap = GEMV_LDS_X_BUDGET / (XN * 512 * (int)sizeof(AT));
+    const int lds_cap = GEMV_LDS_X_BUDGET / XBYTES;
     if (wv > lds_cap) wv = lds_cap;
     if (wv > GEMV_MAX_WAVES) wv = GEMV_MAX_WAVES;
     if (waves > 0 && waves < wv) wv = waves;
+    if (wv < R) wv = R;                                     // (wave v writes tile row v)
     if (wv < 1) wv = 1;
-    const size_t lds = (size_t)wv * XN * 512 * sizeof(AT);
-    hipLaunchKernelGGL((gemv_mfma_kernel<QT, AT, MT, U, XN, DUAL, MOE, R, F32OUT>), dim3(N / TILE_ROWS / R, MOE == 1 ? slots : 1),
-                       dim3(64 * wv), lds, st, x, w, w2, y, M, N, K, act, ids, route_w, ge, n_exp);
+    hipLaunchKernelGGL((gemv_mfma_kernel<QT, AT, MT, U, XN, DUAL, MOE, R, F32, ROWS>),
+                       dim3((N + TILE_ROWS * R - 1) / (TILE_ROWS * R), MOE == 1 ? e.slots : 1), dim3(64 * wv), (size_t)wv * XBYTES, st,
+                       x, w, e.w2, y, bias, M, N, K, e.act, e.ids, e.route_w, e.ge, e.n_exp);
 }
 
-// y in fp32 (see F32OUT): a handful of shapes of the kernel is enough, the path is not a hot one
-template <int QT, typename AT>
-static int launch_gemv_f32out(const void *x, const void *w, void *y, int layout, int M, int N, int K, hipStream_t st) {
-    const bool tiled_ok = layout == LAYOUT_TILED && (N % TILE_ROWS) == 0 && (K % TILE_COLS) == 0;
-    if (layout == LAYOUT_TILED && !tiled_ok) return -5;
-    if (tiled_ok) {
-        for (int m0 = 0; m0 < M; m0 += 16) {
-            const int mc = (M - m0) < 16 ? (M - m0) : 16;
-            const AT *xp = (const AT *)x + (int64_t)m0 * K;
-            AT *yp = (AT *)((float *)y + (int64_t)m0 * N);
-            const uint8_t *wp = (const uint8_t *)w;
-            if (mc <= 2) launch_mfma<QT, AT, 1, 2, 1, false, 0, 1, true>(xp, wp, yp, mc, N, K, 0, st);
-            else if (mc <= 4) launch_mfma<QT, AT, 1, 2, 2, false, 0, 1, true>(xp, wp, yp, mc, N, K, 0, st);
-            else if (mc <= 8) launch_mfma<QT, AT, 2, 1, 2, false, 0, 1, true>(xp, wp, yp, mc, N, K, 0, st);
-            else launch_mfma<QT, AT, 4, 2, 8, false, 0, 1, true>(xp, wp, yp, mc, N, K, 0, st);
-        }
-        return 0;
-    }
-    for (int m0 = 0; m0 < M; m0 += 4)
-        hipLaunchKernelGGL((gemv_generic_kernel<QT, LAYOUT_GGML, AT, 4, true>), dim3((N + 3) / 4), dim3(256), 0, st,
-                           (const AT *)x, (const uint8_t *)w, (AT *)y, m0, M, N, K);
-    return 0;
-}
-
-template <int QT, typename AT>
-static int launch_gemv_t(const void *x, const void *w, void *y, int layout, int M, int N, int K, int waves,
-                         hipStream_t st) {
-    const bool tiled_ok = layout == LAYOUT_TILED && (N % TILE_ROWS) == 0 && (K % TILE_COLS) == 0;
-    if (layout == LAYOUT_TILED && !tiled_ok) return -5;
-    if (tiled_ok) {
-        for (int m0 = 0; m0 < M; m0 += 16) {
-            const int mc = (M - m0) < 16 ? (M - m0) : 16;
-            const AT *xp = (const AT *)x + (int64_t)m0 * K;
-            AT *yp = (AT *)y + (int64_t)m0 * N;
-            // Tiles per wave and round (U), measured on MI355X: 4 when K fits one round of 8 waves and
-            // there are many tile rows to spread over the CUs, else 2 with up to 16 waves and as many
-            // rounds as K needs.  XN = 16-byte chunks of x per lane = ceil(M * U / 4).
-            const bool u4 = (K / TILE_COLS) <= 32 && N >= 8192;
-            const uint8_t *wp = (const uint8_t *)w;
-            if (mc <= 4) {
+template <int QT, typename AT, bool F32, bool ROWS>
+static void launch_gemv_t(const void *x, const void *w, const void *bias, void *y, int M, int N, int K, int waves, hipStream_t st) {
+    using ET = typename std::conditional<F32, float, AT>::type;
+    const int tile_rows = (N + TILE_ROWS - 1) / TILE_ROWS;
+    // tile rows may share x in groups of R when R divides them; a row-major weight's last group may reach past its end
+    auto shares = [&](int R) { return ROWS || tile_rows % R == 0; };
+    const uint8_t *wp = (const uint8_t *)w;
+    const AT *b = (const AT *)bias;
+    for (int m0 = 0; m0 < M; m0 += 16) {
+        const int mc = (M - m0) < 16 ? (M - m0) : 16;
+        const AT *xp = (const AT *)((const ET *)x + (int64_t)m0 * K);
+        AT *yp = (AT *)((ET *)y + (int64_t)m0 * N);
+        // Tiles per wave and round (U), measured on MI355X: 4 when K fits one round of 8 waves and
+        // there are many tile rows to spread over the CUs, else 2 with up to 16 waves and as many
+        // rounds as K needs.  XN = chunks of eight columns of x per lane = ceil(M * U / 4).
+        const bool u4 = !F32 && (K + TILE_COLS - 1) / TILE_COLS <= 32 && N >= 8192;
+        if (mc <= 4) {
+            if constexpr (!F32) {
                 if (u4) {
-                    if (mc == 1) launch_mfma<QT, AT, 1, 4, 1>(xp, wp, yp, mc, N, K, waves, st);
-                    else if (mc == 2) launch_mfma<QT, AT, 1, 4, 2>(xp, wp, yp, mc, N, K, waves, st);
-                    else launch_mfma<QT, AT, 1, 4, 4>(xp, wp, yp, mc, N, K, waves, st);
-                } else {
-                    if (mc <= 2) launch_mfma<QT, AT, 1, 2, 1>(xp, wp, yp, mc, N, K, waves, st);
-                    else launch_mfma<QT, AT, 1, 2, 2>(xp, wp, yp, mc, N, K, waves, st);
+                    if (mc == 1) launch_mfma<QT, AT, 1, 4, 1, false, 0, 1, F32, ROWS>(xp, wp, b, yp, mc, N, K, waves, st);
+                    else if (mc == 2) launch_mfma<QT, AT, 1, 4, 2, false, 0, 1, F32, ROWS>(xp, wp, b, yp, mc, N, K, waves, st);
+                    else launch_mfma<QT, AT, 1, 4, 4, false, 0, 1, F32, ROWS>(xp, wp, b, yp, mc, N, K, waves, st);
+                    continue;
                 }
             }
-            // 5 .. 8 rows: one tile per wave and round with up to 16 waves keeps the x slice of a wave (and with
-            // it the workgroup's LDS footprint) small; two tile rows share x where N leaves enough workgroups
-            // (measured on MI355X, sym_int4: 5-7 % on the Llama-2-7B shapes, 15-20 % on [28672 x 8192] and
-            // [8192 x 28672] against four tiles per wave)
-            else if (mc <= 8 && (N / TILE_ROWS) % 2 == 0 && N >= 8192)
-                launch_mfma<QT, AT, 2, 1, 2, false, 0, 2>(xp, wp, yp, mc, N, K, waves, st);
-            else if (mc <= 8) launch_mfma<QT, AT, 2, 1, 2>(xp, wp, yp, mc, N, K, waves, st);
-            // 9 .. 16 rows of x: share x between 4 or 2 tile rows where N still gives enough workgroups
-            // (measured on MI355X: +25 .. 70 % on [28672 x 8192], +8 .. 24 % on [8192 x 8192])
-            else if ((N / TILE_ROWS) % 4 == 0 && N >= 16384)
-                launch_mfma<QT, AT, 4, 1, 4, false, 0, 4>(xp, wp, yp, mc, N, K, waves, st);
-            else if ((N / TILE_ROWS) % 2 == 0 && N >= 8192 && K >= 8192)
-                launch_mfma<QT, AT, 4, 1, 4, false, 0, 2>(xp, wp, yp, mc, N, K, waves, st);
-            else if ((N / TILE_ROWS) % 2 == 0 && N >= 8192)
-                launch_mfma<QT, AT, 4, 2, 8, false, 0, 2>(xp, wp, yp, mc, N, K, waves, st);
-            else launch_mfma<QT, AT, 4, 2, 8>(xp, wp, yp, mc, N, K, waves, st);
+            if (mc <= 2) launch_mfma<QT, AT, 1, 2, 1, false, 0, 1, F32, ROWS>(xp, wp, b, yp, mc, N, K, waves, st);
+            else launch_mfma<QT, AT, 1, 2, 2, false, 0, 1, F32, ROWS>(xp, wp, b, yp, mc, N, K, waves, st);
         }
-        return 0;
+        // 5 .. 8 rows: one tile per wave and round with up to 16 waves keeps the x slice of a wave (and with
+        // it the workgroup's LDS footprint) small; two tile rows share x where N leaves enough workgroups
+        // (measured on MI355X, sym_int4: 5-7 % on the Llama-2-7B shapes, 15-20 % on [28672 x 8192] and
+        // [8192 x 28672] against four tiles per wave)
+        else if (mc <= 8 && shares(2) && N >= 8192)
+            launch_mfma<QT, AT, 2, 1, 2, false, 0, 2, F32, ROWS>(xp, wp, b, yp, mc, N, K, waves, st);
+        else if (mc <= 8) launch_mfma<QT, AT, 2, 1, 2, false, 0, 1, F32, ROWS>(xp, wp, b, yp, mc, N, K, waves, st);
+        // float32: the two planes of x are twice the LDS, so one tile per wave and round here too
+        else if constexpr (F32) launch_mfma<QT, AT, 4, 1, 4, false, 0, 1, F32, ROWS>(xp, wp, b, yp, mc, N, K, waves, st);
+        // 9 .. 16 rows of x: share x between 4 or 2 tile rows where N still gives enough workgroups
+        // (measured on MI355X: +25 .. 70 % on [28672 x 8192], +8 .. 24 % on [8192 x 8192])
+        else if (shares(4) && N >= 16384)
+            launch_mfma<QT, AT, 4, 1, 4, false, 0, 4, F32, ROWS>(xp, wp, b, yp, mc, N, K, waves, st);
+        else if (shares(2) && N >= 8192 && K >= 8192)
+            launch_mfma<QT, AT, 4, 1, 4, false, 0, 2, F32, ROWS>(xp, wp, b, yp, mc, N, K, waves, st);
+        else if (shares(2) && N >= 8192)
+            launch_mfma<QT, AT, 4, 2, 8, false, 0, 2, F32, ROWS>(xp, wp, b, yp, mc, N, K, waves, st);
+        else launch_mfma<QT, AT, 4, 2, 8, false, 0, 1, F32, ROWS>(xp, wp, b, yp, mc, N, K, waves, st);
     }
-    for (int m0 = 0; m0 < M; m0 += 4)
-        hipLaunchKernelGGL((gemv_generic_kernel<QT, LAYOUT_GGML, AT, 4, false>), dim3((N + 3) / 4), dim3(256), 0, st,
-                           (const AT *)x, (const uint8_t *)w, (AT *)y, m0, M, N, K);
+}
+
+template <int QT, bool ROWS>
+static int launch_gemv_dt(const void *x, const void *w, const void *bias, void *y, int dt, int M, int N, int K, int waves,
+                          hipStream_t st) {
+    if (dt == DT_F16) launch_gemv_t<QT, _Float16, false, ROWS>(x, w, bias, y, M, N, K, waves, st);
+    else if (dt == DT_BF16) launch_gemv_t<QT, __bf16, false, ROWS>(x, w, bias, y, M, N, K, waves, st);
+    else if (dt == DT_F32) launch_gemv_t<QT, __bf16, true, ROWS>(x, w, bias, y, M, N, K, waves, st);
+    else return -4;
     return 0;
 }
 
 template <int QT>
-static int launch_gemv_q(const void *x, const void *w, void *y, int layout, int dt, int M, int N, int K, int waves,
+static int launch_gemv_q(const void *x, const void *w, const void *bias, void *y, int layout, int dt, int M, int N, int K, int waves,
                          hipStream_t st) {
-    if (dt == DT_F16) return launch_gemv_t<QT, _Float16>(x, w, y, layout, M, N, K, waves, st);
-    if (dt == DT_BF16) return launch_gemv_t<QT, __bf16>(x, w, y, layout, M, N, K, waves, st);
-    return -4;
+    if (layout == LAYOUT_TILED) {
+        if (N % TILE_ROWS || K % TILE_COLS) return -5;
+        return launch_gemv_dt<QT, false>(x, w, bias, y, dt, M, N, K, waves, st);
+    }
+    return launch_gemv_dt<QT, true>(x, w, bias, y, dt, M, N, K, waves, st);
 }
 
 template <int QT, typename AT>
@@ -577,17 +615,20 @@ static int launch_mlp_t(const void *x, const void *wg, const void *wu, void *y, 
     // keep the kernel below 80 vector registers, so that a CU holds three workgroups and the 688 workgroups
     // of a [11008 x 4096] pair all run side by side.  With four tiles of each weight the kernel takes 120
     // registers and a third of the workgroups has to wait for a free slot.
-    const uint8_t *g = (const uint8_t *)wg, *u = (const uint8_t *)wu;
+    const uint8_t *g = (const uint8_t *)wg;
+    GemvExtra e;
+    e.w2 = (const uint8_t *)wu;
+    e.act = act;
     for (int m0 = 0; m0 < M; m0 += 16) {             // one pass over both weights per 16 rows
         const int mc = (M - m0) < 16 ? (M - m0) : 16;
         const AT *xp = (const AT *)x + (int64_t)m0 * K;
         AT *yp = (AT *)y + (int64_t)m0 * N;
-        if (mc <= 2) launch_mfma<QT, AT, 1, 2, 1, true>(xp, g, yp, mc, N, K, 8, st, u, act);
-        else if (mc <= 4) launch_mfma<QT, AT, 1, 2, 2, true>(xp, g, yp, mc, N, K, 8, st, u, act);
+        if (mc <= 2) launch_mfma<QT, AT, 1, 2, 1, true>(xp, g, nullptr, yp, mc, N, K, 8, st, e);
+        else if (mc <= 4) launch_mfma<QT, AT, 1, 2, 2, true>(xp, g, nullptr, yp, mc, N, K, 8, st, e);
         // 5 .. 16 rows: one tile of each weight per wave and round with up to 16 waves, as the plain product's
         // kernels that share x between two tile rows
-        else if (mc <= 8) launch_mfma<QT, AT, 2, 1, 2, true>(xp, g, yp, mc, N, K, 0, st, u, act);
-        else launch_mfma<QT, AT, 4, 1, 4, true>(xp, g, yp, mc, N, K, 0, st, u, act);
+        else if (mc <= 8) launch_mfma<QT, AT, 2, 1, 2, true>(xp, g, nullptr, yp, mc, N, K, 0, st, e);
+        else launch_mfma<QT, AT, 4, 1, 4, true>(xp, g, nullptr, yp, mc, N, K, 0, st, e);
     }
     return 0;
 }
@@ -619,10 +660,16 @@ static int launch_moe_t(const void *x, const int32_t *ids, const float *route_w,
                         const void *ups, const void *downs, void *h, void *y, int hidden, int inter, int act,
                         hipStream_t st) {
     // h[slots, inter] = act(x Wg[e]^T) * (x Wu[e]^T), then y[hidden] = sum_j route_w[j] * h[j] Wd[e_j]^T
-    launch_mfma<QT, AT, 1, 4, 1, true, 1>((const AT *)x, (const uint8_t *)gates, (AT *)h, 1, inter, hidden, 0, st,
-                                          (const uint8_t *)ups, act, ids, nullptr, 0, slots, n_exp);
-    launch_mfma<QT, AT, 1, 4, 1, false, 2>((const AT *)h, (const uint8_t *)downs, (AT *)y, 1, hidden, slots * inter, 0,
-                                           st, nullptr, 0, ids, route_w, inter / TILE_COLS, slots, n_exp);
+    GemvExtra e;
+    e.w2 = (const uint8_t *)ups;
+    e.act = act;
+    e.ids = ids;
+    e.route_w = route_w;
+    e.ge = inter / TILE_COLS;
+    e.slots = slots;
+    e.n_exp = n_exp;
+    launch_mfma<QT, AT, 1, 4, 1, true, 1>((const AT *)x, (const uint8_t *)gates, nullptr, (AT *)h, 1, inter, hidden, 0, st, e);
+    launch_mfma<QT, AT, 1, 4, 1, false, 2>((const AT *)h, (const uint8_t *)downs, nullptr, (AT *)y, 1, hidden, slots * inter, 0, st, e);
     return 0;
 }
 
@@ -648,29 +695,17 @@ int launch_moe_gemv(const void *x, const int32_t *ids, const float *route_w, int
     }
 }
 
-// x: bf16 [M, K]; y: float [M, N]
-int launch_gemv_bf16_f32out(const void *x, const void *w, void *y, int qtype, int layout, int M, int N, int K,
-                            hipStream_t st) {
+// y[M, N] = x[M, K] * dequant(w)^T (+ bias, which may be null) in passes of 16 rows; x, bias and y of act_dtype, which may
+// be DT_F32 (see F32)
+int launch_gemv(const void *x, const void *w, const void *bias, void *y, int qtype, int layout, int act_dtype, int M, int N,
+                int K, int waves, hipStream_t st) {
     if (M == 0 || N == 0) return 0;
     switch (qtype) {
-    case QT_SYM_INT4: return launch_gemv_f32out<QT_SYM_INT4, __bf16>(x, w, y, layout, M, N, K, st);
-    case QT_ASYM_INT4: return launch_gemv_f32out<QT_ASYM_INT4, __bf16>(x, w, y, layout, M, N, K, st);
-    case QT_SYM_INT8: return launch_gemv_f32out<QT_SYM_INT8, __bf16>(x, w, y, layout, M, N, K, st);
-    case QT_NF4: return launch_gemv_f32out<QT_NF4, __bf16>(x, w, y, layout, M, N, K, st);
-    case QT_FP8_E4M3: return launch_gemv_f32out<QT_FP8_E4M3, __bf16>(x, w, y, layout, M, N, K, st);
-    default: return -2;
-    }
-}
-
-int launch_gemv(const void *x, const void *w, void *y, int qtype, int layout, int act_dtype, int M, int N, int K,
-                int waves, hipStream_t st) {
-    if (M == 0 || N == 0) return 0;
-    switch (qtype) {
-    case QT_SYM_INT4: return launch_gemv_q<QT_SYM_INT4>(x, w, y, layout, act_dtype, M, N, K, waves, st);
-    case QT_ASYM_INT4: return launch_gemv_q<QT_ASYM_INT4>(x, w, y, layout, act_dtype, M, N, K, waves, st);
-    case QT_SYM_INT8: return launch_gemv_q<QT_SYM_INT8>(x, w, y, layout, act_dtype, M, N, K, waves, st);
-    case QT_NF4: return launch_gemv_q<QT_NF4>(x, w, y, layout, act_dtype, M, N, K, waves, st);
-    case QT_FP8_E4M3: return launch_gemv_q<QT_FP8_E4M3>(x, w, y, layout, act_dtype, M, N, K, waves, st);
+    case QT_SYM_INT4: return launch_gemv_q<QT_SYM_INT4>(x, w, bias, y, layout, act_dtype, M, N, K, waves, st);
+    case QT_ASYM_INT4: return launch_gemv_q<QT_ASYM_INT4>(x, w, bias, y, layout, act_dtype, M, N, K, waves, st);
+    case QT_SYM_INT8: return launch_gemv_q<QT_SYM_INT8>(x, w, bias, y, layout, act_dtype, M, N, K, waves, st);
+    case QT_NF4: return launch_gemv_q<QT_NF4>(x, w, bias, y, layout, act_dtype, M, N, K, waves, st);
+    case QT_FP8_E4M3: return launch_gemv_q<QT_FP8_E4M3>(x, w, bias, y, layout, act_dtype, M, N, K, waves, st);
     default: return -2;
     }
 }

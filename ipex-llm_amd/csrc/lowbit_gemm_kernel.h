@@ -53,6 +53,7 @@ struct GroupArgs {
                                   // half tiles of 64 rows each, to one workgroup apiece
     int chunk;                    // grouped: column tiles per cell of the tile order (see grouped_tile)
     const uint8_t *w_up_one;      // fused form without tables (offsets == nullptr): the up weight
+    const void *bias;             // dense forms: [N] in the activation type, or null
 };
 
 // Which row tile of which group, and which column tile, workgroup `b` of a grouped launch works on.
@@ -779,6 +780,20 @@ __global__ __launch_bounds__(64 * WAVES, (DMA && MB == 4) ? 2 : 1) void gemm_mfm
             return;
         }
     }
+    // The bias of this lane's columns, added to the fp32 sums here (of a K split: by its reduction).  (Starting the
+    // accumulators from it instead moved accumulator blocks around in the main loop of some variants.)
+    typedef AT bias4 __attribute__((ext_vector_type(4)));
+    bias4 bv[GROUPED ? 1 : NB32 * 4];
+    if constexpr (!GROUPED) {
+#pragma unroll
+        for (int c = 0; c < NB32 * 4; c++) {
+            bv[c] = bias4{};
+            if (ga.bias != nullptr) {
+                const int n = n0 + c * 8 + kg * 4;
+                bv[c] = *(const bias4 *)((const AT *)ga.bias + (n < N ? n : N - 4));
+            }
+        }
+    }
     if ((((uintptr_t)y) & 15) == 0) {
         typedef AT at4 __attribute__((ext_vector_type(4)));
         __syncthreads();                                     // every wave is done with its operand reads
@@ -802,7 +817,8 @@ __global__ __launch_bounds__(64 * WAVES, (DMA && MB == 4) ? 2 : 1) void gemm_mfm
                         // (one block for both: registers 0..7 hold the gate's 16 rows, 8..15 the up weight's)
                         if constexpr (DUAL1) o[i] = to_at<AT>(gemm_gate_act(acc[mb][0][q * 4 + i], ga.act) * acc[mb][0][8 + q * 4 + i]);
                         else if constexpr (DUAL) o[i] = to_at<AT>(gemm_gate_act(acc[mb][0][q * 4 + i], ga.act) * acc[mb][1][q * 4 + i]);
-                        else o[i] = to_at<AT>(acc[mb][nb][q * 4 + i]);
+                        else if constexpr (GROUPED) o[i] = to_at<AT>(acc[mb][nb][q * 4 + i]);
+                        else o[i] = to_at<AT>(acc[mb][nb][q * 4 + i] + (float)bv[nb * 4 + q][i]);
                     }
                     *(at4 *)(wpos[nb * 4 + q] + mb * 32 * (CH * 16)) = o;
                 }
@@ -865,7 +881,10 @@ __global__ __launch_bounds__(64 * WAVES, (DMA && MB == 4) ? 2 : 1) void gemm_mfm
                         typedef AT at4 __attribute__((ext_vector_type(4)));
                         at4 o;
 #pragma unroll
-                        for (int i = 0; i < 4; i++) o[i] = to_at<AT>(acc[mb][nb][q * 4 + i]);
+                        for (int i = 0; i < 4; i++) {
+                            if constexpr (GROUPED) o[i] = to_at<AT>(acc[mb][nb][q * 4 + i]);
+                            else o[i] = to_at<AT>(acc[mb][nb][q * 4 + i] + (float)bv[nb * 4 + q][i]);
+                        }
                         *(at4 *)(y + (int64_t)m * N + n) = o;
                     }
                 }

@@ -28,10 +28,7 @@ struct Api {
     decltype(&lowbit_blob_bytes) blob_bytes = nullptr;
     decltype(&lowbit_tileable) tileable = nullptr;
     decltype(&lowbit_workspace_bytes_for) workspace_bytes_for = nullptr;
-    decltype(&lowbit_forward) forward = nullptr;
-    decltype(&lowbit_forward_ws) forward_ws = nullptr;
-    decltype(&lowbit_forward_f32_workspace_bytes) forward_f32_workspace_bytes = nullptr;
-    decltype(&lowbit_forward_f32) forward_f32 = nullptr;
+    decltype(&lowbit_linear) linear = nullptr;
     decltype(&lowbit_mlp_forward) mlp_forward = nullptr;
     decltype(&lowbit_dequantize_rows) dequantize_rows = nullptr;
 } api;
@@ -57,8 +54,6 @@ int dtype_code(at::ScalarType t) {
 
 void *current_stream(const Tensor &t) { return (void *)c10::hip::getCurrentHIPStream(t.device().index()).stream(); }
 
-Tensor bytes_like(const Tensor &t, size_t n) { return at::empty({(int64_t)n}, t.options().dtype(at::kByte)); }
-
 // a tensor of this module's calls: strided, on the GPU
 bool on_gpu(const Tensor &t) { return t.device().is_cuda() && t.layout() == at::kStrided; }
 
@@ -75,22 +70,12 @@ Tensor product(const Tensor &x, const Tensor &w, const Tensor &bias, int qtype, 
                at::IntArrayRef shape) {
     c10::DeviceGuard guard(x.device());
     Tensor y = at::empty(shape, x.options());
-    void *st = current_stream(x);
     const int dt = dtype_code(x.scalar_type());
-    // workspaces come from torch's caching allocator: ordered with the stream, no allocation in the steady state
-    if (dt == LOWBIT_DT_F32) {
-        const size_t bytes = api.forward_f32_workspace_bytes(M, N, K);
-        Tensor ws = bytes_like(x, bytes);
-        check(api.forward_f32((const float *)x.const_data_ptr(), w.const_data_ptr(), (float *)y.data_ptr(), qtype, layout, M, N, K,
-                              ws.data_ptr(), bytes, st), "lowbit_forward_f32");
-    } else if (const size_t bytes = M <= 16 ? 0 : api.workspace_bytes_for(qtype, layout, M, N, K, WORKSPACE_CAP)) {
-        Tensor ws = bytes_like(x, bytes);
-        check(api.forward_ws(x.const_data_ptr(), w.const_data_ptr(), y.data_ptr(), qtype, layout, dt, M, N, K, ws.data_ptr(), bytes,
-                             st), "lowbit_forward_ws");
-    } else {
-        check(api.forward(x.const_data_ptr(), w.const_data_ptr(), y.data_ptr(), qtype, layout, dt, M, N, K, st), "lowbit_forward");
-    }
-    if (bias.defined()) y.add_(bias);
+    // the workspace comes from torch's caching allocator: ordered with the stream, no allocation in the steady state
+    const size_t bytes = M <= 16 || dt == LOWBIT_DT_F32 ? 0 : api.workspace_bytes_for(qtype, layout, M, N, K, WORKSPACE_CAP);
+    const Tensor ws = bytes ? at::empty({(int64_t)bytes}, x.options().dtype(at::kByte)) : Tensor();
+    check(api.linear(x.const_data_ptr(), w.const_data_ptr(), bias.defined() ? bias.const_data_ptr() : nullptr, y.data_ptr(), qtype,
+                     layout, dt, M, N, K, bytes ? ws.data_ptr() : nullptr, bytes, current_stream(x)), "lowbit_linear");
     return y;
 }
 
@@ -116,7 +101,7 @@ Tensor linear(const Tensor &x_in, const Tensor &w, const Tensor &bias, int qtype
     if (!on_gpu(x_in) || x_in.dim() < 1 || x_in.numel() == 0 || dtype_code(x_in.scalar_type()) < 0) return {};
     const int64_t K = x_in.size(-1), M = x_in.numel() / K;
     if (!is_blob(w, x_in, qtype, N, K)) return {};
-    if (bias.defined() && (bias.scalar_type() != x_in.scalar_type() || bias.device() != x_in.device() || bias.numel() != N ||
+    if (bias.defined() && (bias.scalar_type() != x_in.scalar_type() || bias.device() != x_in.device() || bias.numel() != N || !bias.is_contiguous() ||
                            (bias.requires_grad() && c10::GradMode::is_enabled()))) return {};
     const Tensor x = x_in.is_contiguous() ? x_in : x_in.contiguous();
     const int layout = device_layout(qtype, N, K);
@@ -219,8 +204,8 @@ PyObject *py_bind(PyObject *, PyObject *const *args, Py_ssize_t n) {
         }                                                                                          \
         api.name = (decltype(api.name))p;                                                          \
     } while (0)
-    BIND(last_error); BIND(blob_bytes); BIND(tileable); BIND(workspace_bytes_for); BIND(forward); BIND(forward_ws);
-    BIND(forward_f32_workspace_bytes); BIND(forward_f32); BIND(mlp_forward); BIND(dequantize_rows);
+    BIND(last_error); BIND(blob_bytes); BIND(tileable); BIND(workspace_bytes_for); BIND(linear);
+    BIND(mlp_forward); BIND(dequantize_rows);
 #undef BIND
     Py_RETURN_NONE;
 }

@@ -267,6 +267,15 @@ def lowbit_forward_f32(x, w, y, qtype, layout, m, n, k, workspace, workspace_byt
            "lowbit_forward_f32")
 
 
+_lib.lowbit_linear.argtypes = [c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int64, c_int64, c_int64,
+                               c_void_p, c_size_t, c_void_p]
+_lib.lowbit_linear.restype = c_int
+
+
+def lowbit_linear(x, w, bias, y, qtype, layout, dtype, m, n, k, workspace, workspace_bytes, stream):
+    _check(_lib.lowbit_linear(x, w, bias, y, qtype, layout, dtype, m, n, k, workspace, workspace_bytes, stream), "lowbit_linear")
+
+
 _lib.lowbit_noalloc_scratch_bytes.argtypes = []
 _lib.lowbit_noalloc_scratch_bytes.restype = c_size_t
 _lib.lowbit_forward_noalloc.argtypes = [c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int64, c_int64, c_int64,

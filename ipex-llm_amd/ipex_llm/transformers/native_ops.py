@@ -12,8 +12,7 @@ import ipex_llm.ggml.model.llama.llama_cpp as ggml
 from ipex_llm.utils.common import invalidInputError
 from ipex_llm.utils.utils import get_shared_lib_info
 
-_BOUND = ("last_error", "blob_bytes", "tileable", "workspace_bytes_for", "forward", "forward_ws",
-          "forward_f32_workspace_bytes", "forward_f32", "mlp_forward", "dequantize_rows")
+_BOUND = ("last_error", "blob_bytes", "tileable", "workspace_bytes_for", "linear", "mlp_forward", "dequantize_rows")
 
 
 def _load():

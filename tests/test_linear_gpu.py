@@ -1,0 +1,59 @@
+"""lowbit_linear: row-major weights of any shape, float32 activations and the bias, against the oracle."""
+import numpy as np
+import pytest
+import torch
+
+import ipex_llm.ggml.model.llama.llama_cpp as ggml
+import lowbit_oracle as orc
+from gpu_util import ALL, DT, FP8, acts, dev_quantize, stream, weights
+
+pytestmark = pytest.mark.gpu
+GGML, TILED = ggml.LAYOUT_GGML, ggml.LAYOUT_TILED
+TOL = {torch.float16: 2e-3, torch.bfloat16: 8e-3, torch.float32: 3e-5}
+
+
+def _check(qtype, dtype, layout, m, n, k, biased, seed):
+    w, x = weights(seed, (n, k)), acts(seed + 1, m, k, dtype)
+    bias = torch.from_numpy(np.random.default_rng(seed + 2).standard_normal(n).astype(np.float32)).to(dtype) if biased else None
+    blob, xd = dev_quantize(w, qtype, layout), x.cuda()
+    bd = bias.cuda() if biased else None
+    need = ggml.lowbit_workspace_bytes_for(qtype, layout, m, n, k, 64 << 20)
+    ws = torch.empty(max(need, 16), dtype=torch.uint8, device="cuda")
+    # guard rows on both sides: the kernel writes the m x n results and nothing else
+    y = torch.full((m + 2, n), float("nan"), dtype=dtype, device="cuda")
+    if (n * y.element_size()) % 16:
+        y = torch.full(((m + 2) * n + 16,), float("nan"), dtype=dtype, device="cuda")[n % 8:][:(m + 2) * n].view(m + 2, n)
+    ggml.lowbit_linear(xd.data_ptr(), blob.data_ptr(), bd.data_ptr() if biased else None, y[1].data_ptr(), qtype, layout, DT[dtype],
+                       m, n, k, ws.data_ptr() if need else None, need, stream())
+    torch.cuda.synchronize()
+    assert torch.isnan(y[0]).all() and torch.isnan(y[m + 1]).all()
+    want = orc.mul_mat_exact(orc.quantize(w, qtype), x.float().numpy(), (n, k), qtype)
+    if biased:
+        want = want + bias.float().numpy()
+    got = y[1:m + 1].float().cpu().numpy()
+    assert np.abs(got - want).max() <= TOL[dtype] * np.abs(want).max()
+
+
+# rows of x around the kernel's passes and tiles, weight rows around 16, columns around 128 (whole blocks)
+@pytest.mark.parametrize("qtype", ALL)
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("m,n,k", [(1, 1, 128), (2, 17, 64), (3, 37, 192), (5, 48, 4160), (8, 8203, 320), (9, 15, 1088),
+                                   (16, 16401, 128), (13, 8203, 8256), (17, 33, 576), (33, 3200, 1344), (70, 250, 2240),
+                                   (130, 129, 448), (257, 515, 704)])
+def test_row_major_weights_of_any_shape(qtype, dtype, m, n, k):
+    if qtype == FP8:
+        k = (k + 127) // 128 * 128
+    _check(qtype, dtype, GGML, m, n, k, m % 2 == 1, 100 * m + n)
+
+
+@pytest.mark.parametrize("qtype", ALL)
+@pytest.mark.parametrize("m,n,k", [(1, 64, 256), (4, 8192, 384), (7, 8192, 128), (8, 48, 4096), (12, 4096, 1408), (16, 272, 128), (35, 64, 512)])
+def test_float32_activations_in_one_pass(qtype, m, n, k):
+    _check(qtype, torch.float32, TILED, m, n, k, m % 2 == 0, 300 * m + n)
+
+
+# one shape for every kernel of the choice: streaming, ring (cut and whole tiles), GEMM, its K split, narrow and tall tiles
+@pytest.mark.parametrize("qtype,dtype", [(2, torch.float16), (3, torch.bfloat16), (8, torch.float16), (10, torch.bfloat16), (15, torch.bfloat16)])
+@pytest.mark.parametrize("m,n,k", [(3, 512, 256), (40, 4096, 1024), (300, 272, 2048), (512, 16384, 128), (1030, 2048, 256), (200, 1040, 128)])
+def test_bias_of_every_kernel(qtype, dtype, m, n, k):
+    _check(qtype, dtype, TILED, m, n, k, True, 500 * m + n)
