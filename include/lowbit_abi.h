@@ -192,6 +192,17 @@ int lowbit_moe_forward(const void *x, const int32_t *topk_ids, const float *topk
                        const void *const *gates, const void *const *ups, const void *const *downs, void *workspace,
                        void *y, int qtype, int act_dtype, int64_t hidden, int64_t inter, int act, void *stream);
 
+/* A whole mixture-of-experts block for any number of tokens:
+ * y[t, :] = sum_j topk_weight[t, j] * down[e](act(gate[e] x_t) .* up[e] x_t), e = topk_ids[t, j] (int64, [tokens, top_k]);
+ * a pair whose id lies outside [0, n_experts) counts nothing.  topk_weight is [tokens, top_k] of weight_dtype, y [tokens, hidden] 16-byte aligned.  Weight tables
+ * as in lowbit_moe_forward, workspace caller-owned device memory of lowbit_experts_workspace_bytes bytes (16-byte
+ * aligned).  The reference's per-expert loop (models/qwen2_moe.py:375-430) without a host read of the routing. */
+size_t lowbit_experts_workspace_bytes(int64_t tokens, int top_k, int n_experts, int64_t hidden, int64_t inter);
+int lowbit_experts_forward(const void *x, const int64_t *topk_ids, const void *topk_weight, int weight_dtype, int64_t tokens,
+                           int top_k, int n_experts, const void *const *gates, const void *const *ups, const void *const *downs,
+                           void *workspace, size_t workspace_bytes, void *y, int qtype, int act_dtype, int64_t hidden,
+                           int64_t inter, int act, void *stream);
+
 /* The same products with a caller-owned workspace in device memory (16-byte aligned): the GEMM may
  * then split K over more workgroups and sum fp32 partial tiles from the workspace in a second launch,
  * which fills the machine when M is small or N narrow.  No counterpart in the reference (its closed

@@ -15,9 +15,13 @@ int launch_mlp_gemv(const void *x, const void *wg, const void *wu, void *y, int 
                     int K, int act, hipStream_t st);
 int launch_mlp_gemm(const void *x, const void *wg, const void *wu, void *y, int qtype, int act_dtype, int M, int N, int K,
                     int act, hipStream_t st);
-int launch_moe_gemv(const void *x, const int32_t *ids, const float *route_w, int slots, int n_exp, const void *gates,
-                    const void *ups, const void *downs, void *h, void *y, int qtype, int act_dtype, int hidden,
-                    int inter, int act, hipStream_t st);
+int launch_moe_gemv(const void *x, const void *ids, bool ids64, const void *route_w, int route_dtype, int tokens, int top_k,
+                    int n_exp, const void *gates, const void *ups, const void *downs, void *h, void *y, int qtype, int act_dtype,
+                    int hidden, int inter, int act, hipStream_t st);
+size_t experts_workspace_bytes(int tokens, int top_k, int n_exp, int hidden, int inter);
+int launch_experts(const void *x, const int64_t *ids, const void *weight, int w_dtype, int tokens, int top_k, int n_exp,
+                   const void *const *gates, const void *const *ups, const void *const *downs, void *workspace, void *out,
+                   int qtype, int act_dtype, int hidden, int inter, int act, hipStream_t st);
 int launch_quantize(const float *src, void *dst, int qtype, int64_t N, int64_t K, int layout, hipStream_t st);
 int launch_relayout(const void *src, void *dst, int qtype, int64_t N, int64_t K, int src_layout, hipStream_t st);
 int launch_dequantize(const void *w, void *out, int qtype, int64_t N, int64_t K, int layout, int out_dtype,
@@ -494,9 +498,43 @@ int lowbit_moe_forward(const void *x, const int32_t *topk_ids, const float *topk
     if (!x || !topk_ids || !topk_weight || !gates || !ups || !downs || !workspace || !y || !aligned16(x) ||
         !aligned16(workspace))
         return fail(LOWBIT_EARG, "lowbit_moe_forward: null or misaligned pointer");
-    return check_launch(launch_moe_gemv(x, topk_ids, topk_weight, top_k, n_experts, gates, ups, downs, workspace, y, qtype,
-                                        act_dtype, (int)hidden, (int)inter, act, (hipStream_t)stream),
+    return check_launch(launch_moe_gemv(x, topk_ids, false, topk_weight, LOWBIT_DT_F32, 1, top_k, n_experts, gates, ups, downs, workspace,
+                                        y, qtype, act_dtype, (int)hidden, (int)inter, act, (hipStream_t)stream),
                         "lowbit_moe_forward");
+}
+
+static bool experts_sizes_ok(int64_t tokens, int64_t top_k, int64_t n_experts, int64_t hidden, int64_t inter) {
+    return tokens > 0 && top_k > 0 && top_k <= 64 && n_experts > 0 && n_experts <= 4096 && hidden > 0 && inter > 0 &&
+           tokens < (1 << 24) / top_k && hidden < (1 << 23) && inter < (1 << 23) && top_k * inter <= 0x7fffffff;
+}
+
+size_t lowbit_experts_workspace_bytes(int64_t tokens, int top_k, int n_experts, int64_t hidden, int64_t inter) {
+    if (!experts_sizes_ok(tokens, top_k, n_experts, hidden, inter)) return 0;
+    return experts_workspace_bytes((int)tokens, top_k, n_experts, (int)hidden, (int)inter);
+}
+
+int lowbit_experts_forward(const void *x, const int64_t *topk_ids, const void *topk_weight, int weight_dtype, int64_t tokens,
+                           int top_k, int n_experts, const void *const *gates, const void *const *ups, const void *const *downs,
+                           void *workspace, size_t workspace_bytes, void *y, int qtype, int act_dtype, int64_t hidden,
+                           int64_t inter, int act, void *stream) {
+    const char *what = "lowbit_experts_forward";
+    if (int rc = check_weight_shape(what, qtype, inter, hidden, LOWBIT_LAYOUT_TILED)) return rc;
+    if (int rc = check_weight_shape(what, qtype, hidden, inter, LOWBIT_LAYOUT_TILED)) return rc;
+    if (act_dtype != LOWBIT_DT_F16 && act_dtype != LOWBIT_DT_BF16) return fail(LOWBIT_EDTYPE, "%s: activations must be f16 or bf16", what);
+    if (weight_dtype != LOWBIT_DT_F16 && weight_dtype != LOWBIT_DT_BF16 && weight_dtype != LOWBIT_DT_F32)
+        return fail(LOWBIT_EDTYPE, "%s: routing weights must be f16, bf16 or f32", what);
+    if (act != LOWBIT_ACT_SILU && act != LOWBIT_ACT_GELU)
+        return fail(LOWBIT_EARG, "%s: activation must be LOWBIT_ACT_SILU or LOWBIT_ACT_GELU", what);
+    if (tokens == 0) return 0;
+    if (!experts_sizes_ok(tokens, top_k, n_experts, hidden, inter))
+        return fail(LOWBIT_ESIZE, "%s: top_k must be 1 .. 64, experts 1 .. 4096, pairs below 2^24", what);
+    if (!x || !topk_ids || !topk_weight || !gates || !ups || !downs || !y || !aligned16(x) || !aligned16(y) || (((uintptr_t)topk_ids) & 7))
+        return fail(LOWBIT_EARG, "%s: null or misaligned pointer", what);
+    const size_t need = lowbit_experts_workspace_bytes(tokens, top_k, n_experts, hidden, inter);
+    if (!workspace || !aligned16(workspace) || workspace_bytes < need)
+        return fail(LOWBIT_ESIZE, "%s: needs %zu bytes of 16-byte aligned workspace", what, need);
+    return check_launch(launch_experts(x, topk_ids, topk_weight, weight_dtype, (int)tokens, top_k, n_experts, gates, ups, downs, workspace,
+                                       y, qtype, act_dtype, (int)hidden, (int)inter, act, (hipStream_t)stream), what);
 }
 
 static int grouped_any(const char *who, const void *x, const void *const *w, const void *const *w_up, void *y,

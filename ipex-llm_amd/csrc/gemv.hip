@@ -217,6 +217,15 @@ __device__ inline float gate_act(float g, int act) {
 }
 constexpr int GEMV_LDS_X_BUDGET = 64 * 1024;
 
+struct MoeId {
+    int clamped;
+    bool valid;
+};
+__device__ inline MoeId moe_id(const void *ids, bool ids64, int pair, int n_exp) {
+    const int64_t e = ids64 ? ((const int64_t *)ids)[pair] : ((const int32_t *)ids)[pair];
+    return {(int)(e < 0 ? 0 : e < n_exp ? e : n_exp - 1), e >= 0 && e < n_exp};
+}
+
 // One workgroup = one tile row (16 output columns).  Per round, wave w owns U consecutive
 // tiles along K: it first issues every weight load of the round (so the whole slice is in
 // flight at once), then copies its slice of x into a wave-private LDS region, then runs
@@ -230,10 +239,12 @@ constexpr int GEMV_LDS_X_BUDGET = 64 * 1024;
 // python/llm/src/ipex_llm/transformers/models/deepseek.py:290-315).  w / w2 are then tables of
 // weight pointers in device memory and ids[j] names the expert of routing slot j, so that the host
 // never has to read the routing result.
-//   MOE == 1 (with DUAL): blockIdx.y = slot j; row j of y = act(x Wg[e]^T) * (x Wu[e]^T).
-//   MOE == 2: x is the [slots, K / slots] output of the first launch, read as one long vector;
-//             tile g of the K walk belongs to slot g / ge and is scaled by route_w[slot]:
-//             y = sum_j route_w[j] * (x_j Wd[e_j]^T).
+//   MOE == 1 (with DUAL): blockIdx.y = pair of token and slot; row blockIdx.y of y = act(x_t Wg[e]^T) * (x_t Wu[e]^T).
+//   MOE == 2: blockIdx.y = token; x is its [slots, K / slots] part of the first launch's output, read as one long
+//             vector; tile g of the K walk belongs to slot g / ge and is scaled by route_w[slot]:
+//             y_t = sum_j route_w[j] * (x_j Wd[e_j]^T).
+//   ids and route_w are read as the caller has them: 32- or 64-bit ids, weights of any float type.  A 64-bit id outside
+//   [0, n_exp) takes its pair out of the sum; a 32-bit one stands for the nearest expert.
 //
 // F32 (lowbit_forward_f32): x, bias and y are float.  The MFMA operands are 16-bit, so AT is bf16 and each value of x
 // becomes two on its way into LDS, hi = bf16(x) and lo = bf16(x - hi): 16 mantissa bits and fp32's exponent range.  Both
@@ -250,8 +261,9 @@ template <int QT, typename AT, int MT, int U, int XN, bool DUAL, int MOE, int R,
 __global__ __launch_bounds__(1024) void gemv_mfma_kernel(const AT *__restrict__ x, const uint8_t *__restrict__ w,
                                                          const uint8_t *__restrict__ w2, AT *__restrict__ y,
                                                          const AT *__restrict__ bias, int M, int N, int K, int act,
-                                                         const int32_t *__restrict__ ids, const float *__restrict__ route_w,
-                                                         int ge, int n_exp) {
+                                                         const void *__restrict__ ids, bool ids64,
+                                                         const void *__restrict__ route_w, int route_dtype, int ge, int n_exp,
+                                                         int slots) {
     using F = Fmt<QT>;
     using V8 = typename Vec8<AT>::type;
     constexpr bool IS4 = (F::BITS == 4);
@@ -305,17 +317,34 @@ __global__ __launch_bounds__(1024) void gemv_mfma_kernel(const AT *__restrict__ 
         if constexpr (DUAL) wrow2 = (gbytes)w2 + (int64_t)blockIdx.x * G * F::TILE_BYTES;
     } else if constexpr (MOE == 1) {
         // ids come from device memory: clamp, so that a bad id cannot send a load astray
-        const int e = min(max(ids[blockIdx.y], 0), n_exp - 1);
+        const int e = moe_id(ids, ids64, blockIdx.y, n_exp).clamped;
         wrow = (gbytes)((const uint8_t *const *)w)[e] + (int64_t)blockIdx.x * G * F::TILE_BYTES;
         wrow2 = (gbytes)((const uint8_t *const *)w2)[e] + (int64_t)blockIdx.x * G * F::TILE_BYTES;
+        x += (int64_t)(blockIdx.y / slots) * K;
+        y += (int64_t)blockIdx.y * N;
+    } else {
+        x += (int64_t)blockIdx.y * K;
         y += (int64_t)blockIdx.y * N;
     }
-    // MOE == 2: tile g -> slot g / ge; its weight row starts at table[ids[slot]] + blockIdx.x * ge tiles
+    // MOE == 2: tile g -> slot g / ge; its weight row starts at table[ids[slot]] + blockIdx.x * ge tiles.  Lane j looks slot
+    // j up once (at most 64 slots), a tile then asks that lane: per tile, the chain id -> pointer -> weight and the
+    // branches on the types of ids and weights cost 3 us of 6 (60 experts of [1408 x 2048], four slots).
+    uint64_t slot_w = 0;
+    float slot_rw = 0.0f;
+    if constexpr (MOE == 2) {
+        const int pair = blockIdx.y * slots + (lane < slots ? lane : 0);
+        const MoeId id = moe_id(ids, ids64, pair, n_exp);
+        slot_w = (uint64_t)((const uint8_t *const *)w)[id.clamped];
+        slot_rw = route_dtype == DT_F32 ? ((const float *)route_w)[pair]
+                  : route_dtype == DT_F16 ? (float)((const _Float16 *)route_w)[pair] : (float)((const __bf16 *)route_w)[pair];
+        if (ids64 && !id.valid) slot_rw = 0.0f;
+    }
     auto moe_tile = [&](int g, float &rw) -> gbytes {
-        const int slot = g / ge;
-        rw = route_w[slot];
-        return (gbytes)((const uint8_t *const *)w)[min(max(ids[slot], 0), n_exp - 1)] +
-               ((int64_t)blockIdx.x * ge + (g - slot * ge)) * F::TILE_BYTES;
+        const int slot = __builtin_amdgcn_readfirstlane(g / ge);
+        rw = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, slot_rw), slot));
+        const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)slot_w, slot);
+        const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(slot_w >> 32), slot);
+        return (gbytes)((uint64_t)lo | ((uint64_t)hi << 32)) + ((int64_t)blockIdx.x * ge + (g - slot * ge)) * F::TILE_BYTES;
     };
     AT *xs = (AT *)smem + (int64_t)wave * XREGION;          // [XN*64/(SLICE/8)][SLICE], private to this wave
     const AT *xa = xs + m_of_r * SLICE + 8 * c;
@@ -516,9 +545,11 @@ __global__ __launch_bounds__(1024) void gemv_mfma_kernel(const AT *__restrict__ 
 struct GemvExtra {                                          // what the fused forms take besides
     const uint8_t *w2 = nullptr;
     int act = 0;
-    const int32_t *ids = nullptr;
-    const float *route_w = nullptr;
-    int ge = 0, slots = 1, n_exp = 1;
+    const void *ids = nullptr;
+    bool ids64 = false;
+    const void *route_w = nullptr;
+    int route_dtype = DT_F32;
+    int ge = 0, slots = 1, n_exp = 1, tokens = 1;
 };
 
 template <int QT, typename AT, int MT, int U, int XN, bool DUAL = false, int MOE = 0, int R = 1, bool F32 = false, bool ROWS = false>
@@ -535,8 +566,9 @@ static void launch_mfma(const AT *x, const uint8_t *w, const AT *bias, AT *y, in
     if (wv < R) wv = R;                                     // (wave v writes tile row v)
     if (wv < 1) wv = 1;
     hipLaunchKernelGGL((gemv_mfma_kernel<QT, AT, MT, U, XN, DUAL, MOE, R, F32, ROWS>),
-                       dim3((N + TILE_ROWS * R - 1) / (TILE_ROWS * R), MOE == 1 ? e.slots : 1), dim3(64 * wv), (size_t)wv * XBYTES, st,
-                       x, w, e.w2, y, bias, M, N, K, e.act, e.ids, e.route_w, e.ge, e.n_exp);
+                       dim3((N + TILE_ROWS * R - 1) / (TILE_ROWS * R), MOE == 1 ? e.tokens * e.slots : MOE == 2 ? e.tokens : 1), dim3(64 * wv), (size_t)wv * XBYTES, st,
+                       x, w, e.w2, y, bias, M, N, K, e.act, e.ids, e.ids64, e.route_w,
+                       e.route_dtype, e.ge, e.n_exp, e.slots);
 }
 
 template <int QT, typename AT, bool F32, bool ROWS>
@@ -655,42 +687,44 @@ int launch_mlp_gemv(const void *x, const void *wg, const void *wu, void *y, int 
     }
 }
 
+// h[pair, inter] = act(x_t Wg[e]^T) * (x_t Wu[e]^T) for every pair of token and slot, then
+// y[t, hidden] = sum_j route_w[t, j] * (h[t, j] Wd[e_j]^T).  e holds what both launches share.
 template <int QT, typename AT>
-static int launch_moe_t(const void *x, const int32_t *ids, const float *route_w, int slots, int n_exp, const void *gates,
-                        const void *ups, const void *downs, void *h, void *y, int hidden, int inter, int act,
+static int launch_moe_t(const void *x, const void *gates, const void *downs, void *h, void *y, int hidden, int inter, const GemvExtra &e,
                         hipStream_t st) {
-    // h[slots, inter] = act(x Wg[e]^T) * (x Wu[e]^T), then y[hidden] = sum_j route_w[j] * h[j] Wd[e_j]^T
-    GemvExtra e;
-    e.w2 = (const uint8_t *)ups;
-    e.act = act;
-    e.ids = ids;
-    e.route_w = route_w;
-    e.ge = inter / TILE_COLS;
-    e.slots = slots;
-    e.n_exp = n_exp;
     launch_mfma<QT, AT, 1, 4, 1, true, 1>((const AT *)x, (const uint8_t *)gates, nullptr, (AT *)h, 1, inter, hidden, 0, st, e);
-    launch_mfma<QT, AT, 1, 4, 1, false, 2>((const AT *)h, (const uint8_t *)downs, nullptr, (AT *)y, 1, hidden, slots * inter, 0, st, e);
+    launch_mfma<QT, AT, 1, 4, 1, false, 2>((const AT *)h, (const uint8_t *)downs, nullptr, (AT *)y, 1, hidden, e.slots * inter, 0, st, e);
     return 0;
 }
 
 template <int QT>
-static int launch_moe_q(const void *x, const int32_t *ids, const float *route_w, int slots, int n_exp, const void *gates,
-                        const void *ups, const void *downs, void *h, void *y, int dt, int hidden, int inter, int act,
-                        hipStream_t st) {
-    if (dt == DT_F16) return launch_moe_t<QT, _Float16>(x, ids, route_w, slots, n_exp, gates, ups, downs, h, y, hidden, inter, act, st);
-    if (dt == DT_BF16) return launch_moe_t<QT, __bf16>(x, ids, route_w, slots, n_exp, gates, ups, downs, h, y, hidden, inter, act, st);
+static int launch_moe_q(const void *x, const void *gates, const void *downs, void *h, void *y, int dt, int hidden, int inter,
+                        const GemvExtra &e, hipStream_t st) {
+    if (dt == DT_F16) return launch_moe_t<QT, _Float16>(x, gates, downs, h, y, hidden, inter, e, st);
+    if (dt == DT_BF16) return launch_moe_t<QT, __bf16>(x, gates, downs, h, y, hidden, inter, e, st);
     return -4;
 }
 
-int launch_moe_gemv(const void *x, const int32_t *ids, const float *route_w, int slots, int n_exp, const void *gates,
-                    const void *ups, const void *downs, void *h, void *y, int qtype, int act_dtype, int hidden,
-                    int inter, int act, hipStream_t st) {
+int launch_moe_gemv(const void *x, const void *ids, bool ids64, const void *route_w, int route_dtype, int tokens, int top_k,
+                    int n_exp, const void *gates, const void *ups, const void *downs, void *h, void *y, int qtype, int act_dtype,
+                    int hidden, int inter, int act, hipStream_t st) {
+    GemvExtra e;
+    e.w2 = (const uint8_t *)ups;
+    e.act = act;
+    e.ids = ids;
+    e.ids64 = ids64;
+    e.route_w = route_w;
+    e.route_dtype = route_dtype;
+    e.ge = inter / TILE_COLS;
+    e.slots = top_k;
+    e.n_exp = n_exp;
+    e.tokens = tokens;
     switch (qtype) {
-    case QT_SYM_INT4: return launch_moe_q<QT_SYM_INT4>(x, ids, route_w, slots, n_exp, gates, ups, downs, h, y, act_dtype, hidden, inter, act, st);
-    case QT_ASYM_INT4: return launch_moe_q<QT_ASYM_INT4>(x, ids, route_w, slots, n_exp, gates, ups, downs, h, y, act_dtype, hidden, inter, act, st);
-    case QT_SYM_INT8: return launch_moe_q<QT_SYM_INT8>(x, ids, route_w, slots, n_exp, gates, ups, downs, h, y, act_dtype, hidden, inter, act, st);
-    case QT_NF4: return launch_moe_q<QT_NF4>(x, ids, route_w, slots, n_exp, gates, ups, downs, h, y, act_dtype, hidden, inter, act, st);
-    case QT_FP8_E4M3: return launch_moe_q<QT_FP8_E4M3>(x, ids, route_w, slots, n_exp, gates, ups, downs, h, y, act_dtype, hidden, inter, act, st);
+    case QT_SYM_INT4: return launch_moe_q<QT_SYM_INT4>(x, gates, downs, h, y, act_dtype, hidden, inter, e, st);
+    case QT_ASYM_INT4: return launch_moe_q<QT_ASYM_INT4>(x, gates, downs, h, y, act_dtype, hidden, inter, e, st);
+    case QT_SYM_INT8: return launch_moe_q<QT_SYM_INT8>(x, gates, downs, h, y, act_dtype, hidden, inter, e, st);
+    case QT_NF4: return launch_moe_q<QT_NF4>(x, gates, downs, h, y, act_dtype, hidden, inter, e, st);
+    case QT_FP8_E4M3: return launch_moe_q<QT_FP8_E4M3>(x, gates, downs, h, y, act_dtype, hidden, inter, e, st);
     default: return -2;
     }
 }

@@ -31,6 +31,8 @@ struct Api {
     decltype(&lowbit_linear) linear = nullptr;
     decltype(&lowbit_mlp_forward) mlp_forward = nullptr;
     decltype(&lowbit_dequantize_rows) dequantize_rows = nullptr;
+    decltype(&lowbit_experts_workspace_bytes) experts_workspace_bytes = nullptr;
+    decltype(&lowbit_experts_forward) experts_forward = nullptr;
 } api;
 
 constexpr size_t WORKSPACE_CAP = (size_t)256 << 20;      // most that a product borrows for split-K partial sums
@@ -144,6 +146,28 @@ Tensor embedding(const Tensor &ids_in, const Tensor &w, int qtype, int64_t N, in
     return y;
 }
 
+// the experts of a mixture-of-experts block on x [tokens, hidden]; tables: one weight pointer per expert, on x's device
+Tensor experts(const Tensor &x_in, const Tensor &ids_in, const Tensor &weight_in, const Tensor &gates, const Tensor &ups,
+               const Tensor &downs, int qtype, int64_t hidden, int64_t inter, int act) {
+    if (!on_gpu(x_in) || x_in.dim() != 2 || x_in.size(1) != hidden || ids_in.dim() != 2 || ids_in.size(0) != x_in.size(0) ||
+        ids_in.numel() == 0 || ids_in.scalar_type() != at::kLong || weight_in.sizes() != ids_in.sizes() ||
+        ids_in.device() != x_in.device() || weight_in.device() != x_in.device() || gates.device() != x_in.device()) return {};
+    const int dt = dtype_code(x_in.scalar_type()), wdt = dtype_code(weight_in.scalar_type());
+    if ((dt != LOWBIT_DT_F16 && dt != LOWBIT_DT_BF16) || wdt < 0) return {};
+    const int64_t tokens = ids_in.size(0), top_k = ids_in.size(1), n_exp = gates.numel();
+    const size_t bytes = top_k > 64 || n_exp > 4096 ? 0 : api.experts_workspace_bytes(tokens, (int)top_k, (int)n_exp, hidden, inter);
+    if (!bytes) return {};                               // more than the library takes
+    const Tensor x = x_in.contiguous(), ids = ids_in.contiguous(), weight = weight_in.contiguous();
+    c10::DeviceGuard guard(x.device());
+    const Tensor ws = at::empty({(int64_t)bytes}, x.options().dtype(at::kByte));
+    Tensor y = at::empty({tokens, hidden}, x.options());
+    check(api.experts_forward(x.const_data_ptr(), ids.const_data_ptr<int64_t>(), weight.const_data_ptr(), wdt, tokens, (int)top_k,
+                              (int)n_exp, (const void *const *)gates.const_data_ptr(), (const void *const *)ups.const_data_ptr(),
+                              (const void *const *)downs.const_data_ptr(), ws.data_ptr(), bytes, y.data_ptr(), qtype, dt, hidden, inter,
+                              act, current_stream(x)), "lowbit_experts_forward");
+    return y;
+}
+
 // ------------------------------------------------------------------ CPython side
 
 // Arguments by position.  A tensor argument is a torch.Tensor or a Parameter (subclass): anything else, and a value
@@ -205,7 +229,7 @@ PyObject *py_bind(PyObject *, PyObject *const *args, Py_ssize_t n) {
         api.name = (decltype(api.name))p;                                                          \
     } while (0)
     BIND(last_error); BIND(blob_bytes); BIND(tileable); BIND(workspace_bytes_for); BIND(linear);
-    BIND(mlp_forward); BIND(dequantize_rows);
+    BIND(mlp_forward); BIND(dequantize_rows); BIND(experts_workspace_bytes); BIND(experts_forward);
 #undef BIND
     Py_RETURN_NONE;
 }
@@ -261,8 +285,40 @@ PyObject *py_embedding(PyObject *, PyObject *const *args, Py_ssize_t n) {
     });
 }
 
+// experts(x, ids, weights, gates, ups, downs, qtype, hidden, inter, act) -> y or None
+PyObject *py_experts(PyObject *, PyObject *const *args, Py_ssize_t n) {
+    return answer("experts", n, 10, [&] {
+        const Args a{args, n};
+        const Tensor &x = a.tensor(0), &ids = a.tensor(1), &weight = a.tensor(2), &g = a.tensor(3), &u = a.tensor(4), &d = a.tensor(5);
+        const int qtype = (int)a.integer(6), act = (int)a.integer(9);
+        const int64_t hidden = a.integer(7), inter = a.integer(8);
+        NoGil free;
+        return experts(x, ids, weight, g, u, d, qtype, hidden, inter, act);
+    });
+}
+
+// holds(parameter dicts, addresses): whether every dict's "weight" is a tensor whose data lies at the address (bytes of
+// unsigned 64-bit numbers).  What ExpertWeights.check asks of each expert, 180 times for 60 experts: 0.3 us each in Python.
+PyObject *py_holds(PyObject *, PyObject *const *args, Py_ssize_t n) {
+    static PyObject *const weight = PyUnicode_InternFromString("weight");
+    if (n != 2 || !PyTuple_Check(args[0]) || !PyBytes_Check(args[1]) ||
+        PyBytes_GET_SIZE(args[1]) != PyTuple_GET_SIZE(args[0]) * (Py_ssize_t)sizeof(uint64_t)) {
+        PyErr_SetString(PyExc_TypeError, "holds takes a tuple of dicts and as many addresses");
+        return nullptr;
+    }
+    const uint64_t *want = (const uint64_t *)PyBytes_AS_STRING(args[1]);
+    for (Py_ssize_t i = 0; i < PyTuple_GET_SIZE(args[0]); i++) {
+        PyObject *d = PyTuple_GET_ITEM(args[0], i);
+        PyObject *w = PyDict_Check(d) ? PyDict_GetItem(d, weight) : nullptr;
+        if (!w || !THPVariable_Check(w)) Py_RETURN_FALSE;
+        const Tensor &t = THPVariable_Unpack(w);
+        if (!t.has_storage() || (uint64_t)(uintptr_t)t.const_data_ptr() != want[i]) Py_RETURN_FALSE;
+    }
+    Py_RETURN_TRUE;
+}
+
 #define METHOD(name) {#name, (PyCFunction)(void (*)(void))py_##name, METH_FASTCALL, nullptr}
-PyMethodDef methods[] = {METHOD(bind), METHOD(product), METHOD(linear), METHOD(gated), METHOD(embedding),
+PyMethodDef methods[] = {METHOD(bind), METHOD(product), METHOD(linear), METHOD(gated), METHOD(embedding), METHOD(experts), METHOD(holds),
                          {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "lowbit_torch", "native host path of the low-bit layers", -1, methods};
 

@@ -358,6 +358,13 @@ def lowbit_moe_forward(x, topk_ids, topk_weight, top_k, n_experts, gates, ups, d
                                    act_dtype, hidden, inter, act, stream), "lowbit_moe_forward")
 
 
+_lib.lowbit_experts_workspace_bytes.argtypes = [c_int64, c_int, c_int, c_int64, c_int64]
+_lib.lowbit_experts_workspace_bytes.restype = c_size_t
+_lib.lowbit_experts_forward.argtypes = [c_void_p, c_void_p, c_void_p, c_int, c_int64, c_int, c_int, c_void_p, c_void_p, c_void_p,
+                                        c_void_p, c_size_t, c_void_p, c_int, c_int, c_int64, c_int64, c_int, c_void_p]
+_lib.lowbit_experts_forward.restype = c_int
+
+
 def lowbit_dequantize_rows(w, rows, n_rows, dst, qtype, n, k, layout, out_dtype, stream):
     _check(_lib.lowbit_dequantize_rows(w, rows, n_rows, dst, qtype, n, k, layout, out_dtype, stream),
            "lowbit_dequantize_rows")

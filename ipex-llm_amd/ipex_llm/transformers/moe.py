@@ -7,7 +7,7 @@ transformers/models/qwen2_moe.py:375-430).  `moe_ffn_reference` is that loop;
 `moe_ffn_grouped` computes the same thing with two grouped launches over the rows sorted by expert:
 the fused gate/up projection with the activation in its epilogue, then the down projection.
 """
-import ctypes
+import array
 
 import torch
 import torch.nn as nn
@@ -15,6 +15,7 @@ import torch.nn.functional as F
 
 import ipex_llm.ggml.model.llama.llama_cpp as ggml
 from ipex_llm.transformers.low_bit_linear import _DT, _as_u8, _stream
+from ipex_llm.transformers.native_ops import ops
 from ipex_llm.utils.common import invalidInputError
 
 
@@ -47,13 +48,18 @@ class ExpertWeights:
                               "every expert must hold a tiled blob of the common shape on one GPU")
         self.linears = list(linears)
         self.blobs = [_as_u8(lin.weight.data) for lin in linears]        # keeps the storage alive
-        self.ptrs = torch.tensor([b.data_ptr() for b in self.blobs], dtype=torch.int64, device=l0.weight.device)
+        addresses = array.array("Q", [b.data_ptr() for b in self.blobs])
+        self.ptrs = torch.tensor(addresses.tolist(), dtype=torch.int64, device=l0.weight.device)
+        self.held = (tuple(lin._parameters for lin in linears), addresses.tobytes())      # what `holds` compares
+
+    def holds(self, device):
+        """Whether every layer still has the weight that the pointer table, a snapshot, points to."""
+        return self.ptrs.device == device and ops.holds(*self.held)
 
     def check(self, device):
-        """The pointer table is a snapshot: refuse to launch if a layer was moved or re-quantized since."""
-        for lin, blob in zip(self.linears, self.blobs):
-            invalidInputError(lin.weight.data.data_ptr() == blob.data_ptr() and blob.device == device,
-                              "an expert weight was moved or replaced after ExpertWeights was built; build it again")
+        """Refuses to launch if a layer was moved or re-quantized since the table was built."""
+        invalidInputError(self.holds(device),
+                          "an expert weight was moved or replaced after ExpertWeights was built; build it again")
 
 
 def _check_grouped(x_sorted, group_offsets, experts):
@@ -143,20 +149,12 @@ def moe_ffn_reference(hidden, router_logits, w1, w3, w2, top_k=2):
 
 
 def moe_ffn_grouped(hidden, router_logits, g1: ExpertWeights, g3: ExpertWeights, g2: ExpertWeights, top_k=2):
-    """Same result with two grouped launches over the (token, expert) pairs sorted by expert."""
-    n_exp = len(g1.blobs)
+    """Same result in one call of the experts block (csrc/moe.hip)."""
     weights, experts = route_top_k(router_logits, top_k)
-    flat_e = experts.reshape(-1)
-    order = torch.argsort(flat_e, stable=True)
-    tok = torch.div(order, top_k, rounding_mode="floor")
-    counts = torch.bincount(flat_e, minlength=n_exp)
-    offsets = torch.zeros(n_exp + 1, dtype=torch.int32, device=hidden.device)
-    offsets[1:] = torch.cumsum(counts, 0).to(torch.int32)
-    xs = hidden[tok]
-    h = grouped_mlp_forward(xs, offsets, g1, g3)
-    y = grouped_forward(h, offsets, g2) * weights.reshape(-1)[order].unsqueeze(-1).to(hidden.dtype)
-    out = torch.zeros_like(hidden)
-    out.index_add_(0, tok, y)
+    for table in (g1, g3, g2):
+        table.check(hidden.device)
+    out = ops.experts(hidden, experts, weights, g1.ptrs, g3.ptrs, g2.ptrs, g1.qtype, g1.in_len, g1.out_len, 0)
+    invalidInputError(out is not None, "hidden must be [tokens, K] in fp16 / bf16 on the GPU of the experts")
     return out
 
 
@@ -181,8 +179,8 @@ class LowBitExperts(nn.Module):
     `experts(hidden_states [T, H], top_k_index [T, k], top_k_weights [T, k]) -> [T, H]` (MixtralExperts and its
     siblings).  This module takes that one's place: each expert's three weights become LowBitLinear layers
     (`gate[e]`, `up[e]`, `down[e]`, so that save_low_bit / load_low_bit carry them like any other), and on the GPU the
-    call runs as two grouped launches over the (token, expert) pairs sorted by expert, or, for one token, as the two
-    launches of `moe_forward_vec`.  Anywhere else it is the per-expert loop over the LowBitLinear layers."""
+    call is one native call (csrc/moe.hip): two grouped launches over the (token, expert) pairs sorted by expert, or, for
+    few pairs, the streaming kernel.  Anywhere else it is the per-expert loop over the LowBitLinear layers."""
 
     def __init__(self, num_experts, hidden_dim, intermediate_dim, qtype, act_fn, enable_scale_search=False):
         super().__init__()
@@ -221,47 +219,34 @@ class LowBitExperts(nn.Module):
         new.requires_grad_(False)
         return new
 
-    def _expert_tables(self, device):
-        """Pointer tables of the three projections; built on first use and again when a weight has moved."""
+    def _expert_tables(self, x):
+        """Pointer tables of the three projections, built on first use and again when a weight has moved; None where the
+        call is not one for the grouped kernels."""
+        if not x.is_cuda or x.dtype not in (torch.float16, torch.bfloat16) or self.training \
+                or activation_code(self.act_fn) is None:
+            return None
         tables = self.__dict__["_tables"]
-        if tables is not None:
-            try:
-                for t in tables:
-                    t.check(device)
-                return tables
-            except RuntimeError:
-                pass
-        tables = tuple(ExpertWeights(list(layers)) for layers in (self.gate, self.up, self.down))
-        self.__dict__["_tables"] = tables
+        if tables is None or not all(t.holds(x.device) for t in tables):
+            self.__dict__["_tables"] = None
+            w = self.gate[0].weight
+            if not (w.quantized and w.data.device == x.device
+                    and ggml.lowbit_tileable(self.qtype, self.intermediate_dim, self.hidden_dim)
+                    and ggml.lowbit_tileable(self.qtype, self.hidden_dim, self.intermediate_dim)):
+                return None
+            tables = tuple(ExpertWeights(list(layers)) for layers in (self.gate, self.up, self.down))
+            self.__dict__["_tables"] = tables
         return tables
 
-    def _grouped_ok(self, x):
-        w = self.gate[0].weight
-        return (x.device.type == "cuda" and x.dtype in (torch.float16, torch.bfloat16) and not self.training
-                and activation_code(self.act_fn) is not None and w.quantized and w.data.device == x.device
-                and ggml.lowbit_tileable(self.qtype, self.intermediate_dim, self.hidden_dim)
-                and ggml.lowbit_tileable(self.qtype, self.hidden_dim, self.intermediate_dim))
-
     def forward(self, hidden_states, top_k_index, top_k_weights):
-        tokens, top_k = top_k_index.shape
-        if tokens == 0:
+        if top_k_index.shape[0] == 0:
             return torch.zeros_like(hidden_states)
-        if not self._grouped_ok(hidden_states):
+        tables = self._expert_tables(hidden_states)
+        if tables is None:
             return self._loop(hidden_states, top_k_index, top_k_weights)
-        act = activation_code(self.act_fn)
-        g1, g3, g2 = self._expert_tables(hidden_states.device)
-        if tokens == 1:
-            return moe_forward_vec(hidden_states, top_k_index, top_k_weights, g1, g3, g2, act)
-        flat_e = top_k_index.reshape(-1)
-        order = torch.argsort(flat_e, stable=True)
-        tok = torch.div(order, top_k, rounding_mode="floor")
-        offsets = torch.zeros(self.num_experts + 1, dtype=torch.int32, device=hidden_states.device)
-        offsets[1:] = torch.cumsum(torch.bincount(flat_e, minlength=self.num_experts)[:self.num_experts], 0).to(torch.int32)
-        h = grouped_mlp_forward(hidden_states[tok], offsets, g1, g3, act)
-        y = grouped_forward(h, offsets, g2) * top_k_weights.reshape(-1)[order].unsqueeze(-1).to(hidden_states.dtype)
-        out = torch.zeros_like(hidden_states)
-        out.index_add_(0, tok, y)
-        return out
+        g1, g3, g2 = tables
+        y = ops.experts(hidden_states, top_k_index, top_k_weights, g1.ptrs, g3.ptrs, g2.ptrs, self.qtype, self.hidden_dim,
+                        self.intermediate_dim, activation_code(self.act_fn))
+        return self._loop(hidden_states, top_k_index, top_k_weights) if y is None else y
 
     def _loop(self, hidden_states, top_k_index, top_k_weights):
         out = torch.zeros_like(hidden_states)
