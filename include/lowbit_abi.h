@@ -126,6 +126,8 @@ int lowbit_tileable(int qtype, int64_t N, int64_t K);
 
 /* ggml_quantize_tensor on device memory: src fp32 [N, K] -> dst blob in `layout`. */
 int lowbit_quantize(const float *src, void *dst, int qtype, int64_t N, int64_t K, int layout, void *stream);
+/* The same from a source of any element type (LOWBIT_DT_*): 16-bit values are widened to fp32 first, exactly. */
+int lowbit_quantize_from(const void *src, int src_dtype, void *dst, int qtype, int64_t N, int64_t K, int layout, void *stream);
 /* ggml_q_format_convet_cpu2xpu / _xpu2cpu with the shape: src in `src_layout` -> dst in the
  * other layout.  src and dst must not overlap. */
 int lowbit_relayout(const void *src, void *dst, int qtype, int64_t N, int64_t K, int src_layout, void *stream);

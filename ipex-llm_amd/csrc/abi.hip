@@ -22,7 +22,7 @@ size_t experts_workspace_bytes(int tokens, int top_k, int n_exp, int hidden, int
 int launch_experts(const void *x, const int64_t *ids, const void *weight, int w_dtype, int tokens, int top_k, int n_exp,
                    const void *const *gates, const void *const *ups, const void *const *downs, void *workspace, void *out,
                    int qtype, int act_dtype, int hidden, int inter, int act, hipStream_t st);
-int launch_quantize(const float *src, void *dst, int qtype, int64_t N, int64_t K, int layout, hipStream_t st);
+int launch_quantize(const void *src, int src_dtype, void *dst, int qtype, int64_t N, int64_t K, int layout, hipStream_t st);
 int launch_relayout(const void *src, void *dst, int qtype, int64_t N, int64_t K, int src_layout, hipStream_t st);
 int launch_dequantize(const void *w, void *out, int qtype, int64_t N, int64_t K, int layout, int out_dtype,
                       hipStream_t st);
@@ -121,12 +121,16 @@ int lowbit_tileable(int qtype, int64_t N, int64_t K) {
     return qk_size(qtype) != 0 && N > 0 && K > 0 && (N % TILE_ROWS) == 0 && (K % TILE_COLS) == 0;
 }
 
-int lowbit_quantize(const float *src, void *dst, int qtype, int64_t N, int64_t K, int layout, void *stream) {
+int lowbit_quantize_from(const void *src, int src_dtype, void *dst, int qtype, int64_t N, int64_t K, int layout, void *stream) {
     if (int rc = check_weight_shape("lowbit_quantize", qtype, N, K, layout)) return rc;
     if (N * K == 0) return 0;
     if (!src || !dst || !aligned16(src) || !aligned16(dst))
         return fail(LOWBIT_EARG, "lowbit_quantize: pointers must be non-null and 16-byte aligned");
-    return check_launch(launch_quantize(src, dst, qtype, N, K, layout, (hipStream_t)stream), "lowbit_quantize");
+    return check_launch(launch_quantize(src, src_dtype, dst, qtype, N, K, layout, (hipStream_t)stream), "lowbit_quantize");
+}
+
+int lowbit_quantize(const float *src, void *dst, int qtype, int64_t N, int64_t K, int layout, void *stream) {
+    return lowbit_quantize_from(src, LOWBIT_DT_F32, dst, qtype, N, K, layout, stream);
 }
 
 int lowbit_relayout(const void *src, void *dst, int qtype, int64_t N, int64_t K, int src_layout, void *stream) {

@@ -9,7 +9,8 @@
 //
 // Work split: QK/4 adjacent lanes own one block, each lane one float4 of it,
 // so a wave reads 1 KiB of contiguous fp32 per load.  HBM-bound: 4 B read and
-// TS/QK B written per weight.
+// TS/QK B written per weight.  A 16-bit source (the dtype checkpoints come in) is
+// widened in registers, exactly: half the bytes, and no fp32 copy of it made first.
 #include "lowbit_formats.h"
 
 namespace lowbit {
@@ -25,14 +26,14 @@ template <int W> __device__ inline float group_min(float v) {
     return v;
 }
 
-// Signed value of the FIRST element with the largest magnitude in the block.
-// four floats of the source, which is read once: a nontemporal load
-__device__ inline float4 stream4(const float *p) {
-    typedef float f4 __attribute__((ext_vector_type(4)));
-    const f4 v = __builtin_nontemporal_load((const f4 *)p);
-    return make_float4(v[0], v[1], v[2], v[3]);
+// four values of the source, which is read once: a nontemporal load
+template <typename ST> __device__ inline float4 stream4(const ST *p) {
+    typedef ST s4 __attribute__((ext_vector_type(4)));
+    const s4 v = __builtin_nontemporal_load((const s4 *)p);
+    return make_float4((float)v[0], (float)v[1], (float)v[2], (float)v[3]);
 }
 
+// Signed value of the FIRST element with the largest magnitude in the block.
 template <int W> __device__ inline float group_first_absmax_signed(const float4 &v, int lane_in_block) {
     float amax = 0.0f, mx = 0.0f;
     const float e[4] = {v.x, v.y, v.z, v.w};
@@ -124,8 +125,8 @@ __device__ inline void block_codes(const float4 &v, int lib, uint32_t &hdr, uint
 }
 
 // ggml layout: one thread group per block, written where the block lives.
-template <int QT>
-__global__ __launch_bounds__(256) void quantize_kernel(const float *__restrict__ src, uint8_t *__restrict__ dst,
+template <int QT, typename ST>
+__global__ __launch_bounds__(256) void quantize_kernel(const ST *__restrict__ src, uint8_t *__restrict__ dst,
                                                        int64_t n_blocks) {
     using F = Fmt<QT>;
     constexpr int LPB = F::QK / 4;                       // lanes per block
@@ -168,8 +169,8 @@ __global__ __launch_bounds__(256) void quantize_kernel(const float *__restrict__
 // the 16 rows of a tile would arrive from different workgroups at different times.)
 constexpr int QTW = 4;
 
-template <int QT>
-__global__ __launch_bounds__(256) void quantize_tiled_kernel(const float *__restrict__ src, uint8_t *__restrict__ dst,
+template <int QT, typename ST>
+__global__ __launch_bounds__(256) void quantize_tiled_kernel(const ST *__restrict__ src, uint8_t *__restrict__ dst,
                                                              int64_t K) {
     using F = Fmt<QT>;
     constexpr int LPB = F::QK / 4;
@@ -230,7 +231,7 @@ __global__ __launch_bounds__(256) void quantize_tiled_kernel(const float *__rest
     for (int o = threadIdx.x * 16; o < bytes; o += 256 * 16) *(uint4 *)(out + o) = *(const uint4 *)(img + o);
 }
 
-template <int QT> static int launch_q(const float *src, void *dst, int64_t N, int64_t K, int layout, hipStream_t st) {
+template <int QT, typename ST> static int launch_q(const ST *src, void *dst, int64_t N, int64_t K, int layout, hipStream_t st) {
     using F = Fmt<QT>;
     const int64_t n_blocks = N * K / F::QK;
     const int64_t threads = n_blocks * (F::QK / 4);
@@ -238,23 +239,33 @@ template <int QT> static int launch_q(const float *src, void *dst, int64_t N, in
     const int64_t grid = (threads + 255) / 256;
     if (grid > 0x7fffffff) return -3;
     if (layout == LAYOUT_GGML)
-        hipLaunchKernelGGL((quantize_kernel<QT>), dim3((unsigned)grid), dim3(256), 0, st, src, (uint8_t *)dst, n_blocks);
+        hipLaunchKernelGGL((quantize_kernel<QT, ST>), dim3((unsigned)grid), dim3(256), 0, st, src, (uint8_t *)dst, n_blocks);
     else {
         const int64_t strips = (K / TILE_COLS + QTW - 1) / QTW, tile_rows = N / TILE_ROWS;
         if (tile_rows > 65535) return -3;
-        hipLaunchKernelGGL((quantize_tiled_kernel<QT>), dim3((unsigned)strips, (unsigned)tile_rows), dim3(256), 0, st, src,
+        hipLaunchKernelGGL((quantize_tiled_kernel<QT, ST>), dim3((unsigned)strips, (unsigned)tile_rows), dim3(256), 0, st, src,
                            (uint8_t *)dst, K);
     }
     return 0;
 }
 
-int launch_quantize(const float *src, void *dst, int qtype, int64_t N, int64_t K, int layout, hipStream_t st) {
+template <int QT>
+static int launch_q_dt(const void *src, int src_dtype, void *dst, int64_t N, int64_t K, int layout, hipStream_t st) {
+    switch (src_dtype) {
+    case DT_F32: return launch_q<QT>((const float *)src, dst, N, K, layout, st);
+    case DT_F16: return launch_q<QT>((const _Float16 *)src, dst, N, K, layout, st);
+    case DT_BF16: return launch_q<QT>((const __bf16 *)src, dst, N, K, layout, st);
+    default: return -4;
+    }
+}
+
+int launch_quantize(const void *src, int src_dtype, void *dst, int qtype, int64_t N, int64_t K, int layout, hipStream_t st) {
     switch (qtype) {
-    case QT_SYM_INT4: return launch_q<QT_SYM_INT4>(src, dst, N, K, layout, st);
-    case QT_ASYM_INT4: return launch_q<QT_ASYM_INT4>(src, dst, N, K, layout, st);
-    case QT_SYM_INT8: return launch_q<QT_SYM_INT8>(src, dst, N, K, layout, st);
-    case QT_NF4: return launch_q<QT_NF4>(src, dst, N, K, layout, st);
-    case QT_FP8_E4M3: return launch_q<QT_FP8_E4M3>(src, dst, N, K, layout, st);
+    case QT_SYM_INT4: return launch_q_dt<QT_SYM_INT4>(src, src_dtype, dst, N, K, layout, st);
+    case QT_ASYM_INT4: return launch_q_dt<QT_ASYM_INT4>(src, src_dtype, dst, N, K, layout, st);
+    case QT_SYM_INT8: return launch_q_dt<QT_SYM_INT8>(src, src_dtype, dst, N, K, layout, st);
+    case QT_NF4: return launch_q_dt<QT_NF4>(src, src_dtype, dst, N, K, layout, st);
+    case QT_FP8_E4M3: return launch_q_dt<QT_FP8_E4M3>(src, src_dtype, dst, N, K, layout, st);
     default: return -2;
     }
 }

@@ -177,6 +177,8 @@ _lib.lowbit_tileable.argtypes = [c_int, c_int64, c_int64]
 _lib.lowbit_tileable.restype = c_int
 _lib.lowbit_quantize.argtypes = [c_void_p, c_void_p, c_int, c_int64, c_int64, c_int, c_void_p]
 _lib.lowbit_quantize.restype = c_int
+_lib.lowbit_quantize_from.argtypes = [c_void_p, c_int, c_void_p, c_int, c_int64, c_int64, c_int, c_void_p]
+_lib.lowbit_quantize_from.restype = c_int
 _lib.lowbit_relayout.argtypes = [c_void_p, c_void_p, c_int, c_int64, c_int64, c_int, c_void_p]
 _lib.lowbit_relayout.restype = c_int
 _lib.lowbit_dequantize.argtypes = [c_void_p, c_void_p, c_int, c_int64, c_int64, c_int, c_int, c_void_p]
@@ -384,6 +386,10 @@ def lowbit_tileable(qtype, n, k) -> bool:
 
 def lowbit_quantize(src, dst, qtype, n, k, layout, stream):
     _check(_lib.lowbit_quantize(src, dst, qtype, n, k, layout, stream), "lowbit_quantize")
+
+
+def lowbit_quantize_from(src, src_dtype, dst, qtype, n, k, layout, stream):
+    _check(_lib.lowbit_quantize_from(src, src_dtype, dst, qtype, n, k, layout, stream), "lowbit_quantize")
 
 
 def lowbit_relayout(src, dst, qtype, n, k, src_layout, stream):

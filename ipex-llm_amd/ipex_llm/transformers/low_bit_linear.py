@@ -50,6 +50,25 @@ def _stream(device=None):
     return ctypes.c_void_p(torch.cuda.current_stream(device).cuda_stream)
 
 
+def _to_gpu(t, device=_ACCEL):
+    """t.to(device); a large host tensor goes up in chunks through pinned memory."""
+    device = torch.device(device)
+    if t.device.type == "cpu":
+        up = ops.upload(t.detach(), torch.cuda.current_device() if device.index is None else device.index)
+        if up is not None:
+            return up
+    return t.to(device)
+
+
+def _to_device(t, device):
+    """t.to(device); a large GPU tensor comes down to the host in chunks through pinned memory."""
+    if torch.device(device).type == "cpu" and t.device.type == _ACCEL:
+        down = ops.download(t.detach())
+        if down is not None:
+            return down
+    return t.to(device)
+
+
 def _require_gpu(what):
     invalidInputError(torch.cuda.is_available(),
                       f"{what} needs an MI355X: the low-bit kernels have no CPU implementation.")
@@ -87,13 +106,23 @@ def ggml_convert_qtype(tensor: torch.Tensor, qtype: int,
 
     The blob is in the ggml layout unless `layout` asks for the tiled one (only meaningful
     for a GPU destination).  A CUDA source is quantized where it is; a CPU source is staged
-    through the GPU by ggml_quantize_tensor.
+    through the GPU.
     """
+    QK = ggml.ggml_qk_size(qtype)
+    invalidInputError(QK > 0, f"qtype {qtype} has no MI355X kernel in this build "
+                              "(supported: sym_int4, asym_int4, sym_int8, nf4, fp8_e4m3)")
+    invalidInputError(tensor.dtype == torch.float, "Input tensor must be float32")
+    return _pack(tensor, qtype, device, convert_shape_only, imatrix, enable_scale_search, layout)
+
+
+def _pack(tensor, qtype, device=None, convert_shape_only=False, imatrix=None, enable_scale_search=False, layout=None):
+    """ggml_convert_qtype for a tensor of any float type.  Kernels read float32, float16 and bfloat16 as they are: a
+    half-precision checkpoint crosses to the GPU in its own two bytes a weight, and nothing is converted on the host
+    (a [11008 x 4096] float16 layer: 7 ms of 21 in .float(), and twice the bytes over the bus)."""
     QK = ggml.ggml_qk_size(qtype)
     block_size_in_bytes = ggml.ggml_type_size(qtype)
     invalidInputError(QK > 0, f"qtype {qtype} has no MI355X kernel in this build "
                               "(supported: sym_int4, asym_int4, sym_int8, nf4, fp8_e4m3)")
-    invalidInputError(tensor.dtype == torch.float, "Input tensor must be float32")
     invalidInputError(imatrix is None, "imatrix-weighted quantization is not supported")
     invalidInputError(not enable_scale_search, "enable_scale_search is not supported")
     n = tensor.numel()
@@ -107,23 +136,17 @@ def ggml_convert_qtype(tensor: torch.Tensor, qtype: int,
     if layout is None:
         layout = ggml.LAYOUT_GGML
 
-    if tensor.device.type == _ACCEL:
-        src = tensor.contiguous()
-        dst = _blob_like(dst_size, qtype, src.device)
-        if n:
-            with torch.cuda.device(src.device):
-                ggml.lowbit_quantize(src.data_ptr(), dst.data_ptr(), qtype, n // k, k, layout, _stream())
-        return dst if device is None else dst.to(device)
-
-    invalidInputError(layout == ggml.LAYOUT_GGML, "a CPU source can only produce the ggml layout")
-    _require_gpu("ggml_convert_qtype")
-    src = tensor.contiguous()
-    dst = _blob_like(dst_size, qtype, "cpu")
+    on_host = tensor.device.type != _ACCEL
+    if on_host:
+        invalidInputError(layout == ggml.LAYOUT_GGML, "a CPU source can only produce the ggml layout")
+        _require_gpu("ggml_convert_qtype")
+    src = _to_gpu(tensor.detach()) if on_host else tensor
+    src = (src if src.dtype in _DT else src.float()).contiguous()
+    dst = _blob_like(dst_size, qtype, src.device)
     if n:
-        hist = (ctypes.c_int64 * 16)()
-        ggml.ggml_quantize_tensor(ctypes.cast(src.data_ptr(), ctypes.POINTER(ctypes.c_float)),
-                                  ctypes.c_void_p(dst.data_ptr()), qtype, n, k, hist, enable_scale_search)
-    return dst if device is None else dst.to(device)
+        with torch.cuda.device(src.device):
+            ggml.lowbit_quantize_from(src.data_ptr(), _DT[src.dtype], dst.data_ptr(), qtype, n // k, k, layout, _stream())
+    return _to_device(dst, device if device is not None else tensor.device)
 
 
 def _check_blob_dtype(tensor, qtype):
@@ -139,13 +162,13 @@ def _relayout(tensor, qtype, shape, src_layout):
     if device_layout(qtype, shape) == ggml.LAYOUT_GGML:
         return tensor
     _require_gpu("layout conversion")
-    src = tensor if tensor.device.type == _ACCEL else tensor.to(_ACCEL)
+    src = _to_gpu(tensor)
     src = src.contiguous()
     dst = torch.empty_like(src)
     with torch.cuda.device(src.device):
         ggml.lowbit_relayout(src.data_ptr(), dst.data_ptr(), qtype, int(shape[0]), int(shape[-1]),
                              src_layout, _stream())
-    return dst if tensor.device.type == _ACCEL else dst.to(tensor.device)
+    return dst if tensor.device.type == _ACCEL else _to_device(dst, tensor.device)
 
 
 def ggml_q_format_convet_cpu2xpu(tensor: torch.Tensor, num_elem: int, qtype: int, shape=None):
@@ -376,7 +399,7 @@ class FP4Params(torch.nn.Parameter):
     def quantize(self, device=None):
         """In-place quantization to a ggml-layout blob on `device`."""
         if not self.quantized:
-            w = self.data.contiguous().float()
+            w = self.data
             qtype = self.qtype
             if qtype in (MOFQ4, MOFQ8):
                 # mixture-of-formats needs fp4 / picks between two encodings
@@ -385,10 +408,7 @@ class FP4Params(torch.nn.Parameter):
                                   "mixed_fp4 / mixed_fp8 need the fp4 quantizer, which has no MI355X kernel")
                 qtype = SYM_INT4 if qtype == MOFQ4 else SYM_INT8
                 self.qtype = qtype
-            self.data = ggml_convert_qtype(w, qtype, device=device,
-                                           convert_shape_only=self.convert_shape_only,
-                                           imatrix=self.imatrix, in_features=self.in_features,
-                                           enable_scale_search=self.enable_scale_search)
+            self.data = _pack(w, qtype, device, self.convert_shape_only, self.imatrix, self.enable_scale_search)
             if self.data.device.type == _ACCEL:
                 self.data = _relayout(self.data, qtype, w.shape, ggml.LAYOUT_GGML)   # residency rule
             self.quantized = True
@@ -438,13 +458,13 @@ class FP4Params(torch.nn.Parameter):
             # upload first, then quantize / re-tile on the GPU: one H2D copy, no CPU arithmetic
             if not self.quantized:
                 invalidInputError(self.qtype not in (MOFQ4, MOFQ8), "mixed formats are not supported")
-                w = self.data.to(device).contiguous().float()
+                w = _to_gpu(self.data, device)
                 self._shape = w.shape
-                blob = ggml_convert_qtype(w, self.qtype, layout=device_layout(self.qtype, w.shape),
-                                          enable_scale_search=self.enable_scale_search)
+                blob = _pack(w, self.qtype, layout=device_layout(self.qtype, w.shape),
+                             enable_scale_search=self.enable_scale_search)
                 self.quantized = True
             else:
-                blob = ggml_q_format_convet_cpu2xpu(self.data.to(device), reduce(mul, self._shape, 1),
+                blob = ggml_q_format_convet_cpu2xpu(_to_gpu(self.data, device), reduce(mul, self._shape, 1),
                                                     self.qtype, shape=self._shape)
             return self._clone_with(blob)
         if device is not None and device.type == "cpu" and cur == _ACCEL:
@@ -452,11 +472,11 @@ class FP4Params(torch.nn.Parameter):
             if self.quantized:
                 data = ggml_q_format_convet_xpu2cpu(data, reduce(mul, self._shape, 1), self.qtype,
                                                     shape=self._shape)
-            return self._clone_with(data.to(device))
+            return self._clone_with(_to_device(data, device))
         if device is not None and device.type == _ACCEL and cur == _ACCEL and not self.quantized:
-            w = self.data.to(device).contiguous().float()
+            w = self.data.to(device)
             self._shape = w.shape
-            blob = ggml_convert_qtype(w, self.qtype, layout=device_layout(self.qtype, w.shape))
+            blob = _pack(w, self.qtype, layout=device_layout(self.qtype, w.shape))
             self.quantized = True
             return self._clone_with(blob)
         return self._clone_with(super().to(device=device, dtype=None if self.quantized else dtype,

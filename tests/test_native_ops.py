@@ -29,3 +29,29 @@ def test_native_linear_equals_the_python_functions(qname, m, n, k, dtype):
     got = ops.linear(x, w, None, Q[qname], n, True)
     assert got.dtype == dtype and torch.equal(got, want)
     assert ops.linear(x, w, None, Q[qname], n + 1, True) is None                  # a weight of another size
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype,numel", [(torch.float16, (4 << 20) // 2 + 1), (torch.uint8, (8 << 20) + 3), (torch.float32, 3 << 20), (torch.bfloat16, 9 << 20)])
+def test_large_copies_through_pinned_chunks(dtype, numel):
+    t = torch.randint(0, 200, (numel + 5,)).to(dtype)[5:]                        # not at the start of its storage
+    up = ops.upload(t, 0)
+    assert up.device.type == "cuda" and up.dtype == dtype and torch.equal(up, t.cuda())
+    down = ops.download(up)
+    assert down.device.type == "cpu" and torch.equal(down, t)
+    assert ops.upload(t[:100], 0) is None and ops.upload(t[::2], 0) is None and ops.upload(up, 0) is None and ops.download(t) is None
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("qname", ["sym_int4", "asym_int4", "sym_int8", "nf4", "fp8_e4m3"])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("n,k", [(3, 128), (48, 640), (2048, 1152)])
+def test_half_precision_sources_quantize_as_their_float32_values(qname, dtype, n, k):
+    torch.manual_seed(n)
+    w = (torch.randn(n, k) * 0.02).to(dtype)
+    def blob(t, device):
+        return FP4Params(t, qtype=Q[qname]).to(device).data.view(torch.uint8)
+    want, tiled = blob(w.float(), "cpu"), blob(w.float().cuda(), "cuda")
+    for src in (w, w.t().contiguous().t()):                                       # contiguous, and not
+        assert torch.equal(blob(src, "cpu"), want)
+        assert torch.equal(blob(src, "cuda"), tiled) and torch.equal(blob(src.cuda(), "cuda"), tiled)
