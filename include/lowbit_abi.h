@@ -231,11 +231,12 @@ int lowbit_forward_f32(const float *x, const void *w, float *y, int qtype, int l
 
 /* One linear layer: y = x * dequant(w)^T + bias.  x, bias ([N], may be null) and y are of `dtype`, which may be
  * LOWBIT_DT_F32: then as lowbit_forward_f32, and no workspace is used.  With 16-bit activations as lowbit_forward_ws
- * (lowbit_workspace_bytes_for says what to pass; null is valid), the bias added to the fp32 sums before the one
+ * (lowbit_linear_workspace_bytes says what to pass within a budget; null is valid), the bias added to the fp32 sums before the one
  * rounding (a bias that is not 8-byte aligned is valid and slower above 16 rows).  What LowBitLinear.forward computes
  * (low_bit_linear.py:657-687 of the reference). */
 int lowbit_linear(const void *x, const void *w, const void *bias, void *y, int qtype, int layout, int dtype, int64_t M,
                   int64_t N, int64_t K, void *workspace, size_t workspace_bytes, void *stream);
+size_t lowbit_linear_workspace_bytes(int qtype, int layout, int dtype, int64_t M, int64_t N, int64_t K, size_t max_bytes);
 
 /* lowbit_forward_ws without a workspace argument and without any allocation: the partial tiles go to a
  * scratch array that is part of the library's image on every GPU (lowbit_noalloc_scratch_bytes() = 64 MiB,

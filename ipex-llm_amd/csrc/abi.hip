@@ -35,6 +35,9 @@ int launch_gemm_ring(const void *x, const void *w, const void *bias, void *y, in
 int launch_gemm(const void *x, const void *w, const void *bias, void *y, int qtype, int layout, int act_dtype, int M, int N, int K,
                 void *workspace, size_t workspace_bytes, int want_splits, hipStream_t st);
 int launch_gemm_narrow(const void *x, const void *w, const void *bias, void *y, int qtype, int act_dtype, int M, int N, int K, hipStream_t st);
+size_t gemm_rows_workspace_bytes(int M, int N, int K, size_t max_bytes);
+int launch_gemm_rows(const void *x, const void *w, const void *bias, void *y, int qtype, int act_dtype, int M, int N, int K,
+                     void *workspace, size_t workspace_bytes, hipStream_t st);
 double narrow_time_us(int M, int N, int K, int qtype);
 int gemm_splits(int M, int N, int K, size_t ws_bytes, int qtype);
 double gemm_time_us(int M, int N, int K, int splits, int qtype);
@@ -350,6 +353,8 @@ static int forward_any(const char *what, const void *x, const void *w, const voi
     const int m = (int)M, n = (int)N, k = (int)K;
     hipStream_t st = (hipStream_t)stream;
     int splits = 1, rc = 0;
+    if (layout == LOWBIT_LAYOUT_GGML && M > 16)          // (up to 16 rows: one streaming pass)
+        return check_launch(launch_gemm_rows(x, w, bias, y, qtype, act_dtype, m, n, k, workspace, workspace_bytes, st), what);
     switch (plan_forward(qtype, layout, M, N, K, workspace != nullptr, workspace_bytes, !(((uintptr_t)y | (uintptr_t)bias) & 7), &splits)) {
     case PLAN_GEMV: rc = launch_gemv(x, w, bias, y, qtype, layout, act_dtype, m, n, k, 0, st); break;
     case PLAN_RING: rc = launch_gemm_ring(x, w, bias, y, qtype, act_dtype, m, n, k, workspace, workspace_bytes, 0, st); break;
@@ -380,6 +385,13 @@ static int forward_f32(const char *what, const float *x, const void *w, const fl
         return fail(LOWBIT_EARG, "%s: null or misaligned pointer (x, w: 16 bytes)", what);
     if (K % 8) return fail(LOWBIT_ESHAPE, "%s: K must be a multiple of 8", what);
     return check_launch(launch_gemv(x, w, bias, y, qtype, layout, LOWBIT_DT_F32, (int)M, (int)N, (int)K, 0, (hipStream_t)stream), what);
+}
+
+size_t lowbit_linear_workspace_bytes(int qtype, int layout, int dtype, int64_t M, int64_t N, int64_t K, size_t max_bytes) {
+    if (dtype == LOWBIT_DT_F32 || M <= 16) return 0;     // one streaming pass per 16 rows
+    if (layout != LOWBIT_LAYOUT_GGML) return lowbit_workspace_bytes_for(qtype, layout, M, N, K, max_bytes);
+    if (!qk_size(qtype) || N <= 0 || K <= 0 || M > 0x7fffffff || N > 0x7fffffff || K > 0x7fffffff) return 0;
+    return gemm_rows_workspace_bytes((int)M, (int)N, (int)K, max_bytes);
 }
 
 int lowbit_linear(const void *x, const void *w, const void *bias, void *y, int qtype, int layout, int dtype, int64_t M,

@@ -21,6 +21,9 @@ namespace lowbit {
 int launch_gemv(const void *x, const void *w, const void *bias, void *y, int qtype, int layout, int act_dtype, int M, int N, int K,
                 int waves, hipStream_t st);
 
+int launch_gemm_rows(const void *x, const void *w, const void *bias, void *y, int qtype, int act_dtype, int M, int N, int K,
+                     void *workspace, size_t workspace_bytes, hipStream_t st);
+
 // Sums the fp32 partial tiles of the splits (stored in the GEMM's register layout: split, tile, wave,
 // register group, lane) and writes y, rounded once.  One thread per group of 4 consecutive n.
 template <typename AT>
@@ -273,7 +276,8 @@ int launch_gemm(const void *x, const void *w, const void *bias, void *y, int qty
                 void *workspace, size_t workspace_bytes, int want_splits, hipStream_t st) {
     if (M == 0 || N == 0) return 0;
     // the MFMA GEMM reads the tiled layout and stores 8-byte groups of y (N % 4 == 0 is implied
-    // by N % 16 == 0); anything else goes through the streaming kernel in 16-row slices
+    // by N % 16 == 0); row-major weights have their own, a y of another alignment goes through the streaming kernel
+    if (layout == LAYOUT_GGML) return launch_gemm_rows(x, w, bias, y, qtype, act_dtype, M, N, K, workspace, workspace_bytes, st);
     if (layout != LAYOUT_TILED || (N % TILE_ROWS) || (K % TILE_COLS) || (((uintptr_t)y) & 7))
         return launch_gemv(x, w, bias, y, qtype, layout, act_dtype, M, N, K, 0, st);
     float *ws = (float *)workspace;

@@ -16,180 +16,11 @@
 // float32 activations (F32).
 #include "lowbit_mfma.h"
 #include "lowbit_rows.h"
+#include "lowbit_unpack.h"
 
 #include <type_traits>
 
 namespace lowbit {
-
-// ---- codes of one sub-block (8 columns of this lane) -> B operand ----------
-//
-// The operand holds the *unscaled* code value (q - 8, q, int8, e4m3 value, nf4
-// code-book entry); OFFSET<> says what constant is still folded in and has to
-// be removed with the row sum of x (0 for every path below except bf16 4-bit).
-
-template <int QT, typename AT> struct Unpack;
-
-// 4-bit integer codes, fp16: 0x6400 | q is the half 1024 + q; 0x6400 | q << 4 is 1024 + 16 q.
-template <> struct Unpack<QT_SYM_INT4, _Float16> {
-    static constexpr float OFFSET = 0.0f;
-    __device__ static f16x8 run(uint32_t v, const void *, uint32_t magic) {
-        const f16x2 k1032 = {(_Float16)1032.0f, (_Float16)1032.0f};
-        const f16x2 k16th = {(_Float16)0.0625f, (_Float16)0.0625f};
-        const f16x2 k72 = {(_Float16)72.0f, (_Float16)72.0f};
-        const uint32_t v8 = v >> 8;
-        f16x2 t0 = __builtin_bit_cast(f16x2, and_or(v, 0x000f000fu, magic)) - k1032;
-        f16x2 t1 = __builtin_elementwise_fma(__builtin_bit_cast(f16x2, and_or(v, 0x00f000f0u, magic)), k16th, -k72);
-        f16x2 t2 = __builtin_bit_cast(f16x2, and_or(v8, 0x000f000fu, magic)) - k1032;
-        f16x2 t3 = __builtin_elementwise_fma(__builtin_bit_cast(f16x2, and_or(v8, 0x00f000f0u, magic)), k16th, -k72);
-        return f16x8{t0[0], t0[1], t1[0], t1[1], t2[0], t2[1], t3[0], t3[1]};
-    }
-};
-template <> struct Unpack<QT_ASYM_INT4, _Float16> {
-    static constexpr float OFFSET = 0.0f;
-    __device__ static f16x8 run(uint32_t v, const void *, uint32_t magic) {
-        const f16x2 k1024 = {(_Float16)1024.0f, (_Float16)1024.0f};
-        const f16x2 k16th = {(_Float16)0.0625f, (_Float16)0.0625f};
-        const f16x2 k64 = {(_Float16)64.0f, (_Float16)64.0f};
-        const uint32_t v8 = v >> 8;
-        f16x2 t0 = __builtin_bit_cast(f16x2, and_or(v, 0x000f000fu, magic)) - k1024;
-        f16x2 t1 = __builtin_elementwise_fma(__builtin_bit_cast(f16x2, and_or(v, 0x00f000f0u, magic)), k16th, -k64);
-        f16x2 t2 = __builtin_bit_cast(f16x2, and_or(v8, 0x000f000fu, magic)) - k1024;
-        f16x2 t3 = __builtin_elementwise_fma(__builtin_bit_cast(f16x2, and_or(v8, 0x00f000f0u, magic)), k16th, -k64);
-        return f16x8{t0[0], t0[1], t1[0], t1[1], t2[0], t2[1], t3[0], t3[1]};
-    }
-};
-// 4-bit integer codes, bf16: 0x4300 | q is the bf16 128 + q (exact); the constant is removed
-// afterwards through the row sum of x, which a second MFMA against all-ones provides.
-template <int QT> struct UnpackInt4Bf16 {
-    static constexpr float OFFSET = (QT == QT_SYM_INT4) ? 136.0f : 128.0f;
-    __device__ static bf16x8 run(uint32_t v, const void *, uint32_t magic) {
-        u32x4 t;
-        t[0] = and_or(v, 0x000f000fu, magic);
-        t[1] = and_or(v >> 4, 0x000f000fu, magic);
-        t[2] = and_or(v >> 8, 0x000f000fu, magic);
-        t[3] = and_or(v >> 12, 0x000f000fu, magic);
-        return __builtin_bit_cast(bf16x8, t);
-    }
-};
-template <> struct Unpack<QT_SYM_INT4, __bf16> : UnpackInt4Bf16<QT_SYM_INT4> {};
-template <> struct Unpack<QT_ASYM_INT4, __bf16> : UnpackInt4Bf16<QT_ASYM_INT4> {};
-
-// nf4: code-book lookup, two ways.
-//   - From a 16-entry table in LDS: eight 2-byte reads and about twelve vector instructions per dword of codes.
-//   - In registers: the 16 entries, already in the activation type, lie in two byte planes (low bytes, high bytes)
-//     of four registers each; v_perm_b32 looks four codes up at a time in the eight bytes of a register pair -
-//     entries 0..7 and 8..15 separately, a third v_perm_b32 picks per byte by the code's bit 3 - and two more
-//     interleave the planes into 16-bit values: 21 vector instructions per dword of eight codes, no LDS access.
-// Measured on one MI355X on the Llama-3-70B linear set (419 MB of nf4 weights, bf16): at M = 1 from LDS 115.9 us,
-// in registers 123.0, half of the sub-blocks each way 117.7; at M = 16, where x takes its share of the LDS pipe,
-// 171.4 / 156.7 / 165.6.  So up to four rows of x look up in LDS and more rows in registers.  Either way nf4 stays
-// a quarter behind sym_int4 at the same bytes ([28672 x 8192] at M = 1: 31.7 against 25.5 us): the lookups are
-// instructions the integer formats do not issue, whichever unit takes them.
-struct Nf4Planes {
-    uint32_t lo[4], hi[4];        // byte i % 4 of register i / 4 = low / high byte of entry i
-    uint32_t k04, k0123;          // 0x04040404 and 0x03020100 in vector registers: as literals the two would need the
-                                  // one constant slot of v_and_or_b32 twice
-};
-// RESID: what rounding the code book to AT dropped (the second term of the fp32-output variants)
-template <typename AT, bool RESID> __device__ inline Nf4Planes nf4_planes() {
-    Nf4Planes t = {};
-#pragma unroll
-    for (int i = 0; i < 16; i++) {                      // (constants: folded at compile time)
-        const AT main = to_at<AT>(NF4_CODEBOOK[i]);
-        const AT v = RESID ? to_at<AT>(NF4_CODEBOOK[i] - (float)main) : main;
-        const uint32_t b = __builtin_bit_cast(uint16_t, v);
-        t.lo[i / 4] |= (b & 0xffu) << (8 * (i % 4));
-        t.hi[i / 4] |= (b >> 8) << (8 * (i % 4));
-    }
-    asm("v_mov_b32 %0, 0x04040404" : "=v"(t.k04));
-    asm("v_mov_b32 %0, 0x03020100" : "=v"(t.k0123));
-    return t;
-}
-template <typename AT> struct Unpack<QT_NF4, AT> {
-    static constexpr float OFFSET = 0.0f;
-    // four codes, one per byte of `sel` (bits 0..2) and `mrg` (0x03020100 + 4 * bit 3 per byte) -> one byte plane
-    __device__ static uint32_t plane4(const uint32_t (&p)[4], uint32_t sel, uint32_t mrg) {
-        return __builtin_amdgcn_perm(__builtin_amdgcn_perm(p[3], p[2], sel), __builtin_amdgcn_perm(p[1], p[0], sel), mrg);
-    }
-    __device__ static typename Vec8<AT>::type run(uint32_t v, const void *planes_, uint32_t) {
-        const Nf4Planes &t = *(const Nf4Planes *)planes_;
-        // nibbles 0, 2, 4, 6 (columns 0, 4, 1, 5) are the low nibbles of the four bytes, 1, 3, 5, 7 (columns 2, 6,
-        // 3, 7) the high ones
-        const uint32_t sel_e = v & 0x07070707u, mrg_e = and_or(v >> 1, t.k04, t.k0123);
-        const uint32_t sel_o = (v >> 4) & 0x07070707u, mrg_o = and_or(v >> 5, t.k04, t.k0123);
-        const uint32_t lo_e = plane4(t.lo, sel_e, mrg_e), hi_e = plane4(t.hi, sel_e, mrg_e);
-        const uint32_t lo_o = plane4(t.lo, sel_o, mrg_o), hi_o = plane4(t.hi, sel_o, mrg_o);
-        u32x4 r;
-        r[0] = __builtin_amdgcn_perm(hi_e, lo_e, 0x06020400u);      // columns 0, 1: bytes 0 and 2 of the even set
-        r[1] = __builtin_amdgcn_perm(hi_o, lo_o, 0x06020400u);      // columns 2, 3
-        r[2] = __builtin_amdgcn_perm(hi_e, lo_e, 0x07030501u);      // columns 4, 5: bytes 1 and 3
-        r[3] = __builtin_amdgcn_perm(hi_o, lo_o, 0x07030501u);      // columns 6, 7
-        return __builtin_bit_cast(typename Vec8<AT>::type, r);
-    }
-    __device__ static typename Vec8<AT>::type run_lds(uint32_t v, const AT *lut) {
-        typename Vec8<AT>::type r;
-        r[0] = lut[v & 0xf]; r[2] = lut[(v >> 4) & 0xf]; r[4] = lut[(v >> 8) & 0xf]; r[6] = lut[(v >> 12) & 0xf];
-        r[1] = lut[(v >> 16) & 0xf]; r[3] = lut[(v >> 20) & 0xf]; r[5] = lut[(v >> 24) & 0xf]; r[7] = lut[v >> 28];
-        return r;
-    }
-};
-
-// 8-bit codes: two dwords (columns 0..3, 4..7).
-template <int QT, typename AT> struct Unpack8;
-template <> struct Unpack8<QT_SYM_INT8, _Float16> {
-    __device__ static f16x8 run(uint32_t lo, uint32_t hi) {
-        // byte ^ 0x80 = q + 128 (unsigned); 0x6400 | u is the half 1024 + u
-        const f16x2 k1152 = {(_Float16)1152.0f, (_Float16)1152.0f};
-        const uint32_t a = lo ^ 0x80808080u, b = hi ^ 0x80808080u;
-        const uint32_t c64 = 0x64646464u;
-        f16x2 t0 = __builtin_bit_cast(f16x2, __builtin_amdgcn_perm(c64, a, 0x04010400u)) - k1152;
-        f16x2 t1 = __builtin_bit_cast(f16x2, __builtin_amdgcn_perm(c64, a, 0x04030402u)) - k1152;
-        f16x2 t2 = __builtin_bit_cast(f16x2, __builtin_amdgcn_perm(c64, b, 0x04010400u)) - k1152;
-        f16x2 t3 = __builtin_bit_cast(f16x2, __builtin_amdgcn_perm(c64, b, 0x04030402u)) - k1152;
-        return f16x8{t0[0], t0[1], t1[0], t1[1], t2[0], t2[1], t3[0], t3[1]};
-    }
-};
-template <> struct Unpack8<QT_SYM_INT8, __bf16> {
-    __device__ static bf16x8 run(uint32_t lo, uint32_t hi) {
-        bf16x8 r;
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-            r[i] = (__bf16)(float)(int8_t)(lo >> (8 * i));      // |q| <= 128: exact in bf16
-            r[4 + i] = (__bf16)(float)(int8_t)(hi >> (8 * i));
-        }
-        return r;
-    }
-};
-template <> struct Unpack8<QT_FP8_E4M3, _Float16> {
-    __device__ static f16x8 run(uint32_t lo, uint32_t hi) {
-        f16x2 t0 = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(lo, 1.0f, false);
-        f16x2 t1 = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(lo, 1.0f, true);
-        f16x2 t2 = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(hi, 1.0f, false);
-        f16x2 t3 = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(hi, 1.0f, true);
-        return f16x8{t0[0], t0[1], t1[0], t1[1], t2[0], t2[1], t3[0], t3[1]};
-    }
-};
-template <> struct Unpack8<QT_FP8_E4M3, __bf16> {
-    __device__ static bf16x8 run(uint32_t lo, uint32_t hi) {
-        bf16x2 t0 = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(lo, 1.0f, false);
-        bf16x2 t1 = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(lo, 1.0f, true);
-        bf16x2 t2 = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(hi, 1.0f, false);
-        bf16x2 t3 = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(hi, 1.0f, true);
-        return bf16x8{t0[0], t0[1], t1[0], t1[1], t2[0], t2[1], t3[0], t3[1]};
-    }
-};
-
-template <int QT, typename AT> constexpr float code_offset() {
-    if constexpr (Fmt<QT>::BITS == 4) return Unpack<QT, AT>::OFFSET;
-    else return 0.0f;
-}
-
-template <typename AT> __device__ inline typename Vec8<AT>::type ones8() {
-    typename Vec8<AT>::type r;
-#pragma unroll
-    for (int i = 0; i < 8; i++) r[i] = to_at<AT>(1.0f);
-    return r;
-}
 
 // Eight floats -> their bf16 values and those of what the rounding dropped.  inf / nan stay in the first plane only.
 __device__ inline void split_f32(const u32x4 &a, const u32x4 &b, u32x4 &hi, u32x4 &lo) {
@@ -281,13 +112,14 @@ __global__ __launch_bounds__(1024) void gemv_mfma_kernel(const AT *__restrict__ 
     constexpr int NW = DUAL ? 2 : R;
     static_assert(!(DUAL && R != 1) && XN * 1024 >= NW * MT * 256, "bad GEMV shape parameters");
     static_assert(!ROWS || (!DUAL && MOE == 0), "row-major weights: the plain product only");
-    // nf4 code book in the activation type (byte planes in registers).  With fp32 output a second table holds what
-    // the rounding to AT dropped, and a second MFMA per sub-block adds it: the weights then carry 16 mantissa bits
-    // like x does.
+    // nf4 code book in the activation type (byte planes in registers).  With fp32 activations and for row-major weights
+    // (which have always been decoded to fp32) a second table holds what the rounding to AT dropped, and a second
+    // MFMA per sub-block adds it: the weights then carry 16 mantissa bits and more.
+    constexpr bool NF4_LO = QT == QT_NF4 && (F32 || ROWS);
     const Nf4Planes lut_planes = (QT == QT_NF4) ? nf4_planes<AT, false>() : Nf4Planes{};
-    const Nf4Planes lut_lo_planes = (QT == QT_NF4 && F32) ? nf4_planes<AT, true>() : Nf4Planes{};
+    const Nf4Planes lut_lo_planes = NF4_LO ? nf4_planes<AT, true>() : Nf4Planes{};
     const void *const lut = &lut_planes, *const lut_lo = &lut_lo_planes;
-    constexpr bool NF4_IN_LDS = QT == QT_NF4 && MT == 1 && !F32;     // (see Unpack<QT_NF4>)
+    constexpr bool NF4_IN_LDS = QT == QT_NF4 && MT == 1 && !NF4_LO;     // (see Unpack<QT_NF4>)
     __shared__ AT lut_lds[16];
     if constexpr (NF4_IN_LDS) {
         if (threadIdx.x < 16) lut_lds[threadIdx.x] = to_at<AT>(NF4_CODEBOOK[threadIdx.x]);
@@ -487,9 +319,10 @@ __global__ __launch_bounds__(1024) void gemv_mfma_kernel(const AT *__restrict__ 
                     }
                     f32x4 p = mfma16(a[j], b, zero4);
                     if constexpr (F32) p = mfma16(al[j], b, p);
-                    if constexpr (QT == QT_NF4 && F32) {
+                    if constexpr (NF4_LO) {
                         const V8 bl = Unpack<QT, AT>::run(tl.q0[j], lut_lo, magic);
-                        p = mfma16(al[j], bl, mfma16(a[j], bl, p));
+                        p = mfma16(a[j], bl, p);
+                        if constexpr (F32) p = mfma16(al[j], bl, p);
                     }
                     if constexpr (NEED_S) {
                         f32x4 s = mfma16(a[j], ones, zero4);

@@ -75,22 +75,26 @@ template <int QT> __device__ inline void arrange_rows(RowRegs<QT> &t, uint32_t (
 }
 
 // Eight consecutive columns of x (chunk u of a row whose first column is a multiple of 128), stored into the row's
-// LDS image in the order of the steps: 16 bytes at (step * 4 + c) * 16.
-template <int QT> __device__ inline void store_x_rows(uint8_t *row, int u, const u32x4 &x) {
+// LDS image in the order of the steps: lane c's operand of step j is the 16-byte unit j * 4 + c (of its 128 columns).
+// `swizzle` (below 16) is xor-ed onto the unit: a kernel whose lanes read 16 rows 256 bytes apart passes the row, which
+// spreads them over the LDS banks.
+template <int QT> __device__ inline void store_x_rows(uint8_t *row, int u, const u32x4 &x, int swizzle = 0) {
+    const int group = (u >> 4) * 16;
+    auto unit = [&](int j, int c) __attribute__((always_inline)) { return row + (group + ((j * 4 + c) ^ swizzle)) * 16; };
     if constexpr (QT == QT_FP8_E4M3) {
-        *(u32x4 *)(row + (u >> 4) * 256 + (u & 3) * 64 + ((u >> 2) & 3) * 16) = x;
+        *(u32x4 *)unit(u & 3, (u >> 2) & 3) = x;
     } else if constexpr (QT == QT_SYM_INT8) {
-        uint8_t *p = row + (u >> 2) * 64 + (u & 1) * 32 + ((u >> 1) & 1) * 8;
-        *(u32x2 *)p = u32x2{x[0], x[1]};
-        *(u32x2 *)(p + 16) = u32x2{x[2], x[3]};
+        const int j = (u >> 2) & 3, c = 2 * (u & 1), half = ((u >> 1) & 1) * 8;
+        *(u32x2 *)(unit(j, c) + half) = u32x2{x[0], x[1]};
+        *(u32x2 *)(unit(j, c + 1) + half) = u32x2{x[2], x[3]};
     } else {
-        uint8_t *p;
-        if constexpr (QT == QT_NF4) p = row + (u >> 3) * 128 + ((u >> 1) & 1) * 64 + (u & 1) * 32 + ((u >> 2) & 1) * 4;
-        else p = row + (u >> 2) * 64 + (u & 1) * 32 + ((u >> 1) & 1) * 4;
+        const int j = QT == QT_NF4 ? ((u >> 3) & 1) * 2 + ((u >> 1) & 1) : (u >> 2) & 3, c = 2 * (u & 1);
+        const int hi = (QT == QT_NF4 ? (u >> 2) & 1 : (u >> 1) & 1) * 4;
+        uint8_t *const p = unit(j, c) + hi, *const q = unit(j, c + 1) + hi;
         *(uint32_t *)p = __builtin_amdgcn_perm(x[1], x[0], 0x05040100u);          // columns 0, 2
         *(uint32_t *)(p + 8) = __builtin_amdgcn_perm(x[1], x[0], 0x07060302u);    // columns 1, 3
-        *(uint32_t *)(p + 16) = __builtin_amdgcn_perm(x[3], x[2], 0x05040100u);   // columns 4, 6
-        *(uint32_t *)(p + 24) = __builtin_amdgcn_perm(x[3], x[2], 0x07060302u);   // columns 5, 7
+        *(uint32_t *)q = __builtin_amdgcn_perm(x[3], x[2], 0x05040100u);          // columns 4, 6
+        *(uint32_t *)(q + 8) = __builtin_amdgcn_perm(x[3], x[2], 0x07060302u);    // columns 5, 7
     }
 }
 

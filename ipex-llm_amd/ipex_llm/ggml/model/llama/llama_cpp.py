@@ -269,6 +269,14 @@ def lowbit_forward_f32(x, w, y, qtype, layout, m, n, k, workspace, workspace_byt
            "lowbit_forward_f32")
 
 
+_lib.lowbit_linear_workspace_bytes.argtypes = [c_int, c_int, c_int, c_int64, c_int64, c_int64, c_size_t]
+_lib.lowbit_linear_workspace_bytes.restype = c_size_t
+
+
+def lowbit_linear_workspace_bytes(qtype, layout, dtype, m, n, k, max_bytes) -> int:
+    return int(_lib.lowbit_linear_workspace_bytes(qtype, layout, dtype, m, n, k, max_bytes))
+
+
 _lib.lowbit_linear.argtypes = [c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int64, c_int64, c_int64,
                                c_void_p, c_size_t, c_void_p]
 _lib.lowbit_linear.restype = c_int

@@ -17,7 +17,7 @@ def _check(qtype, dtype, layout, m, n, k, biased, seed):
     bias = torch.from_numpy(np.random.default_rng(seed + 2).standard_normal(n).astype(np.float32)).to(dtype) if biased else None
     blob, xd = dev_quantize(w, qtype, layout), x.cuda()
     bd = bias.cuda() if biased else None
-    need = ggml.lowbit_workspace_bytes_for(qtype, layout, m, n, k, 64 << 20)
+    need = ggml.lowbit_linear_workspace_bytes(qtype, layout, DT[dtype], m, n, k, 64 << 20)
     ws = torch.empty(max(need, 16), dtype=torch.uint8, device="cuda")
     # guard rows on both sides: the kernel writes the m x n results and nothing else
     y = torch.full((m + 2, n), float("nan"), dtype=dtype, device="cuda")
