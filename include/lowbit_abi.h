@@ -178,9 +178,9 @@ int lowbit_dequantize_rows(const void *w, const int64_t *rows, int64_t n_rows, v
                            int64_t K, int layout, int out_dtype, void *stream);
 /* xe_linear.mlp_forward_xpu (python/llm/src/ipex_llm/transformers/models/common.py:145-158; signature
  * xpu_ops.py:34-37): y[M, N] = act(x * Wg^T) .* (x * Wu^T) in one launch, both weights tiled [N, K].
- * Any M (the reference fuses at M == 1 only, models/utils.py:246-259): up to 16 rows run the streaming
- * kernel (one pass over both weights; two passes up to 31 rows while a weight has at most 32 MiB), more
- * rows the fused gate/up form of the tiled GEMM (y 8-byte aligned, M < 2^24, K < 2^23). */
+ * Any M (the reference fuses at M == 1 only, models/utils.py:246-259): up to 32 rows, and up
+ * to 64 where a weight has at most 16384 rows, run in one pass over both weights, more rows the fused
+ * gate/up form of the tiled GEMM (y 8-byte aligned, M < 2^24, K < 2^23). */
 int lowbit_mlp_forward(const void *x, const void *w_gate, const void *w_up, void *y, int qtype, int act_dtype,
                        int64_t M, int64_t N, int64_t K, int act, void *stream);
 
@@ -222,8 +222,8 @@ int lowbit_gemm_ws(const void *x, const void *w, void *y, int qtype, int layout,
  * hands them a float x (python/llm/src/ipex_llm/transformers/low_bit_linear.py:657-668: only M > 1 with
  * conver_to_half casts to half first) and what the CPU branch's ggml_compute_forward_mul_mat_q_fp32 returns.
  * x is split into two bf16 planes (16 mantissa bits, fp32's exponent range), the product of the 2M rows is
- * accumulated and stored in fp32 and the halves are added.  The streaming kernel serves every M (16 rows of
- * the planes per pass over the weights): meant for decode and small batches.  workspace: caller-owned device
+ * accumulated and stored in fp32 and the halves are added.  Every M runs in passes over the weights of up to
+ * 32 rows: meant for decode and small batches.  workspace: caller-owned device
  * memory of lowbit_forward_f32_workspace_bytes(M, N, K) bytes, 16-byte aligned. */
 size_t lowbit_forward_f32_workspace_bytes(int64_t M, int64_t N, int64_t K);
 int lowbit_forward_f32(const float *x, const void *w, float *y, int qtype, int layout, int64_t M, int64_t N, int64_t K,

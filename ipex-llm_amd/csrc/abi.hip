@@ -28,6 +28,11 @@ int launch_dequantize(const void *w, void *out, int qtype, int64_t N, int64_t K,
                       hipStream_t st);
 int launch_gemv(const void *x, const void *w, const void *bias, void *y, int qtype, int layout, int act_dtype, int M, int N, int K,
                 int waves, hipStream_t st);
+int launch_gemv_wide(const void *x, const void *w, const void *bias, void *y, int qtype, int layout, int act_dtype, int M, int N, int K,
+                     hipStream_t st);
+bool gemv_wide_applies(int qtype, int layout, int act_dtype, int M, int N, int K);
+int launch_mlp_wide(const void *x, const void *wg, const void *wu, void *y, int qtype, int act_dtype, int M, int N, int K, int act,
+                    hipStream_t st);
 size_t ring_workspace_bytes(int M, int N, int K, int wgs);
 double ring_time_us(int M, int N, int K, int qtype, bool have_ws);
 int launch_gemm_ring(const void *x, const void *w, const void *bias, void *y, int qtype, int act_dtype, int M, int N, int K,
@@ -342,8 +347,11 @@ extern "C" int lowbit_forward_plan(int qtype, int layout, int64_t M, int64_t N, 
     return plan_forward(qtype, layout, M, N, K, have_workspace != 0, have_workspace ? workspace_bytes : 0, true, nullptr);
 }
 
+// linear: lowbit_linear, which is free to take the one-pass kernel (gemv_wide.hip) in place of any planned one; elsewhere it
+// stands in for the streaming kernel's plan only, which is what it is.
 static int forward_any(const char *what, const void *x, const void *w, const void *bias, void *y, int qtype, int layout,
-                       int act_dtype, int64_t M, int64_t N, int64_t K, void *workspace, size_t workspace_bytes, void *stream) {
+                       int act_dtype, int64_t M, int64_t N, int64_t K, void *workspace, size_t workspace_bytes, void *stream,
+                       bool linear = false) {
     if (int rc = check_mm(what, x, w, y, qtype, layout, act_dtype, M, N, K)) return rc;
     if (M * N == 0) return 0;
     if (K == 0) return fail(LOWBIT_ESHAPE, "%s: K == 0", what);
@@ -353,9 +361,15 @@ static int forward_any(const char *what, const void *x, const void *w, const voi
     const int m = (int)M, n = (int)N, k = (int)K;
     hipStream_t st = (hipStream_t)stream;
     int splits = 1, rc = 0;
+    const int plan = linear && gemv_wide_applies(qtype, layout, act_dtype, m, n, k) ? PLAN_GEMV
+        : plan_forward(qtype, layout, M, N, K, workspace != nullptr, workspace_bytes, !(((uintptr_t)y | (uintptr_t)bias) & 7), &splits);
+    if (plan == PLAN_GEMV) {
+        rc = launch_gemv_wide(x, w, bias, y, qtype, layout, act_dtype, m, n, k, st);
+        if (rc <= 0) return check_launch(rc, what);
+    }
     if (layout == LOWBIT_LAYOUT_GGML && M > 16)          // (up to 16 rows: one streaming pass)
         return check_launch(launch_gemm_rows(x, w, bias, y, qtype, act_dtype, m, n, k, workspace, workspace_bytes, st), what);
-    switch (plan_forward(qtype, layout, M, N, K, workspace != nullptr, workspace_bytes, !(((uintptr_t)y | (uintptr_t)bias) & 7), &splits)) {
+    switch (plan) {
     case PLAN_GEMV: rc = launch_gemv(x, w, bias, y, qtype, layout, act_dtype, m, n, k, 0, st); break;
     case PLAN_RING: rc = launch_gemm_ring(x, w, bias, y, qtype, act_dtype, m, n, k, workspace, workspace_bytes, 0, st); break;
     case PLAN_GEMM_SPLIT: rc = launch_gemm(x, w, bias, y, qtype, layout, act_dtype, m, n, k, workspace, workspace_bytes, splits, st); break;
@@ -375,7 +389,7 @@ int lowbit_forward_ws(const void *x, const void *w, void *y, int qtype, int layo
     return forward_any("lowbit_forward_ws", x, w, nullptr, y, qtype, layout, act_dtype, M, N, K, workspace, workspace_bytes, stream);
 }
 
-// ---- fp32 activations: the streaming kernel's F32 form for every M
+// ---- fp32 activations: the one-pass kernel in passes of 32 rows, the streaming kernel for a rest of up to 8
 static int forward_f32(const char *what, const float *x, const void *w, const float *bias, float *y, int qtype, int layout,
                        int64_t M, int64_t N, int64_t K, void *stream) {
     if (int rc = check_weight_shape(what, qtype, N, K, layout)) return rc;
@@ -384,11 +398,19 @@ static int forward_f32(const char *what, const float *x, const void *w, const fl
     if (!x || !w || !y || !aligned16(x) || !aligned16(w) || (((uintptr_t)y | (uintptr_t)bias) & 3))
         return fail(LOWBIT_EARG, "%s: null or misaligned pointer (x, w: 16 bytes)", what);
     if (K % 8) return fail(LOWBIT_ESHAPE, "%s: K must be a multiple of 8", what);
-    return check_launch(launch_gemv(x, w, bias, y, qtype, layout, LOWBIT_DT_F32, (int)M, (int)N, (int)K, 0, (hipStream_t)stream), what);
+    for (int64_t m0 = 0; m0 < M; m0 += 32) {
+        const int m = (int)(M - m0 < 32 ? M - m0 : 32), n = (int)N, k = (int)K;
+        const float *xp = x + m0 * K;
+        float *yp = y + m0 * N;
+        int rc = launch_gemv_wide(xp, w, bias, yp, qtype, layout, LOWBIT_DT_F32, m, n, k, (hipStream_t)stream);
+        if (rc > 0) rc = launch_gemv(xp, w, bias, yp, qtype, layout, LOWBIT_DT_F32, m, n, k, 0, (hipStream_t)stream);
+        if (rc) return check_launch(rc, what);
+    }
+    return check_launch(0, what);
 }
 
 size_t lowbit_linear_workspace_bytes(int qtype, int layout, int dtype, int64_t M, int64_t N, int64_t K, size_t max_bytes) {
-    if (dtype == LOWBIT_DT_F32 || M <= 16) return 0;     // one streaming pass per 16 rows
+    if (dtype == LOWBIT_DT_F32 || M <= 16) return 0;     // one pass over the weights, or one per 32 rows
     if (layout != LOWBIT_LAYOUT_GGML) return lowbit_workspace_bytes_for(qtype, layout, M, N, K, max_bytes);
     if (!qk_size(qtype) || N <= 0 || K <= 0 || M > 0x7fffffff || N > 0x7fffffff || K > 0x7fffffff) return 0;
     return gemm_rows_workspace_bytes((int)M, (int)N, (int)K, max_bytes);
@@ -398,7 +420,7 @@ int lowbit_linear(const void *x, const void *w, const void *bias, void *y, int q
                   int64_t N, int64_t K, void *workspace, size_t workspace_bytes, void *stream) {
     if (dtype == LOWBIT_DT_F32)
         return forward_f32("lowbit_linear", (const float *)x, w, (const float *)bias, (float *)y, qtype, layout, M, N, K, stream);
-    return forward_any("lowbit_linear", x, w, bias, y, qtype, layout, dtype, M, N, K, workspace, workspace_bytes, stream);
+    return forward_any("lowbit_linear", x, w, bias, y, qtype, layout, dtype, M, N, K, workspace, workspace_bytes, stream, true);
 }
 
 // ---- lowbit_forward_f32.  The workspace is part of the interface; the kernel keeps x's two planes in LDS and needs none.
@@ -487,13 +509,14 @@ int lowbit_mlp_forward(const void *x, const void *w_gate, const void *w_up, void
     if (M * N == 0) return 0;
     if (K == 0) return fail(LOWBIT_ESHAPE, "lowbit_mlp_forward: K == 0");
     if (!w_up || !aligned16(w_up)) return fail(LOWBIT_EARG, "lowbit_mlp_forward: null or misaligned pointer");
-    // up to 16 rows (decode): one pass of the streaming kernel over both weights.  17 .. 31 rows: two passes while
-    // a weight is small enough for that to beat the GEMM form (measured on MI355X at M = 24: sym_int4 [11008 x 4096],
-    // 25 MB a weight, 32.1 against 36.7 us; fp8_e4m3 [14336 x 4096], 61 MB, 53.6 against 47.3; nf4 [28672 x 8192],
-    // 125 MB, 152 against 104).  More rows: the fused gate/up form of the tiled MFMA GEMM.
-    if (M <= 16 || (M < 32 && lowbit_blob_bytes(qtype, N * K) <= ((size_t)32 << 20)))
-        return check_launch(launch_mlp_gemv(x, w_gate, w_up, y, qtype, act_dtype, (int)M, (int)N, (int)K, act,
-                                            (hipStream_t)stream), "lowbit_mlp_forward");
+    // up to 64 rows (decode, serving batches): one pass over both weights, by the streaming kernel up to 8 rows and the
+    // kernel that gemv_wide.hip describes above that; more rows: the fused gate/up form of the tiled MFMA GEMM
+    if (M <= 64) {
+        int rc = launch_mlp_wide(x, w_gate, w_up, y, qtype, act_dtype, (int)M, (int)N, (int)K, act, (hipStream_t)stream);
+        if (rc > 0 && M <= 8)
+            rc = launch_mlp_gemv(x, w_gate, w_up, y, qtype, act_dtype, (int)M, (int)N, (int)K, act, (hipStream_t)stream);
+        if (rc <= 0) return check_launch(rc, "lowbit_mlp_forward");
+    }
     if (((uintptr_t)y) & 7) return fail(LOWBIT_EARG, "lowbit_mlp_forward: y must be 8-byte aligned");
     return check_launch(launch_mlp_gemm(x, w_gate, w_up, y, qtype, act_dtype, (int)M, (int)N, (int)K, act,
                                         (hipStream_t)stream), "lowbit_mlp_forward");

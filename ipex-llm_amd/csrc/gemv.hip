@@ -22,30 +22,10 @@
 
 namespace lowbit {
 
-// Eight floats -> their bf16 values and those of what the rounding dropped.  inf / nan stay in the first plane only.
-__device__ inline void split_f32(const u32x4 &a, const u32x4 &b, u32x4 &hi, u32x4 &lo) {
-    bf16x8 h, l;
-#pragma unroll
-    for (int i = 0; i < 8; i++) {
-        const float v = __builtin_bit_cast(float, i < 4 ? a[i] : b[i - 4]);
-        h[i] = (__bf16)v;                                   // round to nearest even
-        const float r = v - (float)h[i];                    // exact: both share the leading bits
-        l[i] = (r - r) == 0.0f ? (__bf16)r : (__bf16)0.0f;
-    }
-    hi = __builtin_bit_cast(u32x4, h);
-    lo = __builtin_bit_cast(u32x4, l);
-}
-
 // ------------------------------------------------------------ MFMA GEMV
 
 constexpr int GEMV_MAX_WAVES = 16;
 
-// activation of the gate branch: 0 = SiLU, 1 = GELU in its tanh form (what Gemma uses)
-__device__ inline float gate_act(float g, int act) {
-    if (act == 0) return g / (1.0f + __expf(-g));
-    const float t = tanhf(0.7978845608028654f * (g + 0.044715f * g * g * g));
-    return 0.5f * g * (1.0f + t);
-}
 constexpr int GEMV_LDS_X_BUDGET = 64 * 1024;
 
 struct MoeId {
@@ -405,7 +385,7 @@ static void launch_mfma(const AT *x, const uint8_t *w, const AT *bias, AT *y, in
 }
 
 template <int QT, typename AT, bool F32, bool ROWS>
-static void launch_gemv_t(const void *x, const void *w, const void *bias, void *y, int M, int N, int K, int waves, hipStream_t st) {
+static int launch_gemv_t(const void *x, const void *w, const void *bias, void *y, int M, int N, int K, int waves, hipStream_t st) {
     using ET = typename std::conditional<F32, float, AT>::type;
     const int tile_rows = (N + TILE_ROWS - 1) / TILE_ROWS;
     // tile rows may share x in groups of R when R divides them; a row-major weight's last group may reach past its end
@@ -439,8 +419,7 @@ static void launch_gemv_t(const void *x, const void *w, const void *bias, void *
         else if (mc <= 8 && shares(2) && N >= 8192)
             launch_mfma<QT, AT, 2, 1, 2, false, 0, 2, F32, ROWS>(xp, wp, b, yp, mc, N, K, waves, st);
         else if (mc <= 8) launch_mfma<QT, AT, 2, 1, 2, false, 0, 1, F32, ROWS>(xp, wp, b, yp, mc, N, K, waves, st);
-        // float32: the two planes of x are twice the LDS, so one tile per wave and round here too
-        else if constexpr (F32) launch_mfma<QT, AT, 4, 1, 4, false, 0, 1, F32, ROWS>(xp, wp, b, yp, mc, N, K, waves, st);
+        else if constexpr (F32) return -7;                  // (9 rows and more: gemv_wide.hip)
         // 9 .. 16 rows of x: share x between 4 or 2 tile rows where N still gives enough workgroups
         // (measured on MI355X: +25 .. 70 % on [28672 x 8192], +8 .. 24 % on [8192 x 8192])
         else if (shares(4) && N >= 16384)
@@ -451,16 +430,16 @@ static void launch_gemv_t(const void *x, const void *w, const void *bias, void *
             launch_mfma<QT, AT, 4, 2, 8, false, 0, 2, F32, ROWS>(xp, wp, b, yp, mc, N, K, waves, st);
         else launch_mfma<QT, AT, 4, 2, 8, false, 0, 1, F32, ROWS>(xp, wp, b, yp, mc, N, K, waves, st);
     }
+    return 0;
 }
 
 template <int QT, bool ROWS>
 static int launch_gemv_dt(const void *x, const void *w, const void *bias, void *y, int dt, int M, int N, int K, int waves,
                           hipStream_t st) {
-    if (dt == DT_F16) launch_gemv_t<QT, _Float16, false, ROWS>(x, w, bias, y, M, N, K, waves, st);
-    else if (dt == DT_BF16) launch_gemv_t<QT, __bf16, false, ROWS>(x, w, bias, y, M, N, K, waves, st);
-    else if (dt == DT_F32) launch_gemv_t<QT, __bf16, true, ROWS>(x, w, bias, y, M, N, K, waves, st);
-    else return -4;
-    return 0;
+    if (dt == DT_F16) return launch_gemv_t<QT, _Float16, false, ROWS>(x, w, bias, y, M, N, K, waves, st);
+    if (dt == DT_BF16) return launch_gemv_t<QT, __bf16, false, ROWS>(x, w, bias, y, M, N, K, waves, st);
+    if (dt == DT_F32) return launch_gemv_t<QT, __bf16, true, ROWS>(x, w, bias, y, M, N, K, waves, st);
+    return -4;
 }
 
 template <int QT>
@@ -484,17 +463,14 @@ static int launch_mlp_t(const void *x, const void *wg, const void *wu, void *y, 
     GemvExtra e;
     e.w2 = (const uint8_t *)wu;
     e.act = act;
-    for (int m0 = 0; m0 < M; m0 += 16) {             // one pass over both weights per 16 rows
-        const int mc = (M - m0) < 16 ? (M - m0) : 16;
-        const AT *xp = (const AT *)x + (int64_t)m0 * K;
-        AT *yp = (AT *)y + (int64_t)m0 * N;
-        if (mc <= 2) launch_mfma<QT, AT, 1, 2, 1, true>(xp, g, nullptr, yp, mc, N, K, 8, st, e);
-        else if (mc <= 4) launch_mfma<QT, AT, 1, 2, 2, true>(xp, g, nullptr, yp, mc, N, K, 8, st, e);
-        // 5 .. 16 rows: one tile of each weight per wave and round with up to 16 waves, as the plain product's
-        // kernels that share x between two tile rows
-        else if (mc <= 8) launch_mfma<QT, AT, 2, 1, 2, true>(xp, g, nullptr, yp, mc, N, K, 0, st, e);
-        else launch_mfma<QT, AT, 4, 1, 4, true>(xp, g, nullptr, yp, mc, N, K, 0, st, e);
-    }
+    const AT *xp = (const AT *)x;
+    AT *yp = (AT *)y;
+    if (M <= 2) launch_mfma<QT, AT, 1, 2, 1, true>(xp, g, nullptr, yp, M, N, K, 8, st, e);
+    else if (M <= 4) launch_mfma<QT, AT, 1, 2, 2, true>(xp, g, nullptr, yp, M, N, K, 8, st, e);
+    // 5 .. 8 rows: one tile of each weight per wave and round with up to 16 waves, as the plain product's
+    // kernels that share x between two tile rows
+    else if (M <= 8) launch_mfma<QT, AT, 2, 1, 2, true>(xp, g, nullptr, yp, M, N, K, 0, st, e);
+    else return -7;
     return 0;
 }
 
@@ -506,7 +482,7 @@ static int launch_mlp_q(const void *x, const void *wg, const void *wu, void *y, 
     return -4;
 }
 
-// y[M, N] = act(x Wg^T) * (x Wu^T) in passes of 16 rows, both weights tiled [N, K]
+// y[M, N] = act(x Wg^T) * (x Wu^T) for up to 8 rows, both weights tiled [N, K]
 int launch_mlp_gemv(const void *x, const void *wg, const void *wu, void *y, int qtype, int act_dtype, int M, int N,
                     int K, int act, hipStream_t st) {
     if (M == 0 || N == 0) return 0;

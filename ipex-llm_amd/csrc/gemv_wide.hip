@@ -1,0 +1,106 @@
+// Where the one-pass kernel for up to 64 rows of x (lowbit_gemv_wide.h) is used, and in which shape.
+#include <hip/hip_runtime.h>
+#include "lowbit_formats.h"
+
+namespace lowbit {
+
+struct WideShape {
+    int r, waves;
+};
+template <int QT>
+int launch_wide_q(const void *x, const void *w, const void *bias, void *y, int layout, int dt, int M, int N, int K, const WideShape &s,
+                  hipStream_t st);
+template <int QT>
+int launch_wide_mlp_q(const void *x, const void *wg, const void *wu, void *y, int dt, int M, int N, int K, int act, const WideShape &s,
+                      hipStream_t st);
+
+// The shape for M rows of x, r = 0: another kernel is the faster one.  T tile rows, G column groups, MB 16-row blocks of x;
+// measured on MI355X over some 900 points (format, shape, M, activation type, layout), each launch on weights not just read.
+//
+// R = ceil(T / 256) tile rows a workgroup: one workgroup per CU then covers the weight, and a larger R only makes fewer
+// workgroups read the same x.  8 waves (12 where a wave holds one tile and 16 rows, at the latency of the walk; 4 where
+// R = 4 and several workgroups share a CU).
+// Every workgroup reads all of x from L2, MB * G * 4 KB: beyond about 0.8 MB (MB * G = 192) the ring kernel and the K splits
+// of the tiled GEMM win, which divide x as well ([4096 x 11008] at 64 rows: 24.2 us against 31).  Beyond 1024 tile rows
+// there are several rounds of workgroups and x comes again in each: only 17 .. 32 rows still pay ([28672 x 8192] at 48
+// rows 106 against 96 us of the GEMM).
+static WideShape wide_shape(int qtype, int layout, int dt, int M, int N, int K) {
+    const int T = (N + TILE_ROWS - 1) / TILE_ROWS, G = (K + TILE_COLS - 1) / TILE_COLS, MB = (M + 15) / 16;
+    const int rounds = (T + 255) / 256;
+    const WideShape none = {0, 0};
+    if (dt == DT_F32) {
+        // Two planes of x: 32 rows at most.  One pass at half the x traffic of the streaming kernel's (9 .. 16 rows on
+        // [28672 x 8192]: 86 -> 59 us) or in place of two (24 rows on [11008 x 4096]: 35.0 -> 31.3); up to 8 rows it loses.
+        if (M <= 8 || M > 32) return none;
+        return {rounds > 1 ? 2 : 1, MB == 2 && rounds > 1 ? 4 : 8};
+    }
+    if (M > 64) return none;
+    if (layout == LAYOUT_GGML) {
+        // From 5 rows on: the streaming kernel reads unaligned weights in smaller pieces ([8008 x 8256], sym_int4, 8 rows:
+        // 19.4 -> 15.2 us; 16 rows of [4001 x 2112] 7.1 -> 4.6).  Not fp8_e4m3, whose rows are whole and aligned, and not
+        // beyond 1024 tile rows, up to 16 rows.  17 .. 64 rows: against the row-major GEMM, whose 64-column tiles leave most
+        // CUs idle at that size ([4001 x 2112], 24 / 64 rows: 11.4 -> 5.8 / 14.8 -> 8.6 us).
+        const bool int4 = qtype == QT_SYM_INT4 || qtype == QT_ASYM_INT4;
+        if (MB == 1) {
+            if (M <= 4 || T > 1024 || qtype == QT_FP8_E4M3) return none;
+            if (rounds == 1) return {1, 12};
+            return {rounds == 3 && !int4 ? 1 : rounds, 8};                  // (more registers per tile: a third of them waits)
+        }
+        if (MB * G > 200 || (MB == 4 && T > 512) || (T > 1024 && (MB > 2 || qtype == QT_SYM_INT8))) return none;
+    } else {
+        if (M <= 8 || (MB == 1 && T > 1024) || (MB > 1 && MB * G > 192) || (MB == 4 && T > 768) || (T > 1024 && MB > 2)) return none;
+    }
+    if (T > 1024) return {4, 4};
+    return {rounds, MB == 1 && rounds == 1 ? 12 : 8};
+}
+
+// The fused gate/up form: R of either weight, so at most 2.  Against two launches' worth of streaming passes and the fused
+// form of the tiled GEMM, which has few tiles at these sizes and walks all of K in each (fp16 sym_int4 [11008 x 4096] at 12 /
+// 24 / 48 rows 18.0 -> 14.2 / 31.1 -> 19.9 / 40.9 -> 28.8 us, [4096 x 16384] at 24 rows 127 -> 26).
+static WideShape wide_mlp_shape(int qtype, int M, int N, int K) {
+    const int T = N / TILE_ROWS, MB = (M + 15) / 16, rounds = (T + 255) / 256;
+    const WideShape none = {0, 0};
+    // 5 .. 8 rows: where the streaming kernel spends more on unpacking than on memory
+    if (M <= 8 && !(M > 4 && (qtype == QT_SYM_INT8 || (qtype == QT_NF4 && T >= 512)))) return none;
+    if (M > 64 || (MB > 2 && T > 1024)) return none;
+    // one tile row of either weight where that takes an odd number of rounds, and with 16 rows and the formats of many
+    // registers (two of them spill); 8 waves where a CU has one workgroup, else 4
+    const bool small = qtype == QT_SYM_INT4 || qtype == QT_NF4;
+    const int r = rounds == 1 || rounds == 3 || (MB == 1 && !small) ? 1 : 2;
+    return {r, (T + r - 1) / r <= 256 ? 8 : 4};
+}
+
+bool gemv_wide_applies(int qtype, int layout, int act_dtype, int M, int N, int K) {
+    return wide_shape(qtype, layout, act_dtype, M, N, K).r != 0;
+}
+
+// 1: not a shape for this kernel
+int launch_gemv_wide(const void *x, const void *w, const void *bias, void *y, int qtype, int layout, int act_dtype, int M, int N, int K,
+                     hipStream_t st) {
+    const WideShape s = wide_shape(qtype, layout, act_dtype, M, N, K);
+    if (!s.r) return 1;
+    switch (qtype) {
+    case QT_SYM_INT4: return launch_wide_q<QT_SYM_INT4>(x, w, bias, y, layout, act_dtype, M, N, K, s, st);
+    case QT_ASYM_INT4: return launch_wide_q<QT_ASYM_INT4>(x, w, bias, y, layout, act_dtype, M, N, K, s, st);
+    case QT_SYM_INT8: return launch_wide_q<QT_SYM_INT8>(x, w, bias, y, layout, act_dtype, M, N, K, s, st);
+    case QT_NF4: return launch_wide_q<QT_NF4>(x, w, bias, y, layout, act_dtype, M, N, K, s, st);
+    case QT_FP8_E4M3: return launch_wide_q<QT_FP8_E4M3>(x, w, bias, y, layout, act_dtype, M, N, K, s, st);
+    default: return -2;
+    }
+}
+
+int launch_mlp_wide(const void *x, const void *wg, const void *wu, void *y, int qtype, int act_dtype, int M, int N, int K, int act,
+                    hipStream_t st) {
+    const WideShape s = wide_mlp_shape(qtype, M, N, K);
+    if (!s.r) return 1;
+    switch (qtype) {
+    case QT_SYM_INT4: return launch_wide_mlp_q<QT_SYM_INT4>(x, wg, wu, y, act_dtype, M, N, K, act, s, st);
+    case QT_ASYM_INT4: return launch_wide_mlp_q<QT_ASYM_INT4>(x, wg, wu, y, act_dtype, M, N, K, act, s, st);
+    case QT_SYM_INT8: return launch_wide_mlp_q<QT_SYM_INT8>(x, wg, wu, y, act_dtype, M, N, K, act, s, st);
+    case QT_NF4: return launch_wide_mlp_q<QT_NF4>(x, wg, wu, y, act_dtype, M, N, K, act, s, st);
+    case QT_FP8_E4M3: return launch_wide_mlp_q<QT_FP8_E4M3>(x, wg, wu, y, act_dtype, M, N, K, act, s, st);
+    default: return -2;
+    }
+}
+
+}  // namespace lowbit

@@ -1,0 +1,304 @@
+// One pass over the weights for up to 64 rows of x (serving batches): y[M,N] = x[M,K] * dequant(W)[N,K]^T.
+//
+// A workgroup owns R tile rows (16 weight rows each) for all of K; its waves take the 128-column groups of K in turn.
+// Each wave copies its group of x (16 * MB rows) into a private part of LDS and multiplies it with R weight tiles, whose
+// registers already are the MFMA operand: exact codes, the block scale applied to the fp32 results, as in the streaming
+// kernel for up to 16 rows (gemv.hip).  The loads of a wave's next group go out before the current one is computed - x
+// into the registers that its LDS copy has freed, the weights into a second set - so that a walk of a few groups costs
+// one memory latency and not one per group.  The waves' partial sums meet in LDS: no workspace, no second launch.
+//
+// What bounds it: every workgroup reads all of x from L2 (40 rows of 4096: 327 KB, against 36 KB of sym_int4 weights per
+// tile row), which is why R tile rows share it, and the scale: MB * 4 FMAs per 8 codes and lane next to some nine
+// instructions of unpacking.  Measured against the kernels it takes the place of (ring and its reduction, K splits of the
+// tiled GEMM, two and three passes of the streaming kernel), each launch on weights it has not just read, sym_int4 fp16:
+// [12288 x 4096] at 9 / 24 / 32 / 48 / 64 rows 10.5 -> 8.4 / 15.1 -> 11.2 / 15.7 -> 11.5 / 19.0 -> 15.7 / 20.5 -> 17.9 us,
+// [4096 x 4096] at 24 / 48 rows 10.5 -> 7.3 / 14.6 -> 9.7, [5632 x 2048] at 32 rows 11.6 -> 6.1; over 504 points (seven
+// shapes and more, five formats, 9 .. 64 rows) the best shape of this kernel is 1.26 times faster on average.
+//
+// This header holds the kernel and the launch code of one weight format; gemv_wide_<format>.hip instantiate it,
+// gemv_wide.hip decides where it is used.
+#pragma once
+#include "lowbit_rows.h"
+#include "lowbit_unpack.h"
+
+#include <type_traits>
+
+namespace lowbit {
+
+// F32: x, bias and y are float, x as two bf16 planes (see gemv.hip).  ROWS: row-major weights of any shape
+// (lowbit_rows.h).  DUAL: the fused gate/up projection, act(x Wg^T) * (x Wu^T): R tile rows of either weight.
+constexpr int wide_max_waves(int mb, int tiles, bool f32) { return !f32 && (mb == 1 || (mb == 2 && tiles == 1)) ? 16 : 8; }
+
+template <int QT, typename AT, int MB, int R, bool F32, bool ROWS, bool DUAL>
+__global__ __launch_bounds__(64 * wide_max_waves(MB, DUAL ? 2 * R : R, F32)) void gemv_wide_kernel(
+    const void *__restrict__ x_, const uint8_t *__restrict__ w, const uint8_t *__restrict__ w_up, const void *__restrict__ bias_,
+    void *__restrict__ y_, int M, int N, int K, int act) {
+    using F = Fmt<QT>;
+    using V8 = typename Vec8<AT>::type;
+    using ET = typename std::conditional<F32, float, AT>::type;
+    constexpr float OFFSET = code_offset<QT, AT>();
+    constexpr bool NEED_S = QT == QT_ASYM_INT4 || OFFSET != 0.0f, NF4 = QT == QT_NF4, NF4_LO = NF4 && (F32 || ROWS);
+    constexpr int NT = DUAL ? 2 * R : R;                     // weight tiles per group; DUAL: R of the gate, R of the up weight
+    static_assert(!DUAL || (!F32 && !ROWS), "the fused form takes 16-bit activations and tiled weights");
+    constexpr int PLANE = 16 * MB * 256, XBYTES = PLANE * (F32 ? 2 : 1), XC = 4 * MB;     // bytes of x in LDS; chunks of 8 per lane
+    extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
+    const ET *const x = (const ET *)x_;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, W = blockDim.x >> 6, r = lane & 15, c = lane >> 4;
+    uint8_t *const xs = smem + wave * XBYTES;
+    const int G = ROWS ? (K + TILE_COLS - 1) / TILE_COLS : K / TILE_COLS, blocks = K / F::QK;
+
+    gbytes wr[NT];                                           // ROWS: this lane's weight row; tiled: the tile row
+#pragma unroll
+    for (int wi = 0; wi < NT; wi++) {
+        const int64_t row = (int64_t)blockIdx.x * R + wi % R;
+        if constexpr (ROWS) {
+            const int64_t n = row * TILE_ROWS + r;
+            wr[wi] = (gbytes)w + (n < N ? n : N - 1) * (int64_t)blocks * F::TS;
+        } else {
+            const int64_t last = N / TILE_ROWS - 1;          // (tile rows past N are computed and not stored)
+            wr[wi] = (gbytes)(wi < R ? w : w_up) + (row < last ? row : last) * (int64_t)G * F::TILE_BYTES;
+        }
+    }
+    // x: 16 consecutive lanes load the 16 chunks of a row's group (256 bytes; F32: 512), four rows per instruction
+    const int u = lane & 15, xrow = lane >> 4;
+    auto load = [&](int g, u32x4 (&xv)[F32 ? 2 * XC : XC], auto &t) __attribute__((always_inline)) {
+        const int col = g * TILE_COLS + u * 8;
+        const bool past = ROWS && col >= K;                  // columns past K read as zero
+#pragma unroll
+        for (int i = 0; i < XC; i++) {
+            const int m = i * 4 + xrow;
+            const u32x4 *p = (const u32x4 *)(x + (int64_t)(m < M ? m : M - 1) * K + (past ? K - 8 : col));
+#pragma unroll
+            for (int h = 0; h < (F32 ? 2 : 1); h++) {
+                xv[i * (F32 ? 2 : 1) + h] = p[h];
+                if constexpr (ROWS) xv[i * (F32 ? 2 : 1) + h] = past ? u32x4{0u, 0u, 0u, 0u} : p[h];
+            }
+        }
+#pragma unroll
+        for (int wi = 0; wi < NT; wi++) {
+            if constexpr (ROWS) load_rows<QT>(wr[wi], g, c, blocks, t[wi]);
+            else load_tile<QT, true>(wr[wi] + (int64_t)g * F::TILE_BYTES, lane, r, t[wi]);
+        }
+    };
+    // Unit v (16 bytes) of row m lies at unit v ^ m % 16: the rows are 256 bytes apart, and a step reads one unit of 16 of
+    // them at a time.
+    auto put = [&](const u32x4 (&xv)[F32 ? 2 * XC : XC]) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < XC; i++) {
+            const int m = i * 4 + xrow;
+            auto one = [&](uint8_t *row, const u32x4 &v) __attribute__((always_inline)) {
+                if constexpr (ROWS) store_x_rows<QT>(row, u, v, m & 15);
+                else *(u32x4 *)(row + (u ^ (m & 15)) * 16) = v;
+            };
+            if constexpr (F32) {
+                u32x4 hi, lo;
+                split_f32(xv[2 * i], xv[2 * i + 1], hi, lo);
+                one(xs + m * 256, hi);
+                one(xs + PLANE + m * 256, lo);
+            } else {
+                one(xs + m * 256, xv[i]);
+            }
+        }
+    };
+
+    f32x4 acc[NT][MB];
+#pragma unroll
+    for (int wi = 0; wi < NT; wi++)
+#pragma unroll
+        for (int mb = 0; mb < MB; mb++) acc[wi][mb] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    const f32x4 zero4 = {0.0f, 0.0f, 0.0f, 0.0f};
+    const V8 ones = ones8<AT>();
+    const Nf4Planes planes = NF4 ? nf4_planes<AT, false>() : Nf4Planes{}, planes_lo = NF4_LO ? nf4_planes<AT, true>() : Nf4Planes{};
+    uint32_t magic;
+    if constexpr (__is_same(AT, _Float16)) asm("v_mov_b32 %0, 0x64006400" : "=v"(magic));
+    else asm("v_mov_b32 %0, 0x43004300" : "=v"(magic));
+
+    typename std::conditional<ROWS, RowRegs<QT>, TileRegs<QT>>::type wc[NT], wn[NT];
+    u32x4 xv[F32 ? 2 * XC : XC];
+    const int first = wave < G ? wave : G - 1;
+    load(first, xv, wn);
+    for (int g = wave; g < G; g += W) {
+#pragma unroll
+        for (int wi = 0; wi < NT; wi++) wc[wi] = wn[wi];
+        // the LDS part is private to the wave, whose LDS operations execute in order: a fence for the compiler is enough
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        put(xv);
+        if (g + W < G) load(g + W, xv, wn);
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        uint32_t hb[NT][4];
+        if constexpr (ROWS) {
+#pragma unroll
+            for (int wi = 0; wi < NT; wi++) arrange_rows<QT>(wc[wi], hb[wi]);
+        }
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            V8 b[NT], bl[NT];
+            float d[NT], e[NT];
+#pragma unroll
+            for (int wi = 0; wi < NT; wi++) {
+                const auto &t = wc[wi];
+                if constexpr (NF4) {
+                    b[wi] = Unpack<QT, AT>::run(t.q0[j], &planes, magic);
+                    if constexpr (NF4_LO) bl[wi] = Unpack<QT, AT>::run(t.q0[j], &planes_lo, magic);
+                } else if constexpr (F::BITS == 4) b[wi] = Unpack<QT, AT>::run(t.q0[j], nullptr, magic);
+                else if (j < 2) b[wi] = Unpack8<QT, AT>::run(t.q0[(2 * j) & 3], t.q0[(2 * j + 1) & 3]);
+                else b[wi] = Unpack8<QT, AT>::run(t.q1[(2 * j) & 3], t.q1[(2 * j + 1) & 3]);
+                float mn;
+                if constexpr (ROWS) hdr_to_scale<QT>(hb[wi][j], d[wi], mn);
+                else tile_scale<QT>(wc[wi], j, d[wi], mn);
+                e[wi] = mn - OFFSET * d[wi];
+            }
+#pragma unroll
+            for (int mb = 0; mb < MB; mb++) {
+                const uint8_t *at = xs + (mb * 16 + r) * 256 + (((j * 4 + c) ^ r) * 16);
+                const V8 a = *(const V8 *)at;
+                V8 al;
+                if constexpr (F32) al = *(const V8 *)(at + PLANE);
+                f32x4 s = zero4;
+                if constexpr (NEED_S) {
+                    s = mfma16(a, ones, zero4);
+                    if constexpr (F32) s = mfma16(al, ones, s);
+                }
+#pragma unroll
+                for (int wi = 0; wi < NT; wi++) {
+                    f32x4 p = mfma16(a, b[wi], zero4);
+                    if constexpr (F32) p = mfma16(al, b[wi], p);
+                    if constexpr (NF4_LO) {
+                        p = mfma16(a, bl[wi], p);
+                        if constexpr (F32) p = mfma16(al, bl[wi], p);
+                    }
+#pragma unroll
+                    for (int i = 0; i < 4; i++) {
+                        acc[wi][mb][i] = fmaf(d[wi], p[i], acc[wi][mb][i]);
+                        if constexpr (NEED_S) acc[wi][mb][i] = fmaf(e[wi], s[i], acc[wi][mb][i]);
+                    }
+                }
+            }
+#pragma unroll
+            for (int wi = 0; wi < NT; wi++)                   // one step after the other: the scheduler would gather all reads first
+#pragma unroll
+                for (int mb = 0; mb < MB; mb++) asm volatile("" : "+v"(acc[wi][mb]));
+        }
+    }
+
+    // The waves' sums meet in their parts of LDS; C layout: lane = 16*grp + weight row, register i = row 4*grp + i of x.
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    constexpr int RS = XBYTES / 16;                          // f32x4 per wave's part: at least NT * MB * 64
+    static_assert(NT * MB * 1024 <= XBYTES, "partial sums fit the x part");
+    f32x4 *const red = (f32x4 *)smem;
+#pragma unroll
+    for (int wi = 0; wi < NT; wi++)
+#pragma unroll
+        for (int mb = 0; mb < MB; mb++) red[wave * RS + (wi * MB + mb) * 64 + lane] = acc[wi][mb];
+    __syncthreads();
+    for (int q = wave; q < R * MB; q += W) {
+        const int wi = q / MB, mb = q % MB;
+        f32x4 s = red[q * 64 + lane], up = zero4;
+        for (int v = 1; v < W; v++) s += red[v * RS + q * 64 + lane];
+        if constexpr (DUAL) {
+            for (int v = 0; v < W; v++) up += red[v * RS + (R * MB + q) * 64 + lane];
+        }
+        const int64_t n = ((int64_t)blockIdx.x * R + wi) * TILE_ROWS + r;
+        if (n >= N) continue;
+        const float bv = bias_ ? (float)((const ET *)bias_)[n] : 0.0f;
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const int m = mb * 16 + c * 4 + i;
+            if (m < M) {
+                const float v = DUAL ? gate_act(s[i], act) * up[i] : s[i] + bv;
+                if constexpr (F32) ((float *)y_)[(int64_t)m * N + n] = v;
+                else ((AT *)y_)[(int64_t)m * N + n] = to_at<AT>(v);
+            }
+        }
+    }
+}
+
+struct WideShape {
+    int r, waves;
+};
+
+template <int QT, typename AT, int MB, int R, bool F32, bool ROWS, bool DUAL>
+static int launch_wide_r(const void *x, const void *w, const void *w_up, const void *bias, void *y, int M, int N, int K, int act,
+                         int waves, hipStream_t st) {
+    constexpr int XBYTES = 16 * MB * 256 * (F32 ? 2 : 1), LDS = 128 * 1024, MOST = wide_max_waves(MB, DUAL ? 2 * R : R, F32);
+    auto kern = gemv_wide_kernel<QT, AT, MB, R, F32, ROWS, DUAL>;
+    const int G = (K + TILE_COLS - 1) / TILE_COLS;
+    int wv = LDS / XBYTES;
+    wv = wv > MOST ? MOST : wv;
+    wv = wv > waves ? waves : wv;
+    wv = wv > G ? G : wv;
+    // the default limit of dynamic LDS is 64 KB; raised once per process (thread-safe static), on the one GPU this library drives
+    static const hipError_t raised = hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, LDS);
+    if (raised != hipSuccess) return -6;
+    hipLaunchKernelGGL(kern, dim3((N + TILE_ROWS * R - 1) / (TILE_ROWS * R)), dim3(64 * wv), (size_t)wv * XBYTES, st, x, (const uint8_t *)w,
+                       (const uint8_t *)w_up, bias, y, M, N, K, act);
+    return 0;
+}
+
+// -7: a shape that is not instantiated (the caller, gemv_wide.hip, asks for none)
+template <int QT, typename AT, int MB, bool F32, bool ROWS>
+static int launch_wide_mb(const void *x, const void *w, const void *bias, void *y, int M, int N, int K, const WideShape &s, hipStream_t st) {
+    if (s.r == 1) return launch_wide_r<QT, AT, MB, 1, F32, ROWS, false>(x, w, nullptr, bias, y, M, N, K, 0, s.waves, st);
+    if (s.r == 2) return launch_wide_r<QT, AT, MB, 2, F32, ROWS, false>(x, w, nullptr, bias, y, M, N, K, 0, s.waves, st);
+    if constexpr (!F32) {
+        if (s.r == 3) return launch_wide_r<QT, AT, MB, 3, F32, ROWS, false>(x, w, nullptr, bias, y, M, N, K, 0, s.waves, st);
+        if constexpr (MB < 4)
+            if (s.r == 4) return launch_wide_r<QT, AT, MB, 4, F32, ROWS, false>(x, w, nullptr, bias, y, M, N, K, 0, s.waves, st);
+    }
+    return -7;
+}
+
+template <int QT, typename AT, bool F32, bool ROWS>
+static int launch_wide_t(const void *x, const void *w, const void *bias, void *y, int M, int N, int K, const WideShape &s, hipStream_t st) {
+    if (M <= 16) return launch_wide_mb<QT, AT, 1, F32, ROWS>(x, w, bias, y, M, N, K, s, st);
+    if (M <= 32) return launch_wide_mb<QT, AT, 2, F32, ROWS>(x, w, bias, y, M, N, K, s, st);
+    if constexpr (!F32) {
+        if (M <= 48) return launch_wide_mb<QT, AT, 3, F32, ROWS>(x, w, bias, y, M, N, K, s, st);
+        if (M <= 64) return launch_wide_mb<QT, AT, 4, F32, ROWS>(x, w, bias, y, M, N, K, s, st);
+    }
+    return -7;
+}
+
+template <int QT>
+int launch_wide_q(const void *x, const void *w, const void *bias, void *y, int layout, int dt, int M, int N, int K, const WideShape &s,
+                  hipStream_t st) {
+    const bool rows = layout == LAYOUT_GGML;
+    if (dt == DT_F16) return rows ? launch_wide_t<QT, _Float16, false, true>(x, w, bias, y, M, N, K, s, st)
+                                  : launch_wide_t<QT, _Float16, false, false>(x, w, bias, y, M, N, K, s, st);
+    if (dt == DT_BF16) return rows ? launch_wide_t<QT, __bf16, false, true>(x, w, bias, y, M, N, K, s, st)
+                                   : launch_wide_t<QT, __bf16, false, false>(x, w, bias, y, M, N, K, s, st);
+    if (dt == DT_F32) return rows ? launch_wide_t<QT, __bf16, true, true>(x, w, bias, y, M, N, K, s, st)
+                                  : launch_wide_t<QT, __bf16, true, false>(x, w, bias, y, M, N, K, s, st);
+    return -4;
+}
+
+template <int QT, typename AT, int MB>
+static int launch_wide_mlp_mb(const void *x, const void *wg, const void *wu, void *y, int M, int N, int K, int act, const WideShape &s,
+                              hipStream_t st) {
+    if (s.r == 1) return launch_wide_r<QT, AT, MB, 1, false, false, true>(x, wg, wu, nullptr, y, M, N, K, act, s.waves, st);
+    if (s.r == 2) return launch_wide_r<QT, AT, MB, 2, false, false, true>(x, wg, wu, nullptr, y, M, N, K, act, s.waves, st);
+    return -7;
+}
+
+// y = act(x wg^T) * (x wu^T) for up to 64 rows
+template <int QT, typename AT>
+static int launch_wide_mlp_t(const void *x, const void *wg, const void *wu, void *y, int M, int N, int K, int act, const WideShape &s,
+                             hipStream_t st) {
+    if (M <= 16) return launch_wide_mlp_mb<QT, AT, 1>(x, wg, wu, y, M, N, K, act, s, st);
+    if (M <= 32) return launch_wide_mlp_mb<QT, AT, 2>(x, wg, wu, y, M, N, K, act, s, st);
+    if (M <= 48) return launch_wide_mlp_mb<QT, AT, 3>(x, wg, wu, y, M, N, K, act, s, st);
+    return M <= 64 ? launch_wide_mlp_mb<QT, AT, 4>(x, wg, wu, y, M, N, K, act, s, st) : -7;
+}
+
+template <int QT>
+int launch_wide_mlp_q(const void *x, const void *wg, const void *wu, void *y, int dt, int M, int N, int K, int act, const WideShape &s,
+                      hipStream_t st) {
+    if (dt == DT_F16) return launch_wide_mlp_t<QT, _Float16>(x, wg, wu, y, M, N, K, act, s, st);
+    if (dt == DT_BF16) return launch_wide_mlp_t<QT, __bf16>(x, wg, wu, y, M, N, K, act, s, st);
+    return -4;
+}
+
+}  // namespace lowbit

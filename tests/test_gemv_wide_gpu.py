@@ -1,0 +1,50 @@
+"""The one-pass kernel for up to 64 rows: rows around its 16-row blocks, tile rows around the 1 .. 4 a workgroup owns, fewer
+and more column groups than waves; both layouts, float32 activations, and the fused gate/up form."""
+import numpy as np
+import pytest
+import torch
+
+import lowbit_oracle as orc
+from gpu_util import ALL, FP8, acts, dev_quantize, weights
+from ipex_llm.transformers.low_bit_linear import mlp_forward_xpu
+from ipex_llm.transformers.models.utils import SILU
+from test_linear_gpu import GGML, TILED, _check
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("qtype", ALL)
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("m,n,k", [(9, 16, 128), (16, 48, 3200), (16, 4112, 256), (17, 1040, 1408), (32, 8208, 128), (33, 4144, 256),
+                                   (48, 12304, 128), (49, 272, 1152), (64, 8224, 256), (64, 16, 6144), (18, 16416, 256), (31, 12304, 640)])
+def test_tiled_weights(qtype, dtype, m, n, k):
+    _check(qtype, dtype, TILED, m, n, k, m % 2 == 0, 700 * m + n)
+
+
+@pytest.mark.parametrize("qtype", ALL)
+@pytest.mark.parametrize("m,n,k", [(5, 4099, 192), (8, 17, 1600), (16, 8201, 128), (17, 4101, 320), (48, 8199, 64), (64, 1023, 1216), (32, 16387, 192)])
+def test_row_major_weights(qtype, m, n, k):
+    if qtype == FP8:
+        k = (k + 127) // 128 * 128
+    _check(qtype, torch.bfloat16, GGML, m, n, k, m % 2 == 0, 800 * m + n)
+
+
+@pytest.mark.parametrize("qtype", ALL)
+@pytest.mark.parametrize("layout,m,n,k", [(TILED, 9, 48, 1408), (TILED, 16, 4112, 128), (TILED, 17, 4112, 384), (TILED, 32, 16, 128),
+                                          (TILED, 75, 64, 512), (GGML, 10, 4099, 192), (GGML, 31, 33, 1088)])
+def test_float32_activations(qtype, layout, m, n, k):
+    if qtype == FP8:
+        k = (k + 127) // 128 * 128
+    _check(qtype, torch.float32, layout, m, n, k, m % 2 == 0, 900 * m + n)
+
+
+@pytest.mark.parametrize("qtype", ALL)
+@pytest.mark.parametrize("m,n,k", [(7, 8208, 128), (9, 16, 128), (16, 4144, 1152), (17, 4112, 128), (33, 8208, 128), (48, 4112, 384),
+                                   (49, 4112, 256), (64, 272, 1408), (32, 16400, 128)])
+def test_fused_gate_up(qtype, m, n, k):
+    dtype = torch.float16 if m % 2 else torch.bfloat16
+    wg, wu, x = weights(m + n, (n, k)), weights(m + n + 1, (n, k)), acts(m, m, k, dtype)
+    y = mlp_forward_xpu(x.cuda(), dev_quantize(wg, qtype, TILED), dev_quantize(wu, qtype, TILED), m, k, n, SILU, qtype).float().cpu().numpy()
+    g, u = (orc.mul_mat_exact(orc.quantize(w, qtype), x.float().numpy(), (n, k), qtype) for w in (wg, wu))
+    want = g / (1.0 + np.exp(-g)) * u
+    assert np.abs(y - want).max() <= (2e-3 if dtype == torch.float16 else 8e-3) * np.abs(want).max()

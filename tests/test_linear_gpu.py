@@ -54,6 +54,6 @@ def test_float32_activations_in_one_pass(qtype, m, n, k):
 
 # one shape for every kernel of the choice: streaming, ring (cut and whole tiles), GEMM, its K split, narrow and tall tiles
 @pytest.mark.parametrize("qtype,dtype", [(2, torch.float16), (3, torch.bfloat16), (8, torch.float16), (10, torch.bfloat16), (15, torch.bfloat16)])
-@pytest.mark.parametrize("m,n,k", [(3, 512, 256), (40, 4096, 1024), (300, 272, 2048), (512, 16384, 128), (1030, 2048, 256), (200, 1040, 128)])
+@pytest.mark.parametrize("m,n,k", [(3, 512, 256), (40, 4096, 1024), (50, 2048, 6400), (300, 272, 2048), (512, 16384, 128), (1030, 2048, 256), (200, 1040, 128)])
 def test_bias_of_every_kernel(qtype, dtype, m, n, k):
     _check(qtype, dtype, TILED, m, n, k, True, 500 * m + n)
