@@ -363,7 +363,8 @@ static int forward_any(const char *what, const void *x, const void *w, const voi
     int splits = 1, rc = 0;
     const int plan = linear && gemv_wide_applies(qtype, layout, act_dtype, m, n, k) ? PLAN_GEMV
         : plan_forward(qtype, layout, M, N, K, workspace != nullptr, workspace_bytes, !(((uintptr_t)y | (uintptr_t)bias) & 7), &splits);
-    if (plan == PLAN_GEMV) {
+    // (a y off the 8-byte boundaries keeps the streaming kernel's passes, and so its bits, at the entry points that say so)
+    if (plan == PLAN_GEMV && (linear || !(((uintptr_t)y) & 7))) {
         rc = launch_gemv_wide(x, w, bias, y, qtype, layout, act_dtype, m, n, k, st);
         if (rc <= 0) return check_launch(rc, what);
     }
