@@ -116,22 +116,34 @@ int gemm_splits(int M, int N, int K, size_t ws_bytes, int qtype) {
 
 // How many column tiles (256 weight rows each) the tall form takes, from the left: whole rounds of one
 // 256 x 256 tile per CU, so that no CU sits idle while another still works on a second tall tile; the 128-row
-// form covers the columns that are left.  0 = the tall form is not used: M not a multiple of 256, too few
-// tiles to fill the machine once, K too long for 24-bit row offsets - or columns left over that would not
-// fill the machine themselves.  Measured on MI355X: a machine full of tall tiles runs 4-7 % (sym_int4) to
-// 10 % (nf4) faster than the 128-row form with two workgroups per CU, which the idle CUs of a thin remainder
-// eat up again ([11008 x 4096] at M = 2048: 32 tall columns + 11 left over, no faster than 688 small tiles).
-static int tall_columns(int M, int N, int K, int n_cus, bool heavy_dequant) {
-    if (M < 2 * GM_TALL || M % GM_TALL || M >= (1 << 24) || K >= (1 << 23)) return 0;
-    const int tiles_m = M / GM_TALL, tiles_n = (N + GN - 1) / GN;
-    const int rounds = tiles_m * tiles_n / n_cus;
+// form covers the columns that are left.  0 = the tall form is not used: a last row tile that is less than half full
+// (the 128-row form computes 128 rows less), too few tiles to fill the machine once, K too long for 24-bit row
+// offsets - or columns left over that cost more than the tall columns gain.  Measured on MI355X: a machine full of tall
+// tiles runs 4-7 % (sym_int4) to 10 % (nf4) faster than the 128-row form with two workgroups per CU ([28672 x 8192] at
+// M = 1000, bf16: sym_int4 440 -> 429, asym_int4 442 -> 418, sym_int8 456 -> 423, fp8_e4m3 420 -> 395 us), which the
+// idle CUs of a thin remainder eat up again.
+//   - sym_int8 and nf4 pay most per weight for the dequantization, which the tall form does half as often: the estimate
+//     of gemm_time_us for both ways, 0.9 of a full 128-row round for a tall one; a remainder of at most one workgroup per
+//     CU costs nf4 1.3 in its register-staged form (nf4 [11008 x 4096] at M = 2047: 207 us without tall tiles, 221 with;
+//     [14336 x 4096] at M = 1990 256 and 243; sym_int8 [28672 x 8192] at M = 700 347 and 332; [11008 x 4096] at
+//     M = 1300, 258 tall tiles, one column left over: 116 us without, 151 with).
+//   - the others with 1.5 workgroups per CU left over (at M = 2048 on [11008 x 4096] sym_int4 +1 %, fp8_e4m3 -3 %).
+static double steps_time(int64_t wgs) {                  // a 128-column step of the 128-row form, see gemm_time_us
+    if (wgs > 512) return 2.68 * (double)((wgs + 255) / 256) / 2.0;
+    return wgs > 256 ? 2.12 + 0.56 * (double)(wgs - 256) / 256.0 : 1.21 + (wgs > 128 ? 0.29 * (double)(wgs - 128) / 128.0 : 0.0);
+}
+static int tall_columns(int M, int N, int K, int n_cus, int qtype) {
+    const int rest = M % GM_TALL;
+    if (M < 2 * GM_TALL || (rest && rest <= GM) || M >= (1 << 24) || K >= (1 << 23)) return 0;
+    const int tiles_m = (M + GM_TALL - 1) / GM_TALL, tiles_n = (N + GN - 1) / GN;
+    const int64_t small_m = (M + GM - 1) / GM;           // row tiles of the 128-row form
+    const int rounds = (int)((int64_t)tiles_m * tiles_n / n_cus);
     if (rounds < 1) return 0;
-    int cols = rounds * n_cus / tiles_m;
+    const int cols = (int)((int64_t)rounds * n_cus / tiles_m);
     if (cols >= tiles_n) return tiles_n;
-    const int left = (tiles_n - cols) * (M / GM);        // 128-row tiles of the remainder
-    // sym_int8 and nf4 pay most per weight for the dequantization, which the tall form does half as often: for them
-    // it wins with any remainder ([11008 x 4096] at M = 2048: +11 % and +5 %; sym_int4 +1 %, fp8_e4m3 -3 %)
-    if (heavy_dequant) return cols;
+    const int64_t left = (tiles_n - cols) * small_m;
+    if (qtype == QT_SYM_INT8 || qtype == QT_NF4)
+        return rounds * 0.9 * 2.68 + steps_time(left) * (qtype == QT_NF4 && left <= n_cus ? 1.3 : 1.0) < 0.98 * steps_time(tiles_n * small_m) ? cols : 0;
     return 2 * left >= 3 * n_cus ? cols : 0;
 }
 
@@ -165,9 +177,9 @@ static int launch_gemm_t(const void *x, const void *w, const void *bias, void *y
     // the tall tiles, which all take the same time, are done)
     GroupArgs ga{};
     ga.bias = bias;
-    const int tall = ws ? 0 : tall_columns(M, N, K, n_cus, QT == QT_SYM_INT8 || QT == QT_NF4);
+    const int tall = ws ? 0 : tall_columns(M, N, K, n_cus, QT);
     if (tall > 0) {
-        const int tiles_m = M / GM_TALL;
+        const int tiles_m = (M + GM_TALL - 1) / GM_TALL;
         const unsigned grid = 8 * (unsigned)(((int64_t)tiles_m * tall + 7) / 8);
         // nf4 runs the tall tile with eight waves of 32 columns (two per SIMD cover each other's waits for the code
         // book reads from LDS: 5-9 % faster than four waves of 64 columns); the other formats are 2-4 % faster

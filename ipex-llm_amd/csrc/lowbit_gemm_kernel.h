@@ -381,16 +381,19 @@ __global__ __launch_bounds__(64 * WAVES, (DMA && MB == 4) ? 2 : 1) void gemm_mfm
     // has registers to spare), and the scalar base changes once per K step: a load is three instructions - M0 from
     // the buffer's base plus an immediate, the wait state that M0 needs, the load.  (With the piece's rows added to
     // the scalar base instead it was six, and a load's slot between two MFMAs overran the 28 cycles the MFMA ahead
-    // of it covers.)  Dense launches hand this form whole 256-row tiles only, so no row is clamped.
+    // of it covers.)  Rows past M read its last row.
     const uint32_t xlane_off = (uint32_t)xr_l[0] * (uint32_t)K * (uint32_t)sizeof(AT) + (uint32_t)xc_l[0];       // even pieces
     const uint32_t xlane_off_odd = (uint32_t)xr_l[1] * (uint32_t)K * (uint32_t)sizeof(AT) + (uint32_t)xc_l[1];   // odd pieces
     const uint64_t xwave_base = (uint64_t)(uintptr_t)x +
-        ((uint64_t)(m0 + (GM / (WAVES / 2)) * (wave % (WAVES / 2))) * (uint64_t)K + (uint64_t)(wave / (WAVES / 2)) * 64u) * sizeof(AT);
+        ((uint64_t)m0 * (uint64_t)K + (uint64_t)(wave / (WAVES / 2)) * 64u) * sizeof(AT);
     uint32_t xpiece_off[(MB32 == 8 && !GROUPED) ? PW : 1];
     if constexpr (MB32 == 8 && !GROUPED) {
 #pragma unroll
-        for (int j = 0; j < PW; j++)            // (whole tile below 2^31 bytes from its first row: K < 2^23)
-            xpiece_off[j] = ((j & 1) ? xlane_off_odd : xlane_off) + (uint32_t)j * 8u * (uint32_t)K * (uint32_t)sizeof(AT);
+        for (int j = 0; j < PW; j++) {          // (whole tile below 2^32 bytes from its first row: K < 2^23)
+            int row = (GM / (WAVES / 2)) * (wave % (WAVES / 2)) + 8 * j + xr_l[j & 1];
+            row = m0 + row < M ? row : M - 1 - m0;
+            xpiece_off[j] = (uint32_t)row * (uint32_t)K * (uint32_t)sizeof(AT) + (uint32_t)xc_l[j & 1];
+        }
     }
     auto dma_x_scalar = [&](int kt, uint8_t *buf, const int j) __attribute__((always_inline)) {
         kt = kt0 + (kt < last ? kt : last);
@@ -989,7 +992,7 @@ __global__ __launch_bounds__(64 * WAVES, (DMA && MB == 4) ? 2 : 1) void gemm_mfm
         // tail tiles and small expert groups: 32-row blocks without rows of x skip their MFMAs
         const int mb_cnt = (M - m0 + 31) / 32;
         if constexpr (MB32 == 8 && !GROUPED) {
-            // the dense launcher hands the tall form whole 256-row tiles only
+            // the dense launcher hands the tall form row tiles that are more than half full
             run(full_t());
         } else if constexpr (MB32 == 8) {
             // one variant per count: only the last block of a variant may then hold rows past the group's end,

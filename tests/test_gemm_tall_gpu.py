@@ -1,0 +1,28 @@
+"""The 256-row tile of the GEMM where M is no multiple of its rows: last row tiles of 129 to 255 rows (rows of x past M),
+one, two and three 128-column steps, a last column tile that is not full, columns left to the 128-row form."""
+import pytest
+import torch
+
+from gpu_util import ALL, DT, NAMES, dev_dequantize, dev_quantize, ggml, stream, weights
+
+pytestmark = pytest.mark.gpu
+TILED = ggml.LAYOUT_TILED
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16], ids=["f16", "bf16"])
+@pytest.mark.parametrize("m,n,k", [(897, 16384, 256), (1023, 16368, 384), (1000, 28672, 128), (767, 38160, 256)])
+@pytest.mark.parametrize("qtype", ALL, ids=NAMES.values())
+def test_last_row_tile(qtype, m, n, k, dtype):
+    blob = dev_quantize(weights(77, (n, k)), qtype, TILED)
+    gen = torch.Generator().manual_seed(m)
+    x = torch.randn((m, k), generator=gen).to(dtype).cuda()
+    y = torch.full((m + 1, n), float("nan"), dtype=dtype, device="cuda")
+    ggml.lowbit_gemm(x.data_ptr(), blob.data_ptr(), y.data_ptr(), qtype, TILED, DT[dtype], m, n, k, stream())
+    w = dev_dequantize(blob, qtype, n, k, TILED, torch.float32).to(dtype).float()
+    want, size = x.double() @ w.double().t(), x.abs().float() @ w.abs().t()
+    assert torch.isnan(y[m]).all()
+    # one rounding of the result; fp32 sums over k terms; 16-bit weights rounded once from the same fp32 value, which
+    # asym_int4 (q * d + m) rounds a second time here
+    eps = torch.finfo(dtype).eps
+    bound = want.abs() * eps / 2 + size * (k * 2.0 ** -24 + (eps if qtype == 3 else 0.0)) + torch.finfo(dtype).smallest_normal
+    assert ((y[:m].double() - want).abs() <= bound).all()
