@@ -123,10 +123,9 @@ int gemm_splits(int M, int N, int K, size_t ws_bytes, int qtype) {
 // M = 1000, bf16: sym_int4 440 -> 429, asym_int4 442 -> 418, sym_int8 456 -> 423, fp8_e4m3 420 -> 395 us), which the
 // idle CUs of a thin remainder eat up again.
 //   - sym_int8 and nf4 pay most per weight for the dequantization, which the tall form does half as often: the estimate
-//     of gemm_time_us for both ways, 0.9 of a full 128-row round for a tall one; a remainder of at most one workgroup per
-//     CU costs nf4 1.3 in its register-staged form (nf4 [11008 x 4096] at M = 2047: 207 us without tall tiles, 221 with;
-//     [14336 x 4096] at M = 1990 256 and 243; sym_int8 [28672 x 8192] at M = 700 347 and 332; [11008 x 4096] at
-//     M = 1300, 258 tall tiles, one column left over: 116 us without, 151 with).
+//     of gemm_time_us for both ways, 0.9 of a full 128-row round for a tall one, nf4's remainder, in narrow tiles, 1.15
+//     (sym_int8 [28672 x 8192] at M = 700 347 us without tall tiles and 332 with; nf4 there 404 and 328, [11008 x 4096] at
+//     M = 2047 207 and 171; [11008 x 4096] at M = 1300, 258 tall tiles, one column left over: 116 us without, 151 with).
 //   - the others with 1.5 workgroups per CU left over (at M = 2048 on [11008 x 4096] sym_int4 +1 %, fp8_e4m3 -3 %).
 static double steps_time(int64_t wgs) {                  // a 128-column step of the 128-row form, see gemm_time_us
     if (wgs > 512) return 2.68 * (double)((wgs + 255) / 256) / 2.0;
@@ -143,7 +142,7 @@ static int tall_columns(int M, int N, int K, int n_cus, int qtype) {
     if (cols >= tiles_n) return tiles_n;
     const int64_t left = (tiles_n - cols) * small_m;
     if (qtype == QT_SYM_INT8 || qtype == QT_NF4)
-        return rounds * 0.9 * 2.68 + steps_time(left) * (qtype == QT_NF4 && left <= n_cus ? 1.3 : 1.0) < 0.98 * steps_time(tiles_n * small_m) ? cols : 0;
+        return rounds * 0.9 * 2.68 + steps_time(left) * (qtype == QT_NF4 ? 1.15 : 1.0) < 0.98 * steps_time(tiles_n * small_m) ? cols : 0;
     return 2 * left >= 3 * n_cus ? cols : 0;
 }
 
@@ -181,16 +180,20 @@ static int launch_gemm_t(const void *x, const void *w, const void *bias, void *y
     if (tall > 0) {
         const int tiles_m = (M + GM_TALL - 1) / GM_TALL;
         const unsigned grid = 8 * (unsigned)(((int64_t)tiles_m * tall + 7) / 8);
-        // nf4 runs the tall tile with eight waves of 32 columns (two per SIMD cover each other's waits for the code
-        // book reads from LDS: 5-9 % faster than four waves of 64 columns); the other formats are 2-4 % faster
-        // with four waves, which read each x operand from LDS once per two MFMAs.
-        if constexpr (QT == QT_NF4)
-            hipLaunchKernelGGL((gemm_mfma_kernel<QT, AT, true, MB32_TALL, false, false, 8>), dim3(grid), dim3(512), 0, st,
-                               (const AT *)x, (const uint8_t *)w, (AT *)y, M, N, K, band_rows(tiles_m), ga, G, (float *)nullptr, 0, tall);
-        else
-            hipLaunchKernelGGL((gemm_mfma_kernel<QT, AT, true, MB32_TALL>), dim3(grid), dim3(256), 0, st,
-                               (const AT *)x, (const uint8_t *)w, (AT *)y, M, N, K, band_rows(tiles_m), ga, G, (float *)nullptr, 0, tall);
+        // (four waves, which read each x operand from LDS once per two MFMAs: 2-4 % faster than eight)
+        hipLaunchKernelGGL((gemm_mfma_kernel<QT, AT, true, MB32_TALL>), dim3(grid), dim3(256), 0, st,
+                           (const AT *)x, (const uint8_t *)w, (AT *)y, M, N, K, band_rows(tiles_m), ga, G, (float *)nullptr, 0, tall);
         if (tall == tiles_n_all) return 0;
+        if constexpr (QT == QT_NF4) {
+            // what is left of nf4 in narrow tiles, which look up in registers too (768 of them: [28672 x 8192] at
+            // M = 1000 483 -> 469 us; where at most one 128 x 256 tile per CU is left, which would take the
+            // register-staged form below, [11008 x 4096] at M = 2047 212 -> 171, [28672 x 8192] at M = 700 404 -> 328)
+            const int left = (N + GN / 2 - 1) / (GN / 2) - 2 * tall, tiles_m = (M + GM - 1) / GM;
+            hipLaunchKernelGGL((gemm_mfma_kernel<QT, AT, true, MB32, false, false, 4, true>),
+                               dim3(8 * (unsigned)(((int64_t)tiles_m * left + 7) / 8)), dim3(256), 0, st, (const AT *)x, (const uint8_t *)w,
+                               (AT *)y, M, N, K, band_rows(tiles_m), ga, G, (float *)nullptr, 2 * tall, left);
+            return 0;
+        }
     }
     const int tn0 = tall, tiles_n = tiles_n_all - tall;
     const int tiles_m = (M + GM - 1) / GM;
@@ -227,12 +230,14 @@ bool narrow_halves(int M, int N) {
 
 // Estimated run time in microseconds of the narrow form, fitted like gemm_time_us (760 launches, 8.5 % rms): a
 // 128-column step takes a workgroup 1.05 us up to 128 workgroups, 1.24 at one per CU, 1.55 - 1.96 once two share a
-// CU; half tiles 0.87 of it.
-double narrow_time_us(int M, int N, int K, int qtype) {
+// CU; half tiles 0.87 of it.  nf4 1.06 with its lookups in registers (80 points, 8 shapes: the choice made with it is
+// 1.5 % above the faster of this form and the rest on average; 14 % at worst, [8192 x 8192] at M = 1300);
+// the entry points whose choices lowbit_forward_plan reports keep the figure from before, 1.24.
+double narrow_time_us(int M, int N, int K, int qtype, bool linear) {
     const int tiles_m = (M + GM - 1) / GM;
     const bool halves = narrow_halves(M, N);
     const double wgs = (double)tiles_m * (double)((N + GN / 2 - 1) / (GN / 2)) * (halves ? 2.0 : 1.0);
-    const double format = qtype == QT_NF4 ? 1.24 : qtype == QT_SYM_INT8 ? 1.11 : qtype == QT_FP8_E4M3 ? 1.05 : 1.0;
+    const double format = qtype == QT_NF4 ? (linear ? 1.06 : 1.24) : qtype == QT_SYM_INT8 ? 1.11 : qtype == QT_FP8_E4M3 ? 1.05 : 1.0;
     const double over128 = wgs > 128.0 ? (wgs - 128.0) / 128.0 : 0.0;
     const double step = wgs <= 256.0 ? 1.05 + 0.20 * over128 : 1.55 + 0.41 * ((wgs < 512.0 ? wgs : 512.0) - 256.0) / 256.0;
     const double rounds = wgs > 512.0 ? (double)(((int64_t)wgs + 255) / 256) / 2.0 : 1.0;

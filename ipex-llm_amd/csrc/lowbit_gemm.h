@@ -136,6 +136,60 @@ template <typename AT> struct Dequant<QT_NF4, AT> {
     }
 };
 
+// nf4 without LDS: 64 codes share a scale, 32 of them belong to one lane, so the lane makes the sixteen scaled weights
+// first - the same fp32 product, rounded once to AT, as above - and picks them by code from byte planes in registers,
+// four codes per v_perm_b32 (the scheme of Unpack<QT_NF4>).  3.9 vector instructions per weight against 3.5 and an LDS
+// read, and it is LDS that bounds the tiles with lookups there: a K step of 128 x 128 has 1030 cycles of MFMA per SIMD
+// and some 1800 of LDS (x in, x out, 512 of lookups), one of 256 x 256 4100 and 3600 or, with eight waves that cover the
+// lookups' latency, 5600.  Measured, bf16, in LDS -> in registers: 256 x 256 tiles, [28672 x 8192] at M = 1024 479 -> 462 us;
+// 128 x 128 tiles, [4096 x 4096] at M = 1024 52.0 -> 43.8 us, [2048 x 2048] 22.3 -> 18.5.  (The 128 x 256 tile is held to
+// 128 vector registers for two workgroups per CU and keeps the lookups in LDS.)
+// The work comes in small units that fit between two MFMAs; the planes of the next 64 columns are built along the way.
+template <typename AT> struct Nf4Scaled {
+    uint32_t lo[4], hi[4];          // planes in use: byte i % 4 of register i / 4 = low / high byte of weight i
+    uint32_t nlo[4], nhi[4];        // planes being built
+    uint32_t e01, e23;
+    uint32_t sel, mrg, lo_e, hi_e, lo_o, hi_o;
+
+    // quad q of the planes of scale d, in three parts
+    __device__ void build(uint32_t h, int half, int q, int part) {
+        const float d = h2f(half ? (h >> 16) : (h & 0xffff));
+        if (part == 0) e01 = pk2<AT>(NF4_CODEBOOK[4 * q] * d, NF4_CODEBOOK[4 * q + 1] * d);
+        else if (part == 1) e23 = pk2<AT>(NF4_CODEBOOK[4 * q + 2] * d, NF4_CODEBOOK[4 * q + 3] * d);
+        else {
+            nlo[q] = __builtin_amdgcn_perm(e23, e01, 0x06040200u);
+            nhi[q] = __builtin_amdgcn_perm(e23, e01, 0x07050301u);
+        }
+    }
+    __device__ void take_built() {
+#pragma unroll
+        for (int q = 0; q < 4; q++) { lo[q] = nlo[q]; hi[q] = nhi[q]; }
+    }
+    __device__ uint32_t plane4(const uint32_t (&p)[4]) const {
+        return __builtin_amdgcn_perm(__builtin_amdgcn_perm(p[3], p[2], sel), __builtin_amdgcn_perm(p[1], p[0], sel), mrg);
+    }
+    // unit u (0..7) of a dword v of eight codes: fills the register pairs 0..3 of w.  (nibbles 0, 2, 4, 6 = columns 0, 4,
+    // 1, 5 are the low nibbles of the bytes, nibbles 1, 3, 5, 7 = columns 2, 6, 3, 7 the high ones)
+    __device__ void unit(uint32_t v, int u, u32x4 &w, uint32_t k04, uint32_t k0123) {
+        if (u == 0) {
+            sel = v & 0x07070707u;
+            mrg = and_or(v >> 1, k04, k0123);
+            lo_e = plane4(lo);
+        } else if (u == 1) {
+            hi_e = plane4(hi);
+            w[0] = __builtin_amdgcn_perm(hi_e, lo_e, 0x06020400u);
+        } else if (u == 2) {
+            sel = (v >> 4) & 0x07070707u;
+            mrg = and_or(v >> 5, k04, k0123);
+            lo_o = plane4(lo);
+        } else if (u == 3) {
+            hi_o = plane4(hi);
+            w[1] = __builtin_amdgcn_perm(hi_o, lo_o, 0x06020400u);
+        } else if (u == 4) w[2] = __builtin_amdgcn_perm(hi_e, lo_e, 0x07030501u);
+        else if (u == 6) w[3] = __builtin_amdgcn_perm(hi_o, lo_o, 0x07030501u);
+    }
+};
+
 // ------------------------------------------------------------------ kernel
 
 typedef float f32x16 __attribute__((ext_vector_type(16)));

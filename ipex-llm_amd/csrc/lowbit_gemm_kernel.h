@@ -219,7 +219,9 @@ __global__ __launch_bounds__(64 * WAVES, (DMA && MB == 4) ? 2 : 1) void gemm_mfm
     __shared__ __attribute__((aligned(16))) uint8_t xs[2 * 8 * MB32 * 1024];
     uint8_t *const xs0 = xs, *const xs1 = xs + 8 * MB32 * 1024;
     __shared__ float lut[16];
-    if constexpr (QT == QT_NF4) {
+    // nf4 weights by lookup in registers (Nf4Scaled): the dense tall form and the narrow one, which have the registers
+    constexpr bool NF4REG = QT == QT_NF4 && !GROUPED && ((MB32 == 8 && WAVES == 4) || NARROW);
+    if constexpr (QT == QT_NF4 && !NF4REG) {
         if (threadIdx.x < 16) lut[threadIdx.x] = NF4_CODEBOOK[threadIdx.x];
     }
 
@@ -556,6 +558,31 @@ __global__ __launch_bounds__(64 * WAVES, (DMA && MB == 4) ? 2 : 1) void gemm_mfm
         return Dequant<QT, AT>::pair(t.lo[nb], ks >> 1, p, ctx);
     };
 
+    Nf4Scaled<AT> nf4[NF4REG ? NB32 : 1];
+    uint32_t k04 = 0, k0123 = 0;
+    if constexpr (NF4REG) {
+        asm("v_mov_b32 %0, 0x04040404" : "=v"(k04));
+        asm("v_mov_b32 %0, 0x03020100" : "=v"(k0123));
+    }
+    // unit u of 16-column step ks: 2 units a register pair.  The planes of columns 64 .. 127 are built during the first
+    // four steps, those of columns 0 .. 63 have been built by the caller (nf4_first).
+    auto nf4_unit = [&](const WRegs &t, int ks, int nb, int u, u32x4 &w) __attribute__((always_inline)) {
+        Nf4Scaled<AT> &z = nf4[NF4REG ? nb : 0];
+        if (u == 0 && (ks & 3) == 0) z.take_built();
+        z.unit(((ks & 1) ? t.hi[nb].q0 : t.lo[nb].q0)[ks >> 1], u, w, k04, k0123);
+        if (ks < 4 && u >= 4 && u < 7) z.build(t.lo[nb].h[0], 1, ks, u - 4);
+    };
+    auto nf4_first = [&](const WRegs &t, int nb, int q) __attribute__((always_inline)) {
+#pragma unroll
+        for (int part = 0; part < 3; part++) nf4[NF4REG ? nb : 0].build(t.lo[nb].h[0], 0, q, part);
+    };
+    // the units [slot * n / slots, (slot + 1) * n / slots) of all weight blocks' n = 8 * NB32
+    auto nf4_slot = [&](const WRegs &t, int ks, int slot, int slots, u32x4 (&w)[NB32]) __attribute__((always_inline)) {
+#pragma unroll
+        for (int u = 0; u < 8 * NB32; u++)
+            if (u >= slot * 8 * NB32 / slots && u < (slot + 1) * 8 * NB32 / slots) nf4_unit(t, ks, u >> 3, u & 7, w[u >> 3]);
+    };
+
     // 8 steps of 16 columns, written in the order the hardware should issue them: after the MFMAs
     // of an m-block its x operand for the NEXT step is requested from LDS, and register pairs of
     // the next step's weights are dequantized after every MFMA, so that LDS latency and the VALU
@@ -578,9 +605,17 @@ __global__ __launch_bounds__(64 * WAVES, (DMA && MB == 4) ? 2 : 1) void gemm_mfm
 #pragma unroll
         for (int mb = 0; mb < MBC; mb++) xv[mb] = *(const V8 *)(cur + xlane[0] + x_piece(0, mb));
 #pragma unroll
-        for (int nb = 0; nb < NB32; nb++)
+        for (int nb = 0; nb < NB32; nb++) {
+            if constexpr (NF4REG) {
 #pragma unroll
-            for (int p = 0; p < 4; p++) wv[nb][p] = dequant_pair(t, 0, nb, p);
+                for (int q = 0; q < 4; q++) nf4_first(t, nb, q);
+#pragma unroll
+                for (int u = 0; u < 8; u++) nf4_unit(t, 0, nb, u, wv[nb]);
+            } else {
+#pragma unroll
+                for (int p = 0; p < 4; p++) wv[nb][p] = dequant_pair(t, 0, nb, p);
+            }
+        }
         // From here on every operand of an MFMA is written at least a 16-column step ahead of it - except with a
         // single row block, where the next step's weights are dequantized right behind the MFMA that precedes
         // their use: those variants keep the two wait states ahead of every MFMA, the others spend them once.
@@ -605,8 +640,9 @@ __global__ __launch_bounds__(64 * WAVES, (DMA && MB == 4) ? 2 : 1) void gemm_mfm
                         // MFMA slots, the first slot of a row block served first (the second is followed by the LDS
                         // read and the loads)
                         const int slot_i = mb * NB32 + nb;
+                        if constexpr (NF4REG) nf4_slot(t, ks + 1, slot_i, SPREAD, wn);
 #pragma unroll
-                        for (int idx = 0; idx < PAIRS; idx++) {
+                        for (int idx = 0; idx < (NF4REG ? 0 : PAIRS); idx++) {
                             if (slot_i >= SPREAD || idx < (slot_i * PAIRS + SPREAD - 1) / SPREAD || idx >= ((slot_i + 1) * PAIRS + SPREAD - 1) / SPREAD) continue;
                             wn[idx >> 2][idx & 3] = dequant_pair(t, ks + 1, idx >> 2, idx & 3);   // (weight block, pair)
                         }
@@ -617,7 +653,7 @@ __global__ __launch_bounds__(64 * WAVES, (DMA && MB == 4) ? 2 : 1) void gemm_mfm
                     // them (the second MFMA then waits 32 cycles with nothing to do, and a dozen instructions follow).
                     // (Not for nf4: its dequantization waits for code book reads from LDS, which the scheduler
                     // starts earlier when it is free to.)
-                    if (nb + 1 < NB32 && QT != QT_NF4) __builtin_amdgcn_sched_barrier(0);
+                    if (nb + 1 < NB32 && (QT != QT_NF4 || NF4REG)) __builtin_amdgcn_sched_barrier(0);
                 }
                 if (ks < 7) xv[mb] = *(const V8 *)(cur + xlane[(ks + 1) % 4] + x_piece(ks + 1, mb));
                 // keep this order: the scheduler does not know how long an MFMA takes and would
@@ -650,9 +686,17 @@ __global__ __launch_bounds__(64 * WAVES, (DMA && MB == 4) ? 2 : 1) void gemm_mfm
 #pragma unroll
         for (int mb = 0; mb < MBC; mb++) xv[mb] = *(const V8 *)(cur + xlane[0] + x_piece(0, mb));
 #pragma unroll
-        for (int nb = 0; nb < NB32; nb++)
+        for (int nb = 0; nb < NB32; nb++) {
+            if constexpr (NF4REG) {
 #pragma unroll
-            for (int p = 0; p < 4; p++) wv[nb][p] = dequant_pair(t, 0, nb, p);
+                for (int q = 0; q < 4; q++) nf4_first(t, nb, q);
+#pragma unroll
+                for (int u = 0; u < 8; u++) nf4_unit(t, 0, nb, u, wv[nb]);
+            } else {
+#pragma unroll
+                for (int p = 0; p < 4; p++) wv[nb][p] = dequant_pair(t, 0, nb, p);
+            }
+        }
         asm volatile("s_nop 1" : "+v"(wv[0]));          // VALU write of an MFMA operand: two wait states
         if constexpr (NB32 == 2) asm volatile("" : "+v"(wv[1]));
     };
@@ -679,22 +723,30 @@ __global__ __launch_bounds__(64 * WAVES, (DMA && MB == 4) ? 2 : 1) void gemm_mfm
                     else mfma_acc<WAIT_STATES>(acc[mb][nb], __builtin_bit_cast(V8, wv[nb]), xv[mb]);
                     if (ks < 7) {
                         const int slot_i = mb * NB32 + nb;
+                        if constexpr (NF4REG) nf4_slot(t, ks + 1, slot_i, SPREAD, wn);
 #pragma unroll
-                        for (int idx = 0; idx < PAIRS; idx++) {
+                        for (int idx = 0; idx < (NF4REG ? 0 : PAIRS); idx++) {
                             if (slot_i >= SPREAD || idx < (slot_i * PAIRS + SPREAD - 1) / SPREAD || idx >= ((slot_i + 1) * PAIRS + SPREAD - 1) / SPREAD) continue;
                             wn[idx >> 2][idx & 3] = dequant_pair(t, ks + 1, idx >> 2, idx & 3);
                         }
                     } else if constexpr (HAS_NEXT && TAIL > 0) {
                         if (mb > BMB) {                  // the next step's first weights, over the slots behind the barrier
                             const int ts = (mb - BMB - 1) * NB32 + nb;
+                            if constexpr (NF4REG) {      // the planes first, one quad of one block at a time
+                                constexpr int BUILD = TSPREAD >= 2 ? TSPREAD / 2 : 1, LOOK = TSPREAD >= 2 ? BUILD : 0;
 #pragma unroll
-                            for (int idx = 0; idx < PAIRS; idx++) {
+                                for (int i = 0; i < 4 * NB32; i++)
+                                    if (i >= ts * 4 * NB32 / BUILD && i < (ts + 1) * 4 * NB32 / BUILD) nf4_first(tn, i >> 2, i & 3);
+                                if (ts >= LOOK) nf4_slot(tn, 0, ts - LOOK, TSPREAD - LOOK, wn);
+                            }
+#pragma unroll
+                            for (int idx = 0; idx < (NF4REG ? 0 : PAIRS); idx++) {
                                 if (ts >= TSPREAD || idx < (ts * PAIRS + TSPREAD - 1) / TSPREAD || idx >= ((ts + 1) * PAIRS + TSPREAD - 1) / TSPREAD) continue;
                                 wn[idx >> 2][idx & 3] = dequant_pair(tn, 0, idx >> 2, idx & 3);
                             }
                         }
                     }
-                    if (nb + 1 < NB32 && QT != QT_NF4) __builtin_amdgcn_sched_barrier(0);
+                    if (nb + 1 < NB32 && (QT != QT_NF4 || NF4REG)) __builtin_amdgcn_sched_barrier(0);
                 }
                 if (ks < 7) xv[mb] = *(const V8 *)(cur + xlane[(ks + 1) % 4] + x_piece(ks + 1, mb));
                 else if (HAS_NEXT && mb > BMB) xv[mb] = *(const V8 *)(nxt + xlane[0] + x_piece(0, mb));
@@ -708,7 +760,11 @@ __global__ __launch_bounds__(64 * WAVES, (DMA && MB == 4) ? 2 : 1) void gemm_mfm
                                                          // and nobody reads this one any more
 #pragma unroll
                         for (int m2 = 0; m2 <= BMB; m2++) xv[m2] = *(const V8 *)(nxt + xlane[0] + x_piece(0, m2));
-                        if constexpr (TAIL == 0) {
+                        if constexpr (TAIL == 0 && NF4REG) {
+#pragma unroll
+                            for (int i = 0; i < 4 * NB32; i++) nf4_first(tn, i >> 2, i & 3);
+                            nf4_slot(tn, 0, 0, 1, wn);
+                        } else if constexpr (TAIL == 0) {
 #pragma unroll
                             for (int idx = 0; idx < PAIRS; idx++) wn[idx >> 2][idx & 3] = dequant_pair(tn, 0, idx >> 2, idx & 3);
                         }

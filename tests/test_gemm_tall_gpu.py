@@ -9,15 +9,12 @@ pytestmark = pytest.mark.gpu
 TILED = ggml.LAYOUT_TILED
 
 
-@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16], ids=["f16", "bf16"])
-@pytest.mark.parametrize("m,n,k", [(897, 16384, 256), (1023, 16368, 384), (1000, 28672, 128), (767, 38160, 256)])
-@pytest.mark.parametrize("qtype", ALL, ids=NAMES.values())
-def test_last_row_tile(qtype, m, n, k, dtype):
+def check(qtype, m, n, k, dtype, gemm):
     blob = dev_quantize(weights(77, (n, k)), qtype, TILED)
     gen = torch.Generator().manual_seed(m)
     x = torch.randn((m, k), generator=gen).to(dtype).cuda()
     y = torch.full((m + 1, n), float("nan"), dtype=dtype, device="cuda")
-    ggml.lowbit_gemm(x.data_ptr(), blob.data_ptr(), y.data_ptr(), qtype, TILED, DT[dtype], m, n, k, stream())
+    gemm(x.data_ptr(), blob.data_ptr(), y.data_ptr(), qtype, TILED, DT[dtype], m, n, k, stream())
     w = dev_dequantize(blob, qtype, n, k, TILED, torch.float32).to(dtype).float()
     want, size = x.double() @ w.double().t(), x.abs().float() @ w.abs().t()
     assert torch.isnan(y[m]).all()
@@ -26,3 +23,17 @@ def test_last_row_tile(qtype, m, n, k, dtype):
     eps = torch.finfo(dtype).eps
     bound = want.abs() * eps / 2 + size * (k * 2.0 ** -24 + (eps if qtype == 3 else 0.0)) + torch.finfo(dtype).smallest_normal
     assert ((y[:m].double() - want).abs() <= bound).all()
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16], ids=["f16", "bf16"])
+@pytest.mark.parametrize("m,n,k", [(897, 16384, 256), (1023, 16368, 384), (1000, 28672, 128), (767, 38160, 256)])
+@pytest.mark.parametrize("qtype", ALL, ids=NAMES.values())
+def test_last_row_tile(qtype, m, n, k, dtype):
+    check(qtype, m, n, k, dtype, ggml.lowbit_gemm)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16], ids=["f16", "bf16"])
+@pytest.mark.parametrize("m,n,k", [(1, 16, 128), (32, 144, 256), (33, 128, 384), (64, 272, 640), (65, 1040, 512), (200, 4096, 1152)])
+def test_narrow_nf4(m, n, k, dtype):
+    """Row blocks 1, 2 and 4 of the narrow tile, whose nf4 lookups are in registers."""
+    check(10, m, n, k, dtype, ggml.lowbit_gemm_narrow)
