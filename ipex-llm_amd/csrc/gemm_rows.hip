@@ -16,6 +16,9 @@
 
 namespace lowbit {
 
+int launch_gemv(const void *x, const void *w, const void *bias, void *y, int qtype, int layout, int act_dtype, int M, int N, int K,
+                int waves, hipStream_t st);
+
 constexpr int RG_WAVES = 4, RG_NB = 2, RG_N = RG_WAVES * RG_NB * TILE_ROWS;      // 128 weight rows per workgroup
 
 // MB: 16-row blocks of x per workgroup.  blockIdx.y: the K split, whose partial sums go to ws in register order.
@@ -262,7 +265,8 @@ int launch_gemm_rows(const void *x, const void *w, const void *bias, void *y, in
                      void *workspace, size_t workspace_bytes, hipStream_t st) {
     if (M == 0 || N == 0) return 0;
     const RowsPlan p = rows_plan(M, N, K, workspace ? workspace_bytes : 0);
-    if (K >= (1 << 23)) return -3;                           // 32-bit offsets within a tile of x
+    if (K >= (1 << 23))                                      // 32-bit offsets within a tile of x: the streaming kernel has 64
+        return launch_gemv(x, w, bias, y, qtype, LAYOUT_GGML, act_dtype, M, N, K, 0, st);
     if ((int64_t)((M + 15) / 16) * ((N + RG_N - 1) / RG_N) > 0x7ffffff) return -3;
     float *ws = (float *)workspace;
     switch (qtype) {

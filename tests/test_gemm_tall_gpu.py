@@ -37,3 +37,19 @@ def test_last_row_tile(qtype, m, n, k, dtype):
 def test_narrow_nf4(m, n, k, dtype):
     """Row blocks 1, 2 and 4 of the narrow tile, whose nf4 lookups are in registers."""
     check(10, m, n, k, dtype, ggml.lowbit_gemm_narrow)
+
+
+def test_row_major_weights_of_very_long_rows():
+    """Rows of x beyond 2^24 bytes: past the 32-bit offsets of the batch kernel for row-major weights."""
+    m, n, k = 17, 3, (1 << 23) + 32
+    gen = torch.Generator(device="cuda").manual_seed(5)
+    w = torch.randn((n, k), generator=gen, device="cuda") * 0.02
+    x = torch.randn((m, k), generator=gen, device="cuda").half()
+    blob = torch.empty(ggml.lowbit_blob_bytes(2, n * k), dtype=torch.uint8, device="cuda")
+    ggml.lowbit_quantize(w.data_ptr(), blob.data_ptr(), 2, n, k, ggml.LAYOUT_GGML, stream())
+    y = torch.empty((m, n), dtype=torch.float16, device="cuda")
+    ggml.lowbit_forward(x.data_ptr(), blob.data_ptr(), y.data_ptr(), 2, ggml.LAYOUT_GGML, DT[torch.float16], m, n, k, stream())
+    w = dev_dequantize(blob, 2, n, k, ggml.LAYOUT_GGML, torch.float32).double()
+    want = torch.stack([(x.double() * w[i]).sum(1) for i in range(n)], 1)
+    # one rounding to 16 bits (sums of about 60); fp32 sums of 2^23 terms, whose rounding errors add up like a random walk
+    assert (y.double() - want).abs().max() <= 2.0 ** -11 * want.abs().max() + 0.05
