@@ -142,7 +142,8 @@ template <typename AT> struct Dequant<QT_NF4, AT> {
 // read, and it is LDS that bounds the tiles with lookups there: a K step of 128 x 128 has 1030 cycles of MFMA per SIMD
 // and some 1800 of LDS (x in, x out, 512 of lookups), one of 256 x 256 4100 and 3600 or, with eight waves that cover the
 // lookups' latency, 5600.  Measured, bf16, in LDS -> in registers: 256 x 256 tiles, [28672 x 8192] at M = 1024 479 -> 462 us;
-// 128 x 128 tiles, [4096 x 4096] at M = 1024 52.0 -> 43.8 us, [2048 x 2048] 22.3 -> 18.5.  (The 128 x 256 tile is held to
+// 128 x 128 tiles, [4096 x 4096] at M = 1024 52.0 -> 43.8 us, [2048 x 2048] 22.3 -> 18.5; 512
+// tokens through two of 8 experts of [14336 x 4096] 591 -> 558, 64 of them with [8192 x 4096] 205 -> 184.  (The 128 x 256 tile is held to
 // 128 vector registers for two workgroups per CU and keeps the lookups in LDS.)
 // The work comes in small units that fit between two MFMAs; the planes of the next 64 columns are built along the way.
 template <typename AT> struct Nf4Scaled {

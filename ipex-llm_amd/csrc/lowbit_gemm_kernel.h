@@ -219,8 +219,8 @@ __global__ __launch_bounds__(64 * WAVES, (DMA && MB == 4) ? 2 : 1) void gemm_mfm
     __shared__ __attribute__((aligned(16))) uint8_t xs[2 * 8 * MB32 * 1024];
     uint8_t *const xs0 = xs, *const xs1 = xs + 8 * MB32 * 1024;
     __shared__ float lut[16];
-    // nf4 weights by lookup in registers (Nf4Scaled): the dense tall form and the narrow one, which have the registers
-    constexpr bool NF4REG = QT == QT_NF4 && !GROUPED && ((MB32 == 8 && WAVES == 4) || NARROW);
+    // nf4 weights by lookup in registers (Nf4Scaled): the tall forms and the narrow one, which have the registers
+    constexpr bool NF4REG = QT == QT_NF4 && (MB32 == 8 || NARROW);
     if constexpr (QT == QT_NF4 && !NF4REG) {
         if (threadIdx.x < 16) lut[threadIdx.x] = NF4_CODEBOOK[threadIdx.x];
     }
