@@ -149,12 +149,19 @@ Tensor embedding(const Tensor &ids_in, const Tensor &w, int qtype, int64_t N, in
     return y;
 }
 
-// the experts of a mixture-of-experts block on x [tokens, hidden]; tables: one weight pointer per expert, on x's device
+// a table of n weight pointers in x's device memory
+bool is_table(const Tensor &t, const Tensor &x, int64_t n) {
+    return t.device() == x.device() && t.layout() == at::kStrided && t.scalar_type() == at::kLong && t.numel() == n && t.is_contiguous();
+}
+
+// the experts of a mixture-of-experts block on x [tokens, hidden]; tables: one weight pointer per expert, on x's device.
+// The caller has checked what the pointers lead to: gate, up [inter, hidden] and down [hidden, inter] weights of one qtype.
 Tensor experts(const Tensor &x_in, const Tensor &ids_in, const Tensor &weight_in, const Tensor &gates, const Tensor &ups,
                const Tensor &downs, int qtype, int64_t hidden, int64_t inter, int act) {
     if (!on_gpu(x_in) || x_in.dim() != 2 || x_in.size(1) != hidden || ids_in.dim() != 2 || ids_in.size(0) != x_in.size(0) ||
         ids_in.numel() == 0 || ids_in.scalar_type() != at::kLong || weight_in.sizes() != ids_in.sizes() ||
-        ids_in.device() != x_in.device() || weight_in.device() != x_in.device() || gates.device() != x_in.device()) return {};
+        ids_in.device() != x_in.device() || weight_in.device() != x_in.device() || !is_table(gates, x_in, gates.numel()) ||
+        !is_table(ups, x_in, gates.numel()) || !is_table(downs, x_in, gates.numel())) return {};
     const int dt = dtype_code(x_in.scalar_type()), wdt = dtype_code(weight_in.scalar_type());
     if ((dt != LOWBIT_DT_F16 && dt != LOWBIT_DT_BF16) || wdt < 0) return {};
     const int64_t tokens = ids_in.size(0), top_k = ids_in.size(1), n_exp = gates.numel();

@@ -51,6 +51,7 @@ class ExpertWeights:
         addresses = array.array("Q", [b.data_ptr() for b in self.blobs])
         self.ptrs = torch.tensor(addresses.tolist(), dtype=torch.int64, device=l0.weight.device)
         self.held = (tuple(lin._parameters for lin in linears), addresses.tobytes())      # what `holds` compares
+        self.shape = (self.out_len, self.in_len, len(self.blobs))
 
     def holds(self, device):
         """Whether every layer still has the weight that the pointer table, a snapshot, points to."""
@@ -148,11 +149,40 @@ def moe_ffn_reference(hidden, router_logits, w1, w3, w2, top_k=2):
     return out
 
 
+def _one_format(gates: ExpertWeights, ups: ExpertWeights, downs: ExpertWeights):
+    """Whether one native call takes the three tables (gate and down weights of one format); refuses tables that do not
+    fit together."""
+    inter, hidden, n_exp = gates.shape
+    invalidInputError(ups.qtype == gates.qtype and ups.shape == gates.shape and downs.shape == (hidden, inter, n_exp),
+                      "gate / up / down experts do not fit together")
+    return downs.qtype == gates.qtype
+
+
+def _grouped_steps(hidden, index, weights, gates: ExpertWeights, ups: ExpertWeights, downs: ExpertWeights, act):
+    """The experts' weighted sum as torch operators around the two grouped launches, for what the native call does not
+    take (down weights of another format than the gate's among it).  A pair whose index names no expert counts nothing."""
+    top_k, n_exp = index.shape[1], len(gates.blobs)
+    expert = index.reshape(-1).to(hidden.device, torch.int64)
+    none = (expert < 0) | (expert >= n_exp)
+    expert, order = torch.sort(expert.masked_fill(none, n_exp), stable=True)
+    offsets = torch.searchsorted(expert, torch.arange(n_exp + 1, device=hidden.device), out_int32=True)
+    tok = torch.div(order, top_k, rounding_mode="floor")
+    h = grouped_mlp_forward(hidden[tok], offsets, gates, ups, act)
+    none = none[order].unsqueeze(-1)
+    w = weights.reshape(-1).to(hidden.device)[order].unsqueeze(-1).to(hidden.dtype).masked_fill(none, 0)
+    y = grouped_forward(h, offsets, downs).masked_fill(none, 0) * w
+    out = torch.zeros_like(hidden)
+    out.index_add_(0, tok, y)
+    return out
+
+
 def moe_ffn_grouped(hidden, router_logits, g1: ExpertWeights, g3: ExpertWeights, g2: ExpertWeights, top_k=2):
     """Same result in one call of the experts block (csrc/moe.hip)."""
     weights, experts = route_top_k(router_logits, top_k)
     for table in (g1, g3, g2):
         table.check(hidden.device)
+    if not _one_format(g1, g3, g2):
+        return _grouped_steps(hidden, experts, weights, g1, g3, g2, 0)
     out = ops.experts(hidden, experts, weights, g1.ptrs, g3.ptrs, g2.ptrs, g1.qtype, g1.in_len, g1.out_len, 0)
     invalidInputError(out is not None, "hidden must be [tokens, K] in fp16 / bf16 on the GPU of the experts")
     return out
@@ -244,8 +274,12 @@ class LowBitExperts(nn.Module):
         if tables is None:
             return self._loop(hidden_states, top_k_index, top_k_weights)
         g1, g3, g2 = tables
-        y = ops.experts(hidden_states, top_k_index, top_k_weights, g1.ptrs, g3.ptrs, g2.ptrs, self.qtype, self.hidden_dim,
-                        self.intermediate_dim, activation_code(self.act_fn))
+        act = activation_code(self.act_fn)
+        if not _one_format(g1, g3, g2):
+            if top_k_index.shape[0] == 1:                # (refuses mixed formats)
+                return moe_forward_vec(hidden_states, top_k_index, top_k_weights, g1, g3, g2, act)
+            return _grouped_steps(hidden_states, top_k_index, top_k_weights, g1, g3, g2, act)
+        y = ops.experts(hidden_states, top_k_index, top_k_weights, g1.ptrs, g3.ptrs, g2.ptrs, g1.qtype, g1.in_len, g1.out_len, act)
         return self._loop(hidden_states, top_k_index, top_k_weights) if y is None else y
 
     def _loop(self, hidden_states, top_k_index, top_k_weights):

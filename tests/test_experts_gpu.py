@@ -4,19 +4,37 @@ import torch
 from torch import nn
 
 from ipex_llm.ggml.quantize import ggml_tensor_qtype as Q
-from ipex_llm.transformers.low_bit_linear import FP4Params
-from ipex_llm.transformers.moe import LowBitExperts
+from ipex_llm.transformers.low_bit_linear import FP4Params, LowBitLinear
+from ipex_llm.transformers.native_ops import ops
+from ipex_llm.transformers.moe import ExpertWeights, LowBitExperts, moe_ffn_grouped, route_top_k
 
 pytestmark = pytest.mark.gpu
+
+
+def _layers(n_exp, n, k, qtype):
+    with torch.device("meta"):
+        layers = nn.ModuleList([LowBitLinear(k, n, qtype, bias=False) for _ in range(n_exp)])
+    for layer in layers:
+        layer._parameters["weight"] = FP4Params(torch.randn(n, k, device="cuda") * 0.05, qtype=qtype).to("cuda")
+    return layers.eval()
 
 
 def _block(n_exp, hidden, inter, qtype):
     with torch.device("meta"):
         block = LowBitExperts(n_exp, hidden, inter, qtype, nn.SiLU())
-    for layers, n, k in ((block.gate, inter, hidden), (block.up, inter, hidden), (block.down, hidden, inter)):
-        for layer in layers:
-            layer._parameters["weight"] = FP4Params(torch.randn(n, k, device="cuda") * 0.05, qtype=qtype).to("cuda")
+    block.gate, block.up = _layers(n_exp, inter, hidden, qtype), _layers(n_exp, inter, hidden, qtype)
+    block.down = _layers(n_exp, hidden, inter, qtype)
     return block.eval()
+
+
+def _tables(block):
+    return [ExpertWeights(list(layers)) for layers in (block.gate, block.up, block.down)]
+
+
+def _close(got, want):
+    """Within what fp16 sums in another order and one rounding more or less differ by."""
+    assert got.dtype == want.dtype and got.shape == want.shape
+    assert (got.float() - want.float()).abs().max() <= 4e-3 * want.float().abs().max()
 
 
 # pairs around a wave, a workgroup and several rounds of the sort; experts around a wave, beyond it, and beyond 512
@@ -55,3 +73,40 @@ def test_experts_follow_a_weight_that_was_replaced():
     block.down[2]._parameters["weight"] = FP4Params(torch.randn(128, 256, device="cuda") * 0.05, qtype=Q["sym_int4"]).to("cuda")
     got, want = block(x, index, weight), block._loop(x, index, weight)
     assert (got.float() - want.float()).abs().max() <= 4e-3 * want.float().abs().max()
+
+
+@pytest.mark.parametrize("qname,down", [("sym_int4", "sym_int8"), ("sym_int8", "sym_int4"), ("fp8_e4m3", "nf4")])
+def test_down_weights_of_another_format(qname, down):
+    torch.manual_seed(6)
+    block = _block(4, 128, 256, Q[qname])
+    block.down = _layers(4, 128, 256, Q[down])
+    x, logits = torch.randn(9, 128, device="cuda").half(), torch.randn(9, 4, device="cuda")
+    weight, index = route_top_k(logits)
+    want = block._loop(x, index, weight)
+    _close(block(x, index, weight), want)
+    _close(moe_ffn_grouped(x, logits, *_tables(block)), want)
+    index[2, 0], weight[2, 0] = 4, float("nan")                                   # a pair without an expert counts nothing
+    got = block(x, index, weight)
+    weight[2, 0], index[2, 0] = 0, 0
+    _close(got, block._loop(x, index, weight))
+    with pytest.raises(RuntimeError, match="fit together"):
+        block(x[:1], index[:1], weight[:1])
+
+
+@pytest.mark.parametrize("table,n_exp,n,k", [(1, 4, 384, 128), (1, 4, 256, 256), (1, 3, 256, 128), (2, 4, 128, 128), (2, 4, 256, 256),
+                                             (2, 3, 128, 256)])
+def test_tables_that_do_not_fit_together_are_refused(table, n_exp, n, k):
+    block = _block(4, 128, 256, Q["sym_int4"])
+    tables = _tables(block)
+    tables[table] = ExpertWeights(list(_layers(n_exp, n, k, Q["sym_int4"])))
+    x, logits = torch.randn(9, 128, device="cuda").half(), torch.randn(9, 4, device="cuda")
+    with pytest.raises(RuntimeError, match="fit together"):
+        moe_ffn_grouped(x, logits, *tables)
+    block.__dict__["_tables"] = tuple(tables)                                     # as after layers were replaced
+    weight, index = route_top_k(logits)
+    for tokens in (1, 9):
+        with pytest.raises(RuntimeError, match="fit together"):
+            block(x[:tokens], index[:tokens], weight[:tokens])
+    g, u, d = (t.ptrs for t in _tables(block))
+    bad = (g, u[:3], d) if table == 1 else (g, u, d.cpu())
+    assert ops.experts(x, index, weight, *bad, Q["sym_int4"], 128, 256, 0) is None
