@@ -159,7 +159,7 @@ bool is_table(const Tensor &t, const Tensor &x, int64_t n) {
 Tensor experts(const Tensor &x_in, const Tensor &ids_in, const Tensor &weight_in, const Tensor &gates, const Tensor &ups,
                const Tensor &downs, int qtype, int64_t hidden, int64_t inter, int act) {
     if (!on_gpu(x_in) || x_in.dim() != 2 || x_in.size(1) != hidden || ids_in.dim() != 2 || ids_in.size(0) != x_in.size(0) ||
-        ids_in.numel() == 0 || ids_in.scalar_type() != at::kLong || weight_in.sizes() != ids_in.sizes() ||
+        ids_in.numel() == 0 || !at::isIntegralType(ids_in.scalar_type(), /*includeBool=*/false) || weight_in.sizes() != ids_in.sizes() ||
         ids_in.device() != x_in.device() || weight_in.device() != x_in.device() || !is_table(gates, x_in, gates.numel()) ||
         !is_table(ups, x_in, gates.numel()) || !is_table(downs, x_in, gates.numel())) return {};
     const int dt = dtype_code(x_in.scalar_type()), wdt = dtype_code(weight_in.scalar_type());
@@ -167,7 +167,7 @@ Tensor experts(const Tensor &x_in, const Tensor &ids_in, const Tensor &weight_in
     const int64_t tokens = ids_in.size(0), top_k = ids_in.size(1), n_exp = gates.numel();
     const size_t bytes = top_k > 64 || n_exp > 4096 ? 0 : api.experts_workspace_bytes(tokens, (int)top_k, (int)n_exp, hidden, inter);
     if (!bytes) return {};                               // more than the library takes
-    const Tensor x = x_in.contiguous(), ids = ids_in.contiguous(), weight = weight_in.contiguous();
+    const Tensor x = x_in.contiguous(), ids = ids_in.to(at::kLong).contiguous(), weight = weight_in.contiguous();
     c10::DeviceGuard guard(x.device());
     const Tensor ws = at::empty({(int64_t)bytes}, x.options().dtype(at::kByte));
     Tensor y = at::empty({tokens, hidden}, x.options());

@@ -110,3 +110,24 @@ def test_tables_that_do_not_fit_together_are_refused(table, n_exp, n, k):
     g, u, d = (t.ptrs for t in _tables(block))
     bad = (g, u[:3], d) if table == 1 else (g, u, d.cpu())
     assert ops.experts(x, index, weight, *bad, Q["sym_int4"], 128, 256, 0) is None
+
+
+@pytest.mark.parametrize("tokens", [1, 3, 9])
+def test_indices_of_other_integer_types_take_the_same_call(tokens):
+    torch.manual_seed(tokens)
+    block = _block(4, 128, 256, Q["sym_int4"])
+    x, index = torch.randn(tokens, 128, device="cuda").half(), torch.randint(0, 4, (tokens, 2), device="cuda")
+    weight = torch.rand(tokens, 2, device="cuda").half()
+    want = block(x, index, weight)
+    for dtype in (torch.int32, torch.int16, torch.uint8):
+        assert torch.equal(block(x, index.to(dtype), weight), want)
+    index32, graph = index.int(), torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):                                                 # nothing in it waits for the host
+        got = block(x, index32, weight)
+    for _ in range(3):
+        got.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(got, want)
+        x.neg_()
+        want = block(x, index, weight)
