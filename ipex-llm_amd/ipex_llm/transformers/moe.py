@@ -122,8 +122,9 @@ def moe_forward_vec(x: torch.Tensor, topk_ids: torch.Tensor, topk_weight: torch.
     for table in (gates, ups, downs):
         table.check(x.device)
     top_k = topk_ids.numel()
-    ids = topk_ids.reshape(-1).to(torch.int32)
-    rw = topk_weight.reshape(-1).to(torch.float32)
+    invalidInputError(topk_weight.numel() >= top_k, "every expert id needs a weight")
+    ids = topk_ids.reshape(-1).to(x.device, torch.int32)
+    rw = topk_weight.reshape(-1).to(x.device, torch.float32)
     xc = x.contiguous()
     work = torch.empty((top_k, inter), dtype=x.dtype, device=x.device)
     y = torch.empty((1, hidden), dtype=x.dtype, device=x.device)
@@ -149,19 +150,24 @@ def moe_ffn_reference(hidden, router_logits, w1, w3, w2, top_k=2):
     return out
 
 
-def _one_format(gates: ExpertWeights, ups: ExpertWeights, downs: ExpertWeights):
-    """Whether one native call takes the three tables (gate and down weights of one format); refuses tables that do not
-    fit together."""
-    inter, hidden, n_exp = gates.shape
-    invalidInputError(ups.qtype == gates.qtype and ups.shape == gates.shape and downs.shape == (hidden, inter, n_exp),
+def _native(hidden, index, weights, gates: ExpertWeights, ups: ExpertWeights, downs: ExpertWeights, act):
+    """The block in one native call (csrc/moe.hip), None for what that does not take; refuses tables that do not fit
+    together."""
+    inter, width, n_exp = gates.shape
+    invalidInputError(ups.qtype == gates.qtype and ups.shape == gates.shape and downs.shape == (width, inter, n_exp),
                       "gate / up / down experts do not fit together")
-    return downs.qtype == gates.qtype
+    if downs.qtype != gates.qtype:                       # the call decodes all three in one format
+        return None
+    return ops.experts(hidden, index, weights, gates.ptrs, ups.ptrs, downs.ptrs, gates.qtype, width, inter, act)
 
 
 def _grouped_steps(hidden, index, weights, gates: ExpertWeights, ups: ExpertWeights, downs: ExpertWeights, act):
     """The experts' weighted sum as torch operators around the two grouped launches, for what the native call does not
-    take (down weights of another format than the gate's among it).  A pair whose index names no expert counts nothing."""
+    take: down weights of another format than the gate's, no tokens, more than 64 experts per token or 4096 in all,
+    indices or weights on another device.  A pair whose index names no expert counts nothing."""
     top_k, n_exp = index.shape[1], len(gates.blobs)
+    invalidInputError(index.shape[0] <= hidden.shape[0] and weights.numel() == index.numel(),
+                      "every row of the indices needs a row of hidden, every index a weight")
     expert = index.reshape(-1).to(hidden.device, torch.int64)
     none = (expert < 0) | (expert >= n_exp)
     expert, order = torch.sort(expert.masked_fill(none, n_exp), stable=True)
@@ -181,11 +187,8 @@ def moe_ffn_grouped(hidden, router_logits, g1: ExpertWeights, g3: ExpertWeights,
     weights, experts = route_top_k(router_logits, top_k)
     for table in (g1, g3, g2):
         table.check(hidden.device)
-    if not _one_format(g1, g3, g2):
-        return _grouped_steps(hidden, experts, weights, g1, g3, g2, 0)
-    out = ops.experts(hidden, experts, weights, g1.ptrs, g3.ptrs, g2.ptrs, g1.qtype, g1.in_len, g1.out_len, 0)
-    invalidInputError(out is not None, "hidden must be [tokens, K] in fp16 / bf16 on the GPU of the experts")
-    return out
+    out = _native(hidden, experts, weights, g1, g3, g2, 0)
+    return _grouped_steps(hidden, experts, weights, g1, g3, g2, 0) if out is None else out
 
 
 def activation_code(act_fn):
@@ -273,14 +276,11 @@ class LowBitExperts(nn.Module):
         tables = self._expert_tables(hidden_states)
         if tables is None:
             return self._loop(hidden_states, top_k_index, top_k_weights)
-        g1, g3, g2 = tables
         act = activation_code(self.act_fn)
-        if not _one_format(g1, g3, g2):
-            if top_k_index.shape[0] == 1:                # (refuses mixed formats)
-                return moe_forward_vec(hidden_states, top_k_index, top_k_weights, g1, g3, g2, act)
-            return _grouped_steps(hidden_states, top_k_index, top_k_weights, g1, g3, g2, act)
-        y = ops.experts(hidden_states, top_k_index, top_k_weights, g1.ptrs, g3.ptrs, g2.ptrs, g1.qtype, g1.in_len, g1.out_len, act)
-        return self._loop(hidden_states, top_k_index, top_k_weights) if y is None else y
+        y = _native(hidden_states, top_k_index, top_k_weights, *tables, act)
+        if y is None and top_k_index.shape[0] == 1 and top_k_index.shape[1] <= 64:
+            return moe_forward_vec(hidden_states, top_k_index, top_k_weights, *tables, act)
+        return _grouped_steps(hidden_states, top_k_index, top_k_weights, *tables, act) if y is None else y
 
     def _loop(self, hidden_states, top_k_index, top_k_weights):
         out = torch.zeros_like(hidden_states)

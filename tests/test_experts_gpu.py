@@ -6,7 +6,7 @@ from torch import nn
 from ipex_llm.ggml.quantize import ggml_tensor_qtype as Q
 from ipex_llm.transformers.low_bit_linear import FP4Params, LowBitLinear
 from ipex_llm.transformers.native_ops import ops
-from ipex_llm.transformers.moe import ExpertWeights, LowBitExperts, moe_ffn_grouped, route_top_k
+from ipex_llm.transformers.moe import ExpertWeights, LowBitExperts, moe_ffn_grouped, moe_ffn_reference, route_top_k
 
 pytestmark = pytest.mark.gpu
 
@@ -131,3 +131,27 @@ def test_indices_of_other_integer_types_take_the_same_call(tokens):
         assert torch.equal(got, want)
         x.neg_()
         want = block(x, index, weight)
+
+
+def test_calls_beyond_the_native_one():
+    torch.manual_seed(7)
+    block = _block(70, 128, 128, Q["sym_int4"])
+    tables = _tables(block)
+    x, logits = torch.randn(5, 128, device="cuda").half(), torch.randn(5, 70, device="cuda")
+    assert moe_ffn_grouped(x[:0], logits[:0], *tables).shape == (0, 128)
+    for top_k in (64, 66):                                                        # at most 64 in the native call
+        weight, index = route_top_k(logits, top_k)
+        want = block._loop(x, index, weight)
+        _close(moe_ffn_grouped(x, logits, *tables, top_k=top_k), want)
+        for tokens in (1, 5):
+            _close(block(x[:tokens], index[:tokens], weight[:tokens]), want[:tokens])
+    weight, index = route_top_k(logits)
+    for tokens in (1, 5):                                                         # routing that stayed on the host
+        want = block(x[:tokens], index[:tokens], weight[:tokens])
+        _close(block(x[:tokens], index[:tokens].cpu(), weight[:tokens].cpu()), want)
+    with pytest.raises(RuntimeError):
+        block(x, index, weight[:4])
+    # more experts than the native call sorts: the same layers again and again
+    g, u, d = ([layers[e % 70] for e in range(4100)] for layers in (block.gate, block.up, block.down))
+    logits = torch.randn(5, 4100, device="cuda")
+    _close(moe_ffn_grouped(x, logits, ExpertWeights(g), ExpertWeights(u), ExpertWeights(d)), moe_ffn_reference(x, logits, g, u, d))
