@@ -62,6 +62,11 @@ void *current_stream(const Tensor &t) { return (void *)c10::hip::getCurrentHIPSt
 // a tensor of this module's calls: strided, on the GPU
 bool on_gpu(const Tensor &t) { return t.device().is_cuda() && t.layout() == at::kStrided; }
 
+// whether the result has to carry a derivative with respect to t, which no call of this module gives it
+bool differentiable(const Tensor &t) {
+    return (t.requires_grad() && c10::GradMode::is_enabled()) || t._fw_grad(/*level=*/0).defined();
+}
+
 // w holds the packed [N, K] weight of this format on x's device
 bool is_blob(const Tensor &w, const Tensor &x, int qtype, int64_t N, int64_t K) {
     if (w.device() != x.device() || w.layout() != at::kStrided || !w.is_contiguous()) return false;
@@ -107,7 +112,7 @@ Tensor linear(const Tensor &x_in, const Tensor &w, const Tensor &bias, int qtype
     const int64_t K = x_in.size(-1), M = x_in.numel() / K;
     if (!is_blob(w, x_in, qtype, N, K)) return {};
     if (bias.defined() && (bias.scalar_type() != x_in.scalar_type() || bias.device() != x_in.device() || bias.numel() != N || !bias.is_contiguous() ||
-                           (bias.requires_grad() && c10::GradMode::is_enabled()))) return {};
+                           differentiable(bias))) return {};
     const Tensor x = x_in.is_contiguous() ? x_in : x_in.contiguous();
     const int layout = device_layout(qtype, N, K);
     const auto shape = with_last(x, N);
@@ -161,7 +166,7 @@ Tensor experts(const Tensor &x_in, const Tensor &ids_in, const Tensor &weight_in
     if (!on_gpu(x_in) || x_in.dim() != 2 || x_in.size(1) != hidden || ids_in.dim() != 2 || ids_in.size(0) != x_in.size(0) ||
         ids_in.numel() == 0 || !at::isIntegralType(ids_in.scalar_type(), /*includeBool=*/false) || weight_in.sizes() != ids_in.sizes() ||
         ids_in.device() != x_in.device() || weight_in.device() != x_in.device() || !is_table(gates, x_in, gates.numel()) ||
-        !is_table(ups, x_in, gates.numel()) || !is_table(downs, x_in, gates.numel())) return {};
+        !is_table(ups, x_in, gates.numel()) || !is_table(downs, x_in, gates.numel()) || differentiable(weight_in)) return {};
     const int dt = dtype_code(x_in.scalar_type()), wdt = dtype_code(weight_in.scalar_type());
     if ((dt != LOWBIT_DT_F16 && dt != LOWBIT_DT_BF16) || wdt < 0) return {};
     const int64_t tokens = ids_in.size(0), top_k = ids_in.size(1), n_exp = gates.numel();

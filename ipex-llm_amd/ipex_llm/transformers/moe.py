@@ -163,8 +163,8 @@ def _native(hidden, index, weights, gates: ExpertWeights, ups: ExpertWeights, do
 
 def _grouped_steps(hidden, index, weights, gates: ExpertWeights, ups: ExpertWeights, downs: ExpertWeights, act):
     """The experts' weighted sum as torch operators around the two grouped launches, for what the native call does not
-    take: down weights of another format than the gate's, no tokens, more than 64 experts per token or 4096 in all,
-    indices or weights on another device.  A pair whose index names no expert counts nothing."""
+    take: routing weights that want a gradient, down weights of another format than the gate's, no tokens, more than 64
+    experts per token or 4096 in all, indices or weights on another device.  A pair whose index names no expert counts nothing."""
     top_k, n_exp = index.shape[1], len(gates.blobs)
     invalidInputError(index.shape[0] <= hidden.shape[0] and weights.numel() == index.numel(),
                       "every row of the indices needs a row of hidden, every index a weight")

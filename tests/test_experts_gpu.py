@@ -155,3 +155,26 @@ def test_calls_beyond_the_native_one():
     g, u, d = ([layers[e % 70] for e in range(4100)] for layers in (block.gate, block.up, block.down))
     logits = torch.randn(5, 4100, device="cuda")
     _close(moe_ffn_grouped(x, logits, ExpertWeights(g), ExpertWeights(u), ExpertWeights(d)), moe_ffn_reference(x, logits, g, u, d))
+
+
+def test_routing_weights_get_their_gradient():
+    torch.manual_seed(8)
+    block = _block(4, 128, 256, Q["sym_int4"])
+    x, logits = torch.randn(9, 128, device="cuda").half(), torch.randn(9, 4, device="cuda").requires_grad_(True)
+    weight, index = route_top_k(logits)
+    index[2, 0] = 4                                                               # a pair without an expert
+    weight = weight.detach().requires_grad_(True)
+    y = block(x, index, weight)
+    with torch.no_grad():
+        one = [block(x, index, torch.nn.functional.one_hot(torch.full((9,), j, device="cuda"), 2).half()) for j in range(2)]
+    _close(y.detach(), block(x, index, weight.detach()))
+    (grad,) = torch.autograd.grad(y.float().sum(), weight)
+    want = torch.stack([t.float().sum(-1) for t in one], -1)
+    assert grad[2, 0] == 0 and (grad - want).abs().max() <= 4e-3 * want.abs().max()
+    (grad,) = torch.autograd.grad(moe_ffn_grouped(x, logits, *_tables(block)).float().pow(2).sum(), logits)
+    assert torch.isfinite(grad).all() and grad.abs().max() > 0
+    with torch.no_grad():
+        assert not block(x, index, weight).requires_grad
+    with torch.autograd.forward_ad.dual_level():
+        dual = torch.autograd.forward_ad.make_dual(weight.detach(), torch.ones_like(weight))
+        assert torch.autograd.forward_ad.unpack_dual(block(x, index, dual)).tangent is not None
