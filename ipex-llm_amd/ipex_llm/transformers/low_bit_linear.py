@@ -142,6 +142,8 @@ def _pack(tensor, qtype, device=None, convert_shape_only=False, imatrix=None, en
         _require_gpu("ggml_convert_qtype")
     src = _to_gpu(tensor.detach()) if on_host else tensor
     src = (src if src.dtype in _DT else src.float()).contiguous()
+    if src.data_ptr() % 16:                              # a view into a flat buffer: the kernel loads 16 bytes at a time
+        src = src.clone()
     dst = _blob_like(dst_size, qtype, src.device)
     if n:
         with torch.cuda.device(src.device):

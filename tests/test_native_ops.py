@@ -55,3 +55,14 @@ def test_half_precision_sources_quantize_as_their_float32_values(qname, dtype, n
     for src in (w, w.t().contiguous().t()):                                       # contiguous, and not
         assert torch.equal(blob(src, "cpu"), want)
         assert torch.equal(blob(src, "cuda"), tiled) and torch.equal(blob(src.cuda(), "cuda"), tiled)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("offset", [1, 3, 4])
+def test_weights_that_start_between_16_byte_boundaries(dtype, offset):
+    flat = torch.randn(offset + 48 * 256, device="cuda").to(dtype)
+    view = flat[offset:].view(48, 256)
+    for place in (lambda p: p.to("cuda"), lambda p: p.quantize("cpu")):
+        got, want = (place(FP4Params(w, qtype=Q["sym_int4"])).data for w in (view, view.clone()))
+        assert torch.equal(got, want)
