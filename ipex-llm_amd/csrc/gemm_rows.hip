@@ -28,8 +28,10 @@ __global__ __launch_bounds__(256, 2) void gemm_rows_kernel(const AT *__restrict_
                                                            int steps, float *__restrict__ ws) {
     using F = Fmt<QT>;
     using V8 = typename Vec8<AT>::type;
-    constexpr float OFFSET = code_offset<QT, AT>();
-    constexpr bool NEED_S = QT == QT_ASYM_INT4 || OFFSET != 0.0f, NF4 = QT == QT_NF4;
+    using Op = Operand<QT, AT, false, true>;
+    constexpr float OFFSET = Op::OFFSET;
+    constexpr bool NEED_S = Op::NEED_S;
+    constexpr int PARTS = Op::PARTS;
     constexpr int BM = 16 * MB, NB = RG_NB;
     __shared__ __attribute__((aligned(16))) uint8_t xs[2][BM * 256];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, r = lane & 15, c = lane >> 4;
@@ -84,10 +86,7 @@ __global__ __launch_bounds__(256, 2) void gemm_rows_kernel(const AT *__restrict_
         for (int nb = 0; nb < NB; nb++) acc[mb][nb] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
     const f32x4 zero4 = {0.0f, 0.0f, 0.0f, 0.0f};
     const V8 ones = ones8<AT>();
-    const Nf4Planes planes = NF4 ? nf4_planes<AT, false>() : Nf4Planes{}, planes_lo = NF4 ? nf4_planes<AT, true>() : Nf4Planes{};
-    uint32_t magic;
-    if constexpr (__is_same(AT, _Float16)) asm("v_mov_b32 %0, 0x64006400" : "=v"(magic));
-    else asm("v_mov_b32 %0, 0x43004300" : "=v"(magic));
+    const Op op;
 
     u32x4 xr[MB];
     RowRegs<QT> wc[NB], wn[NB];
@@ -112,7 +111,7 @@ __global__ __launch_bounds__(256, 2) void gemm_rows_kernel(const AT *__restrict_
             const int j = q / MB, mb = q % MB;
             return *(const V8 *)(cur + (mb * 16 + r) * 256 + (((j * 4 + c) ^ r) * 16));
         };
-        V8 a = read_x(0), b[NB], bl[NB];
+        V8 a = read_x(0), b[NB][PARTS];
         float d[2][NB], e[2][NB];                            // of this step and the one before
         f32x4 p[2][NB], sum[2];
 #pragma unroll
@@ -122,23 +121,20 @@ __global__ __launch_bounds__(256, 2) void gemm_rows_kernel(const AT *__restrict_
                 if (q % MB == 0) {
 #pragma unroll
                     for (int nb = 0; nb < NB; nb++) {
-                        const RowRegs<QT> &t = wc[nb];
-                        if constexpr (NF4) {
-                            b[nb] = Unpack<QT, AT>::run(t.q0[j], &planes, magic);
-                            bl[nb] = Unpack<QT, AT>::run(t.q0[j], &planes_lo, magic);
-                        } else if constexpr (F::BITS == 4) b[nb] = Unpack<QT, AT>::run(t.q0[j], nullptr, magic);
-                        else if (j < 2) b[nb] = Unpack8<QT, AT>::run(t.q0[(2 * j) & 3], t.q0[(2 * j + 1) & 3]);
-                        else b[nb] = Unpack8<QT, AT>::run(t.q1[(2 * j) & 3], t.q1[(2 * j + 1) & 3]);
+#pragma unroll
+                        for (int part = 0; part < PARTS; part++) b[nb][part] = op.get(wc[nb], j, part);
                         float mn;
                         hdr_to_scale<QT>(hb[nb][j], d[j & 1][nb], mn);
                         e[j & 1][nb] = mn - OFFSET * d[j & 1][nb];
+                        d[j & 1][nb] = Op::scale(d[j & 1][nb]);
                     }
                 }
                 if constexpr (NEED_S) sum[q & 1] = mfma16(a, ones, zero4);
 #pragma unroll
                 for (int nb = 0; nb < NB; nb++) {
-                    p[q & 1][nb] = mfma16(a, b[nb], zero4);
-                    if constexpr (NF4) p[q & 1][nb] = mfma16(a, bl[nb], p[q & 1][nb]);
+                    p[q & 1][nb] = zero4;
+#pragma unroll
+                    for (int part = 0; part < PARTS; part++) p[q & 1][nb] = mfma16(a, b[nb][part], p[q & 1][nb]);
                 }
                 if (q + 1 < 4 * MB) a = read_x(q + 1);
             }
@@ -147,10 +143,8 @@ __global__ __launch_bounds__(256, 2) void gemm_rows_kernel(const AT *__restrict_
 #pragma unroll
                 for (int nb = 0; nb < NB; nb++)
 #pragma unroll
-                    for (int i = 0; i < 4; i++) {
-                        acc[mb][nb][i] = fmaf(d[j & 1][nb], p[o][nb][i], acc[mb][nb][i]);
-                        if constexpr (NEED_S) acc[mb][nb][i] = fmaf(e[j & 1][nb], sum[o][i], acc[mb][nb][i]);
-                    }
+                    for (int i = 0; i < 4; i++)
+                        acc[mb][nb][i] = Op::add(acc[mb][nb][i], d[j & 1][nb], p[o][nb][i], e[j & 1][nb], sum[o][i]);
 #pragma unroll
                 for (int nb = 0; nb < NB; nb++) asm volatile("" : "+v"(acc[mb][nb]));
             }

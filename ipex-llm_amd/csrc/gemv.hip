@@ -77,10 +77,9 @@ __global__ __launch_bounds__(1024) void gemv_mfma_kernel(const AT *__restrict__ 
                                                          int slots) {
     using F = Fmt<QT>;
     using V8 = typename Vec8<AT>::type;
-    constexpr bool IS4 = (F::BITS == 4);
-    constexpr bool ASYM = (QT == QT_ASYM_INT4);
-    constexpr float OFFSET = code_offset<QT, AT>();
-    constexpr bool NEED_S = ASYM || OFFSET != 0.0f;
+    using Op = Operand<QT, AT, F32, ROWS>;
+    constexpr float OFFSET = Op::OFFSET;
+    constexpr bool NEED_S = Op::NEED_S;
     constexpr int SLICE = U * TILE_COLS;                    // columns of x per wave and round
     constexpr bool ZERO_X = XN == 1 || ROWS;                // how tiles past K are silenced (see the x loads)
     constexpr int XREGION = XN * 512 * (F32 ? 2 : 1);       // elements of AT in a wave's part of LDS
@@ -92,14 +91,8 @@ __global__ __launch_bounds__(1024) void gemv_mfma_kernel(const AT *__restrict__ 
     constexpr int NW = DUAL ? 2 : R;
     static_assert(!(DUAL && R != 1) && XN * 1024 >= NW * MT * 256, "bad GEMV shape parameters");
     static_assert(!ROWS || (!DUAL && MOE == 0), "row-major weights: the plain product only");
-    // nf4 code book in the activation type (byte planes in registers).  With fp32 activations and for row-major weights
-    // (which have always been decoded to fp32) a second table holds what the rounding to AT dropped, and a second
-    // MFMA per sub-block adds it: the weights then carry 16 mantissa bits and more.
-    constexpr bool NF4_LO = QT == QT_NF4 && (F32 || ROWS);
-    const Nf4Planes lut_planes = (QT == QT_NF4) ? nf4_planes<AT, false>() : Nf4Planes{};
-    const Nf4Planes lut_lo_planes = NF4_LO ? nf4_planes<AT, true>() : Nf4Planes{};
-    const void *const lut = &lut_planes, *const lut_lo = &lut_lo_planes;
-    constexpr bool NF4_IN_LDS = QT == QT_NF4 && MT == 1 && !NF4_LO;     // (see Unpack<QT_NF4>)
+    const Op op;
+    constexpr bool NF4_IN_LDS = QT == QT_NF4 && MT == 1 && Op::PARTS == 1;     // (see Unpack<QT_NF4>)
     __shared__ AT lut_lds[16];
     if constexpr (NF4_IN_LDS) {
         if (threadIdx.x < 16) lut_lds[threadIdx.x] = to_at<AT>(NF4_CODEBOOK[threadIdx.x]);
@@ -166,13 +159,6 @@ __global__ __launch_bounds__(1024) void gemv_mfma_kernel(const AT *__restrict__ 
     for (int i = 0; i < NW * MT; i++) acc[i] = 0.0f;
     const V8 ones = ones8<AT>();
     const f32x4 zero4 = {0.0f, 0.0f, 0.0f, 0.0f};
-    // exponent pattern OR-ed onto 4-bit codes (fp16 1024, bf16 128), held in a vector register: as a
-    // literal it would share the instruction's one constant slot with the nibble mask and split every
-    // v_and_or_b32 into an AND and an OR
-    uint32_t magic;
-    if constexpr (sizeof(AT) == 2 && __is_same(AT, _Float16)) asm("v_mov_b32 %0, 0x64006400" : "=v"(magic));
-    else asm("v_mov_b32 %0, 0x43004300" : "=v"(magic));
-
     for (int g0 = 0; g0 < G; g0 += W * U) {
         const int gw = g0 + wave * U;
         // Straight-line loads (addresses clamped instead of branches, so that the compiler can
@@ -283,9 +269,7 @@ __global__ __launch_bounds__(1024) void gemv_mfma_kernel(const AT *__restrict__ 
                 for (int j = 0; j < 4; j++) {
                     V8 b;
                     if constexpr (NF4_IN_LDS) b = Unpack<QT, AT>::run_lds(tl.q0[j], lut_lds);
-                    else if constexpr (IS4) b = Unpack<QT, AT>::run(tl.q0[j], lut, magic);
-                    else if (j < 2) b = Unpack8<QT, AT>::run(tl.q0[2 * j], tl.q0[2 * j + 1]);
-                    else b = Unpack8<QT, AT>::run(tl.q1[2 * (j - 2)], tl.q1[2 * (j - 2) + 1]);
+                    else b = op.get(tl, j, 0);
                     float d, mn;
                     if constexpr (ROWS) hdr_to_scale<QT>(hb[j], d, mn);
                     else tile_scale<QT>(tl, j, d, mn);
@@ -299,22 +283,21 @@ __global__ __launch_bounds__(1024) void gemv_mfma_kernel(const AT *__restrict__ 
                     }
                     f32x4 p = mfma16(a[j], b, zero4);
                     if constexpr (F32) p = mfma16(al[j], b, p);
-                    if constexpr (NF4_LO) {
-                        const V8 bl = Unpack<QT, AT>::run(tl.q0[j], lut_lo, magic);
-                        p = mfma16(a[j], bl, p);
-                        if constexpr (F32) p = mfma16(al[j], bl, p);
+#pragma unroll
+                    for (int part = 1; part < Op::PARTS; part++) {
+                        b = op.get(tl, j, part);
+                        p = mfma16(a[j], b, p);
+                        if constexpr (F32) p = mfma16(al[j], b, p);
                     }
+                    f32x4 s = zero4;
                     if constexpr (NEED_S) {
-                        f32x4 s = mfma16(a[j], ones, zero4);
+                        s = mfma16(a[j], ones, zero4);
                         if constexpr (F32) s = mfma16(al[j], ones, s);
-                        const float e = mn - OFFSET * d;
-#pragma unroll
-                        for (int i = 0; i < MT; i++)
-                            acc[wi * MT + i] = fmaf(e, s[i], fmaf(d, p[i], acc[wi * MT + i]));
-                    } else {
-#pragma unroll
-                        for (int i = 0; i < MT; i++) acc[wi * MT + i] = fmaf(d, p[i], acc[wi * MT + i]);
                     }
+                    const float e = mn - OFFSET * d;
+                    d = Op::scale(d);
+#pragma unroll
+                    for (int i = 0; i < MT; i++) acc[wi * MT + i] = Op::add(acc[wi * MT + i], d, p[i], e, s[i]);
                 }
             }
     }

@@ -36,8 +36,10 @@ __global__ __launch_bounds__(64 * wide_max_waves(MB, DUAL ? 2 * R : R, F32)) voi
     using F = Fmt<QT>;
     using V8 = typename Vec8<AT>::type;
     using ET = typename std::conditional<F32, float, AT>::type;
-    constexpr float OFFSET = code_offset<QT, AT>();
-    constexpr bool NEED_S = QT == QT_ASYM_INT4 || OFFSET != 0.0f, NF4 = QT == QT_NF4, NF4_LO = NF4 && (F32 || ROWS);
+    using Op = Operand<QT, AT, F32, ROWS>;
+    constexpr float OFFSET = Op::OFFSET;
+    constexpr bool NEED_S = Op::NEED_S;
+    constexpr int PARTS = Op::PARTS;
     constexpr int NT = DUAL ? 2 * R : R;                     // weight tiles per group; DUAL: R of the gate, R of the up weight
     static_assert(!DUAL || (!F32 && !ROWS), "the fused form takes 16-bit activations and tiled weights");
     constexpr int PLANE = 16 * MB * 256, XBYTES = PLANE * (F32 ? 2 : 1), XC = 4 * MB;     // bytes of x in LDS; chunks of 8 per lane
@@ -108,10 +110,7 @@ __global__ __launch_bounds__(64 * wide_max_waves(MB, DUAL ? 2 * R : R, F32)) voi
         for (int mb = 0; mb < MB; mb++) acc[wi][mb] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
     const f32x4 zero4 = {0.0f, 0.0f, 0.0f, 0.0f};
     const V8 ones = ones8<AT>();
-    const Nf4Planes planes = NF4 ? nf4_planes<AT, false>() : Nf4Planes{}, planes_lo = NF4_LO ? nf4_planes<AT, true>() : Nf4Planes{};
-    uint32_t magic;
-    if constexpr (__is_same(AT, _Float16)) asm("v_mov_b32 %0, 0x64006400" : "=v"(magic));
-    else asm("v_mov_b32 %0, 0x43004300" : "=v"(magic));
+    const Op op;
 
     typename std::conditional<ROWS, RowRegs<QT>, TileRegs<QT>>::type wc[NT], wn[NT];
     u32x4 xv[F32 ? 2 * XC : XC];
@@ -134,21 +133,17 @@ __global__ __launch_bounds__(64 * wide_max_waves(MB, DUAL ? 2 * R : R, F32)) voi
         }
 #pragma unroll
         for (int j = 0; j < 4; j++) {
-            V8 b[NT], bl[NT];
+            V8 b[NT][PARTS];
             float d[NT], e[NT];
 #pragma unroll
             for (int wi = 0; wi < NT; wi++) {
-                const auto &t = wc[wi];
-                if constexpr (NF4) {
-                    b[wi] = Unpack<QT, AT>::run(t.q0[j], &planes, magic);
-                    if constexpr (NF4_LO) bl[wi] = Unpack<QT, AT>::run(t.q0[j], &planes_lo, magic);
-                } else if constexpr (F::BITS == 4) b[wi] = Unpack<QT, AT>::run(t.q0[j], nullptr, magic);
-                else if (j < 2) b[wi] = Unpack8<QT, AT>::run(t.q0[(2 * j) & 3], t.q0[(2 * j + 1) & 3]);
-                else b[wi] = Unpack8<QT, AT>::run(t.q1[(2 * j) & 3], t.q1[(2 * j + 1) & 3]);
+#pragma unroll
+                for (int part = 0; part < PARTS; part++) b[wi][part] = op.get(wc[wi], j, part);
                 float mn;
                 if constexpr (ROWS) hdr_to_scale<QT>(hb[wi][j], d[wi], mn);
                 else tile_scale<QT>(wc[wi], j, d[wi], mn);
                 e[wi] = mn - OFFSET * d[wi];
+                d[wi] = Op::scale(d[wi]);
             }
 #pragma unroll
             for (int mb = 0; mb < MB; mb++) {
@@ -163,17 +158,14 @@ __global__ __launch_bounds__(64 * wide_max_waves(MB, DUAL ? 2 * R : R, F32)) voi
                 }
 #pragma unroll
                 for (int wi = 0; wi < NT; wi++) {
-                    f32x4 p = mfma16(a, b[wi], zero4);
-                    if constexpr (F32) p = mfma16(al, b[wi], p);
-                    if constexpr (NF4_LO) {
-                        p = mfma16(a, bl[wi], p);
-                        if constexpr (F32) p = mfma16(al, bl[wi], p);
+                    f32x4 p = zero4;
+#pragma unroll
+                    for (int part = 0; part < PARTS; part++) {
+                        p = mfma16(a, b[wi][part], p);
+                        if constexpr (F32) p = mfma16(al, b[wi][part], p);
                     }
 #pragma unroll
-                    for (int i = 0; i < 4; i++) {
-                        acc[wi][mb][i] = fmaf(d[wi], p[i], acc[wi][mb][i]);
-                        if constexpr (NEED_S) acc[wi][mb][i] = fmaf(e[wi], s[i], acc[wi][mb][i]);
-                    }
+                    for (int i = 0; i < 4; i++) acc[wi][mb][i] = Op::add(acc[wi][mb][i], d[wi], p[i], e[wi], s[i]);
                 }
             }
 #pragma unroll

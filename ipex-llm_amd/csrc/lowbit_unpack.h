@@ -8,8 +8,9 @@ namespace lowbit {
 // ---- codes of one sub-block (8 columns of this lane) -> B operand ----------
 //
 // The operand holds the *unscaled* code value (q - 8, q, int8, e4m3 value, nf4
-// code-book entry); OFFSET<> says what constant is still folded in and has to
+// code-book entry); OFFSET says what constant is still folded in and has to
 // be removed with the row sum of x (0 for every path below except bf16 4-bit).
+// What the kernels use of this, and how, is Operand below.
 
 template <int QT, typename AT> struct Unpack;
 
@@ -74,13 +75,13 @@ struct Nf4Planes {
     uint32_t k04, k0123;          // 0x04040404 and 0x03020100 in vector registers: as literals the two would need the
                                   // one constant slot of v_and_or_b32 twice
 };
-// RESID: what rounding the code book to AT dropped (the second term of the fp32-output variants)
-template <typename AT, bool RESID> __device__ inline Nf4Planes nf4_planes() {
+// PART 0 is the code book rounded to AT, part 1 what the rounding dropped.
+template <typename AT, int PART> __device__ inline Nf4Planes nf4_planes() {
     Nf4Planes t = {};
 #pragma unroll
     for (int i = 0; i < 16; i++) {                      // (constants: folded at compile time)
         const AT main = to_at<AT>(NF4_CODEBOOK[i]);
-        const AT v = RESID ? to_at<AT>(NF4_CODEBOOK[i] - (float)main) : main;
+        const AT v = PART == 1 ? to_at<AT>(NF4_CODEBOOK[i] - (float)main) : main;
         const uint32_t b = __builtin_bit_cast(uint16_t, v);
         t.lo[i / 4] |= (b & 0xffu) << (8 * (i % 4));
         t.hi[i / 4] |= (b >> 8) << (8 * (i % 4));
@@ -117,6 +118,17 @@ template <typename AT> struct Unpack<QT_NF4, AT> {
         return r;
     }
 };
+
+// 4-bit integer codes centred, in bf16: (q - 8) / 16, which v_cvt_off_f32_i4 makes of the low four bits of a byte whose
+// bit 3 is flipped.  14 instructions per dword of codes (the or-ed pattern of UnpackInt4Bf16: 7; a lookup as nf4's: 21).
+__device__ inline bf16x8 centred_bf16(uint32_t v) {
+    const uint32_t lo = v ^ 0x88888888u;
+    uint32_t hi = lo >> 4;
+    asm("" : "+v"(hi));                                 // (its bytes are then picked by the conversion itself)
+    auto code = [](uint32_t byte) { return (__bf16)__builtin_amdgcn_cvt_off_f32_i4((int)byte); };
+    return bf16x8{code(lo), code((lo >> 16) & 0xff), code(hi), code((hi >> 16) & 0xff),
+                  code((lo >> 8) & 0xff), code(lo >> 24), code((hi >> 8) & 0xff), code(hi >> 24)};
+}
 
 // 8-bit codes: two dwords (columns 0..3, 4..7).
 template <int QT, typename AT> struct Unpack8;
@@ -163,10 +175,58 @@ template <> struct Unpack8<QT_FP8_E4M3, __bf16> {
     }
 };
 
-template <int QT, typename AT> constexpr float code_offset() {
-    if constexpr (Fmt<QT>::BITS == 4) return Unpack<QT, AT>::OFFSET;
-    else return 0.0f;
-}
+// The MFMA operand that codes become in a kernel, and what the kernel has to know about it.
+//   PARTS   16-bit operands whose sum is the code's value, one MFMA each
+//   OFFSET  constant still in the value, removed through the row sum of x (NEED_S)
+// Tiled weights with 16-bit activations: one part, the constant as Unpack has it.  F32 (float32 activations): nf4 in two.
+// ROWS (row-major weights): what was decoded to fp32 before the product has operands that keep its precision.
+//   4-bit integers are centred, q - 8.  With the 128 or 136 that Unpack leaves in bf16, fp32 sums some 17 times larger
+//     cancel: float32 activations were off by 3.8e-6 of the result's norm in place of 2.5e-6, and ten times as many bf16
+//     results were not the nearest one.  asym_int4's minimum, mostly near -7.5 scales, goes with the 8, and a step's two
+//     terms meet before they go to the sum, which is then rounded once a step (fp16 results of 8640 columns that are not
+//     the nearest: 1.23 in a thousand with two FMAs, 0.98 this way, 1.05 from weights in fp32).
+template <int QT, typename AT, bool F32, bool ROWS> struct Operand {
+    using V8 = typename Vec8<AT>::type;
+    static constexpr bool NF4 = QT == QT_NF4, INT4 = QT == QT_SYM_INT4 || QT == QT_ASYM_INT4;
+    static constexpr bool CENTRED = ROWS && INT4, CENTRED_BF16 = CENTRED && __is_same(AT, __bf16);
+    static constexpr int PARTS = NF4 && (F32 || ROWS) ? 2 : 1;
+    static constexpr float offset() {
+        if constexpr (CENTRED) return QT == QT_ASYM_INT4 ? -8.0f : 0.0f;
+        else if constexpr (INT4) return Unpack<QT, AT>::OFFSET;
+        else return 0.0f;
+    }
+    static constexpr float OFFSET = offset();
+    static constexpr bool NEED_S = QT == QT_ASYM_INT4 || OFFSET != 0.0f;
+
+    Nf4Planes planes[PARTS];
+    // exponent pattern OR-ed onto 4-bit codes (fp16 1024, bf16 128), held in a vector register: as a literal it would share
+    // the instruction's one constant slot with the nibble mask and split every v_and_or_b32 into an AND and an OR
+    uint32_t magic;
+
+    __device__ Operand() {
+        if constexpr (NF4) planes[0] = nf4_planes<AT, 0>();
+        if constexpr (PARTS > 1) planes[1] = nf4_planes<AT, 1>();
+        if constexpr (__is_same(AT, _Float16)) asm("v_mov_b32 %0, 0x64006400" : "=v"(magic));
+        else asm("v_mov_b32 %0, 0x43004300" : "=v"(magic));
+    }
+    // what a step's product is to be multiplied by, from its block's scale
+    __device__ static float scale(float d) { return CENTRED_BF16 ? 16.0f * d : d; }
+    // sum + d * p + e * s: that times the step's product, e (see OFFSET) times the row sum of x
+    __device__ static float add(float sum, float d, float p, float e, float s) {
+        if constexpr (!NEED_S) return fmaf(d, p, sum);
+        else if constexpr (ROWS) return sum + fmaf(e, s, d * p);
+        else return fmaf(e, s, fmaf(d, p, sum));
+    }
+    // part p of step j's eight codes; t: TileRegs, or RowRegs after arrange_rows
+    template <typename Regs> __device__ V8 get(const Regs &t, int j, int p) const {
+        if constexpr (NF4) return Unpack<QT_NF4, AT>::run(t.q0[j], &planes[p], magic);
+        else if constexpr (CENTRED_BF16) return centred_bf16(t.q0[j]);
+        else if constexpr (CENTRED) return Unpack<QT_SYM_INT4, AT>::run(t.q0[j], nullptr, magic);
+        else if constexpr (INT4) return Unpack<QT, AT>::run(t.q0[j], nullptr, magic);
+        else if (j < 2) return Unpack8<QT, AT>::run(t.q0[(2 * j) & 3], t.q0[(2 * j + 1) & 3]);
+        else return Unpack8<QT, AT>::run(t.q1[(2 * j) & 3], t.q1[(2 * j + 1) & 3]);
+    }
+};
 
 template <typename AT> __device__ inline typename Vec8<AT>::type ones8() {
     typename Vec8<AT>::type r;

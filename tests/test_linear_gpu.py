@@ -5,7 +5,8 @@ import torch
 
 import ipex_llm.ggml.model.llama.llama_cpp as ggml
 import lowbit_oracle as orc
-from gpu_util import ALL, DT, FP8, acts, dev_quantize, stream, weights
+from gpu_util import ALL, DT, FP8, NF4, acts, dev_quantize, stream, weights
+from ipex_llm.transformers.low_bit_linear import FP4Params, LowBitLinear
 
 pytestmark = pytest.mark.gpu
 GGML, TILED = ggml.LAYOUT_GGML, ggml.LAYOUT_TILED
@@ -57,3 +58,33 @@ def test_float32_activations_in_one_pass(qtype, m, n, k):
 @pytest.mark.parametrize("m,n,k", [(3, 512, 256), (40, 4096, 1024), (50, 2048, 6400), (300, 272, 2048), (512, 16384, 128), (1030, 2048, 256), (200, 1040, 128)])
 def test_bias_of_every_kernel(qtype, dtype, m, n, k):
     _check(qtype, dtype, TILED, m, n, k, True, 500 * m + n)
+
+
+# Every form of the row-major kernels: 1 .. 4, 5 .. 8, up to 16 rows, the one-pass kernel, the GEMM with and without K splits
+ROW_MAJOR = [(1, 2000, 4160), (7, 1000, 4160), (12, 1000, 4160), (16, 16399, 1088), (30, 1000, 4160), (70, 1000, 4160), (333, 1000, 4160)]
+
+
+def _row_major(qtype, m, n, k, dtype):
+    if qtype == FP8:
+        n, k = n + 1, (k + 127) // 128 * 128
+    w, x = weights(m, (n, k), outliers=False), acts(m + 1, m, k, dtype)
+    layer = LowBitLinear(k, n, qtype, bias=False, conver_to_half=False).eval()
+    layer.weight = FP4Params(torch.from_numpy(w), qtype=qtype).to("cuda")
+    with torch.no_grad():
+        y = layer(x.cuda()).cpu()
+    return y, x, torch.from_numpy(orc.dequantize(orc.quantize(w, qtype), qtype, (n, k)).astype(np.float64))
+
+
+@pytest.mark.parametrize("qtype", [t for t in ALL if t != NF4])
+@pytest.mark.parametrize("m,n,k", ROW_MAJOR)
+def test_row_major_weights_are_as_exact_as_in_fp32(qtype, m, n, k):
+    """What is left beside the results' own rounding is that of fp32 sums: 2^-24 per step, in at most K / 32 = 136 random
+    steps of at most the result's size, is 7e-7 of the norm."""
+    y, x, w = _row_major(qtype, m, n, k, torch.float32)
+    hi = x.bfloat16().double()
+    want = (hi + (x.double() - hi).bfloat16().double()) @ w.t()                   # float32 activations go in as two bf16 planes
+    assert (y.double() - want).norm() <= 7e-7 * want.norm()
+    y, x, w = _row_major(qtype, m, n, k, torch.bfloat16)
+    want = x.double() @ w.t()
+    # an error of 7e-7 moves a result over a rounding border of bf16 (2^-9 to 2^-8 apart) in 2 * 7e-7 / 2^-9 of the cases
+    assert (y != want.bfloat16()).float().mean() <= 7e-4
