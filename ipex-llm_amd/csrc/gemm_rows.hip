@@ -131,11 +131,7 @@ __global__ __launch_bounds__(256, 2) void gemm_rows_kernel(const AT *__restrict_
                 }
                 if constexpr (NEED_S) sum[q & 1] = mfma16(a, ones, zero4);
 #pragma unroll
-                for (int nb = 0; nb < NB; nb++) {
-                    p[q & 1][nb] = zero4;
-#pragma unroll
-                    for (int part = 0; part < PARTS; part++) p[q & 1][nb] = mfma16(a, b[nb][part], p[q & 1][nb]);
-                }
+                for (int nb = 0; nb < NB; nb++) p[q & 1][nb] = Op::product(a, a, b[nb]);
                 if (q + 1 < 4 * MB) a = read_x(q + 1);
             }
             if (q > 0) {

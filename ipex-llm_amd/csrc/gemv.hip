@@ -267,9 +267,12 @@ __global__ __launch_bounds__(1024) void gemv_mfma_kernel(const AT *__restrict__ 
                 }
 #pragma unroll
                 for (int j = 0; j < 4; j++) {
-                    V8 b;
-                    if constexpr (NF4_IN_LDS) b = Unpack<QT, AT>::run_lds(tl.q0[j], lut_lds);
-                    else b = op.get(tl, j, 0);
+                    V8 b[Op::PARTS];
+#pragma unroll
+                    for (int part = 0; part < Op::PARTS; part++) {
+                        if constexpr (NF4_IN_LDS) b[part] = Unpack<QT, AT>::run_lds(tl.q0[j], lut_lds);
+                        else b[part] = op.get(tl, j, part);
+                    }
                     float d, mn;
                     if constexpr (ROWS) hdr_to_scale<QT>(hb[j], d, mn);
                     else tile_scale<QT>(tl, j, d, mn);
@@ -281,14 +284,7 @@ __global__ __launch_bounds__(1024) void gemv_mfma_kernel(const AT *__restrict__ 
                         d = live ? d : 0.0f;
                         mn = live ? mn : 0.0f;
                     }
-                    f32x4 p = mfma16(a[j], b, zero4);
-                    if constexpr (F32) p = mfma16(al[j], b, p);
-#pragma unroll
-                    for (int part = 1; part < Op::PARTS; part++) {
-                        b = op.get(tl, j, part);
-                        p = mfma16(a[j], b, p);
-                        if constexpr (F32) p = mfma16(al[j], b, p);
-                    }
+                    const f32x4 p = Op::product(a[j], al[j], b);
                     f32x4 s = zero4;
                     if constexpr (NEED_S) {
                         s = mfma16(a[j], ones, zero4);

@@ -158,12 +158,7 @@ __global__ __launch_bounds__(64 * wide_max_waves(MB, DUAL ? 2 * R : R, F32)) voi
                 }
 #pragma unroll
                 for (int wi = 0; wi < NT; wi++) {
-                    f32x4 p = zero4;
-#pragma unroll
-                    for (int part = 0; part < PARTS; part++) {
-                        p = mfma16(a, b[wi][part], p);
-                        if constexpr (F32) p = mfma16(al, b[wi][part], p);
-                    }
+                    const f32x4 p = Op::product(a, al, b[wi]);
 #pragma unroll
                     for (int i = 0; i < 4; i++) acc[wi][mb][i] = Op::add(acc[wi][mb][i], d[wi], p[i], e[wi], s[i]);
                 }

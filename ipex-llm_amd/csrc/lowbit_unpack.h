@@ -75,14 +75,13 @@ struct Nf4Planes {
     uint32_t k04, k0123;          // 0x04040404 and 0x03020100 in vector registers: as literals the two would need the
                                   // one constant slot of v_and_or_b32 twice
 };
-// PART 0 is the code book rounded to AT, part 1 what the rounding dropped.
-template <typename AT, int PART> __device__ inline Nf4Planes nf4_planes() {
+// PART 0 is the code book times SCALE rounded to AT, the next parts what the rounding of those before dropped.
+template <typename AT, int PART, int SCALE> __device__ inline Nf4Planes nf4_planes() {
     Nf4Planes t = {};
 #pragma unroll
     for (int i = 0; i < 16; i++) {                      // (constants: folded at compile time)
-        const AT main = to_at<AT>(NF4_CODEBOOK[i]);
-        const AT v = PART == 1 ? to_at<AT>(NF4_CODEBOOK[i] - (float)main) : main;
-        const uint32_t b = __builtin_bit_cast(uint16_t, v);
+        const float v0 = NF4_CODEBOOK[i] * (float)SCALE, v1 = v0 - (float)to_at<AT>(v0), v2 = v1 - (float)to_at<AT>(v1);
+        const uint32_t b = __builtin_bit_cast(uint16_t, to_at<AT>(PART == 0 ? v0 : PART == 1 ? v1 : v2));
         t.lo[i / 4] |= (b & 0xffu) << (8 * (i % 4));
         t.hi[i / 4] |= (b >> 8) << (8 * (i % 4));
     }
@@ -185,11 +184,16 @@ template <> struct Unpack8<QT_FP8_E4M3, __bf16> {
 //     results were not the nearest one.  asym_int4's minimum, mostly near -7.5 scales, goes with the 8, and a step's two
 //     terms meet before they go to the sum, which is then rounded once a step (fp16 results of 8640 columns that are not
 //     the nearest: 1.23 in a thousand with two FMAs, 0.98 this way, 1.05 from weights in fp32).
+//   nf4's code book has 24 mantissa bits: three parts in bf16, which hold it exactly (two were off by up to 5e-6 of an entry:
+//     3.5e-6 of the result's norm with float32 activations, 2.6 bf16 results in a thousand not the nearest one, 0.17 from
+//     weights in fp32), two in fp16 with the book scaled by 2^14, which keeps the second one clear of fp16's subnormal
+//     numbers: three of the 16 entries are then off by one in the 24th bit, the others exact.
 template <int QT, typename AT, bool F32, bool ROWS> struct Operand {
     using V8 = typename Vec8<AT>::type;
     static constexpr bool NF4 = QT == QT_NF4, INT4 = QT == QT_SYM_INT4 || QT == QT_ASYM_INT4;
     static constexpr bool CENTRED = ROWS && INT4, CENTRED_BF16 = CENTRED && __is_same(AT, __bf16);
-    static constexpr int PARTS = NF4 && (F32 || ROWS) ? 2 : 1;
+    static constexpr int PARTS = !NF4 ? 1 : ROWS ? (__is_same(AT, __bf16) ? 3 : 2) : F32 ? 2 : 1;
+    static constexpr int NF4_SCALE = NF4 && ROWS && __is_same(AT, _Float16) ? 1 << 14 : 1;
     static constexpr float offset() {
         if constexpr (CENTRED) return QT == QT_ASYM_INT4 ? -8.0f : 0.0f;
         else if constexpr (INT4) return Unpack<QT, AT>::OFFSET;
@@ -204,18 +208,31 @@ template <int QT, typename AT, bool F32, bool ROWS> struct Operand {
     uint32_t magic;
 
     __device__ Operand() {
-        if constexpr (NF4) planes[0] = nf4_planes<AT, 0>();
-        if constexpr (PARTS > 1) planes[1] = nf4_planes<AT, 1>();
+        if constexpr (NF4) planes[0] = nf4_planes<AT, 0, NF4_SCALE>();
+        if constexpr (PARTS > 1) planes[1] = nf4_planes<AT, 1, NF4_SCALE>();
+        if constexpr (PARTS > 2) planes[2] = nf4_planes<AT, 2, NF4_SCALE>();
         if constexpr (__is_same(AT, _Float16)) asm("v_mov_b32 %0, 0x64006400" : "=v"(magic));
         else asm("v_mov_b32 %0, 0x43004300" : "=v"(magic));
     }
     // what a step's product is to be multiplied by, from its block's scale
-    __device__ static float scale(float d) { return CENTRED_BF16 ? 16.0f * d : d; }
+    __device__ static float scale(float d) { return CENTRED_BF16 ? 16.0f * d : d * (1.0f / NF4_SCALE); }
     // sum + d * p + e * s: that times the step's product, e (see OFFSET) times the row sum of x
     __device__ static float add(float sum, float d, float p, float e, float s) {
         if constexpr (!NEED_S) return fmaf(d, p, sum);
         else if constexpr (ROWS) return sum + fmaf(e, s, d * p);
         else return fmaf(e, s, fmaf(d, p, sum));
+    }
+    // a step's product; al: what x's first plane leaves (F32).  The largest first: an MFMA drops more of a small sum that it
+    // is given beside large products than of small products beside a large sum (fp16, 8640 columns: 1.48 in a thousand not
+    // the nearest result the other way round, 1.14 this way).  The smallest parts of both are below fp32.
+    __device__ static f32x4 product(const V8 &a, const V8 &al, const V8 (&b)[PARTS]) {
+        f32x4 p = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int part = 0; part < PARTS; part++) {
+            p = mfma16(a, b[part], p);
+            if (F32 && part < 2) p = mfma16(al, b[part], p);
+        }
+        return p;
     }
     // part p of step j's eight codes; t: TileRegs, or RowRegs after arrange_rows
     template <typename Regs> __device__ V8 get(const Regs &t, int j, int p) const {

@@ -5,7 +5,7 @@ import torch
 
 import ipex_llm.ggml.model.llama.llama_cpp as ggml
 import lowbit_oracle as orc
-from gpu_util import ALL, DT, FP8, NF4, acts, dev_quantize, stream, weights
+from gpu_util import ALL, DT, FP8, acts, dev_quantize, stream, weights
 from ipex_llm.transformers.low_bit_linear import FP4Params, LowBitLinear
 
 pytestmark = pytest.mark.gpu
@@ -75,7 +75,7 @@ def _row_major(qtype, m, n, k, dtype):
     return y, x, torch.from_numpy(orc.dequantize(orc.quantize(w, qtype), qtype, (n, k)).astype(np.float64))
 
 
-@pytest.mark.parametrize("qtype", [t for t in ALL if t != NF4])
+@pytest.mark.parametrize("qtype", ALL)
 @pytest.mark.parametrize("m,n,k", ROW_MAJOR)
 def test_row_major_weights_are_as_exact_as_in_fp32(qtype, m, n, k):
     """What is left beside the results' own rounding is that of fp32 sums: 2^-24 per step, in at most K / 32 = 136 random
