@@ -167,20 +167,29 @@ __global__ __launch_bounds__(256, 2) void gemm_rows_kernel(const AT *__restrict_
         const int n = n0 + nb * TILE_ROWS + r;
         if (n >= N) continue;
         const float bv = bias ? (float)bias[n] : 0.0f;
+        uint32_t again = 0;                                   // results that are not finite, see dot_fp32
 #pragma unroll
         for (int mb = 0; mb < MB; mb++)
 #pragma unroll
             for (int i = 0; i < 4; i++) {
                 const int m = m0 + mb * 16 + c * 4 + i;
-                if (m < M) y[(int64_t)m * N + n] = to_at<AT>(acc[mb][nb][i] + bv);
+                if (m < M) {
+                    y[(int64_t)m * N + n] = to_at<AT>(acc[mb][nb][i] + bv);
+                    again |= __builtin_isfinite(acc[mb][nb][i]) ? 0u : 1u << (mb * 4 + i);
+                }
             }
+        for (; again; again &= again - 1) {
+            const int bit = __builtin_ctz(again), m = m0 + bit / 4 * 16 + c * 4 + bit % 4;
+            y[(int64_t)m * N + n] = to_at<AT>(dot_fp32<QT, true>(x + (int64_t)m * K, w, n, K) + bv);
+        }
     }
 }
 
 // Sums the splits and writes y, rounded once: one thread per four rows of one column.
-template <typename AT, int MB>
-__global__ __launch_bounds__(256) void gemm_rows_reduce_kernel(const f32x4 *__restrict__ ws, const AT *__restrict__ bias,
-                                                               AT *__restrict__ y, int M, int N, int tiles, int splits) {
+template <int QT, typename AT, int MB>
+__global__ __launch_bounds__(256) void gemm_rows_reduce_kernel(const f32x4 *__restrict__ ws, const AT *__restrict__ x,
+                                                               const uint8_t *__restrict__ w, const AT *__restrict__ bias,
+                                                               AT *__restrict__ y, int M, int N, int K, int tiles, int splits) {
     constexpr int PER_TILE = RG_WAVES * MB * RG_NB * 64;     // a multiple of 256
     const int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x;
     const int tiles_m = (M + 16 * MB - 1) / (16 * MB);
@@ -195,6 +204,11 @@ __global__ __launch_bounds__(256) void gemm_rows_reduce_kernel(const f32x4 *__re
 #pragma unroll
     for (int i = 0; i < 4; i++)
         if (m + i < M) y[(int64_t)(m + i) * N + n] = to_at<AT>(a[i] + bv);
+    for (int i = 0; i < 4; i++) {                            // results that are not finite, see dot_fp32
+        const float sum = i == 0 ? a[0] : i == 1 ? a[1] : i == 2 ? a[2] : a[3];
+        if (m + i < M && !__builtin_isfinite(sum))
+            y[(int64_t)(m + i) * N + n] = to_at<AT>(dot_fp32<QT, true>(x + (int64_t)(m + i) * K, w, n, K) + bv);
+    }
 }
 
 struct RowsPlan {
@@ -230,8 +244,9 @@ static void launch_rows_m(const void *x, const void *w, const void *bias, void *
     hipLaunchKernelGGL((gemm_rows_kernel<QT, AT, MB>), dim3((p.tiles + 7) / 8 * 8, p.splits), dim3(256), 0, st, (const AT *)x,
                        (const uint8_t *)w, (const AT *)bias, (AT *)y, M, N, K, p.steps, ws);
     if (ws)
-        hipLaunchKernelGGL((gemm_rows_reduce_kernel<AT, MB>), dim3((unsigned)((int64_t)p.tiles * RG_WAVES * MB * RG_NB * 64 / 256)), dim3(256),
-                           0, st, (const f32x4 *)ws, (const AT *)bias, (AT *)y, M, N, p.tiles, p.splits);
+        hipLaunchKernelGGL((gemm_rows_reduce_kernel<QT, AT, MB>), dim3((unsigned)((int64_t)p.tiles * RG_WAVES * MB * RG_NB * 64 / 256)),
+                           dim3(256), 0, st, (const f32x4 *)ws, (const AT *)x, (const uint8_t *)w, (const AT *)bias, (AT *)y, M, N, K,
+                           p.tiles, p.splits);
 }
 
 template <int QT, typename AT>

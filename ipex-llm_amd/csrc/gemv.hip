@@ -37,6 +37,11 @@ __device__ inline MoeId moe_id(const void *ids, bool ids64, int pair, int n_exp)
     return {(int)(e < 0 ? 0 : e < n_exp ? e : n_exp - 1), e >= 0 && e < n_exp};
 }
 
+__device__ inline float load_route_w(const void *w, int dtype, int pair) {
+    return dtype == DT_F32 ? ((const float *)w)[pair]
+           : dtype == DT_F16 ? (float)((const _Float16 *)w)[pair] : (float)((const __bf16 *)w)[pair];
+}
+
 // One workgroup = one tile row (16 output columns).  Per round, wave w owns U consecutive
 // tiles along K: it first issues every weight load of the round (so the whole slice is in
 // flight at once), then copies its slice of x into a wave-private LDS region, then runs
@@ -80,6 +85,9 @@ __global__ __launch_bounds__(1024) void gemv_mfma_kernel(const AT *__restrict__ 
     using Op = Operand<QT, AT, F32, ROWS>;
     constexpr float OFFSET = Op::OFFSET;
     constexpr bool NEED_S = Op::NEED_S;
+    // Row-major weights and the experts' pairs were products with decoded weights before they came here; tiled weights up to
+    // eight rows never were.
+    constexpr bool AGAIN = ROWS || MOE != 0;
     constexpr int SLICE = U * TILE_COLS;                    // columns of x per wave and round
     constexpr bool ZERO_X = XN == 1 || ROWS;                // how tiles past K are silenced (see the x loads)
     constexpr int XREGION = XN * 512 * (F32 ? 2 : 1);       // elements of AT in a wave's part of LDS
@@ -140,8 +148,7 @@ __global__ __launch_bounds__(1024) void gemv_mfma_kernel(const AT *__restrict__ 
         const int pair = blockIdx.y * slots + (lane < slots ? lane : 0);
         const MoeId id = moe_id(ids, ids64, pair, n_exp);
         slot_w = (uint64_t)((const uint8_t *const *)w)[id.clamped];
-        slot_rw = route_dtype == DT_F32 ? ((const float *)route_w)[pair]
-                  : route_dtype == DT_F16 ? (float)((const _Float16 *)route_w)[pair] : (float)((const __bf16 *)route_w)[pair];
+        slot_rw = load_route_w(route_w, route_dtype, pair);
         if (ids64 && !id.valid) slot_rw = 0.0f;
     }
     auto moe_tile = [&](int g, float &rw) -> gbytes {
@@ -310,23 +317,50 @@ __global__ __launch_bounds__(1024) void gemv_mfma_kernel(const AT *__restrict__ 
     // wave v sums and writes tile row v of the R rows (DUAL: wave 0 combines both weights)
     if (wave < (DUAL ? 1 : R)) {
         const int grp = lane >> 4, col = lane & 15;
-#pragma unroll
-        for (int i = 0; i < MT; i++) {
-            float s = 0.0f;
-            for (int ww = 0; ww < W; ww++) s += red[ww * RS + (wave * MT + i) * 64 + lane];
-            if constexpr (DUAL) {
-                float u = 0.0f;
-                for (int ww = 0; ww < W; ww++) u += red[ww * RS + (MT + i) * 64 + lane];
-                s = gate_act(s, act) * u;
-            }
-            const int m = grp * MT + i;
-            const int64_t n = ((int64_t)blockIdx.x * R + wave) * 16 + col;
-            if (m >= M || (ROWS && n >= N)) continue;
+        const int64_t n = ((int64_t)blockIdx.x * R + wave) * 16 + col;
+        auto store = [&](int m, float s, float up) __attribute__((always_inline)) {
+            if constexpr (DUAL) s = gate_act(s, act) * up;
             if constexpr (F32) {
                 ((float *)y)[(int64_t)m * N + n] = bias ? s + ((const float *)bias)[n] : s;
             } else {
                 if constexpr (!DUAL && MOE == 0) s += bias ? (float)bias[n] : 0.0f;
                 y[(int64_t)m * N + n] = to_at<AT>(s);
+            }
+        };
+        uint32_t again = 0;                                 // AGAIN: results that are not finite, see dot_fp32
+#pragma unroll
+        for (int i = 0; i < MT; i++) {
+            float s = 0.0f, up = 0.0f;
+            for (int ww = 0; ww < W; ww++) s += red[ww * RS + (wave * MT + i) * 64 + lane];
+            if constexpr (DUAL) {
+                for (int ww = 0; ww < W; ww++) up += red[ww * RS + (MT + i) * 64 + lane];
+            }
+            const int m = grp * MT + i;
+            if (m >= M || (ROWS && n >= N)) continue;
+            store(m, s, up);
+            if constexpr (AGAIN) again |= __builtin_isfinite(s) && __builtin_isfinite(up) ? 0u : 1u << i;
+        }
+        for (; AGAIN && again; again &= again - 1) {
+            const int m = grp * MT + __builtin_ctz(again);
+            using ET = typename std::conditional<F32, float, AT>::type;
+            const ET *row = (const ET *)x + (int64_t)m * K;
+            if constexpr (MOE == 0) {
+                store(m, dot_fp32<QT, ROWS>(row, w, n, K), 0.0f);
+            } else if constexpr (MOE == 1) {
+                const int e = moe_id(ids, ids64, blockIdx.y, n_exp).clamped;
+                store(m, dot_fp32<QT, false>(row, ((const uint8_t *const *)w)[e], n, K),
+                      dot_fp32<QT, false>(row, ((const uint8_t *const *)w2)[e], n, K));
+            } else {
+                float s = 0.0f;
+                for (int slot = 0; slot < slots; slot++) {
+                    const int pair = blockIdx.y * slots + slot;
+                    const MoeId id = moe_id(ids, ids64, pair, n_exp);
+                    if (ids64 && !id.valid) continue;
+                    s += load_route_w(route_w, route_dtype, pair) *
+                         dot_fp32<QT, false>(row + (int64_t)slot * ge * TILE_COLS, ((const uint8_t *const *)w)[id.clamped], n,
+                                             (int64_t)ge * TILE_COLS);
+                }
+                store(m, s, 0.0f);
             }
         }
     }

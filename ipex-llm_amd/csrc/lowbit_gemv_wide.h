@@ -65,16 +65,13 @@ __global__ __launch_bounds__(64 * wide_max_waves(MB, DUAL ? 2 * R : R, F32)) voi
     const int u = lane & 15, xrow = lane >> 4;
     auto load = [&](int g, u32x4 (&xv)[F32 ? 2 * XC : XC], auto &t) __attribute__((always_inline)) {
         const int col = g * TILE_COLS + u * 8;
-        const bool past = ROWS && col >= K;                  // columns past K read as zero
+        const bool past = ROWS && col >= K;                  // (put makes zeros of columns past K)
 #pragma unroll
         for (int i = 0; i < XC; i++) {
             const int m = i * 4 + xrow;
             const u32x4 *p = (const u32x4 *)(x + (int64_t)(m < M ? m : M - 1) * K + (past ? K - 8 : col));
 #pragma unroll
-            for (int h = 0; h < (F32 ? 2 : 1); h++) {
-                xv[i * (F32 ? 2 : 1) + h] = p[h];
-                if constexpr (ROWS) xv[i * (F32 ? 2 : 1) + h] = past ? u32x4{0u, 0u, 0u, 0u} : p[h];
-            }
+            for (int h = 0; h < (F32 ? 2 : 1); h++) xv[i * (F32 ? 2 : 1) + h] = p[h];
         }
 #pragma unroll
         for (int wi = 0; wi < NT; wi++) {
@@ -84,7 +81,10 @@ __global__ __launch_bounds__(64 * wide_max_waves(MB, DUAL ? 2 * R : R, F32)) voi
     };
     // Unit v (16 bytes) of row m lies at unit v ^ m % 16: the rows are 256 bytes apart, and a step reads one unit of 16 of
     // them at a time.
-    auto put = [&](const u32x4 (&xv)[F32 ? 2 * XC : XC]) __attribute__((always_inline)) {
+    auto put = [&](int g, const u32x4 (&xv)[F32 ? 2 * XC : XC]) __attribute__((always_inline)) {
+        // (here and not where they are loaded: there the select would wait for the loads, in front of the previous group)
+        const bool past = ROWS && g * TILE_COLS + u * 8 >= K;
+        const u32x4 none = {0u, 0u, 0u, 0u};
 #pragma unroll
         for (int i = 0; i < XC; i++) {
             const int m = i * 4 + xrow;
@@ -94,11 +94,11 @@ __global__ __launch_bounds__(64 * wide_max_waves(MB, DUAL ? 2 * R : R, F32)) voi
             };
             if constexpr (F32) {
                 u32x4 hi, lo;
-                split_f32(xv[2 * i], xv[2 * i + 1], hi, lo);
+                split_f32(past ? none : xv[2 * i], past ? none : xv[2 * i + 1], hi, lo);
                 one(xs + m * 256, hi);
                 one(xs + PLANE + m * 256, lo);
             } else {
-                one(xs + m * 256, xv[i]);
+                one(xs + m * 256, past ? none : xv[i]);
             }
         }
     };
@@ -122,7 +122,7 @@ __global__ __launch_bounds__(64 * wide_max_waves(MB, DUAL ? 2 * R : R, F32)) voi
         // the LDS part is private to the wave, whose LDS operations execute in order: a fence for the compiler is enough
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
         __builtin_amdgcn_wave_barrier();
-        put(xv);
+        put(g, xv);
         if (g + W < G) load(g + W, xv, wn);
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
         __builtin_amdgcn_wave_barrier();
@@ -191,14 +191,24 @@ __global__ __launch_bounds__(64 * wide_max_waves(MB, DUAL ? 2 * R : R, F32)) voi
         const int64_t n = ((int64_t)blockIdx.x * R + wi) * TILE_ROWS + r;
         if (n >= N) continue;
         const float bv = bias_ ? (float)((const ET *)bias_)[n] : 0.0f;
+        auto store = [&](int m, float s, float up) __attribute__((always_inline)) {
+            const float v = DUAL ? gate_act(s, act) * up : s + bv;
+            if constexpr (F32) ((float *)y_)[(int64_t)m * N + n] = v;
+            else ((AT *)y_)[(int64_t)m * N + n] = to_at<AT>(v);
+        };
+        uint32_t again = 0;                                   // results that are not finite, see dot_fp32
 #pragma unroll
         for (int i = 0; i < 4; i++) {
             const int m = mb * 16 + c * 4 + i;
             if (m < M) {
-                const float v = DUAL ? gate_act(s[i], act) * up[i] : s[i] + bv;
-                if constexpr (F32) ((float *)y_)[(int64_t)m * N + n] = v;
-                else ((AT *)y_)[(int64_t)m * N + n] = to_at<AT>(v);
+                store(m, s[i], up[i]);
+                again |= __builtin_isfinite(s[i]) && __builtin_isfinite(up[i]) ? 0u : 1u << i;
             }
+        }
+        for (; again; again &= again - 1) {
+            const int m = mb * 16 + c * 4 + __builtin_ctz(again);
+            const ET *row = x + (int64_t)m * K;
+            store(m, dot_fp32<QT, ROWS>(row, w, n, K), DUAL ? dot_fp32<QT, ROWS>(row, w_up, n, K) : 0.0f);
         }
     }
 }

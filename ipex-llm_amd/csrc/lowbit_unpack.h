@@ -266,6 +266,47 @@ __device__ inline void split_f32(const u32x4 &a, const u32x4 &b, u32x4 &hi, u32x
     lo = __builtin_bit_cast(u32x4, l);
 }
 
+// ---- results that are not finite
+//
+// The kernels multiply activations by codes and apply scale, minimum and the parts of a value afterwards.  An infinity among
+// the activations then meets a code of zero whose weight is not zero, terms d * inf and e * inf of opposite signs, or parts
+// of opposite signs: NaN, where the weight times it is a signed infinity.  (And sums of codes can overflow where the weights'
+// do not.)  So a kernel computes a result that is not finite once more: x's row times weights decoded to fp32, column by
+// column.  A test per result; time goes only into calls that have one.  weights: row n of w is meant.
+template <int QT, bool ROWS, typename ET>
+__device__ inline float dot_fp32(const ET *x, const uint8_t *w, int64_t n, int64_t K) {
+    using F = Fmt<QT>;
+    float sum = 0.0f;
+    for (int64_t sb = 0; sb < K / 32 && sum == sum; sb++) {       // (32 columns of one block)
+        const uint8_t *codes, *hdr;
+        const int part = (int)(sb % (F::QK / 32)), r = (int)(n % TILE_ROWS), j = (int)(sb % 4);
+        if constexpr (ROWS) {
+            hdr = w + (n * (K / F::QK) + sb / (F::QK / 32)) * F::TS;
+            codes = hdr + F::HDR;
+        } else {
+            const uint8_t *tile = w + tile_offset<QT>(n, K, (int)sb);
+            hdr = tile + tile_hdr_offset<QT>(r, j);
+            codes = tile + (F::BITS == 4 ? j * 4 : j / 2 * 1024 + j % 2 * 8) + r * 16;
+        }
+        uint32_t h = *(const uint16_t *)hdr;
+        if constexpr (F::HDR == 4) h |= (uint32_t)((const uint16_t *)hdr)[1] << 16;
+        float d, m;
+        hdr_to_scale<QT>(h, d, m);
+#pragma unroll 4
+        for (int i = 0; i < 32; i++) {
+            uint32_t c;
+            if constexpr (!ROWS) {                                // column group i / 8 of the tile, see lowbit_formats.h
+                const int nibble = (i & 1) * 4 + (i % 8 >> 1);
+                c = F::BITS == 8 ? codes[i / 8 * 256 + i % 8] : codes[i / 8 * 256 + nibble / 2] >> nibble % 2 * 4;
+            } else if constexpr (F::BITS == 8) c = codes[part * 32 + i];
+            else if constexpr (QT == QT_NF4) c = codes[i] >> part * 4;
+            else c = codes[i % 16] >> i / 16 * 4;
+            sum = fmaf((float)x[sb * 32 + i], decode<QT>(F::BITS == 4 ? c & 15u : c, d, m), sum);
+        }
+    }
+    return sum;
+}
+
 // activation of the gate branch: 0 = SiLU, 1 = GELU in its tanh form (what Gemma uses)
 __device__ inline float gate_act(float g, int act) {
     if (act == 0) return g / (1.0f + __expf(-g));

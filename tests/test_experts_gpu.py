@@ -4,7 +4,7 @@ import torch
 from torch import nn
 
 from ipex_llm.ggml.quantize import ggml_tensor_qtype as Q
-from ipex_llm.transformers.low_bit_linear import FP4Params, LowBitLinear
+from ipex_llm.transformers.low_bit_linear import FP4Params, LowBitLinear, dequant
 from ipex_llm.transformers.native_ops import ops
 from ipex_llm.transformers.moe import ExpertWeights, LowBitExperts, moe_ffn_grouped, moe_ffn_reference, route_top_k
 
@@ -178,3 +178,23 @@ def test_routing_weights_get_their_gradient():
     with torch.autograd.forward_ad.dual_level():
         dual = torch.autograd.forward_ad.make_dual(weight.detach(), torch.ones_like(weight))
         assert torch.autograd.forward_ad.unpack_dual(block(x, index, dual)).tangent is not None
+
+
+@pytest.mark.parametrize("qname", ["sym_int4", "asym_int4", "nf4", "sym_int8"])
+@pytest.mark.parametrize("tokens", [1, 3])
+def test_an_activation_that_overflows_meets_the_weights(qname, tokens):
+    """One of an expert's intermediate values is beyond fp16: its column of the down weights decides what the results are."""
+    torch.manual_seed(9)
+    block = _block(4, 128, 256, Q[qname])
+    for layers in (block.gate, block.up):
+        for layer in layers:
+            w = torch.rand(256, 128, device="cuda") * 0.02
+            w[17] = 5.0
+            layer._parameters["weight"] = FP4Params(w, qtype=Q[qname]).to("cuda")
+    x = torch.rand(tokens, 128, device="cuda").half() + 1                         # gate and up are 900 and more there, 3 at most elsewhere
+    index, weight = torch.arange(tokens, device="cuda")[:, None], torch.full((tokens, 1), 0.5, device="cuda")
+    y = block(x, index, weight).float().cpu()
+    for t in range(tokens):
+        down = block.down[t].weight
+        col = dequant(torch.empty(0, device="cuda"), down.data, Q[qname], shape=(128, 256)).view(128, 256)[:, 17].cpu()
+        assert torch.equal(y[t].isnan(), col == 0) and torch.equal(y[t] == float("inf"), col > 0) and torch.equal(y[t] == -float("inf"), col < 0)

@@ -8,7 +8,7 @@ import lowbit_oracle as orc
 from gpu_util import ALL, FP8, acts, dev_quantize, weights
 from ipex_llm.transformers.low_bit_linear import mlp_forward_xpu
 from ipex_llm.transformers.models.utils import SILU
-from test_linear_gpu import GGML, TILED, _check
+from test_linear_gpu import GGML, TILED, _check, classes
 
 pytestmark = pytest.mark.gpu
 
@@ -48,3 +48,17 @@ def test_fused_gate_up(qtype, m, n, k):
     g, u = (orc.mul_mat_exact(orc.quantize(w, qtype), x.float().numpy(), (n, k), qtype) for w in (wg, wu))
     want = g / (1.0 + np.exp(-g)) * u
     assert np.abs(y - want).max() <= (2e-3 if dtype == torch.float16 else 8e-3) * np.abs(want).max()
+
+
+@pytest.mark.parametrize("qtype", ALL)
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("m,n,k", [(9, 48, 256), (24, 4112, 128), (64, 48, 256)])
+def test_fused_gate_up_with_infinities(qtype, dtype, m, n, k):
+    wg, wu, x = weights(m, (n, k)), weights(m + 1, (n, k)), acts(m, m, k, dtype)
+    x[0, 5], x[m // 2, k - 3] = float("inf"), -float("inf")
+    y = mlp_forward_xpu(x.cuda(), dev_quantize(wg, qtype, TILED), dev_quantize(wu, qtype, TILED), m, k, n, SILU, qtype).float().cpu().numpy()
+    with np.errstate(all="ignore"):
+        g, u = (x.double().numpy() @ orc.dequantize(orc.quantize(w, qtype), qtype, (n, k)).astype(np.float64).T for w in (wg, wu))
+        want = g / (1.0 + np.exp(-g)) * u
+    assert (classes(y) == classes(want)).all()
+    assert (classes(want) > 1).any() and (classes(want) == 0).any()

@@ -88,3 +88,33 @@ def test_row_major_weights_are_as_exact_as_in_fp32(qtype, m, n, k):
     want = x.double() @ w.t()
     # an error of 7e-7 moves a result over a rounding border of bf16 (2^-9 to 2^-8 apart) in 2 * 7e-7 / 2^-9 of the cases
     assert (y != want.bfloat16()).float().mean() <= 7e-4
+
+
+def classes(t):
+    """0 finite, 1 nan, 2 +inf, 3 -inf"""
+    return np.isnan(t) * 1 + np.isposinf(t) * 2 + np.isneginf(t) * 3
+
+
+# row-major weights in every form, and tiled ones in the one-pass kernel (1 .. 4 tile rows, 16 .. 64 rows)
+@pytest.mark.parametrize("qtype", ALL)
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("m,n,k", [(1, 37, 640), (4, 8203, 192), (8, 37, 640), (8, 8203, 192), (12, 37, 192), (12, 16399, 64), (24, 37, 192), (70, 37, 192),
+                                   (333, 300, 2112), (9, 48, 256), (24, 4112, 256), (40, 8208, 128), (31, 12304, 128), (64, 48, 256)])
+def test_infinities_meet_the_weights_and_not_their_codes(qtype, dtype, m, n, k):
+    if qtype == FP8:
+        k = (k + 127) // 128 * 128
+    w, x = weights(m, (n, k)), acts(m + 1, m, k, dtype)
+    x[0, 5], x[m // 2, k - 3] = float("inf"), -float("inf")
+    if m > 2:
+        x[m - 1, 7] = float("nan")
+    if dtype != torch.float16 and m > 3:
+        x[1, 3] = 1e38                                                            # finite: its codes' sums need not be
+    layer = LowBitLinear(k, n, qtype, bias=True, conver_to_half=False).eval()
+    layer.weight = FP4Params(torch.from_numpy(w), qtype=qtype).to("cuda")
+    layer.bias = torch.nn.Parameter(torch.randn(n).to(dtype).cuda(), requires_grad=False)
+    with torch.no_grad(), np.errstate(invalid="ignore"):
+        y = layer(x.cuda()).float().cpu().numpy()
+        want = x.double().numpy() @ orc.dequantize(orc.quantize(w, qtype), qtype, (n, k)).astype(np.float64).T
+    assert (classes(y) == classes(want)).all()
+    if m > 1:
+        assert (classes(want) != 0).any() and (classes(want) == 0).any()
