@@ -57,16 +57,19 @@ static WideShape wide_shape(int qtype, int layout, int dt, int M, int N, int K) 
 // The fused gate/up form: R of either weight, so at most 2.  Against two launches' worth of streaming passes and the fused
 // form of the tiled GEMM, which has few tiles at these sizes and walks all of K in each (fp16 sym_int4 [11008 x 4096] at 12 /
 // 24 / 48 rows 18.0 -> 14.2 / 31.1 -> 19.9 / 40.9 -> 28.8 us, [4096 x 16384] at 24 rows 127 -> 26).
-static WideShape wide_mlp_shape(int qtype, int M, int N, int K) {
+static WideShape wide_mlp_shape(int qtype, int act_dtype, int M, int N, int K) {
     const int T = N / TILE_ROWS, MB = (M + 15) / 16, rounds = (T + 255) / 256;
     const WideShape none = {0, 0};
     // 5 .. 8 rows: where the streaming kernel spends more on unpacking than on memory
     if (M <= 8 && !(M > 4 && (qtype == QT_SYM_INT8 || (qtype == QT_NF4 && T >= 512)))) return none;
     if (M > 64 || (MB > 2 && T > 1024)) return none;
-    // one tile row of either weight where that takes an odd number of rounds, and with 16 rows and the formats of many
-    // registers (two of them spill); 8 waves where a CU has one workgroup, else 4
+    // One tile row of either weight where that takes an odd number of rounds, with 16 rows and the formats of many registers,
+    // and with 49 .. 64 rows where two spill (all but nf4 and fp16 sym_int4; 56 rows on [8192 x 4096], one / two: sym_int8
+    // 27.5 / 57.7 us, asym_int4 27.6 / 43.3, fp8_e4m3 26.7 / 30.6; nf4 27.7 / 25.2).  8 waves where a CU has one workgroup,
+    // else 4.
     const bool small = qtype == QT_SYM_INT4 || qtype == QT_NF4;
-    const int r = rounds == 1 || rounds == 3 || (MB == 1 && !small) ? 1 : 2;
+    const bool spills = MB == 4 && qtype != QT_NF4 && !(qtype == QT_SYM_INT4 && act_dtype == DT_F16);
+    const int r = rounds == 1 || rounds == 3 || (MB == 1 && !small) || spills ? 1 : 2;
     return {r, (T + r - 1) / r <= 256 ? 8 : 4};
 }
 
@@ -91,7 +94,7 @@ int launch_gemv_wide(const void *x, const void *w, const void *bias, void *y, in
 
 int launch_mlp_wide(const void *x, const void *wg, const void *wu, void *y, int qtype, int act_dtype, int M, int N, int K, int act,
                     hipStream_t st) {
-    const WideShape s = wide_mlp_shape(qtype, M, N, K);
+    const WideShape s = wide_mlp_shape(qtype, act_dtype, M, N, K);
     if (!s.r) return 1;
     switch (qtype) {
     case QT_SYM_INT4: return launch_wide_mlp_q<QT_SYM_INT4>(x, wg, wu, y, act_dtype, M, N, K, act, s, st);
