@@ -470,3 +470,18 @@ def test_workspace_query_with_a_budget_names_what_the_plan_uses():
                     assert ggml.lowbit_forward_plan(qtype, 1, m, n, k, need > 0, need) == (plan if need else ggml.lowbit_forward_plan(qtype, 1, m, n, k, False))
                 assert ggml.lowbit_workspace_bytes_for(qtype, 1, m, n, k, 1 << 40) <= ggml.lowbit_workspace_bytes(m, n, k)
         assert ggml.lowbit_workspace_bytes_for(qtype, 0, 512, 4096, 4096, 1 << 30) == 0      # ggml layout: any-shape kernel
+
+
+def test_linear_asks_for_a_workspace_only_where_its_kernel_uses_one():
+    """lowbit_linear takes the one-pass kernel at 17 .. 64 rows of these shapes, whatever workspace it is given; beyond, the
+    ring kernel, K splits and the row-major GEMM leave partial sums.  Host arithmetic only."""
+    def need(layout, m, n, k, dtype=ggml.DT_F16, qtype=Q["sym_int4"]):
+        return ggml.lowbit_linear_workspace_bytes(qtype, layout, dtype, m, n, k, 256 << 20)
+    tiled, rows = ggml.LAYOUT_TILED, ggml.LAYOUT_GGML
+    for m, n, k in ((17, 11008, 4096), (40, 11008, 4096), (64, 4096, 4096)):
+        assert need(tiled, m, n, k) == 0
+    assert need(tiled, 100, 4096, 4096) > 0 and need(tiled, 48, 4096, 11008) > 0        # the latter: too much x for one pass
+    assert need(rows, 40, 4001, 2112) == 0 and need(rows, 64, 1023, 1216) == 0
+    assert need(rows, 333, 3200, 8640) > 0
+    assert need(tiled, 100, 4096, 4096, ggml.DT_F32) == 0 and need(tiled, 16, 4096, 4096) == 0
+    assert need(tiled, 1 << 40, 4096, 4096) == 0 and need(tiled, 40, 4096, 4096, qtype=99) == 0
