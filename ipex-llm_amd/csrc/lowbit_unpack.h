@@ -177,21 +177,21 @@ template <> struct Unpack8<QT_FP8_E4M3, __bf16> {
 // The MFMA operand that codes become in a kernel, and what the kernel has to know about it.
 //   PARTS   16-bit operands whose sum is the code's value, one MFMA each
 //   OFFSET  constant still in the value, removed through the row sum of x (NEED_S)
-// Tiled weights with 16-bit activations: one part, the constant as Unpack has it.  F32 (float32 activations): nf4 in two.
-// ROWS (row-major weights): what was decoded to fp32 before the product has operands that keep its precision.
+// Tiled weights with 16-bit activations: one part, the constant as Unpack has it.  F32 (float32 activations) and ROWS
+// (row-major weights, which were decoded to fp32 before the product): operands that keep the result's precision.
 //   4-bit integers are centred, q - 8.  With the 128 or 136 that Unpack leaves in bf16, fp32 sums some 17 times larger
-//     cancel: float32 activations were off by 3.8e-6 of the result's norm in place of 2.5e-6, and ten times as many bf16
-//     results were not the nearest one.  asym_int4's minimum, mostly near -7.5 scales, goes with the 8, and a step's two
+//     cancel, and x's second plane loses bits beside the first one's: float32 activations were off by 3.8e-6 of the
+//     result's norm in place of 2.5e-6, and ten times as many bf16 results were not the nearest one.  asym_int4's minimum, mostly near -7.5 scales, goes with the 8, and a step's two
 //     terms meet before they go to the sum, which is then rounded once a step (fp16 results of 8640 columns that are not
 //     the nearest: 1.23 in a thousand with two FMAs, 0.98 this way, 1.05 from weights in fp32).
-//   nf4's code book has 24 mantissa bits: three parts in bf16, which hold it exactly (two were off by up to 5e-6 of an entry:
-//     3.5e-6 of the result's norm with float32 activations, 2.6 bf16 results in a thousand not the nearest one, 0.17 from
-//     weights in fp32), two in fp16 with the book scaled by 2^14, which keeps the second one clear of fp16's subnormal
-//     numbers: three of the 16 entries are then off by one in the 24th bit, the others exact.
+//   nf4's code book has 24 mantissa bits.  ROWS: three parts in bf16, which hold it exactly (two are off by up to 5e-6 of an
+//     entry: 3.5e-6 of the result's norm with float32 activations, 2.6 bf16 results in a thousand not the nearest one, 0.17
+//     from weights in fp32), two in fp16 with the book scaled by 2^14, which keeps the second one clear of fp16's subnormal
+//     numbers: three of the 16 entries are then off by one in the 24th bit, the others exact.  Tiled with F32: two parts.
 template <int QT, typename AT, bool F32, bool ROWS> struct Operand {
     using V8 = typename Vec8<AT>::type;
     static constexpr bool NF4 = QT == QT_NF4, INT4 = QT == QT_SYM_INT4 || QT == QT_ASYM_INT4;
-    static constexpr bool CENTRED = ROWS && INT4, CENTRED_BF16 = CENTRED && __is_same(AT, __bf16);
+    static constexpr bool CENTRED = INT4 && (ROWS || F32), CENTRED_BF16 = CENTRED && __is_same(AT, __bf16);
     static constexpr int PARTS = !NF4 ? 1 : ROWS ? (__is_same(AT, __bf16) ? 3 : 2) : F32 ? 2 : 1;
     static constexpr int NF4_SCALE = NF4 && ROWS && __is_same(AT, _Float16) ? 1 << 14 : 1;
     static constexpr float offset() {
@@ -219,7 +219,7 @@ template <int QT, typename AT, bool F32, bool ROWS> struct Operand {
     // sum + d * p + e * s: that times the step's product, e (see OFFSET) times the row sum of x
     __device__ static float add(float sum, float d, float p, float e, float s) {
         if constexpr (!NEED_S) return fmaf(d, p, sum);
-        else if constexpr (ROWS) return sum + fmaf(e, s, d * p);
+        else if constexpr (CENTRED) return sum + fmaf(e, s, d * p);
         else return fmaf(e, s, fmaf(d, p, sum));
     }
     // a step's product; al: what x's first plane leaves (F32).  The largest first: an MFMA drops more of a small sum that it

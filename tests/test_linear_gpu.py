@@ -5,7 +5,7 @@ import torch
 
 import ipex_llm.ggml.model.llama.llama_cpp as ggml
 import lowbit_oracle as orc
-from gpu_util import ALL, DT, FP8, acts, dev_quantize, stream, weights
+from gpu_util import ALL, DT, FP8, NF4, acts, dev_quantize, stream, weights
 from ipex_llm.transformers.low_bit_linear import FP4Params, LowBitLinear
 
 pytestmark = pytest.mark.gpu
@@ -64,8 +64,8 @@ def test_bias_of_every_kernel(qtype, dtype, m, n, k):
 ROW_MAJOR = [(1, 2000, 4160), (7, 1000, 4160), (12, 1000, 4160), (16, 16399, 1088), (30, 1000, 4160), (70, 1000, 4160), (333, 1000, 4160)]
 
 
-def _row_major(qtype, m, n, k, dtype):
-    if qtype == FP8:
+def _plain(qtype, m, n, k, dtype):
+    if qtype == FP8 and k % 128:
         n, k = n + 1, (k + 127) // 128 * 128
     w, x = weights(m, (n, k), outliers=False), acts(m + 1, m, k, dtype)
     layer = LowBitLinear(k, n, qtype, bias=False, conver_to_half=False).eval()
@@ -80,14 +80,25 @@ def _row_major(qtype, m, n, k, dtype):
 def test_row_major_weights_are_as_exact_as_in_fp32(qtype, m, n, k):
     """What is left beside the results' own rounding is that of fp32 sums: 2^-24 per step, in at most K / 32 = 136 random
     steps of at most the result's size, is 7e-7 of the norm."""
-    y, x, w = _row_major(qtype, m, n, k, torch.float32)
+    y, x, w = _plain(qtype, m, n, k, torch.float32)
     hi = x.bfloat16().double()
     want = (hi + (x.double() - hi).bfloat16().double()) @ w.t()                   # float32 activations go in as two bf16 planes
     assert (y.double() - want).norm() <= 7e-7 * want.norm()
-    y, x, w = _row_major(qtype, m, n, k, torch.bfloat16)
+    y, x, w = _plain(qtype, m, n, k, torch.bfloat16)
     want = x.double() @ w.t()
     # an error of 7e-7 moves a result over a rounding border of bf16 (2^-9 to 2^-8 apart) in 2 * 7e-7 / 2^-9 of the cases
     assert (y != want.bfloat16()).float().mean() <= 7e-4
+
+
+# streaming up to 8 rows in its shapes, the one-pass kernel beyond
+@pytest.mark.parametrize("qtype", [t for t in ALL if t != NF4])                   # (nf4: the code book in two bf16 parts)
+@pytest.mark.parametrize("m,n,k", [(1, 4096, 4096), (3, 1024, 4096), (8, 1024, 4096), (7, 8192, 1024), (12, 4096, 4096), (16, 8192, 1024),
+                                   (24, 1024, 4096), (70, 4112, 2048)])
+def test_tiled_weights_with_float32_activations_are_as_exact_as_fp32_sums(qtype, m, n, k):
+    y, x, w = _plain(qtype, m, n, k, torch.float32)
+    hi = x.bfloat16().double()
+    want = (hi + (x.double() - hi).bfloat16().double()) @ w.t()
+    assert (y.double() - want).norm() <= 7e-7 * want.norm()                       # (K / 32 = 128 steps at most, as above)
 
 
 def classes(t):
