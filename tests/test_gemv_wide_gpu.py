@@ -22,11 +22,12 @@ def test_tiled_weights(qtype, dtype, m, n, k):
 
 
 @pytest.mark.parametrize("qtype", ALL)
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("m,n,k", [(5, 4099, 192), (8, 17, 1600), (16, 8201, 128), (17, 4101, 320), (48, 8199, 64), (64, 1023, 1216), (32, 16387, 192)])
-def test_row_major_weights(qtype, m, n, k):
+def test_row_major_weights(qtype, dtype, m, n, k):
     if qtype == FP8:
         k = (k + 127) // 128 * 128
-    _check(qtype, torch.bfloat16, GGML, m, n, k, m % 2 == 0, 800 * m + n)
+    _check(qtype, dtype, GGML, m, n, k, m % 2 == 0, 800 * m + n)
 
 
 @pytest.mark.parametrize("qtype", ALL)

@@ -3,7 +3,8 @@ import pytest
 import torch
 
 from ipex_llm.ggml.quantize import ggml_tensor_qtype as Q
-from ipex_llm.transformers.low_bit_linear import FP4Params, batch_forward, forward_new
+from ipex_llm.transformers.low_bit_linear import (FP4Params, batch_forward, dequantize_rows, forward_new, mlp_forward_xpu,
+                                                  use_batch_forward)
 from ipex_llm.transformers.native_ops import ops
 
 
@@ -66,3 +67,44 @@ def test_weights_that_start_between_16_byte_boundaries(dtype, offset):
     for place in (lambda p: p.to("cuda"), lambda p: p.quantize("cpu")):
         got, want = (place(FP4Params(w, qtype=Q["sym_int4"])).data for w in (view, view.clone()))
         assert torch.equal(got, want)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("qname", ["sym_int4", "asym_int4", "sym_int8", "nf4", "fp8_e4m3"])
+@pytest.mark.parametrize("m,n,k", [(1, 64, 256), (2, 64, 128), (48, 80, 128), (49, 64, 384), (49, 80, 256), (64, 64, 256), (65, 64, 256)])
+def test_float32_batches_follow_use_batch_forward(qname, m, n, k):
+    torch.manual_seed(m + n)
+    w, x = FP4Params(torch.randn(n, k) * 0.02, qtype=Q[qname]).to("cuda"), torch.randn(m, k, device="cuda")
+    stays = m == 1 or use_batch_forward(x, Q[qname], n)
+    want = (batch_forward if stays else forward_new)(x, w.data, Q[qname], n, layout=w.blob_layout)
+    assert torch.equal(ops.linear(x, w, None, Q[qname], n, True), want)
+    assert torch.equal(ops.linear(x, w, None, Q[qname], n, False), batch_forward(x, w.data, Q[qname], n, layout=w.blob_layout))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("qname", ["sym_int4", "nf4", "fp8_e4m3"])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("m,act", [(1, 0), (6, 1), (40, 0), (70, 1)])
+def test_native_gated_equals_mlp_forward_xpu(qname, dtype, m, act):
+    torch.manual_seed(m)
+    wg, wu = (FP4Params(torch.randn(272, 256) * 0.05, qtype=Q[qname]).to("cuda") for _ in range(2))
+    x = torch.randn(1, m, 512, device="cuda").to(dtype)[..., :256]                # three dimensions, rows that are not contiguous
+    got = ops.gated(x, wg, wu, Q[qname], 272, act)
+    want = mlp_forward_xpu(x.contiguous().view(m, 256), wg.data, wu.data, m, 256, 272, act, Q[qname])
+    assert got.shape == (1, m, 272) and got.dtype == dtype and torch.equal(got[0], want)
+    assert ops.gated(x.float(), wg, wu, Q[qname], 272, act) is None
+    assert ops.gated(x, wg, FP4Params(torch.randn(272, 384), qtype=Q[qname]).to("cuda"), Q[qname], 272, act) is None
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("qname", ["sym_int4", "asym_int4", "sym_int8", "nf4", "fp8_e4m3"])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("n,k", [(48, 256), (37, 128)])
+def test_native_embedding_equals_the_python_steps(qname, dtype, n, k):
+    torch.manual_seed(n)
+    table, like = FP4Params(torch.randn(n, k), qtype=Q[qname]).to("cuda"), torch.empty(0, dtype=dtype, device="cuda")
+    ids = torch.randint(0, n, (3, 8), device="cuda")[:, ::2]
+    got = ops.embedding(ids, table, Q[qname], n, k, like)
+    want = dequantize_rows(ids.contiguous(), table.data, Q[qname], k, n, layout=table.blob_layout).to(dtype)
+    assert got.shape == (3, 4, k) and got.dtype == dtype and torch.equal(got, want)
+    assert ops.embedding(ids.int(), table, Q[qname], n, k, like) is None and ops.embedding(ids, table, Q[qname], n + 1, k, like) is None
