@@ -100,8 +100,8 @@ def main():
     ap.add_argument("--mlp-only", action="store_true",
                     help="only the gated MLP at prefill: gate and up as two launches plus the activation, and as one fused launch")
     ap.add_argument("--choice-only", action="store_true",
-                    help="only the check of the kernel choice: lowbit_forward_ws against every kernel it chooses from, "
-                         "timed on the same inputs (--choice-full: the 40 shapes the estimates were fitted on)")
+                    help="only the check of the kernel choice: lowbit_forward_ws, and lowbit_linear, against every kernel the former "
+                         "chooses from, timed on the same inputs (--choice-full: the 40 shapes the estimates were fitted on)")
     ap.add_argument("--choice-full", action="store_true")
     ap.add_argument("--moe-only", action="store_true",
                     help="run only the Mixtral expert FFN legs (fp8_e4m3, 512 tokens top-2, and one token)")
@@ -274,7 +274,8 @@ def main():
     def choice_check(full):
         """lowbit_forward_ws against every kernel it chooses from - GEMV passes, the ring kernel, narrow tiles, the
         GEMM at 1 .. 16 K splits - on the same inputs, each launch on weights it has not just read (several copies
-        per graph replay).  Reports how far the pick lies above the fastest alternative."""
+        per graph replay).  Reports how far the pick lies above the fastest alternative, and the same for lowbit_linear,
+        which converted models call and which has the one-pass kernel to choose from besides."""
         F16, BF16 = (torch.float16, ggml.DT_F16), (torch.bfloat16, ggml.DT_BF16)
         if full:
             cases = ([(2, F16, sh) for sh in ((11008, 4096), (4096, 4096), (4096, 11008), (12288, 4096), (22016, 4096), (1024, 8192),
@@ -314,6 +315,9 @@ def main():
                     return min(time_graph(g, 4, 2 if i == 0 else 0) for i in range(3)) / copies * 1e3
                 need = max(16, ggml.lowbit_workspace_bytes(m, n, k))
                 alt = {}
+                lin = ggml.lowbit_linear_workspace_bytes(qt, ggml.LAYOUT_TILED, dt, m, n, k, 256 << 20)
+                t_linear = timed(lambda b, st: ggml.lowbit_linear(x.data_ptr(), b.data_ptr(), None, y.data_ptr(), *a,
+                                                                  ws.data_ptr() if lin else None, lin, st))
                 t_pick = timed(lambda b, st: ggml.lowbit_forward_ws(x.data_ptr(), b.data_ptr(), y.data_ptr(), *a, ws.data_ptr(), need, st))
                 if m <= 128:
                     alt["gemv"] = timed(lambda b, st: ggml.lowbit_gemv(x.data_ptr(), b.data_ptr(), y.data_ptr(), *a, 0, st))
@@ -331,12 +335,16 @@ def main():
                 points.append({"qtype": qt, "act": "f16" if dt == ggml.DT_F16 else "bf16", "N": n, "K": k, "M": m,
                                "pick": names[ggml.lowbit_forward_plan(qt, ggml.LAYOUT_TILED, m, n, k, True, need)],
                                "pick_us": round(t_pick, 1), "best": best, "best_us": round(alt[best], 1),
-                               "above_best": round(t_pick / alt[best], 3)})
+                               "above_best": round(t_pick / alt[best], 3), "linear_us": round(t_linear, 1),
+                               "linear_above_best": round(t_linear / min(t_linear, alt[best]), 3)})
             del blobs
         ratios = sorted(p["above_best"] for p in points)
         return {"kernel_choice": {"points": len(points), "mean_above_best": round(sum(ratios) / len(ratios), 4),
                                   "median": ratios[len(ratios) // 2], "more_than_10_percent_above": sum(r > 1.1 for r in ratios),
                                   "worst": sorted(points, key=lambda p: -p["above_best"])[:8],
+                                  "linear_mean_above_best": round(sum(p["linear_above_best"] for p in points) / len(points), 4),
+                                  "linear_worst": sorted(points, key=lambda p: -p["linear_above_best"])[:4],
+                                  "sum_of_linear_ms": round(sum(p["linear_us"] for p in points) / 1e3, 3),
                                   "sum_of_picks_ms": round(sum(p["pick_us"] for p in points) / 1e3, 3),
                                   "sum_of_bests_ms": round(sum(p["best_us"] for p in points) / 1e3, 3)}}
 
@@ -622,7 +630,7 @@ def main():
             extra["sweep_merged_qkv_fused_mlp"] = hbm(sweep_bytes(args.m), ms7, launches_per_step=4 * N_LAYERS,
                                                       note="what a converted Llama runs per token: qkv_proj, o_proj, "
                                                            "mlp_forward_xpu, down_proj")
-        # the same four launches per layer at M = 4 / 8 (lowbit_mlp_forward fuses gate and up at up to 16 rows)
+        # the same four launches per layer at M = 4 / 8 (lowbit_mlp_forward fuses gate and up)
         for m in (4, 8):
             if m == args.m:
                 continue
