@@ -143,7 +143,8 @@ int lowbit_forward(const void *x, const void *w, void *y, int qtype, int layout,
                    int64_t N, int64_t K, void *stream);
 /* Which kernel lowbit_forward (have_workspace = 0) or lowbit_forward_ws (a non-null workspace of
  * workspace_bytes) runs for a shape with an 8-byte aligned y, without running anything: the streaming GEMV in 16-row passes, the ring kernel for batch
- * sizes, or the MFMA GEMM with or without a K split or in narrow tiles.  Negative for an unknown qtype.  Host arithmetic only. */
+ * sizes, or the MFMA GEMM with or without a K split or in narrow tiles.  Negative for an unknown qtype.  Host arithmetic only.
+ * (Not lowbit_linear, which is freer to choose, see there.) */
 #define LOWBIT_PLAN_GEMV 0
 #define LOWBIT_PLAN_RING 1
 #define LOWBIT_PLAN_GEMM 2
@@ -231,7 +232,9 @@ int lowbit_forward_f32(const float *x, const void *w, float *y, int qtype, int l
 
 /* One linear layer: y = x * dequant(w)^T + bias.  x, bias ([N], may be null) and y are of `dtype`, which may be
  * LOWBIT_DT_F32: then as lowbit_forward_f32, and no workspace is used.  With 16-bit activations as lowbit_forward_ws
- * (lowbit_linear_workspace_bytes says what to pass within a budget; null is valid), the bias added to the fp32 sums before the one
+ * (lowbit_linear_workspace_bytes says what to pass within a budget; null is valid), but for two choices that the other entry
+ * points, whose kernel a caller may rely on, do not make: the one-pass kernel at 9 .. 64 rows in place of the ring kernel, a K
+ * split or several streaming passes, and narrow tiles for nf4 more often.  The bias is added to the fp32 sums before the one
  * rounding (a bias that is not 8-byte aligned is valid and slower above 16 rows).  What LowBitLinear.forward computes
  * (low_bit_linear.py:657-687 of the reference). */
 int lowbit_linear(const void *x, const void *w, const void *bias, void *y, int qtype, int layout, int dtype, int64_t M,

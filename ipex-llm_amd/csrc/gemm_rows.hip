@@ -7,9 +7,10 @@
 //
 // The operands are those of lowbit_rows.h: exact codes, and the block scale applied to the fp32 result of each
 // v_mfma_f32_16x16x32, so nothing of a weight is rounded to 16 bits.  That scale is what bounds it: one FMA per result
-// and 32 columns is as much vector time as the MFMA takes matrix time, and unpacking adds to it - the reason for many
-// rows of x per unpacked weight (MB = 8) where M allows.  333 rows on [3200 x 8640] sym_int4: 272 us as 21 streaming
-// passes, 52 us here (357 TFLOP/s).
+// and 32 columns (asym_int4: three operations) is as much vector time as the MFMA takes matrix time, and unpacking adds to
+// it - the reason for many rows of x per unpacked weight (MB = 8) where M allows.  333 rows on [3200 x 8640], 272 us as 21
+// streaming passes in sym_int4: 51.6 us with the reduction (357 TFLOP/s) in sym_int4, 67 in asym_int4, 70 (fp16) and 85
+// (bf16, three MFMAs per step) in nf4, 55 in sym_int8, 49 in fp8_e4m3 ([3201 x 8704]).
 #include "lowbit_mfma.h"
 #include "lowbit_rows.h"
 #include "lowbit_unpack.h"

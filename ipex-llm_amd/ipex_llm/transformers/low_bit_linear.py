@@ -108,9 +108,6 @@ def ggml_convert_qtype(tensor: torch.Tensor, qtype: int,
     for a GPU destination).  A CUDA source is quantized where it is; a CPU source is staged
     through the GPU.
     """
-    QK = ggml.ggml_qk_size(qtype)
-    invalidInputError(QK > 0, f"qtype {qtype} has no MI355X kernel in this build "
-                              "(supported: sym_int4, asym_int4, sym_int8, nf4, fp8_e4m3)")
     invalidInputError(tensor.dtype == torch.float, "Input tensor must be float32")
     return _pack(tensor, qtype, device, convert_shape_only, imatrix, enable_scale_search, layout)
 
@@ -236,8 +233,9 @@ def use_batch_forward(x: torch.Tensor, qtype: int, output_len: int):
     48 rows - 64 when K is a multiple of 256 and the output length one of 64 - and more than one row.  What differs
     between the two branches here is what it is in the reference: batch_forward takes x in the dtype it has (a
     float32 x stays float32), forward_new at more than one row computes in half precision.  The kernels behind
-    both are chosen by the row count alone (up to 16 rows one pass of the streaming kernel, then the ring kernel,
-    then the tiled GEMM)."""
+    both are the same, chosen by layout, rows, shape and format (lowbit_linear: the streaming kernel for a few
+    rows, the one-pass kernel up to 64, then the ring kernel and the GEMMs).  csrc/torch_ops.cpp holds the same rule
+    (batch_stays_f32) for the native call."""
     batch_size = x.shape[0]
     hard_condition = (
         x.dtype in (torch.float, torch.half)
@@ -331,8 +329,9 @@ def dequantize_rows(x: torch.Tensor, w: torch.Tensor, qtype: int, state_size: in
 def mlp_forward_xpu(x: torch.Tensor, weight1: torch.Tensor, weight2: torch.Tensor, batch_size: int,
                     state_size: int, output_size: int, act_type: int, qtype: int):
     """xe_linear.mlp_forward_xpu (models/common.py:152-156, xpu_ops.py:34-37):
-    act(x @ W1^T) * (x @ W2^T) in one launch; act_type 0 = SiLU, 1 = GELU (tanh form).  Any number of rows:
-    up to 16 run the streaming kernel, more the fused gate/up form of the tiled GEMM (made for prefill batches)."""
+    act(x @ W1^T) * (x @ W2^T) in one launch; act_type 0 = SiLU, 1 = GELU (tanh form).  Any number of rows: up to 64
+    (32 for weights of more than 16384 rows) one pass over both weights, by the streaming kernel up to 8 rows and by the
+    one-pass kernel beyond, more the fused gate/up form of the tiled GEMM (made for prefill batches)."""
     invalidInputError(x.dim() == 2 and x.shape == (batch_size, state_size) and x.device.type == _ACCEL,
                       "mlp_forward_xpu expects x of shape [batch_size, state_size] on the GPU")
     invalidInputError(ggml.lowbit_tileable(qtype, output_size, state_size),

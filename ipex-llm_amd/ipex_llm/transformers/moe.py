@@ -3,9 +3,11 @@
 The reference has no fused path for a Mixtral-style block at prefill: the Hugging Face block
 loops over the experts and calls each expert's (converted) LowBitLinear on the rows routed to
 it, then index_adds the weighted result (the same pattern as the reference's own
-transformers/models/qwen2_moe.py:375-430).  `moe_ffn_reference` is that loop;
-`moe_ffn_grouped` computes the same thing with two grouped launches over the rows sorted by expert:
-the fused gate/up projection with the activation in its epilogue, then the down projection.
+transformers/models/qwen2_moe.py:375-430).  `moe_ffn_reference` is that loop; `moe_ffn_grouped` and
+`LowBitExperts` compute the same thing in one native call (csrc/moe.hip): the (token, expert) pairs sorted by
+expert, the fused gate/up projection with the activation in its epilogue, the down projection and the weighted
+sum - or, while there are no more pairs than experts, two launches of the streaming kernel.  What that call does
+not take runs as torch operators around the two grouped launches (`_grouped_steps`).
 """
 import array
 
@@ -212,8 +214,9 @@ class LowBitExperts(nn.Module):
     `experts(hidden_states [T, H], top_k_index [T, k], top_k_weights [T, k]) -> [T, H]` (MixtralExperts and its
     siblings).  This module takes that one's place: each expert's three weights become LowBitLinear layers
     (`gate[e]`, `up[e]`, `down[e]`, so that save_low_bit / load_low_bit carry them like any other), and on the GPU the
-    call is one native call (csrc/moe.hip): two grouped launches over the (token, expert) pairs sorted by expert, or, for
-    few pairs, the streaming kernel.  Anywhere else it is the per-expert loop over the LowBitLinear layers."""
+    call is one native call (see the head of this file).  With anything else - host tensors, float32 activations,
+    training, an activation the kernels do not know, shapes without a tiled layout - it is the per-expert loop over the
+    LowBitLinear layers."""
 
     def __init__(self, num_experts, hidden_dim, intermediate_dim, qtype, act_fn, enable_scale_search=False):
         super().__init__()
