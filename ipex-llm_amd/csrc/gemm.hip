@@ -228,15 +228,37 @@ bool narrow_halves(int M, int N) {
     return M > GM / 2 && tiles * 2 <= 256;
 }
 
+static int64_t narrow_workgroups(int M, int N) {
+    const int64_t tiles = (int64_t)((M + GM - 1) / GM) * ((N + GN / 2 - 1) / (GN / 2));
+    return narrow_halves(M, N) ? 2 * tiles : tiles;
+}
+
+// Whether a launch of narrow tiles takes two groups of waves per workgroup, each on one half of K (KS in the kernel): as
+// long as a CU has one workgroup and K eight steps.  One wave per SIMD cannot cover its own loads and dequantization; two
+// workgroups per CU do that for each other, and there the form loses what its sums cost at the end.  One group / two:
+// [2048 x 2048] at M = 256 16.4 / 13.6 us in sym_int4 fp16, 17.8 / 15.0 in nf4 bf16, [4096 x 4096] at M = 512 31.4 / 27.3
+// and 36.0 / 29.7, [12288 x 4096] at M = 256 40.1 / 33.7 and 42.2 / 37.6; [1024 x 1024], eight steps, at M = 128 / 512
+// 8.5 / 8.1 and 10.3 / 9.4; 344 workgroups ([11008 x 4096] at M = 512) 56.0 / 65.2.
+static bool narrow_two_groups(int M, int N, int K) { return narrow_workgroups(M, N) <= 256 && K / TILE_COLS >= 8; }
+
 // Estimated run time in microseconds of the narrow form, fitted like gemm_time_us (760 launches, 8.5 % rms): a
 // 128-column step takes a workgroup 1.05 us up to 128 workgroups, 1.24 at one per CU, 1.55 - 1.96 once two share a
 // CU; half tiles 0.87 of it.  nf4 1.06 with its lookups in registers (80 points, 8 shapes: the choice made with it is
 // 1.5 % above the faster of this form and the rest on average; 14 % at worst, [8192 x 8192] at M = 1300);
 // the entry points whose choices lowbit_forward_plan reports keep the figure from before, 1.24.
+// Two groups of waves (lowbit_linear's estimate only): 888 launches, 6.8 % rms; a pair of steps takes 1.49 us, a million
+// weights 0.12 us; scaled by 0.91, with which the shortest estimate is 1.2 % above the fastest kernel on average (600
+// points, ten shapes, 40 .. 1024 rows; 22 % at worst, nf4 [8192 x 8192] at 72 rows).
 double narrow_time_us(int M, int N, int K, int qtype, bool linear) {
     const int tiles_m = (M + GM - 1) / GM;
     const bool halves = narrow_halves(M, N);
-    const double wgs = (double)tiles_m * (double)((N + GN / 2 - 1) / (GN / 2)) * (halves ? 2.0 : 1.0);
+    const double wgs = (double)narrow_workgroups(M, N);
+    if (linear && narrow_two_groups(M, N, K)) {
+        const double format = qtype == QT_NF4 ? 1.12 : qtype == QT_SYM_INT8 ? 1.16 : qtype == QT_FP8_E4M3 ? 1.14 : 1.0;
+        const double over128 = wgs > 128.0 ? (wgs - 128.0) / 128.0 : 0.0, fill = (double)M / ((double)tiles_m * GM);
+        return 0.91 * (3.86 + 0.97 * over128 + 0.123e-6 * (double)N * (double)K +
+                       (double)((K / TILE_COLS + 1) / 2) * 1.485 * format * (1.0 + 0.17 * over128) * (halves ? 0.79 : 1.0) * (0.69 + 0.31 * fill));
+    }
     const double format = qtype == QT_NF4 ? (linear ? 1.06 : 1.24) : qtype == QT_SYM_INT8 ? 1.11 : qtype == QT_FP8_E4M3 ? 1.05 : 1.0;
     const double over128 = wgs > 128.0 ? (wgs - 128.0) / 128.0 : 0.0;
     const double step = wgs <= 256.0 ? 1.05 + 0.20 * over128 : 1.55 + 0.41 * ((wgs < 512.0 ? wgs : 512.0) - 256.0) / 256.0;
@@ -256,8 +278,12 @@ static int launch_gemm_narrow_t(const void *x, const void *w, const void *bias, 
     ga.bias = bias;
     ga.split_tail = halves ? (int)(((int64_t)tiles_m * tiles_n) / 8) + 1 : 0;
     dim3 grid(8 * (unsigned)(((int64_t)tiles_m * tiles_n + 7) / 8 + ga.split_tail), 1);
-    hipLaunchKernelGGL((gemm_mfma_kernel<QT, AT, true, MB32, false, false, 4, true>), grid, dim3(256), 0, st, (const AT *)x,
+    if (narrow_two_groups(M, N, K))
+        hipLaunchKernelGGL((gemm_mfma_kernel<QT, AT, true, MB32, false, false, 4, true, 2>), grid, dim3(512), 0, st, (const AT *)x,
                        (const uint8_t *)w, (AT *)y, M, N, K, band_rows(tiles_m), ga, G, (float *)nullptr, 0, tiles_n);
+    else
+        hipLaunchKernelGGL((gemm_mfma_kernel<QT, AT, true, MB32, false, false, 4, true>), grid, dim3(256), 0, st, (const AT *)x,
+                           (const uint8_t *)w, (AT *)y, M, N, K, band_rows(tiles_m), ga, G, (float *)nullptr, 0, tiles_n);
     return 0;
 }
 

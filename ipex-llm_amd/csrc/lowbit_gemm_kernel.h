@@ -201,8 +201,11 @@ __device__ inline float gemm_gate_act(float g, int act) {
 // NARROW (dense 128-row DMA form only): 128 weight rows per workgroup instead of 256, one 32-row block per wave -
 // twice the workgroups for a product whose 256-column tiles leave compute units idle, without the partial sums
 // of a K split.
-template <int QT, typename AT, bool DMA, int MB, bool GROUPED = false, bool DUAL = false, int WAVES = 4, bool NARROW = false>
-__global__ __launch_bounds__(64 * WAVES, (DMA && MB == 4) ? 2 : 1) void gemm_mfma_kernel(const AT *__restrict__ x, const uint8_t *__restrict__ w,
+// KS == 2 (narrow form only): two groups of WAVES waves on the same tile, each with its own x buffers and accumulators, the
+// first on the first half of the K steps, the second on the rest; `meet` adds their sums.  Two waves per SIMD cover each
+// other's waits and dequantization where the tiles of a product are no more than one per CU (narrow_two_groups).
+template <int QT, typename AT, bool DMA, int MB, bool GROUPED = false, bool DUAL = false, int WAVES = 4, bool NARROW = false, int KS = 1>
+__global__ __launch_bounds__(64 * WAVES * KS, (DMA && MB == 4) ? 2 : 1) void gemm_mfma_kernel(const AT *__restrict__ x, const uint8_t *__restrict__ w,
                                                         AT *__restrict__ y, int M, int N, int K, int band_m,
                                                         const GroupArgs ga, int k_steps,
                                                         float *__restrict__ ws, int tn0, int tn_cnt) {
@@ -212,12 +215,15 @@ __global__ __launch_bounds__(64 * WAVES, (DMA && MB == 4) ? 2 : 1) void gemm_mfm
     static_assert(!DUAL || (GROUPED && MB == 8), "the fused gate/up form exists for grouped launches of the tall form");
     static_assert(WAVES == 4 || (WAVES == 8 && MB == 8 && DMA), "eight waves: tall form only");
     static_assert(!NARROW || (DMA && MB == 4 && WAVES == 4 && !GROUPED && !DUAL), "the narrow tile is a dense 128-row DMA form");
+    static_assert(KS == 1 || (KS == 2 && NARROW), "two groups of waves: the narrow tile");
     constexpr int MB32 = MB, GM = 32 * MB;            // shadow the 128-row constants of the file
     constexpr int GN = NARROW ? lowbit::GN / 2 : lowbit::GN;
     constexpr int NB32 = GN / WAVES / 32;             // 32-row weight blocks per wave: 2, or 1 with eight waves or a narrow tile
     // x block of a K step: 8 * MB32 pieces of 1 KiB (layout below), double buffered
-    __shared__ __attribute__((aligned(16))) uint8_t xs[2 * 8 * MB32 * 1024];
-    uint8_t *const xs0 = xs, *const xs1 = xs + 8 * MB32 * 1024;
+    __shared__ __attribute__((aligned(16))) uint8_t xs[KS * 2 * 8 * MB32 * 1024];
+    const int wave_wg = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);        // uniform: scalar address arithmetic
+    const int half_k = KS == 2 ? wave_wg / WAVES : 0, wave = KS == 2 ? wave_wg % WAVES : wave_wg;
+    uint8_t *const xs0 = xs + half_k * (2 * 8 * MB32 * 1024), *const xs1 = xs0 + 8 * MB32 * 1024;
     __shared__ float lut[16];
     // nf4 weights by lookup in registers (Nf4Scaled): the tall forms and the narrow one, which have the registers
     constexpr bool NF4REG = QT == QT_NF4 && (MB32 == 8 || NARROW);
@@ -226,7 +232,6 @@ __global__ __launch_bounds__(64 * WAVES, (DMA && MB == 4) ? 2 : 1) void gemm_mfm
     }
 
     const int lane = threadIdx.x & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);   // uniform: scalar address arithmetic
     const int G = K / TILE_COLS;
     const int n_tiles = N / TILE_ROWS;
 
@@ -362,8 +367,12 @@ __global__ __launch_bounds__(64 * WAVES, (DMA && MB == 4) ? 2 : 1) void gemm_mfm
     // Split-K: with a workspace the grid has a second dimension, workgroup (t, s) walks the K steps
     // s * k_steps .. and leaves its fp32 partial tile in ws[s]; a second kernel sums the splits.  It
     // fills the machine when the output alone has too few tiles (small M, narrow N).
-    const int kt0 = ws ? blockIdx.y * k_steps : 0;
-    const int Gs = ws ? (k_steps < G - kt0 ? k_steps : G - kt0) : G;
+    const int kt_wg = ws ? blockIdx.y * k_steps : 0;
+    const int Gs_wg = ws ? (k_steps < G - kt_wg ? k_steps : G - kt_wg) : G;
+    // KS == 2: the first group of waves walks the first half of the steps (one more where their number is odd)
+    const int Gs_first = KS == 2 ? (Gs_wg + 1) / 2 : Gs_wg;
+    const int kt0 = half_k ? kt_wg + Gs_first : kt_wg;
+    const int Gs = half_k ? Gs_wg - Gs_first : Gs_first;
     const int last = Gs - 1;
     // the same loads one at a time, for spreading them over a step: a burst of 8 + 6 loads per wave,
     // from eight waves at once, queues up at the CU's address unit and the waves stand still meanwhile
@@ -781,8 +790,9 @@ __global__ __launch_bounds__(64 * WAVES, (DMA && MB == 4) ? 2 : 1) void gemm_mfm
     typedef std::integral_constant<int, MB32> full_t;
     auto nothing = [](int, int) __attribute__((always_inline)) {};
 
-    auto epilogue = [&](auto &acc, auto mbc_) __attribute__((always_inline)) {
-        constexpr int MBC = decltype(mbc_)::value;
+    // for the 32-row blocks MB0 .. MBC - 1
+    auto epilogue = [&](auto &acc, auto mb0_, auto mbc_) __attribute__((always_inline)) {
+        constexpr int MB0 = decltype(mb0_)::value, MBC = decltype(mbc_)::value;
         // The lane's number, asked for anew: the values derived from threadIdx at the head of the kernel would
         // have to stay in registers (or, where those run out, in scratch memory with a reload inside the K loop)
         // all the way down to here.
@@ -792,7 +802,7 @@ __global__ __launch_bounds__(64 * WAVES, (DMA && MB == 4) ? 2 : 1) void gemm_mfm
     // before its result may be read; 64 are spent).  The accumulators are operands of the statement,
     // so that no read of them can be scheduled ahead of it.
 #pragma unroll
-    for (int mb = 0; mb < MBC; mb++) {
+    for (int mb = MB0; mb < MBC; mb++) {
         if constexpr (NB32 == 2)
             asm volatile("s_nop 7\n\ts_nop 7\n\ts_nop 7\n\ts_nop 7\n\ts_nop 7\n\ts_nop 7\n\ts_nop 7\n\ts_nop 7"
                          : "+a"(acc[mb][0]), "+a"(acc[mb][1]));
@@ -824,7 +834,7 @@ __global__ __launch_bounds__(64 * WAVES, (DMA && MB == 4) ? 2 : 1) void gemm_mfm
             const int64_t n_tiles_all = GROUPED ? (int64_t)gridDim.x : (int64_t)((M + GM - 1) / GM) * ((N + GN - 1) / GN);
             float *const wp = ws + ((((int64_t)blockIdx.y * n_tiles_all + tile_id) * WAVES + wave) * (MB32 * NB32 * 4)) * 256 + lane * 4;
 #pragma unroll
-            for (int mb = 0; mb < MBC; mb++) {
+            for (int mb = MB0; mb < MBC; mb++) {
 #pragma unroll
                 for (int nb = 0; nb < NB32; nb++) {
                     asm volatile("" : "+a"(acc[mb][nb]));            // (stay in accumulation registers up to here)
@@ -861,7 +871,7 @@ __global__ __launch_bounds__(64 * WAVES, (DMA && MB == 4) ? 2 : 1) void gemm_mfm
 #pragma unroll
         for (int c = 0; c < CH; c++) wpos[c] = stage + i32 * (CH * 16) + ((c ^ (i32 & (CH - 1))) * 16) + kg * 8;
 #pragma unroll
-        for (int mb = 0; mb < MBC; mb++) {
+        for (int mb = MB0; mb < MBC; mb++) {
 #pragma unroll
             for (int nb = 0; nb < (DUAL ? 1 : NB32); nb++) {
                 // (keeps the block in its accumulation registers up to here: the compiler would otherwise read
@@ -895,7 +905,7 @@ __global__ __launch_bounds__(64 * WAVES, (DMA && MB == 4) ? 2 : 1) void gemm_mfm
         AT *const yp = y + (int64_t)(m0 + row_l) * N + n;
         const uint8_t *const rpos = stage + lane * 16;
 #pragma unroll
-        for (int j0 = 0; j0 < MBC * 32 / RPI; j0 += 8) {
+        for (int j0 = MB0 * 32 / RPI; j0 < MBC * 32 / RPI; j0 += 8) {
             u32x4 v[8];
 #pragma unroll
             for (int j = j0; j < j0 + 8 && j < MBC * 32 / RPI; j++) v[j - j0] = *(const u32x4 *)(rpos + j * 1024);
@@ -906,7 +916,7 @@ __global__ __launch_bounds__(64 * WAVES, (DMA && MB == 4) ? 2 : 1) void gemm_mfm
         return;
     }
 #pragma unroll
-    for (int mb = 0; mb < MBC; mb++) {
+    for (int mb = MB0; mb < MBC; mb++) {
         const int m = m0 + mb * 32 + i32;
         if constexpr (DUAL) {
             // both blocks hold the same 32 columns of y: the gate branch in block 0, the up branch in block 1
@@ -954,6 +964,61 @@ __global__ __launch_bounds__(64 * WAVES, (DMA && MB == 4) ? 2 : 1) void gemm_mfm
             }
         }
     }
+    };
+
+    typedef std::integral_constant<int, 0> first_t;
+    // KS == 2: the two groups' sums meet in LDS.  Each group keeps one half of the row blocks, hands the other half's sums
+    // over and stores what it kept: 4 KiB per wave and block, in the x buffers of both.
+    auto meet = [&](auto &acc, auto mbc_) __attribute__((always_inline)) {
+        constexpr int MBC = decltype(mbc_)::value, KEEP = (MBC + 1) / 2;
+        typedef std::integral_constant<int, KEEP> keep_t;
+        const int lane = fresh_lane_id();
+        if (Gs < Gs_first) __syncthreads();                  // the barrier of the step that the second group has not
+#pragma unroll
+        for (int mb = 0; mb < MBC; mb++) {                   // MFMA results on their way, see the epilogue
+            if constexpr (NB32 == 2) asm volatile("s_nop 7\n\ts_nop 7\n\ts_nop 7" : "+a"(acc[mb][0]), "+a"(acc[mb][1]));
+            else asm volatile("s_nop 7\n\ts_nop 7\n\ts_nop 7" : "+a"(acc[mb][0]));
+        }
+        __syncthreads();                                     // every wave is done with its operand reads
+        f32x4 *const part = (f32x4 *)xs + wave * (MBC * NB32 * 256) + lane;
+        auto hand = [&](auto from_, auto to_) __attribute__((always_inline)) {
+#pragma unroll
+            for (int mb = decltype(from_)::value; mb < decltype(to_)::value; mb++)
+#pragma unroll
+                for (int nb = 0; nb < NB32; nb++) {
+                    asm volatile("" : "+a"(acc[mb][nb]));
+#pragma unroll
+                    for (int q = 0; q < 4; q++)
+                        part[((mb * NB32 + nb) * 4 + q) * 64] = f32x4{acc[mb][nb][q * 4], acc[mb][nb][q * 4 + 1], acc[mb][nb][q * 4 + 2], acc[mb][nb][q * 4 + 3]};
+                    __builtin_amdgcn_sched_barrier(0);       // one block at a time (register footprint)
+                }
+        };
+        auto take = [&](auto from_, auto to_) __attribute__((always_inline)) {
+#pragma unroll
+            for (int mb = decltype(from_)::value; mb < decltype(to_)::value; mb++)
+#pragma unroll
+                for (int nb = 0; nb < NB32; nb++) {
+                    asm volatile("" : "+a"(acc[mb][nb]));
+#pragma unroll
+                    for (int q = 0; q < 4; q++) {
+                        const f32x4 v = part[((mb * NB32 + nb) * 4 + q) * 64];
+#pragma unroll
+                        for (int i = 0; i < 4; i++) acc[mb][nb][q * 4 + i] += v[i];
+                    }
+                    asm volatile("" : "+a"(acc[mb][nb]));
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+        };
+        if (half_k) hand(first_t(), keep_t());
+        else hand(keep_t(), mbc_);
+        __syncthreads();
+        if (half_k) {
+            take(keep_t(), mbc_);
+            epilogue(acc, keep_t(), mbc_);
+        } else {
+            take(first_t(), keep_t());
+            epilogue(acc, first_t(), keep_t());
+        }
     };
 
     if constexpr (DMA) {
@@ -1020,7 +1085,7 @@ __global__ __launch_bounds__(64 * WAVES, (DMA && MB == 4) ? 2 : 1) void gemm_mfm
                 }
 #undef LOWBIT_DEEP_STEP
                 wait_all_loads();                   // the loads past the end (clamped re-reads) must not outlive the wave's registers
-                epilogue(acc, mbc);
+                epilogue(acc, first_t(), mbc);
                 return;
             }
             dma_x(0, xs0, mbc, xg);
@@ -1043,7 +1108,8 @@ __global__ __launch_bounds__(64 * WAVES, (DMA && MB == 4) ? 2 : 1) void gemm_mfm
             // (the compiler may move an accumulator block to other registers where the variants of the loop meet
             // and does not know that the block written last is still in the MFMA pipe: leave it the time to land)
             asm volatile("s_nop 7\n\ts_nop 7\n\ts_nop 1" : "+a"(acc[MBC - 1][NB32 - 1]));
-            epilogue(acc, mbc);
+            if constexpr (KS == 2) meet(acc, mbc);
+            else epilogue(acc, first_t(), mbc);
         };
         // tail tiles and small expert groups: 32-row blocks without rows of x skip their MFMAs
         const int mb_cnt = (M - m0 + 31) / 32;
@@ -1105,7 +1171,7 @@ __global__ __launch_bounds__(64 * WAVES, (DMA && MB == 4) ? 2 : 1) void gemm_mfm
         LOWBIT_GEMM_STEP(5, xs1, xs0, xa, xb, w2, w1)
     }
 #undef LOWBIT_GEMM_STEP
-    epilogue(acc, full_t());
+    epilogue(acc, first_t(), full_t());
     }
 }
 

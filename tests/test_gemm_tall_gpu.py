@@ -9,11 +9,11 @@ pytestmark = pytest.mark.gpu
 TILED = ggml.LAYOUT_TILED
 
 
-def check(qtype, m, n, k, dtype, gemm):
+def check(qtype, m, n, k, dtype, gemm, shift=0):
     blob = dev_quantize(weights(77, (n, k)), qtype, TILED)
     gen = torch.Generator().manual_seed(m)
     x = torch.randn((m, k), generator=gen).to(dtype).cuda()
-    y = torch.full((m + 1, n), float("nan"), dtype=dtype, device="cuda")
+    y = torch.full(((m + 1) * n + shift,), float("nan"), dtype=dtype, device="cuda")[shift:].view(m + 1, n)
     gemm(x.data_ptr(), blob.data_ptr(), y.data_ptr(), qtype, TILED, DT[dtype], m, n, k, stream())
     w = dev_dequantize(blob, qtype, n, k, TILED, torch.float32).to(dtype).float()
     want, size = x.double() @ w.double().t(), x.abs().float() @ w.abs().t()
@@ -37,6 +37,15 @@ def test_last_row_tile(qtype, m, n, k, dtype):
 def test_narrow_nf4(m, n, k, dtype):
     """Row blocks 1, 2 and 4 of the narrow tile, whose nf4 lookups are in registers."""
     check(10, m, n, k, dtype, ggml.lowbit_gemm_narrow)
+
+
+@pytest.mark.parametrize("m,n,k,shift", [(1, 16, 1024, 0), (33, 144, 1152, 4), (64, 272, 1024, 0), (65, 1040, 1152, 0), (129, 144, 1408, 4),
+                                         (250, 2048, 1152, 0), (2048, 2048, 1024, 0), (2040, 2064, 1024, 0), (100, 512, 896, 0)])
+@pytest.mark.parametrize("qtype", ALL, ids=NAMES.values())
+def test_narrow_two_groups(qtype, m, n, k, shift):
+    """Two groups of waves on one tile: 1, 2 and 4 row blocks, half tiles, an odd number of K steps, a last column tile that
+    is not full, a y off the 16-byte boundaries; 256 workgroups and 272, eight K steps and seven, where the form ends."""
+    check(qtype, m, n, k, torch.bfloat16 if n % 32 else torch.float16, ggml.lowbit_gemm_narrow, shift)
 
 
 def test_row_major_weights_of_very_long_rows():
