@@ -241,6 +241,14 @@ int lowbit_linear(const void *x, const void *w, const void *bias, void *y, int q
                   int64_t N, int64_t K, void *workspace, size_t workspace_bytes, void *stream);
 size_t lowbit_linear_workspace_bytes(int qtype, int layout, int dtype, int64_t M, int64_t N, int64_t K, size_t max_bytes);
 
+/* The gradient of lowbit_linear with respect to x: grad_x[M, K] = grad[M, N] * dequant(w)[N, K], from a tiled weight; grad and
+ * grad_x are f16 or bf16, 16-byte aligned.  Same weights (one rounding to act_dtype) and sums (fp32, one rounding) as
+ * lowbit_dequantize to act_dtype followed by a dense product, which is what the reference does
+ * (low_bit_linear.py:519-541).  lowbit_backward_applies: 1 where this is the faster of the two ways on MI355X. */
+int lowbit_backward(const void *grad, const void *w, void *grad_x, int qtype, int act_dtype, int64_t M, int64_t N, int64_t K,
+                    void *stream);
+int lowbit_backward_applies(int qtype, int layout, int act_dtype, int64_t M, int64_t N, int64_t K);
+
 /* lowbit_forward_ws without a workspace argument and without any allocation: the partial tiles go to a
  * scratch array that is part of the library's image on every GPU (lowbit_noalloc_scratch_bytes() = 64 MiB,
  * held by each GPU the library runs on until the process ends).  No counterpart in the reference; it is for

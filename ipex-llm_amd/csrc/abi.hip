@@ -43,6 +43,8 @@ int launch_gemm_narrow(const void *x, const void *w, const void *bias, void *y, 
 size_t gemm_rows_workspace_bytes(int M, int N, int K, size_t max_bytes);
 int launch_gemm_rows(const void *x, const void *w, const void *bias, void *y, int qtype, int act_dtype, int M, int N, int K,
                      void *workspace, size_t workspace_bytes, hipStream_t st);
+bool gemm_back_applies(int qtype, int M, int N, int K);
+int launch_gemm_back(const void *g, const void *w, void *gx, int qtype, int act_dtype, int M, int N, int K, hipStream_t st);
 double narrow_time_us(int M, int N, int K, int qtype, bool linear);
 int gemm_splits(int M, int N, int K, size_t ws_bytes, int qtype);
 double gemm_time_us(int M, int N, int K, int splits, int qtype);
@@ -504,6 +506,26 @@ int lowbit_dequantize_rows(const void *w, const int64_t *rows, int64_t n_rows, v
         return fail(LOWBIT_EARG, "lowbit_dequantize_rows: null or misaligned pointer");
     return check_launch(launch_dequantize_rows(w, rows, n_rows, dst, qtype, N, K, layout, out_dtype,
                                                (hipStream_t)stream), "lowbit_dequantize_rows");
+}
+
+int lowbit_backward_applies(int qtype, int layout, int act_dtype, int64_t M, int64_t N, int64_t K) {
+    if (layout != LOWBIT_LAYOUT_TILED || (act_dtype != LOWBIT_DT_F16 && act_dtype != LOWBIT_DT_BF16) || !lowbit_tileable(qtype, N, K) ||
+        M <= 0 || M > 0x7fffffff || N > 0x7fffffff || K > 0x7fffffff) return 0;
+    return gemm_back_applies(qtype, (int)M, (int)N, (int)K);
+}
+
+int lowbit_backward(const void *grad, const void *w, void *grad_x, int qtype, int act_dtype, int64_t M, int64_t N, int64_t K,
+                    void *stream) {
+    const char *what = "lowbit_backward";
+    if (int rc = check_weight_shape(what, qtype, N, K, LOWBIT_LAYOUT_TILED)) return rc;
+    if (M < 0 || M > 0x7fffffff) return fail(LOWBIT_EARG, "%s: bad M", what);
+    if (act_dtype != LOWBIT_DT_F16 && act_dtype != LOWBIT_DT_BF16)
+        return fail(LOWBIT_EDTYPE, "%s: gradients must be f16 or bf16", what);
+    if (M * K == 0) return 0;
+    if (N == 0) return fail(LOWBIT_ESHAPE, "%s: N == 0", what);
+    if (!grad || !w || !grad_x || !aligned16(grad) || !aligned16(w) || !aligned16(grad_x))
+        return fail(LOWBIT_EARG, "%s: null or misaligned pointer (16 bytes)", what);
+    return check_launch(launch_gemm_back(grad, w, grad_x, qtype, act_dtype, (int)M, (int)N, (int)K, (hipStream_t)stream), what);
 }
 
 int lowbit_mlp_forward(const void *x, const void *w_gate, const void *w_up, void *y, int qtype, int act_dtype,

@@ -211,6 +211,20 @@ _lib.lowbit_gemm_narrow.argtypes = [c_void_p, c_void_p, c_void_p, c_int, c_int, 
 _lib.lowbit_gemm_narrow.restype = c_int
 
 
+_lib.lowbit_backward.argtypes = [c_void_p, c_void_p, c_void_p, c_int, c_int, c_int64, c_int64, c_int64, c_void_p]
+_lib.lowbit_backward.restype = c_int
+_lib.lowbit_backward_applies.argtypes = [c_int, c_int, c_int, c_int64, c_int64, c_int64]
+_lib.lowbit_backward_applies.restype = c_int
+
+
+def lowbit_backward(grad, w, grad_x, qtype, act_dtype, m, n, k, stream):
+    _check(_lib.lowbit_backward(grad, w, grad_x, qtype, act_dtype, m, n, k, stream), "lowbit_backward")
+
+
+def lowbit_backward_applies(qtype, layout, act_dtype, m, n, k):
+    return bool(_lib.lowbit_backward_applies(qtype, layout, act_dtype, m, n, k))
+
+
 _lib.lowbit_forward_plan.argtypes = [c_int, c_int, c_int64, c_int64, c_int64, c_int, c_size_t]
 _lib.lowbit_forward_plan.restype = c_int
 PLAN_GEMV, PLAN_RING, PLAN_GEMM, PLAN_GEMM_SPLIT, PLAN_GEMM_NARROW = 0, 1, 2, 3, 4
