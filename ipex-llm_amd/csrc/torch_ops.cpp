@@ -12,10 +12,14 @@
 // the error.
 #include <torch/csrc/autograd/python_variable.h>
 #include <torch/csrc/Exceptions.h>
+#include <torch/csrc/autograd/function.h>
+#include <torch/csrc/autograd/functions/utils.h>
 #include <ATen/ATen.h>
 #include <c10/core/DeviceGuard.h>
 #include <c10/core/Event.h>
 #include <c10/core/GradMode.h>
+#include <c10/core/impl/LocalDispatchKeySet.h>
+#include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <c10/hip/HIPStream.h>
 
 #include <algorithm>
@@ -34,6 +38,9 @@ struct Api {
     decltype(&lowbit_linear) linear = nullptr;
     decltype(&lowbit_mlp_forward) mlp_forward = nullptr;
     decltype(&lowbit_dequantize_rows) dequantize_rows = nullptr;
+    decltype(&lowbit_dequantize) dequantize = nullptr;
+    decltype(&lowbit_backward) backward = nullptr;
+    decltype(&lowbit_backward_applies) backward_applies = nullptr;
     decltype(&lowbit_experts_workspace_bytes) experts_workspace_bytes = nullptr;
     decltype(&lowbit_experts_forward) experts_forward = nullptr;
 } api;
@@ -122,6 +129,85 @@ Tensor linear(const Tensor &x_in, const Tensor &w, const Tensor &bias, int qtype
         return y;
     }
     return product(x, w, bias, qtype, layout, M, N, K, shape);
+}
+
+// ---- training: the same product below trained parameters
+//
+// What bounded a small step was the host: a layer's forward and backward took some 110 us of Python, ctypes and the
+// interpreter lock taken in autograd's thread, around 20 us of GPU time (77 rows on [1200 x 1024]).
+
+// no transform (vmap, grad), trace or dispatch mode that wants to see the operators
+bool nothing_watches(const Tensor &t) {
+    using c10::DispatchKey;
+    const c10::DispatchKeySet on = c10::impl::tls_local_dispatch_key_set().included_;
+    if (on.has(DispatchKey::FuncTorchDynamicLayerFrontMode) || on.has(DispatchKey::Tracer) || on.has(DispatchKey::Functionalize) ||
+        c10::impl::TorchDispatchModeTLS::any_modes_set()) return false;
+    return !t.key_set().has_any(c10::DispatchKeySet({DispatchKey::Python, DispatchKey::FuncTorchBatched, DispatchKey::FuncTorchGradWrapper,
+                                                     DispatchKey::Batched, DispatchKey::Functionalize}));
+}
+
+// The gradient that flows on to x.  A node and not a torch::autograd::Function: it holds the weight as MatMulLowBit's context
+// does, as it is when the backward runs, past saved-tensor hooks and through repeated backwards.
+struct ProductBackward : public torch::autograd::Node {
+    Tensor w;
+    int qtype = 0, layout = 0;
+    int64_t N = 0, K = 0;
+    at::ScalarType dtype = at::kHalf;
+    at::DimVector x_shape;
+
+    std::string name() const override { return "MatMulLowBitBackward"; }
+
+    torch::autograd::variable_list apply(torch::autograd::variable_list &&grads) override {
+        if (!grads[0].defined() || !task_should_compute_output(0)) return {Tensor()};
+        const Tensor grad = grads[0].to(dtype).reshape({-1, N});
+        const int64_t M = grad.size(0);
+        c10::DeviceGuard guard(grad.device());
+        if (!is_blob(w, grad, qtype, N, K)) throw Failed("the low-bit weight is not where the forward found it");
+        const int dt = dtype_code(dtype);
+        void *const stream = current_stream(grad);
+        const bool tracked = (c10::GradMode::is_enabled() && grad.requires_grad()) || !nothing_watches(grad);
+        if (!tracked && api.backward_applies(qtype, layout, dt, M, N, K)) {
+            const Tensor g = grad.contiguous();
+            if ((((uintptr_t)g.const_data_ptr() | (uintptr_t)w.const_data_ptr()) & 15) == 0) {
+                Tensor gx = at::empty(x_shape, g.options());
+                check(api.backward(g.const_data_ptr(), w.const_data_ptr(), gx.data_ptr(), qtype, dt, M, N, K, stream), "lowbit_backward");
+                return {gx};
+            }
+        }
+        // (tracked: a second derivative, or a transform over the backward, goes through the dense product)
+        const Tensor dense = at::empty({N, K}, w.options().dtype(dtype));
+        check(api.dequantize(w.const_data_ptr(), dense.data_ptr(), qtype, N, K, layout, dt, stream), "lowbit_dequantize");
+        return {at::matmul(grad, dense).view(x_shape)};
+    }
+};
+
+// LowBitLinear in training on a 16-bit x that wants a gradient, where the weight and bias want none; an undefined tensor when
+// this is not the plain case
+Tensor linear_train(const Tensor &x_in, const Tensor &w, const Tensor &bias, int qtype, int64_t N) {
+    if (!on_gpu(x_in) || x_in.dim() < 1 || x_in.numel() == 0 || !x_in.requires_grad() || !c10::GradMode::is_enabled()) return {};
+    const int dt = dtype_code(x_in.scalar_type());
+    const int64_t K = x_in.size(-1), M = x_in.numel() / K;
+    if ((dt != LOWBIT_DT_F16 && dt != LOWBIT_DT_BF16) || !nothing_watches(x_in) || x_in._fw_grad(/*level=*/0).defined() ||
+        !is_blob(w, x_in, qtype, N, K) || w.requires_grad()) return {};
+    if (bias.defined() && (bias.scalar_type() != x_in.scalar_type() || bias.device() != x_in.device() || bias.numel() != N || !bias.is_contiguous() ||
+                           bias.requires_grad() || differentiable(bias))) return {};
+    Tensor y;
+    auto node = std::shared_ptr<ProductBackward>(new ProductBackward(), torch::autograd::deleteNode);
+    node->set_next_edges(torch::autograd::collect_next_edges(x_in));
+    node->w = w;
+    node->qtype = qtype;
+    node->layout = device_layout(qtype, N, K);
+    node->N = N;
+    node->K = K;
+    node->dtype = x_in.scalar_type();
+    node->x_shape.assign(x_in.sizes().begin(), x_in.sizes().end());
+    {
+        c10::AutoGradMode no_grad(false);
+        const Tensor x = x_in.detach().contiguous();
+        y = product(x, w, bias, qtype, node->layout, M, N, K, with_last(x, N));
+    }
+    torch::autograd::set_history(y, node);
+    return y;
 }
 
 // act(x Wg^T) * (x Wu^T) for 16-bit x and tiled weights; an undefined tensor when this is not the plain case
@@ -313,7 +399,7 @@ PyObject *py_bind(PyObject *, PyObject *const *args, Py_ssize_t n) {
         api.name = (decltype(api.name))p;                                                          \
     } while (0)
     BIND(last_error); BIND(blob_bytes); BIND(tileable); BIND(linear_workspace_bytes); BIND(linear);
-    BIND(mlp_forward); BIND(dequantize_rows); BIND(experts_workspace_bytes); BIND(experts_forward);
+    BIND(mlp_forward); BIND(dequantize_rows); BIND(dequantize); BIND(backward); BIND(backward_applies); BIND(experts_workspace_bytes); BIND(experts_forward);
 #undef BIND
     Py_RETURN_NONE;
 }
@@ -341,6 +427,19 @@ PyObject *py_linear(PyObject *, PyObject *const *args, Py_ssize_t n) {
         const bool half = a.truth(5);
         NoGil free;
         return linear(x, w, bias, qtype, N, half);
+    });
+}
+
+// linear_train(x, weight, bias or None, qtype, out_len) -> y or None
+PyObject *py_linear_train(PyObject *, PyObject *const *args, Py_ssize_t n) {
+    return answer("linear_train", n, 5, [&] {
+        const Args a{args, n};
+        const Tensor &x = a.tensor(0), &w = a.tensor(1);
+        const Tensor bias = a.optional(2);
+        const int qtype = (int)a.integer(3);
+        const int64_t N = a.integer(4);
+        NoGil free;
+        return linear_train(x, w, bias, qtype, N);
     });
 }
 
@@ -423,7 +522,7 @@ PyObject *py_holds(PyObject *, PyObject *const *args, Py_ssize_t n) {
 }
 
 #define METHOD(name) {#name, (PyCFunction)(void (*)(void))py_##name, METH_FASTCALL, nullptr}
-PyMethodDef methods[] = {METHOD(bind), METHOD(product), METHOD(linear), METHOD(gated), METHOD(embedding), METHOD(experts), METHOD(upload),
+PyMethodDef methods[] = {METHOD(bind), METHOD(product), METHOD(linear), METHOD(linear_train), METHOD(gated), METHOD(embedding), METHOD(experts), METHOD(upload),
                          METHOD(download), METHOD(holds),
                          {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "lowbit_torch", "native host path of the low-bit layers", -1, methods};

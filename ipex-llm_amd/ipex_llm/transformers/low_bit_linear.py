@@ -587,6 +587,15 @@ class LowBitLinear(nn.Linear):
         is_training = self.training and not torch.is_inference_mode_enabled()
         if is_training and self.compute_dtype is not None and x.device.type == _ACCEL:
             x = x.to(self.compute_dtype)
+        if is_training and not self.act_order and self.mp_group is None:
+            # a 16-bit x that wants a gradient: one native call either way (None: not the plain case, the steps below)
+            params = self._parameters
+            weight = params["weight"]
+            if weight.quantized and weight._shape is not None and weight.qtype == self.qtype:
+                y = ops.linear_train(reshape_lm_head_input(x) if self.optimize_lm_head else x, weight, params["bias"], self.qtype,
+                                     self.out_len)
+                if y is not None:
+                    return y
 
         if self.bias is not None and self.bias.dtype != x.dtype:
             self.bias.data = self.bias.data.to(x.dtype)

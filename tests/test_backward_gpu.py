@@ -1,8 +1,9 @@
-"""The gradient that flows on below a low-bit linear, from the packed weight."""
+"""The gradient that flows on below a low-bit linear: the kernel that reads the packed weight, and the layer around it."""
 import pytest
 import torch
 
 from gpu_util import ALL, DT, NAMES, dev_dequantize, dev_quantize, ggml, stream, weights
+from ipex_llm.transformers.low_bit_linear import FP4Params, LowBitLinear, MatMulLowBit
 
 pytestmark = pytest.mark.gpu
 TILED = ggml.LAYOUT_TILED
@@ -37,3 +38,62 @@ def test_kernel(qtype, m, n, k, dtype):
     want = grad[:1].float().cpu() @ w.float().cpu()
     assert torch.equal(out[:1].float().cpu().isnan(), want.isnan()) and torch.equal(out[:1].float().cpu().isinf(), want.isinf())
     assert m == 1 or close(out[1:m], grad[1:], w, dtype)
+
+
+def layer_of(qtype, n, k, bias=None):
+    with torch.device("meta"):
+        layer = LowBitLinear(k, n, qtype, bias=bias is not None)
+    layer._parameters["weight"] = FP4Params(torch.from_numpy(weights(9, (n, k))), qtype=qtype).to("cuda")
+    if bias is not None:
+        layer._parameters["bias"] = torch.nn.Parameter(bias, requires_grad=False)
+    return layer.train()
+
+
+@pytest.mark.parametrize("m,n,k", [(100, 1024, 2560), (100, 4096, 512), (70, 528, 1056)], ids=["packed", "dense", "row-major"])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16], ids=["f16", "bf16"])
+def test_layer_in_training(m, n, k, dtype):
+    """Both ways of the gradient and both layouts, against the autograd function in Python; x and its gradient of other strides."""
+    gen = torch.Generator().manual_seed(3)
+    layer = layer_of(2, n, k, torch.randn(n, generator=gen).to(dtype).cuda())
+    layout = layer.weight.blob_layout
+    assert ggml.lowbit_backward_applies(2, layout, DT[dtype], m, n, k) == (layout == TILED and n < 2 * k)
+    x = torch.randn((2, k, m // 2), generator=gen).to(dtype).cuda().transpose(1, 2).requires_grad_(True)
+    y = layer(x)
+    assert y.grad_fn.name() == "MatMulLowBitBackward" and y.shape == (2, m // 2, n)
+    with torch.inference_mode():
+        assert torch.equal(y, layer.eval()(x.detach()))
+    layer.train()
+    w = dev_dequantize(layer.weight.data.view(torch.uint8), 2, n, k, layout, dtype)
+    grad = torch.randn((2, n, m // 2), generator=gen).to(dtype).cuda().transpose(1, 2)
+    for _ in range(2):                                       # nothing is freed by the first backward
+        (gx,) = torch.autograd.grad(y, x, grad)
+        assert gx.shape == x.shape and close(gx.reshape(m, k), grad.reshape(m, n), w, dtype)
+    (gs,) = torch.autograd.grad(y.sum(), x)                  # a gradient of strides 0
+    assert close(gs.reshape(m, k), torch.ones((m, n), dtype=dtype, device="cuda"), w, dtype)
+    product = MatMulLowBit.apply(x.detach().reshape(m, k).requires_grad_(True), layer.weight, n).view(y.shape)
+    eps = torch.finfo(dtype).eps                             # that rounds the product and the sum with the bias, the layer the sum
+    assert ((product + layer.bias - y).abs() <= eps * (product.abs() / 2 + y.abs())).all()
+
+
+def test_derivatives_that_the_node_leaves_to_operators():
+    """A second derivative, a batch of gradients, a forward-mode tangent and a saved-tensor hook, as MatMulLowBit has them."""
+    m, n, k = 24, 64, 128
+    layer = layer_of(2, n, k)
+    w = dev_dequantize(layer.weight.data.view(torch.uint8), 2, n, k, TILED, torch.float16)
+    x = torch.randn((m, k), device="cuda").half().requires_grad_(True)
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: pytest.fail("nothing is saved"), lambda t: t):
+        y = layer(x)
+    grad = torch.randn((m, n), device="cuda").half().requires_grad_(True)
+    (gx,) = torch.autograd.grad(y, x, grad, create_graph=True)
+    (gg,) = torch.autograd.grad(gx, grad, torch.ones_like(gx), retain_graph=True)
+    assert torch.allclose(gg.float(), w.float().sum(1).expand(m, n), rtol=2e-3, atol=2e-3)
+    batch = torch.randn((3, m, n), device="cuda").half()
+    (gb,) = torch.autograd.grad(y, x, batch, is_grads_batched=True, retain_graph=True)
+    for i in range(3):
+        assert close(gb[i], batch[i], w, torch.float16)
+    with torch.autograd.forward_ad.dual_level():
+        dual = torch.autograd.forward_ad.make_dual(x, torch.ones_like(x))
+        with pytest.raises(RuntimeError):
+            layer(dual)
+    with torch.no_grad():
+        assert not layer(x).requires_grad
