@@ -630,8 +630,8 @@ __global__ __launch_bounds__(64 * WAVES * KS, (DMA && MB == 4) ? 2 : 1) void gem
         // their use: those variants keep the two wait states ahead of every MFMA, the others spend them once.
         constexpr bool WAIT_STATES = MBC * NB32 < 4;
         if constexpr (!WAIT_STATES) {
-            asm volatile("s_nop 1" : "+v"(wv[0]));
-            if constexpr (NB32 == 2) asm volatile("" : "+v"(wv[1]));
+            if constexpr (NB32 == 2) asm volatile("s_nop 1" : "+v"(wv[0]), "+v"(wv[1]));
+            else asm volatile("s_nop 1" : "+v"(wv[0]));
         }
 #pragma unroll
         for (int ks = 0; ks < 8; ks++) {
@@ -642,7 +642,8 @@ __global__ __launch_bounds__(64 * WAVES * KS, (DMA && MB == 4) ? 2 : 1) void gem
                 for (int nb = 0; nb < NB32; nb++) {
                     // (a wave with one weight block uses what the step before dequantized last in the very first MFMA of a
                     // step, and where the compiler puts that last instruction is its choice: the two wait states stay)
-                    if (NB32 == 1 && mb == 0) mfma_acc<true>(acc[mb][nb], __builtin_bit_cast(V8, wv[nb]), xv[mb]);
+                    // (the last step's are held here by nothing but their use: there too)
+                    if ((NB32 == 1 || (ks == 7 && nb == 0)) && mb == 0) mfma_acc<true>(acc[mb][nb], __builtin_bit_cast(V8, wv[nb]), xv[mb]);
                     else mfma_acc<WAIT_STATES>(acc[mb][nb], __builtin_bit_cast(V8, wv[nb]), xv[mb]);
                     if (ks < 7) {
                         // pairs [ceil(slot * PAIRS / SLOTS), ceil((slot + 1) * PAIRS / SLOTS)): spread evenly over the
@@ -654,6 +655,11 @@ __global__ __launch_bounds__(64 * WAVES * KS, (DMA && MB == 4) ? 2 : 1) void gem
                         for (int idx = 0; idx < (NF4REG ? 0 : PAIRS); idx++) {
                             if (slot_i >= SPREAD || idx < (slot_i * PAIRS + SPREAD - 1) / SPREAD || idx >= ((slot_i + 1) * PAIRS + SPREAD - 1) / SPREAD) continue;
                             wn[idx >> 2][idx & 3] = dequant_pair(t, ks + 1, idx >> 2, idx & 3);   // (weight block, pair)
+                        }
+                        // (here and not where the next step uses them)
+                        if (slot_i == SPREAD - 1) {
+                            if constexpr (NB32 == 2) asm volatile("" : "+v"(wn[0]), "+v"(wn[1]));
+                            else asm volatile("" : "+v"(wn[0]));
                         }
                     }
                     // An MFMA occupies its pipe for 32 cycles and the wave issues in order: what stands between two
@@ -706,8 +712,9 @@ __global__ __launch_bounds__(64 * WAVES * KS, (DMA && MB == 4) ? 2 : 1) void gem
                 for (int p = 0; p < 4; p++) wv[nb][p] = dequant_pair(t, 0, nb, p);
             }
         }
-        asm volatile("s_nop 1" : "+v"(wv[0]));          // VALU write of an MFMA operand: two wait states
-        if constexpr (NB32 == 2) asm volatile("" : "+v"(wv[1]));
+        // VALU write of an MFMA operand: two wait states
+        if constexpr (NB32 == 2) asm volatile("s_nop 1" : "+v"(wv[0]), "+v"(wv[1]));
+        else asm volatile("s_nop 1" : "+v"(wv[0]));
     };
     auto step_ahead = [&](auto &acc, const uint8_t *cur, const uint8_t *nxt, const WRegs &t, const WRegs &tn, auto mbc_,
                           auto &xv, u32x4 (&wv)[NB32], auto &&between) __attribute__((always_inline)) {
@@ -1059,7 +1066,8 @@ __global__ __launch_bounds__(64 * WAVES * KS, (DMA && MB == 4) ? 2 : 1) void gem
                 // tile saved 7 % of its time, removing the weight loads 21 %).  These variants have registers to
                 // spare, so the weights run two steps ahead, through three register sets, and a step ends when
                 // everything but the weight loads it has just issued has landed.  x keeps its two LDS buffers and
-                // one step of prefetch (it comes from L2).  Three weight sets and two buffers: a period of six.
+                // one step of prefetch (it comes from L2).
+                constexpr int XBUF = 8 * MB32 * 1024;
                 constexpr int WLOADS = NB32 * ((F::BITS == 8 ? 2 : 1) * 2 + 1);      // load instructions of load_w_nb, all blocks
                 WRegs w2;
                 dma_x(0, xs0, mbc, xg);
@@ -1067,24 +1075,51 @@ __global__ __launch_bounds__(64 * WAVES * KS, (DMA && MB == 4) ? 2 : 1) void gem
                 load_w(1, w1);
                 wait_all_loads();
                 __syncthreads();
-#define LOWBIT_DEEP_STEP(i, cur, nxt, wc, wl)                                                                  \
-                if (kt + (i) < Gs) {                                                                           \
-                    compute(acc, cur, wc, mbc, [&](const int point, const int points) __attribute__((always_inline)) { \
-                        fetch_units_deep(kt + (i) + 1, nxt, kt + (i) + 2, wl, point, points, mbc, xg); \
-                    });                                                                                        \
-                    wait_loads_but<WLOADS>();                                                                  \
-                    __syncthreads();                                                                           \
+                // The x buffers are told apart by an offset, so that three steps are a period, and the last one to three steps
+                // stand apart from the loop: with a way out between its steps the compiler moved the sets of weight
+                // registers where the ways met, which waits for the loads on their way into them - a step then lasted as
+                // long as a load again, however early it had been issued.
+                int cur = 0;
+                auto deep_step = [&](int kt, WRegs &wc, WRegs &wl) __attribute__((always_inline)) {
+                    // (nothing of this step ahead of the barrier that it begins behind: the checker of the assembly pairs
+                    // the wait there with the loads ahead of it)
+#pragma unroll
+                    for (int nb = 0; nb < NB32; nb++) {
+                        asm volatile("" : "+v"(wc.lo[nb].q0));
+                        if constexpr (F::BITS == 8) asm volatile("" : "+v"(wc.lo[nb].q1));
+                    }
+                    compute(acc, xs0 + cur, wc, mbc, [&](const int point, const int points) __attribute__((always_inline)) {
+                        fetch_units_deep(kt + 1, xs0 + (XBUF - cur), kt + 2, wl, point, points, mbc, xg);
+                    });
+                    wait_loads_but<WLOADS>();
+                    __syncthreads();
+                    cur = XBUF - cur;
+                };
+                int kt = 0;
+                for (; kt + 3 < Gs; kt += 3) {
+                    deep_step(kt, w0, w2);
+                    deep_step(kt + 1, w1, w0);
+                    deep_step(kt + 2, w2, w1);
                 }
-                for (int kt = 0; kt < Gs; kt += 6) {
-                    LOWBIT_DEEP_STEP(0, xs0, xs1, w0, w2)
-                    LOWBIT_DEEP_STEP(1, xs1, xs0, w1, w0)
-                    LOWBIT_DEEP_STEP(2, xs0, xs1, w2, w1)
-                    LOWBIT_DEEP_STEP(3, xs1, xs0, w0, w2)
-                    LOWBIT_DEEP_STEP(4, xs0, xs1, w1, w0)
-                    LOWBIT_DEEP_STEP(5, xs1, xs0, w2, w1)
+                if (kt < Gs) {
+                    deep_step(kt, w0, w2);
+                    if (kt + 1 < Gs) {
+                        deep_step(kt + 1, w1, w0);
+                        if (kt + 2 < Gs) deep_step(kt + 2, w2, w1);
+                    }
                 }
-#undef LOWBIT_DEEP_STEP
                 wait_all_loads();                   // the loads past the end (clamped re-reads) must not outlive the wave's registers
+                // (and they are made: a step ends by counting its loads)
+                auto used = [](const WRegs &t) __attribute__((always_inline)) {
+#pragma unroll
+                    for (int nb = 0; nb < NB32; nb++) {
+                        asm volatile("" :: "v"(t.lo[nb].q0), "v"(t.hi[nb].q0), "v"(t.lo[nb].h[0]));
+                        if constexpr (F::BITS == 8) asm volatile("" :: "v"(t.lo[nb].q1), "v"(t.hi[nb].q1));
+                    }
+                };
+                used(w0);
+                used(w1);
+                used(w2);
                 epilogue(acc, first_t(), mbc);
                 return;
             }
