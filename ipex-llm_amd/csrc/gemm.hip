@@ -151,15 +151,6 @@ static int split_tail_tiles(int M, int64_t tiles, int n_cus) {
     return half_tiles(M, tiles, n_cus) ? (int)(tiles / 8) + 1 : 0;
 }
 
-// Row tiles per band of the kernel's tile order (see the kernel): the row tiles are cut into at most 8 bands, a
-// power of two of them, so that a band of x (band_m * rows per tile * K activations) stays small enough for an
-// XCD's L2 where M allows it.
-static int band_rows(int tiles_m) {
-    int bands = 1;
-    while (bands * 2 <= 8 && bands * 2 <= tiles_m) bands *= 2;
-    return (tiles_m + bands - 1) / bands;
-}
-
 template <int QT, typename AT>
 static int launch_gemm_t(const void *x, const void *w, const void *bias, void *y, int M, int N, int K, float *ws, int splits,
                          hipStream_t st) {

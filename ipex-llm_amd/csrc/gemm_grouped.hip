@@ -4,13 +4,15 @@
 // LowBitLinear on the rows routed to it (python/llm/src/ipex_llm/transformers/models/qwen2_moe.py:375-430
 // is the pattern; the gated MLP of an expert is models/common.py:145-158).
 //
-// Two forms of the tiled MFMA GEMM kernel serve it:
+// Three forms of the tiled MFMA GEMM kernel serve it:
 //   - 128-row tiles, two workgroups per compute unit: a group of r rows takes ceil(r / 128) row tiles, each
 //     of which walks (loads and dequantizes) the group's weights once;
 //   - 256-row tiles ("tall"), one workgroup per compute unit: one walk for up to 256 rows, only the 32-row
 //     blocks that hold rows are computed.  With a hundred and more rows per group - a prefill batch spread over
 //     the experts - every group above 128 rows would otherwise walk its weights twice.
-// The tall form also has the fused gate/up variant (act(x Wg^T) * (x Wu^T) in one pass over x) and can split
+//   - the narrow tile of the dense GEMM (128 rows by 128 weight rows, one or two groups of waves) where the tiles are few:
+//     twice the workgroups of the 128-row form, four times those of the tall one's fused variant.
+// The tall form also has the fused gate/up variant (act(x Wg^T) * (x Wu^T) in one pass over x), as has the narrow tile, and can split
 // K over a second grid dimension when the output alone has too few tiles for the machine (the down
 // projection: few columns, long K); the fp32 partial tiles go through a workspace and a second kernel.
 //
@@ -28,8 +30,8 @@ int launch_grouped_q(const void *x, const void *const *w, const void *const *w_u
                      hipStream_t st);
 
 template <int QT>
-int launch_mlp_gemm_q(const void *x, const void *wg, const void *wu, void *y, int dt, int M, int N, int K, int act, int waves,
-                      bool one_round, hipStream_t st);
+int launch_mlp_gemm_q(const void *x, const void *wg, const void *wu, void *y, int dt, int M, int N, int K, int act,
+                      const GroupedPlan &plan, hipStream_t st);
 
 static int device_cus() {
     static const int n_cus = [] {
@@ -77,6 +79,20 @@ static bool grouped_one_round(int total_rows, int n_groups, int tiles_n, bool ta
     return row_tiles >= 8 && (int64_t)row_tiles * tiles_n * splits <= (int64_t)device_cus() * (tall ? 1 : 2);
 }
 
+// Whether a grouped launch takes narrow tiles (128 rows by 128 weight rows, of both weights 64), and with how many groups of
+// waves: 2 while its tiles (an estimate: the host never sees the offsets) are one per CU at most and K has eight steps, 1
+// while they are two per CU, 0 beyond.  The fused form's tall tiles are a quarter as many and leave CUs idle there, whole
+// experts, us: 15 of [896 x 2048] in nf4 with 114 tokens, two each, 54.9 -> 46.4, 9 of [640 x 1920] in sym_int8 with 93
+// tokens, four each, 44.5 -> 39.7, 9 of [1536 x 3968] in sym_int4 with 496 tokens 122.9 -> 109.4; more tiles: 12 of
+// [7168 x 2048] in fp8_e4m3 with 300 tokens 169.7 / 178.7, 8 of [14336 x 4096] with 512 492 / 586.
+static int grouped_narrow(int total_rows, int n_groups, int tiles_n, int K) {
+    const int rows = G_GM_TALL / 2;
+    const int row_tiles = total_rows > 64 * n_groups ? total_rows / rows + (n_groups + 1) / 2 : n_groups;
+    const int64_t tiles = (int64_t)row_tiles * tiles_n;
+    if (tiles > 2 * device_cus()) return 0;
+    return tiles <= device_cus() && K / TILE_COLS >= 8 ? 2 : 1;
+}
+
 GroupedPlan grouped_plan(int total_rows, int n_groups, int N, int K, size_t ws_bytes) {
     const int tiles_n = (N + G_GN - 1) / G_GN, G = K / TILE_COLS;
     const int row_tiles = total_rows / G_GM_TALL > n_groups ? total_rows / G_GM_TALL : n_groups;   // estimate of the tiles that hold rows
@@ -86,6 +102,12 @@ GroupedPlan grouped_plan(int total_rows, int n_groups, int N, int K, size_t ws_b
     const size_t per_split = tall_split_bytes(total_rows, n_groups, N);
     while (s > 1 && (size_t)s * per_split > ws_bytes) s--;
     if (s < 1) s = 1;
+    // Narrow tiles in place of either unsplit form (the same experts, down projection: 54.9 -> 46.9, 44.5 -> 42.4, 122.9 ->
+    // 116.4), and of two splits where each tile has a CU and groups are small: the halves of K then meet without a second
+    // launch (16 of [2048 x 4096] in nf4 with 300 tokens, two each, 126.0 -> 119.7).
+    const int tiles_narrow = (N + G_GN / 2 - 1) / (G_GN / 2), narrow = grouped_narrow(total_rows, n_groups, tiles_narrow, K);
+    if (s == 1 ? narrow > 0 : s == 2 && narrow == 2 && total_rows <= 96 * n_groups)
+        return {false, 1, 4 * narrow, grouped_one_round(total_rows, n_groups, tiles_narrow, false, 1), narrow};
     const bool tall = s > 1 || (int64_t)total_rows > (int64_t)n_groups * 96;
     return {tall, s, grouped_waves(total_rows, n_groups, false), grouped_one_round(total_rows, n_groups, tiles_n, tall, s)};
 }
@@ -93,10 +115,10 @@ GroupedPlan grouped_plan(int total_rows, int n_groups, int N, int K, size_t ws_b
 // What launch_grouped_gemm would do for a plain grouped product: {tall, splits, waves, grid.x}.
 void grouped_plan_query(int total_rows, int n_groups, int N, int K, size_t ws_bytes, int out[4]) {
     const GroupedPlan p = grouped_plan(total_rows, n_groups, N, K, ws_bytes);
-    const int tiles_n = (N + G_GN - 1) / G_GN;
+    const int tiles_n = p.narrow ? (N + G_GN / 2 - 1) / (G_GN / 2) : (N + G_GN - 1) / G_GN;
     out[0] = p.tall;
     out[1] = p.splits;
-    out[2] = p.tall ? p.waves : 4;
+    out[2] = p.tall || p.narrow ? p.waves : 4;
     out[3] = p.tall ? tall_grid(total_rows, n_groups, tiles_n, p.one_round)
                     : grouped_grid(grouped_max_row_tiles(total_rows, n_groups, G_GM_TALL / 2), tiles_n, grouped_chunk(tiles_n, p.one_round));
 }
@@ -104,6 +126,13 @@ void grouped_plan_query(int total_rows, int n_groups, int N, int K, size_t ws_by
 size_t grouped_workspace_bytes(int total_rows, int n_groups, int N, int K) {
     const GroupedPlan p = grouped_plan(total_rows, n_groups, N, K, (size_t)-1);
     return p.splits > 1 ? (size_t)p.splits * tall_split_bytes(total_rows, n_groups, N) : 0;
+}
+
+static GroupedPlan grouped_mlp_plan(int total_rows, int n_groups, int N, int K) {
+    const int tiles_narrow = (N + G_GN / 4 - 1) / (G_GN / 4), narrow = grouped_narrow(total_rows, n_groups, tiles_narrow, K);
+    if (narrow) return {false, 1, 4 * narrow, grouped_one_round(total_rows, n_groups, tiles_narrow, false, 1), narrow};
+    return {true, 1, grouped_waves(total_rows, n_groups, true),
+            grouped_one_round(total_rows, n_groups, (N + G_GN / 2 - 1) / (G_GN / 2), true, 1)};
 }
 
 // y[rows of group e] = x[rows of group e] * dequant(w[e])^T, or, with w_up, act(x w[e]^T) * (x w_up[e]^T).
@@ -114,8 +143,7 @@ int launch_grouped_gemm(const void *x, const void *const *w, const void *const *
     if (total_rows == 0 || N == 0 || n_groups == 0) return 0;
     if (total_rows >= (1 << 24) || K >= (1 << 23)) return -3;        // 24-bit row offsets in the kernel
     float *ws = (float *)workspace;
-    const GroupedPlan plan = w_up ? GroupedPlan{true, 1, grouped_waves(total_rows, n_groups, true),
-                                                grouped_one_round(total_rows, n_groups, (N + G_GN / 2 - 1) / (G_GN / 2), true, 1)}
+    const GroupedPlan plan = w_up ? grouped_mlp_plan(total_rows, n_groups, N, K)
                                   : grouped_plan(total_rows, n_groups, N, K, ws ? workspace_bytes : 0);
     switch (qtype) {
     case QT_SYM_INT4: return launch_grouped_q<QT_SYM_INT4>(x, w, w_up, y, offsets, n_groups, total_rows, act_dtype, N, K, act, plan, ws, st);
@@ -127,6 +155,25 @@ int launch_grouped_gemm(const void *x, const void *const *w, const void *const *
     }
 }
 
+// Which tiles a dense gated MLP takes: narrow ones (64 columns of both weights), in halves of 64 rows and with two groups of
+// waves, while they are one per CU at most (eight K steps and more); with one group while they are two per CU and M more
+// than 128, and where the tall tiles of 256 x 128 would be little more than one per CU, so that most CUs wait for the
+// others' second.  400 points, eight shapes, M = 65 .. 2048, five formats: 1.4 times as fast as tall tiles alone on
+// average, 1.6 on the 290 where narrow ones are taken, 0.95 at worst.  Tall / narrow, sym_int4 fp16, us:
+// [3584 x 1152] at M = 128 / 512 18.1 / 10.8 and 31.6 / 15.8, [8064 x 3840] at M = 128 / 384 43.5 / 25.1 and 77.7 / 54.3,
+// [11008 x 4096] at M = 128 / 256 / 768 49.3 / 33.1, 81.2 / 56.4 and 183 / 149; but at M = 512 / 2048 90 / 100 and 319 / 335.
+static GroupedPlan mlp_plan(int M, int N, int K) {
+    const int rows = G_GM_TALL / 2, tiles_m = (M + rows - 1) / rows, cus = device_cus();
+    const int64_t tiles = (int64_t)tiles_m * ((N + G_GN / 4 - 1) / (G_GN / 4));
+    const int tall_n = (N + G_GN / 2 - 1) / (G_GN / 2);
+    const int64_t tall = (int64_t)((M + G_GM_TALL - 1) / G_GM_TALL) * tall_n;
+    GroupedPlan plan = {true, 1, grouped_waves(M, 1, true), grouped_one_round(M, 1, tall_n, true, 1)};
+    if (tiles <= cus && K / TILE_COLS >= 8) plan.narrow = 2;
+    else if ((tiles <= 2 * cus && (M > rows || tiles <= cus)) || (tall > cus && tall * 20 <= (int64_t)cus * 27)) plan.narrow = 1;
+    plan.halves = plan.narrow && M > rows / 2 && 2 * tiles <= cus;
+    return plan;
+}
+
 // y = act(x wg^T) * (x wu^T) for a dense gated MLP of M rows: the fused gate/up form of the grouped kernel on one
 // group, its weights passed as arguments (nothing is read from tables in device memory).  Measured on MI355X
 // against the two products as separate launches plus the activation as an elementwise kernel, sym_int4
@@ -136,14 +183,13 @@ int launch_mlp_gemm(const void *x, const void *wg, const void *wu, void *y, int 
                     int act, hipStream_t st) {
     if (M == 0 || N == 0) return 0;
     if (M >= (1 << 24) || K >= (1 << 23)) return -3;                 // 24-bit row offsets in the kernel
-    const int waves = grouped_waves(M, 1, true);
-    const bool one_round = grouped_one_round(M, 1, (N + G_GN / 2 - 1) / (G_GN / 2), true, 1);
+    const GroupedPlan plan = mlp_plan(M, N, K);
     switch (qtype) {
-    case QT_SYM_INT4: return launch_mlp_gemm_q<QT_SYM_INT4>(x, wg, wu, y, act_dtype, M, N, K, act, waves, one_round, st);
-    case QT_ASYM_INT4: return launch_mlp_gemm_q<QT_ASYM_INT4>(x, wg, wu, y, act_dtype, M, N, K, act, waves, one_round, st);
-    case QT_SYM_INT8: return launch_mlp_gemm_q<QT_SYM_INT8>(x, wg, wu, y, act_dtype, M, N, K, act, waves, one_round, st);
-    case QT_NF4: return launch_mlp_gemm_q<QT_NF4>(x, wg, wu, y, act_dtype, M, N, K, act, waves, one_round, st);
-    case QT_FP8_E4M3: return launch_mlp_gemm_q<QT_FP8_E4M3>(x, wg, wu, y, act_dtype, M, N, K, act, waves, one_round, st);
+    case QT_SYM_INT4: return launch_mlp_gemm_q<QT_SYM_INT4>(x, wg, wu, y, act_dtype, M, N, K, act, plan, st);
+    case QT_ASYM_INT4: return launch_mlp_gemm_q<QT_ASYM_INT4>(x, wg, wu, y, act_dtype, M, N, K, act, plan, st);
+    case QT_SYM_INT8: return launch_mlp_gemm_q<QT_SYM_INT8>(x, wg, wu, y, act_dtype, M, N, K, act, plan, st);
+    case QT_NF4: return launch_mlp_gemm_q<QT_NF4>(x, wg, wu, y, act_dtype, M, N, K, act, plan, st);
+    case QT_FP8_E4M3: return launch_mlp_gemm_q<QT_FP8_E4M3>(x, wg, wu, y, act_dtype, M, N, K, act, plan, st);
     default: return -2;
     }
 }

@@ -4,13 +4,15 @@
 // LowBitLinear on the rows routed to it (python/llm/src/ipex_llm/transformers/models/qwen2_moe.py:375-430
 // is the pattern; the gated MLP of an expert is models/common.py:145-158).
 //
-// Two forms of the tiled MFMA GEMM kernel serve it:
+// Three forms of the tiled MFMA GEMM kernel serve it:
 //   - 128-row tiles, two workgroups per compute unit: a group of r rows takes ceil(r / 128) row tiles, each
 //     of which walks (loads and dequantizes) the group's weights once;
 //   - 256-row tiles ("tall"), one workgroup per compute unit: one walk for up to 256 rows, only the 32-row
 //     blocks that hold rows are computed.  With a hundred and more rows per group - a prefill batch spread over
 //     the experts - every group above 128 rows would otherwise walk its weights twice.
-// The tall form also has the fused gate/up variant (act(x Wg^T) * (x Wu^T) in one pass over x) and can split
+//   - the narrow tile of the dense GEMM (128 rows by 128 weight rows, one or two groups of waves) where the tiles are few:
+//     twice the workgroups of the 128-row form, four times those of the tall one's fused variant.
+// The tall form also has the fused gate/up variant (act(x Wg^T) * (x Wu^T) in one pass over x), as has the narrow tile, and can split
 // K over a second grid dimension when the output alone has too few tiles for the machine (the down
 // projection: few columns, long K); the fp32 partial tiles go through a workspace and a second kernel.
 //
@@ -65,6 +67,18 @@ __global__ __launch_bounds__(256) void grouped_splitk_reduce_kernel(const float 
 template <int QT, typename AT>
 static int launch_grouped_t(const void *x, const void *const *w, void *y, const int32_t *offsets, int n_groups,
                             int total_rows, int N, int K, const GroupedPlan &plan, float *ws, hipStream_t st) {
+    if (plan.narrow) {
+        const int tiles_n = (N + GN / 2 - 1) / (GN / 2), G = K / TILE_COLS, chunk = grouped_chunk(tiles_n, plan.one_round);
+        const GroupArgs ga = {offsets, (const uint8_t *const *)w, nullptr, n_groups, 0, 0, chunk};
+        const int grid = grouped_grid(grouped_max_row_tiles(total_rows, n_groups, GM), tiles_n, chunk);
+        if (plan.narrow == 2)
+            hipLaunchKernelGGL((gemm_mfma_kernel<QT, AT, true, MB32, true, false, 4, true, 2>), dim3(grid), dim3(512), 0, st, (const AT *)x,
+                               (const uint8_t *)nullptr, (AT *)y, 0, N, K, 1, ga, G, (float *)nullptr, 0, tiles_n);
+        else
+            hipLaunchKernelGGL((gemm_mfma_kernel<QT, AT, true, MB32, true, false, 4, true, 1>), dim3(grid), dim3(256), 0, st, (const AT *)x,
+                               (const uint8_t *)nullptr, (AT *)y, 0, N, K, 1, ga, G, (float *)nullptr, 0, tiles_n);
+        return 0;
+    }
     const int tiles_n = (N + GN - 1) / GN, G = K / TILE_COLS;
     const int chunk = grouped_chunk(tiles_n, plan.one_round);
     const GroupArgs ga = {offsets, (const uint8_t *const *)w, nullptr, n_groups, 0, 0, chunk};
@@ -92,6 +106,18 @@ template <int QT, typename AT>
 static int launch_grouped_mlp_t(const void *x, const void *const *wg, const void *const *wu, void *y,
                                 const int32_t *offsets, int n_groups, int total_rows, int N, int K, int act,
                                 const GroupedPlan &plan, hipStream_t st) {
+    if (plan.narrow) {
+        const int tiles_n = (N + GN / 4 - 1) / (GN / 4), G = K / TILE_COLS, chunk = grouped_chunk(tiles_n, plan.one_round);   // 64 columns of both
+        const GroupArgs ga = {offsets, (const uint8_t *const *)wg, (const uint8_t *const *)wu, n_groups, act, 0, chunk};
+        const int grid = grouped_grid(grouped_max_row_tiles(total_rows, n_groups, GM), tiles_n, chunk);
+        if (plan.narrow == 2)
+            hipLaunchKernelGGL((gemm_mfma_kernel<QT, AT, true, MB32, true, true, 4, true, 2>), dim3(grid), dim3(512), 0, st, (const AT *)x,
+                               (const uint8_t *)nullptr, (AT *)y, 0, N, K, 1, ga, G, (float *)nullptr, 0, tiles_n);
+        else
+            hipLaunchKernelGGL((gemm_mfma_kernel<QT, AT, true, MB32, true, true, 4, true, 1>), dim3(grid), dim3(256), 0, st, (const AT *)x,
+                               (const uint8_t *)nullptr, (AT *)y, 0, N, K, 1, ga, G, (float *)nullptr, 0, tiles_n);
+        return 0;
+    }
     const int tiles_n = (N + GN / 2 - 1) / (GN / 2), G = K / TILE_COLS;      // 128 columns of both weights per workgroup
     const int chunk = grouped_chunk(tiles_n, plan.one_round);
     const GroupArgs ga = {offsets, (const uint8_t *const *)wg, (const uint8_t *const *)wu, n_groups, act, 0, chunk};
@@ -113,13 +139,28 @@ static int launch_grouped_mlp_t(const void *x, const void *const *wg, const void
 // The fused gate/up form on a dense gated MLP: y = act(x wg^T) * (x wu^T) for all M rows of x, the two weights
 // given directly (no tables in device memory: see GroupArgs).
 template <int QT, typename AT>
-static int launch_mlp_gemm_t(const void *x, const void *wg, const void *wu, void *y, int M, int N, int K, int act, int waves,
-                             bool one_round, hipStream_t st) {
+static int launch_mlp_gemm_t(const void *x, const void *wg, const void *wu, void *y, int M, int N, int K, int act,
+                             const GroupedPlan &plan, hipStream_t st) {
+    if (plan.narrow) {
+        const int tiles_n = (N + GN / 4 - 1) / (GN / 4), G = K / TILE_COLS, tiles_m = (M + GM - 1) / GM;
+        GroupArgs ga{};
+        ga.act = act;
+        ga.w_up_one = (const uint8_t *)wu;
+        ga.split_tail = plan.halves ? (int)(((int64_t)tiles_m * tiles_n) / 8) + 1 : 0;
+        const dim3 grid(8 * (unsigned)(((int64_t)tiles_m * tiles_n + 7) / 8 + ga.split_tail));
+        if (plan.narrow == 2)
+            hipLaunchKernelGGL((gemm_mfma_kernel<QT, AT, true, MB32, false, true, 4, true, 2>), grid, dim3(512), 0, st, (const AT *)x,
+                               (const uint8_t *)wg, (AT *)y, M, N, K, band_rows(tiles_m), ga, G, (float *)nullptr, 0, tiles_n);
+        else
+            hipLaunchKernelGGL((gemm_mfma_kernel<QT, AT, true, MB32, false, true, 4, true, 1>), grid, dim3(256), 0, st, (const AT *)x,
+                               (const uint8_t *)wg, (AT *)y, M, N, K, band_rows(tiles_m), ga, G, (float *)nullptr, 0, tiles_n);
+        return 0;
+    }
     const int tiles_n = (N + GN / 2 - 1) / (GN / 2), G = K / TILE_COLS;
-    const int chunk = grouped_chunk(tiles_n, one_round);
+    const int chunk = grouped_chunk(tiles_n, plan.one_round);
     const GroupArgs ga = {nullptr, nullptr, nullptr, 1, act, 0, chunk, (const uint8_t *)wu};
     const int n_wg = grouped_grid((M + GM_TALL - 1) / GM_TALL, tiles_n, chunk);
-    if (waves == 8 || QT == QT_NF4) {                 // (nf4: see launch_grouped_mlp_t)
+    if (plan.waves == 8 || QT == QT_NF4) {            // (nf4: see launch_grouped_mlp_t)
         hipLaunchKernelGGL((gemm_mfma_kernel<QT, AT, true, MB32_TALL, true, true, 8>), dim3(n_wg), dim3(512), 0, st, (const AT *)x,
                            (const uint8_t *)wg, (AT *)y, M, N, K, 1, ga, G, (float *)nullptr, 0, tiles_n);
         return 0;
@@ -131,10 +172,10 @@ static int launch_mlp_gemm_t(const void *x, const void *wg, const void *wu, void
 }
 
 template <int QT>
-int launch_mlp_gemm_q(const void *x, const void *wg, const void *wu, void *y, int dt, int M, int N, int K, int act, int waves,
-                      bool one_round, hipStream_t st) {
-    if (dt == DT_F16) return launch_mlp_gemm_t<QT, _Float16>(x, wg, wu, y, M, N, K, act, waves, one_round, st);
-    if (dt == DT_BF16) return launch_mlp_gemm_t<QT, __bf16>(x, wg, wu, y, M, N, K, act, waves, one_round, st);
+int launch_mlp_gemm_q(const void *x, const void *wg, const void *wu, void *y, int dt, int M, int N, int K, int act,
+                      const GroupedPlan &plan, hipStream_t st) {
+    if (dt == DT_F16) return launch_mlp_gemm_t<QT, _Float16>(x, wg, wu, y, M, N, K, act, plan, st);
+    if (dt == DT_BF16) return launch_mlp_gemm_t<QT, __bf16>(x, wg, wu, y, M, N, K, act, plan, st);
     return -4;
 }
 

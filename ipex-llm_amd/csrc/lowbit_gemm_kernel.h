@@ -212,9 +212,9 @@ __global__ __launch_bounds__(64 * WAVES * KS, (DMA && MB == 4) ? 2 : 1) void gem
     using F = Fmt<QT>;
     using V8 = typename Vec8<AT>::type;
     static_assert(MB == 4 || (MB == 8 && DMA), "row tiles of 128 rows, or 256 rows in the DMA form");
-    static_assert(!DUAL || (GROUPED && MB == 8), "the fused gate/up form exists for grouped launches of the tall form");
+    static_assert(!DUAL || (GROUPED && MB == 8) || NARROW, "the fused gate/up form: grouped launches of the tall form, narrow tiles");
     static_assert(WAVES == 4 || (WAVES == 8 && MB == 8 && DMA), "eight waves: tall form only");
-    static_assert(!NARROW || (DMA && MB == 4 && WAVES == 4 && !GROUPED && !DUAL), "the narrow tile is a dense 128-row DMA form");
+    static_assert(!NARROW || (DMA && MB == 4 && WAVES == 4), "the narrow tile is a 128-row DMA form");
     static_assert(KS == 1 || (KS == 2 && NARROW), "two groups of waves: the narrow tile");
     constexpr int MB32 = MB, GM = 32 * MB;            // shadow the 128-row constants of the file
     constexpr int GN = NARROW ? lowbit::GN / 2 : lowbit::GN;
@@ -271,6 +271,7 @@ __global__ __launch_bounds__(64 * WAVES * KS, (DMA && MB == 4) ? 2 : 1) void gem
             if (m0 >= M) return;                                                     // (a last row tile of at most 64 rows)
             M = M < m0 + GM / 2 ? M : m0 + GM / 2;                                   // rows past the half are clamped / not stored
         }
+        w_up = ga.w_up_one;
     } else if (DUAL && ga.offsets == nullptr) {
         // one group of all M rows: the cells are dealt as in a grouped launch, a row tile is 256 rows of x
         int idx;
@@ -1210,5 +1211,13 @@ __global__ __launch_bounds__(64 * WAVES * KS, (DMA && MB == 4) ? 2 : 1) void gem
     }
 }
 
+// Row tiles per band of the kernel's tile order (see the kernel): the row tiles are cut into at most 8 bands, a
+// power of two of them, so that a band of x (band_m * rows per tile * K activations) stays small enough for an
+// XCD's L2 where M allows it.
+inline int band_rows(int tiles_m) {
+    int bands = 1;
+    while (bands * 2 <= 8 && bands * 2 <= tiles_m) bands *= 2;
+    return (tiles_m + bands - 1) / bands;
+}
 
 }  // namespace lowbit

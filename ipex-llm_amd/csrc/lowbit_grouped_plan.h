@@ -11,10 +11,12 @@ constexpr int G_GN = 256, G_GM_TALL = 256;
 // How a grouped launch runs: chosen on the host from the row count, never from the rows per group, which only
 // the device knows.
 struct GroupedPlan {
-    bool tall;      // 256-row tiles (always for the fused gate/up form)
+    bool tall;      // 256-row tiles
     int splits;     // K splits of the tall form (1 = none)
-    int waves;      // waves per workgroup of the tall form: 4 (64 weight rows each) or 8 (32 each, two per SIMD)
+    int waves;      // waves per workgroup of the tall form: 4 (64 weight rows each) or 8 (32 each, two per SIMD); of narrow tiles
     bool one_round; // the launch's workgroups (expected count) all fit the machine at once
+    int narrow = 0; // narrow tiles, with one or two groups of waves (0: not)
+    bool halves = false;   // narrow tiles of a dense gated MLP: in halves of 64 rows
 };
 
 // Upper bound of the number of `rows`-row tiles: every group adds at most one partly filled tile.

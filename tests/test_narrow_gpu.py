@@ -1,0 +1,69 @@
+"""Gated MLPs and grouped products around the sizes where their tiles change: narrow ones with two groups of waves and one, 128-row
+and tall ones."""
+import pytest
+import torch
+
+from gpu_util import ALL, DT, NAMES, dev_dequantize, dev_quantize, ggml, stream, weights
+
+pytestmark = pytest.mark.gpu
+TILED = ggml.LAYOUT_TILED
+
+
+def products(x, blob, qtype, n, k):
+    """x w^T in fp64 with the weights that the GEMM forms make, rounded once to x's type, and the bound of its error: fp32 sums of k
+    terms; asym_int4 (q * d + m) rounds a second time in dev_dequantize"""
+    w = dev_dequantize(blob, qtype, n, k, TILED, torch.float32).to(x.dtype).double()
+    size = x.double().abs() @ w.abs().t()
+    return x.double() @ w.t(), size * (k * 2.0 ** -24 + (torch.finfo(x.dtype).eps if qtype == 3 else 0.0))
+
+
+def mlp_close(y, x, blobs, qtype, n, k, act):
+    """act(x Wg^T) * (x Wu^T), rounded once; exp2 and rcp of an ulp each; the activation's slope is at most 1.13"""
+    (g, dg), (u, du) = (products(x, b, qtype, n, k) for b in blobs)
+    a = torch.nn.functional.silu(g) if act == 0 else torch.nn.functional.gelu(g, approximate="tanh")
+    eps = torch.finfo(x.dtype).eps
+    # (tanh as 1 - 2 / (1 + e^2u) cancels: an absolute 2^-23 of g)
+    bound = (a * u).abs() * (eps / 2 + 2.0 ** -20) + 1.13 * dg * u.abs() + a.abs() * du + dg * du + (g * u).abs() * 2.0 ** -21 + \
+        torch.finfo(x.dtype).smallest_normal
+    return ((y.double() - a * u).abs() <= bound).all()
+
+
+# 64 rows and two groups of waves per tile: 1, 2, 3 and 4 row blocks, an odd number of K steps, a last tile of 16 columns; one
+# group: fewer than eight steps, more than one tile per CU, tall tiles little more than one per CU; tall tiles beyond
+@pytest.mark.parametrize("m,n,k", [(65, 144, 1152), (100, 2064, 1024), (130, 1040, 1408), (256, 4096, 1024), (200, 272, 640), (300, 6400, 256),
+                                   (260, 16400, 256), (513, 11008, 128), (384, 24576, 256)])
+@pytest.mark.parametrize("qtype", ALL, ids=NAMES.values())
+def test_gated_mlp_tiles(qtype, m, n, k):
+    dtype, act = (torch.bfloat16, 1) if k % 512 == 128 else (torch.float16, 0)
+    blobs = [dev_quantize(weights(60 + i, (n, k)), qtype, TILED) for i in range(2)]
+    x = torch.randn((m, k), generator=torch.Generator().manual_seed(m)).to(dtype).cuda()
+    y = torch.full((m + 1, n), float("nan"), dtype=dtype, device="cuda")
+    ggml.lowbit_mlp_forward(x.data_ptr(), blobs[0].data_ptr(), blobs[1].data_ptr(), y.data_ptr(), qtype, DT[dtype], m, n, k, act, stream())
+    assert torch.isnan(y[m]).all() and mlp_close(y[:m], x, blobs, qtype, n, k, act)
+
+
+@pytest.mark.parametrize("rows,n,k", [((3, 0, 40, 129, 1), 144, 1152), ((130, 257, 64), 2064, 1024), ((5, 31, 33), 272, 640), ((200, 9), 16400, 256),
+                                      ((300, 100, 20), 40960, 128)])
+@pytest.mark.parametrize("qtype", ALL, ids=NAMES.values())
+def test_grouped_tiles(qtype, rows, n, k):
+    """Groups of no, few and more than 128 rows in narrow tiles with two groups of waves and one, and in the forms beyond; the plain
+    product and the fused gate/up."""
+    dtype = torch.float16 if n % 32 else torch.bfloat16
+    offsets = torch.tensor([0, *rows]).cumsum(0).int().cuda()
+    total = sum(rows)
+    blobs = [[dev_quantize(weights(10 * e + i, (n, k)), qtype, TILED) for e in range(len(rows))] for i in range(2)]
+    tables = [torch.tensor([b.data_ptr() for b in bs], device="cuda") for bs in blobs]
+    x = torch.randn((total, k), generator=torch.Generator().manual_seed(1)).to(dtype).cuda()
+    y = torch.full((total + 1, n), float("nan"), dtype=dtype, device="cuda")
+    h = torch.full_like(y, float("nan"))
+    ggml.lowbit_grouped_forward(x.data_ptr(), tables[0].data_ptr(), y.data_ptr(), offsets.data_ptr(), len(rows), total, qtype, DT[dtype], n, k,
+                                stream())
+    ggml.lowbit_grouped_mlp_forward(x.data_ptr(), tables[0].data_ptr(), tables[1].data_ptr(), h.data_ptr(), offsets.data_ptr(), len(rows),
+                                    total, qtype, DT[dtype], n, k, 0, stream())
+    assert torch.isnan(y[total]).all() and torch.isnan(h[total]).all()
+    for e, (a, b) in enumerate(zip(offsets.tolist(), offsets.tolist()[1:])):
+        if a == b:
+            continue
+        want, bound = products(x[a:b], blobs[0][e], qtype, n, k)
+        assert ((y[a:b].double() - want).abs() <= want.abs() * torch.finfo(dtype).eps / 2 + bound + torch.finfo(dtype).smallest_normal).all()
+        assert mlp_close(h[a:b], x[a:b], (blobs[0][e], blobs[1][e]), qtype, n, k, 0)
