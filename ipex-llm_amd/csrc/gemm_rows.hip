@@ -1,28 +1,103 @@
 // Batches of more than 16 rows against weights in the row-major (ggml) layout, any shape: y[M,N] = x[M,K] dequant(W)[N,K]^T.
 //
 // Untileable weights (out_features no multiple of 16 or in_features no multiple of 128) had the streaming kernel only: a
-// pass over the weights per 16 rows of x.  Here a workgroup of four waves owns 16 * MB rows of x by 128 weight
+// pass over the weights per 16 rows of x.  Here a workgroup of four waves owns 32 * MB rows of x by 128 weight
 // rows; its waves split the weight rows, share the block of x in LDS (two buffers, one 128-column step of prefetch
-// through registers) and use every unpacked weight for all rows.
+// by LDS-DMA) and use every unpacked weight for all rows.
 //
-// The operands are those of lowbit_rows.h: exact codes, and the block scale applied to the fp32 result of each
-// v_mfma_f32_16x16x32, so nothing of a weight is rounded to 16 bits.  That scale is what bounds it: one FMA per result
-// and 32 columns (asym_int4: three operations) is as much vector time as the MFMA takes matrix time, and unpacking adds to
-// it - the reason for many rows of x per unpacked weight (MB = 8) where M allows.  333 rows on [3200 x 8640], 272 us as 21
-// streaming passes in sym_int4: 51.6 us with the reduction (357 TFLOP/s) in sym_int4, 67 in asym_int4, 70 (fp16) and 85
-// (bf16, three MFMAs per step) in nf4, 55 in sym_int8, 49 in fp8_e4m3 ([3201 x 8704]).
+// The operands are exact codes, and the block scale is applied to the fp32 result of a block's MFMAs, so nothing of a weight
+// is rounded to 16 bits.  That scale bounds the formats with blocks of 32: 16 FMAs (asym_int4: 48 operations) to two
+// v_mfma_f32_32x32x16, and the two do not overlap fully - an MFMA takes the issue of about 2.5 FMAs from either wave of a
+// SIMD.  Hence the 32 x 32 form (half the MFMAs of 16 x 16 x 32 for the same work: 21.0 against 24.7 ns per 32768 products
+// and 8 FMAs), one scaling per block of nf4 and fp8_e4m3 in place of one per 32 columns, and x by LDS-DMA in its own order: the
+// weights are unpacked so that a lane's eight codes are eight consecutive columns, where before x was permuted on its way
+// through registers.  The loads are spread over the step (8 KB of LDS-DMA per wave over its first half, the weights in
+// the middle): all at its head they waited for each other, 7 % of the time in sym_int4 and 13 % in fp8_e4m3.  sym_int8, whose six
+// loads touch the same lines, fetches those by the first code and the headers at the head (another 4 %, and 9 % where the
+// weights come from HBM: 128 rows on [32003 x 4096] 84 / 76 us; fp8_e4m3 loses 5).  Left: the memory
+// system (without the loads of x a step is 15 % shorter), and without FMAs, x and weights still 60 % of it.
+// Eight waves on 256 weight rows, which halve x's traffic, gain 5 - 9 % on [8008 x 8256] and lose as much elsewhere.
+// 333 rows on [3200 x 8640] with the reduction, before (16 x 16 x 32, x through registers) / now: sym_int4 49.9 / 42.0 us
+// (438 TFLOP/s), asym_int4 68.6 / 62.0, sym_int8 54.3 / 46, nf4 68.2 / 57.9 (fp16, two MFMAs per product) and 83.5 / 69.3
+// (bf16, three), fp8_e4m3 45.9 / 34.5 ([3201 x 8704]); 2000 rows on [4001 x 4160] 109.2 / 93.7 in sym_int4, 96.4 / 73.3 in
+// fp8_e4m3.
 #include "lowbit_mfma.h"
 #include "lowbit_rows.h"
 #include "lowbit_unpack.h"
+
+#include <type_traits>
 
 namespace lowbit {
 
 int launch_gemv(const void *x, const void *w, const void *bias, void *y, int qtype, int layout, int act_dtype, int M, int N, int K,
                 int waves, hipStream_t st);
 
-constexpr int RG_WAVES = 4, RG_NB = 2, RG_N = RG_WAVES * RG_NB * TILE_ROWS;      // 128 weight rows per workgroup
+constexpr int RG_WAVES = 4, RG_N = RG_WAVES * 32;        // 128 weight rows per workgroup, 32 per wave
 
-// MB: 16-row blocks of x per workgroup.  blockIdx.y: the K split, whose partial sums go to ws in register order.
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+__device__ inline f32x16 mfma32(f16x8 a, f16x8 b, f32x16 c) { return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0); }
+__device__ inline f32x16 mfma32(bf16x8 a, bf16x8 b, f32x16 c) { return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0); }
+
+// Codes and headers of 32 weight rows by 128 columns, lane l = 32 * c + r holding 16-byte pieces of row r:
+//   sym_int4, asym_int4   blocks c and 2 + c of the four
+//   nf4                   half c of either block's 32 bytes
+//   8 bits                bytes 16c .. 16c+15 of each 32 columns; sym_int8: headers of blocks c and 2 + c
+template <int QT> struct RowRegs32 {
+    static constexpr int NQ = Fmt<QT>::BITS == 8 ? 4 : 2, NH = QT == QT_FP8_E4M3 ? 1 : 2;
+    u32x4 q[NQ];
+    uint32_t h[NH];
+};
+// Blocks past the end of the row are read from its last one (their scale is made zero).
+template <int QT> __device__ inline void load_rows32(gbytes row, int g, int c, int blocks, RowRegs32<QT> &t, int from = 0, int to = RowRegs32<QT>::NQ) {
+    using F = Fmt<QT>;
+    constexpr int PER = TILE_COLS / F::QK;                   // blocks per group of columns
+    auto block = [&](int i) __attribute__((always_inline)) {
+        const int b = g * PER + i;
+        return row + (int64_t)(b < blocks ? b : blocks - 1) * F::TS;
+    };
+#pragma unroll
+    for (int i = from; i < to; i++) {
+        const gbytes p = QT == QT_NF4 ? block(i) + 16 * c : QT == QT_SYM_INT8 ? block(i) + 16 * c
+                       : QT == QT_FP8_E4M3 ? block(0) + 32 * i + 16 * c : block(2 * i + c);
+        t.q[i] = *(const __attribute__((address_space(1))) u32x4_a2 *)(p + F::HDR);
+    }
+    if (from > 0) return;                                    // (the headers come with the first piece)
+#pragma unroll
+    for (int i = 0; i < RowRegs32<QT>::NH; i++) {
+        const gbytes p = QT == QT_NF4 ? block(i) : QT == QT_FP8_E4M3 ? block(0) : block(2 * i + c);
+        if constexpr (F::HDR == 2) t.h[i] = *(const __attribute__((address_space(1))) uint16_t *)p;
+        else t.h[i] = *(const __attribute__((address_space(1))) u32_a2 *)p;
+    }
+}
+// After this sub-step j (32 columns) has its codes in q[j / 2][2 * (j & 1)] and the next dword (4 bits) or in q[j] (8 bits),
+// and its block's header in hb[j], in all lanes.
+template <int QT> __device__ inline void arrange_rows32(RowRegs32<QT> &t, uint32_t (&hb)[4]) {
+    if constexpr (QT == QT_FP8_E4M3) {
+        hb[0] = hb[1] = hb[2] = hb[3] = t.h[0];
+    } else if constexpr (QT == QT_NF4) {
+        hb[0] = hb[1] = t.h[0];
+        hb[2] = hb[3] = t.h[1];
+    } else {
+#pragma unroll
+        for (int i = 0; i < 2; i++) {
+            const auto h = __builtin_amdgcn_permlane32_swap(t.h[i], t.h[i], false, false);
+            hb[2 * i] = h[0];
+            hb[2 * i + 1] = h[1];
+            if constexpr (QT != QT_SYM_INT8) {               // lane c: dwords 2c, 2c+1 of both blocks
+                const auto a = __builtin_amdgcn_permlane32_swap(t.q[i][0], t.q[i][2], false, false);
+                const auto b = __builtin_amdgcn_permlane32_swap(t.q[i][1], t.q[i][3], false, false);
+                t.q[i] = u32x4{a[0], b[0], a[1], b[1]};
+            }
+        }
+    }
+}
+// MFMA s of sub-step j takes eight columns per lane, of which lane c's are unit rows32_unit + c * rows32_lane of a row's 16.
+template <int QT> constexpr int rows32_unit(int j, int s) {
+    return Fmt<QT>::BITS == 8 ? 4 * j + s : QT == QT_NF4 ? 8 * (j / 2) + 4 * s + (j & 1) : 4 * j + 2 * s;
+}
+template <int QT> constexpr int rows32_lane() { return Fmt<QT>::BITS == 8 || QT == QT_NF4 ? 2 : 1; }
+
+// MB: 32-row blocks of x per workgroup.  blockIdx.y: the K split, whose partial sums go to ws in register order.
 template <int QT, typename AT, int MB>
 __global__ __launch_bounds__(256, 2) void gemm_rows_kernel(const AT *__restrict__ x, const uint8_t *__restrict__ w,
                                                            const AT *__restrict__ bias, AT *__restrict__ y, int M, int N, int K,
@@ -33,156 +108,199 @@ __global__ __launch_bounds__(256, 2) void gemm_rows_kernel(const AT *__restrict_
     constexpr float OFFSET = Op::OFFSET;
     constexpr bool NEED_S = Op::NEED_S;
     constexpr int PARTS = Op::PARTS;
-    constexpr int BM = 16 * MB, NB = RG_NB;
-    __shared__ __attribute__((aligned(16))) uint8_t xs[2][BM * 256];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, r = lane & 15, c = lane >> 4;
+    constexpr int BM = 32 * MB, XBYTES = BM * 256, PIECES = 2 * MB;      // 1 KB pieces of x (four rows) per wave and step
+    constexpr int SUB = F::QK / 32, NS = 4 / SUB;            // sub-steps of 32 columns per scale; scales per step
+    __shared__ __attribute__((aligned(1024))) uint8_t xs[2 * XBYTES];
+    const int lane = threadIdx.x & 63, r = lane & 31, c = lane >> 5;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
 
     // Workgroups go to the XCDs in turn (id % 8): each XCD takes a run of the tiles, row tile by row tile within a column
     // tile, so that its L2 serves a column's weights to all their row tiles.
     const int tiles_m = (M + BM - 1) / BM, tiles = tiles_m * ((N + RG_N - 1) / RG_N), per_xcd = (tiles + 7) / 8;
     const int tile = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
     if (tile >= tiles) return;                               // whole workgroup leaves
-    const int m0 = tile % tiles_m * BM, n0 = tile / tiles_m * RG_N + wave * (NB * TILE_ROWS);
+    const int m0 = tile % tiles_m * BM, n0 = tile / tiles_m * RG_N + wave * 32;
 
     const int blocks = K / F::QK, G = (K + TILE_COLS - 1) / TILE_COLS;
     const int g0 = blockIdx.y * steps, g1 = g0 + steps < G ? g0 + steps : G;
-    gbytes wr[NB];
+    const int n = n0 + r;
+    const gbytes wr = (gbytes)w + (int64_t)(n < N ? n : N - 1) * blocks * F::TS;
+
+    // x goes to LDS by itself: the 16 units (16 bytes) of a row's 128 columns in order, but for unit v of row m at v ^ m % 16,
+    // so that the 32 rows that an MFMA operand takes a unit of spread over the banks.  A wave's piece i is rows 16i + 4 * wave
+    // and the next three; rows past M are copies of the last one.
+    const int xrow = 4 * wave + (lane >> 4), xunit = (lane & 15) ^ xrow;
+    uint32_t xoff[PIECES];                                   // bytes from the tile's first row (K < 2^23)
 #pragma unroll
-    for (int nb = 0; nb < NB; nb++) {
-        const int n = n0 + nb * TILE_ROWS + r;
-        wr[nb] = (gbytes)w + (int64_t)(n < N ? n : N - 1) * blocks * F::TS;
-    }
-    // this thread's chunks of the x block: 16 lanes per row
-    const int u = threadIdx.x & 15, xrow = threadIdx.x >> 4;
-    const uint8_t *const xtile = (const uint8_t *)(x + (int64_t)m0 * K);
-    uint32_t xoff[MB];                                       // bytes from the tile's first row (K < 2^23)
-#pragma unroll
-    for (int i = 0; i < MB; i++) {
+    for (int i = 0; i < PIECES; i++) {
         const int m = i * 16 + xrow;
         xoff[i] = (uint32_t)(m0 + m < M ? m : M - 1 - m0) * (uint32_t)K * 2u;
     }
-    auto load_x = [&](int g, u32x4 (&v)[MB]) __attribute__((always_inline)) {
-        const int col = g * TILE_COLS + u * 8;
-        const bool past = col >= K;                          // columns past K read as zero (from the row's first ones)
-        const uint32_t at = past ? 0 : (uint32_t)col * 2u;
+    const uint64_t xtile = (uint64_t)(uintptr_t)(x + (int64_t)m0 * K);
+    const uint32_t xs_at = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t *)xs;
+    auto dma_x = [&](int g, int buf, int p0, int p1) __attribute__((always_inline)) {
+        // (past K: the group's first columns, times a scale of zero; from inline assembly, because the compiler would wait for
+        // an LDS-DMA ahead of every later LDS access - a step ends by waiting for it)
+        const uint32_t at = g * TILE_COLS + xunit * 8 < K ? (uint32_t)xunit * 16u : 0u;
+        const uint64_t src = xtile + (uint64_t)g * (TILE_COLS * sizeof(AT));
+        const uint32_t to = xs_at + buf + wave * 1024;
 #pragma unroll
-        for (int i = 0; i < MB; i++) {
-            v[i] = *(const u32x4 *)(xtile + (xoff[i] + at));
-            v[i] = past ? u32x4{0u, 0u, 0u, 0u} : v[i];
-        }
+        for (int i = p0; i < p1; i++)
+            asm volatile("s_add_u32 m0, %2, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
+                         :: "v"(xoff[i] + at), "s"(src), "s"(to), "n"(i * 4096) : "memory", "m0", "scc");
     };
-    auto load_w = [&](int g, RowRegs<QT> (&t)[NB]) __attribute__((always_inline)) {
-#pragma unroll
-        for (int nb = 0; nb < NB; nb++) load_rows<QT>(wr[nb], g, c, blocks, t[nb]);
-    };
-    auto put_x = [&](uint8_t *buf, const u32x4 (&v)[MB]) __attribute__((always_inline)) {
-#pragma unroll
-        for (int i = 0; i < MB; i++) store_x_rows<QT>(buf + (i * 16 + xrow) * 256, u, v[i], xrow);
+    auto land = [&]() __attribute__((always_inline)) {
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __syncthreads();
     };
 
-    f32x4 acc[MB][NB];
+    f32x16 acc[MB];
+    const f32x16 zero16 = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-    for (int mb = 0; mb < MB; mb++)
-#pragma unroll
-        for (int nb = 0; nb < NB; nb++) acc[mb][nb] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-    const f32x4 zero4 = {0.0f, 0.0f, 0.0f, 0.0f};
+    for (int mb = 0; mb < MB; mb++) acc[mb] = zero16;
     const V8 ones = ones8<AT>();
     const Op op;
 
-    u32x4 xr[MB];
-    RowRegs<QT> wc[NB], wn[NB];
-    load_x(g0, xr);
-    load_w(g0, wc);
-    put_x(xs[0], xr);
-    __syncthreads();
-    for (int g = g0; g < g1; g++) {
-        const uint8_t *cur = xs[(g - g0) & 1];
-        const bool more = g + 1 < g1;
-        if (more) {
-            load_x(g + 1, xr);
-            load_w(g + 1, wn);
+    RowRegs32<QT> wc, wn;
+    load_rows32<QT>(wr, g0, c, blocks, wc);
+    dma_x(g0, 0, 0, PIECES);
+    land();
+    // A step of 128 columns; the last one (more = false) loads nothing.  It stands apart from the loop: with a condition around
+    // the loads the compiler merged the registers of this step's weights with the next one's where the ways met, and so
+    // waited for the loads that it had just issued.
+    int cur = 0;
+    auto step = [&](int g, auto more_) __attribute__((always_inline)) {
+        constexpr bool more = decltype(more_)::value;
+        if constexpr (more) {
         }
-        uint32_t hb[NB][4];
-#pragma unroll
-        for (int nb = 0; nb < NB; nb++) arrange_rows<QT>(wc[nb], hb[nb]);
-        // Unit q = (step j, 16-row block mb), in the order the hardware should issue them: the MFMAs of a unit, the LDS
-        // read of the next one's x, then the scaling of the unit before, whose results have landed meanwhile.  Left
-        // alone the scheduler issues the step's reads and MFMAs together and runs out of registers.
-        auto read_x = [&](int q) __attribute__((always_inline)) {
-            const int j = q / MB, mb = q % MB;
-            return *(const V8 *)(cur + (mb * 16 + r) * 256 + (((j * 4 + c) ^ r) * 16));
+        uint32_t hb[4];
+        arrange_rows32<QT>(wc, hb);
+        // MFMA o of the step: 32-row block mb, MFMA s of sub-step j, in the order of the units below
+        constexpr int EARLY = QT == QT_SYM_INT8 ? 1 : 0;     // pieces of the weights loaded at the step's head
+        constexpr int PER = 2 * SUB, OPS = NS * MB * PER, AHEAD = 3;
+        const uint8_t *const base = xs + cur;
+        const int at = r * 256 + ((c * rows32_lane<QT>()) ^ (r & 15)) * 16;
+        auto read_x = [&](int o) __attribute__((always_inline)) {
+            const int q = o / PER, t = o % PER, mb = q % MB, j = q / MB * SUB + t / 2;
+            return *(const V8 *)(base + mb * 8192 + (at ^ (rows32_unit<QT>(j, t % 2) * 16)));
         };
-        V8 a = read_x(0), b[NB][PARTS];
-        float d[2][NB], e[2][NB];                            // of this step and the one before
-        f32x4 p[2][NB], sum[2];
+        V8 a[AHEAD + 1], b[SUB == 1 ? 2 : 1][PER][PARTS];
+        float d[2], e[2];                                    // of this scale and the next or the one before
+        f32x16 p[2], sum[2];
+        auto unpack = [&](int sc) __attribute__((always_inline)) {
 #pragma unroll
-        for (int q = 0; q <= 4 * MB; q++) {
-            if (q < 4 * MB) {
-                const int j = q / MB;
-                if (q % MB == 0) {
+            for (int jj = 0; jj < SUB; jj++) {
+                const int j = sc * SUB + jj;
 #pragma unroll
-                    for (int nb = 0; nb < NB; nb++) {
+                for (int part = 0; part < PARTS; part++) {
+                    V8 (&to)[PER][PARTS] = b[SUB == 1 ? sc & 1 : 0];
+                    RowRegs<QT> t;
+                    if constexpr (F::BITS == 8) {
+                        t.q0 = wc.q[j];
+                        to[2 * jj][part] = op.get(t, 0, part);
+                        to[2 * jj + 1][part] = op.get(t, 1, part);
+                    } else {
+                        // bytes 0, 2, 1, 3: the unpacking then leaves low 0, 1, high 0, 1, low 2, 3, high 2, 3
+                        V8 v[2];
 #pragma unroll
-                        for (int part = 0; part < PARTS; part++) b[nb][part] = op.get(wc[nb], j, part);
-                        float mn;
-                        hdr_to_scale<QT>(hb[nb][j], d[j & 1][nb], mn);
-                        e[j & 1][nb] = mn - OFFSET * d[j & 1][nb];
-                        d[j & 1][nb] = Op::scale(d[j & 1][nb]);
+                        for (int i = 0; i < 2; i++) {
+                            const uint32_t dw = wc.q[j / 2][2 * (j & 1) + i];
+                            t.q0[0] = __builtin_amdgcn_perm(dw, dw, 0x03010200u);
+                            v[i] = op.get(t, 0, part);
+                        }
+                        to[2 * jj][part] = __builtin_shufflevector(v[0], v[1], 0, 1, 4, 5, 8, 9, 12, 13);
+                        to[2 * jj + 1][part] = __builtin_shufflevector(v[0], v[1], 2, 3, 6, 7, 10, 11, 14, 15);
                     }
                 }
-                if constexpr (NEED_S) sum[q & 1] = mfma16(a, ones, zero4);
-#pragma unroll
-                for (int nb = 0; nb < NB; nb++) p[q & 1][nb] = Op::product(a, a, b[nb]);
-                if (q + 1 < 4 * MB) a = read_x(q + 1);
             }
-            if (q > 0) {
-                const int o = (q - 1) & 1, mb = (q - 1) % MB, j = (q - 1) / MB;
+            float mn;
+            hdr_to_scale<QT>(hb[sc * SUB], d[sc & 1], mn);
+            e[sc & 1] = mn - OFFSET * d[sc & 1];
+            d[sc & 1] = Op::scale(d[sc & 1]);
+            asm volatile("" : "+v"(d[sc & 1]), "+v"(e[sc & 1]));      // (in fp32: not converted again in every FMA)
+            if constexpr (!more) {                           // blocks past the end of the rows
+                const bool past = g * NS + sc >= blocks;
+                d[sc & 1] = past ? 0.0f : d[sc & 1];
+                e[sc & 1] = past ? 0.0f : e[sc & 1];
+            }
+        };
 #pragma unroll
-                for (int nb = 0; nb < NB; nb++)
+        for (int o = 0; o < AHEAD && o < OPS; o++) a[o] = read_x(o);
+        if constexpr (SUB == 1) unpack(0);
+        // Unit q = (scale sc, 32-row block mb), in the order the hardware should issue them: an MFMA, the LDS read of x three
+        // MFMAs ahead, a part of the scaling of the unit before, whose results have landed meanwhile, and so on; and the
+        // unpacking of the next sub-step's weights (nf4 and fp8: of this scale's, ahead of its first unit).
+        auto scale_some = [&](int q, int from, int to) __attribute__((always_inline)) {
+            const int mb = q % MB, sc = q / MB;
 #pragma unroll
-                    for (int i = 0; i < 4; i++)
-                        acc[mb][nb][i] = Op::add(acc[mb][nb][i], d[j & 1][nb], p[o][nb][i], e[j & 1][nb], sum[o][i]);
+            for (int i = from; i < to; i++) acc[mb][i] = Op::add(acc[mb][i], d[sc & 1], p[q & 1][i], e[sc & 1], sum[q & 1][i]);
+        };
 #pragma unroll
-                for (int nb = 0; nb < NB; nb++) asm volatile("" : "+v"(acc[mb][nb]));
+        for (int q = 0; q < NS * MB; q++) {
+            const int sc = q / MB;
+            if (SUB > 1 && q % MB == 0) {
+                unpack(sc);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            p[q & 1] = zero16;
+            sum[q & 1] = zero16;
+#pragma unroll
+            for (int t = 0; t < PER; t++) {
+                const int o = q * PER + t;
+                if constexpr (more) {                        // the next step's x over the first half, its weights in the middle
+#pragma unroll
+                    for (int i = 0; i < PIECES; i++)
+                        if (o == i * OPS / (2 * PIECES)) dma_x(g + 1, XBYTES - cur, i, i + 1);
+                    if (EARLY && o == 0) load_rows32<QT>(wr, g + 1, c, blocks, wn, 0, 1);
+                    if (o == OPS / 2) load_rows32<QT>(wr, g + 1, c, blocks, wn, EARLY);
+                }
+                const V8 v = a[o % (AHEAD + 1)];
+                if constexpr (NEED_S) sum[q & 1] = mfma32(v, ones, sum[q & 1]);
+#pragma unroll
+                for (int part = 0; part < PARTS; part++) p[q & 1] = mfma32(v, b[SUB == 1 ? sc & 1 : 0][t][part], p[q & 1]);
+                if (o + AHEAD < OPS) a[(o + AHEAD) % (AHEAD + 1)] = read_x(o + AHEAD);
+                if (q > 0) scale_some(q - 1, t * 16 / PER, (t + 1) * 16 / PER);
+                if (SUB == 1 && t == 1 && q % MB == MB / 2 && sc + 1 < NS) unpack(sc + 1);
+                __builtin_amdgcn_sched_barrier(0);
             }
         }
-        if (more) {
-            put_x(xs[(g + 1 - g0) & 1], xr);
-#pragma unroll
-            for (int nb = 0; nb < NB; nb++) wc[nb] = wn[nb];
+        scale_some(NS * MB - 1, 0, 16);
+        if constexpr (more) {
+            land();
+            wc = wn;
+            cur = XBYTES - cur;
         }
-        __syncthreads();
-    }
+    };
+    int g = g0;
+    for (; g + 1 < g1; g++) step(g, std::true_type{});
+    step(g, std::false_type{});
 
-    // C layout: lane = 16*grp + column (weight row), register i = row 4*grp + i of x
+    // C layout: lane = 32 * c + column (weight row), register 4q + i = row 8q + 4c + i of x
     if (ws) {
-        f32x4 *part = (f32x4 *)ws + (((int64_t)blockIdx.y * tiles + tile) * RG_WAVES + wave) * (MB * NB * 64) + lane;
+        f32x4 *part = (f32x4 *)ws + (((int64_t)blockIdx.y * tiles + tile) * RG_WAVES + wave) * (MB * 4 * 64) + lane;
 #pragma unroll
         for (int mb = 0; mb < MB; mb++)
 #pragma unroll
-            for (int nb = 0; nb < NB; nb++) part[(mb * NB + nb) * 64] = acc[mb][nb];
+            for (int q = 0; q < 4; q++)
+                part[(mb * 4 + q) * 64] = f32x4{acc[mb][4 * q], acc[mb][4 * q + 1], acc[mb][4 * q + 2], acc[mb][4 * q + 3]};
         return;
     }
+    if (n >= N) return;
+    const float bv = bias ? (float)bias[n] : 0.0f;
+    uint64_t again = 0;                                       // results that are not finite, see dot_fp32
 #pragma unroll
-    for (int nb = 0; nb < NB; nb++) {
-        const int n = n0 + nb * TILE_ROWS + r;
-        if (n >= N) continue;
-        const float bv = bias ? (float)bias[n] : 0.0f;
-        uint32_t again = 0;                                   // results that are not finite, see dot_fp32
+    for (int mb = 0; mb < MB; mb++)
 #pragma unroll
-        for (int mb = 0; mb < MB; mb++)
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-                const int m = m0 + mb * 16 + c * 4 + i;
-                if (m < M) {
-                    y[(int64_t)m * N + n] = to_at<AT>(acc[mb][nb][i] + bv);
-                    again |= __builtin_isfinite(acc[mb][nb][i]) ? 0u : 1u << (mb * 4 + i);
-                }
+        for (int i = 0; i < 16; i++) {
+            const int m = m0 + mb * 32 + i / 4 * 8 + c * 4 + i % 4;
+            if (m < M) {
+                y[(int64_t)m * N + n] = to_at<AT>(acc[mb][i] + bv);
+                again |= __builtin_isfinite(acc[mb][i]) ? 0ull : 1ull << (mb * 16 + i);
             }
-        for (; again; again &= again - 1) {
-            const int bit = __builtin_ctz(again), m = m0 + bit / 4 * 16 + c * 4 + bit % 4;
-            y[(int64_t)m * N + n] = to_at<AT>(dot_fp32<QT, true>(x + (int64_t)m * K, w, n, K) + bv);
         }
+    for (; again; again &= again - 1) {
+        const int bit = __builtin_ctzll(again), m = m0 + bit / 4 * 8 + c * 4 + bit % 4;
+        y[(int64_t)m * N + n] = to_at<AT>(dot_fp32<QT, true>(x + (int64_t)m * K, w, n, K) + bv);
     }
 }
 
@@ -191,13 +309,13 @@ template <int QT, typename AT, int MB>
 __global__ __launch_bounds__(256) void gemm_rows_reduce_kernel(const f32x4 *__restrict__ ws, const AT *__restrict__ x,
                                                                const uint8_t *__restrict__ w, const AT *__restrict__ bias,
                                                                AT *__restrict__ y, int M, int N, int K, int tiles, int splits) {
-    constexpr int PER_TILE = RG_WAVES * MB * RG_NB * 64;     // a multiple of 256
+    constexpr int PER_TILE = RG_WAVES * MB * 4 * 64;         // a multiple of 256
     const int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    const int tiles_m = (M + 16 * MB - 1) / (16 * MB);
+    const int tiles_m = (M + 32 * MB - 1) / (32 * MB);
     const int tile = (int)(t / PER_TILE), in = (int)(t % PER_TILE);
-    const int lane = in & 63, nb = (in >> 6) % RG_NB, mb = (in >> 6) / RG_NB % MB, wave = (in >> 6) / (RG_NB * MB);
-    const int m = tile % tiles_m * 16 * MB + mb * 16 + (lane >> 4) * 4;
-    const int n = tile / tiles_m * RG_N + (wave * RG_NB + nb) * TILE_ROWS + (lane & 15);
+    const int lane = in & 63, q = (in >> 6) & 3, mb = (in >> 8) % MB, wave = (in >> 8) / MB;
+    const int m = tile % tiles_m * 32 * MB + mb * 32 + q * 8 + (lane >> 5) * 4;
+    const int n = tile / tiles_m * RG_N + wave * 32 + (lane & 31);
     if (m >= M || n >= N) return;
     f32x4 a = ws[t];
     for (int s = 1; s < splits; s++) a += ws[(int64_t)s * tiles * PER_TILE + t];
@@ -216,15 +334,22 @@ struct RowsPlan {
     int mb, tiles, steps, splits;
     size_t ws_bytes;
 };
-// Rows of x per workgroup: 128 where that pads M by little more than 64 would, fewer for small batches.  K splits:
-// until the workgroups are about two per CU (the kernel's occupancy), of at least four steps each.
+// Rows of x per workgroup: 128 where that pads M by little more than 64 would, fewer for small batches and where 128 leave
+// CUs idle, K too short to be split for them (200 rows on [1001 x 1088] 13.8 -> 12.1 us in sym_int4, 19.0 -> 15.4 in nf4; 128
+// rows on [4001 x 2112] 17.4 -> 14.9 and 22.6 -> 19.8; with both forms at two workgroups per CU 64 rows lose, 256 rows on
+// [30003 x 4096] 92 -> 124).  K splits: until the workgroups are about two per CU (the kernel's occupancy), of at
+// least four steps each.
 static RowsPlan rows_plan(int M, int N, int K, size_t ws_bytes) {
     RowsPlan p;
     const int pad64 = (M + 63) / 64 * 64, pad128 = (M + 127) / 128 * 128;
-    p.mb = M <= 32 ? 2 : M <= 64 || pad128 * 8 > pad64 * 9 ? 4 : 8;
-    p.tiles = ((M + 16 * p.mb - 1) / (16 * p.mb)) * ((N + RG_N - 1) / RG_N);
+    p.mb = M <= 32 ? 1 : M <= 64 || pad128 * 8 > pad64 * 9 ? 2 : 4;
+    p.tiles = ((M + 32 * p.mb - 1) / (32 * p.mb)) * ((N + RG_N - 1) / RG_N);
     const int G = (K + TILE_COLS - 1) / TILE_COLS;
-    const size_t per_split = (size_t)p.tiles * 16 * p.mb * RG_N * sizeof(float);
+    if (p.mb == 4 && (int64_t)p.tiles * (G / 4 > 1 ? G / 4 : 1) <= 256) {
+        p.mb = 2;
+        p.tiles = ((M + 63) / 64) * ((N + RG_N - 1) / RG_N);
+    }
+    const size_t per_split = (size_t)p.tiles * 32 * p.mb * RG_N * sizeof(float);
     int s = 512 / p.tiles;
     s = s > G / 4 ? G / 4 : s;
     s = s > 16 ? 16 : s;
@@ -245,7 +370,7 @@ static void launch_rows_m(const void *x, const void *w, const void *bias, void *
     hipLaunchKernelGGL((gemm_rows_kernel<QT, AT, MB>), dim3((p.tiles + 7) / 8 * 8, p.splits), dim3(256), 0, st, (const AT *)x,
                        (const uint8_t *)w, (const AT *)bias, (AT *)y, M, N, K, p.steps, ws);
     if (ws)
-        hipLaunchKernelGGL((gemm_rows_reduce_kernel<QT, AT, MB>), dim3((unsigned)((int64_t)p.tiles * RG_WAVES * MB * RG_NB * 64 / 256)),
+        hipLaunchKernelGGL((gemm_rows_reduce_kernel<QT, AT, MB>), dim3((unsigned)((int64_t)p.tiles * RG_WAVES * MB * 4 * 64 / 256)),
                            dim3(256), 0, st, (const f32x4 *)ws, (const AT *)x, (const uint8_t *)w, (const AT *)bias, (AT *)y, M, N, K,
                            p.tiles, p.splits);
 }
@@ -253,9 +378,9 @@ static void launch_rows_m(const void *x, const void *w, const void *bias, void *
 template <int QT, typename AT>
 static int launch_rows_t(const void *x, const void *w, const void *bias, void *y, int M, int N, int K, const RowsPlan &p, float *ws,
                          hipStream_t st) {
-    if (p.mb == 2) launch_rows_m<QT, AT, 2>(x, w, bias, y, M, N, K, p, ws, st);
-    else if (p.mb == 4) launch_rows_m<QT, AT, 4>(x, w, bias, y, M, N, K, p, ws, st);
-    else launch_rows_m<QT, AT, 8>(x, w, bias, y, M, N, K, p, ws, st);
+    if (p.mb == 1) launch_rows_m<QT, AT, 1>(x, w, bias, y, M, N, K, p, ws, st);
+    else if (p.mb == 2) launch_rows_m<QT, AT, 2>(x, w, bias, y, M, N, K, p, ws, st);
+    else launch_rows_m<QT, AT, 4>(x, w, bias, y, M, N, K, p, ws, st);
     return 0;
 }
 
