@@ -44,11 +44,19 @@ __global__ __launch_bounds__(64 * wide_max_waves(MB, DUAL ? 2 * R : R, F32)) voi
     constexpr bool NEED_S = Op::NEED_S;
     constexpr int PARTS = Op::PARTS;
     constexpr int NT = DUAL ? 2 * R : R;                     // weight tiles per group; DUAL: R of the gate, R of the up weight
+    // PEEL: a wave's last group, which loads nothing, stands apart from the loop, and the order of the products is given.  With a
+    // condition around the loads the compiler merged the registers of two groups' weights where the ways met, in the middle of the
+    // products, and waited there for the loads that it had just issued; and it let most products wait for their MFMA.  It takes
+    // some 40 registers more, so only where they are there: with spills a kernel took up to 1.6 times as long.  Old / new
+    // form, fp16 sym_int4: 40 rows on [11008 x 4096] 16.3 / 14.7 us, on [6144 x 2048] 8.6 / 7.7, 64 on [4096 x 4096] 13.7 / 12.2,
+    // 12 on [11008 x 4096] 9.4 / 8.7; 1.05 on average.  Row-major weights and float32 activations: level, not taken.
+    constexpr bool PEEL = !ROWS && !F32 && NT * MB <= (QT == QT_ASYM_INT4 ? 6 : QT == QT_SYM_INT8 || NEED_S ? 8 : 9);
     static_assert(!DUAL || (!F32 && !ROWS), "the fused form takes 16-bit activations and tiled weights");
     constexpr int PLANE = 16 * MB * 256, XBYTES = PLANE * (F32 ? 2 : 1), XC = 4 * MB;     // bytes of x in LDS; chunks of 8 per lane
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
     const ET *const x = (const ET *)x_;
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, W = blockDim.x >> 6, r = lane & 15, c = lane >> 4;
+    const int lane = threadIdx.x & 63, W = blockDim.x >> 6, r = lane & 15, c = lane >> 4;
+    const int wave = PEEL ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : threadIdx.x >> 6;
     uint8_t *const xs = smem + wave * XBYTES;
     const int G = ROWS ? (K + TILE_COLS - 1) / TILE_COLS : K / TILE_COLS, blocks = K / F::QK;
 
@@ -71,8 +79,15 @@ __global__ __launch_bounds__(64 * wide_max_waves(MB, DUAL ? 2 * R : R, F32)) voi
         const bool past = ROWS && col >= K;                  // (put makes zeros of columns past K)
 #pragma unroll
         for (int i = 0; i < XC; i++) {
-            const int m = i * 4 + xrow;
-            const u32x4 *p = (const u32x4 *)(x + (int64_t)(m < M ? m : M - 1) * K + (past ? K - 8 : col));
+            const u32x4 *p;
+            if constexpr (PEEL) {                            // a scalar base per instruction, one lane offset
+                const int first = 4 * i < M ? 4 * i : (M - 1) & ~3, left = M - 1 - first;       // rows past M: the last one
+                const uint32_t at = (uint32_t)xrow * (uint32_t)K, most = (uint32_t)(left < 3 ? left : 3) * (uint32_t)K;
+                p = (const u32x4 *)(x + (int64_t)first * K + g * TILE_COLS + ((at < most ? at : most) + (uint32_t)u * 8u));
+            } else {
+                const int m = i * 4 + xrow;
+                p = (const u32x4 *)(x + (int64_t)(m < M ? m : M - 1) * K + (past ? K - 8 : col));
+            }
 #pragma unroll
             for (int h = 0; h < (F32 ? 2 : 1); h++) xv[i * (F32 ? 2 : 1) + h] = p[h];
         }
@@ -117,59 +132,124 @@ __global__ __launch_bounds__(64 * wide_max_waves(MB, DUAL ? 2 * R : R, F32)) voi
 
     typename std::conditional<ROWS, RowRegs<QT>, TileRegs<QT>>::type wc[NT], wn[NT];
     u32x4 xv[F32 ? 2 * XC : XC];
-    const int first = wave < G ? wave : G - 1;
-    load(first, xv, wn);
-    for (int g = wave; g < G; g += W) {
-#pragma unroll
-        for (int wi = 0; wi < NT; wi++) wc[wi] = wn[wi];
-        // the LDS part is private to the wave, whose LDS operations execute in order: a fence for the compiler is enough
-        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        put(g, xv);
-        if (g + W < G) load(g + W, xv, wn);
-        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        uint32_t hb[NT][4];
-        if constexpr (ROWS) {
-#pragma unroll
-            for (int wi = 0; wi < NT; wi++) arrange_rows<QT>(wc[wi], hb[wi]);
-        }
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-            V8 b[NT][PARTS];
-            float d[NT], e[NT];
+    if constexpr (PEEL) {
+        load(wave, xv, wn);                                  // (no more waves than groups)
+        auto hold = [](auto &t) __attribute__((always_inline)) {
+            asm volatile("" : "+v"(t.q0));
+            if constexpr (F::BITS == 8) asm volatile("" : "+v"(t.q1));
+        };
+        auto group = [&](int g, auto more_) __attribute__((always_inline)) {
+            constexpr bool more = decltype(more_)::value;
 #pragma unroll
             for (int wi = 0; wi < NT; wi++) {
+                wc[wi] = wn[wi];
+                hold(wc[wi]);
+            }
+            // the LDS part is private to the wave, whose LDS operations execute in order: a fence for the compiler is enough
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            put(g, xv);
+            if constexpr (more) load(g + W, xv, wn);
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            // Unit q = (step j, 16-row block mb), in the order the hardware should issue them: the MFMAs of a unit, the LDS read of
+            // the next one's x, the scaling of the unit before, whose results have landed meanwhile.
+            auto read_x = [&](int q) __attribute__((always_inline)) {
+                return *(const V8 *)(xs + (q % MB * 16 + r) * 256 + (((q / MB * 4 + c) ^ r) * 16));
+            };
+            V8 a[2], b[NT][PARTS];
+            float d[2][NT], e[2][NT];                             // of this step and the one before
+            f32x4 p[2][NT], s[2];
+            a[0] = read_x(0);
 #pragma unroll
-                for (int part = 0; part < PARTS; part++) b[wi][part] = op.get(wc[wi], j, part);
-                float mn;
-                if constexpr (ROWS) hdr_to_scale<QT>(hb[wi][j], d[wi], mn);
-                else tile_scale<QT>(wc[wi], j, d[wi], mn);
-                e[wi] = mn - OFFSET * d[wi];
-                d[wi] = Op::scale(d[wi]);
+            for (int q = 0; q <= 4 * MB; q++) {
+                if (q < 4 * MB) {
+                    const int j = q / MB;
+                    if (q % MB == 0) {
+#pragma unroll
+                        for (int wi = 0; wi < NT; wi++) {
+#pragma unroll
+                            for (int part = 0; part < PARTS; part++) b[wi][part] = op.get(wc[wi], j, part);
+                            float mn;
+                            tile_scale<QT>(wc[wi], j, d[j & 1][wi], mn);
+                            e[j & 1][wi] = mn - OFFSET * d[j & 1][wi];
+                            d[j & 1][wi] = Op::scale(d[j & 1][wi]);
+                        }
+                    }
+                    s[q & 1] = NEED_S ? mfma16(a[q & 1], ones, zero4) : zero4;
+#pragma unroll
+                    for (int wi = 0; wi < NT; wi++) p[q & 1][wi] = Op::product(a[q & 1], a[q & 1], b[wi]);
+                    if (q + 1 < 4 * MB) a[(q + 1) & 1] = read_x(q + 1);
+                }
+                if (q > 0) {
+                    const int o = (q - 1) & 1, mb = (q - 1) % MB, j = (q - 1) / MB;
+#pragma unroll
+                    for (int wi = 0; wi < NT; wi++)
+#pragma unroll
+                        for (int i = 0; i < 4; i++)
+                            acc[wi][mb][i] = Op::add(acc[wi][mb][i], d[j & 1][wi], p[o][wi][i], e[j & 1][wi], s[o][i]);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        };
+        int g = wave;
+        for (; g + W < G; g += W) group(g, std::true_type{});
+        group(g, std::false_type{});
+    } else {
+        const int first = wave < G ? wave : G - 1;
+        load(first, xv, wn);
+        for (int g = wave; g < G; g += W) {
+#pragma unroll
+            for (int wi = 0; wi < NT; wi++) wc[wi] = wn[wi];
+            // the LDS part is private to the wave, whose LDS operations execute in order: a fence for the compiler is enough
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            put(g, xv);
+            if (g + W < G) load(g + W, xv, wn);
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            uint32_t hb[NT][4];
+            if constexpr (ROWS) {
+#pragma unroll
+                for (int wi = 0; wi < NT; wi++) arrange_rows<QT>(wc[wi], hb[wi]);
             }
 #pragma unroll
-            for (int mb = 0; mb < MB; mb++) {
-                const uint8_t *at = xs + (mb * 16 + r) * 256 + (((j * 4 + c) ^ r) * 16);
-                const V8 a = *(const V8 *)at;
-                V8 al;
-                if constexpr (F32) al = *(const V8 *)(at + PLANE);
-                f32x4 s = zero4;
-                if constexpr (NEED_S) {
-                    s = mfma16(a, ones, zero4);
-                    if constexpr (F32) s = mfma16(al, ones, s);
-                }
+            for (int j = 0; j < 4; j++) {
+                V8 b[NT][PARTS];
+                float d[NT], e[NT];
 #pragma unroll
                 for (int wi = 0; wi < NT; wi++) {
-                    const f32x4 p = Op::product(a, al, b[wi]);
 #pragma unroll
-                    for (int i = 0; i < 4; i++) acc[wi][mb][i] = Op::add(acc[wi][mb][i], d[wi], p[i], e[wi], s[i]);
+                    for (int part = 0; part < PARTS; part++) b[wi][part] = op.get(wc[wi], j, part);
+                    float mn;
+                    if constexpr (ROWS) hdr_to_scale<QT>(hb[wi][j], d[wi], mn);
+                    else tile_scale<QT>(wc[wi], j, d[wi], mn);
+                    e[wi] = mn - OFFSET * d[wi];
+                    d[wi] = Op::scale(d[wi]);
                 }
+#pragma unroll
+                for (int mb = 0; mb < MB; mb++) {
+                    const uint8_t *at = xs + (mb * 16 + r) * 256 + (((j * 4 + c) ^ r) * 16);
+                    const V8 a = *(const V8 *)at;
+                    V8 al;
+                    if constexpr (F32) al = *(const V8 *)(at + PLANE);
+                    f32x4 s = zero4;
+                    if constexpr (NEED_S) {
+                        s = mfma16(a, ones, zero4);
+                        if constexpr (F32) s = mfma16(al, ones, s);
+                    }
+#pragma unroll
+                    for (int wi = 0; wi < NT; wi++) {
+                        const f32x4 p = Op::product(a, al, b[wi]);
+#pragma unroll
+                        for (int i = 0; i < 4; i++) acc[wi][mb][i] = Op::add(acc[wi][mb][i], d[wi], p[i], e[wi], s[i]);
+                    }
+                }
+#pragma unroll
+                for (int wi = 0; wi < NT; wi++)                   // one step after the other: the scheduler would gather all reads first
+#pragma unroll
+                    for (int mb = 0; mb < MB; mb++) asm volatile("" : "+v"(acc[wi][mb]));
             }
-#pragma unroll
-            for (int wi = 0; wi < NT; wi++)                   // one step after the other: the scheduler would gather all reads first
-#pragma unroll
-                for (int mb = 0; mb < MB; mb++) asm volatile("" : "+v"(acc[wi][mb]));
         }
     }
 
