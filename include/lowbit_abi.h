@@ -234,8 +234,9 @@ int lowbit_forward_f32(const float *x, const void *w, float *y, int qtype, int l
  * LOWBIT_DT_F32: then as lowbit_forward_f32, and no workspace is used.  With 16-bit activations as lowbit_forward_ws
  * (lowbit_linear_workspace_bytes says what to pass within a budget; null is valid), but for two choices that the other entry
  * points, whose kernel a caller may rely on, do not make: the one-pass kernel at 9 .. 64 rows in place of the ring kernel, a K
- * split or several streaming passes, and narrow tiles for nf4 more often.  The bias is added to the fp32 sums before the one
- * rounding (a bias that is not 8-byte aligned is valid and slower above 16 rows).  What LowBitLinear.forward computes
+ * split or several streaming passes, and narrow tiles more often (two groups of waves share such a tile's K where CUs
+ * would idle).  The bias is added to the fp32 sums before the one rounding (a bias that is not 8-byte aligned is valid and
+ * slower above 16 rows).  What LowBitLinear.forward computes
  * (low_bit_linear.py:657-687 of the reference). */
 int lowbit_linear(const void *x, const void *w, const void *bias, void *y, int qtype, int layout, int dtype, int64_t M,
                   int64_t N, int64_t K, void *workspace, size_t workspace_bytes, void *stream);
@@ -282,13 +283,15 @@ int lowbit_grouped_forward(const void *x, const void *const *w, void *y, const i
 /* The same with a workspace (caller-owned device memory, 16-byte aligned, lowbit_grouped_workspace_bytes(...)
  * bytes; null / 0 is valid): when the output alone has too few tiles for the machine - few columns, long K, the
  * down projection of an expert - K is split over a second grid dimension and the fp32 partial tiles are summed
- * from the workspace by a second kernel.  lowbit_grouped_workspace_bytes returns 0 for shapes that do not split. */
+ * from the workspace by a second kernel.  lowbit_grouped_workspace_bytes returns 0 for shapes that do not split; few rows per
+ * group run in tiles of 128 x 128 without a split where those fill the machine. */
 size_t lowbit_grouped_workspace_bytes(int n_groups, int64_t total_rows, int64_t N, int64_t K);
 int lowbit_grouped_forward_ws(const void *x, const void *const *w, void *y, const int32_t *group_offsets,
                               int n_groups, int64_t total_rows, int qtype, int act_dtype, int64_t N, int64_t K,
                               void *workspace, size_t workspace_bytes, void *stream);
 /* Host arithmetic only (no GPU call, like lowbit_forward_plan): how lowbit_grouped_forward(_ws) would run the
- * shape.  plan4 = {256-row tiles (1) or 128-row tiles (0), K splits, waves per workgroup, workgroups per split}.
+ * shape.  plan4 = {256-row tiles (1) or 128-row tiles, of 256 or 128 weight rows (0), K splits, waves per workgroup,
+ * workgroups per split}.
  * Every workgroup of a split launch owns one 256 x 256 fp32 tile of the workspace: splits x workgroups x 256 KiB
  * never exceeds lowbit_grouped_workspace_bytes.  No counterpart in the reference (its expert loop has no plan). */
 int lowbit_grouped_forward_plan(int n_groups, int64_t total_rows, int64_t N, int64_t K, int have_workspace,

@@ -1082,7 +1082,7 @@ __global__ __launch_bounds__(64 * WAVES * KS, (DMA && MB == 4) ? 2 : 1) void gem
                 // long as a load again, however early it had been issued.
                 int cur = 0;
                 auto deep_step = [&](int kt, WRegs &wc, WRegs &wl) __attribute__((always_inline)) {
-                    // (nothing of this step ahead of the barrier that it begins behind: the checker of the assembly pairs
+                    // (nothing of this step ahead of the barrier that it begins behind: the test of the assembly pairs
                     // the wait there with the loads ahead of it)
 #pragma unroll
                     for (int nb = 0; nb < NB32; nb++) {
