@@ -165,7 +165,7 @@ struct ProductBackward : public torch::autograd::Node {
         if (!is_blob(w, grad, qtype, N, K)) throw Failed("the low-bit weight is not where the forward found it");
         const int dt = dtype_code(dtype);
         void *const stream = current_stream(grad);
-        const bool tracked = (c10::GradMode::is_enabled() && grad.requires_grad()) || !nothing_watches(grad);
+        const bool tracked = differentiable(grad) || !nothing_watches(grad);
         if (!tracked && api.backward_applies(qtype, layout, dt, M, N, K)) {
             const Tensor g = grad.contiguous();
             if ((((uintptr_t)g.const_data_ptr() | (uintptr_t)w.const_data_ptr()) & 15) == 0) {
@@ -174,7 +174,7 @@ struct ProductBackward : public torch::autograd::Node {
                 return {gx};
             }
         }
-        // (tracked: a second derivative, or a transform over the backward, goes through the dense product)
+        // (tracked: a second derivative, a tangent or a transform over the backward goes through the dense product)
         const Tensor dense = at::empty({N, K}, w.options().dtype(dtype));
         check(api.dequantize(w.const_data_ptr(), dense.data_ptr(), qtype, N, K, layout, dt, stream), "lowbit_dequantize");
         return {at::matmul(grad, dense).view(x_shape)};

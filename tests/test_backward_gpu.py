@@ -75,9 +75,11 @@ def test_layer_in_training(m, n, k, dtype):
     assert ((product + layer.bias - y).abs() <= eps * (product.abs() / 2 + y.abs())).all()
 
 
-def test_derivatives_that_the_node_leaves_to_operators():
-    """A second derivative, a batch of gradients, a forward-mode tangent and a saved-tensor hook, as MatMulLowBit has them."""
-    m, n, k = 24, 64, 128
+@pytest.mark.parametrize("m,n,k", [(24, 64, 128), (100, 1024, 2560)], ids=["dense", "packed"])
+def test_derivatives_that_the_node_leaves_to_operators(m, n, k):
+    """A second derivative, a batch of gradients, tangents and a saved-tensor hook, as MatMulLowBit has them, at sizes where a plain
+    gradient comes from the packed weight and where it does not."""
+    assert ggml.lowbit_backward_applies(2, TILED, DT[torch.float16], m, n, k) == (n > 64)
     layer = layer_of(2, n, k)
     w = dev_dequantize(layer.weight.data.view(torch.uint8), 2, n, k, TILED, torch.float16)
     x = torch.randn((m, k), device="cuda").half().requires_grad_(True)
@@ -85,13 +87,17 @@ def test_derivatives_that_the_node_leaves_to_operators():
         y = layer(x)
     grad = torch.randn((m, n), device="cuda").half().requires_grad_(True)
     (gx,) = torch.autograd.grad(y, x, grad, create_graph=True)
-    (gg,) = torch.autograd.grad(gx, grad, torch.ones_like(gx), retain_graph=True)
-    assert torch.allclose(gg.float(), w.float().sum(1).expand(m, n), rtol=2e-3, atol=2e-3)
+    v = torch.randn((m, k), device="cuda").half()
+    (gg,) = torch.autograd.grad(gx, grad, v, retain_graph=True)
+    assert close(gg, v, w.t(), torch.float16)
     batch = torch.randn((3, m, n), device="cuda").half()
     (gb,) = torch.autograd.grad(y, x, batch, is_grads_batched=True, retain_graph=True)
     for i in range(3):
         assert close(gb[i], batch[i], w, torch.float16)
     with torch.autograd.forward_ad.dual_level():
+        (gt,) = torch.autograd.grad(y, x, torch.autograd.forward_ad.make_dual(batch[0], batch[1]))
+        primal, tangent = torch.autograd.forward_ad.unpack_dual(gt)
+        assert close(primal, batch[0], w, torch.float16) and close(tangent, batch[1], w, torch.float16)
         dual = torch.autograd.forward_ad.make_dual(x, torch.ones_like(x))
         with pytest.raises(RuntimeError):
             layer(dual)
