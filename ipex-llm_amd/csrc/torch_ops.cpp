@@ -158,8 +158,10 @@ struct ProductBackward : public torch::autograd::Node {
     std::string name() const override { return "MatMulLowBitBackward"; }
 
     torch::autograd::variable_list apply(torch::autograd::variable_list &&grads) override {
-        if (!grads[0].defined() || !task_should_compute_output(0)) return {Tensor()};
-        const Tensor grad = grads[0].to(dtype).reshape({-1, N});
+        if (!task_should_compute_output(0)) return {Tensor()};
+        // (a gradient that a function above left out counts as zeros, as autograd functions in Python are given it)
+        const Tensor grad = grads[0].defined() ? grads[0].to(dtype).reshape({-1, N})
+                                               : at::zeros({c10::multiply_integers(x_shape) / K, N}, w.options().dtype(dtype));
         const int64_t M = grad.size(0);
         c10::DeviceGuard guard(grad.device());
         if (!is_blob(w, grad, qtype, N, K)) throw Failed("the low-bit weight is not where the forward found it");

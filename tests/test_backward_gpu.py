@@ -103,3 +103,23 @@ def test_derivatives_that_the_node_leaves_to_operators(m, n, k):
             layer(dual)
     with torch.no_grad():
         assert not layer(x).requires_grad
+
+
+class LeavesOut(torch.autograd.Function):
+    @staticmethod
+    def forward(ctx, y):
+        return y.clone()
+
+    @staticmethod
+    def backward(ctx, grad):
+        return None
+
+
+@pytest.mark.parametrize("m,n,k", [(24, 64, 128), (100, 1024, 2560)], ids=["dense", "packed"])
+def test_a_gradient_that_is_left_out_counts_as_zeros(m, n, k):
+    """As MatMulLowBit, an autograd function in Python, is given it."""
+    layer = layer_of(2, n, k)
+    x = torch.randn((2, m // 2, k), device="cuda").half().requires_grad_(True)
+    for product in (layer, lambda t: MatMulLowBit.apply(t.view(m, k), layer.weight, n)):
+        (gx,) = torch.autograd.grad(LeavesOut.apply(product(x)).sum(), x)
+        assert gx.shape == x.shape and gx.dtype == x.dtype and not gx.any()
