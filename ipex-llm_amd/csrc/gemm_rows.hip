@@ -11,16 +11,16 @@
 // SIMD.  Hence the 32 x 32 form (half the MFMAs of 16 x 16 x 32 for the same work: 21.0 against 24.7 ns per 32768 products
 // and 8 FMAs), one scaling per block of nf4 and fp8_e4m3 in place of one per 32 columns, and x by LDS-DMA in its own order: the
 // weights are unpacked so that a lane's eight codes are eight consecutive columns, where before x was permuted on its way
-// through registers.  The loads are spread over the step (8 KB of LDS-DMA per wave over its first half, the weights in
-// the middle): all at its head they waited for each other, 7 % of the time in sym_int4 and 13 % in fp8_e4m3.  sym_int8, whose six
-// loads touch the same lines, fetches those by the first code and the headers at the head (another 4 %, and 9 % where the
-// weights come from HBM: 128 rows on [32003 x 4096] 84 / 76 us; fp8_e4m3 loses 5).  Left: the memory
-// system (without the loads of x a step is 15 % shorter), and without FMAs, x and weights still 60 % of it.
+// through registers.  The loads are spread over the step: 8 KB of LDS-DMA per wave over its first half, half of the weights at
+// its head and half in the middle (fp8_e4m3: all in the middle, 5 - 15 % faster than with some at the head).  Everything at
+// the head waits for each other, 7 % of the time in sym_int4 and 13 % in fp8_e4m3; all weights in the middle, the others
+// lose 2 % on average and up to 8 where the weights come from HBM (180 rows on [27966 x 9696] in asym_int4 325 / 313 us).
+// Left: the memory system (without the loads of x a step is 15 % shorter), and without FMAs, x and weights still 60 % of it.
 // Eight waves on 256 weight rows, which halve x's traffic, gain 5 - 9 % on [8008 x 8256] and lose as much elsewhere.
-// 333 rows on [3200 x 8640] with the reduction, before (16 x 16 x 32, x through registers) / now: sym_int4 49.9 / 42.0 us
-// (438 TFLOP/s), asym_int4 68.6 / 62.0, sym_int8 54.3 / 46, nf4 68.2 / 57.9 (fp16, two MFMAs per product) and 83.5 / 69.3
-// (bf16, three), fp8_e4m3 45.9 / 34.5 ([3201 x 8704]); 2000 rows on [4001 x 4160] 109.2 / 93.7 in sym_int4, 96.4 / 73.3 in
-// fp8_e4m3.
+// 333 rows on [3200 x 8640] with the reduction, 16 x 16 x 32 and x through registers / now: sym_int4 52.0 / 42.5 us (433
+// TFLOP/s), asym_int4 67.3 / 64.7, sym_int8 56.3 / 48.6, nf4 70.4 / 59.8 (fp16, two MFMAs per product) and 85.9 / 73.4 (bf16,
+// three), fp8_e4m3 51.2 / 38.9 ([3201 x 8704]); 2000 rows on [4001 x 4160] 115.2 / 92.1 in sym_int4, 125.4 / 107.1 in
+// sym_int8; 1.23 times as fast on average over 1000 points, 3 of them slower by 5 to 8 %.
 #include "lowbit_mfma.h"
 #include "lowbit_rows.h"
 #include "lowbit_unpack.h"
@@ -38,56 +38,95 @@ typedef float f32x16 __attribute__((ext_vector_type(16)));
 __device__ inline f32x16 mfma32(f16x8 a, f16x8 b, f32x16 c) { return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0); }
 __device__ inline f32x16 mfma32(bf16x8 a, bf16x8 b, f32x16 c) { return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0); }
 
-// Codes and headers of 32 weight rows by 128 columns, lane l = 32 * c + r holding 16-byte pieces of row r:
-//   sym_int4, asym_int4   blocks c and 2 + c of the four
-//   nf4                   half c of either block's 32 bytes
-//   8 bits                bytes 16c .. 16c+15 of each 32 columns; sym_int8: headers of blocks c and 2 + c
+// Codes and headers of 32 weight rows by 128 columns, in 16-byte pieces:
+//   sym_int4, sym_int8  lane l = 16 * b + r holds block b of rows r and 16 + r (sym_int8: two pieces each), as the streaming
+//                       kernel's lanes do: the loads that touch a row's lines then follow each other.  With 32 rows to a load
+//                       and a block's half to a lane the lines of a wave's 32 rows, with four waves as much as the L1 holds,
+//                       were often gone before the last load of them (sym_int8: 30 rows on [17069 x 9600] 89.6 us, now 66.4)
+//   asym_int4           lane 32 * c + r: blocks c and 2 + c of row r (its scale leaves the vector units no time for twice the
+//                       lane swaps: in sets 1 % slower over 600 points)
+//   nf4                 lane 32 * c + r: half c of either block's 32 bytes of row r
+//   fp8_e4m3            lane 32 * c + r: bytes 16c .. 16c+15 of each 32 columns of row r
 template <int QT> struct RowRegs32 {
+    static constexpr bool SETS = QT == QT_SYM_INT4 || QT == QT_SYM_INT8;       // pieces in two sets of 16 rows
     static constexpr int NQ = Fmt<QT>::BITS == 8 ? 4 : 2, NH = QT == QT_FP8_E4M3 ? 1 : 2;
     u32x4 q[NQ];
     uint32_t h[NH];
 };
-// Blocks past the end of the row are read from its last one (their scale is made zero).
-template <int QT> __device__ inline void load_rows32(gbytes row, int g, int c, int blocks, RowRegs32<QT> &t, int from = 0, int to = RowRegs32<QT>::NQ) {
+// row: the lane's weight row, SETS: those of either set.  Blocks past the end of the row are read from its last one (their
+// scale is made zero).
+template <int QT> __device__ inline void load_rows32(const gbytes (&row)[2], int g, int lane, int blocks, RowRegs32<QT> &t, int from = 0, int to = RowRegs32<QT>::NQ) {
     using F = Fmt<QT>;
+    using R = RowRegs32<QT>;
     constexpr int PER = TILE_COLS / F::QK;                   // blocks per group of columns
-    auto block = [&](int i) __attribute__((always_inline)) {
+    const int c = lane >> 5;
+    auto block = [&](gbytes row, int i) __attribute__((always_inline)) {
         const int b = g * PER + i;
         return row + (int64_t)(b < blocks ? b : blocks - 1) * F::TS;
     };
+    auto header = [&](gbytes p) __attribute__((always_inline)) -> uint32_t {
+        if constexpr (F::HDR == 2) return *(const __attribute__((address_space(1))) uint16_t *)p;
+        else return *(const __attribute__((address_space(1))) u32_a2 *)p;
+    };
 #pragma unroll
     for (int i = from; i < to; i++) {
-        const gbytes p = QT == QT_NF4 ? block(i) + 16 * c : QT == QT_SYM_INT8 ? block(i) + 16 * c
-                       : QT == QT_FP8_E4M3 ? block(0) + 32 * i + 16 * c : block(2 * i + c);
+        constexpr int EACH = R::NQ / 2;                      // SETS: pieces per set
+        const gbytes p = R::SETS ? block(row[i / EACH], lane >> 4) + i % EACH * 16 : QT == QT_NF4 ? block(row[0], i) + 16 * c
+                       : QT == QT_FP8_E4M3 ? block(row[0], 0) + 32 * i + 16 * c : block(row[0], 2 * i + c);
+        if (R::SETS && i % EACH == 0) t.h[i / EACH] = header(p);
         t.q[i] = *(const __attribute__((address_space(1))) u32x4_a2 *)(p + F::HDR);
     }
-    if (from > 0) return;                                    // (the headers come with the first piece)
+    if constexpr (!R::SETS) {
+        if (from > 0) return;                                // (the headers come with the first piece)
 #pragma unroll
-    for (int i = 0; i < RowRegs32<QT>::NH; i++) {
-        const gbytes p = QT == QT_NF4 ? block(i) : QT == QT_FP8_E4M3 ? block(0) : block(2 * i + c);
-        if constexpr (F::HDR == 2) t.h[i] = *(const __attribute__((address_space(1))) uint16_t *)p;
-        else t.h[i] = *(const __attribute__((address_space(1))) u32_a2 *)p;
+        for (int i = 0; i < R::NH; i++) t.h[i] = header(block(row[0], QT == QT_ASYM_INT4 ? 2 * i + c : i));
     }
 }
-// After this sub-step j (32 columns) has its codes in q[j / 2][2 * (j & 1)] and the next dword (4 bits) or in q[j] (8 bits),
-// and its block's header in hb[j], in all lanes.
+// After this lane 32 * c + r has half c of sub-step j (32 columns) of row r in q[j / 2][2 * (j & 1)] and the next dword (4 bits) or
+// in q[j] (8 bits), and its block's header in hb[j].
 template <int QT> __device__ inline void arrange_rows32(RowRegs32<QT> &t, uint32_t (&hb)[4]) {
     if constexpr (QT == QT_FP8_E4M3) {
         hb[0] = hb[1] = hb[2] = hb[3] = t.h[0];
     } else if constexpr (QT == QT_NF4) {
         hb[0] = hb[1] = t.h[0];
         hb[2] = hb[3] = t.h[1];
-    } else {
+    } else if constexpr (QT == QT_ASYM_INT4) {
 #pragma unroll
         for (int i = 0; i < 2; i++) {
             const auto h = __builtin_amdgcn_permlane32_swap(t.h[i], t.h[i], false, false);
+            const auto a = __builtin_amdgcn_permlane32_swap(t.q[i][0], t.q[i][2], false, false);
+            const auto b = __builtin_amdgcn_permlane32_swap(t.q[i][1], t.q[i][3], false, false);
             hb[2 * i] = h[0];
             hb[2 * i + 1] = h[1];
-            if constexpr (QT != QT_SYM_INT8) {               // lane c: dwords 2c, 2c+1 of both blocks
-                const auto a = __builtin_amdgcn_permlane32_swap(t.q[i][0], t.q[i][2], false, false);
-                const auto b = __builtin_amdgcn_permlane32_swap(t.q[i][1], t.q[i][3], false, false);
-                t.q[i] = u32x4{a[0], b[0], a[1], b[1]};
+            t.q[i] = u32x4{a[0], b[0], a[1], b[1]};
+        }
+    } else {
+        // the set changes places with bit 0 of the block, then the half (4 bits: dwords 0, 1 and 2, 3) with bit 1
+        constexpr bool WIDE = Fmt<QT>::BITS == 8;
+        const RowRegs32<QT> in = t;
+#pragma unroll
+        for (int d = 0; d < (WIDE ? 4 : 2); d++) {
+            uint32_t m[2][2];                                // [block % 2][half]
+#pragma unroll
+            for (int half = 0; half < 2; half++) {
+                const auto v = WIDE ? __builtin_amdgcn_permlane16_swap(in.q[half][d], in.q[WIDE ? 2 + half : 0][d], false, false)
+                                    : __builtin_amdgcn_permlane16_swap(in.q[0][(2 * half + d) % 4], in.q[1][(2 * half + d) % 4], false, false);
+                m[0][half] = v[0];
+                m[1][half] = v[1];
             }
+#pragma unroll
+            for (int odd = 0; odd < 2; odd++) {
+                const auto v = __builtin_amdgcn_permlane32_swap(m[odd][0], m[odd][1], false, false);
+                t.q[WIDE ? odd : 0][WIDE ? d : 2 * odd + d] = v[0];
+                t.q[WIDE ? 2 + odd : 1][WIDE ? d : 2 * odd + d] = v[1];
+            }
+        }
+        const auto h = __builtin_amdgcn_permlane16_swap(t.h[0], t.h[1], false, false);
+#pragma unroll
+        for (int odd = 0; odd < 2; odd++) {
+            const auto v = __builtin_amdgcn_permlane32_swap(h[odd], h[odd], false, false);
+            hb[odd] = v[0];
+            hb[2 + odd] = v[1];
         }
     }
 }
@@ -124,7 +163,12 @@ __global__ __launch_bounds__(256, 2) void gemm_rows_kernel(const AT *__restrict_
     const int blocks = K / F::QK, G = (K + TILE_COLS - 1) / TILE_COLS;
     const int g0 = blockIdx.y * steps, g1 = g0 + steps < G ? g0 + steps : G;
     const int n = n0 + r;
-    const gbytes wr = (gbytes)w + (int64_t)(n < N ? n : N - 1) * blocks * F::TS;
+    gbytes wr[2];
+#pragma unroll
+    for (int i = 0; i < 2; i++) {
+        const int row = RowRegs32<QT>::SETS ? n0 + 16 * i + (lane & 15) : n;
+        wr[i] = (gbytes)w + (int64_t)(row < N ? row : N - 1) * blocks * F::TS;
+    }
 
     // x goes to LDS by itself: the 16 units (16 bytes) of a row's 128 columns in order, but for unit v of row m at v ^ m % 16,
     // so that the 32 rows that an MFMA operand takes a unit of spread over the banks.  A wave's piece i is rows 16i + 4 * wave
@@ -162,7 +206,7 @@ __global__ __launch_bounds__(256, 2) void gemm_rows_kernel(const AT *__restrict_
     const Op op;
 
     RowRegs32<QT> wc, wn;
-    load_rows32<QT>(wr, g0, c, blocks, wc);
+    load_rows32<QT>(wr, g0, lane, blocks, wc);
     dma_x(g0, 0, 0, PIECES);
     land();
     // A step of 128 columns; the last one (more = false) loads nothing.  It stands apart from the loop: with a condition around
@@ -171,12 +215,10 @@ __global__ __launch_bounds__(256, 2) void gemm_rows_kernel(const AT *__restrict_
     int cur = 0;
     auto step = [&](int g, auto more_) __attribute__((always_inline)) {
         constexpr bool more = decltype(more_)::value;
-        if constexpr (more) {
-        }
         uint32_t hb[4];
         arrange_rows32<QT>(wc, hb);
         // MFMA o of the step: 32-row block mb, MFMA s of sub-step j, in the order of the units below
-        constexpr int EARLY = QT == QT_SYM_INT8 ? 1 : 0;     // pieces of the weights loaded at the step's head
+        constexpr int EARLY = QT == QT_FP8_E4M3 ? 0 : RowRegs32<QT>::NQ / 2;    // pieces of the weights loaded at the step's head
         constexpr int PER = 2 * SUB, OPS = NS * MB * PER, AHEAD = 3;
         const uint8_t *const base = xs + cur;
         const int at = r * 256 + ((c * rows32_lane<QT>()) ^ (r & 15)) * 16;
@@ -251,8 +293,8 @@ __global__ __launch_bounds__(256, 2) void gemm_rows_kernel(const AT *__restrict_
 #pragma unroll
                     for (int i = 0; i < PIECES; i++)
                         if (o == i * OPS / (2 * PIECES)) dma_x(g + 1, XBYTES - cur, i, i + 1);
-                    if (EARLY && o == 0) load_rows32<QT>(wr, g + 1, c, blocks, wn, 0, 1);
-                    if (o == OPS / 2) load_rows32<QT>(wr, g + 1, c, blocks, wn, EARLY);
+                    if (EARLY && o == 0) load_rows32<QT>(wr, g + 1, lane, blocks, wn, 0, EARLY);
+                    if (o == OPS / 2) load_rows32<QT>(wr, g + 1, lane, blocks, wn, EARLY);
                 }
                 const V8 v = a[o % (AHEAD + 1)];
                 if constexpr (NEED_S) sum[q & 1] = mfma32(v, ones, sum[q & 1]);

@@ -5,7 +5,7 @@ import pytest
 import torch
 
 import lowbit_oracle as orc
-from gpu_util import ALL, DT, FP8, acts, dev_quantize, ggml, stream, weights
+from gpu_util import ALL, DT, FP8, acts, dev_dequantize, dev_quantize, ggml, stream, weights
 from test_linear_gpu import GGML, _check, classes
 
 pytestmark = pytest.mark.gpu
@@ -35,3 +35,36 @@ def test_infinities_at_the_columns_read_past_the_end(qtype):
         want = x.double().numpy() @ orc.dequantize(orc.quantize(w, qtype), qtype, (n, k)).astype(np.float64).T
     assert (classes(y.float().cpu().numpy()) == classes(want)).all()
     assert (classes(want) > 0).any() and (classes(want) == 0).any()
+
+
+# Tiles of 128 rows, which take more than 256 tiles times splits: K splits where the steps are four times as many or more
+@pytest.mark.parametrize("qtype", ALL)
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("m,n,k,splits", [(333, 3201, 2240, 4), (229, 16523, 192, 1), (97, 16771, 1088, 2), (128, 33003, 96, 1)])
+def test_tiles_of_128_rows(qtype, dtype, m, n, k, splits):
+    """With a workspace and without; last steps of one to three blocks; infinities and a nan among the activations, also at columns
+    that are read past the end."""
+    if qtype in (FP8, 10):
+        k = (k + 127) // 128 * 128 if qtype == FP8 else (k + 63) // 64 * 64
+    tiles = (m + 127) // 128 * ((n + 127) // 128)
+    need = ggml.lowbit_linear_workspace_bytes(qtype, GGML, DT[dtype], m, n, k, 256 << 20)
+    assert need == (splits * tiles * 128 * 128 * 4 if splits > 1 else 0) and tiles * max((k + 127) // 128 // 4, 1) > 256
+    blob, x = dev_quantize(weights(m, (n, k)), qtype, GGML), acts(m, m, k, dtype).cuda()
+    w = dev_dequantize(blob, qtype, n, k, GGML, torch.float32).double()
+    ws, bias = torch.empty(max(need, 16), dtype=torch.uint8, device="cuda"), torch.randn(n, device="cuda").to(dtype)
+    for odd in (False, True):
+        if odd:
+            x[3, k - k % 128 - 128 if k % 128 == 0 else k - k % 128], x[m // 2, k - 3], x[m - 1, 5] = float("inf"), -float("inf"), float("nan")
+        want = x.double() @ w.t()
+        # fp32 sums of at most k / 32 scaled partial sums, themselves fp32; the sum with the bias; one rounding
+        size = x.double().nan_to_num(posinf=0.0, neginf=0.0).abs() @ w.t().abs()
+        bound = size * (k // 32 + 8) * 2.0 ** -24 + (want + bias).abs() * torch.finfo(dtype).eps / 2 * (1 + 2.0 ** -10) + torch.finfo(dtype).smallest_normal
+        for workspace in (ws.data_ptr() if need else None, None):
+            y = torch.full((m + 2, n), float("nan"), dtype=dtype, device="cuda")
+            ggml.lowbit_linear(x.data_ptr(), blob.data_ptr(), bias.data_ptr(), y[1].data_ptr(), qtype, GGML, DT[dtype], m, n, k, workspace,
+                               need if workspace else 0, stream())
+            assert torch.isnan(y[0]).all() and torch.isnan(y[m + 1]).all()
+            got, finite = y[1:m + 1].double(), want.isfinite()
+            assert ((got - want - bias).abs() <= bound)[finite].all()
+            assert (got.isnan() == want.isnan()).all() and (got == want)[want.isinf()].all()
+            assert finite.all() != odd
