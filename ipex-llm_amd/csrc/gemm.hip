@@ -238,24 +238,25 @@ static bool narrow_two_groups(int M, int N, int K) { return narrow_workgroups(M,
 // 1.5 % above the faster of this form and the rest on average; 14 % at worst, [8192 x 8192] at M = 1300);
 // the entry points whose choices lowbit_forward_plan reports keep the figure from before, 1.24.
 // Two groups of waves (lowbit_linear's estimate only): 888 launches, 6.8 % rms; a pair of steps takes 1.49 us, a million
-// weights 0.12 us; scaled by 0.91, with which the shortest estimate is 1.2 % above the fastest kernel on average (600
-// points, ten shapes, 40 .. 1024 rows; 22 % at worst, nf4 [8192 x 8192] at 72 rows).
+// weights 0.12 us; scaled by 0.91.  Never above the estimate of one group, which two groups did not exceed at any of 2500
+// random points: the fit is too long for wide weights of few steps ([26304 x 2432] at 88 rows in sym_int4 26.1 us; where it
+// passed them over, 37.6).  Against the choice with one group the one made with this is 6.2 % faster on average over 2164
+// of them; 20 are slower by 3 to 11 % (a larger scale loses as much elsewhere).
 double narrow_time_us(int M, int N, int K, int qtype, bool linear) {
     const int tiles_m = (M + GM - 1) / GM;
     const bool halves = narrow_halves(M, N);
     const double wgs = (double)narrow_workgroups(M, N);
-    if (linear && narrow_two_groups(M, N, K)) {
-        const double format = qtype == QT_NF4 ? 1.12 : qtype == QT_SYM_INT8 ? 1.16 : qtype == QT_FP8_E4M3 ? 1.14 : 1.0;
-        const double over128 = wgs > 128.0 ? (wgs - 128.0) / 128.0 : 0.0, fill = (double)M / ((double)tiles_m * GM);
-        return 0.91 * (3.86 + 0.97 * over128 + 0.123e-6 * (double)N * (double)K +
-                       (double)((K / TILE_COLS + 1) / 2) * 1.485 * format * (1.0 + 0.17 * over128) * (halves ? 0.79 : 1.0) * (0.69 + 0.31 * fill));
-    }
     const double format = qtype == QT_NF4 ? (linear ? 1.06 : 1.24) : qtype == QT_SYM_INT8 ? 1.11 : qtype == QT_FP8_E4M3 ? 1.05 : 1.0;
     const double over128 = wgs > 128.0 ? (wgs - 128.0) / 128.0 : 0.0;
     const double step = wgs <= 256.0 ? 1.05 + 0.20 * over128 : 1.55 + 0.41 * ((wgs < 512.0 ? wgs : 512.0) - 256.0) / 256.0;
     const double rounds = wgs > 512.0 ? (double)(((int64_t)wgs + 255) / 256) / 2.0 : 1.0;
     const double fill = (double)M / ((double)tiles_m * GM);
-    return 0.5 + (double)(K / TILE_COLS) * step * format * rounds * (halves ? 0.87 : 1.0) * (0.84 + 0.16 * fill);
+    const double one = 0.5 + (double)(K / TILE_COLS) * step * format * rounds * (halves ? 0.87 : 1.0) * (0.84 + 0.16 * fill);
+    if (!linear || !narrow_two_groups(M, N, K)) return one;
+    const double format2 = qtype == QT_NF4 ? 1.12 : qtype == QT_SYM_INT8 ? 1.16 : qtype == QT_FP8_E4M3 ? 1.14 : 1.0;
+    const double two = 0.91 * (3.86 + 0.97 * over128 + 0.123e-6 * (double)N * (double)K +
+                                (double)((K / TILE_COLS + 1) / 2) * 1.485 * format2 * (1.0 + 0.17 * over128) * (halves ? 0.79 : 1.0) * (0.69 + 0.31 * fill));
+    return two < one ? two : one;
 }
 
 // The narrow form of the 128-row DMA kernel: tiles of 128 x 128, or 64 x 128 (narrow_halves).

@@ -485,3 +485,14 @@ def test_linear_asks_for_a_workspace_only_where_its_kernel_uses_one():
     assert need(rows, 333, 3200, 8640) > 0
     assert need(tiled, 100, 4096, 4096, ggml.DT_F32) == 0 and need(tiled, 16, 4096, 4096) == 0
     assert need(tiled, 1 << 40, 4096, 4096) == 0 and need(tiled, 40, 4096, 4096, qtype=99) == 0
+
+
+def test_two_groups_of_waves_are_not_estimated_longer_than_one():
+    """lowbit_linear's estimate of narrow tiles: at wide weights of few steps, [26304 x 2432] at 88 rows, the fit of the form with two
+    groups alone is above the form with one, which it never exceeds, and loses to slower kernels."""
+    time_us = ggml._lib["_ZN6lowbit14narrow_time_usEiiiib"]          # lowbit::narrow_time_us(M, N, K, qtype, linear)
+    time_us.argtypes, time_us.restype = [ctypes.c_int] * 4 + [ctypes.c_bool], ctypes.c_double
+    for qtype in (2, 3, 8, 15):                                       # (nf4: another figure for one group too)
+        for m, n, k in [(88, 26304, 2432), (360, 10416, 1152), (116, 15568, 1024), (43, 26352, 1280), (256, 2048, 2048), (586, 3216, 6016)]:
+            assert time_us(m, n, k, qtype, True) <= time_us(m, n, k, qtype, False)
+    assert ggml.lowbit_linear_workspace_bytes(2, ggml.LAYOUT_TILED, ggml.DT_F16, 256, 2048, 2048, 256 << 20) == 0
