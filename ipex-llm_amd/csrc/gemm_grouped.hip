@@ -79,18 +79,39 @@ static bool grouped_one_round(int total_rows, int n_groups, int tiles_n, bool ta
     return row_tiles >= 8 && (int64_t)row_tiles * tiles_n * splits <= (int64_t)device_cus() * (tall ? 1 : 2);
 }
 
+// Narrow tiles of a grouped launch: how many groups of waves (0: another form) and the column tiles per cell.
+struct NarrowPlan {
+    int groups, chunk;
+};
+
 // Whether a grouped launch takes narrow tiles (128 rows by 128 weight rows, of both weights 64), and with how many groups of
 // waves: 2 while its tiles (an estimate: the host never sees the offsets) are one per CU at most and K has eight steps, 1
 // while they are two per CU, 0 beyond.  The fused form's tall tiles are a quarter as many and leave CUs idle there, whole
 // experts, us: 15 of [896 x 2048] in nf4 with 114 tokens, two each, 54.9 -> 46.4, 9 of [640 x 1920] in sym_int8 with 93
 // tokens, four each, 44.5 -> 39.7, 9 of [1536 x 3968] in sym_int4 with 496 tokens 122.9 -> 109.4; more tiles: 12 of
 // [7168 x 2048] in fp8_e4m3 with 300 tokens 169.7 / 178.7, 8 of [14336 x 4096] with 512 492 / 586.
-static int grouped_narrow(int total_rows, int n_groups, int tiles_n, int K) {
-    const int rows = G_GM_TALL / 2;
-    const int row_tiles = total_rows > 64 * n_groups ? total_rows / rows + (n_groups + 1) / 2 : n_groups;
+// A group counts as one row tile up to 64 rows on average, else as half a tile more than its rows fill, and as whole tiles at
+// least if all have the same (21 of [1872 x 2304] with 2924 tokens in sym_int8 are 630 tiles: 42.8 us in the 128-row form, 66.6 in
+// narrow tiles).
+// The cells are the largest ones with which no XCD gets more tiles than its CUs hold at once - whole rows of column tiles, an
+// eighth, halves of that - because the tiles are about as many as the CUs hold, and a cell more than the others is a second
+// round.  A row tile more than the estimate is reckoned with where groups may be uneven.  Whole rows whatever the XCDs' shares,
+// as before / now, us: 18 of [720 x 3712] in sym_int8 with 202 tokens, fused, 43.7 / 24.2, 10 of [1088 x 10752] in fp8_e4m3 with
+// 178 110 / 69, 18 of [1600 x 1664] in sym_int4 with 179, plain, 21.0 / 13.8, 10 of [6032 x 9856] with 300 203 / 104.
+// Random sizes against the forms that narrow tiles replaced: 1.17 times as fast over 3800 fused launches and 1.22 over 6000
+// plain ones, 2 and 1 % of them slower by more than 4 % (at worst 0.79 and 0.75: tiles that all but fill the CUs).
+static NarrowPlan grouped_narrow(int total_rows, int n_groups, int tiles_n, int K) {
+    const int rows = G_GM_TALL / 2, cus = device_cus();
+    const int uneven = total_rows / rows + (n_groups + 1) / 2, even = (total_rows / n_groups + rows - 1) / rows * n_groups;
+    const int row_tiles = total_rows > 64 * n_groups ? (uneven > even ? uneven : even) : n_groups;
     const int64_t tiles = (int64_t)row_tiles * tiles_n;
-    if (tiles > 2 * device_cus()) return 0;
-    return tiles <= device_cus() && K / TILE_COLS >= 8 ? 2 : 1;
+    if (tiles > 2 * cus) return {0, 0};
+    const int groups = tiles <= cus && K / TILE_COLS >= 8 ? 2 : 1, most = cus / 8 * (groups == 2 ? 1 : 2);
+    const int unsure = total_rows > 32 * n_groups ? 1 : 0;
+    const bool whole = row_tiles >= 8 && grouped_grid(row_tiles + unsure, tiles_n, tiles_n) <= 8 * most;
+    int chunk = whole ? tiles_n : (tiles_n + 7) / 8;
+    while (chunk > 1 && grouped_grid(row_tiles, tiles_n, chunk) > 8 * most) chunk = (chunk + 1) / 2;
+    return {groups, chunk};
 }
 
 GroupedPlan grouped_plan(int total_rows, int n_groups, int N, int K, size_t ws_bytes) {
@@ -105,11 +126,11 @@ GroupedPlan grouped_plan(int total_rows, int n_groups, int N, int K, size_t ws_b
     // Narrow tiles in place of either unsplit form (the same experts, down projection: 54.9 -> 46.9, 44.5 -> 42.4, 122.9 ->
     // 116.4), and of two splits where each tile has a CU and groups are small: the halves of K then meet without a second
     // launch (16 of [2048 x 4096] in nf4 with 300 tokens, two each, 126.0 -> 119.7).
-    const int tiles_narrow = (N + G_GN / 2 - 1) / (G_GN / 2), narrow = grouped_narrow(total_rows, n_groups, tiles_narrow, K);
-    if (s == 1 ? narrow > 0 : s == 2 && narrow == 2 && total_rows <= 96 * n_groups)
-        return {false, 1, 4 * narrow, grouped_one_round(total_rows, n_groups, tiles_narrow, false, 1), narrow};
+    const NarrowPlan narrow = grouped_narrow(total_rows, n_groups, (N + G_GN / 2 - 1) / (G_GN / 2), K);
+    if (s == 1 ? narrow.groups > 0 : s == 2 && narrow.groups == 2 && total_rows <= 96 * n_groups)
+        return {false, 1, 4 * narrow.groups, narrow.chunk, narrow.groups};
     const bool tall = s > 1 || (int64_t)total_rows > (int64_t)n_groups * 96;
-    return {tall, s, grouped_waves(total_rows, n_groups, false), grouped_one_round(total_rows, n_groups, tiles_n, tall, s)};
+    return {tall, s, grouped_waves(total_rows, n_groups, false), grouped_chunk(tiles_n, grouped_one_round(total_rows, n_groups, tiles_n, tall, s))};
 }
 
 // What launch_grouped_gemm would do for a plain grouped product: {tall, splits, waves, grid.x}.
@@ -119,8 +140,7 @@ void grouped_plan_query(int total_rows, int n_groups, int N, int K, size_t ws_by
     out[0] = p.tall;
     out[1] = p.splits;
     out[2] = p.tall || p.narrow ? p.waves : 4;
-    out[3] = p.tall ? tall_grid(total_rows, n_groups, tiles_n, p.one_round)
-                    : grouped_grid(grouped_max_row_tiles(total_rows, n_groups, G_GM_TALL / 2), tiles_n, grouped_chunk(tiles_n, p.one_round));
+    out[3] = grouped_grid(grouped_max_row_tiles(total_rows, n_groups, p.tall ? G_GM_TALL : G_GM_TALL / 2), tiles_n, p.chunk);
 }
 
 size_t grouped_workspace_bytes(int total_rows, int n_groups, int N, int K) {
@@ -129,10 +149,10 @@ size_t grouped_workspace_bytes(int total_rows, int n_groups, int N, int K) {
 }
 
 static GroupedPlan grouped_mlp_plan(int total_rows, int n_groups, int N, int K) {
-    const int tiles_narrow = (N + G_GN / 4 - 1) / (G_GN / 4), narrow = grouped_narrow(total_rows, n_groups, tiles_narrow, K);
-    if (narrow) return {false, 1, 4 * narrow, grouped_one_round(total_rows, n_groups, tiles_narrow, false, 1), narrow};
-    return {true, 1, grouped_waves(total_rows, n_groups, true),
-            grouped_one_round(total_rows, n_groups, (N + G_GN / 2 - 1) / (G_GN / 2), true, 1)};
+    const NarrowPlan narrow = grouped_narrow(total_rows, n_groups, (N + G_GN / 4 - 1) / (G_GN / 4), K);
+    if (narrow.groups) return {false, 1, 4 * narrow.groups, narrow.chunk, narrow.groups};
+    const int tiles_n = (N + G_GN / 2 - 1) / (G_GN / 2);
+    return {true, 1, grouped_waves(total_rows, n_groups, true), grouped_chunk(tiles_n, grouped_one_round(total_rows, n_groups, tiles_n, true, 1))};
 }
 
 // y[rows of group e] = x[rows of group e] * dequant(w[e])^T, or, with w_up, act(x w[e]^T) * (x w_up[e]^T).
@@ -167,7 +187,7 @@ static GroupedPlan mlp_plan(int M, int N, int K) {
     const int64_t tiles = (int64_t)tiles_m * ((N + G_GN / 4 - 1) / (G_GN / 4));
     const int tall_n = (N + G_GN / 2 - 1) / (G_GN / 2);
     const int64_t tall = (int64_t)((M + G_GM_TALL - 1) / G_GM_TALL) * tall_n;
-    GroupedPlan plan = {true, 1, grouped_waves(M, 1, true), grouped_one_round(M, 1, tall_n, true, 1)};
+    GroupedPlan plan = {true, 1, grouped_waves(M, 1, true), grouped_chunk(tall_n, grouped_one_round(M, 1, tall_n, true, 1))};
     if (tiles <= cus && K / TILE_COLS >= 8) plan.narrow = 2;
     else if ((tiles <= 2 * cus && (M > rows || tiles <= cus)) || (tall > cus && tall * 20 <= (int64_t)cus * 27)) plan.narrow = 1;
     plan.halves = plan.narrow && M > rows / 2 && 2 * tiles <= cus;

@@ -68,7 +68,7 @@ template <int QT, typename AT>
 static int launch_grouped_t(const void *x, const void *const *w, void *y, const int32_t *offsets, int n_groups,
                             int total_rows, int N, int K, const GroupedPlan &plan, float *ws, hipStream_t st) {
     if (plan.narrow) {
-        const int tiles_n = (N + GN / 2 - 1) / (GN / 2), G = K / TILE_COLS, chunk = grouped_chunk(tiles_n, plan.one_round);
+        const int tiles_n = (N + GN / 2 - 1) / (GN / 2), G = K / TILE_COLS, chunk = plan.chunk;
         const GroupArgs ga = {offsets, (const uint8_t *const *)w, nullptr, n_groups, 0, 0, chunk};
         const int grid = grouped_grid(grouped_max_row_tiles(total_rows, n_groups, GM), tiles_n, chunk);
         if (plan.narrow == 2)
@@ -80,7 +80,7 @@ static int launch_grouped_t(const void *x, const void *const *w, void *y, const 
         return 0;
     }
     const int tiles_n = (N + GN - 1) / GN, G = K / TILE_COLS;
-    const int chunk = grouped_chunk(tiles_n, plan.one_round);
+    const int chunk = plan.chunk;
     const GroupArgs ga = {offsets, (const uint8_t *const *)w, nullptr, n_groups, 0, 0, chunk};
     if (!plan.tall) {
         const int grid = grouped_grid(grouped_max_row_tiles(total_rows, n_groups, GM), tiles_n, chunk);
@@ -107,7 +107,7 @@ static int launch_grouped_mlp_t(const void *x, const void *const *wg, const void
                                 const int32_t *offsets, int n_groups, int total_rows, int N, int K, int act,
                                 const GroupedPlan &plan, hipStream_t st) {
     if (plan.narrow) {
-        const int tiles_n = (N + GN / 4 - 1) / (GN / 4), G = K / TILE_COLS, chunk = grouped_chunk(tiles_n, plan.one_round);   // 64 columns of both
+        const int tiles_n = (N + GN / 4 - 1) / (GN / 4), G = K / TILE_COLS, chunk = plan.chunk;   // 64 columns of both
         const GroupArgs ga = {offsets, (const uint8_t *const *)wg, (const uint8_t *const *)wu, n_groups, act, 0, chunk};
         const int grid = grouped_grid(grouped_max_row_tiles(total_rows, n_groups, GM), tiles_n, chunk);
         if (plan.narrow == 2)
@@ -119,7 +119,7 @@ static int launch_grouped_mlp_t(const void *x, const void *const *wg, const void
         return 0;
     }
     const int tiles_n = (N + GN / 2 - 1) / (GN / 2), G = K / TILE_COLS;      // 128 columns of both weights per workgroup
-    const int chunk = grouped_chunk(tiles_n, plan.one_round);
+    const int chunk = plan.chunk;
     const GroupArgs ga = {offsets, (const uint8_t *const *)wg, (const uint8_t *const *)wu, n_groups, act, 0, chunk};
     const int n_wg = grouped_grid(grouped_max_row_tiles(total_rows, n_groups, GM_TALL), tiles_n, chunk);
     // nf4 always takes the eight-wave form: its two waves per SIMD cover each other's code book reads (the dense
@@ -157,7 +157,7 @@ static int launch_mlp_gemm_t(const void *x, const void *wg, const void *wu, void
         return 0;
     }
     const int tiles_n = (N + GN / 2 - 1) / (GN / 2), G = K / TILE_COLS;
-    const int chunk = grouped_chunk(tiles_n, plan.one_round);
+    const int chunk = plan.chunk;
     const GroupArgs ga = {nullptr, nullptr, nullptr, 1, act, 0, chunk, (const uint8_t *)wu};
     const int n_wg = grouped_grid((M + GM_TALL - 1) / GM_TALL, tiles_n, chunk);
     if (plan.waves == 8 || QT == QT_NF4) {            // (nf4: see launch_grouped_mlp_t)

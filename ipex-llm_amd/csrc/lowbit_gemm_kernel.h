@@ -68,8 +68,8 @@ struct GroupArgs {
 //     for x to arrive from beyond L2);
 //   - with chunk = ceil(tiles_n / 8) every XCD gets one cell of every row tile: equal shares however uneven the
 //     groups are (a group per XCD was 9-12 % slower with 10 to 300 rows per group);
-//   - with chunk = tiles_n a row tile is one cell: all its column tiles on one XCD, for launches of a single round,
-//     where shares do not matter.
+//   - with chunk = tiles_n a row tile is one cell: all its column tiles on one XCD, for launches of a single round.
+//     Shares matter there only where they make a second round of the largest one (narrow tiles: grouped_narrow).
 // Workgroups beyond an XCD's last cell leave at once; they are the last of that XCD's sequence (workgroups go to
 // the compute units of an XCD in turn: idle ones between working ones leave units idle).
 struct GroupTile {

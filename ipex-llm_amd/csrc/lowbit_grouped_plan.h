@@ -14,7 +14,7 @@ struct GroupedPlan {
     bool tall;      // 256-row tiles
     int splits;     // K splits of the tall form (1 = none)
     int waves;      // waves per workgroup of the tall form: 4 (64 weight rows each) or 8 (32 each, two per SIMD); of narrow tiles
-    bool one_round; // the launch's workgroups (expected count) all fit the machine at once
+    int chunk;      // column tiles per cell of the tile order (grouped_tile in lowbit_gemm_kernel.h)
     int narrow = 0; // narrow tiles, with one or two groups of waves (0: not)
     bool halves = false;   // narrow tiles of a dense gated MLP: in halves of 64 rows
 };
@@ -22,9 +22,8 @@ struct GroupedPlan {
 // Upper bound of the number of `rows`-row tiles: every group adds at most one partly filled tile.
 inline int grouped_max_row_tiles(int total_rows, int n_groups, int rows) { return total_rows / rows + n_groups; }
 
-// Column tiles per cell of the tile order (grouped_tile in lowbit_gemm_kernel.h): a whole row of column tiles when
-// the launch is a single round of workgroups, else an eighth of it, so that every XCD gets an equal share of
-// every row tile.
+// Column tiles per cell of the 128-row and the tall form: a whole row of column tiles when the launch is a single round of
+// workgroups, else an eighth of it, so that every XCD gets an equal share of every row tile.
 inline int grouped_chunk(int tiles_n, bool one_round) { return one_round ? tiles_n : (tiles_n + 7) / 8; }
 
 // Workgroups (grid.x) of a grouped launch over at most `row_tiles` row tiles: 8 XCDs x the most cells one of them

@@ -310,3 +310,25 @@ def test_lane_lookup_agrees_with_the_walk_over_the_offsets(n_groups):
             got = [grouped_tile_lanes(offs, tiles_n, chunk, b) for b in range(n_wg)]
             assert got == [grouped_tile(offs, tiles_n, chunk, b) for b in range(n_wg)]
             assert sum(g is not None for g in got) == row_tiles * tiles_n
+
+
+def test_no_xcd_gets_a_second_round_of_narrow_tiles():
+    """Narrow tiles are chosen where they are one (two groups of waves) or two per CU at most: then no XCD may get more of them than
+    its 32 CUs hold.  Up to 127 rows a group has one row tile, and the launch is as large as the estimate says."""
+    import ctypes
+    import ipex_llm.ggml.model.llama.llama_cpp as ggml
+    plan = (ctypes.c_int * 4)()
+    seen = set()
+    for groups in range(1, 60):
+        for n in range(16, 8000, 208):
+            for k in (512, 1536, 4096):
+                tiles = groups * ((n + 127) // 128)
+                assert ggml._lib.lowbit_grouped_forward_plan(groups, 100, n, k, 0, 0, plan) == 0
+                tall, splits, waves, wgs = plan
+                if tall or splits > 1 or tiles > 512:
+                    continue
+                two = tiles <= 256 and k >= 1024
+                assert waves == (8 if two else 4)
+                assert wgs <= (256 if two else 512), (groups, n, k, wgs)
+                seen.add((two, wgs))
+    assert len(seen) > 50
