@@ -40,7 +40,13 @@ __host__ __device__ inline uint32_t wide_row_chunks(int xrow, int left, int K) {
     return at < most ? at : most;
 }
 
-template <int QT, typename AT, int MB, int R, bool F32, bool ROWS, bool DUAL>
+// Whether a form's last group stands apart (PEEL in the kernel)
+template <int QT, typename AT, int MB, int R, bool F32, bool ROWS, bool DUAL> constexpr bool wide_peels() {
+    return !ROWS && !F32 && (DUAL ? 2 * R : R) * MB <= (QT == QT_ASYM_INT4 ? 6 : QT == QT_SYM_INT8 || Operand<QT, AT, F32, ROWS>::NEED_S ? 8 : 9);
+}
+
+// CROWD: the fused form without PEEL, see launch_wide_r
+template <int QT, typename AT, int MB, int R, bool F32, bool ROWS, bool DUAL, bool CROWD = false>
 __global__ __launch_bounds__(64 * wide_max_waves(MB, DUAL ? 2 * R : R, F32)) void gemv_wide_kernel(
     const void *__restrict__ x_, const uint8_t *__restrict__ w, const uint8_t *__restrict__ w_up, const void *__restrict__ bias_,
     void *__restrict__ y_, int M, int N, int K, int act) {
@@ -58,7 +64,7 @@ __global__ __launch_bounds__(64 * wide_max_waves(MB, DUAL ? 2 * R : R, F32)) voi
     // some 40 registers more, so only where they are there: with spills a kernel took up to 1.6 times as long.  Old / new
     // form, fp16 sym_int4: 40 rows on [11008 x 4096] 16.3 / 14.7 us, on [6144 x 2048] 8.6 / 7.7, 64 on [4096 x 4096] 13.7 / 12.2,
     // 12 on [11008 x 4096] 9.4 / 8.7; 1.05 on average.  Row-major weights and float32 activations: level, not taken.
-    constexpr bool PEEL = !ROWS && !F32 && NT * MB <= (QT == QT_ASYM_INT4 ? 6 : QT == QT_SYM_INT8 || NEED_S ? 8 : 9);
+    constexpr bool PEEL = !CROWD && wide_peels<QT, AT, MB, R, F32, ROWS, DUAL>();
     static_assert(!DUAL || (!F32 && !ROWS), "the fused form takes 16-bit activations and tiled weights");
     constexpr int PLANE = 16 * MB * 256, XBYTES = PLANE * (F32 ? 2 : 1), XC = 4 * MB;     // bytes of x in LDS; chunks of 8 per lane
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
@@ -307,6 +313,18 @@ struct WideShape {
     int r, waves;
 };
 
+// Workgroups of four waves that the GPU holds at once, in either form
+struct WideRoom {
+    int peel, crowd;
+};
+inline WideRoom wide_room(const void *peel, const void *crowd, size_t lds) {
+    int dev = 0, cus = 0, a = 0, b = 0;
+    if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
+        hipOccupancyMaxActiveBlocksPerMultiprocessor(&a, peel, 256, lds) != hipSuccess ||
+        hipOccupancyMaxActiveBlocksPerMultiprocessor(&b, crowd, 256, lds) != hipSuccess) return {0, 0};
+    return {a * cus, b * cus};
+}
+
 template <int QT, typename AT, int MB, int R, bool F32, bool ROWS, bool DUAL>
 static int launch_wide_r(const void *x, const void *w, const void *w_up, const void *bias, void *y, int M, int N, int K, int act,
                          int waves, hipStream_t st) {
@@ -320,8 +338,16 @@ static int launch_wide_r(const void *x, const void *w, const void *w_up, const v
     // the default limit of dynamic LDS is 64 KB; raised once per process (thread-safe static), on the one GPU this library drives
     static const hipError_t raised = hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, LDS);
     if (raised != hipSuccess) return -6;
-    hipLaunchKernelGGL(kern, dim3((N + TILE_ROWS * R - 1) / (TILE_ROWS * R)), dim3(64 * wv), (size_t)wv * XBYTES, st, x, (const uint8_t *)w,
-                       (const uint8_t *)w_up, bias, y, M, N, K, act);
+    const int wgs = (N + TILE_ROWS * R - 1) / (TILE_ROWS * R);
+    if constexpr (DUAL && wide_peels<QT, AT, MB, R, F32, ROWS, DUAL>()) {
+        // The registers of PEEL let a CU hold fewer workgroups of four waves, in several of these forms two in place of three:
+        // with more than that the others wait for a second round.  With PEEL / without: 22 rows on [9376 x 768] in bf16 sym_int4
+        // 9.0 / 7.4 us, 37 on [10336 x 768] in fp16 nf4 11.0 / 9.8, 26 on [9920 x 1152] in bf16 sym_int8 12.3 / 10.5.
+        auto crowd = gemv_wide_kernel<QT, AT, MB, R, F32, ROWS, DUAL, true>;
+        static const WideRoom room = wide_room((const void *)kern, (const void *)crowd, 4 * XBYTES);
+        if (wv == 4 && room.crowd > room.peel && wgs > room.peel) kern = crowd;
+    }
+    hipLaunchKernelGGL(kern, dim3(wgs), dim3(64 * wv), (size_t)wv * XBYTES, st, x, (const uint8_t *)w, (const uint8_t *)w_up, bias, y, M, N, K, act);
     return 0;
 }
 

@@ -5,7 +5,7 @@ import pytest
 import torch
 
 import lowbit_oracle as orc
-from gpu_util import ALL, FP8, acts, dev_quantize, weights
+from gpu_util import ALL, FP8, NF4, acts, dev_dequantize, dev_quantize, weights
 from ipex_llm.transformers.low_bit_linear import mlp_forward_xpu
 from ipex_llm.transformers.models.utils import SILU
 from test_linear_gpu import GGML, TILED, _check, classes
@@ -49,6 +49,25 @@ def test_fused_gate_up(qtype, m, n, k):
     g, u = (orc.mul_mat_exact(orc.quantize(w, qtype), x.float().numpy(), (n, k), qtype) for w in (wg, wu))
     want = g / (1.0 + np.exp(-g)) * u
     assert np.abs(y - want).max() <= (2e-3 if dtype == torch.float16 else 8e-3) * np.abs(want).max()
+
+
+@pytest.mark.parametrize("qtype", ALL)
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("m,n,k", [(12, 16400, 640), (20, 8336, 512), (40, 8336, 640), (48, 12304, 1152)])
+def test_fused_gate_up_of_many_workgroups(qtype, dtype, m, n, k):
+    """More workgroups of four waves than the GPU holds at once in the form of more registers; K of as many groups as waves, and more."""
+    blobs = [dev_quantize(weights(m + i, (n, k)), qtype, TILED) for i in range(2)]
+    x = acts(m, m, k, dtype).cuda()
+    y = mlp_forward_xpu(x, *blobs, m, k, n, SILU, qtype).double()
+    eps = torch.finfo(dtype).eps
+    # fp32 sums of exact products; the levels of nf4 are rounded to x's type
+    err = k * 2.0 ** -24 + (eps / 2 if qtype == NF4 else 0.0)
+    (g, dg), (u, du) = ((x.double() @ w.t(), x.double().abs() @ w.abs().t() * err)
+                        for w in (dev_dequantize(b, qtype, n, k, TILED, torch.float32).double() for b in blobs))
+    a = g * torch.sigmoid(g)
+    # one rounding; exp2 and rcp of an ulp each; silu's slope is at most 1.13
+    bound = (a * u).abs() * (eps / 2 + 2.0 ** -20) + 1.13 * dg * u.abs() + a.abs() * du + dg * du + torch.finfo(dtype).smallest_normal
+    assert ((y - a * u).abs() <= bound).all()
 
 
 @pytest.mark.parametrize("qtype", ALL)
