@@ -73,7 +73,7 @@ __device__ inline float load_route_w(const void *w, int dtype, int pair) {
 // kernel.  A row of a tile is 72 .. 136 contiguous bytes instead of a 1 KiB tile; a workgroup's waves take
 // neighbouring columns, so lines are shared within the workgroup only.  (One wave per weight row and a scalar decode
 // per weight, four rows of x a pass, took 74 us per pass for [32003 x 4096] in asym_int4: two at eight rows, which now take
-// 26.2 us in bf16.)
+// 27.1 us in bf16, 25.8 in fp16.)
 template <int QT, typename AT, int MT, int U, int XN, bool DUAL, int MOE, int R, bool F32, bool ROWS>
 __global__ __launch_bounds__(1024) void gemv_mfma_kernel(const AT *__restrict__ x, const uint8_t *__restrict__ w,
                                                          const uint8_t *__restrict__ w2, AT *__restrict__ y,
@@ -91,6 +91,12 @@ __global__ __launch_bounds__(1024) void gemv_mfma_kernel(const AT *__restrict__ 
     constexpr bool AGAIN = ROWS || MOE != 0;
     constexpr int SLICE = U * TILE_COLS;                    // columns of x per wave and round
     constexpr bool ZERO_X = XN == 1 || ROWS;                // how tiles past K are silenced (see the x loads)
+    // With two planes of x that gains nothing and loses up to 15 % (5 rows on [2593 x 11648] in fp8_e4m3 13.8 -> 16.2 us), and the
+    // forms left out with 16 bits lose up to 12 % at some sizes (3 rows on [32003 x 4096] in sym_int8 50 -> 52, 8 rows in asym_int4
+    // 28.8 -> 30.1).  10000 random sizes: 1.008 times as fast with it as without, at worst 0.91 (asym_int4, 4 rows on
+    // [3505 x 9792] 9.2 -> 10.1).
+    constexpr bool ZERO_LATE = ROWS && XN > 1 && !F32 && !(MT == 2 && (QT == QT_FP8_E4M3 || QT == QT_ASYM_INT4)) &&
+                               !(MT == 1 && XN == 4 && QT == QT_SYM_INT8);
     constexpr int XREGION = XN * 512 * (F32 ? 2 : 1);       // elements of AT in a wave's part of LDS
 
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
@@ -187,23 +193,22 @@ __global__ __launch_bounds__(1024) void gemv_mfma_kernel(const AT *__restrict__ 
             // one select per round where zeroing the scales is one per sub-block (M = 1: [11008 x 4096] 6.23 ->
             // 6.15 us, [28672 x 8192] 24.8 -> 23.8); with more chunks per lane the same change cost 5-20 %, and
             // those shapes zero the scales (below).
-            // Row-major weights with more chunks select where x goes to LDS: here the select waits for x in front of the loads
-            // of the weights ([32003 x 4096] at 8 rows 27.0 -> 26.2 us in asym_int4, 56.0 -> 53.2 in sym_int8, at 3 rows 22.5 -> 21.0
-            // in asym_int4; 1.03 times over 60 points, sym_int8 at 3 rows 50 -> 52 the one loss).  With one chunk the
-            // compiler has moved it behind them by itself.
+            // Row-major weights with more chunks select where x goes to LDS (ZERO_LATE): here the select waits for x in front of
+            // the loads of the weights (8 rows on [32003 x 4096] in sym_int8 56.0 -> 53.2 us).  With one chunk the compiler has
+            // moved it behind them by itself.
             const bool past = col >= K;
             col = past ? K - 8 : col;
             if constexpr (F32) {
                 const u32x4 *xp = (const u32x4 *)((const float *)x + (int64_t)m * K + col);
                 xv[2 * i] = xp[0];
                 xv[2 * i + 1] = xp[1];
-                if constexpr (ZERO_X && XN == 1) {
+                if constexpr (ZERO_X && !ZERO_LATE) {
                     xv[2 * i] = past ? u32x4{0u, 0u, 0u, 0u} : xv[2 * i];
                     xv[2 * i + 1] = past ? u32x4{0u, 0u, 0u, 0u} : xv[2 * i + 1];
                 }
             } else {
                 xv[i] = *(const u32x4 *)(x + (int64_t)m * K + col);
-                if constexpr (ZERO_X && XN == 1) xv[i] = past ? u32x4{0u, 0u, 0u, 0u} : xv[i];
+                if constexpr (ZERO_X && !ZERO_LATE) xv[i] = past ? u32x4{0u, 0u, 0u, 0u} : xv[i];
             }
         }
         __builtin_amdgcn_sched_barrier(0);                  // keep the x loads ahead of the weight loads
@@ -250,13 +255,9 @@ __global__ __launch_bounds__(1024) void gemv_mfma_kernel(const AT *__restrict__ 
                 if constexpr (ROWS) store_x_rows<QT>((uint8_t *)(plane + at / (SLICE / 8) * SLICE), at % (SLICE / 8), v);
                 else *(u32x4 *)(plane + at * 8) = v;
             };
-            if constexpr (ZERO_X && XN > 1) {
+            if constexpr (ZERO_LATE) {
                 const bool past = (int)(gw * TILE_COLS + at % (SLICE / 8) * 8) >= K;
-#pragma unroll
-                for (int h = 0; h < (F32 ? 2 : 1); h++) {
-                    u32x4 &v = xv[(F32 ? 2 : 1) * i + h];
-                    v = past ? u32x4{0u, 0u, 0u, 0u} : v;
-                }
+                xv[i] = past ? u32x4{0u, 0u, 0u, 0u} : xv[i];
             }
             if constexpr (F32) {
                 u32x4 hi, lo;
