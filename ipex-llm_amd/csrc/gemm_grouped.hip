@@ -178,18 +178,19 @@ int launch_grouped_gemm(const void *x, const void *const *w, const void *const *
 // Which tiles a dense gated MLP takes: narrow ones (64 columns of both weights), in halves of 64 rows and with two groups of
 // waves, while they are one per CU at most (eight K steps and more); with one group while they are two per CU and M more
 // than 128, and where the tall tiles of 256 x 128 would be little more than one per CU, so that most CUs wait for the
-// others' second.  400 points, eight shapes, M = 65 .. 2048, five formats: 1.4 times as fast as tall tiles alone on
-// average, 1.6 on the 290 where narrow ones are taken, 0.95 at worst.  Tall / narrow, sym_int4 fp16, us:
+// others' second - a last row tile of 64 rows at most is soon done and does not count ([12032 x 5120] at 522 rows in asym_int4
+// 137 / 161).  3086 random sizes, M = 65 .. 2048, five formats: 1.84 times as fast as tall tiles alone on average, 0.94 at
+// worst.  Tall / narrow, sym_int4 fp16, us:
 // [3584 x 1152] at M = 128 / 512 18.1 / 10.8 and 31.6 / 15.8, [8064 x 3840] at M = 128 / 384 43.5 / 25.1 and 77.7 / 54.3,
 // [11008 x 4096] at M = 128 / 256 / 768 49.3 / 33.1, 81.2 / 56.4 and 183 / 149; but at M = 512 / 2048 90 / 100 and 319 / 335.
 static GroupedPlan mlp_plan(int M, int N, int K) {
     const int rows = G_GM_TALL / 2, tiles_m = (M + rows - 1) / rows, cus = device_cus();
     const int64_t tiles = (int64_t)tiles_m * ((N + G_GN / 4 - 1) / (G_GN / 4));
     const int tall_n = (N + G_GN / 2 - 1) / (G_GN / 2);
-    const int64_t tall = (int64_t)((M + G_GM_TALL - 1) / G_GM_TALL) * tall_n;
+    const int64_t tall = (int64_t)((M + G_GM_TALL - 1) / G_GM_TALL) * tall_n, tall_long = (int64_t)((M + G_GM_TALL - 65) / G_GM_TALL) * tall_n;
     GroupedPlan plan = {true, 1, grouped_waves(M, 1, true), grouped_chunk(tall_n, grouped_one_round(M, 1, tall_n, true, 1))};
     if (tiles <= cus && K / TILE_COLS >= 8) plan.narrow = 2;
-    else if ((tiles <= 2 * cus && (M > rows || tiles <= cus)) || (tall > cus && tall * 20 <= (int64_t)cus * 27)) plan.narrow = 1;
+    else if ((tiles <= 2 * cus && (M > rows || tiles <= cus)) || (tall_long > cus && tall * 20 <= (int64_t)cus * 27)) plan.narrow = 1;
     plan.halves = plan.narrow && M > rows / 2 && 2 * tiles <= cus;
     return plan;
 }

@@ -42,6 +42,13 @@ def test_gated_mlp_tiles(qtype, m, n, k):
     assert torch.isnan(y[m]).all() and mlp_close(y[:m], x, blobs, qtype, n, k, act)
 
 
+@pytest.mark.parametrize("m,n,k", [(400, 16400, 256), (600, 11008, 128), (576, 11008, 256), (577, 11008, 256)])
+@pytest.mark.parametrize("qtype", ALL, ids=NAMES.values())
+def test_gated_mlp_tiles_around_a_second_round(qtype, m, n, k):
+    """Tall tiles little more than one per CU: narrow ones in their place, but not with a last row tile of 64 rows at most."""
+    test_gated_mlp_tiles(qtype, m, n, k)
+
+
 @pytest.mark.parametrize("rows,n,k", [((3, 0, 40, 129, 1), 144, 1152), ((130, 257, 64), 2064, 1024), ((5, 31, 33), 272, 640), ((200, 9), 16400, 256),
                                       ((300, 100, 20), 40960, 128)])
 @pytest.mark.parametrize("qtype", ALL, ids=NAMES.values())
