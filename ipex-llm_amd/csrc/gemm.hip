@@ -238,7 +238,8 @@ static bool narrow_two_groups(int M, int N, int K) { return narrow_workgroups(M,
 // 1.5 % above the faster of this form and the rest on average; 14 % at worst, [8192 x 8192] at M = 1300);
 // the entry points whose choices lowbit_forward_plan reports keep the figure from before, 1.24.
 // Two groups of waves (lowbit_linear's estimate only): 888 launches, 6.8 % rms; a pair of steps takes 1.49 us, a million
-// weights 0.12 us; scaled by 0.91.  Never above the estimate of one group, which two groups did not exceed at any of 2500
+// weights 0.12 us; scaled by 0.91, in the 8-bit formats by 0.955 (4900 points on weights that were not just read: chosen within
+// 1.3 % of the faster way on average as with 0.91, but 96 of them 5 % slower than the other way where it were 271).  Never above the estimate of one group, which two groups did not exceed at any of 2500
 // random points: the fit is too long for wide weights of few steps ([26304 x 2432] at 88 rows in sym_int4 26.1 us; where it
 // passed them over, 37.6).  Against the choice with one group the one made with this is 6.2 % faster on average over 2164
 // of them; 20 are slower by 3 to 11 % (a larger scale loses as much elsewhere).
@@ -254,7 +255,8 @@ double narrow_time_us(int M, int N, int K, int qtype, bool linear) {
     const double one = 0.5 + (double)(K / TILE_COLS) * step * format * rounds * (halves ? 0.87 : 1.0) * (0.84 + 0.16 * fill);
     if (!linear || !narrow_two_groups(M, N, K)) return one;
     const double format2 = qtype == QT_NF4 ? 1.12 : qtype == QT_SYM_INT8 ? 1.16 : qtype == QT_FP8_E4M3 ? 1.14 : 1.0;
-    const double two = 0.91 * (3.86 + 0.97 * over128 + 0.123e-6 * (double)N * (double)K +
+    const double two = (qtype == QT_SYM_INT8 || qtype == QT_FP8_E4M3 ? 0.955 : 0.91) *
+                       (3.86 + 0.97 * over128 + 0.123e-6 * (double)N * (double)K +
                                 (double)((K / TILE_COLS + 1) / 2) * 1.485 * format2 * (1.0 + 0.17 * over128) * (halves ? 0.79 : 1.0) * (0.69 + 0.31 * fill));
     return two < one ? two : one;
 }

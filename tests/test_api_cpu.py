@@ -496,3 +496,10 @@ def test_two_groups_of_waves_are_not_estimated_longer_than_one():
         for m, n, k in [(88, 26304, 2432), (360, 10416, 1152), (116, 15568, 1024), (43, 26352, 1280), (256, 2048, 2048), (586, 3216, 6016)]:
             assert time_us(m, n, k, qtype, True) <= time_us(m, n, k, qtype, False)
     assert ggml.lowbit_linear_workspace_bytes(2, ggml.LAYOUT_TILED, ggml.DT_F16, 256, 2048, 2048, 256 << 20) == 0
+
+
+def test_narrow_tiles_of_8_bits_are_not_estimated_too_short():
+    """sym_int8 and fp8_e4m3 at sizes where lowbit_linear took narrow tiles of two groups that were 15 to 20 % slower than the ring kernel
+    or a K split; both of those ask for a workspace, narrow tiles do not."""
+    for qtype, m, n, k in [(8, 166, 5216, 4352), (8, 1087, 1600, 7424), (8, 89, 6944, 3328), (15, 365, 3376, 4352)]:
+        assert ggml.lowbit_linear_workspace_bytes(qtype, ggml.LAYOUT_TILED, ggml.DT_F16, m, n, k, 256 << 20) > 0
