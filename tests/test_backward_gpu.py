@@ -40,6 +40,16 @@ def test_kernel(qtype, m, n, k, dtype):
     assert m == 1 or close(out[1:m], grad[1:], w, dtype)
 
 
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16], ids=["f16", "bf16"])
+@pytest.mark.parametrize("m,n,k", [(1030, 1200, 2048), (2100, 1616, 1024), (1024, 1664, 2176)])
+@pytest.mark.parametrize("qtype", ALL, ids=NAMES.values())
+def test_kernel_of_128_rows_over_many_steps(qtype, m, n, k, dtype):
+    """Row tiles of 128 (more than 256 of 64), each group of waves past its loop's period of six: 19 and 26 steps, a last one of 48
+    and of 16 weight rows and whole ones."""
+    assert (m + 63) // 64 * (k // 128) > 256
+    test_kernel(qtype, m, n, k, dtype)
+
+
 def layer_of(qtype, n, k, bias=None):
     with torch.device("meta"):
         layer = LowBitLinear(k, n, qtype, bias=bias is not None)
@@ -123,3 +133,34 @@ def test_a_gradient_that_is_left_out_counts_as_zeros(m, n, k):
     for product in (layer, lambda t: MatMulLowBit.apply(t.view(m, k), layer.weight, n)):
         (gx,) = torch.autograd.grad(LeavesOut.apply(product(x)).sum(), x)
         assert gx.shape == x.shape and gx.dtype == x.dtype and not gx.any()
+
+
+class Operators(torch.utils._python_dispatch.TorchDispatchMode):
+    def __init__(self):
+        super().__init__()
+        self.seen = []
+
+    def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+        self.seen.append(func._schema.name)
+        return func(*args, **(kwargs or {}))
+
+
+def test_transforms_and_modes_get_what_the_autograd_function_gives():
+    """A transform that MatMulLowBit refuses is refused, a dispatch mode sees the operators of the backward, and a trace holds the
+    layer: at a size where a plain gradient comes from the packed weight."""
+    m, n, k = 100, 1024, 2560
+    assert ggml.lowbit_backward_applies(2, TILED, DT[torch.float16], m, n, k)
+    layer = layer_of(2, n, k)
+    w = dev_dequantize(layer.weight.data.view(torch.uint8), 2, n, k, TILED, torch.float16)
+    x = torch.randn((m, k), device="cuda").half().requires_grad_(True)
+    grad = torch.randn((m, n), device="cuda").half()
+    for product in (layer, lambda t: MatMulLowBit.apply(t, layer.weight, n)):
+        with pytest.raises(RuntimeError):
+            torch.func.grad(lambda t: product(t).sum())(x)
+        with pytest.raises(RuntimeError):
+            torch.func.vmap(product)(x.view(4, m // 4, k))
+        with Operators() as mode:
+            (gx,) = torch.autograd.grad(product(x), x, grad)
+        assert "aten::mm" in mode.seen and close(gx, grad, w, torch.float16)
+    traced = torch.jit.trace(layer, x, check_trace=False)
+    assert torch.equal(traced(x), layer(x))

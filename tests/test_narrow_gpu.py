@@ -74,3 +74,45 @@ def test_grouped_tiles(qtype, rows, n, k):
         want, bound = products(x[a:b], blobs[0][e], qtype, n, k)
         assert ((y[a:b].double() - want).abs() <= want.abs() * torch.finfo(dtype).eps / 2 + bound + torch.finfo(dtype).smallest_normal).all()
         assert mlp_close(h[a:b], x[a:b], (blobs[0][e], blobs[1][e]), qtype, n, k, 0)
+
+
+def random_blob(qtype, n, k, seed):
+    w = torch.randn((n, k), generator=torch.Generator("cuda").manual_seed(seed), device="cuda") * 0.02
+    blob = torch.empty(ggml.lowbit_blob_bytes(qtype, n * k), dtype=torch.uint8, device="cuda")
+    ggml.lowbit_quantize(w.data_ptr(), blob.data_ptr(), qtype, n, k, TILED, stream())
+    return blob
+
+
+# 1 .. 8 row blocks of 32 per tall tile, eight waves (up to 192 rows per group) and four
+@pytest.mark.parametrize("rows", [(5, 33, 70, 100, 130, 170, 200, 256), (300, 700, 250, 513)], ids=["eight waves", "four waves"])
+@pytest.mark.parametrize("k", [384, 512, 640, 768, 896])
+@pytest.mark.parametrize("qtype", ALL, ids=NAMES.values())
+def test_tall_tiles_over_several_steps(qtype, k, rows):
+    """The tall forms, fused and plain, where narrow tiles would be more than two per CU: three to seven K steps, so that the
+    pipeline of two steps ahead runs its loop of three and ends with one, two and three steps after it."""
+    dtype = torch.bfloat16 if k % 256 else torch.float16
+    offsets = torch.tensor([0, *rows]).cumsum(0).int().cuda()
+    total, groups = sum(rows), len(rows)
+    x = torch.randn((total, k), generator=torch.Generator().manual_seed(k)).to(dtype).cuda()
+    for fused, n in ((True, 5136), (False, 10256)):
+        blobs = [random_blob(qtype, n, k, 7 * k + i) for i in range(3)]
+        of = lambda e, up: blobs[(e + up) % 3]
+        tables = [torch.tensor([of(e, up).data_ptr() for e in range(groups)], device="cuda") for up in range(2)]
+        # more narrow tiles than two per CU of 256, were every group's rows to fill theirs; the plain product says what it takes
+        assert sum((r + 127) // 128 for r in rows) * ((n + 63) // 64 if fused else (n + 127) // 128) > 512
+        y = torch.full((total + 1, n), float("nan"), dtype=dtype, device="cuda")
+        if fused:
+            ggml.lowbit_grouped_mlp_forward(x.data_ptr(), tables[0].data_ptr(), tables[1].data_ptr(), y.data_ptr(), offsets.data_ptr(), groups,
+                                            total, qtype, DT[dtype], n, k, 0, stream())
+        else:
+            tall, splits = ggml.lowbit_grouped_forward_plan(groups, total, n, k, False)[:2]
+            assert (tall, splits) == (1, 1)
+            ggml.lowbit_grouped_forward(x.data_ptr(), tables[0].data_ptr(), y.data_ptr(), offsets.data_ptr(), groups, total, qtype, DT[dtype],
+                                        n, k, stream())
+        assert torch.isnan(y[total]).all()
+        for e, (a, b) in enumerate(zip(offsets.tolist(), offsets.tolist()[1:])):
+            if fused:
+                assert mlp_close(y[a:b], x[a:b], (of(e, 0), of(e, 1)), qtype, n, k, 0)
+            else:
+                want, bound = products(x[a:b], of(e, 0), qtype, n, k)
+                assert ((y[a:b].double() - want).abs() <= want.abs() * torch.finfo(dtype).eps / 2 + bound + torch.finfo(dtype).smallest_normal).all()
