@@ -1,12 +1,9 @@
 // Where the one-pass kernel for up to 64 rows of x (lowbit_gemv_wide.h) is used, and in which shape.
 #include <hip/hip_runtime.h>
-#include "lowbit_formats.h"
+#include "lowbit_wide_plan.h"
 
 namespace lowbit {
 
-struct WideShape {
-    int r, waves;
-};
 template <int QT>
 int launch_wide_q(const void *x, const void *w, const void *bias, void *y, int layout, int dt, int M, int N, int K, const WideShape &s,
                   hipStream_t st);
@@ -64,12 +61,9 @@ static WideShape wide_mlp_shape(int qtype, int act_dtype, int M, int N, int K) {
     if (M <= 8 && !(M > 4 && (qtype == QT_SYM_INT8 || (qtype == QT_NF4 && T >= 512)))) return none;
     if (M > 64 || (MB > 2 && T > 1024)) return none;
     // One tile row of either weight where that takes an odd number of rounds, with 16 rows and the formats of many registers,
-    // and with 49 .. 64 rows where two spill (all but nf4 and fp16 sym_int4; 56 rows on [8192 x 4096], one / two: sym_int8
-    // 27.5 / 57.7 us, asym_int4 27.6 / 43.3, fp8_e4m3 26.7 / 30.6; nf4 27.7 / 25.2).  8 waves where a CU has one workgroup,
-    // else 4.
+    // and with 49 .. 64 rows where two spill.  8 waves where a CU has one workgroup, else 4.
     const bool small = qtype == QT_SYM_INT4 || qtype == QT_NF4;
-    const bool spills = MB == 4 && qtype != QT_NF4 && !(qtype == QT_SYM_INT4 && act_dtype == DT_F16);
-    const int r = rounds == 1 || rounds == 3 || (MB == 1 && !small) || spills ? 1 : 2;
+    const int r = rounds == 1 || rounds == 3 || (MB == 1 && !small) || !wide_mlp_two_rows(qtype, act_dtype == DT_F16, MB) ? 1 : 2;
     return {r, (T + r - 1) / r <= 256 ? 8 : 4};
 }
 

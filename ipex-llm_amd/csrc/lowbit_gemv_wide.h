@@ -20,6 +20,7 @@
 #pragma once
 #include "lowbit_rows.h"
 #include "lowbit_unpack.h"
+#include "lowbit_wide_plan.h"
 
 #include <type_traits>
 
@@ -309,10 +310,6 @@ __global__ __launch_bounds__(64 * wide_max_waves(MB, DUAL ? 2 * R : R, F32)) voi
     }
 }
 
-struct WideShape {
-    int r, waves;
-};
-
 // Workgroups of four waves that the GPU holds at once, in either form
 struct WideRoom {
     int peel, crowd;
@@ -392,7 +389,8 @@ template <int QT, typename AT, int MB>
 static int launch_wide_mlp_mb(const void *x, const void *wg, const void *wu, void *y, int M, int N, int K, int act, const WideShape &s,
                               hipStream_t st) {
     if (s.r == 1) return launch_wide_r<QT, AT, MB, 1, false, false, true>(x, wg, wu, nullptr, y, M, N, K, act, s.waves, st);
-    if (s.r == 2) return launch_wide_r<QT, AT, MB, 2, false, false, true>(x, wg, wu, nullptr, y, M, N, K, act, s.waves, st);
+    if constexpr (wide_mlp_two_rows(QT, __is_same(AT, _Float16), MB))
+        if (s.r == 2) return launch_wide_r<QT, AT, MB, 2, false, false, true>(x, wg, wu, nullptr, y, M, N, K, act, s.waves, st);
     return -7;
 }
 
