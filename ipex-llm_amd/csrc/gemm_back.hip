@@ -12,12 +12,12 @@
 // steps, the second on the rest, each with its own LDS buffers (two of each operand); their sums meet in LDS at the end.
 // Within a group a wave owns all the rows by 32 columns.  What a step needs is loaded three steps ahead, into three sets of
 // registers, and goes to LDS during the step before it.  (g by LDS-DMA instead, which the compiler does not count among
-// the loads in flight, made it wait for the youngest ones: 43 us in place of 38 for 128 rows on [4096 x 4096].)
+// the loads in flight, made it wait for the youngest ones and an earlier version a seventh slower.)
 //
-// What bounds it, 128 rows on [4096 x 4096] in sym_int4 (39 us, 1.05 us a pair of steps): LDS is busy 54 % of the time, the
-// MFMA pipes 38 %, the vector units 30 %; two waves per SIMD that meet at a barrier per step overlap them badly.  Taking the
-// MFMAs out saves 2 us, the dequantization with its writes to LDS 12, g's way into LDS 10.  64 rows by 64 columns per wave,
-// whose operands are a fifth less LDS traffic, and the writes ahead of the MFMAs are level with this.
+// What bounds it, 128 rows on [4096 x 4096] in sym_int4 (33.7 us in a kernel trace, 1.05 us a pair of steps): LDS is busy 54 % of
+// the time, the MFMA pipes 38 %, the vector units 30 %; two waves per SIMD that meet at a barrier per step overlap them badly.
+// Of an earlier version's 39 us the MFMAs were 2, the dequantization with its writes to LDS 12, g's way into LDS 10.  64 rows
+// by 64 columns per wave, whose operands are a fifth less LDS traffic, and the writes ahead of the MFMAs are level with this.
 #include "lowbit_gemm.h"
 
 namespace lowbit {
@@ -275,11 +275,13 @@ static int launch_back_q(const void *g, const void *w, void *gx, int dt, int M, 
     return -4;
 }
 
-// Whether this kernel is the faster way, against dequantizing W and torch's dense product (260 random points, M = 64 .. 2048,
-// N = 1024 .. 14336, K = 1024 .. 8192, five formats): while its tiles are one per CU at most - the 152 points that are taken
-// are 1.32 times faster on average, 0.92 at worst; with a second round of tiles it is 0.6 - 1.2 times as fast - and as long
-// as the walk along N is no longer than twice K, or than four times K with a third of the CUs at work ([9504 x 1280] at 178
-// rows in nf4 104 us against 52; [4096 x 4096] at 128 / 1024 rows in sym_int4 30 against 46 and 49 against 58).
+// Whether this kernel is the faster way, against dequantizing W and torch's dense product: while its tiles are one per CU at
+// most - with a second round it is 0.6 - 1.2 times as fast - and as long as the walk along N is no longer than twice K, or than
+// four times K with a third of the CUs at work ([9504 x 1280] at 178 rows in nf4 104 us against 52; [4096 x 4096] at 128 / 1024
+// rows in sym_int4 28 against 45 and 45 against 56).  4900 random sizes that are taken, M = 32 .. 4096, N = 512 .. 16000,
+// K = 512 .. 12000, five formats, time on the GPU alone: 1.64 times as fast on average; 31 are more than 5 % slower, 0.79 at
+// worst ([3200 x 1920] at 85 rows in nf4 28.7 us against 22.6: the dense product's time jumps between neighbouring sizes).
+// Narrower limits lose more than they save.
 bool gemm_back_applies(int qtype, int M, int N, int K) {
     const bool tall = back_tiles(M, K, 64) > 256;
     const int64_t tiles = back_tiles(M, K, tall ? 128 : 64);

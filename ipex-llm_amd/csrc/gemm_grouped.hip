@@ -98,8 +98,9 @@ struct NarrowPlan {
 // round.  A row tile more than the estimate is reckoned with where groups may be uneven.  Whole rows whatever the XCDs' shares,
 // as before / now, us: 18 of [720 x 3712] in sym_int8 with 202 tokens, fused, 43.7 / 24.2, 10 of [1088 x 10752] in fp8_e4m3 with
 // 178 110 / 69, 18 of [1600 x 1664] in sym_int4 with 179, plain, 21.0 / 13.8, 10 of [6032 x 9856] with 300 203 / 104.
-// Random sizes against the forms that narrow tiles replaced: 1.17 times as fast over 3800 fused launches and 1.22 over 6000
-// plain ones, 2 and 1 % of them slower by more than 4 % (at worst 0.79 and 0.75: tiles that all but fill the CUs).
+// Random sizes against the forms that narrow tiles replaced: 1.18 times as fast over 2650 fused launches and 1.22 over 4030 plain
+// ones; 2 and 1 % of them are slower by more than 4 %, 0.80 and 0.68 at worst: uneven groups whose tiles are more than the
+// estimate and than the CUs hold, which are 1.3 times as fast on average all the same.
 static NarrowPlan grouped_narrow(int total_rows, int n_groups, int tiles_n, int K) {
     const int rows = G_GM_TALL / 2, cus = device_cus();
     const int uneven = total_rows / rows + (n_groups + 1) / 2, even = (total_rows / n_groups + rows - 1) / rows * n_groups;
@@ -191,6 +192,7 @@ static GroupedPlan mlp_plan(int M, int N, int K) {
     GroupedPlan plan = {true, 1, grouped_waves(M, 1, true), grouped_chunk(tall_n, grouped_one_round(M, 1, tall_n, true, 1))};
     if (tiles <= cus && K / TILE_COLS >= 8) plan.narrow = 2;
     else if ((tiles <= 2 * cus && (M > rows || tiles <= cus)) || (tall_long > cus && tall * 20 <= (int64_t)cus * 27)) plan.narrow = 1;
+    if (plan.narrow) plan.waves = 4 * plan.narrow;
     plan.halves = plan.narrow && M > rows / 2 && 2 * tiles <= cus;
     return plan;
 }

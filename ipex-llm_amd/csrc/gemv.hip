@@ -73,7 +73,7 @@ __device__ inline float load_route_w(const void *w, int dtype, int pair) {
 // kernel.  A row of a tile is 72 .. 136 contiguous bytes instead of a 1 KiB tile; a workgroup's waves take
 // neighbouring columns, so lines are shared within the workgroup only.  (One wave per weight row and a scalar decode
 // per weight, four rows of x a pass, took 74 us per pass for [32003 x 4096] in asym_int4: two at eight rows, which now take
-// 27.1 us in bf16, 25.8 in fp16.)
+// 29.8 us in bf16, 29.0 in fp16.)
 template <int QT, typename AT, int MT, int U, int XN, bool DUAL, int MOE, int R, bool F32, bool ROWS>
 __global__ __launch_bounds__(1024) void gemv_mfma_kernel(const AT *__restrict__ x, const uint8_t *__restrict__ w,
                                                          const uint8_t *__restrict__ w2, AT *__restrict__ y,

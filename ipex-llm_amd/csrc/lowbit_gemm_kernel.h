@@ -193,12 +193,12 @@ __device__ inline float gemm_gate_act(float g, int act) {
 
 // GROUPED: the launch covers the row tiles of all groups (see GroupArgs); the tall form then takes one row
 // tile for up to 256 rows of a group and runs only the 32-row blocks that hold rows.
-// DUAL (grouped tall form only): the fused gate/up projection of a gated MLP.  The wave's two 32-row weight
+// DUAL (tall and narrow forms): the fused gate/up projection of a gated MLP.  The wave's two 32-row weight
 // blocks are the same 32 rows of the gate and of the up weight (a workgroup covers 128 columns of both), and
-// the epilogue stores act(gate) * up.  With eight waves a wave has one 32-row block: its first tile (16 rows) is
-// the gate's, its second the same 16 rows of the up weight, so that both products of an output element still
+// the epilogue stores act(gate) * up.  With eight waves or a narrow tile a wave has one 32-row block: its first tile (16
+// rows) is the gate's, its second the same 16 rows of the up weight, so that both products of an output element still
 // end in the same lane (accumulator i and i + 8).
-// NARROW (dense 128-row DMA form only): 128 weight rows per workgroup instead of 256, one 32-row block per wave -
+// NARROW (128-row DMA form, dense or grouped): 128 weight rows per workgroup instead of 256, one 32-row block per wave -
 // twice the workgroups for a product whose 256-column tiles leave compute units idle, without the partial sums
 // of a K split.
 // KS == 2 (narrow form only): two groups of WAVES waves on the same tile, each with its own x buffers and accumulators, the
