@@ -249,6 +249,12 @@ size_t lowbit_linear_workspace_bytes(int qtype, int layout, int dtype, int64_t M
 int lowbit_backward(const void *grad, const void *w, void *grad_x, int qtype, int act_dtype, int64_t M, int64_t N, int64_t K,
                     void *stream);
 int lowbit_backward_applies(int qtype, int layout, int act_dtype, int64_t M, int64_t N, int64_t K);
+/* The same with a workspace (16-byte aligned device memory, contents undefined before and after): where the result has too
+ * few tiles for the GPU, several workgroups share a tile's walk along N and their fp32 sums meet in the workspace.  With
+ * less than lowbit_backward_workspace_bytes (or null) the walk is shared less, or not at all. */
+int lowbit_backward_ws(const void *grad, const void *w, void *grad_x, int qtype, int act_dtype, int64_t M, int64_t N, int64_t K,
+                       void *workspace, size_t workspace_bytes, void *stream);
+size_t lowbit_backward_workspace_bytes(int qtype, int64_t M, int64_t N, int64_t K);
 
 /* lowbit_forward_ws without a workspace argument and without any allocation: the partial tiles go to a
  * scratch array that is part of the library's image on every GPU (lowbit_noalloc_scratch_bytes() = 64 MiB,

@@ -44,7 +44,9 @@ size_t gemm_rows_workspace_bytes(int M, int N, int K, size_t max_bytes);
 int launch_gemm_rows(const void *x, const void *w, const void *bias, void *y, int qtype, int act_dtype, int M, int N, int K,
                      void *workspace, size_t workspace_bytes, hipStream_t st);
 bool gemm_back_applies(int qtype, int M, int N, int K);
-int launch_gemm_back(const void *g, const void *w, void *gx, int qtype, int act_dtype, int M, int N, int K, hipStream_t st);
+size_t back_workspace_bytes(int qtype, int M, int N, int K);
+int launch_gemm_back(const void *g, const void *w, void *gx, int qtype, int act_dtype, int M, int N, int K, void *ws, size_t ws_bytes,
+                     hipStream_t st);
 double narrow_time_us(int M, int N, int K, int qtype, bool linear);
 int gemm_splits(int M, int N, int K, size_t ws_bytes, int qtype);
 double gemm_time_us(int M, int N, int K, int splits, int qtype);
@@ -514,8 +516,18 @@ int lowbit_backward_applies(int qtype, int layout, int act_dtype, int64_t M, int
     return gemm_back_applies(qtype, (int)M, (int)N, (int)K);
 }
 
+size_t lowbit_backward_workspace_bytes(int qtype, int64_t M, int64_t N, int64_t K) {
+    if (!lowbit_tileable(qtype, N, K) || M <= 0 || M > 0x7fffffff || N > 0x7fffffff || K > 0x7fffffff) return 0;
+    return back_workspace_bytes(qtype, (int)M, (int)N, (int)K);
+}
+
 int lowbit_backward(const void *grad, const void *w, void *grad_x, int qtype, int act_dtype, int64_t M, int64_t N, int64_t K,
                     void *stream) {
+    return lowbit_backward_ws(grad, w, grad_x, qtype, act_dtype, M, N, K, nullptr, 0, stream);
+}
+
+int lowbit_backward_ws(const void *grad, const void *w, void *grad_x, int qtype, int act_dtype, int64_t M, int64_t N, int64_t K,
+                       void *workspace, size_t workspace_bytes, void *stream) {
     const char *what = "lowbit_backward";
     if (int rc = check_weight_shape(what, qtype, N, K, LOWBIT_LAYOUT_TILED)) return rc;
     if (M < 0 || M > 0x7fffffff) return fail(LOWBIT_EARG, "%s: bad M", what);
@@ -525,7 +537,9 @@ int lowbit_backward(const void *grad, const void *w, void *grad_x, int qtype, in
     if (N == 0) return fail(LOWBIT_ESHAPE, "%s: N == 0", what);
     if (!grad || !w || !grad_x || !aligned16(grad) || !aligned16(w) || !aligned16(grad_x))
         return fail(LOWBIT_EARG, "%s: null or misaligned pointer (16 bytes)", what);
-    return check_launch(launch_gemm_back(grad, w, grad_x, qtype, act_dtype, (int)M, (int)N, (int)K, (hipStream_t)stream), what);
+    if (workspace && !aligned16(workspace)) return fail(LOWBIT_EARG, "%s: misaligned workspace (16 bytes)", what);
+    return check_launch(launch_gemm_back(grad, w, grad_x, qtype, act_dtype, (int)M, (int)N, (int)K, workspace, workspace_bytes,
+                                         (hipStream_t)stream), what);
 }
 
 int lowbit_mlp_forward(const void *x, const void *w_gate, const void *w_up, void *y, int qtype, int act_dtype,

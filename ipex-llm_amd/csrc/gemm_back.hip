@@ -18,6 +18,7 @@
 // the time, the MFMA pipes 38 %, the vector units 30 %; two waves per SIMD that meet at a barrier per step overlap them badly.
 // Of an earlier version's 39 us the MFMAs were 2, the dequantization with its writes to LDS 12, g's way into LDS 10.  64 rows
 // by 64 columns per wave, whose operands are a fifth less LDS traffic, and the writes ahead of the MFMAs are level with this.
+// Few tiles leave CUs idle: then several workgroups share a tile's walk (back_plan).
 #include "lowbit_gemm.h"
 
 namespace lowbit {
@@ -30,9 +31,12 @@ __device__ inline f32x16 mfma32(bf16x8 a, bf16x8 b, f32x16 c) { return __builtin
 constexpr int BACK_N = 64;                                   // weight rows per step
 constexpr int BACK_WBYTES = BACK_N * TILE_COLS * 2;          // of scaled weights in LDS per step
 
+// ws != null: workgroup (tile, s) walks the steps s * split_steps .. of N only and leaves its fp32 sums there for
+// back_reduce_kernel.
 template <int QT, typename AT, int MBW>
 __global__ __launch_bounds__(512, 2) void gemm_back_kernel(const AT *__restrict__ g, const uint8_t *__restrict__ w,
-                                                           AT *__restrict__ gx, int M, int N, int K) {
+                                                           AT *__restrict__ gx, int M, int N, int K, f32x4 *__restrict__ ws,
+                                                           int split_steps) {
     using F = Fmt<QT>;
     using V8 = typename Vec8<AT>::type;
     constexpr int BM = 64 * MBW, GBYTES = BM * BACK_N * 2, GROUP = 2 * (GBYTES + BACK_WBYTES);
@@ -48,13 +52,14 @@ __global__ __launch_bounds__(512, 2) void gemm_back_kernel(const AT *__restrict_
     if ((int)(blockIdx.x >> 3) >= count) return;             // whole workgroup leaves
     const int tile = first + (blockIdx.x >> 3), m0 = tile % tiles_m * BM, kt = tile / tiles_m;
 
-    const int steps = (N + BACK_N - 1) / BACK_N, steps_first = (steps + 1) / 2;
-    const int s0 = half ? steps_first : 0, S = half ? steps - steps_first : steps_first, last = S > 0 ? S - 1 : 0;
+    const int all_steps = (N + BACK_N - 1) / BACK_N, split_s0 = ws ? blockIdx.y * split_steps : 0;
+    const int steps = ws && split_steps < all_steps - split_s0 ? split_steps : all_steps - split_s0, steps_first = (steps + 1) / 2;
+    const int s0 = split_s0 + (half ? steps_first : 0), S = half ? steps - steps_first : steps_first, last = S > 0 ? S - 1 : 0;
     const int row_tiles = N / TILE_ROWS;
     // which step of the whole walk; past this group's last one: a re-read that nobody uses (a group may have no step at all)
     auto step_at = [&](int s) __attribute__((always_inline)) {
         s = s0 + (s < last ? s : last);
-        return s < steps ? s : steps - 1;
+        return s < split_s0 + steps ? s : split_s0 + steps - 1;
     };
 
     // ---- the weights: this wave's tile of a step
@@ -232,6 +237,16 @@ __global__ __launch_bounds__(512, 2) void gemm_back_kernel(const AT *__restrict_
     };
     // C layout: lane = 32 * kg + row of g, register i = column 8 * (i / 4) + 4 * kg + i % 4
     auto finish = [&](int from) __attribute__((always_inline)) {
+        if (ws) {
+            f32x4 *const to = ws + (((int64_t)blockIdx.y * T + tile) * 8 + wave_wg) * (MBW * 256) + lane;
+#pragma unroll
+            for (int mb = from; mb < from + MBW; mb++)
+#pragma unroll
+                for (int q = 0; q < 4; q++)
+                    to[((mb - from) * 4 + q) * 64] = part[(mb * 4 + q) * 64] +
+                        f32x4{acc[mb][q * 4], acc[mb][q * 4 + 1], acc[mb][q * 4 + 2], acc[mb][q * 4 + 3]};
+            return;
+        }
 #pragma unroll
         for (int mb = from; mb < from + MBW; mb++) {
             const int m = m0 + mb * 32 + i32;
@@ -254,51 +269,127 @@ __global__ __launch_bounds__(512, 2) void gemm_back_kernel(const AT *__restrict_
     else finish(0);
 }
 
-// Tiles of gx with 64 or 128 rows each: 64 while those are no more than one per CU.
+// Adds the partial sums of the splits (as gemm_back_kernel leaves them: split, tile, wave, row block, register group, lane) in
+// order and rounds once.  One thread per group of four columns.
+template <typename AT, int MBW>
+__global__ __launch_bounds__(256) void back_reduce_kernel(const f32x4 *__restrict__ ws, AT *__restrict__ gx, int M, int K, int64_t per_split,
+                                                          int splits) {
+    const int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x;           // (a split's sums are whole blocks of threads)
+    const int lane = (int)(t & 63), q = (int)(t >> 6) & 3, mb = (int)(t >> 8) % MBW;
+    const int64_t tw = (t >> 8) / MBW;
+    const int wave_wg = (int)(tw & 7), tiles_m = (M + 64 * MBW - 1) / (64 * MBW);
+    const int m = (int)((tw >> 3) % tiles_m) * (64 * MBW) + ((wave_wg >> 2) * MBW + mb) * 32 + (lane & 31);
+    const int k = (int)((tw >> 3) / tiles_m) * TILE_COLS + (wave_wg & 3) * 32 + 8 * q + 4 * (lane >> 5);
+    f32x4 a = ws[t];
+    for (int s = 1; s < splits; s++) a += ws[s * per_split + t];
+    typedef AT at4 __attribute__((ext_vector_type(4)));
+    at4 o;
+#pragma unroll
+    for (int i = 0; i < 4; i++) o[i] = to_at<AT>(a[i]);
+    if (m < M) *(at4 *)(gx + (int64_t)m * K + k) = o;
+}
+
+// Tiles of gx with 64 or 128 rows each.
 static int64_t back_tiles(int M, int K, int rows) { return (int64_t)((M + rows - 1) / rows) * (K / TILE_COLS); }
 
-template <int QT, typename AT>
-static int launch_back_t(const void *g, const void *w, void *gx, int M, int N, int K, hipStream_t st) {
-    const bool tall = back_tiles(M, K, 64) > 256;
-    const int64_t tiles = back_tiles(M, K, tall ? 128 : 64);
+// How the tiles are cut: what takes the shortest by the estimate below, while the workgroups are one per CU at most (a workgroup's
+// LDS fills a CU).  Where the result has fewer tiles than the GPU CUs, several workgroups share a tile's walk along N.
+// Estimated microseconds, fitted to 258 random sizes (M = 24 .. 2048, N = 1024 .. 14336, K = 1024 .. 8192, five formats, both
+// types) with up to 16 splits each: 6 % rms, the plan it picks within 2 % of the best on average.  A pair of steps takes 0.78
+// (64 rows) or 1.03 (128), a launch 4.7 or 6.2, a second one that adds the splits 1.0 and 0.021 per 64 rows by 128 columns of fp32
+// sums.  Splits are charged 12 instead of that 1.0: their workspace and launch cost the host 6, and where the GPU waits for the host
+// anyway a step with them is the longer one (498 rows on [2000 x 1280] 42 -> 49, its kernel 18 -> 13).  Whole training steps against the choice without splits, us: 307 rows on [3360 x 1408] in nf4 65 -> 51, 234 on
+// [7616 x 2432] 77 -> 50, 329 on [11456 x 4224] 168 -> 128, 125 on [9104 x 6272] in sym_int8 104 -> 89; the kernels alone 1.34 times
+// as fast over those 258 sizes, 0.90 at worst.
+struct BackPlan {
+    int rows, splits;             // rows of g per tile; workgroups that share a tile's walk along N
+};
+static double back_time_us(int qtype, int64_t tiles, int rows, int N, int splits) {
+    const int steps = (N + BACK_N - 1) / BACK_N, per = (steps + splits - 1) / splits;
+    const double format = qtype == QT_NF4 ? 1.2 : qtype == QT_SYM_INT4 || qtype == QT_ASYM_INT4 ? 1.06 : 0.99;
+    const double t = (rows == 64 ? 4.7 : 6.2) + (rows == 64 ? 0.78 : 1.03) * format * ((per + 1) / 2);
+    return splits > 1 ? t + 12.0 + 0.021 * (double)splits * (double)tiles * rows / 64 : t;
+}
+static size_t back_split_bytes(int M, int K, int rows) { return (size_t)back_tiles(M, K, rows) * rows * TILE_COLS * sizeof(float); }
+
+static BackPlan back_plan(int qtype, int M, int N, int K, size_t ws_bytes) {
+    const int steps = (N + BACK_N - 1) / BACK_N;
+    BackPlan best = {128, 1};
+    double best_us = 1e30;
+    auto consider = [&](int rows, int s) {
+        const double us = back_time_us(qtype, back_tiles(M, K, rows), rows, N, s);
+        if (us < best_us) {
+            best = {rows, s};
+            best_us = us;
+        }
+    };
+    for (int rows = 64; rows <= 128; rows += 64)
+        if (back_tiles(M, K, rows) <= 256) consider(rows, 1);
+    if (best_us < 18.0) return best;                         // (no split is estimated shorter)
+    for (int rows = 64; rows <= 128; rows += 64)
+        for (int s = 2; s <= 16 && back_tiles(M, K, rows) * s <= 256 && 2 * s <= steps && s * back_split_bytes(M, K, rows) <= ws_bytes; s++)
+            if ((steps + s - 1) / s < (steps + s - 2) / (s - 1)) consider(rows, s);        // (fewer steps than with one split less)
+    return best;
+}
+
+size_t back_workspace_bytes(int qtype, int M, int N, int K) {
+    const BackPlan p = back_plan(qtype, M, N, K, (size_t)-1);
+    return p.splits > 1 ? (size_t)p.splits * back_split_bytes(M, K, p.rows) : 0;
+}
+
+template <int QT, typename AT, int MBW>
+static int launch_back_m(const void *g, const void *w, void *gx, int M, int N, int K, int splits, void *ws, hipStream_t st) {
+    const int64_t tiles = back_tiles(M, K, 64 * MBW);
     if (tiles > (1 << 28)) return -3;
-    const dim3 grid(8 * (unsigned)((tiles + 7) / 8));
-    if (tall) hipLaunchKernelGGL((gemm_back_kernel<QT, AT, 2>), grid, dim3(512), 0, st, (const AT *)g, (const uint8_t *)w, (AT *)gx, M, N, K);
-    else hipLaunchKernelGGL((gemm_back_kernel<QT, AT, 1>), grid, dim3(512), 0, st, (const AT *)g, (const uint8_t *)w, (AT *)gx, M, N, K);
+    const int steps = (N + BACK_N - 1) / BACK_N, per = (steps + splits - 1) / splits, ny = (steps + per - 1) / per;
+    if (ny == 1) ws = nullptr;
+    hipLaunchKernelGGL((gemm_back_kernel<QT, AT, MBW>), dim3(8 * (unsigned)((tiles + 7) / 8), ny), dim3(512), 0, st, (const AT *)g,
+                       (const uint8_t *)w, (AT *)gx, M, N, K, (f32x4 *)ws, per);
+    if (ws) {
+        const int64_t per_split = tiles * 8 * MBW * 256;                 // groups of four sums
+        hipLaunchKernelGGL((back_reduce_kernel<AT, MBW>), dim3((unsigned)(per_split / 256)), dim3(256), 0, st, (const f32x4 *)ws, (AT *)gx,
+                           M, K, per_split, ny);
+    }
     return 0;
 }
 
+template <int QT, typename AT>
+static int launch_back_t(const void *g, const void *w, void *gx, int M, int N, int K, void *ws, size_t ws_bytes, hipStream_t st) {
+    const BackPlan p = back_plan(QT, M, N, K, ws ? ws_bytes : 0);
+    if (p.rows == 128) return launch_back_m<QT, AT, 2>(g, w, gx, M, N, K, p.splits, ws, st);
+    return launch_back_m<QT, AT, 1>(g, w, gx, M, N, K, p.splits, ws, st);
+}
+
 template <int QT>
-static int launch_back_q(const void *g, const void *w, void *gx, int dt, int M, int N, int K, hipStream_t st) {
-    if (dt == DT_F16) return launch_back_t<QT, _Float16>(g, w, gx, M, N, K, st);
-    if (dt == DT_BF16) return launch_back_t<QT, __bf16>(g, w, gx, M, N, K, st);
+static int launch_back_q(const void *g, const void *w, void *gx, int dt, int M, int N, int K, void *ws, size_t ws_bytes, hipStream_t st) {
+    if (dt == DT_F16) return launch_back_t<QT, _Float16>(g, w, gx, M, N, K, ws, ws_bytes, st);
+    if (dt == DT_BF16) return launch_back_t<QT, __bf16>(g, w, gx, M, N, K, ws, ws_bytes, st);
     return -4;
 }
 
-// Whether this kernel is the faster way, against dequantizing W and torch's dense product: while its tiles are one per CU at
-// most - with a second round it is 0.6 - 1.2 times as fast - and as long as the walk along N is no longer than twice K, or than
-// four times K with a third of the CUs at work ([9504 x 1280] at 178 rows in nf4 104 us against 52; [4096 x 4096] at 128 / 1024
-// rows in sym_int4 28 against 45 and 45 against 56).  4900 random sizes that are taken, M = 32 .. 4096, N = 512 .. 16000,
-// K = 512 .. 12000, five formats, time on the GPU alone: 1.64 times as fast on average; 31 are more than 5 % slower, 0.79 at
-// worst ([3200 x 1920] at 85 rows in nf4 28.7 us against 22.6: the dense product's time jumps between neighbouring sizes).
-// Narrower limits lose more than they save.
+// Whether this kernel is the faster way, against dequantizing W and torch's dense product: while its tiles of 128 rows are one per
+// CU at most (with a second round it is 0.6 - 1.3 times as fast), and there are 20 workgroups or more: one of the 258
+// sizes above is slower by more than 3 % (1064 rows on [13984 x 2816] in nf4 153 us against 137).  A K below 1024 leaves few column tiles, and there the walk along N is to be
+// no longer than four times K over 20 tiles at least.
 bool gemm_back_applies(int qtype, int M, int N, int K) {
-    const bool tall = back_tiles(M, K, 64) > 256;
-    const int64_t tiles = back_tiles(M, K, tall ? 128 : 64);
+    const BackPlan p = back_plan(qtype, M, N, K, (size_t)-1);
+    const int64_t tiles = back_tiles(M, K, p.rows);
     if (tiles > 256 || N >= (1 << 23)) return false;
-    return N <= 2 * (int64_t)K ? tiles >= 20 : qtype != QT_NF4 && tiles >= 80 && N <= 4 * (int64_t)K;
+    if (K < 1024) return tiles >= 20 && N <= (qtype == QT_NF4 ? 2 : 4) * (int64_t)K;
+    return tiles * p.splits >= 20;
 }
 
 // gx[M, K] = g[M, N] * dequant(w)[N, K]; w tiled, g and gx 16-byte aligned, N below 2^23 (32-bit offsets within a row tile)
-int launch_gemm_back(const void *g, const void *w, void *gx, int qtype, int act_dtype, int M, int N, int K, hipStream_t st) {
+int launch_gemm_back(const void *g, const void *w, void *gx, int qtype, int act_dtype, int M, int N, int K, void *ws, size_t ws_bytes,
+                     hipStream_t st) {
     if (M == 0 || K == 0) return 0;
     if (N >= (1 << 23)) return -3;
     switch (qtype) {
-    case QT_SYM_INT4: return launch_back_q<QT_SYM_INT4>(g, w, gx, act_dtype, M, N, K, st);
-    case QT_ASYM_INT4: return launch_back_q<QT_ASYM_INT4>(g, w, gx, act_dtype, M, N, K, st);
-    case QT_SYM_INT8: return launch_back_q<QT_SYM_INT8>(g, w, gx, act_dtype, M, N, K, st);
-    case QT_NF4: return launch_back_q<QT_NF4>(g, w, gx, act_dtype, M, N, K, st);
-    case QT_FP8_E4M3: return launch_back_q<QT_FP8_E4M3>(g, w, gx, act_dtype, M, N, K, st);
+    case QT_SYM_INT4: return launch_back_q<QT_SYM_INT4>(g, w, gx, act_dtype, M, N, K, ws, ws_bytes, st);
+    case QT_ASYM_INT4: return launch_back_q<QT_ASYM_INT4>(g, w, gx, act_dtype, M, N, K, ws, ws_bytes, st);
+    case QT_SYM_INT8: return launch_back_q<QT_SYM_INT8>(g, w, gx, act_dtype, M, N, K, ws, ws_bytes, st);
+    case QT_NF4: return launch_back_q<QT_NF4>(g, w, gx, act_dtype, M, N, K, ws, ws_bytes, st);
+    case QT_FP8_E4M3: return launch_back_q<QT_FP8_E4M3>(g, w, gx, act_dtype, M, N, K, ws, ws_bytes, st);
     default: return -2;
     }
 }

@@ -221,6 +221,20 @@ def lowbit_backward(grad, w, grad_x, qtype, act_dtype, m, n, k, stream):
     _check(_lib.lowbit_backward(grad, w, grad_x, qtype, act_dtype, m, n, k, stream), "lowbit_backward")
 
 
+_lib.lowbit_backward_ws.argtypes = [c_void_p, c_void_p, c_void_p, c_int, c_int, c_int64, c_int64, c_int64, c_void_p, c_size_t, c_void_p]
+_lib.lowbit_backward_ws.restype = c_int
+_lib.lowbit_backward_workspace_bytes.argtypes = [c_int, c_int64, c_int64, c_int64]
+_lib.lowbit_backward_workspace_bytes.restype = c_size_t
+
+
+def lowbit_backward_ws(grad, w, grad_x, qtype, act_dtype, m, n, k, workspace, workspace_bytes, stream):
+    _check(_lib.lowbit_backward_ws(grad, w, grad_x, qtype, act_dtype, m, n, k, workspace, workspace_bytes, stream), "lowbit_backward_ws")
+
+
+def lowbit_backward_workspace_bytes(qtype, m, n, k):
+    return _lib.lowbit_backward_workspace_bytes(qtype, m, n, k)
+
+
 def lowbit_backward_applies(qtype, layout, act_dtype, m, n, k):
     return bool(_lib.lowbit_backward_applies(qtype, layout, act_dtype, m, n, k))
 

@@ -164,3 +164,23 @@ def test_transforms_and_modes_get_what_the_autograd_function_gives():
         assert "aten::mm" in mode.seen and close(gx, grad, w, torch.float16)
     traced = torch.jit.trace(layer, x, check_trace=False)
     assert torch.equal(traced(x), layer(x))
+
+
+@pytest.mark.parametrize("m,n,k,rows", [(24, 4096, 1024, 64), (65, 2992, 1152, 64), (139, 4096, 2304, 64), (300, 6160, 1152, 64), (500, 8208, 2048, 128)])
+@pytest.mark.parametrize("qtype", ALL, ids=NAMES.values())
+def test_shared_walks(qtype, m, n, k, rows):
+    """Several workgroups on a tile's walk along N: last splits of other lengths than the first, a last step of 16 and 48 rows, row tiles
+    with rows past M; no more of the workspace is written than was asked for, and with half of it the answer is as good."""
+    dtype = torch.bfloat16 if qtype in (3, 15) else torch.float16
+    need = ggml.lowbit_backward_workspace_bytes(qtype, m, n, k)
+    per_split = -(-m // rows) * rows * k * 4
+    assert need >= 2 * per_split and need % per_split == 0 and need // per_split * (per_split // (rows * 512)) <= 256
+    blob = dev_quantize(weights(5, (n, k)), qtype, TILED)
+    grad = torch.randn((m, n), generator=torch.Generator().manual_seed(m)).to(dtype).cuda()
+    w = dev_dequantize(blob, qtype, n, k, TILED, dtype)
+    for size in (need, need // 2 // 16 * 16, 0):
+        ws = torch.full((need + 64,), 255, dtype=torch.uint8, device="cuda")
+        out = torch.full((m + 1, k), float("nan"), dtype=dtype, device="cuda")
+        ggml.lowbit_backward_ws(grad.data_ptr(), blob.data_ptr(), out.data_ptr(), qtype, DT[dtype], m, n, k, ws.data_ptr(), size, stream())
+        assert torch.isnan(out[m]).all() and close(out[:m], grad, w, dtype)
+        assert (ws[size:] == 255).all()
