@@ -43,10 +43,21 @@ static int device_cus() {
     return n_cus;
 }
 
+// Groups of more than 64 rows on average: how unevenly long they are then decides when a launch ends.
+static bool long_groups(int total_rows, int n_groups) { return total_rows > 64 * n_groups; }
+
+// Column tiles per cell of a plain tall launch: an eighth of a row tile, with long groups a single round of workgroups included.  A
+// row tile per XCD keeps its x in one L2, but gives the XCD of the longest group, or of a ninth row tile, twice the others' work
+// (512 tokens through two of 8 experts of [14336 x 4096], whole experts, us: fp8_e4m3 528 -> 498, sym_int4 482 -> 468; 600 through
+// four of 16 of [4096 x 2048] in sym_int8 241 -> 232; but 200 through two of those 8, 50 rows each, 298 -> 302).
+static int tall_chunk(int total_rows, int n_groups, int tiles_n, bool one_round) {
+    return grouped_chunk(tiles_n, one_round && !long_groups(total_rows, n_groups));
+}
+
 // Bytes of workspace per K split of the tall form: a partial tile per workgroup of the launch, whichever of the two
 // tile orders it takes (the grid, and with it a workgroup's slot in the workspace, depends on the order).
 static int tall_grid(int total_rows, int n_groups, int tiles_n, bool one_round) {
-    return grouped_grid(grouped_max_row_tiles(total_rows, n_groups, G_GM_TALL), tiles_n, grouped_chunk(tiles_n, one_round));
+    return grouped_grid(grouped_max_row_tiles(total_rows, n_groups, G_GM_TALL), tiles_n, tall_chunk(total_rows, n_groups, tiles_n, one_round));
 }
 static size_t tall_split_bytes(int total_rows, int n_groups, int N) {
     const int tiles_n = (N + G_GN - 1) / G_GN;
@@ -131,7 +142,10 @@ GroupedPlan grouped_plan(int total_rows, int n_groups, int N, int K, size_t ws_b
     if (s == 1 ? narrow.groups > 0 : s == 2 && narrow.groups == 2 && total_rows <= 96 * n_groups)
         return {false, 1, 4 * narrow.groups, narrow.chunk, narrow.groups};
     const bool tall = s > 1 || (int64_t)total_rows > (int64_t)n_groups * 96;
-    return {tall, s, grouped_waves(total_rows, n_groups, false), grouped_chunk(tiles_n, grouped_one_round(total_rows, n_groups, tiles_n, tall, s))};
+    const bool one_round = grouped_one_round(total_rows, n_groups, tiles_n, tall, s);
+    GroupedPlan plan = {tall, s, grouped_waves(total_rows, n_groups, false), tall ? tall_chunk(total_rows, n_groups, tiles_n, one_round) : grouped_chunk(tiles_n, one_round)};
+    plan.longest_first = tall && long_groups(total_rows, n_groups);
+    return plan;
 }
 
 // What launch_grouped_gemm would do for a plain grouped product: {tall, splits, waves, grid.x}.
@@ -153,7 +167,9 @@ static GroupedPlan grouped_mlp_plan(int total_rows, int n_groups, int N, int K) 
     const NarrowPlan narrow = grouped_narrow(total_rows, n_groups, (N + G_GN / 4 - 1) / (G_GN / 4), K);
     if (narrow.groups) return {false, 1, 4 * narrow.groups, narrow.chunk, narrow.groups};
     const int tiles_n = (N + G_GN / 2 - 1) / (G_GN / 2);
-    return {true, 1, grouped_waves(total_rows, n_groups, true), grouped_chunk(tiles_n, grouped_one_round(total_rows, n_groups, tiles_n, true, 1))};
+    GroupedPlan plan = {true, 1, grouped_waves(total_rows, n_groups, true), grouped_chunk(tiles_n, grouped_one_round(total_rows, n_groups, tiles_n, true, 1))};
+    plan.longest_first = long_groups(total_rows, n_groups);
+    return plan;
 }
 
 // y[rows of group e] = x[rows of group e] * dequant(w[e])^T, or, with w_up, act(x w[e]^T) * (x w_up[e]^T).

@@ -38,12 +38,12 @@ static_assert(4 * (MB32_TALL * (GN / 4 / 32) * 4) * 64 * 4 == GM_TALL * GN && 8 
 template <typename AT, int WAVES>
 __global__ __launch_bounds__(256) void grouped_splitk_reduce_kernel(const float *__restrict__ ws, AT *__restrict__ y,
                                                                     const int32_t *__restrict__ offsets, int n_groups,
-                                                                    int N, int tiles_n, int chunk, int n_wg, int splits) {
+                                                                    int N, int tiles_n, int chunk, int n_wg, int splits, bool longest_first) {
     constexpr int NBW = GN / WAVES / 32;                               // 32-row weight blocks per wave of the GEMM
     constexpr int REGS = MB32_TALL * NBW * 4;                          // groups of 4 accumulators per lane and wave
     const int b = blockIdx.x / WAVES, wave = blockIdx.x % WAVES;       // workgroup and wave of the GEMM
     GroupTile gt;
-    if (!grouped_tile<GM_TALL>(offsets, n_groups, tiles_n, chunk, b, gt)) return;
+    if (!grouped_tile<GM_TALL>(offsets, n_groups, tiles_n, chunk, b, longest_first, gt)) return;
     const int lane = threadIdx.x & 63;
     const int64_t per_split = (int64_t)n_wg * WAVES * REGS * 64 * 4;   // floats
     const float *base = ws + ((int64_t)(b * WAVES + wave) * REGS * 64 + lane) * 4;
@@ -69,7 +69,7 @@ static int launch_grouped_t(const void *x, const void *const *w, void *y, const 
                             int total_rows, int N, int K, const GroupedPlan &plan, float *ws, hipStream_t st) {
     if (plan.narrow) {
         const int tiles_n = (N + GN / 2 - 1) / (GN / 2), G = K / TILE_COLS, chunk = plan.chunk;
-        const GroupArgs ga = {offsets, (const uint8_t *const *)w, nullptr, n_groups, 0, 0, chunk};
+        const GroupArgs ga = {offsets, (const uint8_t *const *)w, nullptr, n_groups, 0, 0, chunk, nullptr, nullptr, plan.longest_first};
         const int grid = grouped_grid(grouped_max_row_tiles(total_rows, n_groups, GM), tiles_n, chunk);
         if (plan.narrow == 2)
             hipLaunchKernelGGL((gemm_mfma_kernel<QT, AT, true, MB32, true, false, 4, true, 2>), dim3(grid), dim3(512), 0, st, (const AT *)x,
@@ -81,7 +81,7 @@ static int launch_grouped_t(const void *x, const void *const *w, void *y, const 
     }
     const int tiles_n = (N + GN - 1) / GN, G = K / TILE_COLS;
     const int chunk = plan.chunk;
-    const GroupArgs ga = {offsets, (const uint8_t *const *)w, nullptr, n_groups, 0, 0, chunk};
+    const GroupArgs ga = {offsets, (const uint8_t *const *)w, nullptr, n_groups, 0, 0, chunk, nullptr, nullptr, plan.longest_first};
     if (!plan.tall) {
         const int grid = grouped_grid(grouped_max_row_tiles(total_rows, n_groups, GM), tiles_n, chunk);
         hipLaunchKernelGGL((gemm_mfma_kernel<QT, AT, true, MB32, true>), dim3(grid), dim3(256), 0, st, (const AT *)x,
@@ -97,7 +97,7 @@ static int launch_grouped_t(const void *x, const void *const *w, void *y, const 
                        (const uint8_t *)nullptr, (AT *)y, 0, N, K, 1, ga, k_steps, ws, 0, tiles_n);
     if (ws) {
         hipLaunchKernelGGL((grouped_splitk_reduce_kernel<AT, 4>), dim3((unsigned)(n_wg * 4)), dim3(256), 0, st, ws,
-                           (AT *)y, offsets, n_groups, N, tiles_n, chunk, n_wg, ny);
+                           (AT *)y, offsets, n_groups, N, tiles_n, chunk, n_wg, ny, plan.longest_first);
     }
     return 0;
 }
@@ -108,7 +108,7 @@ static int launch_grouped_mlp_t(const void *x, const void *const *wg, const void
                                 const GroupedPlan &plan, hipStream_t st) {
     if (plan.narrow) {
         const int tiles_n = (N + GN / 4 - 1) / (GN / 4), G = K / TILE_COLS, chunk = plan.chunk;   // 64 columns of both
-        const GroupArgs ga = {offsets, (const uint8_t *const *)wg, (const uint8_t *const *)wu, n_groups, act, 0, chunk};
+        const GroupArgs ga = {offsets, (const uint8_t *const *)wg, (const uint8_t *const *)wu, n_groups, act, 0, chunk, nullptr, nullptr, plan.longest_first};
         const int grid = grouped_grid(grouped_max_row_tiles(total_rows, n_groups, GM), tiles_n, chunk);
         if (plan.narrow == 2)
             hipLaunchKernelGGL((gemm_mfma_kernel<QT, AT, true, MB32, true, true, 4, true, 2>), dim3(grid), dim3(512), 0, st, (const AT *)x,
@@ -120,7 +120,7 @@ static int launch_grouped_mlp_t(const void *x, const void *const *wg, const void
     }
     const int tiles_n = (N + GN / 2 - 1) / (GN / 2), G = K / TILE_COLS;      // 128 columns of both weights per workgroup
     const int chunk = plan.chunk;
-    const GroupArgs ga = {offsets, (const uint8_t *const *)wg, (const uint8_t *const *)wu, n_groups, act, 0, chunk};
+    const GroupArgs ga = {offsets, (const uint8_t *const *)wg, (const uint8_t *const *)wu, n_groups, act, 0, chunk, nullptr, nullptr, plan.longest_first};
     const int n_wg = grouped_grid(grouped_max_row_tiles(total_rows, n_groups, GM_TALL), tiles_n, chunk);
     // nf4 always takes the eight-wave form: its two waves per SIMD cover each other's code book reads (the dense
     // tall form gains 5-9 % from it), and with four waves, two weight blocks and the lookups' temporaries the fused

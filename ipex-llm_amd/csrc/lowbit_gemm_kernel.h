@@ -54,6 +54,7 @@ struct GroupArgs {
     int chunk;                    // grouped: column tiles per cell of the tile order (see grouped_tile)
     const uint8_t *w_up_one;      // fused form without tables (offsets == nullptr): the up weight
     const void *bias;             // dense forms: [N] in the activation type, or null
+    bool longest_first;           // grouped, up to 64 groups: order of the partly filled row tiles (see grouped_tile)
 };
 
 // Which row tile of which group, and which column tile, workgroup `b` of a grouped launch works on.
@@ -70,6 +71,11 @@ struct GroupArgs {
 //     groups are (a group per XCD was 9-12 % slower with 10 to 300 rows per group);
 //   - with chunk = tiles_n a row tile is one cell: all its column tiles on one XCD, for launches of a single round.
 //     Shares matter there only where they make a second round of the largest one (narrow tiles: grouped_narrow).
+//   - the partly filled row tiles of long groups come longest first (up to 64 groups): the launch then ends on short ones.  Rows
+//     per expert are uneven in earnest, and the launch waited for whichever tile came last: 600 tokens, three of 6 experts of
+//     [8192 x 4096] in sym_int8, whole experts, 481 -> 443 us, 450 tokens, four of 16 of [6144 x 3072] in asym_int4 351 -> 341;
+//     but 200 tokens, two of 8 of [14336 x 4096] in sym_int4 (50 rows each: tiles that wait for HBM, which mixed lengths share
+//     better) 303 -> 310.
 // Workgroups beyond an XCD's last cell leave at once; they are the last of that XCD's sequence (workgroups go to
 // the compute units of an XCD in turn: idle ones between working ones leave units idle).
 struct GroupTile {
@@ -97,9 +103,10 @@ __device__ inline bool grouped_cell(int row_tiles, int tiles_n, int chunk, int b
 // gate/up launch of 64 groups x [1408 x 2048] with 6144 rows took 158 us that way and takes 125 us this way
 // (60 groups, 2048 rows: 114 -> 87; 8 groups: no difference).  Every wave of the workgroup calls this with all
 // lanes active.
+// longest_first: the partly filled row tiles with more 32-row blocks first, equal ones in the groups' order.
 template <int ROWS>
 __device__ inline bool grouped_tile_lanes(const int32_t *__restrict__ offsets, int n_groups, int tiles_n, int chunk, int b,
-                                          GroupTile &t) {
+                                          bool longest_first, GroupTile &t) {
     const int lane = threadIdx.x & 63;
     const bool on = lane < n_groups;
     const int r0 = on ? offsets[lane] : 0, r1 = on ? offsets[lane + 1] : 0;
@@ -118,8 +125,18 @@ __device__ inline bool grouped_tile_lanes(const int32_t *__restrict__ offsets, i
     if (!grouped_cell(full + __popcll(pm), tiles_n, chunk, b, idx, t.tile_n)) return false;
     const bool want_full = idx < full;
     if (!want_full) idx -= full;
-    const uint64_t hit = want_full ? __ballot(incl - f <= idx && idx < incl)
-                                   : __ballot(p && __popcll(pm & ((1ull << lane) - 1ull)) == idx);
+    int place = __popcll(pm & ((1ull << lane) - 1ull));  // of this group's partly filled tile among them
+    if (longest_first) {
+        const int blocks = (rows % ROWS + 31) / 32;
+        place = 0;
+#pragma unroll
+        for (int c = ROWS / 32; c >= 1; c--) {
+            const uint64_t same = __ballot(blocks == c);
+            if (blocks == c) place += __popcll(same & ((1ull << lane) - 1ull));
+            else if (blocks < c) place += __popcll(same);
+        }
+    }
+    const uint64_t hit = want_full ? __ballot(incl - f <= idx && idx < incl) : __ballot(p && place == idx);
     if (!hit) return false;
     const int g = __ffsll((unsigned long long)hit) - 1;
     const int gf = __builtin_amdgcn_readlane(f, g);
@@ -130,8 +147,8 @@ __device__ inline bool grouped_tile_lanes(const int32_t *__restrict__ offsets, i
 }
 template <int ROWS>
 __device__ inline bool grouped_tile(const int32_t *__restrict__ offsets, int n_groups, int tiles_n, int chunk, int b,
-                                    GroupTile &t) {
-    if (n_groups <= 64) return grouped_tile_lanes<ROWS>(offsets, n_groups, tiles_n, chunk, b, t);
+                                    bool longest_first, GroupTile &t) {
+    if (n_groups <= 64) return grouped_tile_lanes<ROWS>(offsets, n_groups, tiles_n, chunk, b, longest_first, t);
     int full = 0, part = 0;
     for (int e = 0; e < n_groups; e++) {
         const int rows = offsets[e + 1] - offsets[e];
@@ -288,7 +305,7 @@ __global__ __launch_bounds__(64 * WAVES * KS, (DMA && MB == 4) ? 2 : 1) void gem
             if constexpr (DUAL) w_up_lane = (uint64_t)ga.w_up[lane];
         }
         GroupTile gt;
-        if (!grouped_tile<GM>(ga.offsets, ga.n_groups, tn_cnt, ga.chunk, blockIdx.x, gt)) return;    // whole workgroup leaves
+        if (!grouped_tile<GM>(ga.offsets, ga.n_groups, tn_cnt, ga.chunk, blockIdx.x, ga.longest_first, gt)) return;    // whole workgroup leaves
         // (the compiler does not see that what comes out of the walk is the same in every lane)
         tile_n = __builtin_amdgcn_readfirstlane(gt.tile_n);
         m0 = __builtin_amdgcn_readfirstlane(gt.m0);

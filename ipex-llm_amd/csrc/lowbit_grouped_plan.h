@@ -17,6 +17,7 @@ struct GroupedPlan {
     int chunk;      // column tiles per cell of the tile order (grouped_tile in lowbit_gemm_kernel.h)
     int narrow = 0; // narrow tiles, with one or two groups of waves (0: not)
     bool halves = false;   // narrow tiles of a dense gated MLP: in halves of 64 rows
+    bool longest_first = false;   // order of the partly filled row tiles (grouped_tile)
 };
 
 // Upper bound of the number of `rows`-row tiles: every group adds at most one partly filled tile.

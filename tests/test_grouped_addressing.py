@@ -48,7 +48,7 @@ def grouped_tile(offs, tiles_n, chunk, b):
     return None
 
 
-def grouped_tile_lanes(offs, tiles_n, chunk, b):
+def grouped_tile_lanes(offs, tiles_n, chunk, b, longest_first=False):
     """The same answer found the way a wave finds it for up to 64 groups (grouped_tile_lanes): lane e holds group
     e's offsets, an inclusive prefix sum over the lanes counts whole row tiles, a ballot marks the groups with a
     partly filled one, and the group comes out of a ballot over 'my range of row tiles holds idx'."""
@@ -89,7 +89,18 @@ def grouped_tile_lanes(offs, tiles_n, chunk, b):
         hit = [l for l in lanes if incl[l] - f[l] <= idx < incl[l]]
     else:
         idx -= full
-        hit = [l for l in lanes if p[l] and bin(pm & ((1 << l) - 1)).count("1") == idx]
+        place = [bin(pm & ((1 << l) - 1)).count("1") for l in lanes]
+        if longest_first:
+            blocks = [(rows[l] % ROWS + 31) // 32 for l in lanes]
+            place = [0] * 64
+            for c in range(ROWS // 32, 0, -1):
+                same = sum(1 << l for l in lanes if blocks[l] == c)
+                for l in lanes:
+                    if blocks[l] == c:
+                        place[l] += bin(same & ((1 << l) - 1)).count("1")
+                    elif blocks[l] < c:
+                        place[l] += bin(same).count("1")
+        hit = [l for l in lanes if p[l] and place[l] == idx]
     if not hit:
         return None
     g = hit[0]
@@ -310,6 +321,21 @@ def test_lane_lookup_agrees_with_the_walk_over_the_offsets(n_groups):
             got = [grouped_tile_lanes(offs, tiles_n, chunk, b) for b in range(n_wg)]
             assert got == [grouped_tile(offs, tiles_n, chunk, b) for b in range(n_wg)]
             assert sum(g is not None for g in got) == row_tiles * tiles_n
+
+
+@pytest.mark.parametrize("n_groups", [1, 9, 64])
+def test_longest_first_holds_every_tile_once_and_ends_on_the_shortest(n_groups):
+    rng = np.random.default_rng(n_groups + 100)
+    for _ in range(6):
+        counts = rng.integers(0, 2 * ROWS, n_groups)
+        offs = [0] + [int(v) for v in np.cumsum(counts)]
+        n_wg = grouped_grid(offs[-1] // ROWS + n_groups, 5, 2)
+        got = [grouped_tile_lanes(offs, 5, 2, b, True) for b in range(n_wg)]
+        want = [grouped_tile(offs, 5, 2, b) for b in range(n_wg)]
+        assert sorted(t for t in got if t) == sorted(t for t in want if t)
+        order = [grouped_tile_lanes(offs, 1, 1, b, True) for b in range(grouped_grid(offs[-1] // ROWS + n_groups, 1, 1))]
+        blocks = [min(-(-(t[2] - t[1]) // 32), 8) for t in order if t]
+        assert blocks == sorted(blocks, reverse=True)
 
 
 def test_no_xcd_gets_a_second_round_of_narrow_tiles():
