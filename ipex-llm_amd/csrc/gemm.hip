@@ -28,9 +28,9 @@ int launch_gemm_rows(const void *x, const void *w, const void *bias, void *y, in
 // register group, lane) and writes y, rounded once.  One thread per group of 4 consecutive n.
 template <typename AT>
 __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float *__restrict__ ws, AT *__restrict__ y,
-                                                            const AT *__restrict__ bias, int M, int N, int splits) {
+                                                            const AT *__restrict__ bias, int M, int N, int splits, int tile_rows) {
     const int tiles_n = (N + GN - 1) / GN;
-    const int64_t n_tiles_all = (int64_t)((M + GM - 1) / GM) * tiles_n;
+    const int64_t n_tiles_all = (int64_t)((M + tile_rows - 1) / tile_rows) * tiles_n;
     const int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x;       // (tile, wave, group, lane)
     if (t >= n_tiles_all * 4 * (MB32 * NB32 * 4) * 64) return;
     const int lane = (int)(t & 63);
@@ -38,9 +38,9 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float *__restr
     const int wave = (int)((t >> 6) / (MB32 * NB32 * 4) % 4);
     const int64_t tile_id = (t >> 6) / (MB32 * NB32 * 4) / 4;
     const int mb = grp / (NB32 * 4), nb = grp / 4 % NB32, q = grp % 4;
-    const int m = (int)(tile_id / tiles_n) * GM + mb * 32 + (lane & 31);
+    const int m = (int)(tile_id / tiles_n) * tile_rows + mb * 32 + (lane & 31);
     const int n = (int)(tile_id % tiles_n) * GN + wave * GN_WAVE + nb * 32 + q * 8 + (lane >> 5) * 4;
-    if (m >= M || n >= N) return;
+    if (mb * 32 >= tile_rows || m >= M || n >= N) return;
     const int64_t per_split = n_tiles_all * 4 * (MB32 * NB32 * 4) * 64 * 4;     // floats
     f32x4 a = *(const f32x4 *)(ws + t * 4);
     for (int s = 1; s < splits; s++) a += *(const f32x4 *)(ws + (int64_t)s * per_split + t * 4);
@@ -170,6 +170,8 @@ static int launch_gemm_t(const void *x, const void *w, const void *bias, void *y
     const int tall = ws ? 0 : tall_columns(M, N, K, n_cus, QT);
     if (tall > 0) {
         const int tiles_m = (M + GM_TALL - 1) / GM_TALL;
+        ga.tile_rows = GM_TALL;
+        ga.row_tiles = tiles_m;
         const unsigned grid = 8 * (unsigned)(((int64_t)tiles_m * tall + 7) / 8);
         // (four waves, which read each x operand from LDS once per two MFMAs: 2-4 % faster than eight)
         hipLaunchKernelGGL((gemm_mfma_kernel<QT, AT, true, MB32_TALL>), dim3(grid), dim3(256), 0, st,
@@ -180,6 +182,8 @@ static int launch_gemm_t(const void *x, const void *w, const void *bias, void *y
             // M = 1000 483 -> 469 us; where at most one 128 x 256 tile per CU is left, which would take the
             // register-staged form below, [11008 x 4096] at M = 2047 212 -> 171, [28672 x 8192] at M = 700 404 -> 328)
             const int left = (N + GN / 2 - 1) / (GN / 2) - 2 * tall, tiles_m = (M + GM - 1) / GM;
+            ga.tile_rows = GM;
+            ga.row_tiles = tiles_m;
             hipLaunchKernelGGL((gemm_mfma_kernel<QT, AT, true, MB32, false, false, 4, true>),
                                dim3(8 * (unsigned)(((int64_t)tiles_m * left + 7) / 8)), dim3(256), 0, st, (const AT *)x, (const uint8_t *)w,
                                (AT *)y, M, N, K, band_rows(tiles_m), ga, G, (float *)nullptr, 2 * tall, left);
@@ -194,6 +198,8 @@ static int launch_gemm_t(const void *x, const void *w, const void *bias, void *y
     const bool fits24 = M < (1 << 24) && K < (1 << 23);              // 24-bit row offsets
     const bool dma = fits24 && (QT != QT_NF4 || tiles_m * tiles_n * ny > 256);
     ga.split_tail = (dma && !ws) ? split_tail_tiles(M, (int64_t)tiles_m * tiles_n, n_cus) : 0;
+    ga.tile_rows = dma && !ga.split_tail ? dense_tile_rows(M) : GM;
+    ga.row_tiles = tiles_m;
     dim3 grid(8 * (unsigned)(((int64_t)tiles_m * tiles_n + 7) / 8 + ga.split_tail), ny);
     // Two forms of the kernel.  The DMA form (x straight into LDS, one K step of prefetch, 128 vector registers)
     // lets a CU hold two workgroups that cover each other's waits, and is 4-8 % ahead with a single workgroup per
@@ -208,7 +214,7 @@ static int launch_gemm_t(const void *x, const void *w, const void *bias, void *y
     if (ws) {
         const int64_t threads = (int64_t)tiles_m * tiles_n * (GM * GN / 4);
         hipLaunchKernelGGL((splitk_reduce_kernel<AT>), dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, st, ws,
-                           (AT *)y, (const AT *)bias, M, N, ny);
+                           (AT *)y, (const AT *)bias, M, N, ny, ga.tile_rows);
     }
     return 0;
 }
@@ -271,6 +277,8 @@ static int launch_gemm_narrow_t(const void *x, const void *w, const void *bias, 
     GroupArgs ga{};
     ga.bias = bias;
     ga.split_tail = halves ? (int)(((int64_t)tiles_m * tiles_n) / 8) + 1 : 0;
+    ga.tile_rows = halves ? GM : dense_tile_rows(M);
+    ga.row_tiles = tiles_m;
     dim3 grid(8 * (unsigned)(((int64_t)tiles_m * tiles_n + 7) / 8 + ga.split_tail), 1);
     if (narrow_two_groups(M, N, K))
         hipLaunchKernelGGL((gemm_mfma_kernel<QT, AT, true, MB32, false, false, 4, true, 2>), grid, dim3(512), 0, st, (const AT *)x,

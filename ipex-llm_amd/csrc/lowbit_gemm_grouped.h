@@ -69,7 +69,7 @@ static int launch_grouped_t(const void *x, const void *const *w, void *y, const 
                             int total_rows, int N, int K, const GroupedPlan &plan, float *ws, hipStream_t st) {
     if (plan.narrow) {
         const int tiles_n = (N + GN / 2 - 1) / (GN / 2), G = K / TILE_COLS, chunk = plan.chunk;
-        const GroupArgs ga = {offsets, (const uint8_t *const *)w, nullptr, n_groups, 0, 0, chunk, nullptr, nullptr, plan.longest_first};
+        const GroupArgs ga = {offsets, (const uint8_t *const *)w, nullptr, {n_groups}, 0, {plan.longest_first}, {chunk}};
         const int grid = grouped_grid(grouped_max_row_tiles(total_rows, n_groups, GM), tiles_n, chunk);
         if (plan.narrow == 2)
             hipLaunchKernelGGL((gemm_mfma_kernel<QT, AT, true, MB32, true, false, 4, true, 2>), dim3(grid), dim3(512), 0, st, (const AT *)x,
@@ -81,7 +81,7 @@ static int launch_grouped_t(const void *x, const void *const *w, void *y, const 
     }
     const int tiles_n = (N + GN - 1) / GN, G = K / TILE_COLS;
     const int chunk = plan.chunk;
-    const GroupArgs ga = {offsets, (const uint8_t *const *)w, nullptr, n_groups, 0, 0, chunk, nullptr, nullptr, plan.longest_first};
+    const GroupArgs ga = {offsets, (const uint8_t *const *)w, nullptr, {n_groups}, 0, {plan.longest_first}, {chunk}};
     if (!plan.tall) {
         const int grid = grouped_grid(grouped_max_row_tiles(total_rows, n_groups, GM), tiles_n, chunk);
         hipLaunchKernelGGL((gemm_mfma_kernel<QT, AT, true, MB32, true>), dim3(grid), dim3(256), 0, st, (const AT *)x,
@@ -108,7 +108,7 @@ static int launch_grouped_mlp_t(const void *x, const void *const *wg, const void
                                 const GroupedPlan &plan, hipStream_t st) {
     if (plan.narrow) {
         const int tiles_n = (N + GN / 4 - 1) / (GN / 4), G = K / TILE_COLS, chunk = plan.chunk;   // 64 columns of both
-        const GroupArgs ga = {offsets, (const uint8_t *const *)wg, (const uint8_t *const *)wu, n_groups, act, 0, chunk, nullptr, nullptr, plan.longest_first};
+        const GroupArgs ga = {offsets, (const uint8_t *const *)wg, (const uint8_t *const *)wu, {n_groups}, act, {plan.longest_first}, {chunk}};
         const int grid = grouped_grid(grouped_max_row_tiles(total_rows, n_groups, GM), tiles_n, chunk);
         if (plan.narrow == 2)
             hipLaunchKernelGGL((gemm_mfma_kernel<QT, AT, true, MB32, true, true, 4, true, 2>), dim3(grid), dim3(512), 0, st, (const AT *)x,
@@ -120,7 +120,7 @@ static int launch_grouped_mlp_t(const void *x, const void *const *wg, const void
     }
     const int tiles_n = (N + GN / 2 - 1) / (GN / 2), G = K / TILE_COLS;      // 128 columns of both weights per workgroup
     const int chunk = plan.chunk;
-    const GroupArgs ga = {offsets, (const uint8_t *const *)wg, (const uint8_t *const *)wu, n_groups, act, 0, chunk, nullptr, nullptr, plan.longest_first};
+    const GroupArgs ga = {offsets, (const uint8_t *const *)wg, (const uint8_t *const *)wu, {n_groups}, act, {plan.longest_first}, {chunk}};
     const int n_wg = grouped_grid(grouped_max_row_tiles(total_rows, n_groups, GM_TALL), tiles_n, chunk);
     // nf4 always takes the eight-wave form: its two waves per SIMD cover each other's code book reads (the dense
     // tall form gains 5-9 % from it), and with four waves, two weight blocks and the lookups' temporaries the fused
@@ -147,6 +147,8 @@ static int launch_mlp_gemm_t(const void *x, const void *wg, const void *wu, void
         ga.act = act;
         ga.w_up_one = (const uint8_t *)wu;
         ga.split_tail = plan.halves ? (int)(((int64_t)tiles_m * tiles_n) / 8) + 1 : 0;
+        ga.tile_rows = plan.halves ? GM : dense_tile_rows(M);
+        ga.row_tiles = tiles_m;
         const dim3 grid(8 * (unsigned)(((int64_t)tiles_m * tiles_n + 7) / 8 + ga.split_tail));
         if (plan.narrow == 2)
             hipLaunchKernelGGL((gemm_mfma_kernel<QT, AT, true, MB32, false, true, 4, true, 2>), grid, dim3(512), 0, st, (const AT *)x,
@@ -158,7 +160,7 @@ static int launch_mlp_gemm_t(const void *x, const void *wg, const void *wu, void
     }
     const int tiles_n = (N + GN / 2 - 1) / (GN / 2), G = K / TILE_COLS;
     const int chunk = plan.chunk;
-    const GroupArgs ga = {nullptr, nullptr, nullptr, 1, act, 0, chunk, (const uint8_t *)wu};
+    const GroupArgs ga = {nullptr, nullptr, nullptr, {1}, act, {0}, {chunk}, (const uint8_t *)wu};
     const int n_wg = grouped_grid((M + GM_TALL - 1) / GM_TALL, tiles_n, chunk);
     if (plan.waves == 8 || QT == QT_NF4) {            // (nf4: see launch_grouped_mlp_t)
         hipLaunchKernelGGL((gemm_mfma_kernel<QT, AT, true, MB32_TALL, true, true, 8>), dim3(n_wg), dim3(512), 0, st, (const AT *)x,

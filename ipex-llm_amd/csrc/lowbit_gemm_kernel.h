@@ -43,18 +43,28 @@ constexpr int GM_TALL = 256, MB32_TALL = GM_TALL / 32;
 // (and w_up[e] in the fused gate/up form); all pointers are device memory.
 // The fused gate/up form also runs a dense gated MLP - one group that holds all M rows - without any table in
 // device memory: offsets == nullptr, the gate weight is the kernel's own `w` argument, the up weight w_up_one.
+// Fields that only dense and only grouped launches need share their place: the kernel's arguments stay within two lines of 64
+// bytes.
 struct GroupArgs {
     const int32_t *offsets;
     const uint8_t *const *w;
     const uint8_t *const *w_up;
-    int n_groups;
+    union {
+        int n_groups;
+        int row_tiles;            // dense: how many row tiles
+    };
     int act;                      // activation of the gate branch in the fused form: 0 = SiLU, 1 = tanh-GELU
-    int split_tail;               // dense 128-row DMA form: the last split_tail tiles of every XCD's share go out as two
+    union {
+        int split_tail;           // dense 128-row DMA form: the last split_tail tiles of every XCD's share go out as two
                                   // half tiles of 64 rows each, to one workgroup apiece
-    int chunk;                    // grouped: column tiles per cell of the tile order (see grouped_tile)
+        int longest_first;        // grouped, up to 64 groups: order of the partly filled row tiles (see grouped_tile)
+    };
+    union {
+        int chunk;                // grouped: column tiles per cell of the tile order (see grouped_tile)
+        int tile_rows;            // dense: rows from one row tile to the next (see dense_tile_rows)
+    };
     const uint8_t *w_up_one;      // fused form without tables (offsets == nullptr): the up weight
     const void *bias;             // dense forms: [N] in the activation type, or null
-    bool longest_first;           // grouped, up to 64 groups: order of the partly filled row tiles (see grouped_tile)
 };
 
 // Which row tile of which group, and which column tile, workgroup `b` of a grouped launch works on.
@@ -261,8 +271,9 @@ __global__ __launch_bounds__(64 * WAVES * KS, (DMA && MB == 4) ? 2 : 1) void gem
     // tiles are a second round for an XCD whose 32 CUs hold 64 workgroups.
     int m0, tile_n;
     const uint8_t *w_up = nullptr;
+    int row_tile = 0;
     if constexpr (!GROUPED) {
-        const int tiles_m = (M + GM - 1) / GM, tiles_n = tn_cnt;
+        const int pitch = ga.tile_rows, tiles_m = ga.row_tiles, tiles_n = tn_cnt;
         const int64_t T = (int64_t)tiles_m * tiles_n;
         const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
         const int first = (int)(T * xcd / 8), count = (int)(T * (xcd + 1) / 8) - first;
@@ -282,8 +293,10 @@ __global__ __launch_bounds__(64 * WAVES * KS, (DMA && MB == 4) ? 2 : 1) void gem
         const int band = line / per_band, r = line - band * per_band;
         const int rows_b = tiles_m - band * band_m < band_m ? tiles_m - band * band_m : band_m;   // the last band may be short
         tile_n = r / rows_b + tn0;
-        m0 = (band * band_m + r % rows_b) * GM;
-        if (half >= 0) {
+        row_tile = band * band_m + r % rows_b;
+        m0 = row_tile * pitch;
+        if (half < 0) M = M < m0 + pitch ? M : m0 + pitch;                           // rows past the tile are clamped / not stored
+        else {
             m0 += (GM / 2) * half;
             if (m0 >= M) return;                                                     // (a last row tile of at most 64 rows)
             M = M < m0 + GM / 2 ? M : m0 + GM / 2;                                   // rows past the half are clamped / not stored
@@ -855,8 +868,8 @@ __global__ __launch_bounds__(64 * WAVES * KS, (DMA && MB == 4) ? 2 : 1) void gem
             // store is 1 KiB contiguous, straight from the accumulation registers, whole tiles whatever M and N
             // (the workspace holds whole tiles; the reduction kernel reads what lies inside y and undoes the layout).
             // dense: tiles in row-major order; grouped: in the order of the launch
-            const int64_t tile_id = GROUPED ? (int64_t)blockIdx.x : (int64_t)(m0 / GM) * ((N + GN - 1) / GN) + tile_n;
-            const int64_t n_tiles_all = GROUPED ? (int64_t)gridDim.x : (int64_t)((M + GM - 1) / GM) * ((N + GN - 1) / GN);
+            const int64_t tile_id = GROUPED ? (int64_t)blockIdx.x : (int64_t)row_tile * ((N + GN - 1) / GN) + tile_n;
+            const int64_t n_tiles_all = GROUPED ? (int64_t)gridDim.x : (int64_t)ga.row_tiles * ((N + GN - 1) / GN);
             float *const wp = ws + ((((int64_t)blockIdx.y * n_tiles_all + tile_id) * WAVES + wave) * (MB32 * NB32 * 4)) * 256 + lane * 4;
 #pragma unroll
             for (int mb = MB0; mb < MBC; mb++) {
@@ -1164,7 +1177,8 @@ __global__ __launch_bounds__(64 * WAVES * KS, (DMA && MB == 4) ? 2 : 1) void gem
             if constexpr (KS == 2) meet(acc, mbc);
             else epilogue(acc, first_t(), mbc);
         };
-        // tail tiles and small expert groups: 32-row blocks without rows of x skip their MFMAs
+        // tail tiles and small expert groups: 32-row blocks without rows of x skip their MFMAs (three blocks instead of four:
+        // 94 rows on [8464 x 19200] in sym_int4 63.9 -> 56.0 us, 90 on [9104 x 6272] in sym_int8 38.2 -> 34.7)
         const int mb_cnt = (M - m0 + 31) / 32;
         if constexpr (MB32 == 8 && !GROUPED) {
             // the dense launcher hands the tall form row tiles that are more than half full
@@ -1186,6 +1200,8 @@ __global__ __launch_bounds__(64 * WAVES * KS, (DMA && MB == 4) ? 2 : 1) void gem
             run(std::integral_constant<int, 1>());
         } else if (mb_cnt <= 2) {
             run(std::integral_constant<int, 2>());
+        } else if (mb_cnt == 3) {
+            run(std::integral_constant<int, 3>());
         } else {
             run(full_t());
         }
@@ -1226,6 +1242,15 @@ __global__ __launch_bounds__(64 * WAVES * KS, (DMA && MB == 4) ? 2 : 1) void gem
 #undef LOWBIT_GEMM_STEP
     epilogue(acc, first_t(), full_t());
     }
+}
+
+// Rows from one row tile to the next in the dense 128-row DMA forms: as many 32-row blocks in every tile as in the others where
+// that is fewer than four, because the launch lasts as long as its fullest tiles: 129 .. 192 and 257 .. 288 rows in tiles of 96.
+// Tiles of 128 and a rest / of 96, us: 150 rows on [8464 x 8192] in sym_int4 43.9 / 42.0, 176 on [14336 x 4096] in nf4 34.2 / 31.5,
+// 270 on [11008 x 4096] in asym_int4 42.8 / 39.3, a layer of [4096 x 4096] and [11008 x 4096] at 160 rows 145 / 136.
+inline int dense_tile_rows(int M) {
+    const int tiles = (M + GM - 1) / GM, blocks = (M + 31) / 32;
+    return tiles > 1 ? (blocks + tiles - 1) / tiles * 32 : GM;
 }
 
 // Row tiles per band of the kernel's tile order (see the kernel): the row tiles are cut into at most 8 bands, a

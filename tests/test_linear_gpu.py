@@ -64,6 +64,15 @@ def test_bias_of_every_kernel(qtype, dtype, m, n, k):
 ROW_MAJOR = [(1, 2000, 4160), (7, 1000, 4160), (12, 1000, 4160), (16, 16399, 1088), (30, 1000, 4160), (70, 1000, 4160), (333, 1000, 4160)]
 
 
+@pytest.mark.parametrize("qtype,dtype", [(2, torch.float16), (3, torch.bfloat16), (8, torch.float16), (10, torch.bfloat16), (15, torch.bfloat16)])
+@pytest.mark.parametrize("m", [65, 96, 97, 129, 161, 192, 193, 257, 288, 289])
+@pytest.mark.parametrize("n,k", [(1040, 4096), (2064, 1152), (16400, 256)], ids=["splits", "narrow", "wide"])
+def test_row_tiles_of_three_blocks(qtype, dtype, m, n, k):
+    """Three 32-row blocks in a tile, as a last one and as the height of all (129 .. 192 and 257 .. 288 rows), and the counts beside
+    them; with K splits, in narrow tiles and in 128 x 256 tiles."""
+    _check(qtype, dtype, ggml.LAYOUT_TILED, m, n, k, m % 2 == 1, m + n)
+
+
 def _plain(qtype, m, n, k, dtype):
     if qtype == FP8 and k % 128:
         n, k = n + 1, (k + 127) // 128 * 128

@@ -42,6 +42,12 @@ def test_gated_mlp_tiles(qtype, m, n, k):
     assert torch.isnan(y[m]).all() and mlp_close(y[:m], x, blobs, qtype, n, k, act)
 
 
+@pytest.mark.parametrize("m,n,k", [(90, 5008, 1152), (176, 8208, 256), (192, 11008, 1024), (270, 4112, 1152), (288, 11024, 256)])
+@pytest.mark.parametrize("qtype", ALL, ids=NAMES.values())
+def test_gated_mlp_in_row_tiles_of_three_blocks(qtype, m, n, k):
+    test_gated_mlp_tiles(qtype, m, n, k)
+
+
 @pytest.mark.parametrize("m,n,k", [(400, 16400, 256), (600, 11008, 128), (576, 11008, 256), (577, 11008, 256)])
 @pytest.mark.parametrize("qtype", ALL, ids=NAMES.values())
 def test_gated_mlp_tiles_around_a_second_round(qtype, m, n, k):
