@@ -40,7 +40,7 @@ int launch_gemm_ring(const void *x, const void *w, const void *bias, void *y, in
 int launch_gemm(const void *x, const void *w, const void *bias, void *y, int qtype, int layout, int act_dtype, int M, int N, int K,
                 void *workspace, size_t workspace_bytes, int want_splits, hipStream_t st);
 int launch_gemm_narrow(const void *x, const void *w, const void *bias, void *y, int qtype, int act_dtype, int M, int N, int K, hipStream_t st);
-size_t gemm_rows_workspace_bytes(int M, int N, int K, size_t max_bytes);
+size_t gemm_rows_workspace_bytes(int qtype, int act_dtype, int M, int N, int K, size_t max_bytes);
 int launch_gemm_rows(const void *x, const void *w, const void *bias, void *y, int qtype, int act_dtype, int M, int N, int K,
                      void *workspace, size_t workspace_bytes, hipStream_t st);
 bool gemm_back_applies(int qtype, int M, int N, int K);
@@ -422,7 +422,7 @@ size_t lowbit_linear_workspace_bytes(int qtype, int layout, int dtype, int64_t M
     if (!qk_size(qtype) || N <= 0 || K <= 0 || M > 0x7fffffff || N > 0x7fffffff || K > 0x7fffffff) return 0;
     if (gemv_wide_applies(qtype, layout, dtype, (int)M, (int)N, (int)K)) return 0;       // one pass, as forward_any chooses
     if (layout != LOWBIT_LAYOUT_GGML) return workspace_for(qtype, layout, M, N, K, max_bytes, true);
-    return gemm_rows_workspace_bytes((int)M, (int)N, (int)K, max_bytes);
+    return gemm_rows_workspace_bytes(qtype, dtype, (int)M, (int)N, (int)K, max_bytes);
 }
 
 int lowbit_linear(const void *x, const void *w, const void *bias, void *y, int qtype, int layout, int dtype, int64_t M,

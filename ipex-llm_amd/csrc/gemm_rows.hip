@@ -136,7 +136,7 @@ template <int QT> constexpr int rows32_unit(int j, int s) {
 }
 template <int QT> constexpr int rows32_lane() { return Fmt<QT>::BITS == 8 || QT == QT_NF4 ? 2 : 1; }
 
-// MB: 32-row blocks of x per workgroup.  blockIdx.y: the K split, whose partial sums go to ws in register order.
+// MB: 32-row blocks of x per workgroup, 1 .. 5.  blockIdx.y: the K split, whose partial sums go to ws in register order.
 template <int QT, typename AT, int MB>
 __global__ __launch_bounds__(256, 2) void gemm_rows_kernel(const AT *__restrict__ x, const uint8_t *__restrict__ w,
                                                            const AT *__restrict__ bias, AT *__restrict__ y, int M, int N, int K,
@@ -329,7 +329,7 @@ __global__ __launch_bounds__(256, 2) void gemm_rows_kernel(const AT *__restrict_
     }
     if (n >= N) return;
     const float bv = bias ? (float)bias[n] : 0.0f;
-    uint64_t again = 0;                                       // results that are not finite, see dot_fp32
+    uint64_t again[2] = {0, 0};                               // results that are not finite, see dot_fp32: of blocks 0 .. 3, and 4
 #pragma unroll
     for (int mb = 0; mb < MB; mb++)
 #pragma unroll
@@ -337,12 +337,15 @@ __global__ __launch_bounds__(256, 2) void gemm_rows_kernel(const AT *__restrict_
             const int m = m0 + mb * 32 + i / 4 * 8 + c * 4 + i % 4;
             if (m < M) {
                 y[(int64_t)m * N + n] = to_at<AT>(acc[mb][i] + bv);
-                again |= __builtin_isfinite(acc[mb][i]) ? 0ull : 1ull << (mb * 16 + i);
+                again[mb / 4] |= __builtin_isfinite(acc[mb][i]) ? 0ull : 1ull << (mb % 4 * 16 + i);
             }
         }
-    for (; again; again &= again - 1) {
-        const int bit = __builtin_ctzll(again), m = m0 + bit / 4 * 8 + c * 4 + bit % 4;
+    while (again[0] | again[1]) {
+        const int high = again[0] == 0, bit = __builtin_ctzll(high ? again[1] : again[0]);
+        const int m = m0 + high * 128 + bit / 4 * 8 + c * 4 + bit % 4;
         y[(int64_t)m * N + n] = to_at<AT>(dot_fp32<QT, true>(x + (int64_t)m * K, w, n, K) + bv);
+        if (high) again[1] &= again[1] - 1;
+        else again[0] &= again[0] - 1;
     }
 }
 
@@ -375,23 +378,17 @@ __global__ __launch_bounds__(256) void gemm_rows_reduce_kernel(const f32x4 *__re
 struct RowsPlan {
     int mb, tiles, steps, splits;
     size_t ws_bytes;
+    double cost;                  // in steps of one row block, two workgroups per CU
 };
-// Rows of x per workgroup: 128 where that pads M by little more than 64 would, fewer for small batches and where 128 leave
-// CUs idle, K too short to be split for them (200 rows on [1001 x 1088] 13.8 -> 12.1 us in sym_int4, 19.0 -> 15.4 in nf4; 128
-// rows on [4001 x 2112] 17.4 -> 14.9 and 22.6 -> 19.8; with both forms at two workgroups per CU 64 rows lose, 256 rows on
-// [30003 x 4096] 92 -> 124).  K splits: until the workgroups are about two per CU (the kernel's occupancy), of at
-// least four steps each.
-static RowsPlan rows_plan(int M, int N, int K, size_t ws_bytes) {
+// With row tiles of 32 * mb rows.  K splits: until the workgroups are about two per CU (the kernel's occupancy), of at least four
+// steps each.  cost: a step reckons its weights as two row blocks, a workgroup that has a CU to itself takes 0.7 of the time, a split
+// costs 2 and 5 per round of fp32 tiles.
+static RowsPlan rows_plan_of(int mb, int M, int N, int K, size_t ws_bytes) {
     RowsPlan p;
-    const int pad64 = (M + 63) / 64 * 64, pad128 = (M + 127) / 128 * 128;
-    p.mb = M <= 32 ? 1 : M <= 64 || pad128 * 8 > pad64 * 9 ? 2 : 4;
-    p.tiles = ((M + 32 * p.mb - 1) / (32 * p.mb)) * ((N + RG_N - 1) / RG_N);
+    p.mb = mb;
+    p.tiles = ((M + 32 * mb - 1) / (32 * mb)) * ((N + RG_N - 1) / RG_N);
     const int G = (K + TILE_COLS - 1) / TILE_COLS;
-    if (p.mb == 4 && (int64_t)p.tiles * (G / 4 > 1 ? G / 4 : 1) <= 256) {
-        p.mb = 2;
-        p.tiles = ((M + 63) / 64) * ((N + RG_N - 1) / RG_N);
-    }
-    const size_t per_split = (size_t)p.tiles * 32 * p.mb * RG_N * sizeof(float);
+    const size_t per_split = (size_t)p.tiles * 32 * mb * RG_N * sizeof(float);
     int s = 512 / p.tiles;
     s = s > G / 4 ? G / 4 : s;
     s = s > 16 ? 16 : s;
@@ -400,10 +397,38 @@ static RowsPlan rows_plan(int M, int N, int K, size_t ws_bytes) {
     p.steps = (G + s - 1) / s;
     p.splits = (G + p.steps - 1) / p.steps;
     p.ws_bytes = p.splits > 1 ? p.splits * per_split : 0;
+    const int64_t wgs = (int64_t)p.tiles * p.splits, per_cu = (wgs + 255) / 256;
+    p.cost = p.steps * (mb + 2.0) * ((double)(per_cu / 2) + (per_cu % 2 ? 0.7 : 0.0)) + (p.splits > 1 ? 2.0 + 5.0 * (double)wgs * mb / 512 : 0.0);
+    return p;
+}
+// Row tiles of 128 where they pad M by little more than 64 would, fewer for small batches and where 128 leave
+// CUs idle, K too short to be split for them (200 rows on [1001 x 1088] 13.8 -> 12.1 us in sym_int4, 19.0 -> 15.4 in nf4; 128
+// rows on [4001 x 2112] 17.4 -> 14.9 and 22.6 -> 19.8; with both forms at two workgroups per CU 64 rows lose, 256 rows on
+// [30003 x 4096] 92 -> 124).  Tiles of 96 or 160 rows where their estimate is 8 % shorter: 80 rows on [9001 x 4096] in
+// asym_int4 34.4 -> 28.3 us, 129 on [17563 x 3968] 78.5 -> 69.2 and in sym_int8 77.2 -> 53.5, 310 on [4677 x 4096] in sym_int4
+// 36.8 -> 31.6; 1.025 times as fast over 330 random sizes, one of them slower by more than 4 % (143 rows on [5823 x 9216] in
+// fp8_e4m3, 9 %).
+static RowsPlan rows_plan(int qtype, int act_dtype, int M, int N, int K, size_t ws_bytes) {
+    const int pad64 = (M + 63) / 64 * 64, pad128 = (M + 127) / 128 * 128;
+    RowsPlan p = rows_plan_of(M <= 32 ? 1 : M <= 64 || pad128 * 8 > pad64 * 9 ? 2 : 4, M, N, K, ws_bytes);
+    const int G = (K + TILE_COLS - 1) / TILE_COLS;
+    if (p.mb == 4 && (int64_t)p.tiles * (G / 4 > 1 ? G / 4 : 1) <= 256) return rows_plan_of(2, M, N, K, ws_bytes);
+    if (M <= 32) return p;
+    double best = 0.92 * p.cost;
+    for (int mb = 3; mb <= 5; mb += 2) {
+        if (mb == 5 && qtype == QT_NF4 && act_dtype == DT_BF16) continue;    // (nf4's three bf16 parts would spill)
+        const RowsPlan other = rows_plan_of(mb, M, N, K, ws_bytes);
+        if (other.cost < best) {
+            p = other;
+            best = other.cost;
+        }
+    }
     return p;
 }
 
-size_t gemm_rows_workspace_bytes(int M, int N, int K, size_t max_bytes) { return rows_plan(M, N, K, max_bytes).ws_bytes; }
+size_t gemm_rows_workspace_bytes(int qtype, int act_dtype, int M, int N, int K, size_t max_bytes) {
+    return rows_plan(qtype, act_dtype, M, N, K, max_bytes).ws_bytes;
+}
 
 template <int QT, typename AT, int MB>
 static void launch_rows_m(const void *x, const void *w, const void *bias, void *y, int M, int N, int K, const RowsPlan &p, float *ws,
@@ -422,7 +447,9 @@ static int launch_rows_t(const void *x, const void *w, const void *bias, void *y
                          hipStream_t st) {
     if (p.mb == 1) launch_rows_m<QT, AT, 1>(x, w, bias, y, M, N, K, p, ws, st);
     else if (p.mb == 2) launch_rows_m<QT, AT, 2>(x, w, bias, y, M, N, K, p, ws, st);
-    else launch_rows_m<QT, AT, 4>(x, w, bias, y, M, N, K, p, ws, st);
+    else if (p.mb == 3) launch_rows_m<QT, AT, 3>(x, w, bias, y, M, N, K, p, ws, st);
+    else if (p.mb == 4) launch_rows_m<QT, AT, 4>(x, w, bias, y, M, N, K, p, ws, st);
+    else if constexpr (QT != QT_NF4 || __is_same(AT, _Float16)) launch_rows_m<QT, AT, 5>(x, w, bias, y, M, N, K, p, ws, st);
     return 0;
 }
 
@@ -437,7 +464,7 @@ static int launch_rows_q(const void *x, const void *w, const void *bias, void *y
 int launch_gemm_rows(const void *x, const void *w, const void *bias, void *y, int qtype, int act_dtype, int M, int N, int K,
                      void *workspace, size_t workspace_bytes, hipStream_t st) {
     if (M == 0 || N == 0) return 0;
-    const RowsPlan p = rows_plan(M, N, K, workspace ? workspace_bytes : 0);
+    const RowsPlan p = rows_plan(qtype, act_dtype, M, N, K, workspace ? workspace_bytes : 0);
     if (K >= (1 << 23))                                      // 32-bit offsets within a tile of x: the streaming kernel has 64
         return launch_gemv(x, w, bias, y, qtype, LAYOUT_GGML, act_dtype, M, N, K, 0, st);
     if ((int64_t)((M + 15) / 16) * ((N + RG_N - 1) / RG_N) > 0x7ffffff) return -3;

@@ -68,3 +68,19 @@ def test_tiles_of_128_rows(qtype, dtype, m, n, k, splits):
             assert ((got - want - bias).abs() <= bound)[finite].all()
             assert (got.isnan() == want.isnan()).all() and (got == want)[want.isinf()].all()
             assert finite.all() != odd
+
+
+@pytest.mark.parametrize("qtype", ALL)
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("m,n,k", [(65, 9001, 2112), (96, 33001, 576), (180, 12001, 704), (129, 9001, 4160), (159, 9011, 4288)])
+def test_tiles_of_96_and_160_rows(qtype, dtype, m, n, k):
+    """Tiles of three and five 32-row blocks, with and without K splits; infinities in the last block's rows."""
+    if qtype in (FP8, 10):
+        k = (k + 127) // 128 * 128 if qtype == FP8 else (k + 63) // 64 * 64
+    _check(qtype, dtype, GGML, m, n, k, m % 2 == 0, 1300 * m + n)
+    blob, x = dev_quantize(weights(m, (37, k)), qtype, GGML), acts(m, m, k, dtype).cuda()
+    x[m - 1, k - 1], x[m - 2, 3] = float("inf"), -float("inf")
+    y = torch.empty((m, 37), dtype=dtype, device="cuda")
+    ggml.lowbit_linear(x.data_ptr(), blob.data_ptr(), None, y.data_ptr(), qtype, GGML, DT[dtype], m, 37, k, None, 0, stream())
+    want = x.double() @ dev_dequantize(blob, qtype, 37, k, GGML, torch.float32).double().t()
+    assert (classes(y.float().cpu().numpy()) == classes(want.cpu().numpy())).all()
