@@ -3,11 +3,12 @@
 //
 // The reference loops over the experts in Python (python/llm/src/ipex_llm/transformers/models/qwen2_moe.py:375-430: a
 // `where`, two index selects and an index_add per expert); its closed decode kernel takes one token
-// (models/deepseek.py:290-315).  Three small kernels stand around the products of gemm_grouped.hip:
-//   route    the stable counting sort of the pairs, in one workgroup
-//   gather   the rows of x in that order
+// (models/deepseek.py:290-315).  Two small kernels stand around the products of gemm_grouped.hip:
+//   sort     the stable counting sort of the pairs and the rows of x in that order (more than 4096 pairs: two launches, the
+//            sort in one workgroup)
 //   combine  out[t] = sum_j weight[t, j] * y[position of pair (t, j)], in fp32, rounded once
-// They are latency, not bandwidth: 1024 pairs over 8 experts with rows of 4096 take 6.1 + 6.3 + 5.4 us.  (The same steps
+// They are latency, not bandwidth: 1024 pairs over 8 experts with rows of 4096 take 5.4 us to combine, and took 6.1 + 6.3 to sort and
+// gather in two launches.  (The same steps
 // as torch operators - argsort, bincount, cumsum, index, mul, index_add - were 17 launches and 105 us, with bincount
 // waiting for the GPU in the middle of them.)
 //
@@ -106,6 +107,51 @@ __global__ __launch_bounds__(256) void moe_gather_kernel(const u32x4 *__restrict
     for (int c = threadIdx.x; c < chunks; c += 256) to[c] = from[c];
 }
 
+// Both at once for up to MOE_SORT_PAIRS pairs: workgroup p counts the pairs that come before pair p - those of lower experts, and the
+// earlier ones of its own - and copies its row of x there; workgroup pairs + e writes offsets[e].  pairs^2 ids come out of L2, which
+// costs less than a second launch that waits for a single workgroup's sort (39 pairs over 5 experts 3.3 + 3.4 us in a kernel
+// trace, 472 over 10 4.4 + 3.9, 1024 over 8 6.4 + 6.1).  Whole experts: 118 tokens, four of 10 of [1408 x 1664], 46.2 -> 40.5 us, 600,
+// four of 60 of [768 x 1024], 81.2 -> 69.4.
+constexpr int MOE_SORT_PAIRS = 4096;
+__global__ __launch_bounds__(256) void moe_sort_gather_kernel(const int64_t *__restrict__ ids, const u32x4 *__restrict__ x, int pairs,
+                                                              int n_exp, int32_t *__restrict__ offsets, int32_t *__restrict__ pos,
+                                                              u32x4 *__restrict__ xs, int top_k, int chunks) {
+    __shared__ int32_t part[4];
+    const int b = blockIdx.x, t = threadIdx.x;
+    const bool is_pair = b < pairs;
+    constexpr int HELD = 2;                              // 16-byte pieces of the row on their way while the pairs are counted
+    const u32x4 *const from = x + (int64_t)(is_pair ? b / top_k : 0) * chunks;
+    u32x4 held[HELD] = {};
+#pragma unroll
+    for (int i = 0; i < HELD; i++)
+        if (is_pair && t + i * 256 < chunks) held[i] = from[t + i * 256];
+    const int64_t own = is_pair ? ids[b] : b - pairs;
+    int before = 0;
+    for (int j0 = t; j0 - t < pairs; j0 += 2048) {
+        int64_t e[8];
+#pragma unroll
+        for (int i = 0; i < 8; i++) e[i] = j0 + i * 256 < pairs ? ids[j0 + i * 256] : -1;
+#pragma unroll
+        for (int i = 0; i < 8; i++)
+            before += __popcll(__ballot(e[i] >= 0 && e[i] < n_exp && (e[i] < own || (is_pair && e[i] == own && j0 + i * 256 < b))));
+    }
+    if ((t & 63) == 0) part[t >> 6] = before;
+    __syncthreads();
+    before = part[0] + part[1] + part[2] + part[3];
+    if (!is_pair) {
+        if (t == 0) offsets[own] = before;
+        return;
+    }
+    const bool valid = own >= 0 && own < n_exp;
+    if (t == 0) pos[b] = valid ? before : -1;
+    if (!valid) return;                                  // pairs without an expert have no row
+    u32x4 *const to = xs + (int64_t)before * chunks;
+#pragma unroll
+    for (int i = 0; i < HELD; i++)
+        if (t + i * 256 < chunks) to[t + i * 256] = held[i];
+    for (int c = t + HELD * 256; c < chunks; c += 256) to[c] = from[c];
+}
+
 // Eight columns of one token per lane.
 template <typename AT, typename WT>
 __global__ __launch_bounds__(256) void moe_combine_kernel(const AT *__restrict__ y, const int32_t *__restrict__ pos,
@@ -192,10 +238,15 @@ int launch_experts(const void *x, const int64_t *ids, const void *weight, int w_
     int32_t *const offsets = (int32_t *)(ws + at.offsets), *const order = (int32_t *)(ws + at.order), *const pos = (int32_t *)(ws + at.pos);
     void *const xs = ws + at.xs, *const y = ws + at.y;
     const int waves = n_exp <= 512 ? 16 : 2;          // at most 48 KiB of counters
-    hipLaunchKernelGGL(moe_route_kernel, dim3(1), dim3(64 * waves), (size_t)n_exp * (waves + 1) * sizeof(int32_t), st, ids, pairs, n_exp,
-                       offsets, order, pos);
-    hipLaunchKernelGGL(moe_gather_kernel, dim3(pairs), dim3(256), 0, st, (const u32x4 *)x, order, offsets + n_exp, (u32x4 *)xs, top_k,
-                       hidden / 8);
+    if (pairs <= MOE_SORT_PAIRS && n_exp <= 512) {
+        hipLaunchKernelGGL(moe_sort_gather_kernel, dim3(pairs + n_exp + 1), dim3(256), 0, st, ids, (const u32x4 *)x, pairs, n_exp, offsets,
+                           pos, (u32x4 *)xs, top_k, hidden / 8);
+    } else {
+        hipLaunchKernelGGL(moe_route_kernel, dim3(1), dim3(64 * waves), (size_t)n_exp * (waves + 1) * sizeof(int32_t), st, ids, pairs, n_exp,
+                           offsets, order, pos);
+        hipLaunchKernelGGL(moe_gather_kernel, dim3(pairs), dim3(256), 0, st, (const u32x4 *)x, order, offsets + n_exp, (u32x4 *)xs, top_k,
+                           hidden / 8);
+    }
     if (int rc = launch_grouped_gemm(xs, gates, ups, h, offsets, n_exp, pairs, qtype, act_dtype, inter, hidden, act, nullptr, 0, st))
         return rc;
     if (int rc = launch_grouped_gemm(h, downs, nullptr, y, offsets, n_exp, pairs, qtype, act_dtype, hidden, inter, 0, ws + at.split,

@@ -64,6 +64,21 @@ def test_experts_equal_the_loop_over_their_layers(qname, dtype, tokens, top_k, n
         assert (again.float() - want.float()).abs().max() <= tol * want.float().abs().max()
 
 
+@pytest.mark.parametrize("tokens,top_k,n_exp,hidden", [(85, 3, 8, 128), (86, 3, 8, 2048), (1024, 4, 16, 256), (1025, 4, 16, 256), (683, 3, 512, 128),
+                                                       (9, 2, 4, 4224)])
+def test_pairs_around_the_rounds_of_their_counting(tokens, top_k, n_exp, hidden):
+    """255 and 258 pairs, 4096 and beyond (the two launches), 2049, 512 experts; rows of 16 pieces up to more than the 512 held; two
+    pairs without an expert."""
+    torch.manual_seed(tokens)
+    block = _block(n_exp, hidden, 128, Q["sym_int4"])
+    x = torch.randn(tokens, hidden, device="cuda").half()
+    weight, index = torch.topk(torch.softmax(torch.randn(tokens, n_exp, device="cuda"), -1), top_k, dim=-1)
+    index[0, 0], index[tokens - 1, top_k - 1] = -1, n_exp
+    got = block(x, index, weight.half())
+    weight[0, 0], index[0, 0], weight[tokens - 1, top_k - 1], index[tokens - 1, top_k - 1] = 0, 0, 0, 0
+    _close(got, block._loop(x, index, weight.half()))
+
+
 def test_experts_follow_a_weight_that_was_replaced():
     torch.manual_seed(5)
     block = _block(4, 128, 256, Q["sym_int4"])
