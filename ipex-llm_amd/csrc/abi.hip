@@ -50,6 +50,7 @@ int launch_gemm_back(const void *g, const void *w, void *gx, int qtype, int act_
 double narrow_time_us(int M, int N, int K, int qtype, bool linear);
 int gemm_splits(int M, int N, int K, size_t ws_bytes, int qtype);
 double gemm_time_us(int M, int N, int K, int splits, int qtype);
+bool gemm_prefers_tall(int qtype, int act_dtype, int M, int N, int K);
 int launch_grouped_gemm(const void *x, const void *const *w, const void *const *w_up, void *y, const int32_t *offsets,
                         int n_groups, int total_rows, int qtype, int act_dtype, int N, int K, int act, void *workspace,
                         size_t workspace_bytes, hipStream_t st);
@@ -285,10 +286,11 @@ static double gemv_time_us(int qtype, int64_t M, int64_t N, int64_t K) {
 
 // which kernel, and for PLAN_GEMM_SPLIT into how many K splits
 static int plan_forward(int qtype, int layout, int64_t M, int64_t N, int64_t K, bool have_ws, size_t workspace_bytes,
-                        bool y_aligned8, int *splits_out, bool linear = false) {
+                        bool y_aligned8, int *splits_out, bool linear = false, int act_dtype = LOWBIT_DT_F16) {
     if (splits_out) *splits_out = 1;
     if (M <= 16 || layout != LOWBIT_LAYOUT_TILED || !y_aligned8) return PLAN_GEMV;            // the MFMA kernels store 8 bytes and more
     if (M > 0x7fffffff || N > 0x7fffffff || K > 0x7fffffff || K < 128) return PLAN_GEMM;     // reports the error
+    if (linear && gemm_prefers_tall(qtype, act_dtype, (int)M, (int)N, (int)K)) return PLAN_GEMM;
     const int splits = have_ws ? gemm_splits((int)M, (int)N, (int)K, workspace_bytes, qtype) : 1;
     double best_t = gemm_time_us((int)M, (int)N, (int)K, splits, qtype);
     int best = splits > 1 ? PLAN_GEMM_SPLIT : PLAN_GEMM;
@@ -330,11 +332,11 @@ size_t lowbit_workspace_bytes(int64_t M, int64_t N, int64_t K) {
 
 // What lowbit_forward_ws will use of a workspace of at most max_bytes for this format and shape: the bytes of the
 // plan it then picks (0 when that plan leaves no partial tiles).
-static size_t workspace_for(int qtype, int layout, int64_t M, int64_t N, int64_t K, size_t max_bytes, bool linear) {
+static size_t workspace_for(int qtype, int layout, int64_t M, int64_t N, int64_t K, size_t max_bytes, bool linear, int act_dtype = LOWBIT_DT_F16) {
     if (!qk_size(qtype) || M <= 0 || N <= 0 || K <= 0 || M > 0x7fffffff || N > 0x7fffffff || K > 0x7fffffff) return 0;
     int splits = 1;
     if (max_bytes < 16) return 0;
-    switch (plan_forward(qtype, layout, M, N, K, true, max_bytes, true, &splits, linear)) {
+    switch (plan_forward(qtype, layout, M, N, K, true, max_bytes, true, &splits, linear, act_dtype)) {
     case PLAN_RING: {
         // (a run that cuts no tile needs no bytes, but the plan is only made for a caller that brings a workspace)
         const size_t need = ring_workspace_bytes((int)M, (int)N, (int)K, 0);
@@ -369,7 +371,7 @@ static int forward_any(const char *what, const void *x, const void *w, const voi
     hipStream_t st = (hipStream_t)stream;
     int splits = 1, rc = 0;
     const int plan = linear && gemv_wide_applies(qtype, layout, act_dtype, m, n, k) ? PLAN_GEMV
-        : plan_forward(qtype, layout, M, N, K, workspace != nullptr, workspace_bytes, !(((uintptr_t)y | (uintptr_t)bias) & 7), &splits, linear);
+        : plan_forward(qtype, layout, M, N, K, workspace != nullptr, workspace_bytes, !(((uintptr_t)y | (uintptr_t)bias) & 7), &splits, linear, act_dtype);
     // (a y off the 8-byte boundaries keeps the streaming kernel's passes, and so its bits, at the entry points that say so)
     if (plan == PLAN_GEMV && (linear || !(((uintptr_t)y) & 7))) {
         rc = launch_gemv_wide(x, w, bias, y, qtype, layout, act_dtype, m, n, k, st);
@@ -421,7 +423,7 @@ size_t lowbit_linear_workspace_bytes(int qtype, int layout, int dtype, int64_t M
     if (dtype == LOWBIT_DT_F32 || M <= 16) return 0;     // one pass over the weights, or one per 32 rows
     if (!qk_size(qtype) || N <= 0 || K <= 0 || M > 0x7fffffff || N > 0x7fffffff || K > 0x7fffffff) return 0;
     if (gemv_wide_applies(qtype, layout, dtype, (int)M, (int)N, (int)K)) return 0;       // one pass, as forward_any chooses
-    if (layout != LOWBIT_LAYOUT_GGML) return workspace_for(qtype, layout, M, N, K, max_bytes, true);
+    if (layout != LOWBIT_LAYOUT_GGML) return workspace_for(qtype, layout, M, N, K, max_bytes, true, dtype);
     return gemm_rows_workspace_bytes(qtype, dtype, (int)M, (int)N, (int)K, max_bytes);
 }
 

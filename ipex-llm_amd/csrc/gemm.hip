@@ -114,26 +114,47 @@ int gemm_splits(int M, int N, int K, size_t ws_bytes, int qtype) {
     return best;
 }
 
-// How many column tiles (256 weight rows each) the tall form takes, from the left: whole rounds of one
-// 256 x 256 tile per CU, so that no CU sits idle while another still works on a second tall tile; the 128-row
-// form covers the columns that are left.  0 = the tall form is not used: a last row tile that is less than half full
-// (the 128-row form computes 128 rows less), too few tiles to fill the machine once, K too long for 24-bit row
-// offsets - or columns left over that cost more than the tall columns gain.  Measured on MI355X: a machine full of tall
-// tiles runs 4-7 % (sym_int4) to 10 % (nf4) faster than the 128-row form with two workgroups per CU ([28672 x 8192] at
-// M = 1000, bf16: sym_int4 440 -> 429, asym_int4 442 -> 418, sym_int8 456 -> 423, fp8_e4m3 420 -> 395 us), which the
-// idle CUs of a thin remainder eat up again.
+// How many column tiles (256 weight rows each) the tall form takes, from the left; the 128-row form covers the columns that are
+// left.  0 = the tall form is not used: a last row tile that is less than half full (the 128-row form computes 128 rows less), K too
+// long for 24-bit row offsets, or one of the rules below.  A launch of tall tiles takes 3.3 us per K step and whole round of one
+// tile per CU and 1.75 + 1.3 f for a round of which a part f is filled (fewer CUs at work run faster), 8 us per round: fitted to 500
+// random sizes, M = 140 .. 2048, five formats, both types, 3 % rms in each.  Hence
+//   - all columns in up to one round, from 0.52 of it on and where 128-row tiles would be more than one per CU ([12288 x 4096] at M =
+//     700 in nf4 118 -> 83 us, at M = 1000 in bf16 sym_int4 114 -> 95, in fp16 100 -> 95; 0.4 to 0.5 of a round 1.2 times the time);
+//   - all columns where the last round is whole or half full at least (0.65 of it in fp16 and 4-bit integers, which cost the 128-row
+//     form least), from 8 steps on ([28672 x 8192] at M = 1000, 1.75 rounds: nf4 431 -> 403 us, bf16 sym_int4 435 -> 393, fp16 402 ->
+//     386, fp8_e4m3 404 -> 385);
+//   - else whole rounds, so that no CU sits idle while another works on one more tall tile, where the rest costs less than they gain:
+//     fp8_e4m3 and 4-bit integers in bf16 from 16 steps on ([12288 x 4096] at M = 1500 in bf16 sym_int4 168 -> 157; fewer steps lose
+//     up to 16 %).  None of the 500 sizes is slower by more than 2 % with these three than without, and the 180 that they change are
+//     1.07 times as fast;
 //   - sym_int8 and nf4 pay most per weight for the dequantization, which the tall form does half as often: the estimate
 //     of gemm_time_us for both ways, 0.9 of a full 128-row round for a tall one, nf4's remainder, in narrow tiles, 1.15
 //     (sym_int8 [28672 x 8192] at M = 700 347 us without tall tiles and 332 with; nf4 there 404 and 328, [11008 x 4096] at
-//     M = 2047 207 and 171; [11008 x 4096] at M = 1300, 258 tall tiles, one column left over: 116 us without, 151 with).
+//     M = 2047 207 and 171; [11008 x 4096] at M = 1300, 258 tall tiles, one column left over: 116 us without, 151 with);
 //   - the others with 1.5 workgroups per CU left over (at M = 2048 on [11008 x 4096] sym_int4 +1 %, fp8_e4m3 -3 %).
 static double steps_time(int64_t wgs) {                  // a 128-column step of the 128-row form, see gemm_time_us
     if (wgs > 512) return 2.68 * (double)((wgs + 255) / 256) / 2.0;
     return wgs > 256 ? 2.12 + 0.56 * (double)(wgs - 256) / 256.0 : 1.21 + (wgs > 128 ? 0.29 * (double)(wgs - 128) / 128.0 : 0.0);
 }
-static int tall_columns(int M, int N, int K, int n_cus, int qtype) {
+static bool tall_fits(int M, int K) {
     const int rest = M % GM_TALL;
-    if (M < 2 * GM_TALL || (rest && rest <= GM) || M >= (1 << 24) || K >= (1 << 23)) return 0;
+    return M >= GM_TALL && !(rest && rest <= GM) && M < (1 << 24) && K < (1 << 23);
+}
+// by the first three rules, 0: none of them
+static int tall_by_rounds(int M, int N, int K, int n_cus, int qtype, bool f16) {
+    if (!tall_fits(M, K)) return 0;
+    const int tiles_m = (M + GM_TALL - 1) / GM_TALL, tiles_n = (N + GN - 1) / GN;
+    const int64_t tiles = (int64_t)tiles_m * tiles_n, small = (int64_t)((M + GM - 1) / GM) * tiles_n;
+    if (tiles <= n_cus) return small > n_cus && tiles * 100 >= (int64_t)n_cus * 52 ? tiles_n : 0;
+    const bool int4 = qtype == QT_SYM_INT4 || qtype == QT_ASYM_INT4;
+    const int64_t last = tiles % n_cus;
+    if (last == 0 || (last * 100 >= (int64_t)n_cus * (int4 && f16 ? 65 : 50) && K >= 8 * TILE_COLS)) return tiles_n;
+    return ((int4 && !f16) || qtype == QT_FP8_E4M3) && K >= 16 * TILE_COLS ? (int)(tiles / n_cus * n_cus / tiles_m) : 0;
+}
+static int tall_columns(int M, int N, int K, int n_cus, int qtype, bool f16) {
+    if (const int cols = tall_by_rounds(M, N, K, n_cus, qtype, f16)) return cols;
+    if (M < 2 * GM_TALL || !tall_fits(M, K)) return 0;
     const int tiles_m = (M + GM_TALL - 1) / GM_TALL, tiles_n = (N + GN - 1) / GN;
     const int64_t small_m = (M + GM - 1) / GM;           // row tiles of the 128-row form
     const int rounds = (int)((int64_t)tiles_m * tiles_n / n_cus);
@@ -144,6 +165,21 @@ static int tall_columns(int M, int N, int K, int n_cus, int qtype) {
     if (qtype == QT_SYM_INT8 || qtype == QT_NF4)
         return rounds * 0.9 * 2.68 + steps_time(left) * (qtype == QT_NF4 ? 1.15 : 1.0) < 0.98 * steps_time(tiles_n * small_m) ? cols : 0;
     return 2 * left >= 3 * n_cus ? cols : 0;
+}
+
+static int gemm_cus() {
+    static const int n_cus = [] {
+        int dev = 0, n = 0;
+        if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
+            n = 256;
+        return n > 0 ? n : 256;
+    }();
+    return n_cus;
+}
+
+// Whether lowbit_linear takes tall tiles whatever the estimates of the other kernels say.
+bool gemm_prefers_tall(int qtype, int act_dtype, int M, int N, int K) {
+    return tall_by_rounds(M, N, K, gemm_cus(), qtype, act_dtype == DT_F16) > 0;
 }
 
 // How many tiles at the end of each XCD's share of a 128-row launch go out as two half tiles: all of them or none.
@@ -157,17 +193,12 @@ static int launch_gemm_t(const void *x, const void *w, const void *bias, void *y
     if (splits <= 1) ws = nullptr;
     const int G = K / TILE_COLS;
     const int tiles_n_all = (N + GN - 1) / GN;
-    static const int n_cus = [] {
-        int dev = 0, n = 0;
-        if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
-            n = 256;
-        return n > 0 ? n : 256;
-    }();
+    const int n_cus = gemm_cus();
     // tall form on the left columns, 128-row form on the rest (both in the same stream, the second starts when
     // the tall tiles, which all take the same time, are done)
     GroupArgs ga{};
     ga.bias = bias;
-    const int tall = ws ? 0 : tall_columns(M, N, K, n_cus, QT);
+    const int tall = ws ? 0 : tall_columns(M, N, K, n_cus, QT, __is_same(AT, _Float16));
     if (tall > 0) {
         const int tiles_m = (M + GM_TALL - 1) / GM_TALL;
         ga.tile_rows = GM_TALL;

@@ -33,6 +33,14 @@ def test_last_row_tile(qtype, m, n, k, dtype):
 
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16], ids=["f16", "bf16"])
+@pytest.mark.parametrize("m,n,k", [(385, 17136, 256), (700, 11520, 384), (512, 32752, 128), (897, 24832, 1024), (1000, 20496, 2048)])
+@pytest.mark.parametrize("qtype", ALL, ids=NAMES.values())
+def test_rounds_that_are_partly_filled(qtype, m, n, k, dtype):
+    """All columns in tall tiles: half a round and more of them, a last round that is half full; and whole rounds with a rest."""
+    check(qtype, m, n, k, dtype, ggml.lowbit_gemm)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16], ids=["f16", "bf16"])
 @pytest.mark.parametrize("m,n,k", [(1, 16, 128), (32, 144, 256), (33, 128, 384), (64, 272, 640), (65, 1040, 512), (200, 4096, 1152)])
 def test_narrow_nf4(m, n, k, dtype):
     """Row blocks 1, 2 and 4 of the narrow tile, whose nf4 lookups are in registers."""
