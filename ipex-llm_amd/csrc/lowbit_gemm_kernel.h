@@ -271,12 +271,22 @@ __global__ __launch_bounds__(64 * WAVES * KS, (DMA && MB == 4) ? 2 : 1) void gem
     // tiles are a second round for an XCD whose 32 CUs hold 64 workgroups.
     int m0, tile_n;
     const uint8_t *w_up = nullptr;
-    int row_tile = 0;
+    int row_tile = 0, split = blockIdx.y;
     if constexpr (!GROUPED) {
         const int pitch = ga.tile_rows, tiles_m = ga.row_tiles, tiles_n = tn_cnt;
         const int64_t T = (int64_t)tiles_m * tiles_n;
-        const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
-        const int first = (int)(T * xcd / 8), count = (int)(T * (xcd + 1) / 8) - first;
+        const int xcd = blockIdx.x & 7;
+        int slot = blockIdx.x >> 3, first = (int)(T * xcd / 8), count = (int)(T * (xcd + 1) / 8) - first;
+        if (ws) {
+            // K splits: the line holds every tile's splits side by side.  With an eighth of the tiles for every XCD in each
+            // split, 50 tiles in five splits - 250 workgroups - put 35 on some XCDs, whose 32 CUs then took turns (178 rows on
+            // [6288 x 14720] in bf16 sym_int4 76.0 us, with four splits 57.5).  Split by split instead, every XCD reads from all
+            // rows of the weight (284 rows on [2512 x 3968] in fp8_e4m3 22.5 us a tile's splits side by side, 26.5).
+            const int64_t U = T * gridDim.y;
+            first = (int)(U * xcd / 8);
+            count = (int)(U * (xcd + 1) / 8) - first;
+            slot += blockIdx.y * (gridDim.x >> 3);
+        }
         // A launch with fewer tiles than compute units goes out in half tiles, twice as many workgroups (the
         // launcher says how many tiles at the end of each XCD's share are cut: all of them or none).
         int idx = slot, half = -1;
@@ -288,7 +298,12 @@ __global__ __launch_bounds__(64 * WAVES * KS, (DMA && MB == 4) ? 2 : 1) void gem
             }
         }
         if (idx >= count) return;                                                    // whole workgroup leaves
-        const int line = first + idx;
+        int line = first + idx;
+        if (ws) {
+            const int tile = line / (int)gridDim.y;
+            split = line - tile * (int)gridDim.y;
+            line = tile;
+        }
         const int per_band = band_m * tiles_n;
         const int band = line / per_band, r = line - band * per_band;
         const int rows_b = tiles_m - band * band_m < band_m ? tiles_m - band * band_m : band_m;   // the last band may be short
@@ -395,10 +410,10 @@ __global__ __launch_bounds__(64 * WAVES * KS, (DMA && MB == 4) ? 2 : 1) void gem
     }
     const uint64_t xone_base = (uint64_t)(uintptr_t)x + (uint64_t)m0 * (uint64_t)K * sizeof(AT);
     constexpr int PW = 8 * MB32 / WAVES;                  // pieces of 1 KiB (8 rows of a half row) a wave fetches per K step
-    // Split-K: with a workspace the grid has a second dimension, workgroup (t, s) walks the K steps
+    // Split-K: with a workspace the grid has a second dimension, the workgroup of tile t and split s walks the K steps
     // s * k_steps .. and leaves its fp32 partial tile in ws[s]; a second kernel sums the splits.  It
     // fills the machine when the output alone has too few tiles (small M, narrow N).
-    const int kt_wg = ws ? blockIdx.y * k_steps : 0;
+    const int kt_wg = ws ? split * k_steps : 0;
     const int Gs_wg = ws ? (k_steps < G - kt_wg ? k_steps : G - kt_wg) : G;
     // KS == 2: the first group of waves walks the first half of the steps (one more where their number is odd)
     const int Gs_first = KS == 2 ? (Gs_wg + 1) / 2 : Gs_wg;
@@ -870,7 +885,7 @@ __global__ __launch_bounds__(64 * WAVES * KS, (DMA && MB == 4) ? 2 : 1) void gem
             // dense: tiles in row-major order; grouped: in the order of the launch
             const int64_t tile_id = GROUPED ? (int64_t)blockIdx.x : (int64_t)row_tile * ((N + GN - 1) / GN) + tile_n;
             const int64_t n_tiles_all = GROUPED ? (int64_t)gridDim.x : (int64_t)ga.row_tiles * ((N + GN - 1) / GN);
-            float *const wp = ws + ((((int64_t)blockIdx.y * n_tiles_all + tile_id) * WAVES + wave) * (MB32 * NB32 * 4)) * 256 + lane * 4;
+            float *const wp = ws + ((((int64_t)split * n_tiles_all + tile_id) * WAVES + wave) * (MB32 * NB32 * 4)) * 256 + lane * 4;
 #pragma unroll
             for (int mb = MB0; mb < MBC; mb++) {
 #pragma unroll

@@ -5,7 +5,7 @@ import torch
 
 import ipex_llm.ggml.model.llama.llama_cpp as ggml
 import lowbit_oracle as orc
-from gpu_util import ALL, DT, FP8, NF4, acts, dev_quantize, stream, weights
+from gpu_util import ALL, DT, FP8, NF4, acts, dev_dequantize, dev_quantize, stream, weights
 from ipex_llm.transformers.low_bit_linear import FP4Params, LowBitLinear
 
 pytestmark = pytest.mark.gpu
@@ -138,3 +138,20 @@ def test_infinities_meet_the_weights_and_not_their_codes(qtype, dtype, m, n, k):
     assert (classes(y) == classes(want)).all()
     if m > 1:
         assert (classes(want) != 0).any() and (classes(want) == 0).any()
+
+
+# tiles times splits that eighths of either do not divide: 1 tile in 16 splits, 9 in 5 to 7, 50 in 5, more than 256 workgroups
+@pytest.mark.parametrize("qtype,dtype", [(2, torch.float16), (3, torch.bfloat16), (8, torch.float16), (10, torch.bfloat16), (15, torch.bfloat16)])
+@pytest.mark.parametrize("m,n,k", [(70, 256, 8192), (300, 784, 4096), (178, 6288, 1920), (100, 2320, 2176)])
+@pytest.mark.parametrize("splits", [2, 5, 7, 16])
+def test_k_splits_over_the_xcds(qtype, dtype, m, n, k, splits):
+    blob, x = dev_quantize(weights(m, (n, k)), qtype, TILED), acts(m, m, k, dtype).cuda()
+    if k // 128 < 2 * splits:
+        splits = k // 256
+    tiles = (m + 127) // 128 * ((n + 255) // 256)
+    ws = torch.full((tiles * splits * 128 * 256 * 4 + 64,), 255, dtype=torch.uint8, device="cuda")
+    y = torch.full((m + 1, n), float("nan"), dtype=dtype, device="cuda")
+    ggml.lowbit_gemm_ws(x.data_ptr(), blob.data_ptr(), y.data_ptr(), qtype, TILED, DT[dtype], m, n, k, ws.data_ptr(), ws.numel() - 64, splits, stream())
+    want = x.double() @ dev_dequantize(blob, qtype, n, k, TILED, torch.float32).double().t()
+    assert torch.isnan(y[m]).all() and (ws[-64:] == 255).all()
+    assert ((y[:m].double() - want).abs().max() <= TOL[dtype] * want.abs().max())
