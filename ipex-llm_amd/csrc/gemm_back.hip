@@ -47,12 +47,13 @@ __global__ __launch_bounds__(512, 2) void gemm_back_kernel(const AT *__restrict_
     // Workgroups go to the XCDs in turn (id % 8): each takes a run of the tiles, the row tiles of a column tile side by side,
     // so that its L2 serves a column's weights to all of them.
     const int tiles_m = (M + BM - 1) / BM, G = K / TILE_COLS;
-    const int64_t T = (int64_t)tiles_m * G;
-    const int xcd = blockIdx.x & 7, first = (int)(T * xcd / 8), count = (int)(T * (xcd + 1) / 8) - first;
-    if ((int)(blockIdx.x >> 3) >= count) return;             // whole workgroup leaves
-    const int tile = first + (blockIdx.x >> 3), m0 = tile % tiles_m * BM, kt = tile / tiles_m;
+    // (a run of tiles and splits, a tile's side by side: with an eighth of the tiles in every split XCDs differ by up to a tile's splits)
+    const int64_t T = (int64_t)tiles_m * G, units = T * gridDim.y;
+    const int xcd = blockIdx.x & 7, unit = (int)(units * xcd / 8) + (int)((blockIdx.x >> 3) + blockIdx.y * (gridDim.x >> 3));
+    if (unit >= (int)(units * (xcd + 1) / 8)) return;        // whole workgroup leaves
+    const int tile = unit / (int)gridDim.y, split = unit - tile * (int)gridDim.y, m0 = tile % tiles_m * BM, kt = tile / tiles_m;
 
-    const int all_steps = (N + BACK_N - 1) / BACK_N, split_s0 = ws ? blockIdx.y * split_steps : 0;
+    const int all_steps = (N + BACK_N - 1) / BACK_N, split_s0 = ws ? split * split_steps : 0;
     const int steps = ws && split_steps < all_steps - split_s0 ? split_steps : all_steps - split_s0, steps_first = (steps + 1) / 2;
     const int s0 = split_s0 + (half ? steps_first : 0), S = half ? steps - steps_first : steps_first, last = S > 0 ? S - 1 : 0;
     const int row_tiles = N / TILE_ROWS;
@@ -238,7 +239,7 @@ __global__ __launch_bounds__(512, 2) void gemm_back_kernel(const AT *__restrict_
     // C layout: lane = 32 * kg + row of g, register i = column 8 * (i / 4) + 4 * kg + i % 4
     auto finish = [&](int from) __attribute__((always_inline)) {
         if (ws) {
-            f32x4 *const to = ws + (((int64_t)blockIdx.y * T + tile) * 8 + wave_wg) * (MBW * 256) + lane;
+            f32x4 *const to = ws + (((int64_t)split * T + tile) * 8 + wave_wg) * (MBW * 256) + lane;
 #pragma unroll
             for (int mb = from; mb < from + MBW; mb++)
 #pragma unroll

@@ -136,7 +136,7 @@ template <int QT> constexpr int rows32_unit(int j, int s) {
 }
 template <int QT> constexpr int rows32_lane() { return Fmt<QT>::BITS == 8 || QT == QT_NF4 ? 2 : 1; }
 
-// MB: 32-row blocks of x per workgroup, 1 .. 5.  blockIdx.y: the K split, whose partial sums go to ws in register order.
+// MB: 32-row blocks of x per workgroup, 1 .. 5.  gridDim.y: the K splits, whose partial sums go to ws in register order.
 template <int QT, typename AT, int MB>
 __global__ __launch_bounds__(256, 2) void gemm_rows_kernel(const AT *__restrict__ x, const uint8_t *__restrict__ w,
                                                            const AT *__restrict__ bias, AT *__restrict__ y, int M, int N, int K,
@@ -155,13 +155,17 @@ __global__ __launch_bounds__(256, 2) void gemm_rows_kernel(const AT *__restrict_
 
     // Workgroups go to the XCDs in turn (id % 8): each XCD takes a run of the tiles, row tile by row tile within a column
     // tile, so that its L2 serves a column's weights to all their row tiles.
-    const int tiles_m = (M + BM - 1) / BM, tiles = tiles_m * ((N + RG_N - 1) / RG_N), per_xcd = (tiles + 7) / 8;
-    const int tile = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
-    if (tile >= tiles) return;                               // whole workgroup leaves
+    // (with K splits a run of tiles and splits, a tile's side by side: an eighth of the tiles in every split leaves XCDs with up to
+    // a tile's splits more than others)
+    const int tiles_m = (M + BM - 1) / BM, tiles = tiles_m * ((N + RG_N - 1) / RG_N), xcd = blockIdx.x & 7;
+    const int64_t units = (int64_t)tiles * gridDim.y;
+    const int first = (int)(units * xcd / 8), unit = first + (int)((blockIdx.x >> 3) + blockIdx.y * (gridDim.x >> 3));
+    if (unit >= (int)(units * (xcd + 1) / 8)) return;        // whole workgroup leaves
+    const int tile = unit / (int)gridDim.y, split = unit - tile * (int)gridDim.y;
     const int m0 = tile % tiles_m * BM, n0 = tile / tiles_m * RG_N + wave * 32;
 
     const int blocks = K / F::QK, G = (K + TILE_COLS - 1) / TILE_COLS;
-    const int g0 = blockIdx.y * steps, g1 = g0 + steps < G ? g0 + steps : G;
+    const int g0 = split * steps, g1 = g0 + steps < G ? g0 + steps : G;
     const int n = n0 + r;
     gbytes wr[2];
 #pragma unroll
@@ -319,7 +323,7 @@ __global__ __launch_bounds__(256, 2) void gemm_rows_kernel(const AT *__restrict_
 
     // C layout: lane = 32 * c + column (weight row), register 4q + i = row 8q + 4c + i of x
     if (ws) {
-        f32x4 *part = (f32x4 *)ws + (((int64_t)blockIdx.y * tiles + tile) * RG_WAVES + wave) * (MB * 4 * 64) + lane;
+        f32x4 *part = (f32x4 *)ws + (((int64_t)split * tiles + tile) * RG_WAVES + wave) * (MB * 4 * 64) + lane;
 #pragma unroll
         for (int mb = 0; mb < MB; mb++)
 #pragma unroll
