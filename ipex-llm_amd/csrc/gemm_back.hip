@@ -14,8 +14,9 @@
 // registers, and goes to LDS during the step before it.  (g by LDS-DMA instead, which the compiler does not count among
 // the loads in flight, made it wait for the youngest ones and an earlier version a seventh slower.)
 //
-// What bounds it, 128 rows on [4096 x 4096] in sym_int4 (33.7 us in a kernel trace, 1.05 us a pair of steps): LDS is busy 54 % of
-// the time, the MFMA pipes 38 %, the vector units 30 %; two waves per SIMD that meet at a barrier per step overlap them badly.
+// What bounds it, 128 rows on [4096 x 4096] in sym_int4 (unsplit 33.7 us in a kernel trace, 1.05 us a pair of steps; split 16.8
+// and 4.1 for the sums): LDS is busy 54 % of the time, the MFMA pipes 38 %, the vector units 30 %; two waves per SIMD that meet
+// at a barrier per step overlap them badly.
 // Of an earlier version's 39 us the MFMAs were 2, the dequantization with its writes to LDS 12, g's way into LDS 10.  64 rows
 // by 64 columns per wave, whose operands are a fifth less LDS traffic, and the writes ahead of the MFMAs are level with this.
 // Few tiles leave CUs idle: then several workgroups share a tile's walk (back_plan).
@@ -47,7 +48,9 @@ __global__ __launch_bounds__(512, 2) void gemm_back_kernel(const AT *__restrict_
     // Workgroups go to the XCDs in turn (id % 8): each takes a run of the tiles, the row tiles of a column tile side by side,
     // so that its L2 serves a column's weights to all of them.
     const int tiles_m = (M + BM - 1) / BM, G = K / TILE_COLS;
-    // (a run of tiles and splits, a tile's side by side: with an eighth of the tiles in every split XCDs differ by up to a tile's splits)
+    // (What is dealt is tiles times splits, a tile's side by side: with an eighth of the tiles in every split the XCDs differ by up to
+    // as many workgroups as there are splits, and those above a workgroup per CU wait.  125 rows on [9104 x 6272] in sym_int8, a
+    // training step with the forward's splits dealt likewise: 89 -> 65 us.)
     const int64_t T = (int64_t)tiles_m * G, units = T * gridDim.y;
     const int xcd = blockIdx.x & 7, unit = (int)(units * xcd / 8) + (int)((blockIdx.x >> 3) + blockIdx.y * (gridDim.x >> 3));
     if (unit >= (int)(units * (xcd + 1) / 8)) return;        // whole workgroup leaves
@@ -299,9 +302,10 @@ static int64_t back_tiles(int M, int K, int rows) { return (int64_t)((M + rows -
 // types) with up to 16 splits each: 6 % rms, the plan it picks within 2 % of the best on average.  A pair of steps takes 0.78
 // (64 rows) or 1.03 (128), a launch 4.7 or 6.2, a second one that adds the splits 1.0 and 0.021 per 64 rows by 128 columns of fp32
 // sums.  Splits are charged 12 instead of that 1.0: their workspace and launch cost the host 6, and where the GPU waits for the host
-// anyway a step with them is the longer one (498 rows on [2000 x 1280] 42 -> 49, its kernel 18 -> 13).  Whole training steps against the choice without splits, us: 307 rows on [3360 x 1408] in nf4 65 -> 51, 234 on
-// [7616 x 2432] 77 -> 50, 329 on [11456 x 4224] 168 -> 128, 125 on [9104 x 6272] in sym_int8 104 -> 89; the kernels alone 1.34 times
-// as fast over those 258 sizes, 0.90 at worst.
+// anyway a step with them is the longer one (498 rows on [2000 x 1280] 42 -> 49, its kernel 18 -> 13).  Whole training steps against the choice without
+// splits, us: 307 rows on [3360 x 1408] in nf4 65 -> 51, 234 on [7616 x 2432] 77 -> 50, 329 on [11456 x 4224] 168 -> 128, 125 on
+// [9104 x 6272] in sym_int8 104 -> 89 (65 with this kernel's and the forward's splits dealt evenly to the XCDs); the kernels alone
+// 1.34 times as fast over those 258 sizes, 0.90 at worst.
 struct BackPlan {
     int rows, splits;             // rows of g per tile; workgroups that share a tile's walk along N
 };
