@@ -15,6 +15,7 @@
 //   and stores 8 contiguous bytes of y at a time.
 // FLOP per launch: 2*M*N*K; MFMA-bound (fp16 / bf16 dense peak).
 #include "lowbit_gemm_kernel.h"
+#include "lowbit_splits.h"
 
 namespace lowbit {
 
@@ -31,19 +32,16 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float *__restr
                                                             const AT *__restrict__ bias, int M, int N, int splits, int tile_rows) {
     const int tiles_n = (N + GN - 1) / GN;
     const int64_t n_tiles_all = (int64_t)((M + tile_rows - 1) / tile_rows) * tiles_n;
-    const int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x;       // (tile, wave, group, lane)
-    if (t >= n_tiles_all * 4 * (MB32 * NB32 * 4) * 64) return;
-    const int lane = (int)(t & 63);
-    const int grp = (int)((t >> 6) % (MB32 * NB32 * 4));
-    const int wave = (int)((t >> 6) / (MB32 * NB32 * 4) % 4);
-    const int64_t tile_id = (t >> 6) / (MB32 * NB32 * 4) / 4;
+    const int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x;       // (tile, wave, group, lane): a block's groups are of one wave
+    constexpr int BLOCKS = MB32 * NB32 * 4 / 4;                      // blocks of threads per wave
+    const int lane = threadIdx.x & 63, grp = (int)(blockIdx.x % BLOCKS) * 4 + (threadIdx.x >> 6);
+    const int wave = (int)(blockIdx.x / BLOCKS % 4), tile_id = (int)(blockIdx.x / (4 * BLOCKS));
     const int mb = grp / (NB32 * 4), nb = grp / 4 % NB32, q = grp % 4;
-    const int m = (int)(tile_id / tiles_n) * tile_rows + mb * 32 + (lane & 31);
-    const int n = (int)(tile_id % tiles_n) * GN + wave * GN_WAVE + nb * 32 + q * 8 + (lane >> 5) * 4;
+    const int m = tile_id / tiles_n * tile_rows + mb * 32 + (lane & 31);
+    const int n = tile_id % tiles_n * GN + wave * GN_WAVE + nb * 32 + q * 8 + (lane >> 5) * 4;
     if (mb * 32 >= tile_rows || m >= M || n >= N) return;
     const int64_t per_split = n_tiles_all * 4 * (MB32 * NB32 * 4) * 64 * 4;     // floats
-    f32x4 a = *(const f32x4 *)(ws + t * 4);
-    for (int s = 1; s < splits; s++) a += *(const f32x4 *)(ws + (int64_t)s * per_split + t * 4);
+    const f32x4 a = sum_splits((const f32x4 *)ws + t, per_split / 4, splits);
     typedef AT at4 __attribute__((ext_vector_type(4)));
     at4 o;
 #pragma unroll

@@ -21,6 +21,7 @@
 // by 64 columns per wave, whose operands are a fifth less LDS traffic, and the writes ahead of the MFMAs are level with this.
 // Few tiles leave CUs idle: then several workgroups share a tile's walk (back_plan).
 #include "lowbit_gemm.h"
+#include "lowbit_splits.h"
 
 namespace lowbit {
 
@@ -279,13 +280,11 @@ template <typename AT, int MBW>
 __global__ __launch_bounds__(256) void back_reduce_kernel(const f32x4 *__restrict__ ws, AT *__restrict__ gx, int M, int K, int64_t per_split,
                                                           int splits) {
     const int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x;           // (a split's sums are whole blocks of threads)
-    const int lane = (int)(t & 63), q = (int)(t >> 6) & 3, mb = (int)(t >> 8) % MBW;
-    const int64_t tw = (t >> 8) / MBW;
-    const int wave_wg = (int)(tw & 7), tiles_m = (M + 64 * MBW - 1) / (64 * MBW);
-    const int m = (int)((tw >> 3) % tiles_m) * (64 * MBW) + ((wave_wg >> 2) * MBW + mb) * 32 + (lane & 31);
-    const int k = (int)((tw >> 3) / tiles_m) * TILE_COLS + (wave_wg & 3) * 32 + 8 * q + 4 * (lane >> 5);
-    f32x4 a = ws[t];
-    for (int s = 1; s < splits; s++) a += ws[s * per_split + t];
+    const int lane = threadIdx.x & 63, q = threadIdx.x >> 6, mb = (int)(blockIdx.x % MBW), tw = (int)(blockIdx.x / MBW);
+    const int wave_wg = tw & 7, tiles_m = (M + 64 * MBW - 1) / (64 * MBW);
+    const int m = (tw >> 3) % tiles_m * (64 * MBW) + ((wave_wg >> 2) * MBW + mb) * 32 + (lane & 31);
+    const int k = (tw >> 3) / tiles_m * TILE_COLS + (wave_wg & 3) * 32 + 8 * q + 4 * (lane >> 5);
+    const f32x4 a = sum_splits(ws + t, per_split, splits);
     typedef AT at4 __attribute__((ext_vector_type(4)));
     at4 o;
 #pragma unroll

@@ -155,3 +155,16 @@ def test_k_splits_over_the_xcds(qtype, dtype, m, n, k, splits):
     want = x.double() @ dev_dequantize(blob, qtype, n, k, TILED, torch.float32).double().t()
     assert torch.isnan(y[m]).all() and (ws[-64:] == 255).all()
     assert ((y[:m].double() - want).abs().max() <= TOL[dtype] * want.abs().max())
+
+
+# parts that are summed in one round of loads (up to 9), in one and a rest, and in two: a part left out or added twice is a tenth of y
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("splits", [3, 4, 6, 8, 9, 10, 14, 16])
+def test_sums_of_splits(dtype, splits):
+    m, n, k, qtype = 137, 272, 256 * splits, 8
+    blob, x = dev_quantize(weights(splits, (n, k)), qtype, TILED), acts(splits, m, k, dtype).cuda()
+    ws = torch.empty(2 * 2 * 128 * 256 * 4 * splits, dtype=torch.uint8, device="cuda")
+    y = torch.empty(m, n, dtype=dtype, device="cuda")
+    ggml.lowbit_gemm_ws(x.data_ptr(), blob.data_ptr(), y.data_ptr(), qtype, TILED, DT[dtype], m, n, k, ws.data_ptr(), ws.numel(), splits, stream())
+    want = x.double() @ dev_dequantize(blob, qtype, n, k, TILED, torch.float32).double().t()
+    assert ((y.double() - want).abs().max() <= TOL[dtype] * want.abs().max())
