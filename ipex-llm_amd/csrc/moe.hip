@@ -152,7 +152,32 @@ __global__ __launch_bounds__(256) void moe_sort_gather_kernel(const int64_t *__r
     for (int c = t + HELD * 256; c < chunks; c += 256) to[c] = from[c];
 }
 
-// Eight columns of one token per lane.
+// U pairs of one token: their places and weights on their way together, then their rows; added in order.
+template <int U, typename AT, typename WT>
+__device__ inline void combine_pairs(float (&sum)[8], const AT *__restrict__ y, const int32_t *__restrict__ pos, const WT *__restrict__ weight,
+                                     int N) {
+    using V8 = typename Vec8<AT>::type;
+    int p[U];
+    float w[U];
+    V8 v[U];
+#pragma unroll
+    for (int j = 0; j < U; j++) {
+        p[j] = pos[j];
+        w[j] = (float)weight[j];
+    }
+#pragma unroll
+    for (int j = 0; j < U; j++) v[j] = *(const V8 *)(y + (int64_t)(p[j] < 0 ? 0 : p[j]) * N);    // (a pair without an expert: any row, not added)
+#pragma unroll
+    for (int j = 0; j < U; j++) {
+        if (p[j] < 0) continue;
+#pragma unroll
+        for (int i = 0; i < 8; i++) sum[i] = fmaf(w[j], (float)v[j][i], sum[i]);
+    }
+}
+
+// Eight columns of one token per lane.  Bound by latency (3.8 us in a trace at 472 pairs of 1664 columns, 1.6 MB): a pair's place, its weight and
+// its row one after the other, pair by pair, were three waits per pair; four pairs at a time are two (118 tokens, four of 10 experts
+// of [1024 x 1664] in asym_int4, the whole call 34.9 -> 33.6 us, 32 tokens, two of 13, 30.2 -> 29.0, 512 of [14336 x 4096] 498 -> 496).
 template <typename AT, typename WT>
 __global__ __launch_bounds__(256) void moe_combine_kernel(const AT *__restrict__ y, const int32_t *__restrict__ pos,
                                                           const WT *__restrict__ weight, AT *__restrict__ out, int top_k, int N) {
@@ -160,14 +185,14 @@ __global__ __launch_bounds__(256) void moe_combine_kernel(const AT *__restrict__
     const int t = blockIdx.y, n = (blockIdx.x * 256 + threadIdx.x) * 8;
     if (n >= N) return;
     float sum[8] = {};
-    for (int j = 0; j < top_k; j++) {
-        const int p = pos[t * top_k + j];
-        if (p < 0) continue;
-        const float w = (float)weight[t * top_k + j];
-        const V8 v = *(const V8 *)(y + (int64_t)p * N + n);
-#pragma unroll
-        for (int i = 0; i < 8; i++) sum[i] = fmaf(w, (float)v[i], sum[i]);
-    }
+    y += n;
+    pos += t * top_k;
+    weight += t * top_k;
+    int left = top_k;
+    for (; left >= 4; left -= 4, pos += 4, weight += 4) combine_pairs<4>(sum, y, pos, weight, N);
+    if (left == 3) combine_pairs<3>(sum, y, pos, weight, N);
+    else if (left == 2) combine_pairs<2>(sum, y, pos, weight, N);
+    else if (left == 1) combine_pairs<1>(sum, y, pos, weight, N);
     V8 o;
 #pragma unroll
     for (int i = 0; i < 8; i++) o[i] = to_at<AT>(sum[i]);

@@ -79,6 +79,20 @@ def test_pairs_around_the_rounds_of_their_counting(tokens, top_k, n_exp, hidden)
     _close(got, block._loop(x, index, weight.half()))
 
 
+@pytest.mark.parametrize("top_k", [1, 2, 3, 4, 5, 7, 8, 9])
+def test_experts_per_token_summed_in_fours_and_a_rest(top_k):
+    """Pairs without an expert at the start, at the end, and all of one token: its row is zero."""
+    torch.manual_seed(top_k)
+    block = _block(10, 256, 128, Q["sym_int8"])
+    x = torch.randn(21, 256, device="cuda").half()
+    weight, index = torch.topk(torch.softmax(torch.randn(21, 10, device="cuda"), -1), top_k, dim=-1)
+    index[0, 0], index[20, top_k - 1], index[7] = -1, 10, -1
+    got = block(x, index, weight.half())
+    weight[0, 0], index[0, 0], weight[20, top_k - 1], index[20, top_k - 1], weight[7], index[7] = 0, 0, 0, 0, 0, 0
+    _close(got, block._loop(x, index, weight.half()))
+    assert (got[7] == 0).all()
+
+
 def test_experts_follow_a_weight_that_was_replaced():
     torch.manual_seed(5)
     block = _block(4, 128, 256, Q["sym_int4"])
