@@ -213,9 +213,11 @@ static int launch_gemm_t(const void *x, const void *w, const void *bias, void *y
             const int left = (N + GN / 2 - 1) / (GN / 2) - 2 * tall, tiles_m = (M + GM - 1) / GM;
             ga.tile_rows = GM;
             ga.row_tiles = tiles_m;
-            hipLaunchKernelGGL((gemm_mfma_kernel<QT, AT, true, MB32, false, false, 4, true>),
-                               dim3(8 * (unsigned)(((int64_t)tiles_m * left + 7) / 8)), dim3(256), 0, st, (const AT *)x, (const uint8_t *)w,
-                               (AT *)y, M, N, K, band_rows(tiles_m), ga, G, (float *)nullptr, 2 * tall, left);
+            narrow_form(false, three_blocks(M, GM), [&](auto, auto three) {
+                hipLaunchKernelGGL((gemm_mfma_kernel<QT, AT, true, MB32, false, false, 4, true, 1, decltype(three)::value>),
+                                   dim3(8 * (unsigned)(((int64_t)tiles_m * left + 7) / 8)), dim3(256), 0, st, (const AT *)x, (const uint8_t *)w,
+                                   (AT *)y, M, N, K, band_rows(tiles_m), ga, G, (float *)nullptr, 2 * tall, left);
+            });
             return 0;
         }
     }
@@ -234,7 +236,10 @@ static int launch_gemm_t(const void *x, const void *w, const void *bias, void *y
     // lets a CU hold two workgroups that cover each other's waits, and is 4-8 % ahead with a single workgroup per
     // CU as well - except with nf4, whose code book reads compete with the DMA for LDS: there the register-staged
     // form with its deeper prefetch is 4 % faster while there is at most one workgroup per CU.
-    if (dma)
+    if (dma && !ga.split_tail && three_blocks(M, ga.tile_rows))
+        hipLaunchKernelGGL((gemm_mfma_kernel<QT, AT, true, MB32, false, false, 4, false, 1, true>), grid, dim3(256), 0, st, (const AT *)x,
+                           (const uint8_t *)w, (AT *)y, M, N, K, band_m, ga, k_steps, ws, tn0, tiles_n);
+    else if (dma)
         hipLaunchKernelGGL((gemm_mfma_kernel<QT, AT, true, MB32>), grid, dim3(256), 0, st, (const AT *)x, (const uint8_t *)w,
                            (AT *)y, M, N, K, band_m, ga, k_steps, ws, tn0, tiles_n);
     else
@@ -309,12 +314,12 @@ static int launch_gemm_narrow_t(const void *x, const void *w, const void *bias, 
     ga.tile_rows = halves ? GM : dense_tile_rows(M);
     ga.row_tiles = tiles_m;
     dim3 grid(8 * (unsigned)(((int64_t)tiles_m * tiles_n + 7) / 8 + ga.split_tail), 1);
-    if (narrow_two_groups(M, N, K))
-        hipLaunchKernelGGL((gemm_mfma_kernel<QT, AT, true, MB32, false, false, 4, true, 2>), grid, dim3(512), 0, st, (const AT *)x,
-                       (const uint8_t *)w, (AT *)y, M, N, K, band_rows(tiles_m), ga, G, (float *)nullptr, 0, tiles_n);
-    else
-        hipLaunchKernelGGL((gemm_mfma_kernel<QT, AT, true, MB32, false, false, 4, true>), grid, dim3(256), 0, st, (const AT *)x,
-                           (const uint8_t *)w, (AT *)y, M, N, K, band_rows(tiles_m), ga, G, (float *)nullptr, 0, tiles_n);
+    auto launch = [&](auto groups, auto three) {
+        constexpr int KS = decltype(groups)::value;
+        hipLaunchKernelGGL((gemm_mfma_kernel<QT, AT, true, MB32, false, false, 4, true, KS, decltype(three)::value>), grid, dim3(256 * KS), 0, st,
+                           (const AT *)x, (const uint8_t *)w, (AT *)y, M, N, K, band_rows(tiles_m), ga, G, (float *)nullptr, 0, tiles_n);
+    };
+    narrow_form(narrow_two_groups(M, N, K), !halves && three_blocks(M, ga.tile_rows), launch);
     return 0;
 }
 

@@ -150,12 +150,12 @@ static int launch_mlp_gemm_t(const void *x, const void *wg, const void *wu, void
         ga.tile_rows = plan.halves ? GM : dense_tile_rows(M);
         ga.row_tiles = tiles_m;
         const dim3 grid(8 * (unsigned)(((int64_t)tiles_m * tiles_n + 7) / 8 + ga.split_tail));
-        if (plan.narrow == 2)
-            hipLaunchKernelGGL((gemm_mfma_kernel<QT, AT, true, MB32, false, true, 4, true, 2>), grid, dim3(512), 0, st, (const AT *)x,
-                               (const uint8_t *)wg, (AT *)y, M, N, K, band_rows(tiles_m), ga, G, (float *)nullptr, 0, tiles_n);
-        else
-            hipLaunchKernelGGL((gemm_mfma_kernel<QT, AT, true, MB32, false, true, 4, true, 1>), grid, dim3(256), 0, st, (const AT *)x,
-                               (const uint8_t *)wg, (AT *)y, M, N, K, band_rows(tiles_m), ga, G, (float *)nullptr, 0, tiles_n);
+        auto launch = [&](auto groups, auto three) {
+            constexpr int KS = decltype(groups)::value;
+            hipLaunchKernelGGL((gemm_mfma_kernel<QT, AT, true, MB32, false, true, 4, true, KS, decltype(three)::value>), grid, dim3(256 * KS), 0, st,
+                               (const AT *)x, (const uint8_t *)wg, (AT *)y, M, N, K, band_rows(tiles_m), ga, G, (float *)nullptr, 0, tiles_n);
+        };
+        narrow_form(plan.narrow == 2, !plan.halves && three_blocks(M, ga.tile_rows), launch);
         return 0;
     }
     const int tiles_n = (N + GN / 2 - 1) / (GN / 2), G = K / TILE_COLS;

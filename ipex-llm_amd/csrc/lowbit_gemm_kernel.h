@@ -231,7 +231,12 @@ __device__ inline float gemm_gate_act(float g, int act) {
 // KS == 2 (narrow form only): two groups of WAVES waves on the same tile, each with its own x buffers and accumulators, the
 // first on the first half of the K steps, the second on the rest; `meet` adds their sums.  Two waves per SIMD cover each
 // other's waits and dequantization where the tiles of a product are no more than one per CU (narrow_two_groups).
-template <int QT, typename AT, bool DMA, int MB, bool GROUPED = false, bool DUAL = false, int WAVES = 4, bool NARROW = false, int KS = 1>
+// THREE (dense 128-row DMA forms): some row tile of the launch holds 65 to 96 rows (three_blocks), which a loop of its own walks.
+// Not part of every launch's kernel: a fourth copy of the loop costs registers and spills in the others (two more spilled in asym_int4
+// with fp16 and sym_int8, up to 8 more registers), 1.01 times the time over 230 random launches that never run it.  Here the copy for
+// one block is left out, which no such launch has.
+template <int QT, typename AT, bool DMA, int MB, bool GROUPED = false, bool DUAL = false, int WAVES = 4, bool NARROW = false, int KS = 1,
+          bool THREE = false>
 __global__ __launch_bounds__(64 * WAVES * KS, (DMA && MB == 4) ? 2 : 1) void gemm_mfma_kernel(const AT *__restrict__ x, const uint8_t *__restrict__ w,
                                                         AT *__restrict__ y, int M, int N, int K, int band_m,
                                                         const GroupArgs ga, int k_steps,
@@ -243,6 +248,7 @@ __global__ __launch_bounds__(64 * WAVES * KS, (DMA && MB == 4) ? 2 : 1) void gem
     static_assert(WAVES == 4 || (WAVES == 8 && MB == 8 && DMA), "eight waves: tall form only");
     static_assert(!NARROW || (DMA && MB == 4 && WAVES == 4), "the narrow tile is a 128-row DMA form");
     static_assert(KS == 1 || (KS == 2 && NARROW), "two groups of waves: the narrow tile");
+    static_assert(!THREE || (DMA && MB == 4 && !GROUPED), "three row blocks: a dense 128-row DMA form");
     constexpr int MB32 = MB, GM = 32 * MB;            // shadow the 128-row constants of the file
     constexpr int GN = NARROW ? lowbit::GN / 2 : lowbit::GN;
     constexpr int NB32 = GN / WAVES / 32;             // 32-row weight blocks per wave: 2, or 1 with eight waves or a narrow tile
@@ -1211,13 +1217,17 @@ __global__ __launch_bounds__(64 * WAVES * KS, (DMA && MB == 4) ? 2 : 1) void gem
             case 7: run(std::integral_constant<int, 7>()); break;
             default: run(full_t()); break;
             }
-        } else if (mb_cnt <= 1) {
+        } else if (!THREE && mb_cnt <= 1) {
             run(std::integral_constant<int, 1>());
         } else if (mb_cnt <= 2) {
             run(std::integral_constant<int, 2>());
-        } else if (mb_cnt == 3) {
-            run(std::integral_constant<int, 3>());
         } else {
+            if constexpr (THREE || GROUPED) {
+                if (mb_cnt == 3) {
+                    run(std::integral_constant<int, 3>());
+                    return;
+                }
+            }
             run(full_t());
         }
     } else {
@@ -1266,6 +1276,17 @@ __global__ __launch_bounds__(64 * WAVES * KS, (DMA && MB == 4) ? 2 : 1) void gem
 inline int dense_tile_rows(int M) {
     const int tiles = (M + GM - 1) / GM, blocks = (M + 31) / 32;
     return tiles > 1 ? (blocks + tiles - 1) / tiles * 32 : GM;
+}
+
+// Whether a launch with that many rows per row tile has one of 65 to 96 rows (half tiles of 64 rows apart).
+inline bool three_blocks(int M, int tile_rows) { return tile_rows == 96 || (M % GM > 64 && M % GM <= 96); }
+
+// launch(KS, THREE) with the kernel's template arguments, as integral constants, for a dense launch of narrow tiles.
+template <typename F> inline void narrow_form(bool two_groups, bool three, F &&launch) {
+    typedef std::integral_constant<int, 1> one_t;
+    typedef std::integral_constant<int, 2> two_t;
+    if (two_groups) three ? launch(two_t(), std::true_type()) : launch(two_t(), std::false_type());
+    else three ? launch(one_t(), std::true_type()) : launch(one_t(), std::false_type());
 }
 
 // Row tiles per band of the kernel's tile order (see the kernel): the row tiles are cut into at most 8 bands, a

@@ -41,11 +41,12 @@ def listings(tmp_path_factory):
 def test_generated_assembly_respects_the_mfma_hazards(unit, listings):
     listing = listings[unit]
     assert isinstance(listing, str), "hipcc failed on %s with code %s" % (unit, listing)
-    # the 128-row DMA form (not the narrow one) is held to 128 vector registers, for two workgroups per compute unit, and spills a few;
-    # the grouped tall form with eight waves (two per SIMD, 128 vector registers each) may spill outside its loops
-    out = subprocess.run([sys.executable, CHECKER, listing, "--allow-scratch", "Lb1ELi4ELb0ELb0ELi4ELb0E", "Lb1ELi4ELb1ELb0ELi4ELb0E",
-                          "--allow-scratch-outside-loops", "Li8ELb1ELb1ELi8E"],
-                         capture_output=True, text=True)
+    # Nothing spills inside a loop.  Outside loops: the 128 x 256 DMA form, which is held to 128 vector registers for two workgroups per
+    # compute unit, in the 8-bit formats, its grouped variant in asym_int4 with fp16 as well, and the grouped tall form with eight
+    # waves (two per SIMD, 128 vector registers each).
+    spills = ["ILi%dE%sLb1ELi4ELb%dELb0ELi4ELb0E" % (qtype, at, grouped) for qtype in (8, 15) for at in ("DF16_", "DF16b") for grouped in (0, 1)]
+    out = subprocess.run([sys.executable, CHECKER, listing, "--allow-scratch-outside-loops", "ILi3EDF16_Lb1ELi4ELb1ELb0ELi4ELb0E",
+                          "Li8ELb1ELb1ELi8E"] + spills, capture_output=True, text=True)
     assert out.returncode == 0, out.stdout[-4000:]
     assert out.stdout.count(": ok") >= 3, out.stdout
 

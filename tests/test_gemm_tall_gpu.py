@@ -40,6 +40,12 @@ def test_rounds_that_are_partly_filled(qtype, m, n, k, dtype):
     check(qtype, m, n, k, dtype, ggml.lowbit_gemm)
 
 
+@pytest.mark.parametrize("qtype", ALL, ids=NAMES.values())
+def test_rest_of_the_columns_ends_on_three_blocks(qtype):
+    """2016 rows: a last tall tile of 224 rows, and what is left of the columns in tiles of 128 rows, the last of 96."""
+    check(qtype, 2016, 11008, 512, torch.bfloat16, ggml.lowbit_gemm)
+
+
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16], ids=["f16", "bf16"])
 @pytest.mark.parametrize("m,n,k", [(1, 16, 128), (32, 144, 256), (33, 128, 384), (64, 272, 640), (65, 1040, 512), (200, 4096, 1152)])
 def test_narrow_nf4(m, n, k, dtype):

@@ -73,6 +73,13 @@ def test_row_tiles_of_three_blocks(qtype, dtype, m, n, k):
     _check(qtype, dtype, ggml.LAYOUT_TILED, m, n, k, m % 2 == 1, m + n)
 
 
+@pytest.mark.parametrize("qtype,dtype", [(2, torch.float16), (3, torch.float16), (8, torch.bfloat16), (10, torch.float16), (15, torch.float16)])
+@pytest.mark.parametrize("m", [224, 225, 352, 480])
+@pytest.mark.parametrize("n,k", [(1040, 4096), (2064, 1152), (16400, 256)], ids=["splits", "narrow", "wide"])
+def test_last_row_tile_of_three_blocks_behind_whole_ones(qtype, dtype, m, n, k):
+    _check(qtype, dtype, ggml.LAYOUT_TILED, m, n, k, m % 2 == 1, m + n)
+
+
 def _plain(qtype, m, n, k, dtype):
     if qtype == FP8 and k % 128:
         n, k = n + 1, (k + 127) // 128 * 128
