@@ -46,16 +46,25 @@ __global__ __launch_bounds__(512, 2) void gemm_back_kernel(const AT *__restrict_
     const int lane = threadIdx.x & 63;
     const int wave_wg = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), half = wave_wg >> 2, wave = wave_wg & 3;
 
+    const uint32_t grid_x = gridDim.x, splits = gridDim.y;
+    // (one wait for all arguments: left alone the compiler loads each where it is first used, a scalar load's time apiece)
+    asm volatile("" :: "s"(g), "s"(w), "s"(M), "s"(N), "s"(K), "s"(ws), "s"(split_steps), "s"(grid_x), "s"(splits));
+
     // Workgroups go to the XCDs in turn (id % 8): each takes a run of the tiles, the row tiles of a column tile side by side,
     // so that its L2 serves a column's weights to all of them.
     const int tiles_m = (M + BM - 1) / BM, G = K / TILE_COLS;
     // (What is dealt is tiles times splits, a tile's side by side: with an eighth of the tiles in every split the XCDs differ by up to
     // as many workgroups as there are splits, and those above a workgroup per CU wait.  125 rows on [9104 x 6272] in sym_int8, a
     // training step with the forward's splits dealt likewise: 89 -> 65 us.)
-    const int64_t T = (int64_t)tiles_m * G, units = T * gridDim.y;
-    const int xcd = blockIdx.x & 7, unit = (int)(units * xcd / 8) + (int)((blockIdx.x >> 3) + blockIdx.y * (gridDim.x >> 3));
-    if (unit >= (int)(units * (xcd + 1) / 8)) return;        // whole workgroup leaves
-    const int tile = unit / (int)gridDim.y, split = unit - tile * (int)gridDim.y, m0 = tile % tiles_m * BM, kt = tile / tiles_m;
+    const uint32_t units = (uint32_t)(tiles_m * G * splits), xcd = blockIdx.x & 7;           // (2^28 at most, see launch_back_m)
+    const uint32_t unit = (units * xcd >> 3) + (blockIdx.x >> 3) + blockIdx.y * (grid_x >> 3);
+    if (unit >= units * (xcd + 1) >> 3) return;              // whole workgroup leaves
+    int tile = (int)unit, split = 0;
+    if (ws) {
+        tile = (int)(unit / splits);
+        split = (int)(unit - tile * splits);
+    }
+    const int m0 = tile % tiles_m * BM, kt = tile / tiles_m;
 
     const int all_steps = (N + BACK_N - 1) / BACK_N, split_s0 = ws ? split * split_steps : 0;
     const int steps = ws && split_steps < all_steps - split_s0 ? split_steps : all_steps - split_s0, steps_first = (steps + 1) / 2;
@@ -243,7 +252,7 @@ __global__ __launch_bounds__(512, 2) void gemm_back_kernel(const AT *__restrict_
     // C layout: lane = 32 * kg + row of g, register i = column 8 * (i / 4) + 4 * kg + i % 4
     auto finish = [&](int from) __attribute__((always_inline)) {
         if (ws) {
-            f32x4 *const to = ws + (((int64_t)split * T + tile) * 8 + wave_wg) * (MBW * 256) + lane;
+            f32x4 *const to = ws + (((int64_t)split * (tiles_m * G) + tile) * 8 + wave_wg) * (MBW * 256) + lane;
 #pragma unroll
             for (int mb = from; mb < from + MBW; mb++)
 #pragma unroll

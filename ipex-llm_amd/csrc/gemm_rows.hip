@@ -154,16 +154,24 @@ __global__ __launch_bounds__(256, 2) void gemm_rows_kernel(const AT *__restrict_
     const int lane = threadIdx.x & 63, r = lane & 31, c = lane >> 5;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
 
+    const int grid_x = gridDim.x, splits = gridDim.y;
+    // (one wait for all arguments: left alone the compiler loads each where it is first used, a scalar load's time apiece)
+    asm volatile("" :: "s"(x), "s"(w), "s"(M), "s"(N), "s"(K), "s"(steps), "s"(ws), "s"(grid_x), "s"(splits));
+
     // Workgroups go to the XCDs in turn (id % 8): each XCD takes a run of the tiles, row tile by row tile within a column
     // tile, so that its L2 serves a column's weights to all their row tiles.
     // (With K splits what is dealt is tiles times splits, a tile's side by side: an eighth of the tiles in every split leaves some
     // XCDs with up to as many workgroups more as there are splits.  156 rows on [1281 x 6592] in asym_int4 took 1.23 times as
     // long, 136 on [1785 x 13248] in nf4 1.25, 85 random sizes 1.008 on average.)
     const int tiles_m = (M + BM - 1) / BM, tiles = tiles_m * ((N + RG_N - 1) / RG_N), xcd = blockIdx.x & 7;
-    const int64_t units = (int64_t)tiles * gridDim.y;
-    const int first = (int)(units * xcd / 8), unit = first + (int)((blockIdx.x >> 3) + blockIdx.y * (gridDim.x >> 3));
-    if (unit >= (int)(units * (xcd + 1) / 8)) return;        // whole workgroup leaves
-    const int tile = unit / (int)gridDim.y, split = unit - tile * (int)gridDim.y;
+    int tile = (tiles * xcd >> 3) + (int)(blockIdx.x >> 3), split = 0;       // (tiles below 2^27, see launch_gemm_rows)
+    if (ws) {
+        const int units = tiles * splits, first = units * xcd >> 3, count = (units * (xcd + 1) >> 3) - first;
+        const int place = (int)((blockIdx.x >> 3) + blockIdx.y * (grid_x >> 3));
+        if (place >= count) return;
+        tile = (first + place) / splits;
+        split = first + place - tile * splits;
+    } else if (tile >= tiles * (xcd + 1) >> 3) return;       // whole workgroup leaves
     const int m0 = tile % tiles_m * BM, n0 = tile / tiles_m * RG_N + wave * 32;
 
     const int blocks = K / F::QK, G = (K + TILE_COLS - 1) / TILE_COLS;

@@ -280,6 +280,9 @@ __global__ __launch_bounds__(64 * WAVES * KS, (DMA && MB == 4) ? 2 : 1) void gem
     int row_tile = 0, split = blockIdx.y;
     if constexpr (!GROUPED) {
         const int pitch = ga.tile_rows, tiles_m = ga.row_tiles, tiles_n = tn_cnt;
+        const int grid_x = gridDim.x, splits = gridDim.y;
+        // (one wait for the arguments that say which tile: left alone the compiler loads M behind the first of them)
+        asm volatile("" :: "s"(M), "s"(band_m), "s"(tn0), "s"(tn_cnt), "s"(ws), "s"(pitch), "s"(tiles_m), "s"(ga.split_tail), "s"(grid_x), "s"(splits));
         const int64_t T = (int64_t)tiles_m * tiles_n;
         const int xcd = blockIdx.x & 7;
         int slot = blockIdx.x >> 3, first = (int)(T * xcd / 8), count = (int)(T * (xcd + 1) / 8) - first;
@@ -288,10 +291,10 @@ __global__ __launch_bounds__(64 * WAVES * KS, (DMA && MB == 4) ? 2 : 1) void gem
             // split, 50 tiles in five splits - 250 workgroups - put 35 on some XCDs, whose 32 CUs then took turns (178 rows on
             // [6288 x 14720] in bf16 sym_int4 76.0 us, with four splits 57.5).  Split by split instead, every XCD reads from all
             // rows of the weight (284 rows on [2512 x 3968] in fp8_e4m3 22.5 us a tile's splits side by side, 26.5).
-            const int64_t U = T * gridDim.y;
+            const int64_t U = T * splits;
             first = (int)(U * xcd / 8);
             count = (int)(U * (xcd + 1) / 8) - first;
-            slot += blockIdx.y * (gridDim.x >> 3);
+            slot += (int)blockIdx.y * (grid_x >> 3);
         }
         // A launch with fewer tiles than compute units goes out in half tiles, twice as many workgroups (the
         // launcher says how many tiles at the end of each XCD's share are cut: all of them or none).
@@ -306,8 +309,8 @@ __global__ __launch_bounds__(64 * WAVES * KS, (DMA && MB == 4) ? 2 : 1) void gem
         if (idx >= count) return;                                                    // whole workgroup leaves
         int line = first + idx;
         if (ws) {
-            const int tile = line / (int)gridDim.y;
-            split = line - tile * (int)gridDim.y;
+            const int tile = line / splits;
+            split = line - tile * splits;
             line = tile;
         }
         const int per_band = band_m * tiles_n;

@@ -22,6 +22,7 @@ FLAGS = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-ffp-contract=o
 
 UNITS = ([os.path.basename(p) for p in sorted(glob.glob(os.path.join(CSRC, "gemm_grouped_*.hip")))]
          + ["gemm.hip", "gemm_ring.hip", "gemm_rows.hip"])
+HEADS = {"gemm.hip": ("gemm_mfma_kernel", 2), "gemm_rows.hip": ("gemm_rows_kernel", 1), "gemm_back.hip": ("gemm_back_kernel", 1)}
 
 
 @pytest.fixture(scope="module")
@@ -29,7 +30,7 @@ def listings(tmp_path_factory):
     """unit -> path of its assembly listing (or the compiler's return code), all units compiled concurrently"""
     out_dir = tmp_path_factory.mktemp("asm")
     procs = {}
-    for unit in UNITS:
+    for unit in sorted(set(UNITS) | set(HEADS)):
         listing = str(out_dir / (unit + ".s"))
         procs[unit] = (listing, subprocess.Popen([HIPCC] + FLAGS + ["-c", os.path.join(CSRC, unit), "-o", listing],
                                                  cwd=CSRC, stderr=subprocess.DEVNULL))
@@ -49,6 +50,27 @@ def test_generated_assembly_respects_the_mfma_hazards(unit, listings):
                           "Li8ELb1ELb1ELi8E"] + spills, capture_output=True, text=True)
     assert out.returncode == 0, out.stdout[-4000:]
     assert out.stdout.count(": ok") >= 3, out.stdout
+
+
+@pytest.mark.skipif(not os.path.exists(HIPCC), reason="no hipcc")
+@pytest.mark.parametrize("unit", sorted(HEADS))
+def test_a_workgroup_waits_for_its_arguments_once(unit, listings):
+    """Ahead of its first load of x or weights a workgroup waits for scalar loads once (the dense GEMM: once for what says which tile,
+    once for the pointers), not each time it first uses an argument: 0.1 us and more apiece, of launches of 7 to 20 us."""
+    kernel, most = HEADS[unit]
+    waits, name = {}, None
+    for line in open(listings[unit]):
+        if line.startswith("_Z") and line.split(";")[0].rstrip().endswith(":"):
+            name = line if kernel in line else None
+            waits[name], pending, done = 0, False, name is None
+        elif name and not done:
+            text = line.strip()
+            pending |= text.startswith("s_load")
+            done = text.startswith(("global_load", "s_endpgm"))
+            if pending and text.startswith("s_waitcnt") and "lgkmcnt" in text:
+                waits[name], pending = waits[name] + 1, False
+    waits.pop(None, None)
+    assert len(waits) >= 18 and max(waits.values()) <= most, {n: w for n, w in waits.items() if w > most}
 
 
 def test_the_checker_sees_a_copy_of_a_fresh_accumulator(tmp_path):
