@@ -84,3 +84,14 @@ def test_tiles_of_96_and_160_rows(qtype, dtype, m, n, k):
     ggml.lowbit_linear(x.data_ptr(), blob.data_ptr(), None, y.data_ptr(), qtype, GGML, DT[dtype], m, 37, k, None, 0, stream())
     want = x.double() @ dev_dequantize(blob, qtype, 37, k, GGML, torch.float32).double().t()
     assert (classes(y.float().cpu().numpy()) == classes(want.cpu().numpy())).all()
+
+
+@pytest.mark.parametrize("qtype,dtype", [(2, torch.float16), (3, torch.bfloat16), (8, torch.float16), (10, torch.bfloat16), (15, torch.float16)])
+@pytest.mark.parametrize("m,n,k,splits", [(56, 8670, 2176, 4), (52, 17372, 1408, 2), (60, 16383, 1664, 3), (60, 16500, 1664, 3)])
+def test_short_last_splits(qtype, dtype, m, n, k, splits):
+    """Last splits that are shorter than the others, of workgroups that are a few more than the CUs (they go out last), as many more as
+    there are tiles, and more than that."""
+    tiles, steps = -(-n // 128), -(-(k // 128) // splits)
+    assert ggml.lowbit_linear_workspace_bytes(qtype, GGML, DT[dtype], m, n, k, 256 << 20) == splits * tiles * 64 * 128 * 4
+    assert splits * steps > k // 128
+    _check(qtype, dtype, GGML, m, n, k, False, m + n)
