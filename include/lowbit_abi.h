@@ -255,6 +255,8 @@ int lowbit_backward_applies(int qtype, int layout, int act_dtype, int64_t M, int
 int lowbit_backward_ws(const void *grad, const void *w, void *grad_x, int qtype, int act_dtype, int64_t M, int64_t N, int64_t K,
                        void *workspace, size_t workspace_bytes, void *stream);
 size_t lowbit_backward_workspace_bytes(int qtype, int64_t M, int64_t N, int64_t K);
+/* 1 where lowbit_backward_ws with that much workspace is the faster of the two ways (lowbit_backward_applies: with none). */
+int lowbit_backward_ws_applies(int qtype, int layout, int act_dtype, int64_t M, int64_t N, int64_t K, size_t workspace_bytes);
 
 /* lowbit_forward_ws without a workspace argument and without any allocation: the partial tiles go to a
  * scratch array that is part of the library's image on every GPU (lowbit_noalloc_scratch_bytes() = 64 MiB,

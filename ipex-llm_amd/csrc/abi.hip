@@ -43,7 +43,7 @@ int launch_gemm_narrow(const void *x, const void *w, const void *bias, void *y, 
 size_t gemm_rows_workspace_bytes(int qtype, int act_dtype, int M, int N, int K, size_t max_bytes);
 int launch_gemm_rows(const void *x, const void *w, const void *bias, void *y, int qtype, int act_dtype, int M, int N, int K,
                      void *workspace, size_t workspace_bytes, hipStream_t st);
-bool gemm_back_applies(int qtype, int M, int N, int K);
+bool gemm_back_applies(int qtype, int M, int N, int K, size_t ws_bytes);
 size_t back_workspace_bytes(int qtype, int M, int N, int K);
 int launch_gemm_back(const void *g, const void *w, void *gx, int qtype, int act_dtype, int M, int N, int K, void *ws, size_t ws_bytes,
                      hipStream_t st);
@@ -513,9 +513,13 @@ int lowbit_dequantize_rows(const void *w, const int64_t *rows, int64_t n_rows, v
 }
 
 int lowbit_backward_applies(int qtype, int layout, int act_dtype, int64_t M, int64_t N, int64_t K) {
+    return lowbit_backward_ws_applies(qtype, layout, act_dtype, M, N, K, 0);
+}
+
+int lowbit_backward_ws_applies(int qtype, int layout, int act_dtype, int64_t M, int64_t N, int64_t K, size_t workspace_bytes) {
     if (layout != LOWBIT_LAYOUT_TILED || (act_dtype != LOWBIT_DT_F16 && act_dtype != LOWBIT_DT_BF16) || !lowbit_tileable(qtype, N, K) ||
         M <= 0 || M > 0x7fffffff || N > 0x7fffffff || K > 0x7fffffff) return 0;
-    return gemm_back_applies(qtype, (int)M, (int)N, (int)K);
+    return gemm_back_applies(qtype, (int)M, (int)N, (int)K, workspace_bytes);
 }
 
 size_t lowbit_backward_workspace_bytes(int qtype, int64_t M, int64_t N, int64_t K) {

@@ -384,10 +384,15 @@ static int launch_back_q(const void *g, const void *w, void *gx, int dt, int M, 
 // CU at most (with a second round it is 0.6 - 1.3 times as fast), and there are 20 workgroups or more: one of the 258
 // sizes above is slower by more than 3 % (1064 rows on [13984 x 2816] in nf4 153 us against 137).  A K below 1024 leaves few column tiles, and there the walk along N is to be
 // no longer than four times K over 20 tiles at least.
-bool gemm_back_applies(int qtype, int M, int N, int K) {
-    const BackPlan p = back_plan(qtype, M, N, K, (size_t)-1);
+// With less workspace than the plan asks for the walks are longer: then it is the faster way from 20 tiles on while N is no longer than
+// twice K, and from 80 on up to four times (4900 random sizes, 1.64 times as fast on average, 31 more than 5 % slower, 0.79 at worst).
+bool gemm_back_applies(int qtype, int M, int N, int K, size_t ws_bytes) {
+    BackPlan p = back_plan(qtype, M, N, K, (size_t)-1);
+    const bool shared = p.splits == 1 || (size_t)p.splits * back_split_bytes(M, K, p.rows) <= ws_bytes;
+    if (!shared) p = back_plan(qtype, M, N, K, 0);
     const int64_t tiles = back_tiles(M, K, p.rows);
     if (tiles > 256 || N >= (1 << 23)) return false;
+    if (!shared) return N <= 2 * (int64_t)K ? tiles >= 20 : qtype != QT_NF4 && tiles >= 80 && N <= 4 * (int64_t)K;
     if (K < 1024) return tiles >= 20 && N <= (qtype == QT_NF4 ? 2 : 4) * (int64_t)K;
     return tiles * p.splits >= 20;
 }

@@ -41,7 +41,7 @@ struct Api {
     decltype(&lowbit_dequantize) dequantize = nullptr;
     decltype(&lowbit_backward_ws) backward_ws = nullptr;
     decltype(&lowbit_backward_workspace_bytes) backward_workspace_bytes = nullptr;
-    decltype(&lowbit_backward_applies) backward_applies = nullptr;
+    decltype(&lowbit_backward_ws_applies) backward_ws_applies = nullptr;
     decltype(&lowbit_experts_workspace_bytes) experts_workspace_bytes = nullptr;
     decltype(&lowbit_experts_forward) experts_forward = nullptr;
 } api;
@@ -169,11 +169,11 @@ struct ProductBackward : public torch::autograd::Node {
         const int dt = dtype_code(dtype);
         void *const stream = current_stream(grad);
         const bool tracked = differentiable(grad) || !nothing_watches(grad);
-        if (!tracked && api.backward_applies(qtype, layout, dt, M, N, K)) {
+        const size_t bytes = tracked ? 0 : api.backward_workspace_bytes(qtype, M, N, K);
+        if (!tracked && api.backward_ws_applies(qtype, layout, dt, M, N, K, bytes)) {
             const Tensor g = grad.contiguous();
             if ((((uintptr_t)g.const_data_ptr() | (uintptr_t)w.const_data_ptr()) & 15) == 0) {
                 Tensor gx = at::empty(x_shape, g.options());
-                const size_t bytes = api.backward_workspace_bytes(qtype, M, N, K);
                 const Tensor ws = bytes ? at::empty({(int64_t)bytes}, g.options().dtype(at::kByte)) : Tensor();
                 check(api.backward_ws(g.const_data_ptr(), w.const_data_ptr(), gx.data_ptr(), qtype, dt, M, N, K,
                                       bytes ? ws.data_ptr() : nullptr, bytes, stream), "lowbit_backward");
@@ -405,7 +405,7 @@ PyObject *py_bind(PyObject *, PyObject *const *args, Py_ssize_t n) {
         api.name = (decltype(api.name))p;                                                          \
     } while (0)
     BIND(last_error); BIND(blob_bytes); BIND(tileable); BIND(linear_workspace_bytes); BIND(linear);
-    BIND(mlp_forward); BIND(dequantize_rows); BIND(dequantize); BIND(backward_ws); BIND(backward_workspace_bytes); BIND(backward_applies); BIND(experts_workspace_bytes); BIND(experts_forward);
+    BIND(mlp_forward); BIND(dequantize_rows); BIND(dequantize); BIND(backward_ws); BIND(backward_workspace_bytes); BIND(backward_ws_applies); BIND(experts_workspace_bytes); BIND(experts_forward);
 #undef BIND
     Py_RETURN_NONE;
 }

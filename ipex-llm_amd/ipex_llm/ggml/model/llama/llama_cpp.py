@@ -239,6 +239,14 @@ def lowbit_backward_applies(qtype, layout, act_dtype, m, n, k):
     return bool(_lib.lowbit_backward_applies(qtype, layout, act_dtype, m, n, k))
 
 
+_lib.lowbit_backward_ws_applies.argtypes = [c_int, c_int, c_int, c_int64, c_int64, c_int64, c_size_t]
+_lib.lowbit_backward_ws_applies.restype = c_int
+
+
+def lowbit_backward_ws_applies(qtype, layout, act_dtype, m, n, k, workspace_bytes):
+    return bool(_lib.lowbit_backward_ws_applies(qtype, layout, act_dtype, m, n, k, workspace_bytes))
+
+
 _lib.lowbit_forward_plan.argtypes = [c_int, c_int, c_int64, c_int64, c_int64, c_int, c_size_t]
 _lib.lowbit_forward_plan.restype = c_int
 PLAN_GEMV, PLAN_RING, PLAN_GEMM, PLAN_GEMM_SPLIT, PLAN_GEMM_NARROW = 0, 1, 2, 3, 4

@@ -503,3 +503,14 @@ def test_narrow_tiles_of_8_bits_are_not_estimated_too_short():
     or a K split; both of those ask for a workspace, narrow tiles do not."""
     for qtype, m, n, k in [(8, 166, 5216, 4352), (8, 1087, 1600, 7424), (8, 89, 6944, 3328), (15, 365, 3376, 4352)]:
         assert ggml.lowbit_linear_workspace_bytes(qtype, ggml.LAYOUT_TILED, ggml.DT_F16, m, n, k, 256 << 20) > 0
+
+
+def test_backward_applies_speaks_for_the_call_without_a_workspace():
+    """24 rows on [4096 x 1024]: eight workgroups without splits.  100 rows on [1024 x 2560]: the call plans no splits."""
+    need = ggml.lowbit_backward_workspace_bytes(2, 24, 4096, 1024)
+    assert need > 0 and not ggml.lowbit_backward_applies(2, ggml.LAYOUT_TILED, ggml.DT_F16, 24, 4096, 1024)
+    for size, want in ((0, False), (need - 1, False), (need, True), (2 * need, True)):
+        assert ggml.lowbit_backward_ws_applies(2, ggml.LAYOUT_TILED, ggml.DT_F16, 24, 4096, 1024, size) is want
+    assert not ggml.lowbit_backward_ws_applies(2, ggml.LAYOUT_GGML, ggml.DT_F16, 24, 4096, 1024, need)
+    assert ggml.lowbit_backward_workspace_bytes(2, 100, 1024, 2560) == 0
+    assert ggml.lowbit_backward_applies(2, ggml.LAYOUT_TILED, ggml.DT_F16, 100, 1024, 2560)
