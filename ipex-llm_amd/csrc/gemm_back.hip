@@ -381,9 +381,14 @@ static int launch_back_q(const void *g, const void *w, void *gx, int dt, int M, 
 }
 
 // Whether this kernel is the faster way, against dequantizing W and torch's dense product: while its tiles of 128 rows are one per
-// CU at most (with a second round it is 0.6 - 1.3 times as fast), and there are 20 workgroups or more: one of the 258
-// sizes above is slower by more than 3 % (1064 rows on [13984 x 2816] in nf4 153 us against 137).  A K below 1024 leaves few column tiles, and there the walk along N is to be
-// no longer than four times K over 20 tiles at least.
+// CU at most (with a second round it is 0.6 - 1.3 times as fast), and there are 20 workgroups or more.  A K below 1024 leaves few
+// column tiles, and there the walk along N is to be no longer than four times K over 20 tiles at least.  Over 1150 random sizes, M =
+// 200 .. 2048, N = 4096 .. 152000, K = 1024 .. 8192: shared walks 1.8 times as fast and never slower, tiles of 64 rows 1.17 (11 of
+// 180 slower by more than 3 %), unshared tiles of 128 rows
+//   - 1.2 in fp8_e4m3, never slower, and 1.07 in the integers where N is more than four times K (1.2 below): 28 of 111 are slower by
+//     more than 3 %, 0.78 at worst, because the dense product's rate varies from 320 to 830 TFLOP/s between neighbouring sizes;
+//   - in nf4, which takes 1.2 of the others' time, 1.06 up to N = 2.5 K and 0.98 beyond (187 of 336 slower by more than 3 %, 0.69 at
+//     worst; 1064 rows on [13984 x 2816] 153 us against 137): not taken there.
 // With less workspace than the plan asks for the walks are longer: then it is the faster way from 20 tiles on while N is no longer than
 // twice K, and from 80 on up to four times (4900 random sizes, 1.64 times as fast on average, 31 more than 5 % slower, 0.79 at worst).
 bool gemm_back_applies(int qtype, int M, int N, int K, size_t ws_bytes) {
@@ -394,6 +399,7 @@ bool gemm_back_applies(int qtype, int M, int N, int K, size_t ws_bytes) {
     if (tiles > 256 || N >= (1 << 23)) return false;
     if (!shared) return N <= 2 * (int64_t)K ? tiles >= 20 : qtype != QT_NF4 && tiles >= 80 && N <= 4 * (int64_t)K;
     if (K < 1024) return tiles >= 20 && N <= (qtype == QT_NF4 ? 2 : 4) * (int64_t)K;
+    if (qtype == QT_NF4 && p.rows == 128 && p.splits == 1 && 2 * (int64_t)N > 5 * (int64_t)K) return false;
     return tiles * p.splits >= 20;
 }
 

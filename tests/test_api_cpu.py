@@ -514,3 +514,12 @@ def test_backward_applies_speaks_for_the_call_without_a_workspace():
     assert not ggml.lowbit_backward_ws_applies(2, ggml.LAYOUT_GGML, ggml.DT_F16, 24, 4096, 1024, need)
     assert ggml.lowbit_backward_workspace_bytes(2, 100, 1024, 2560) == 0
     assert ggml.lowbit_backward_applies(2, ggml.LAYOUT_TILED, ggml.DT_F16, 100, 1024, 2560)
+
+
+def test_long_walks_of_nf4_go_to_the_dense_product():
+    """Whole GPUs of unshared 128-row tiles: N up to 2.5 K.  Shared walks, 64-row tiles and the other formats: any N."""
+    def applies(qtype, m, n, k):
+        return ggml.lowbit_backward_ws_applies(qtype, ggml.LAYOUT_TILED, ggml.DT_BF16, m, n, k, ggml.lowbit_backward_workspace_bytes(qtype, m, n, k))
+    assert applies(10, 1024, 10240, 4096) and not applies(10, 1024, 10256, 4096) and not applies(10, 1064, 13984, 2816)
+    assert applies(10, 256, 32000, 4096) and ggml.lowbit_backward_workspace_bytes(10, 256, 32000, 4096) > 0
+    assert all(applies(q, 1024, 128256, 4096) for q in (2, 3, 8, 15)) and not applies(10, 1024, 128256, 4096)
