@@ -523,3 +523,17 @@ def test_long_walks_of_nf4_go_to_the_dense_product():
     assert applies(10, 1024, 10240, 4096) and not applies(10, 1024, 10256, 4096) and not applies(10, 1064, 13984, 2816)
     assert applies(10, 256, 32000, 4096) and ggml.lowbit_backward_workspace_bytes(10, 256, 32000, 4096) > 0
     assert all(applies(q, 1024, 128256, 4096) for q in (2, 3, 8, 15)) and not applies(10, 1024, 128256, 4096)
+
+
+def test_a_workspace_of_the_size_asked_for_gets_the_plan_it_was_sized_for():
+    """Asked again within its own answer, lowbit_linear_workspace_bytes gives the same: the launch plans within those bytes."""
+    rng = np.random.default_rng(7)
+    sizes = [(2, 0, 67, 15073, 1792), (10, 0, 463, 6179, 960), (2, 0, 2032, 744, 2112), (15, 0, 263, 1829, 2240)]
+    sizes += [(int(rng.choice([2, 3, 8, 10, 15])), i % 2, int(2 ** rng.uniform(4.1, 11)), 16 * int(2 ** rng.uniform(2, 11)) + 3 * (1 - i % 2),
+               128 * int(2 ** rng.uniform(0, 7))) for i in range(4000)]
+    for qtype, layout, m, n, k in sizes:
+        for dt in (ggml.DT_F16, ggml.DT_BF16):
+            for budget in (256 << 20, int(2 ** rng.uniform(15, 26))):
+                need = ggml.lowbit_linear_workspace_bytes(qtype, layout, dt, m, n, k, budget)
+                assert need <= budget
+                assert ggml.lowbit_linear_workspace_bytes(qtype, layout, dt, m, n, k, need) == need, (qtype, layout, dt, m, n, k, budget)
