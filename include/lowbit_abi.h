@@ -232,10 +232,11 @@ int lowbit_forward_f32(const float *x, const void *w, float *y, int qtype, int l
 
 /* One linear layer: y = x * dequant(w)^T + bias.  x, bias ([N], may be null) and y are of `dtype`, which may be
  * LOWBIT_DT_F32: then as lowbit_forward_f32, and no workspace is used.  With 16-bit activations as lowbit_forward_ws
- * (lowbit_linear_workspace_bytes says what to pass within a budget; null is valid), but for two choices that the other entry
+ * (lowbit_linear_workspace_bytes says what to pass within a budget; null is valid), but for three choices that the other entry
  * points, whose kernel a caller may rely on, do not make: the one-pass kernel at 9 .. 64 rows in place of the ring kernel, a K
- * split or several streaming passes, and narrow tiles more often (two groups of waves share such a tile's K where CUs
- * would idle).  The bias is added to the fp32 sums before the one rounding (a bias that is not 8-byte aligned is valid and
+ * split or several streaming passes; narrow tiles more often (two groups of waves share such a tile's K where CUs
+ * would idle); and tiles of 256 rows ahead of all estimates where they fill the GPU's rounds well (the rounds depend on the
+ * activation type).  The bias is added to the fp32 sums before the one rounding (a bias that is not 8-byte aligned is valid and
  * slower above 16 rows).  What LowBitLinear.forward computes
  * (low_bit_linear.py:657-687 of the reference). */
 int lowbit_linear(const void *x, const void *w, const void *bias, void *y, int qtype, int layout, int dtype, int64_t M,

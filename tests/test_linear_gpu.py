@@ -80,6 +80,13 @@ def test_last_row_tile_of_three_blocks_behind_whole_ones(qtype, dtype, m, n, k):
     _check(qtype, dtype, ggml.LAYOUT_TILED, m, n, k, m % 2 == 1, m + n)
 
 
+@pytest.mark.parametrize("m,n,k,dtype", [(385, 17136, 256, torch.float16), (700, 11520, 384, torch.bfloat16)])
+@pytest.mark.parametrize("qtype", ALL)
+def test_rounds_of_tall_tiles_that_are_partly_filled(qtype, m, n, k, dtype):
+    """Tiles of 256 rows over half a round of the GPU and more, which lowbit_linear takes ahead of the estimates."""
+    _check(qtype, dtype, ggml.LAYOUT_TILED, m, n, k, True, m + n)
+
+
 def _plain(qtype, m, n, k, dtype):
     if qtype == FP8 and k % 128:
         n, k = n + 1, (k + 127) // 128 * 128
