@@ -5,11 +5,13 @@ import pytest
 import torch
 
 import lowbit_oracle as orc
+import ipex_llm.ggml.model.llama.llama_cpp as ggml
 from ipex_llm.ggml.quantize import ggml_tensor_qtype as Q
 from ipex_llm.transformers.low_bit_linear import FP4Params, LowBitLinear
 from ipex_llm.transformers.moe import (ExpertWeights, grouped_forward, grouped_mlp_forward, moe_ffn_grouped,
                                        moe_ffn_reference, route_top_k)
 from gpu_util import weights
+from test_grouped_addressing import grouped_tile_lanes
 
 pytestmark = pytest.mark.gpu
 
@@ -46,6 +48,43 @@ def test_grouped_forward_matches_oracle_per_group(qname, dtype):
             tol = 2e-3 if dtype == torch.float16 else 8e-3
             assert np.abs(y[r0:r0 + c] - want).max() <= tol * np.abs(want).max(), (e, c)
         r0 += c
+
+
+@pytest.mark.parametrize("n_exp,top,k,longest_first", [(1, 500, 2048, True), (9, 300, 2048, True), (12, 259, 2048, True), (9, 70, 4096, False)])
+def test_workgroups_take_the_row_tiles_longest_first(n_exp, top, k, longest_first):
+    """Which tile each workgroup of a tall launch takes, read from the partial sums it leaves in the workspace (its own place of
+    256 x 256 floats): row r of x times a column of tile t's weights is (r + 1) / 2^t there, in split 0.  Groups of up to 64 rows on average keep the
+    groups' order."""
+    n = 1280
+    rng = np.random.default_rng(n_exp + top)
+    counts = [int(c) for c in rng.integers(1, top, n_exp)]
+    counts[0] = top
+    rows, offs = sum(counts), [0] + [int(v) for v in np.cumsum(counts)]
+    assert (rows > 64 * n_exp) == longest_first
+    w = np.zeros((n, k), dtype=np.float32)
+    w[:, 0] = 0.5 ** (np.arange(n) // 256)
+    lin = LowBitLinear(k, n, Q["sym_int4"], bias=False)
+    lin.weight = FP4Params(torch.from_numpy(w), qtype=Q["sym_int4"]).to("cuda")
+    table = ExpertWeights([lin.eval()] * n_exp)
+    x = torch.zeros((rows, k), dtype=torch.float16)
+    x[:, 0] = torch.arange(1, rows + 1)
+    x, y, at = x.cuda(), torch.empty((rows, n), dtype=torch.float16, device="cuda"), torch.tensor(offs, dtype=torch.int32, device="cuda")
+    need = ggml.lowbit_grouped_workspace_bytes(n_exp, rows, n, k)
+    tall, splits, waves, n_wg = ggml.lowbit_grouped_forward_plan(n_exp, rows, n, k, True, need)
+    assert tall and splits >= 2 and waves == 4 and rows < 2048
+    ws = torch.full((need // 4,), float("nan"), device="cuda")
+    ggml.lowbit_grouped_forward_ws(x.data_ptr(), table.ptrs.data_ptr(), y.data_ptr(), at.data_ptr(), n_exp, rows, Q["sym_int4"], ggml.DT_F16, n, k,
+                                   ws.data_ptr(), need, torch.cuda.current_stream().cuda_stream)
+    first = ws[:n_wg * 65536].view(n_wg, 65536)[:, :128].cpu().numpy().reshape(n_wg, 32, 4)     # rows 0 .. 31 of the tile, four columns
+    chunk = 1 if longest_first else 5                   # column tiles per cell: an eighth of a row, or all of it in a single round
+    for b in range(n_wg):
+        tile = grouped_tile_lanes(offs, 5, chunk, b, longest_first)
+        if tile is None:
+            assert np.isnan(first[b]).all()
+            continue
+        _, m0, end, tn = tile
+        for i in range(min(32, end - m0)):
+            assert (first[b, i] == (m0 + i + 1) * 0.5 ** tn).all(), (b, i)
 
 
 # Row counts that put the launch on the 256-row form (more than 96 rows per group on average): a tile for
