@@ -14,7 +14,7 @@
 // registers, and goes to LDS during the step before it.  (g by LDS-DMA instead, which the compiler does not count among
 // the loads in flight, made it wait for the youngest ones and an earlier version a seventh slower.)
 //
-// What bounds it, 128 rows on [4096 x 4096] in sym_int4 (unsplit 33.7 us in a kernel trace, 1.05 us a pair of steps; split 16.0
+// What bounds it, 128 rows on [4096 x 4096] in sym_int4 (unsplit 33.7 us in a kernel trace, 1.05 us a pair of steps; split 15.9
 // and 4.0 for the sums): LDS is busy 54 % of the time, the MFMA pipes 38 %, the vector units 30 %; two waves per SIMD that meet
 // at a barrier per step overlap them badly.
 // Of an earlier version's 39 us the MFMAs were 2, the dequantization with its writes to LDS 12, g's way into LDS 10.  64 rows

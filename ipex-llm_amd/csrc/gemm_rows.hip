@@ -427,7 +427,7 @@ static RowsPlan rows_plan_of(int mb, int M, int N, int K, size_t ws_bytes) {
 // rows on [4001 x 2112] 17.4 -> 14.9 and 22.6 -> 19.8; with both forms at two workgroups per CU 64 rows lose, 256 rows on
 // [30003 x 4096] 92 -> 124).  Tiles of 96 or 160 rows where their estimate is 8 % shorter: 80 rows on [9001 x 4096] in
 // asym_int4 34.4 -> 28.3 us, 129 on [17563 x 3968] 78.5 -> 69.2 and in sym_int8 77.2 -> 53.5, 310 on [4677 x 4096] in sym_int4
-// 36.8 -> 31.6; 1.025 times as fast over 330 random sizes, one of them slower by more than 4 % (143 rows on [5823 x 9216] in
+// 37.8 -> 32.2, sym_int8 54.9 -> 37.0, nf4 47.3 -> 39.8; 1.025 times as fast over 330 random sizes, one of them slower by more than 4 % (143 rows on [5823 x 9216] in
 // fp8_e4m3, 9 %).
 static RowsPlan rows_plan_within(int qtype, int act_dtype, int M, int N, int K, size_t ws_bytes) {
     const int pad64 = (M + 63) / 64 * 64, pad128 = (M + 127) / 128 * 128;

@@ -234,7 +234,10 @@ __device__ inline float gemm_gate_act(float g, int act) {
 // THREE (dense 128-row DMA forms): some row tile of the launch holds 65 to 96 rows (three_blocks), which a loop of its own walks.
 // Not part of every launch's kernel: a fourth copy of the loop costs registers and spills in the others (two more spilled in asym_int4
 // with fp16 and sym_int8, up to 8 more registers), 1.01 times the time over 230 random launches that never run it.  Here the copy for
-// one block is left out, which no such launch has.
+// one block is left out, which no such launch has.  Grouped launches always have the copy, because the host never sees how many rows
+// a group holds: 401 of the 128 x 256 form, five formats, both types, 12 to 95 rows a group, against the kernel without it: 1.00 to
+// 1.03 times as fast with 12 and 30 rows on average, 1.02 with 48 and 62, 1.05 to 1.10 from 75 on; asym_int4 in fp16, whose two
+// registers spill outside its loops, 0.995 with 12 (0.96 at worst) and 1.09 from 75 on.
 template <int QT, typename AT, bool DMA, int MB, bool GROUPED = false, bool DUAL = false, int WAVES = 4, bool NARROW = false, int KS = 1,
           bool THREE = false>
 __global__ __launch_bounds__(64 * WAVES * KS, (DMA && MB == 4) ? 2 : 1) void gemm_mfma_kernel(const AT *__restrict__ x, const uint8_t *__restrict__ w,

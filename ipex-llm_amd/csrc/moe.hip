@@ -110,7 +110,9 @@ __global__ __launch_bounds__(256) void moe_gather_kernel(const u32x4 *__restrict
 // Both at once for up to MOE_SORT_PAIRS pairs: workgroup p counts the pairs that come before pair p - those of lower experts, and the
 // earlier ones of its own - and copies its row of x there; workgroup pairs + e writes offsets[e].  pairs^2 ids come out of L2, which
 // costs less than a second launch that waits for a single workgroup's sort (39 pairs over 5 experts 3.3 + 3.4 us in a kernel
-// trace, 472 over 10 4.4 + 3.9, 1024 over 8 6.4 + 6.1).  Whole experts: 118 tokens, four of 10 of [1408 x 1664], 46.2 -> 40.5 us, 600,
+// trace, 472 over 10 4.4 + 3.9, 1024 over 8 6.4 + 6.1).  At the limit of 4096 pairs it is still the shorter way: over 8 experts with rows
+// of 4096 18.2 us against 13.1 + 10.8 and the gap between two launches, of 1024 15.4 / 13.1 + 4.8, over 16 of 3072 16.8 / 15.8 +
+// 8.6, over 60 of 2048 15.7 / 23.1 + 6.7; at 2048 pairs 8.6 / 7.5 + 6.4, 8.2 / 7.3 + 4.2, 7.9 / 8.6 + 5.2, 7.3 / 12.6 + 4.7.  Whole experts: 118 tokens, four of 10 of [1408 x 1664], 46.2 -> 40.5 us, 600,
 // four of 60 of [768 x 1024], 81.2 -> 69.4.
 constexpr int MOE_SORT_PAIRS = 4096;
 __global__ __launch_bounds__(256) void moe_sort_gather_kernel(const int64_t *__restrict__ ids, const u32x4 *__restrict__ x, int pairs,
