@@ -430,7 +430,7 @@ static RowsPlan rows_plan_of(int mb, int M, int N, int K, size_t ws_bytes) {
 // 37.8 -> 32.2, sym_int8 54.9 -> 37.0, nf4 47.3 -> 39.8; 1.025 times as fast over 330 random sizes, one of them slower by more than 4 % (143 rows on [5823 x 9216] in
 // fp8_e4m3, 9 %).
 static RowsPlan rows_plan_within(int qtype, int act_dtype, int M, int N, int K, size_t ws_bytes) {
-    const int pad64 = (M + 63) / 64 * 64, pad128 = (M + 127) / 128 * 128;
+    const int64_t pad64 = (M + 63) / 64 * 64, pad128 = (M + 127) / 128 * 128;
     RowsPlan p = rows_plan_of(M <= 32 ? 1 : M <= 64 || pad128 * 8 > pad64 * 9 ? 2 : 4, M, N, K, ws_bytes);
     const int G = (K + TILE_COLS - 1) / TILE_COLS;
     if (p.mb == 4 && (int64_t)p.tiles * (G / 4 > 1 ? G / 4 : 1) <= 256) return rows_plan_of(2, M, N, K, ws_bytes);
@@ -458,8 +458,13 @@ static RowsPlan rows_plan(int qtype, int act_dtype, int M, int N, int K, size_t 
     }
 }
 
+// Sizes whose tiles 32-bit counts do not hold, or barely: neither planned nor launched.
+static bool rows_too_many(int M, int N) {
+    return M > 0x7fffff00 || N > 0x7fffff00 || (int64_t)((M + 15) / 16) * ((N + RG_N - 1) / RG_N) > 0x7ffffff;
+}
+
 size_t gemm_rows_workspace_bytes(int qtype, int act_dtype, int M, int N, int K, size_t max_bytes) {
-    return rows_plan(qtype, act_dtype, M, N, K, max_bytes).ws_bytes;
+    return rows_too_many(M, N) ? 0 : rows_plan(qtype, act_dtype, M, N, K, max_bytes).ws_bytes;
 }
 
 template <int QT, typename AT, int MB>
@@ -496,10 +501,10 @@ static int launch_rows_q(const void *x, const void *w, const void *bias, void *y
 int launch_gemm_rows(const void *x, const void *w, const void *bias, void *y, int qtype, int act_dtype, int M, int N, int K,
                      void *workspace, size_t workspace_bytes, hipStream_t st) {
     if (M == 0 || N == 0) return 0;
-    const RowsPlan p = rows_plan(qtype, act_dtype, M, N, K, workspace ? workspace_bytes : 0);
     if (K >= (1 << 23))                                      // 32-bit offsets within a tile of x: the streaming kernel has 64
         return launch_gemv(x, w, bias, y, qtype, LAYOUT_GGML, act_dtype, M, N, K, 0, st);
-    if ((int64_t)((M + 15) / 16) * ((N + RG_N - 1) / RG_N) > 0x7ffffff) return -3;
+    if (rows_too_many(M, N)) return -3;
+    const RowsPlan p = rows_plan(qtype, act_dtype, M, N, K, workspace ? workspace_bytes : 0);
     float *ws = (float *)workspace;
     switch (qtype) {
     case QT_SYM_INT4: return launch_rows_q<QT_SYM_INT4>(x, w, bias, y, act_dtype, M, N, K, p, ws, st);

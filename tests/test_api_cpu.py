@@ -537,3 +537,11 @@ def test_a_workspace_of_the_size_asked_for_gets_the_plan_it_was_sized_for():
                 need = ggml.lowbit_linear_workspace_bytes(qtype, layout, dt, m, n, k, budget)
                 assert need <= budget
                 assert ggml.lowbit_linear_workspace_bytes(qtype, layout, dt, m, n, k, need) == need, (qtype, layout, dt, m, n, k, budget)
+
+
+def test_row_major_sizes_of_too_many_tiles_are_not_planned():
+    """Their number of tiles does not fit 32 bits: no workspace, where the plan divided by it."""
+    for m, n, k in [(1 << 30, 1 << 30, 4096), (1 << 29, 1 << 20, 1152), (1 << 27, 1 << 23, 128), (0x7fffffff, 0x7fffffff, 4096), (0x7fffffff, 64, 4096),
+                    (64, 0x7fffffff, 4096), (0x7fffff80, 1, 128)]:
+        for qtype in (2, 3, 8, 10, 15):
+            assert ggml.lowbit_linear_workspace_bytes(qtype, ggml.LAYOUT_GGML, ggml.DT_F16, m, n, k, 256 << 20) == 0, (qtype, m, n, k)
