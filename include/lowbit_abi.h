@@ -302,7 +302,8 @@ int lowbit_grouped_forward_ws(const void *x, const void *const *w, void *y, cons
  * shape.  plan4 = {256-row tiles (1) or 128-row tiles, of 256 or 128 weight rows (0), K splits, waves per workgroup,
  * workgroups per split}.
  * Every workgroup of a split launch owns one 256 x 256 fp32 tile of the workspace: splits x workgroups x 256 KiB
- * never exceeds lowbit_grouped_workspace_bytes.  No counterpart in the reference (its expert loop has no plan). */
+ * never exceeds lowbit_grouped_workspace_bytes.  LOWBIT_ESIZE for more tiles than a launch counts.  No counterpart in the reference
+ * (its expert loop has no plan). */
 int lowbit_grouped_forward_plan(int n_groups, int64_t total_rows, int64_t N, int64_t K, int have_workspace,
                                 size_t workspace_bytes, int *plan4);
 /* The gated MLP's first half for all experts in one launch: rows of group e of y [total_rows, N] =

@@ -153,17 +153,27 @@ GroupedPlan grouped_plan(int total_rows, int n_groups, int N, int K, size_t ws_b
     return plan;
 }
 
-// What launch_grouped_gemm would do for a plain grouped product: {tall, splits, waves, grid.x}.
-void grouped_plan_query(int total_rows, int n_groups, int N, int K, size_t ws_bytes, int out[4]) {
+// Sizes whose tiles (the narrowest: 128 rows by 64 columns) or workgroups 32-bit counts do not hold, or barely: neither planned nor
+// launched.
+static bool grouped_too_many(int total_rows, int n_groups, int N) {
+    return total_rows > 0x7fffff00 || N > 0x7fffff00 || n_groups > (1 << 24) ||
+           (int64_t)grouped_max_row_tiles(total_rows, n_groups, G_GM_TALL / 2) * ((N + G_GN / 4 - 1) / (G_GN / 4)) > (1 << 28);
+}
+
+// What launch_grouped_gemm would do for a plain grouped product: {tall, splits, waves, grid.x}.  False: it would refuse.
+bool grouped_plan_query(int total_rows, int n_groups, int N, int K, size_t ws_bytes, int out[4]) {
+    if (grouped_too_many(total_rows, n_groups, N)) return false;
     const GroupedPlan p = grouped_plan(total_rows, n_groups, N, K, ws_bytes);
     const int tiles_n = p.narrow ? (N + G_GN / 2 - 1) / (G_GN / 2) : (N + G_GN - 1) / G_GN;
     out[0] = p.tall;
     out[1] = p.splits;
     out[2] = p.tall || p.narrow ? p.waves : 4;
     out[3] = grouped_grid(grouped_max_row_tiles(total_rows, n_groups, p.tall ? G_GM_TALL : G_GM_TALL / 2), tiles_n, p.chunk);
+    return true;
 }
 
 size_t grouped_workspace_bytes(int total_rows, int n_groups, int N, int K) {
+    if (grouped_too_many(total_rows, n_groups, N)) return 0;
     const GroupedPlan p = grouped_plan(total_rows, n_groups, N, K, (size_t)-1);
     return p.splits > 1 ? (size_t)p.splits * tall_split_bytes(total_rows, n_groups, N) : 0;
 }
@@ -183,7 +193,7 @@ int launch_grouped_gemm(const void *x, const void *const *w, const void *const *
                         int n_groups, int total_rows, int qtype, int act_dtype, int N, int K, int act, void *workspace,
                         size_t workspace_bytes, hipStream_t st) {
     if (total_rows == 0 || N == 0 || n_groups == 0) return 0;
-    if (total_rows >= (1 << 24) || K >= (1 << 23)) return -3;        // 24-bit row offsets in the kernel
+    if (total_rows >= (1 << 24) || K >= (1 << 23) || grouped_too_many(total_rows, n_groups, N)) return -3;   // 24-bit row offsets in the kernel
     float *ws = (float *)workspace;
     const GroupedPlan plan = w_up ? grouped_mlp_plan(total_rows, n_groups, N, K)
                                   : grouped_plan(total_rows, n_groups, N, K, ws ? workspace_bytes : 0);

@@ -545,3 +545,13 @@ def test_row_major_sizes_of_too_many_tiles_are_not_planned():
                     (64, 0x7fffffff, 4096), (0x7fffff80, 1, 128)]:
         for qtype in (2, 3, 8, 10, 15):
             assert ggml.lowbit_linear_workspace_bytes(qtype, ggml.LAYOUT_GGML, ggml.DT_F16, m, n, k, 256 << 20) == 0, (qtype, m, n, k)
+
+
+def test_grouped_sizes_of_too_many_tiles_are_not_planned():
+    """Their number of tiles does not fit 32 bits: no workspace and no plan, where the plan divided by it."""
+    for groups, rows, n, k in [(64, 1 << 29, 1 << 30, 848177450), (1, 1 << 27, 1 << 30, 1 << 23), (8, 1 << 30, 1 << 20, 4096), (64, 1 << 28, 1 << 26, 128),
+                               (1, 0x7fffffff, 256, 4096), (1, 64, 0x7fffffff, 4096), (0x7fffffff, 1, 1, 128)]:
+        assert ggml.lowbit_grouped_workspace_bytes(groups, rows, n, k) == 0, (groups, rows, n, k)
+        with pytest.raises(RuntimeError):
+            ggml.lowbit_grouped_forward_plan(groups, rows, n, k, True, 1 << 30)
+    assert ggml.lowbit_grouped_forward_plan(4096, (1 << 24) - 1, 2048, 4096, True, 1 << 30)[0]
