@@ -26,10 +26,21 @@ static WideShape wide_shape(int qtype, int layout, int dt, int M, int N, int K) 
     const int rounds = (T + 255) / 256;
     const WideShape none = {0, 0};
     if (dt == DT_F32) {
-        // Two planes of x: 32 rows at most.  One pass at half the x traffic of the streaming kernel's (9 .. 16 rows on
-        // [28672 x 8192]: 86 -> 59 us) or in place of two (24 rows on [11008 x 4096]: 35.0 -> 31.3); up to 8 rows it loses.
+        // Two planes of x: 32 rows at most, and twice the x to read, to split and to write to LDS.  One pass at half the x traffic of
+        // the streaming kernel's (9 .. 16 rows on [28672 x 8192]: 86 -> 48) or in place of two; up to 8 rows it loses.
+        // As few workgroups as cover the weight in one round, as with 16-bit activations, now that splitting x is short enough for
+        // x to be shared by three tile rows (two, in two rounds, before): 9 / 24 rows on [11008 x 4096] in sym_int4 18.6 -> 12.8
+        // / 30.4 -> 17.7 us, on [9600 x 8192] 31.7 -> 19.6 / 55.3 -> 29.6.  Four tile rows have the registers for 16 rows
+        // of x only, and row-major weights need more instructions per tile: [14336 x 4096], 9 rows, four / two tile rows 15.2 / 17.2
+        // us.  Beyond 1024 tile rows three with four waves, several workgroups per CU ([18000 x 1024], 9 / 24 rows: 10.3 -> 8.2 / 15.1 ->
+        // 11.8; eight waves 9.9 / 13.9).  12 waves up to 12 rows and one tile row, where the walk's latency counts ([4096 x 4096]
+        // in sym_int4, 9 / 12 / 16 rows, 8 waves / 12: 9.3 / 8.4, 9.4 / 8.9, 9.4 / 9.1 us; [2048 x 3072] at 16 rows 7.6 / 8.2;
+        // fp8_e4m3 on [4096 x 6144] at 12 rows 11.7 / 12.7).
         if (M <= 8 || M > 32) return none;
-        return {rounds > 1 ? 2 : 1, MB == 2 && rounds > 1 ? 4 : 8};
+        const bool int4 = qtype == QT_SYM_INT4 || qtype == QT_ASYM_INT4;
+        if (rounds <= 3) return {rounds, rounds == 1 && M <= 12 && int4 ? 12 : 8};
+        if (rounds == 4) return layout == LAYOUT_TILED && MB == 1 ? WideShape{4, 8} : WideShape{2, 4};
+        return {3, 4};
     }
     if (M > 64) return none;
     if (layout == LAYOUT_GGML) {

@@ -31,7 +31,7 @@ namespace lowbit {
 // wide_max_waves: what gemv_wide.hip asks for at most, and with it the registers a wave may have (256 at 8, 168 at
 // 12).  Four tiles in the 128 that 16 waves leave spilled: 16 rows on [14336 x 4096], asym_int4 bf16 20.6 ->
 // 12.7 us, sym_int8 23.3 -> 16.0.
-constexpr int wide_max_waves(int mb, int tiles, bool f32) { return !f32 && mb == 1 && tiles == 1 ? 12 : 8; }
+constexpr int wide_max_waves(int mb, int tiles) { return mb == 1 && tiles == 1 ? 12 : 8; }
 
 // 16-byte chunks from the first of four 16-bit rows of x to row xrow (0 .. 3) of them, or to the last row where fewer than xrow are
 // left; K is a multiple of 128.  (In elements three rows are past 32 bits from K = 1.4 * 10^9 on; a 64-bit offset costs 0.5 %
@@ -48,7 +48,7 @@ template <int QT, typename AT, int MB, int R, bool F32, bool ROWS, bool DUAL> co
 
 // CROWD: the fused form without PEEL, see launch_wide_r
 template <int QT, typename AT, int MB, int R, bool F32, bool ROWS, bool DUAL, bool CROWD = false>
-__global__ __launch_bounds__(64 * wide_max_waves(MB, DUAL ? 2 * R : R, F32)) void gemv_wide_kernel(
+__global__ __launch_bounds__(64 * wide_max_waves(MB, DUAL ? 2 * R : R)) void gemv_wide_kernel(
     const void *__restrict__ x_, const uint8_t *__restrict__ w, const uint8_t *__restrict__ w_up, const void *__restrict__ bias_,
     void *__restrict__ y_, int M, int N, int K, int act) {
     using F = Fmt<QT>;
@@ -126,7 +126,7 @@ __global__ __launch_bounds__(64 * wide_max_waves(MB, DUAL ? 2 * R : R, F32)) voi
             };
             if constexpr (F32) {
                 u32x4 hi, lo;
-                split_f32(past ? none : xv[2 * i], past ? none : xv[2 * i + 1], hi, lo);
+                split_f32<false>(past ? none : xv[2 * i], past ? none : xv[2 * i + 1], hi, lo);
                 one(xs + m * 256, hi);
                 one(xs + PLANE + m * 256, lo);
             } else {
@@ -325,7 +325,7 @@ inline WideRoom wide_room(const void *peel, const void *crowd, size_t lds) {
 template <int QT, typename AT, int MB, int R, bool F32, bool ROWS, bool DUAL>
 static int launch_wide_r(const void *x, const void *w, const void *w_up, const void *bias, void *y, int M, int N, int K, int act,
                          int waves, hipStream_t st) {
-    constexpr int XBYTES = 16 * MB * 256 * (F32 ? 2 : 1), LDS = 128 * 1024, MOST = wide_max_waves(MB, DUAL ? 2 * R : R, F32);
+    constexpr int XBYTES = 16 * MB * 256 * (F32 ? 2 : 1), LDS = 128 * 1024, MOST = wide_max_waves(MB, DUAL ? 2 * R : R);
     auto kern = gemv_wide_kernel<QT, AT, MB, R, F32, ROWS, DUAL>;
     const int G = (K + TILE_COLS - 1) / TILE_COLS;
     int wv = LDS / XBYTES;
@@ -353,8 +353,8 @@ template <int QT, typename AT, int MB, bool F32, bool ROWS>
 static int launch_wide_mb(const void *x, const void *w, const void *bias, void *y, int M, int N, int K, const WideShape &s, hipStream_t st) {
     if (s.r == 1) return launch_wide_r<QT, AT, MB, 1, F32, ROWS, false>(x, w, nullptr, bias, y, M, N, K, 0, s.waves, st);
     if (s.r == 2) return launch_wide_r<QT, AT, MB, 2, F32, ROWS, false>(x, w, nullptr, bias, y, M, N, K, 0, s.waves, st);
-    if constexpr (!F32) {
-        if (s.r == 3) return launch_wide_r<QT, AT, MB, 3, F32, ROWS, false>(x, w, nullptr, bias, y, M, N, K, 0, s.waves, st);
+    if (s.r == 3) return launch_wide_r<QT, AT, MB, 3, F32, ROWS, false>(x, w, nullptr, bias, y, M, N, K, 0, s.waves, st);
+    if constexpr (!F32 || (MB == 1 && !ROWS)) {
         if constexpr (MB < 4)
             if (s.r == 4) return launch_wide_r<QT, AT, MB, 4, F32, ROWS, false>(x, w, nullptr, bias, y, M, N, K, 0, s.waves, st);
     }

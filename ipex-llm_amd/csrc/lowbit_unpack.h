@@ -252,15 +252,16 @@ template <typename AT> __device__ inline typename Vec8<AT>::type ones8() {
     return r;
 }
 
-// Eight floats -> their bf16 values and those of what the rounding dropped.  inf / nan stay in the first plane only.
-__device__ inline void split_f32(const u32x4 &a, const u32x4 &b, u32x4 &hi, u32x4 &lo) {
+// Eight floats -> their bf16 values and those of what the rounding dropped.  inf / nan stay in the first plane only, or, without KEEP,
+// make NaN of the second: three of six instructions less, for kernels that compute a result that is not finite once more (below).
+template <bool KEEP = true> __device__ inline void split_f32(const u32x4 &a, const u32x4 &b, u32x4 &hi, u32x4 &lo) {
     bf16x8 h, l;
 #pragma unroll
     for (int i = 0; i < 8; i++) {
         const float v = __builtin_bit_cast(float, i < 4 ? a[i] : b[i - 4]);
         h[i] = (__bf16)v;                                   // round to nearest even
         const float r = v - (float)h[i];                    // exact: both share the leading bits
-        l[i] = (r - r) == 0.0f ? (__bf16)r : (__bf16)0.0f;
+        l[i] = !KEEP || (r - r) == 0.0f ? (__bf16)r : (__bf16)0.0f;
     }
     hi = __builtin_bit_cast(u32x4, h);
     lo = __builtin_bit_cast(u32x4, l);

@@ -5,7 +5,8 @@ import pytest
 import torch
 
 import lowbit_oracle as orc
-from gpu_util import ALL, FP8, NF4, acts, dev_dequantize, dev_quantize, weights
+import ipex_llm.ggml.model.llama.llama_cpp as ggml
+from gpu_util import ALL, FP8, NF4, acts, dev_dequantize, dev_quantize, stream, weights
 from ipex_llm.transformers.low_bit_linear import mlp_forward_xpu
 from ipex_llm.transformers.models.utils import SILU
 from test_linear_gpu import GGML, TILED, _check, classes
@@ -37,6 +38,36 @@ def test_float32_activations(qtype, layout, m, n, k):
     if qtype == FP8:
         k = (k + 127) // 128 * 128
     _check(qtype, torch.float32, layout, m, n, k, m % 2 == 0, 900 * m + n)
+
+
+# tile rows that three and four do not divide, 12 waves with fewer and more groups, several workgroups of four waves per CU
+@pytest.mark.parametrize("qtype", ALL)
+@pytest.mark.parametrize("layout,m,n,k", [(TILED, 12, 48, 1664), (TILED, 9, 8224, 256), (TILED, 32, 8240, 1152), (TILED, 16, 12336, 1152),
+                                          (TILED, 17, 12336, 640), (TILED, 10, 16400, 640), (TILED, 24, 16416, 128), (GGML, 12, 33, 1728),
+                                          (GGML, 9, 8215, 1088), (GGML, 31, 8231, 192), (GGML, 16, 12299, 320), (GGML, 18, 16401, 320)])
+def test_float32_activations_shared_by_tile_rows(qtype, layout, m, n, k):
+    if qtype == FP8:
+        k = (k + 127) // 128 * 128
+    _check(qtype, torch.float32, layout, m, n, k, m % 2 == 0, 950 * m + n)
+
+
+@pytest.mark.parametrize("qtype", ALL)
+@pytest.mark.parametrize("layout,m,n,k", [(TILED, 9, 48, 256), (TILED, 20, 8224, 128), (TILED, 16, 12336, 128), (GGML, 17, 8215, 128)])
+def test_float32_activations_beyond_bfloat16(qtype, layout, m, n, k):
+    """Infinities, a NaN, and a finite value that rounds to an infinity in bfloat16: what its second plane would be is not used."""
+    w, x = weights(m + n, (n, k)), acts(m, m, k, torch.float32)
+    x[0, 5], x[m // 2, k - 3], x[1, 7], x[2, 9] = float("inf"), -float("inf"), float("nan"), 3.4e38
+    blob, y = dev_quantize(w, qtype, layout), torch.empty((m, n), dtype=torch.float32, device="cuda")
+    xd = x.cuda()
+    ggml.lowbit_linear(xd.data_ptr(), blob.data_ptr(), None, y.data_ptr(), qtype, layout, ggml.DT_F32, m, n, k, None, 0, stream())
+    got = y.cpu().numpy()
+    dense = orc.dequantize(orc.quantize(w, qtype), qtype, (n, k)).astype(np.float64)
+    with np.errstate(all="ignore"):
+        want = (x.double().numpy() @ dense.T).astype(np.float32)
+    assert (classes(got) == classes(want)).all()
+    assert np.isfinite(want[2]).all() and (classes(want[0]) > 1).any()
+    # float32 sums of products in float32
+    assert np.abs(got[2] - want[2]).max() <= k * 2.0 ** -23 * 3.4e38 * np.abs(dense[:, 9]).max()
 
 
 @pytest.mark.parametrize("qtype", ALL)
