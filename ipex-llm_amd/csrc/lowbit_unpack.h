@@ -225,8 +225,7 @@ template <int QT, typename AT, bool F32, bool ROWS> struct Operand {
     // a step's product; al: what x's first plane leaves (F32).  The largest first: an MFMA drops more of a small sum that it
     // is given beside large products than of small products beside a large sum (fp16, 8640 columns: 1.48 in a thousand not
     // the nearest result the other way round, 1.14 this way).  The smallest parts of both are below fp32.
-    __device__ static f32x4 product(const V8 &a, const V8 &al, const V8 (&b)[PARTS]) {
-        f32x4 p = {0.0f, 0.0f, 0.0f, 0.0f};
+    __device__ static f32x4 product(const V8 &a, const V8 &al, const V8 (&b)[PARTS], f32x4 p = {0.0f, 0.0f, 0.0f, 0.0f}) {
 #pragma unroll
         for (int part = 0; part < PARTS; part++) {
             p = mfma16(a, b[part], p);
