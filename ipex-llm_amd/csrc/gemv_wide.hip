@@ -19,12 +19,17 @@ int launch_wide_mlp_q(const void *x, const void *wg, const void *wu, void *y, in
 // R = 4 and several workgroups share a CU).
 // Every workgroup reads all of x from L2, MB * G * 4 KB: beyond about 0.8 MB (MB * G = 192) the ring kernel and the K splits
 // of the tiled GEMM win, which divide x as well ([4096 x 11008] at 64 rows: 24.2 us against 31).  Beyond 1024 tile rows
-// there are several rounds of workgroups and x comes again in each: only 17 .. 32 rows still pay ([28672 x 8192] at 48
+// there are several rounds of workgroups and x comes again in each: only up to 32 rows still pay ([28672 x 8192] at 48
 // rows 106 against 96 us of the GEMM).
 static WideShape wide_shape(int qtype, int layout, int dt, int M, int N, int K) {
     const int T = (N + TILE_ROWS - 1) / TILE_ROWS, G = (K + TILE_COLS - 1) / TILE_COLS, MB = (M + 15) / 16;
     const int rounds = (T + 255) / 256;
     const WideShape none = {0, 0};
+    // 5 .. 8 rows of x and a weight that three tile rows a workgroup cover in one round, where the streaming kernel's workgroups of
+    // one or two read x more often: from 24 groups on (8 rows, 16-bit activations: 0.79 .. 0.95 of its time on 9728 .. 12288 rows
+    // of 4096 and 8192 columns, sym_int8 on [11008 x 4096] 14.2 -> 11.3 us, asym_int4 in bf16 10.9 -> 9.2, float32 sym_int4 15.2 -> 12.8;
+    // 1.0 .. 1.07 of it with 8 groups).
+    const bool shared_by_three = M > 4 && M <= 8 && layout == LAYOUT_TILED && rounds == 3 && G >= 24;
     if (dt == DT_F32) {
         // Two planes of x: 32 rows at most, and twice the x to read, to split and to write to LDS.  One pass at half the x traffic of
         // the streaming kernel's (9 .. 16 rows on [28672 x 8192]: 86 -> 48) or in place of two; up to 8 rows it loses.
@@ -36,7 +41,7 @@ static WideShape wide_shape(int qtype, int layout, int dt, int M, int N, int K) 
         // 11.8; eight waves 9.9 / 13.9).  12 waves up to 12 rows and one tile row, where the walk's latency counts ([4096 x 4096]
         // in sym_int4, 9 / 12 / 16 rows, 8 waves / 12: 9.3 / 8.4, 9.4 / 8.9, 9.4 / 9.1 us; [2048 x 3072] at 16 rows 7.6 / 8.2;
         // fp8_e4m3 on [4096 x 6144] at 12 rows 11.7 / 12.7).
-        if (M <= 8 || M > 32) return none;
+        if (M > 32 || (M <= 8 && !shared_by_three)) return none;
         const bool int4 = qtype == QT_SYM_INT4 || qtype == QT_ASYM_INT4;
         if (rounds <= 3) return {rounds, rounds == 1 && M <= 12 && int4 ? 12 : 8};
         if (rounds == 4) return layout == LAYOUT_TILED && MB == 1 ? WideShape{4, 8} : WideShape{2, 4};
@@ -45,18 +50,42 @@ static WideShape wide_shape(int qtype, int layout, int dt, int M, int N, int K) 
     if (M > 64) return none;
     if (layout == LAYOUT_GGML) {
         // From 5 rows on: the streaming kernel reads unaligned weights in smaller pieces ([8008 x 8256], sym_int4, 8 rows:
-        // 19.4 -> 15.2 us; 16 rows of [4001 x 2112] 7.1 -> 4.6).  Not fp8_e4m3, whose rows are whole and aligned, and not
-        // beyond 1024 tile rows, up to 16 rows.  17 .. 64 rows: against the row-major GEMM, whose 64-column tiles leave most
+        // 19.4 -> 15.2 us; 16 rows of [4001 x 2112] 7.1 -> 4.6).  Not fp8_e4m3, whose rows are whole and aligned, up to 16 rows.  17 .. 64 rows: against the row-major GEMM, whose 64-column tiles leave most
         // CUs idle at that size ([4001 x 2112], 24 / 64 rows: 11.4 -> 5.8 / 14.8 -> 8.6 us).
         const bool int4 = qtype == QT_SYM_INT4 || qtype == QT_ASYM_INT4;
         if (MB == 1) {
+            // Beyond 1024 tile rows 9 .. 16 rows and 24 groups or more (9 / 16 rows on [17001 x 4096] 0.72 .. 0.85 / 0.75 .. 0.85 of
+            // the streaming kernel's time over the formats, on [50001 x 4096] 0.81 .. 0.95 / 0.81 .. 0.98, on [17001 x 1024] 0.88 ..
+            // 1.05); between 1537 and 2048, where that kernel's rounds come out even, four waves with four tile rows, and not fp8_e4m3
+            // (1.03), nor asym_int4 up to 12 rows (9 / 16 rows on [32003 x 4096] 1.04 / 0.88; sym_int4 0.97 / 0.92).
+            if (T > 1024 && M > 8 && G >= 24) {
+                if (T <= 1536 || T > 2048) return {2, 8};
+                if (qtype != QT_FP8_E4M3 && (qtype != QT_ASYM_INT4 || M > 12)) return {4, 4};
+            }
             if (M <= 4 || T > 1024 || qtype == QT_FP8_E4M3) return none;
             if (rounds == 1) return {1, 12};
             return {rounds == 3 && !int4 ? 1 : rounds, 8};                  // (more registers per tile: a third of them waits)
         }
         if (MB * G > 200 || (MB == 4 && T > 512) || (T > 1024 && (MB > 2 || qtype == QT_SYM_INT8))) return none;
     } else {
-        if (M <= 8 || (MB == 1 && T > 1024) || (MB > 1 && MB * G > 192) || (MB == 4 && T > 768) || (T > 1024 && MB > 2)) return none;
+        // Up to 16 rows and beyond 1024 tile rows: workgroups of four waves, two to a CU, and as many tile rows as let 512 of them cover
+        // the weight, in several rounds three.  9 and 16 rows, over the formats and types: 0.74 .. 0.96 of the streaming kernel's time on
+        // 17008 .. 24576 weight rows (sym_int4 on [22016 x 4096] 17.6 -> 14.2 us), 0.86 .. 1.0 on [28672 x 4096] (level with 8 groups, not
+        // taken), 0.85 .. 0.95 on 36000 rows.  5 .. 8 rows: asym_int4 and sym_int8, whose unpacking is what the streaming kernel spends its time
+        // on there (0.86 .. 0.92 on [20480 x 4096] and [24576 x 4096], 1.0 .. 1.08 on [17008 x 4096]; the other formats 0.97 .. 1.06).
+        const WideShape many = T <= 1536 || T > 2048 ? WideShape{3, 4} : WideShape{4, 4};
+        if (M <= 8) {
+            if (shared_by_three) return {3, 8};
+            // two tile rows from 64 groups on (8 rows on [5008 x 11008] 0.86 .. 0.94; just above 256 tile rows half of the CUs would
+            // have nothing, 6 rows on [4272 x 8192] in fp8_e4m3 1.08), 512 of them in the 8-bit formats only (0.91 .. 0.93,
+            // the others 0.99 .. 1.04)
+            const bool eight_bit = qtype == QT_SYM_INT8 || qtype == QT_FP8_E4M3;
+            if (M > 4 && rounds == 2 && T >= 304 && G >= 64 && (T < 512 || eight_bit)) return {2, 8};
+            if (M > 4 && T >= 1216 && G >= 24 && (qtype == QT_ASYM_INT4 || qtype == QT_SYM_INT8)) return many;
+            return none;
+        }
+        if (MB == 1 && T > 1024) return T > 1536 && T <= 2048 && G < 24 ? none : many;
+        if ((MB > 1 && MB * G > 192) || (MB == 4 && T > 768) || (T > 1024 && MB > 2)) return none;
     }
     if (T > 1024) return {4, 4};
     return {rounds, MB == 1 && rounds == 1 ? 12 : 8};

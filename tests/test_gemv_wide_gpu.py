@@ -6,7 +6,7 @@ import torch
 
 import lowbit_oracle as orc
 import ipex_llm.ggml.model.llama.llama_cpp as ggml
-from gpu_util import ALL, FP8, NF4, acts, dev_dequantize, dev_quantize, stream, weights
+from gpu_util import ALL, DT, FP8, NF4, acts, dev_dequantize, dev_quantize, stream, weights
 from ipex_llm.transformers.low_bit_linear import mlp_forward_xpu
 from ipex_llm.transformers.models.utils import SILU
 from test_linear_gpu import GGML, TILED, _check, classes
@@ -38,6 +38,33 @@ def test_float32_activations(qtype, layout, m, n, k):
     if qtype == FP8:
         k = (k + 127) // 128 * 128
     _check(qtype, torch.float32, layout, m, n, k, m % 2 == 0, 900 * m + n)
+
+
+# where 5 to 16 rows go to this kernel: around 512, 768, 1024, 1536 and 2048 tile rows, 24 and 64 groups
+@pytest.mark.parametrize("qtype,dtype", [(2, torch.float16), (3, torch.bfloat16), (8, torch.float16), (10, torch.bfloat16), (15, torch.bfloat16)])
+@pytest.mark.parametrize("layout,m,n,k", [(TILED, 5, 8208, 3072), (TILED, 8, 12288, 3072), (TILED, 7, 4112, 8192), (TILED, 8, 8192, 8192),
+                                          (TILED, 6, 19456, 3072), (TILED, 8, 24592, 3072), (TILED, 9, 16400, 256), (TILED, 16, 24576, 128),
+                                          (TILED, 12, 24592, 3072), (TILED, 9, 32784, 128), (GGML, 9, 16401, 3072), (GGML, 16, 24577, 3072),
+                                          (GGML, 13, 32769, 3072)])
+def test_few_rows_of_many_tile_rows(qtype, dtype, layout, m, n, k):
+    w = np.random.default_rng(m + n).standard_normal((n, k), dtype=np.float32) * 0.02
+    blob, x = dev_quantize(w, qtype, layout), acts(m, m, k, dtype).cuda()
+    y = torch.full((m + 1, n), float("nan"), dtype=dtype, device="cuda")
+    x_inf = x.clone()
+    x_inf[0, 5], x_inf[m - 1, k - 3] = float("inf"), -float("inf")
+    dense = dev_dequantize(blob, qtype, n, k, layout, torch.float32).double()
+    ggml.lowbit_linear(x.data_ptr(), blob.data_ptr(), None, y.data_ptr(), qtype, layout, DT[dtype], m, n, k, None, 0, stream())
+    want, eps = x.double() @ dense.t(), torch.finfo(dtype).eps
+    # one rounding, those of fp32 sums over k / 32 blocks of 32 products each, of codes that carry 17 times their value at most, and of
+    # nf4's levels to x's type
+    err = 2.0 ** -24 * 2 * 17 * (k / 32 + 33) + (eps / 2 if qtype == NF4 else 0.0)
+    bound = want.abs() * eps / 2 + x.double().abs().sum(1, keepdim=True) * dense.abs().amax(1) * err + torch.finfo(dtype).smallest_normal
+    assert ((y[:m].double() - want).abs() <= bound).all() and torch.isnan(y[m]).all()
+    if m > 8 or layout == GGML:                            # (fewer rows may go to the streaming kernel, which gives NaN for some of these)
+        ggml.lowbit_linear(x_inf.data_ptr(), blob.data_ptr(), None, y.data_ptr(), qtype, layout, DT[dtype], m, n, k, None, 0, stream())
+        want = torch.where(dense[:, 5] == 0, torch.nan, torch.copysign(torch.full_like(dense[:, 5], torch.inf), dense[:, 5]))
+        assert torch.equal(torch.nan_to_num(y[0].float(), nan=7.0, posinf=1.0, neginf=-1.0),
+                           torch.nan_to_num(want.float(), nan=7.0, posinf=1.0, neginf=-1.0))
 
 
 # tile rows that three and four do not divide, 12 waves with fewer and more groups, several workgroups of four waves per CU
