@@ -29,7 +29,9 @@ int launch_dequantize(const void *w, void *out, int qtype, int64_t N, int64_t K,
 int launch_gemv(const void *x, const void *w, const void *bias, void *y, int qtype, int layout, int act_dtype, int M, int N, int K,
                 int waves, hipStream_t st);
 int launch_gemv_wide(const void *x, const void *w, const void *bias, void *y, int qtype, int layout, int act_dtype, int M, int N, int K,
-                     hipStream_t st);
+                     bool batch, hipStream_t st);
+double gemv_wide_batch_us(int qtype, int layout, int M, int N, int K);
+double gemm_rows_us(int qtype, int act_dtype, int M, int N, int K);
 bool gemv_wide_applies(int qtype, int layout, int act_dtype, int M, int N, int K);
 int launch_mlp_wide(const void *x, const void *wg, const void *wu, void *y, int qtype, int act_dtype, int M, int N, int K, int act,
                     hipStream_t st);
@@ -284,9 +286,10 @@ static double gemv_time_us(int qtype, int64_t M, int64_t N, int64_t K) {
     return 0.9 * t;
 }
 
-// which kernel, and for PLAN_GEMM_SPLIT into how many K splits
+// which kernel, and for PLAN_GEMM_SPLIT into how many K splits; *us_out: its estimate, 0 where none was made
 static int plan_forward(int qtype, int layout, int64_t M, int64_t N, int64_t K, bool have_ws, size_t workspace_bytes,
-                        bool y_aligned8, int *splits_out, bool linear = false, int act_dtype = LOWBIT_DT_F16) {
+                        bool y_aligned8, int *splits_out, bool linear = false, int act_dtype = LOWBIT_DT_F16, double *us_out = nullptr) {
+    if (us_out) *us_out = 0.0;
     if (splits_out) *splits_out = 1;
     if (M <= 16 || layout != LOWBIT_LAYOUT_TILED || !y_aligned8) return PLAN_GEMV;            // the MFMA kernels store 8 bytes and more
     if (M > 0x7fffffff || N > 0x7fffffff || K > 0x7fffffff || K < 128) return PLAN_GEMM;     // reports the error
@@ -306,8 +309,35 @@ static int plan_forward(int qtype, int layout, int64_t M, int64_t N, int64_t K, 
         const double t = ring_time_us((int)M, (int)N, (int)K, qtype, true);
         if (t < best_t) { best_t = t; best = PLAN_RING; }
     }
+    if (us_out) *us_out = best_t;
     if (best == PLAN_GEMM_SPLIT && splits_out) *splits_out = splits;
     return best;
+}
+
+// Whether lowbit_linear takes the one-pass kernel, 16-bit activations: what gemv_wide.hip names up to 64 rows, and otherwise where its
+// estimate is 5 % below that of the kernel that else takes the size.  Those of the tiled kernels are 0.82 to 0.91 of what they take at 65
+// rows and more on weights so small: fitted to 700 random sizes (M = 65 .. 900, N to 16384, K to 14000), 5 to 10 % rms.  Of these and of
+// 250 row-major ones 533 and 150 change kernel, 0.68 and 0.65 of the time, three of them more than 3 % longer, 1.10 at worst.  Does not depend
+// on the workspace that a call brings: the other kernel's is taken to be there.
+static bool one_pass_applies(int qtype, int layout, int act_dtype, int64_t M, int64_t N, int64_t K) {
+    const int m = (int)M, n = (int)N, k = (int)K;
+    if (gemv_wide_applies(qtype, layout, act_dtype, m, n, k)) return true;
+    const double us = gemv_wide_batch_us(qtype, layout, m, n, k);
+    if (us <= 0.0) return false;
+    double other = 0.0;
+    if (layout == LOWBIT_LAYOUT_GGML) {
+        other = gemm_rows_us(qtype, act_dtype, m, n, k);
+    } else {
+        plan_forward(qtype, layout, M, N, K, true, (size_t)256 << 20, true, nullptr, true, act_dtype, &other);
+        if (other > 0.0) switch (qtype) {
+        case LOWBIT_QT_SYM_INT4: other = 2.40 + 0.946 * other; break;
+        case LOWBIT_QT_ASYM_INT4: other = 2.73 + 0.928 * other; break;
+        case LOWBIT_QT_SYM_INT8: other = 2.61 + 0.854 * other; break;
+        case LOWBIT_QT_NF4: other = 3.32 + 0.920 * other; break;
+        default: other = 2.24 + 0.877 * other; break;
+        }
+    }
+    return us < 0.95 * other;
 }
 
 static size_t plan_workspace(int plan, int splits, int64_t M, int64_t N, int64_t K) {
@@ -370,11 +400,12 @@ static int forward_any(const char *what, const void *x, const void *w, const voi
     const int m = (int)M, n = (int)N, k = (int)K;
     hipStream_t st = (hipStream_t)stream;
     int splits = 1, rc = 0;
-    const int plan = linear && gemv_wide_applies(qtype, layout, act_dtype, m, n, k) ? PLAN_GEMV
+    const bool one_pass = linear && one_pass_applies(qtype, layout, act_dtype, M, N, K);
+    const int plan = one_pass ? PLAN_GEMV
         : plan_forward(qtype, layout, M, N, K, workspace != nullptr, workspace_bytes, !(((uintptr_t)y | (uintptr_t)bias) & 7), &splits, linear, act_dtype);
     // (a y off the 8-byte boundaries keeps the streaming kernel's passes, and so its bits, at the entry points that say so)
     if (plan == PLAN_GEMV && (linear || !(((uintptr_t)y) & 7))) {
-        rc = launch_gemv_wide(x, w, bias, y, qtype, layout, act_dtype, m, n, k, st);
+        rc = launch_gemv_wide(x, w, bias, y, qtype, layout, act_dtype, m, n, k, one_pass, st);
         if (rc <= 0) return check_launch(rc, what);
     }
     if (layout == LOWBIT_LAYOUT_GGML && M > 16)          // (up to 16 rows: one streaming pass)
@@ -399,7 +430,7 @@ int lowbit_forward_ws(const void *x, const void *w, void *y, int qtype, int layo
     return forward_any("lowbit_forward_ws", x, w, nullptr, y, qtype, layout, act_dtype, M, N, K, workspace, workspace_bytes, stream);
 }
 
-// ---- fp32 activations: the one-pass kernel in passes of 32 rows, the streaming kernel for a rest of up to 8
+// ---- fp32 activations: the one-pass kernel, above 32 rows (64 on small weights) in passes of 32, the streaming kernel for a rest of up to 8
 static int forward_f32(const char *what, const float *x, const void *w, const float *bias, float *y, int qtype, int layout,
                        int64_t M, int64_t N, int64_t K, void *stream) {
     if (int rc = check_weight_shape(what, qtype, N, K, layout)) return rc;
@@ -408,11 +439,15 @@ static int forward_f32(const char *what, const float *x, const void *w, const fl
     if (!x || !w || !y || !aligned16(x) || !aligned16(w) || (((uintptr_t)y | (uintptr_t)bias) & 3))
         return fail(LOWBIT_EARG, "%s: null or misaligned pointer (x, w: 16 bytes)", what);
     if (K % 8) return fail(LOWBIT_ESHAPE, "%s: K must be a multiple of 8", what);
+    if (M > 32 && M <= 64) {                             // in one launch, where the weight is small enough
+        const int rc = launch_gemv_wide(x, w, bias, y, qtype, layout, LOWBIT_DT_F32, (int)M, (int)N, (int)K, false, (hipStream_t)stream);
+        if (rc <= 0) return check_launch(rc, what);
+    }
     for (int64_t m0 = 0; m0 < M; m0 += 32) {
         const int m = (int)(M - m0 < 32 ? M - m0 : 32), n = (int)N, k = (int)K;
         const float *xp = x + m0 * K;
         float *yp = y + m0 * N;
-        int rc = launch_gemv_wide(xp, w, bias, yp, qtype, layout, LOWBIT_DT_F32, m, n, k, (hipStream_t)stream);
+        int rc = launch_gemv_wide(xp, w, bias, yp, qtype, layout, LOWBIT_DT_F32, m, n, k, false, (hipStream_t)stream);
         if (rc > 0) rc = launch_gemv(xp, w, bias, yp, qtype, layout, LOWBIT_DT_F32, m, n, k, 0, (hipStream_t)stream);
         if (rc) return check_launch(rc, what);
     }
@@ -422,7 +457,7 @@ static int forward_f32(const char *what, const float *x, const void *w, const fl
 size_t lowbit_linear_workspace_bytes(int qtype, int layout, int dtype, int64_t M, int64_t N, int64_t K, size_t max_bytes) {
     if (dtype == LOWBIT_DT_F32 || M <= 16) return 0;     // one pass over the weights, or one per 32 rows
     if (!qk_size(qtype) || N <= 0 || K <= 0 || M > 0x7fffffff || N > 0x7fffffff || K > 0x7fffffff) return 0;
-    if (gemv_wide_applies(qtype, layout, dtype, (int)M, (int)N, (int)K)) return 0;       // one pass, as forward_any chooses
+    if (one_pass_applies(qtype, layout, dtype, M, N, K)) return 0;       // as forward_any chooses
     if (layout != LOWBIT_LAYOUT_GGML) return workspace_for(qtype, layout, M, N, K, max_bytes, true, dtype);
     return gemm_rows_workspace_bytes(qtype, dtype, (int)M, (int)N, (int)K, max_bytes);
 }

@@ -91,6 +91,68 @@ static WideShape wide_shape(int qtype, int layout, int dt, int M, int N, int K) 
     return {rounds, MB == 1 && rounds == 1 ? 12 : 8};
 }
 
+// What a launch takes whose workgroups are one per CU at most, 8 waves each, with r tile rows and 16 * mb rows of x to a workgroup:
+// microseconds, fitted to 1250 sizes (M = 17 .. 900, N to 16384, K to 14000) in up to three shapes each, 6 to 10 % rms.  A launch; per
+// 1024 columns what goes with the groups, with x, with the weights and with their products; the sums; x out of L2.
+static double wide_us(int qtype, int layout, int r, int mb, int M, int T, int G) {
+    static const double fit[2][5][7] = {                    // row-major, tiled; sym_int4, asym_int4, sym_int8, nf4, fp8_e4m3
+        {{2.680, 0.076, 0.200, 0.466, 0.032, 0.249, 0.020}, {2.423, 0.326, 0.100, 0.390, 0.114, 0.296, 0.042},
+         {2.388, 0.297, 0.040, 0.653, 0.088, 0.299, 0.036}, {3.236, 0.000, 0.000, 0.814, 0.158, 0.110, 0.057},
+         {2.751, 0.133, 0.065, 0.365, 0.125, 0.135, 0.028}},
+        {{2.975, 0.190, 0.075, 0.163, 0.126, 0.127, 0.038}, {3.089, 0.058, 0.118, 0.221, 0.132, 0.078, 0.038},
+         {2.974, 0.087, 0.177, 0.415, 0.074, 0.094, 0.031}, {2.817, 0.170, 0.081, 0.279, 0.061, 0.160, 0.043},
+         {3.052, 0.223, 0.102, 0.288, 0.096, 0.065, 0.034}}};
+    const double(&f)[7] = fit[layout == LAYOUT_TILED][qtype == QT_SYM_INT4 ? 0 : qtype == QT_ASYM_INT4 ? 1 : qtype == QT_SYM_INT8 ? 2 : qtype == QT_NF4 ? 3 : 4];
+    const double wgs = (double)((T + r - 1) / r) * ((M + 16 * mb - 1) / (16 * mb));
+    return f[0] + (G + 7) / 8 * (f[1] + f[2] * mb + f[3] * r + f[4] * r * mb) + f[5] * r * mb + f[6] * wgs / 256 * G * mb;
+}
+
+// Rows of x dealt to several workgroups: so many rows and tile rows to each that the workgroups are one per CU at most and the estimate is
+// the shortest; r = 0: there is no such shape.  (r * mb: more than nine products of 16 x 16, six in asym_int4, spill.)
+static WideShape wide_batch_shape(int qtype, int layout, int M, int N, int K, double *us) {
+    WideShape best = {0, 0};
+    if (M <= 16 || M > 1024 || K > 16384) return best;
+    const int T = (N + TILE_ROWS - 1) / TILE_ROWS, G = (K + TILE_COLS - 1) / TILE_COLS;
+    for (int r = 1; r <= 4; r++)
+        for (int mb = 1; mb <= 4 && r * mb <= (qtype == QT_ASYM_INT4 ? 6 : 9); mb++) {
+            if ((int64_t)((T + r - 1) / r) * ((M + 16 * mb - 1) / (16 * mb)) > 256) continue;
+            const double t = wide_us(qtype, layout, r, mb, M, T, G);
+            if (!best.r || t < *us) {
+                best = {r, 8, mb};
+                *us = t;
+            }
+        }
+    return best;
+}
+
+// Microseconds with rows dealt that way, 0 where there is no such shape: for the choice between this and the other kernels.  (What it takes
+// the place of there: the K splits, half tiles and narrow tiles of the GEMMs, whose few tiles leave CUs idle or walk K at the latency of a
+// step, and their sums.  128 rows on [2048 x 2048] 15.2 -> 7.0 us, 72 on [4096 x 4096] 19.3 -> 12.4, 217 on [1001 x 1024] row-major
+// 11.3 -> 6.2, averages of the formats.)
+double gemv_wide_batch_us(int qtype, int layout, int M, int N, int K) {
+    double us = 0.0;
+    return wide_batch_shape(qtype, layout, M, N, K, &us).r ? us : 0.0;
+}
+
+// batch: also the sizes that wide_shape leaves to other kernels
+static WideShape wide_shape_for(int qtype, int layout, int dt, int M, int N, int K, bool batch) {
+    const WideShape s = wide_shape(qtype, layout, dt, M, N, K);
+    const int T = (N + TILE_ROWS - 1) / TILE_ROWS, MB = (M + 15) / 16;
+    if (dt == DT_F32) {
+        // Up to 64 rows: 16 to a workgroup where the workgroups are then one per CU at most, with up to three tile rows (four in place of
+        // two passes: 33 rows and more).  Two blocks of x take a workgroup longer than three tile rows (see wide_shape).
+        for (int r = 1; MB > 1 && MB <= 4 && r <= (MB > 2 && layout == LAYOUT_TILED ? 4 : 3); r++)
+            if ((T + r - 1) / r * MB <= 256) return {r, 8, 1};
+        return s;
+    }
+    if (M <= 16 || (M > 64 && !batch) || (s.r && T > 1024)) return s;
+    // 17 .. 64 rows, where the estimate is 5 % shorter: 122 of 250 random sizes 0.81 of the time, 74 of 200 row-major ones 0.79
+    double us = 0.0;
+    const WideShape dealt = wide_batch_shape(qtype, layout, M, N, K, &us);
+    if (!s.r) return batch ? dealt : s;
+    return dealt.r && us < 0.95 * wide_us(qtype, layout, s.r, MB, M, T, (K + TILE_COLS - 1) / TILE_COLS) ? dealt : s;
+}
+
 // The fused gate/up form: R of either weight, so at most 2.  Against two launches' worth of streaming passes and the fused
 // form of the tiled GEMM, which has few tiles at these sizes and walks all of K in each (fp16 sym_int4 [11008 x 4096] at 12 /
 // 24 / 48 rows 18.0 -> 14.2 / 31.1 -> 19.9 / 40.9 -> 28.8 us, [4096 x 16384] at 24 rows 127 -> 26).
@@ -111,10 +173,10 @@ bool gemv_wide_applies(int qtype, int layout, int act_dtype, int M, int N, int K
     return wide_shape(qtype, layout, act_dtype, M, N, K).r != 0;
 }
 
-// 1: not a shape for this kernel
+// 1: not a shape for this kernel; batch: see wide_shape_for
 int launch_gemv_wide(const void *x, const void *w, const void *bias, void *y, int qtype, int layout, int act_dtype, int M, int N, int K,
-                     hipStream_t st) {
-    const WideShape s = wide_shape(qtype, layout, act_dtype, M, N, K);
+                     bool batch, hipStream_t st) {
+    const WideShape s = wide_shape_for(qtype, layout, act_dtype, M, N, K, batch);
     if (!s.r) return 1;
     switch (qtype) {
     case QT_SYM_INT4: return launch_wide_q<QT_SYM_INT4>(x, w, bias, y, layout, act_dtype, M, N, K, s, st);

@@ -1,4 +1,5 @@
-// One pass over the weights for up to 64 rows of x (serving batches): y[M,N] = x[M,K] * dequant(W)[N,K]^T.
+// One pass over the weights for up to 64 rows of x (serving batches): y[M,N] = x[M,K] * dequant(W)[N,K]^T.  More rows, where the
+// weight is small: so many rows to a workgroup, that the workgroups are one per CU (gemv_wide.hip).
 //
 // A workgroup owns R tile rows (16 weight rows each) for all of K; its waves take the 128-column groups of K in turn.
 // Each wave copies its group of x (16 * MB rows) into a private part of LDS and multiplies it with R weight tiles, whose
@@ -74,7 +75,11 @@ __global__ __launch_bounds__(64 * wide_max_waves(MB, DUAL ? 2 * R : R)) void gem
     static_assert(!DUAL || (!F32 && !ROWS), "the fused form takes 16-bit activations and tiled weights");
     constexpr int PLANE = 16 * MB * 256, XBYTES = PLANE * (F32 ? 2 : 1), XC = 4 * MB;     // bytes of x in LDS; chunks of 8 per lane
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
-    const ET *const x = (const ET *)x_;
+    // (blockIdx.y: which 16 * MB rows of x)
+    const int m0 = (int)blockIdx.y * 16 * MB;
+    const ET *const x = (const ET *)x_ + (int64_t)m0 * K;
+    ET *const y = (ET *)y_ + (int64_t)m0 * N;
+    M = M - m0 < 16 * MB ? M - m0 : 16 * MB;
     const int lane = threadIdx.x & 63, W = blockDim.x >> 6, r = lane & 15, c = lane >> 4;
     const int wave = PEEL ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : threadIdx.x >> 6;
     uint8_t *const xs = smem + wave * XBYTES;
@@ -301,8 +306,8 @@ __global__ __launch_bounds__(64 * wide_max_waves(MB, DUAL ? 2 * R : R)) void gem
         const float bv = bias_ ? (float)((const ET *)bias_)[n] : 0.0f;
         auto store = [&](int m, float s, float up) __attribute__((always_inline)) {
             const float v = DUAL ? gate_act(s, act) * up : s + bv;
-            if constexpr (F32) ((float *)y_)[(int64_t)m * N + n] = v;
-            else ((AT *)y_)[(int64_t)m * N + n] = to_at<AT>(v);
+            if constexpr (F32) y[(int64_t)m * N + n] = v;
+            else y[(int64_t)m * N + n] = to_at<AT>(v);
         };
         uint32_t again = 0;                                   // results that are not finite, see dot_fp32
 #pragma unroll
@@ -355,7 +360,7 @@ static int launch_wide_r(const void *x, const void *w, const void *w_up, const v
         static const WideRoom room = wide_room((const void *)kern, (const void *)crowd, 4 * XBYTES);
         if (wv == 4 && room.crowd > room.peel && wgs > room.peel) kern = crowd;
     }
-    hipLaunchKernelGGL(kern, dim3(wgs), dim3(64 * wv), (size_t)wv * XBYTES, st, x, (const uint8_t *)w, (const uint8_t *)w_up, bias, y, M, N, K, act);
+    hipLaunchKernelGGL(kern, dim3(wgs, (M + 16 * MB - 1) / (16 * MB)), dim3(64 * wv), (size_t)wv * XBYTES, st, x, (const uint8_t *)w, (const uint8_t *)w_up, bias, y, M, N, K, act);
     return 0;
 }
 
@@ -374,11 +379,13 @@ static int launch_wide_mb(const void *x, const void *w, const void *bias, void *
 
 template <int QT, typename AT, bool F32, bool ROWS>
 static int launch_wide_t(const void *x, const void *w, const void *bias, void *y, int M, int N, int K, const WideShape &s, hipStream_t st) {
-    if (M <= 16) return launch_wide_mb<QT, AT, 1, F32, ROWS>(x, w, bias, y, M, N, K, s, st);
-    if (M <= 32) return launch_wide_mb<QT, AT, 2, F32, ROWS>(x, w, bias, y, M, N, K, s, st);
+    const int mb = s.mb ? s.mb : (M + 15) / 16;
+    if (M > 16 * mb * 65535) return -7;                      // (blocks of rows are counted in the grid's y)
+    if (mb == 1) return launch_wide_mb<QT, AT, 1, F32, ROWS>(x, w, bias, y, M, N, K, s, st);
+    if (mb == 2) return launch_wide_mb<QT, AT, 2, F32, ROWS>(x, w, bias, y, M, N, K, s, st);
     if constexpr (!F32) {
-        if (M <= 48) return launch_wide_mb<QT, AT, 3, F32, ROWS>(x, w, bias, y, M, N, K, s, st);
-        if (M <= 64) return launch_wide_mb<QT, AT, 4, F32, ROWS>(x, w, bias, y, M, N, K, s, st);
+        if (mb == 3) return launch_wide_mb<QT, AT, 3, F32, ROWS>(x, w, bias, y, M, N, K, s, st);
+        if (mb == 4) return launch_wide_mb<QT, AT, 4, F32, ROWS>(x, w, bias, y, M, N, K, s, st);
     }
     return -7;
 }

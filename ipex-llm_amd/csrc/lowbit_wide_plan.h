@@ -7,6 +7,7 @@ namespace lowbit {
 
 struct WideShape {
     int r, waves;       // tile rows per workgroup (0: another kernel), waves at most
+    int mb = 0;         // 16-row blocks of x per workgroup; 0: all of up to 64 rows
 };
 
 // Whether the fused gate/up form with two tile rows of either weight has the registers for mb 16-row blocks of x: with four it

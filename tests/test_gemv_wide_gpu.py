@@ -40,6 +40,45 @@ def test_float32_activations(qtype, layout, m, n, k):
     _check(qtype, torch.float32, layout, m, n, k, m % 2 == 0, 900 * m + n)
 
 
+# rows dealt to several workgroups: rests of 1 to 4 blocks of rows, tile rows that 1 to 4 a workgroup do not divide, one workgroup and 256
+@pytest.mark.parametrize("qtype", ALL)
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("layout,m,n,k", [(TILED, 17, 1024, 2176), (TILED, 33, 528, 1152), (TILED, 64, 2064, 384), (TILED, 65, 1040, 1152),
+                                          (TILED, 97, 48, 3200), (TILED, 130, 2064, 640), (TILED, 217, 1024, 1408), (TILED, 128, 4096, 2048),
+                                          (TILED, 500, 512, 384), (TILED, 1024, 272, 256), (TILED, 1024, 16, 128), (GGML, 40, 1003, 704),
+                                          (GGML, 66, 1001, 1088), (GGML, 200, 2003, 320), (GGML, 513, 300, 192), (GGML, 1024, 7, 64)])
+def test_rows_dealt_to_several_workgroups(qtype, dtype, layout, m, n, k):
+    if qtype == FP8:
+        k = (k + 127) // 128 * 128
+    assert ggml.lowbit_linear_workspace_bytes(qtype, layout, DT[dtype], m, n, k, 64 << 20) == 0
+    _check(qtype, dtype, layout, m, n, k, m % 2 == 0, 720 * m + n)
+
+
+@pytest.mark.parametrize("qtype", ALL)
+@pytest.mark.parametrize("layout,m,n,k", [(TILED, 17, 1024, 1408), (TILED, 32, 6160, 256), (TILED, 33, 5440, 256), (TILED, 48, 1040, 1152),
+                                          (TILED, 64, 48, 128), (GGML, 20, 3001, 320), (GGML, 40, 1001, 1088), (GGML, 63, 2003, 192)])
+def test_float32_rows_dealt_to_several_workgroups(qtype, layout, m, n, k):
+    if qtype == FP8:
+        k = (k + 127) // 128 * 128
+    _check(qtype, torch.float32, layout, m, n, k, m % 2 == 0, 730 * m + n)
+
+
+@pytest.mark.parametrize("qtype", ALL)
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("layout,m,n,k", [(TILED, 100, 1040, 256), (GGML, 70, 301, 320)])
+def test_infinities_in_rows_dealt_to_several_workgroups(qtype, dtype, layout, m, n, k):
+    if qtype == FP8:
+        k = (k + 127) // 128 * 128
+    w, x = weights(m, (n, k)), acts(m + 1, m, k, dtype)
+    x[0, 5], x[m // 2, k - 3], x[m - 1, 7] = float("inf"), -float("inf"), float("nan")
+    blob, xd = dev_quantize(w, qtype, layout), x.cuda()
+    y = torch.empty((m, n), dtype=dtype, device="cuda")
+    ggml.lowbit_linear(xd.data_ptr(), blob.data_ptr(), None, y.data_ptr(), qtype, layout, DT[dtype], m, n, k, None, 0, stream())
+    with np.errstate(all="ignore"):
+        want = x.double().numpy() @ orc.dequantize(orc.quantize(w, qtype), qtype, (n, k)).astype(np.float64).T
+    assert (classes(y.float().cpu().numpy()) == classes(want)).all()
+
+
 # where 5 to 16 rows go to this kernel: around 512, 768, 1024, 1536 and 2048 tile rows, 24 and 64 groups
 @pytest.mark.parametrize("qtype,dtype", [(2, torch.float16), (3, torch.bfloat16), (8, torch.float16), (10, torch.bfloat16), (15, torch.bfloat16)])
 @pytest.mark.parametrize("layout,m,n,k", [(TILED, 5, 8208, 3072), (TILED, 8, 12288, 3072), (TILED, 7, 4112, 8192), (TILED, 8, 8192, 8192),
