@@ -233,8 +233,8 @@ int lowbit_forward_f32(const float *x, const void *w, float *y, int qtype, int l
 /* One linear layer: y = x * dequant(w)^T + bias.  x, bias ([N], may be null) and y are of `dtype`, which may be
  * LOWBIT_DT_F32: then as lowbit_forward_f32, and no workspace is used.  With 16-bit activations as lowbit_forward_ws
  * (lowbit_linear_workspace_bytes says what to pass within a budget; null is valid), but for three choices that the other entry
- * points, whose kernel a caller may rely on, do not make: the one-pass kernel at 9 .. 64 rows in place of the ring kernel, a K
- * split or several streaming passes; narrow tiles more often (two groups of waves share such a tile's K where CUs
+ * points, whose kernel a caller may rely on, do not make: the one-pass kernel at 5 .. 64 rows, and up to 1024 on small weights, in
+ * place of the ring kernel, a K split, row-major tiles or several streaming passes; narrow tiles more often (two groups of waves share such a tile's K where CUs
  * would idle); and tiles of 256 rows ahead of all estimates where they fill the GPU's rounds well (the rounds depend on the
  * activation type).  The bias is added to the fp32 sums before the one rounding (a bias that is not 8-byte aligned is valid and
  * slower above 16 rows).  What LowBitLinear.forward computes
@@ -242,6 +242,9 @@ int lowbit_forward_f32(const float *x, const void *w, float *y, int qtype, int l
 int lowbit_linear(const void *x, const void *w, const void *bias, void *y, int qtype, int layout, int dtype, int64_t M,
                   int64_t N, int64_t K, void *workspace, size_t workspace_bytes, void *stream);
 size_t lowbit_linear_workspace_bytes(int qtype, int layout, int dtype, int64_t M, int64_t N, int64_t K, size_t max_bytes);
+/* What the call then uses of it: less where the one-pass kernel takes sizes that it takes by estimate (17 rows and more, small weights)
+ * and needs none, whatever it is given. */
+size_t lowbit_linear_scratch_bytes(int qtype, int layout, int dtype, int64_t M, int64_t N, int64_t K, size_t max_bytes);
 
 /* The gradient of lowbit_linear with respect to x: grad_x[M, K] = grad[M, N] * dequant(w)[N, K], from a tiled weight; grad and
  * grad_x are f16 or bf16, 16-byte aligned.  Same weights (one rounding to act_dtype) and sums (fp32, one rounding) as

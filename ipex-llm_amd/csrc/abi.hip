@@ -457,9 +457,15 @@ static int forward_f32(const char *what, const float *x, const void *w, const fl
 size_t lowbit_linear_workspace_bytes(int qtype, int layout, int dtype, int64_t M, int64_t N, int64_t K, size_t max_bytes) {
     if (dtype == LOWBIT_DT_F32 || M <= 16) return 0;     // one pass over the weights, or one per 32 rows
     if (!qk_size(qtype) || N <= 0 || K <= 0 || M > 0x7fffffff || N > 0x7fffffff || K > 0x7fffffff) return 0;
-    if (one_pass_applies(qtype, layout, dtype, M, N, K)) return 0;       // as forward_any chooses
+    if (gemv_wide_applies(qtype, layout, dtype, (int)M, (int)N, (int)K)) return 0;       // one pass, as forward_any chooses
     if (layout != LOWBIT_LAYOUT_GGML) return workspace_for(qtype, layout, M, N, K, max_bytes, true, dtype);
     return gemm_rows_workspace_bytes(qtype, dtype, (int)M, (int)N, (int)K, max_bytes);
+}
+
+size_t lowbit_linear_scratch_bytes(int qtype, int layout, int dtype, int64_t M, int64_t N, int64_t K, size_t max_bytes) {
+    const bool sizes_ok = qk_size(qtype) && M > 16 && N > 0 && K > 0 && M <= 0x7fffffff && N <= 0x7fffffff && K <= 0x7fffffff;
+    if (dtype != LOWBIT_DT_F32 && sizes_ok && one_pass_applies(qtype, layout, dtype, M, N, K)) return 0;
+    return lowbit_linear_workspace_bytes(qtype, layout, dtype, M, N, K, max_bytes);
 }
 
 int lowbit_linear(const void *x, const void *w, const void *bias, void *y, int qtype, int layout, int dtype, int64_t M,

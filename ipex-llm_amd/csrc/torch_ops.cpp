@@ -34,7 +34,7 @@ struct Api {
     decltype(&lowbit_last_error) last_error = nullptr;
     decltype(&lowbit_blob_bytes) blob_bytes = nullptr;
     decltype(&lowbit_tileable) tileable = nullptr;
-    decltype(&lowbit_linear_workspace_bytes) linear_workspace_bytes = nullptr;
+    decltype(&lowbit_linear_scratch_bytes) linear_scratch_bytes = nullptr;
     decltype(&lowbit_linear) linear = nullptr;
     decltype(&lowbit_mlp_forward) mlp_forward = nullptr;
     decltype(&lowbit_dequantize_rows) dequantize_rows = nullptr;
@@ -90,7 +90,7 @@ Tensor product(const Tensor &x, const Tensor &w, const Tensor &bias, int qtype, 
     Tensor y = at::empty(shape, x.options());
     const int dt = dtype_code(x.scalar_type());
     // the workspace comes from torch's caching allocator: ordered with the stream, no allocation in the steady state
-    const size_t bytes = M <= 16 ? 0 : api.linear_workspace_bytes(qtype, layout, dt, M, N, K, WORKSPACE_CAP);
+    const size_t bytes = M <= 16 ? 0 : api.linear_scratch_bytes(qtype, layout, dt, M, N, K, WORKSPACE_CAP);
     const Tensor ws = bytes ? at::empty({(int64_t)bytes}, x.options().dtype(at::kByte)) : Tensor();
     check(api.linear(x.const_data_ptr(), w.const_data_ptr(), bias.defined() ? bias.const_data_ptr() : nullptr, y.data_ptr(), qtype,
                      layout, dt, M, N, K, bytes ? ws.data_ptr() : nullptr, bytes, current_stream(x)), "lowbit_linear");
@@ -404,7 +404,7 @@ PyObject *py_bind(PyObject *, PyObject *const *args, Py_ssize_t n) {
         }                                                                                          \
         api.name = (decltype(api.name))p;                                                          \
     } while (0)
-    BIND(last_error); BIND(blob_bytes); BIND(tileable); BIND(linear_workspace_bytes); BIND(linear);
+    BIND(last_error); BIND(blob_bytes); BIND(tileable); BIND(linear_scratch_bytes); BIND(linear);
     BIND(mlp_forward); BIND(dequantize_rows); BIND(dequantize); BIND(backward_ws); BIND(backward_workspace_bytes); BIND(backward_ws_applies); BIND(experts_workspace_bytes); BIND(experts_forward);
 #undef BIND
     Py_RETURN_NONE;

@@ -313,6 +313,14 @@ def lowbit_linear_workspace_bytes(qtype, layout, dtype, m, n, k, max_bytes) -> i
     return int(_lib.lowbit_linear_workspace_bytes(qtype, layout, dtype, m, n, k, max_bytes))
 
 
+_lib.lowbit_linear_scratch_bytes.argtypes = _lib.lowbit_linear_workspace_bytes.argtypes
+_lib.lowbit_linear_scratch_bytes.restype = c_size_t
+
+
+def lowbit_linear_scratch_bytes(qtype, layout, dtype, m, n, k, max_bytes) -> int:
+    return int(_lib.lowbit_linear_scratch_bytes(qtype, layout, dtype, m, n, k, max_bytes))
+
+
 _lib.lowbit_linear.argtypes = [c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int64, c_int64, c_int64,
                                c_void_p, c_size_t, c_void_p]
 _lib.lowbit_linear.restype = c_int

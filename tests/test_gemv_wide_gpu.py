@@ -50,7 +50,7 @@ def test_float32_activations(qtype, layout, m, n, k):
 def test_rows_dealt_to_several_workgroups(qtype, dtype, layout, m, n, k):
     if qtype == FP8:
         k = (k + 127) // 128 * 128
-    assert ggml.lowbit_linear_workspace_bytes(qtype, layout, DT[dtype], m, n, k, 64 << 20) == 0
+    assert ggml.lowbit_linear_scratch_bytes(qtype, layout, DT[dtype], m, n, k, 64 << 20) == 0
     _check(qtype, dtype, layout, m, n, k, m % 2 == 0, 720 * m + n)
 
 
