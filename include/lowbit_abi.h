@@ -184,6 +184,10 @@ int lowbit_dequantize_rows(const void *w, const int64_t *rows, int64_t n_rows, v
  * gate/up form of the tiled GEMM (y 8-byte aligned, M < 2^24, K < 2^23). */
 int lowbit_mlp_forward(const void *x, const void *w_gate, const void *w_up, void *y, int qtype, int act_dtype,
                        int64_t M, int64_t N, int64_t K, int act, void *stream);
+/* The same, what a converted model's MLP calls: on small weights the one-pass kernel, whose weights are not rounded to 16 bits, takes up to
+ * 1024 rows where it is estimated to be the faster one. */
+int lowbit_gated_mlp(const void *x, const void *w_gate, const void *w_up, void *y, int qtype, int act_dtype,
+                     int64_t M, int64_t N, int64_t K, int act, void *stream);
 
 /* xe_linear.moe_forward_vec (python/llm/src/ipex_llm/transformers/models/deepseek.py:290-315): one
  * token through its top_k experts without the host reading the routing result.

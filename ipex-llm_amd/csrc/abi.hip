@@ -34,7 +34,7 @@ double gemv_wide_batch_us(int qtype, int layout, int M, int N, int K);
 double gemm_rows_us(int qtype, int act_dtype, int M, int N, int K);
 bool gemv_wide_applies(int qtype, int layout, int act_dtype, int M, int N, int K);
 int launch_mlp_wide(const void *x, const void *wg, const void *wu, void *y, int qtype, int act_dtype, int M, int N, int K, int act,
-                    hipStream_t st);
+                    bool batch, hipStream_t st);
 size_t ring_workspace_bytes(int M, int N, int K, int wgs);
 double ring_time_us(int M, int N, int K, int qtype, bool have_ws);
 int launch_gemm_ring(const void *x, const void *w, const void *bias, void *y, int qtype, int act_dtype, int M, int N, int K,
@@ -589,25 +589,35 @@ int lowbit_backward_ws(const void *grad, const void *w, void *grad_x, int qtype,
                                          (hipStream_t)stream), what);
 }
 
-int lowbit_mlp_forward(const void *x, const void *w_gate, const void *w_up, void *y, int qtype, int act_dtype,
-                       int64_t M, int64_t N, int64_t K, int act, void *stream) {
-    if (int rc = check_mm("lowbit_mlp_forward", x, w_gate, y, qtype, LOWBIT_LAYOUT_TILED, act_dtype, M, N, K)) return rc;
+// linear: also the sizes above 64 rows where the one-pass kernel is estimated shorter
+static int mlp_any(const char *who, const void *x, const void *w_gate, const void *w_up, void *y, int qtype, int act_dtype,
+                       int64_t M, int64_t N, int64_t K, int act, void *stream, bool linear) {
+    if (int rc = check_mm(who, x, w_gate, y, qtype, LOWBIT_LAYOUT_TILED, act_dtype, M, N, K)) return rc;
     if (act != LOWBIT_ACT_SILU && act != LOWBIT_ACT_GELU)
-        return fail(LOWBIT_EARG, "lowbit_mlp_forward: activation must be LOWBIT_ACT_SILU or LOWBIT_ACT_GELU");
+        return fail(LOWBIT_EARG, "%s: activation must be LOWBIT_ACT_SILU or LOWBIT_ACT_GELU", who);
     if (M * N == 0) return 0;
-    if (K == 0) return fail(LOWBIT_ESHAPE, "lowbit_mlp_forward: K == 0");
-    if (!w_up || !aligned16(w_up)) return fail(LOWBIT_EARG, "lowbit_mlp_forward: null or misaligned pointer");
-    // up to 64 rows (decode, serving batches): one pass over both weights, by the streaming kernel up to 8 rows and the
-    // kernel that gemv_wide.hip describes above that; more rows: the fused gate/up form of the tiled MFMA GEMM
-    if (M <= 64) {
-        int rc = launch_mlp_wide(x, w_gate, w_up, y, qtype, act_dtype, (int)M, (int)N, (int)K, act, (hipStream_t)stream);
-        if (rc > 0 && M <= 8)
-            rc = launch_mlp_gemv(x, w_gate, w_up, y, qtype, act_dtype, (int)M, (int)N, (int)K, act, (hipStream_t)stream);
-        if (rc <= 0) return check_launch(rc, "lowbit_mlp_forward");
-    }
-    if (((uintptr_t)y) & 7) return fail(LOWBIT_EARG, "lowbit_mlp_forward: y must be 8-byte aligned");
+    if (K == 0) return fail(LOWBIT_ESHAPE, "%s: K == 0", who);
+    if (!w_up || !aligned16(w_up)) return fail(LOWBIT_EARG, "%s: null or misaligned pointer", who);
+    // up to 64 rows (decode, serving batches), more on small weights: one pass over both weights, by the streaming kernel up to 8 rows
+    // and the kernel that gemv_wide.hip describes above that; else the fused gate/up form of the tiled MFMA GEMM
+    if (M > 64 && (((uintptr_t)y) & 7)) return fail(LOWBIT_EARG, "%s: y must be 8-byte aligned", who);
+    int rc = launch_mlp_wide(x, w_gate, w_up, y, qtype, act_dtype, (int)M, (int)N, (int)K, act, linear, (hipStream_t)stream);
+    if (rc > 0 && M <= 8)
+        rc = launch_mlp_gemv(x, w_gate, w_up, y, qtype, act_dtype, (int)M, (int)N, (int)K, act, (hipStream_t)stream);
+    if (rc <= 0) return check_launch(rc, who);
+    if (((uintptr_t)y) & 7) return fail(LOWBIT_EARG, "%s: y must be 8-byte aligned", who);
     return check_launch(launch_mlp_gemm(x, w_gate, w_up, y, qtype, act_dtype, (int)M, (int)N, (int)K, act,
-                                        (hipStream_t)stream), "lowbit_mlp_forward");
+                                        (hipStream_t)stream), who);
+}
+
+int lowbit_mlp_forward(const void *x, const void *w_gate, const void *w_up, void *y, int qtype, int act_dtype, int64_t M, int64_t N, int64_t K,
+                       int act, void *stream) {
+    return mlp_any("lowbit_mlp_forward", x, w_gate, w_up, y, qtype, act_dtype, M, N, K, act, stream, false);
+}
+
+int lowbit_gated_mlp(const void *x, const void *w_gate, const void *w_up, void *y, int qtype, int act_dtype, int64_t M, int64_t N, int64_t K,
+                     int act, void *stream) {
+    return mlp_any("lowbit_gated_mlp", x, w_gate, w_up, y, qtype, act_dtype, M, N, K, act, stream, true);
 }
 
 int lowbit_moe_forward(const void *x, const int32_t *topk_ids, const float *topk_weight, int top_k, int n_experts,

@@ -91,6 +91,10 @@ static WideShape wide_shape(int qtype, int layout, int dt, int M, int N, int K) 
     return {rounds, MB == 1 && rounds == 1 ? 12 : 8};
 }
 
+static int format_index(int qtype) {
+    return qtype == QT_SYM_INT4 ? 0 : qtype == QT_ASYM_INT4 ? 1 : qtype == QT_SYM_INT8 ? 2 : qtype == QT_NF4 ? 3 : 4;
+}
+
 // What a launch takes whose workgroups are one per CU at most, 8 waves each, with r tile rows and 16 * mb rows of x to a workgroup:
 // microseconds, fitted to 1250 sizes (M = 17 .. 900, N to 16384, K to 14000) in up to three shapes each, 6 to 10 % rms.  A launch; per
 // 1024 columns what goes with the groups, with x, with the weights and with their products; the sums; x out of L2.
@@ -102,7 +106,7 @@ static double wide_us(int qtype, int layout, int r, int mb, int M, int T, int G)
         {{2.975, 0.190, 0.075, 0.163, 0.126, 0.127, 0.038}, {3.089, 0.058, 0.118, 0.221, 0.132, 0.078, 0.038},
          {2.974, 0.087, 0.177, 0.415, 0.074, 0.094, 0.031}, {2.817, 0.170, 0.081, 0.279, 0.061, 0.160, 0.043},
          {3.052, 0.223, 0.102, 0.288, 0.096, 0.065, 0.034}}};
-    const double(&f)[7] = fit[layout == LAYOUT_TILED][qtype == QT_SYM_INT4 ? 0 : qtype == QT_ASYM_INT4 ? 1 : qtype == QT_SYM_INT8 ? 2 : qtype == QT_NF4 ? 3 : 4];
+    const double(&f)[7] = fit[layout == LAYOUT_TILED][format_index(qtype)];
     const double wgs = (double)((T + r - 1) / r) * ((M + 16 * mb - 1) / (16 * mb));
     return f[0] + (G + 7) / 8 * (f[1] + f[2] * mb + f[3] * r + f[4] * r * mb) + f[5] * r * mb + f[6] * wgs / 256 * G * mb;
 }
@@ -169,6 +173,33 @@ static WideShape wide_mlp_shape(int qtype, int act_dtype, int M, int N, int K) {
     return {r, (T + r - 1) / r <= 256 ? 8 : 4};
 }
 
+// The fused form with rows of x dealt to several workgroups, as wide_batch_shape, r of either weight; r = 0: no such shape, or the fused
+// form of the tiled GEMM is the faster one.  Fitted to 920 launches (M = 17 .. 600, N to 16384, K to 14000), 7 to 8 % rms.  17 .. 64 rows: ahead of
+// the shapes with all rows to a workgroup (172 of 183 random sizes 0.87 of the time, one 3 % longer).  More: against narrow tiles, which
+// while they are one per CU take 4 to 5 us and 0.54 to 0.65 per 128 columns (118 of 147 random sizes 0.61 of the time, none longer).
+static WideShape wide_mlp_batch_shape(int qtype, int M, int N, int K) {
+    static const double fit[5][7] = {{3.495, 0.036, 0.213, 0.220, 0.080, 0.044, 0.030}, {3.097, 0.004, 0.097, 0.235, 0.141, 0.139, 0.041},
+                                     {3.434, 0.091, 0.134, 0.416, 0.039, 0.063, 0.043}, {3.493, 0.000, 0.116, 0.322, 0.085, 0.088, 0.031},
+                                     {3.293, 0.115, 0.195, 0.351, 0.018, 0.054, 0.043}};
+    static const double tiled[5][2] = {{4.36, 0.579}, {4.32, 0.537}, {4.05, 0.580}, {4.84, 0.648}, {4.20, 0.545}};
+    WideShape best = {0, 0};
+    if (M <= 16 || M > 1024 || K > 16384) return best;
+    const int T = N / TILE_ROWS, G = K / TILE_COLS, q = format_index(qtype);
+    const double(&f)[7] = fit[q];
+    double us = M <= 64 ? 1e30 : 0.95 * (tiled[q][0] + tiled[q][1] * G);
+    for (int r = 1; r <= 2; r++)
+        for (int mb = 1; r * mb <= 4; mb++) {
+            const int64_t wgs = (int64_t)((T + r - 1) / r) * ((M + 16 * mb - 1) / (16 * mb));
+            if (wgs > 256) continue;
+            const double t = f[0] + (G + 7) / 8 * (f[1] + f[2] * mb + f[3] * 2 * r + f[4] * 2 * r * mb) + f[5] * 2 * r * mb + f[6] * (double)wgs / 256 * G * mb;
+            if (t < us) {
+                best = {r, 8, mb};
+                us = t;
+            }
+        }
+    return best;
+}
+
 bool gemv_wide_applies(int qtype, int layout, int act_dtype, int M, int N, int K) {
     return wide_shape(qtype, layout, act_dtype, M, N, K).r != 0;
 }
@@ -189,8 +220,10 @@ int launch_gemv_wide(const void *x, const void *w, const void *bias, void *y, in
 }
 
 int launch_mlp_wide(const void *x, const void *wg, const void *wu, void *y, int qtype, int act_dtype, int M, int N, int K, int act,
-                    hipStream_t st) {
-    const WideShape s = wide_mlp_shape(qtype, act_dtype, M, N, K);
+                    bool batch, hipStream_t st) {
+    WideShape s = {0, 0};
+    if (M <= 64 || batch) s = wide_mlp_batch_shape(qtype, M, N, K);
+    if (!s.r) s = wide_mlp_shape(qtype, act_dtype, M, N, K);
     if (!s.r) return 1;
     switch (qtype) {
     case QT_SYM_INT4: return launch_wide_mlp_q<QT_SYM_INT4>(x, wg, wu, y, act_dtype, M, N, K, act, s, st);

@@ -75,12 +75,16 @@ __global__ __launch_bounds__(64 * wide_max_waves(MB, DUAL ? 2 * R : R)) void gem
     static_assert(!DUAL || (!F32 && !ROWS), "the fused form takes 16-bit activations and tiled weights");
     constexpr int PLANE = 16 * MB * 256, XBYTES = PLANE * (F32 ? 2 : 1), XC = 4 * MB;     // bytes of x in LDS; chunks of 8 per lane
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
+    // (one wait for all arguments and the number of threads: left alone the compiler loaded that one behind the others, a scalar load's time
+    // that 40 rows on [11008 x 4096] took 13.4 -> 14.0 us for)
+    const int threads = (int)blockDim.x;
+    asm volatile("" :: "s"(x_), "s"(w), "s"(M), "s"(N), "s"(K), "s"(threads));
     // (blockIdx.y: which 16 * MB rows of x)
     const int m0 = (int)blockIdx.y * 16 * MB;
     const ET *const x = (const ET *)x_ + (int64_t)m0 * K;
     ET *const y = (ET *)y_ + (int64_t)m0 * N;
     M = M - m0 < 16 * MB ? M - m0 : 16 * MB;
-    const int lane = threadIdx.x & 63, W = blockDim.x >> 6, r = lane & 15, c = lane >> 4;
+    const int lane = threadIdx.x & 63, W = threads >> 6, r = lane & 15, c = lane >> 4;
     const int wave = PEEL ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : threadIdx.x >> 6;
     uint8_t *const xs = smem + wave * XBYTES;
     const int G = ROWS ? (K + TILE_COLS - 1) / TILE_COLS : K / TILE_COLS, blocks = K / F::QK;
@@ -416,10 +420,12 @@ static int launch_wide_mlp_mb(const void *x, const void *wg, const void *wu, voi
 template <int QT, typename AT>
 static int launch_wide_mlp_t(const void *x, const void *wg, const void *wu, void *y, int M, int N, int K, int act, const WideShape &s,
                              hipStream_t st) {
-    if (M <= 16) return launch_wide_mlp_mb<QT, AT, 1>(x, wg, wu, y, M, N, K, act, s, st);
-    if (M <= 32) return launch_wide_mlp_mb<QT, AT, 2>(x, wg, wu, y, M, N, K, act, s, st);
-    if (M <= 48) return launch_wide_mlp_mb<QT, AT, 3>(x, wg, wu, y, M, N, K, act, s, st);
-    return M <= 64 ? launch_wide_mlp_mb<QT, AT, 4>(x, wg, wu, y, M, N, K, act, s, st) : -7;
+    const int mb = s.mb ? s.mb : (M + 15) / 16;
+    if (M > 16 * mb * 65535) return -7;                      // (blocks of rows are counted in the grid's y)
+    if (mb == 1) return launch_wide_mlp_mb<QT, AT, 1>(x, wg, wu, y, M, N, K, act, s, st);
+    if (mb == 2) return launch_wide_mlp_mb<QT, AT, 2>(x, wg, wu, y, M, N, K, act, s, st);
+    if (mb == 3) return launch_wide_mlp_mb<QT, AT, 3>(x, wg, wu, y, M, N, K, act, s, st);
+    return mb == 4 ? launch_wide_mlp_mb<QT, AT, 4>(x, wg, wu, y, M, N, K, act, s, st) : -7;
 }
 
 template <int QT>

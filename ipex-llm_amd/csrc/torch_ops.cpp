@@ -36,7 +36,7 @@ struct Api {
     decltype(&lowbit_tileable) tileable = nullptr;
     decltype(&lowbit_linear_scratch_bytes) linear_scratch_bytes = nullptr;
     decltype(&lowbit_linear) linear = nullptr;
-    decltype(&lowbit_mlp_forward) mlp_forward = nullptr;
+    decltype(&lowbit_gated_mlp) gated_mlp = nullptr;
     decltype(&lowbit_dequantize_rows) dequantize_rows = nullptr;
     decltype(&lowbit_dequantize) dequantize = nullptr;
     decltype(&lowbit_backward_ws) backward_ws = nullptr;
@@ -226,8 +226,8 @@ Tensor gated(const Tensor &x_in, const Tensor &wg, const Tensor &wu, int qtype, 
     const Tensor x = x_in.is_contiguous() ? x_in : x_in.contiguous();
     c10::DeviceGuard guard(x.device());
     Tensor y = at::empty(with_last(x, N), x.options());
-    check(api.mlp_forward(x.const_data_ptr(), wg.const_data_ptr(), wu.const_data_ptr(), y.data_ptr(), qtype, dt, M, N, K, act,
-                          current_stream(x)), "lowbit_mlp_forward");
+    check(api.gated_mlp(x.const_data_ptr(), wg.const_data_ptr(), wu.const_data_ptr(), y.data_ptr(), qtype, dt, M, N, K, act,
+                          current_stream(x)), "lowbit_gated_mlp");
     return y;
 }
 
@@ -405,7 +405,7 @@ PyObject *py_bind(PyObject *, PyObject *const *args, Py_ssize_t n) {
         api.name = (decltype(api.name))p;                                                          \
     } while (0)
     BIND(last_error); BIND(blob_bytes); BIND(tileable); BIND(linear_scratch_bytes); BIND(linear);
-    BIND(mlp_forward); BIND(dequantize_rows); BIND(dequantize); BIND(backward_ws); BIND(backward_workspace_bytes); BIND(backward_ws_applies); BIND(experts_workspace_bytes); BIND(experts_forward);
+    BIND(gated_mlp); BIND(dequantize_rows); BIND(dequantize); BIND(backward_ws); BIND(backward_workspace_bytes); BIND(backward_ws_applies); BIND(experts_workspace_bytes); BIND(experts_forward);
 #undef BIND
     Py_RETURN_NONE;
 }

@@ -399,6 +399,8 @@ _lib.lowbit_dequantize_rows.restype = c_int
 _lib.lowbit_mlp_forward.argtypes = [c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int64, c_int64, c_int64,
                                     c_int, c_void_p]
 _lib.lowbit_mlp_forward.restype = c_int
+_lib.lowbit_gated_mlp.argtypes = _lib.lowbit_mlp_forward.argtypes
+_lib.lowbit_gated_mlp.restype = c_int
 
 
 _lib.lowbit_moe_forward.argtypes = [c_void_p, c_void_p, c_void_p, c_int, c_int, c_void_p, c_void_p, c_void_p, c_void_p,
@@ -426,6 +428,10 @@ def lowbit_dequantize_rows(w, rows, n_rows, dst, qtype, n, k, layout, out_dtype,
 
 def lowbit_mlp_forward(x, w_gate, w_up, y, qtype, act_dtype, m, n, k, act, stream):
     _check(_lib.lowbit_mlp_forward(x, w_gate, w_up, y, qtype, act_dtype, m, n, k, act, stream), "lowbit_mlp_forward")
+
+
+def lowbit_gated_mlp(x, w_gate, w_up, y, qtype, act_dtype, m, n, k, act, stream):
+    _check(_lib.lowbit_gated_mlp(x, w_gate, w_up, y, qtype, act_dtype, m, n, k, act, stream), "lowbit_gated_mlp")
 
 
 def lowbit_blob_bytes(qtype, n_weights) -> int:

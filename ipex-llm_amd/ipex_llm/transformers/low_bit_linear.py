@@ -330,7 +330,7 @@ def mlp_forward_xpu(x: torch.Tensor, weight1: torch.Tensor, weight2: torch.Tenso
                     state_size: int, output_size: int, act_type: int, qtype: int):
     """xe_linear.mlp_forward_xpu (models/common.py:152-156, xpu_ops.py:34-37):
     act(x @ W1^T) * (x @ W2^T) in one launch; act_type 0 = SiLU, 1 = GELU (tanh form).  Any number of rows: up to 64
-    (32 for weights of more than 16384 rows) one pass over both weights, by the streaming kernel up to 8 rows and by the
+    (32 for weights of more than 16384 rows; more on small weights) one pass over both weights, by the streaming kernel up to 8 rows and by the
     one-pass kernel beyond, more the fused gate/up form of the tiled GEMM (made for prefill batches)."""
     invalidInputError(x.dim() == 2 and x.shape == (batch_size, state_size) and x.device.type == _ACCEL,
                       "mlp_forward_xpu expects x of shape [batch_size, state_size] on the GPU")
@@ -349,7 +349,7 @@ def mlp_forward_xpu(x: torch.Tensor, weight1: torch.Tensor, weight2: torch.Tenso
     xc = (x if x.dtype != torch.float32 else x.half()).contiguous()
     y = torch.empty((batch_size, output_size), dtype=xc.dtype, device=x.device)
     with torch.cuda.device(x.device):
-        ggml.lowbit_mlp_forward(xc.data_ptr(), _as_u8(weight1).data_ptr(), _as_u8(weight2).data_ptr(), y.data_ptr(),
+        ggml.lowbit_gated_mlp(xc.data_ptr(), _as_u8(weight1).data_ptr(), _as_u8(weight2).data_ptr(), y.data_ptr(),
                                 qtype, _DT[xc.dtype], batch_size, output_size, state_size, act_type, _stream())
     return y if y.dtype == x.dtype else y.to(x.dtype)
 

@@ -12,7 +12,7 @@ import ipex_llm.ggml.model.llama.llama_cpp as ggml
 from ipex_llm.utils.common import invalidInputError
 from ipex_llm.utils.utils import get_shared_lib_info
 
-_BOUND = ("last_error", "blob_bytes", "tileable", "linear_scratch_bytes", "linear", "mlp_forward", "dequantize_rows", "dequantize", "backward_ws", "backward_workspace_bytes", "backward_ws_applies",
+_BOUND = ("last_error", "blob_bytes", "tileable", "linear_scratch_bytes", "linear", "gated_mlp", "dequantize_rows", "dequantize", "backward_ws", "backward_workspace_bytes", "backward_ws_applies",
           "experts_workspace_bytes", "experts_forward")
 
 

@@ -148,14 +148,30 @@ def test_fused_gate_up(qtype, m, n, k):
     assert np.abs(y - want).max() <= (2e-3 if dtype == torch.float16 else 8e-3) * np.abs(want).max()
 
 
+def gated_mlp(x, wg, wu, m, k, n, act, qtype):
+    y = torch.full((m + 1, n), float("nan"), dtype=x.dtype, device="cuda")
+    ggml.lowbit_gated_mlp(x.data_ptr(), wg.data_ptr(), wu.data_ptr(), y.data_ptr(), qtype, DT[x.dtype], m, n, k, 0, stream())
+    assert torch.isnan(y[m]).all()
+    return y[:m]
+
+
+# 17 rows and more, dealt to several workgroups
+@pytest.mark.parametrize("qtype", ALL)
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("m,n,k", [(17, 1040, 1152), (33, 272, 640), (64, 2064, 384), (65, 1040, 1408), (130, 1024, 2048), (200, 528, 3200),
+                                   (600, 256, 2176), (1024, 48, 1280)])
+def test_fused_gate_up_rows_dealt(qtype, dtype, m, n, k):
+    test_fused_gate_up_of_many_workgroups(qtype, dtype, m, n, k, gated_mlp)
+
+
 @pytest.mark.parametrize("qtype", ALL)
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("m,n,k", [(12, 16400, 640), (20, 8336, 512), (40, 8336, 640), (48, 12304, 1152)])
-def test_fused_gate_up_of_many_workgroups(qtype, dtype, m, n, k):
+def test_fused_gate_up_of_many_workgroups(qtype, dtype, m, n, k, run=mlp_forward_xpu):
     """More workgroups of four waves than the GPU holds at once in the form of more registers; K of as many groups as waves, and more."""
     blobs = [dev_quantize(weights(m + i, (n, k)), qtype, TILED) for i in range(2)]
     x = acts(m, m, k, dtype).cuda()
-    y = mlp_forward_xpu(x, *blobs, m, k, n, SILU, qtype).double()
+    y = run(x, *blobs, m, k, n, SILU, qtype).double()
     eps = torch.finfo(dtype).eps
     # fp32 sums of exact products; the levels of nf4 are rounded to x's type
     err = k * 2.0 ** -24 + (eps / 2 if qtype == NF4 else 0.0)
