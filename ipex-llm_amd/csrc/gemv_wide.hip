@@ -150,11 +150,13 @@ static WideShape wide_shape_for(int qtype, int layout, int dt, int M, int N, int
         return s;
     }
     if (M <= 16 || (M > 64 && !batch) || (s.r && T > 1024)) return s;
-    // 17 .. 64 rows, where the estimate is 5 % shorter: 122 of 250 random sizes 0.81 of the time, 74 of 200 row-major ones 0.79
+    // 17 .. 64 rows, where the estimate is 5 % shorter: 122 of 250 random sizes 0.81 of the time, 74 of 200 row-major ones 0.79; beyond 64
+    // groups 12 % (18 rows on [5104 x 9728] in asym_int4, estimated 8 % shorter, took 1.06 of the time)
+    const int G = (K + TILE_COLS - 1) / TILE_COLS;
     double us = 0.0;
     const WideShape dealt = wide_batch_shape(qtype, layout, M, N, K, &us);
     if (!s.r) return batch ? dealt : s;
-    return dealt.r && us < 0.95 * wide_us(qtype, layout, s.r, MB, M, T, (K + TILE_COLS - 1) / TILE_COLS) ? dealt : s;
+    return dealt.r && us < (G <= 64 ? 0.95 : 0.88) * wide_us(qtype, layout, s.r, MB, M, T, G) ? dealt : s;
 }
 
 // The fused gate/up form: R of either weight, so at most 2.  Against two launches' worth of streaming passes and the fused

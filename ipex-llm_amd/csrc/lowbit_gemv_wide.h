@@ -103,7 +103,7 @@ __global__ __launch_bounds__(64 * wide_max_waves(MB, DUAL ? 2 * R : R)) void gem
     }
     // x: 16 consecutive lanes load the 16 chunks of a row's group (256 bytes; F32: 512), four rows per instruction
     const int u = lane & 15, xrow = lane >> 4;
-    auto load = [&](int g, u32x4 (&xv)[F32 ? 2 * XC : XC], auto &t) __attribute__((always_inline)) {
+    auto load = [&](int g, u32x4 (&xv)[F32 ? 2 * XC : XC], auto &t, bool first_group = false) __attribute__((always_inline)) {
         const int col = g * TILE_COLS + u * 8;
         const bool past = ROWS && col >= K;                  // (put makes zeros of columns past K)
 #pragma unroll
@@ -118,6 +118,8 @@ __global__ __launch_bounds__(64 * wide_max_waves(MB, DUAL ? 2 * R : R)) void gem
             }
 #pragma unroll
             for (int h = 0; h < (F32 ? 2 : 1); h++) xv[i * (F32 ? 2 : 1) + h] = p[h];
+            // (ahead of the loop each goes out as its address is there: left alone the compiler kept all of them behind the last one's)
+            if (first_group) __builtin_amdgcn_sched_barrier(0);
         }
 #pragma unroll
         for (int wi = 0; wi < NT; wi++) {
@@ -161,7 +163,7 @@ __global__ __launch_bounds__(64 * wide_max_waves(MB, DUAL ? 2 * R : R)) void gem
     typename std::conditional<ROWS, RowRegs<QT>, TileRegs<QT>>::type wc[NT], wn[NT];
     u32x4 xv[F32 ? 2 * XC : XC];
     if constexpr (PEEL) {
-        load(wave, xv, wn);                                  // (no more waves than groups)
+        load(wave, xv, wn, true);                            // (no more waves than groups)
         auto hold = [](auto &t) __attribute__((always_inline)) {
             asm volatile("" : "+v"(t.q0));
             if constexpr (F::BITS == 8) asm volatile("" : "+v"(t.q1));
