@@ -1,4 +1,4 @@
-// Where the one-pass kernel for up to 64 rows of x (lowbit_gemv_wide.h) is used, and in which shape.
+// Where the one-pass kernel (lowbit_gemv_wide.h) is used, for up to 64 rows of x and for more on small weights, and in which shape.
 #include <hip/hip_runtime.h>
 #include "lowbit_wide_plan.h"
 
