@@ -237,8 +237,10 @@ int lowbit_forward_f32(const float *x, const void *w, float *y, int qtype, int l
 /* One linear layer: y = x * dequant(w)^T + bias.  x, bias ([N], may be null) and y are of `dtype`, which may be
  * LOWBIT_DT_F32: then as lowbit_forward_f32, and no workspace is used.  With 16-bit activations as lowbit_forward_ws
  * (lowbit_linear_workspace_bytes says what to pass within a budget; null is valid), but for three choices that the other entry
- * points, whose kernel a caller may rely on, do not make: the one-pass kernel at 5 .. 64 rows, and up to 1024 on small weights, in
- * place of the ring kernel, a K split, row-major tiles or several streaming passes; narrow tiles more often (two groups of waves share such a tile's K where CUs
+ * points, whose kernel a caller may rely on, do not make: the one-pass kernel at 17 .. 64 rows of x, and up to 1024 on small weights, in
+ * place of the ring kernel, a K split, row-major tiles or several streaming passes, and up to 16 rows on more weights than they take
+ * it on (where lowbit_forward(_ws) plans one streaming pass and y is 8-byte aligned, it takes the one-pass kernel in its place at 9 .. 16
+ * rows of x on tiled and 5 .. 16 on row-major weights, up to 16384 weight rows; row-major ones up to 64); narrow tiles more often (two groups of waves share such a tile's K where CUs
  * would idle); and tiles of 256 rows ahead of all estimates where they fill the GPU's rounds well (the rounds depend on the
  * activation type).  The bias is added to the fp32 sums before the one rounding (a bias that is not 8-byte aligned is valid and
  * slower above 16 rows).  What LowBitLinear.forward computes

@@ -29,7 +29,7 @@ int launch_dequantize(const void *w, void *out, int qtype, int64_t N, int64_t K,
 int launch_gemv(const void *x, const void *w, const void *bias, void *y, int qtype, int layout, int act_dtype, int M, int N, int K,
                 int waves, hipStream_t st);
 int launch_gemv_wide(const void *x, const void *w, const void *bias, void *y, int qtype, int layout, int act_dtype, int M, int N, int K,
-                     bool batch, hipStream_t st);
+                     bool linear, hipStream_t st);
 double gemv_wide_batch_us(int qtype, int layout, int M, int N, int K);
 double gemm_rows_us(int qtype, int act_dtype, int M, int N, int K);
 bool gemv_wide_applies(int qtype, int layout, int act_dtype, int M, int N, int K);
@@ -440,14 +440,14 @@ static int forward_f32(const char *what, const float *x, const void *w, const fl
         return fail(LOWBIT_EARG, "%s: null or misaligned pointer (x, w: 16 bytes)", what);
     if (K % 8) return fail(LOWBIT_ESHAPE, "%s: K must be a multiple of 8", what);
     if (M > 32 && M <= 64) {                             // in one launch, where the weight is small enough
-        const int rc = launch_gemv_wide(x, w, bias, y, qtype, layout, LOWBIT_DT_F32, (int)M, (int)N, (int)K, false, (hipStream_t)stream);
+        const int rc = launch_gemv_wide(x, w, bias, y, qtype, layout, LOWBIT_DT_F32, (int)M, (int)N, (int)K, true, (hipStream_t)stream);
         if (rc <= 0) return check_launch(rc, what);
     }
     for (int64_t m0 = 0; m0 < M; m0 += 32) {
         const int m = (int)(M - m0 < 32 ? M - m0 : 32), n = (int)N, k = (int)K;
         const float *xp = x + m0 * K;
         float *yp = y + m0 * N;
-        int rc = launch_gemv_wide(xp, w, bias, yp, qtype, layout, LOWBIT_DT_F32, m, n, k, false, (hipStream_t)stream);
+        int rc = launch_gemv_wide(xp, w, bias, yp, qtype, layout, LOWBIT_DT_F32, m, n, k, true, (hipStream_t)stream);
         if (rc > 0) rc = launch_gemv(xp, w, bias, yp, qtype, layout, LOWBIT_DT_F32, m, n, k, 0, (hipStream_t)stream);
         if (rc) return check_launch(rc, what);
     }

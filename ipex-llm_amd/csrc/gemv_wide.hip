@@ -21,7 +21,9 @@ int launch_wide_mlp_q(const void *x, const void *wg, const void *wu, void *y, in
 // of the tiled GEMM win, which divide x as well ([4096 x 11008] at 64 rows: 24.2 us against 31).  Beyond 1024 tile rows
 // there are several rounds of workgroups and x comes again in each: only up to 32 rows still pay ([28672 x 8192] at 48
 // rows 106 against 96 us of the GEMM).
-static WideShape wide_shape(int qtype, int layout, int dt, int M, int N, int K) {
+// linear: lowbit_linear and float32 activations.  The other entry points, whose kernel a caller may rely on, keep the streaming kernel up to 8
+// rows of tiled weights (4 of row-major ones) and beyond 1024 tile rows.
+static WideShape wide_shape(int qtype, int layout, int dt, int M, int N, int K, bool linear) {
     const int T = (N + TILE_ROWS - 1) / TILE_ROWS, G = (K + TILE_COLS - 1) / TILE_COLS, MB = (M + 15) / 16;
     const int rounds = (T + 255) / 256;
     const WideShape none = {0, 0};
@@ -29,7 +31,7 @@ static WideShape wide_shape(int qtype, int layout, int dt, int M, int N, int K) 
     // one or two read x more often: from 24 groups on (8 rows, 16-bit activations: 0.79 .. 0.95 of its time on 9728 .. 12288 rows
     // of 4096 and 8192 columns, sym_int8 on [11008 x 4096] 14.2 -> 11.3 us, asym_int4 in bf16 10.9 -> 9.2, float32 sym_int4 15.2 -> 12.8;
     // 1.0 .. 1.07 of it with 8 groups).
-    const bool shared_by_three = M > 4 && M <= 8 && layout == LAYOUT_TILED && rounds == 3 && G >= 24;
+    const bool shared_by_three = linear && M > 4 && M <= 8 && layout == LAYOUT_TILED && rounds == 3 && G >= 24;
     if (dt == DT_F32) {
         // Two planes of x: 32 rows at most, and twice the x to read, to split and to write to LDS.  One pass at half the x traffic of
         // the streaming kernel's (9 .. 16 rows on [28672 x 8192]: 86 -> 48) or in place of two; up to 8 rows it loses.
@@ -58,7 +60,7 @@ static WideShape wide_shape(int qtype, int layout, int dt, int M, int N, int K) 
             // the streaming kernel's time over the formats, on [50001 x 4096] 0.81 .. 0.95 / 0.81 .. 0.98, on [17001 x 1024] 0.88 ..
             // 1.05); between 1537 and 2048, where that kernel's rounds come out even, four waves with four tile rows, and not fp8_e4m3
             // (1.03), nor asym_int4 up to 12 rows (9 / 16 rows on [32003 x 4096] 1.04 / 0.88; sym_int4 0.97 / 0.92).
-            if (T > 1024 && M > 8 && G >= 24) {
+            if (linear && T > 1024 && M > 8 && G >= 24) {
                 if (T <= 1536 || T > 2048) return {2, 8};
                 if (qtype != QT_FP8_E4M3 && (qtype != QT_ASYM_INT4 || M > 12)) return {4, 4};
             }
@@ -80,11 +82,11 @@ static WideShape wide_shape(int qtype, int layout, int dt, int M, int N, int K) 
             // have nothing, 6 rows on [4272 x 8192] in fp8_e4m3 1.08), 512 of them in the 8-bit formats only (0.91 .. 0.93,
             // the others 0.99 .. 1.04)
             const bool eight_bit = qtype == QT_SYM_INT8 || qtype == QT_FP8_E4M3;
-            if (M > 4 && rounds == 2 && T >= 304 && G >= 64 && (T < 512 || eight_bit)) return {2, 8};
-            if (M > 4 && T >= 1216 && G >= 24 && (qtype == QT_ASYM_INT4 || qtype == QT_SYM_INT8)) return many;
+            if (linear && M > 4 && rounds == 2 && T >= 304 && G >= 64 && (T < 512 || eight_bit)) return {2, 8};
+            if (linear && M > 4 && T >= 1216 && G >= 24 && (qtype == QT_ASYM_INT4 || qtype == QT_SYM_INT8)) return many;
             return none;
         }
-        if (MB == 1 && T > 1024) return T > 1536 && T <= 2048 && G < 24 ? none : many;
+        if (MB == 1 && T > 1024) return !linear || (T > 1536 && T <= 2048 && G < 24) ? none : many;
         if ((MB > 1 && MB * G > 192) || (MB == 4 && T > 768) || (T > 1024 && MB > 2)) return none;
     }
     if (T > 1024) return {4, 4};
@@ -138,9 +140,9 @@ double gemv_wide_batch_us(int qtype, int layout, int M, int N, int K) {
     return wide_batch_shape(qtype, layout, M, N, K, &us).r ? us : 0.0;
 }
 
-// batch: also the sizes that wide_shape leaves to other kernels
-static WideShape wide_shape_for(int qtype, int layout, int dt, int M, int N, int K, bool batch) {
-    const WideShape s = wide_shape(qtype, layout, dt, M, N, K);
+// linear: also the sizes that wide_shape leaves to other kernels
+static WideShape wide_shape_for(int qtype, int layout, int dt, int M, int N, int K, bool linear) {
+    const WideShape s = wide_shape(qtype, layout, dt, M, N, K, linear);
     const int T = (N + TILE_ROWS - 1) / TILE_ROWS, MB = (M + 15) / 16;
     if (dt == DT_F32) {
         // Up to 64 rows: 16 to a workgroup where the workgroups are then one per CU at most, with up to three tile rows (four in place of
@@ -149,13 +151,13 @@ static WideShape wide_shape_for(int qtype, int layout, int dt, int M, int N, int
             if ((T + r - 1) / r * MB <= 256) return {r, 8, 1};
         return s;
     }
-    if (M <= 16 || (M > 64 && !batch) || (s.r && T > 1024)) return s;
+    if (M <= 16 || (M > 64 && !linear) || (s.r && T > 1024)) return s;
     // 17 .. 64 rows, where the estimate is 5 % shorter: 122 of 250 random sizes 0.81 of the time, 74 of 200 row-major ones 0.79; beyond 64
     // groups 12 % (18 rows on [5104 x 9728] in asym_int4, estimated 8 % shorter, took 1.06 of the time)
     const int G = (K + TILE_COLS - 1) / TILE_COLS;
     double us = 0.0;
     const WideShape dealt = wide_batch_shape(qtype, layout, M, N, K, &us);
-    if (!s.r) return batch ? dealt : s;
+    if (!s.r) return linear ? dealt : s;
     return dealt.r && us < (G <= 64 ? 0.95 : 0.88) * wide_us(qtype, layout, s.r, MB, M, T, G) ? dealt : s;
 }
 
@@ -203,13 +205,13 @@ static WideShape wide_mlp_batch_shape(int qtype, int M, int N, int K) {
 }
 
 bool gemv_wide_applies(int qtype, int layout, int act_dtype, int M, int N, int K) {
-    return wide_shape(qtype, layout, act_dtype, M, N, K).r != 0;
+    return wide_shape(qtype, layout, act_dtype, M, N, K, true).r != 0;
 }
 
-// 1: not a shape for this kernel; batch: see wide_shape_for
+// 1: not a shape for this kernel; linear: see wide_shape and wide_shape_for
 int launch_gemv_wide(const void *x, const void *w, const void *bias, void *y, int qtype, int layout, int act_dtype, int M, int N, int K,
-                     bool batch, hipStream_t st) {
-    const WideShape s = wide_shape_for(qtype, layout, act_dtype, M, N, K, batch);
+                     bool linear, hipStream_t st) {
+    const WideShape s = wide_shape_for(qtype, layout, act_dtype, M, N, K, linear);
     if (!s.r) return 1;
     switch (qtype) {
     case QT_SYM_INT4: return launch_wide_q<QT_SYM_INT4>(x, w, bias, y, layout, act_dtype, M, N, K, s, st);

@@ -106,6 +106,25 @@ def test_few_rows_of_many_tile_rows(qtype, dtype, layout, m, n, k):
                            torch.nan_to_num(want.float(), nan=7.0, posinf=1.0, neginf=-1.0))
 
 
+# the sizes of 5 to 16 rows that only lowbit_linear gives to this kernel
+@pytest.mark.parametrize("qtype,dtype", [(2, torch.float16), (3, torch.bfloat16), (8, torch.float16), (10, torch.bfloat16), (15, torch.bfloat16)])
+@pytest.mark.parametrize("layout,m,n,k", [(TILED, 5, 8208, 3072), (TILED, 8, 12288, 3072), (TILED, 7, 4880, 8192), (TILED, 8, 8192, 8192),
+                                          (TILED, 6, 24592, 3072), (TILED, 9, 16400, 256), (TILED, 12, 24592, 3072), (GGML, 9, 16401, 3072),
+                                          (GGML, 13, 32769, 3072)])
+def test_forward_keeps_the_streaming_kernel(qtype, dtype, layout, m, n, k):
+    """lowbit_forward and lowbit_forward_ws give the streaming kernel's bits, with whatever alignment of y."""
+    blob = dev_quantize(np.random.default_rng(m + n).standard_normal((n, k), dtype=np.float32) * 0.02, qtype, layout)
+    x = acts(m, m, k, dtype).cuda()
+    y = torch.full((4, (m * n + 23) // 8 * 8), float("nan"), dtype=dtype, device="cuda")
+    args = (qtype, layout, DT[dtype], m, n, k)
+    ggml.lowbit_gemv(x.data_ptr(), blob.data_ptr(), y[0].data_ptr(), *args, 0, stream())
+    ggml.lowbit_forward(x.data_ptr(), blob.data_ptr(), y[1].data_ptr(), *args, stream())
+    ggml.lowbit_forward_ws(x.data_ptr(), blob.data_ptr(), y[2].data_ptr(), *args, None, 0, stream())
+    ggml.lowbit_forward(x.data_ptr(), blob.data_ptr(), y[3][1:].data_ptr(), *args, stream())
+    want = y[0, :m * n]
+    assert want.isfinite().all() and torch.equal(y[1, :m * n], want) and torch.equal(y[2, :m * n], want) and torch.equal(y[3, 1:m * n + 1], want)
+
+
 # tile rows that three and four do not divide, 12 waves with fewer and more groups, several workgroups of four waves per CU
 @pytest.mark.parametrize("qtype", ALL)
 @pytest.mark.parametrize("layout,m,n,k", [(TILED, 12, 48, 1664), (TILED, 9, 8224, 256), (TILED, 32, 8240, 1152), (TILED, 16, 12336, 1152),
