@@ -144,12 +144,14 @@ int lowbit_forward(const void *x, const void *w, void *y, int qtype, int layout,
 /* Which kernel lowbit_forward (have_workspace = 0) or lowbit_forward_ws (a non-null workspace of
  * workspace_bytes) runs for a shape with an 8-byte aligned y, without running anything: the streaming GEMV in 16-row passes, the ring kernel for batch
  * sizes, or the MFMA GEMM with or without a K split or in narrow tiles.  Negative for an unknown qtype.  Host arithmetic only.
- * (Not lowbit_linear, which is freer to choose, see there.) */
+ * (Not lowbit_linear, which is freer to choose, see lowbit_linear_plan.) */
 #define LOWBIT_PLAN_GEMV 0
 #define LOWBIT_PLAN_RING 1
 #define LOWBIT_PLAN_GEMM 2
 #define LOWBIT_PLAN_GEMM_SPLIT 3
 #define LOWBIT_PLAN_GEMM_NARROW 4  /* the MFMA GEMM in tiles of 128 weight rows (lowbit_gemm_narrow) */
+#define LOWBIT_PLAN_ONE_PASS 5     /* lowbit_linear_plan only, as is the next */
+#define LOWBIT_PLAN_ROWS 6         /* the MFMA GEMM over row-major weights */
 /* What lowbit_forward_ws makes use of when the caller can spare at most max_bytes of workspace for this format
  * and shape: the size of the partial tiles of the plan it then picks, 0 when that plan has none.  A caller
  * with a budget asks this instead of capping lowbit_workspace_bytes (which carries no format and returns the most
@@ -248,6 +250,10 @@ int lowbit_forward_f32(const float *x, const void *w, float *y, int qtype, int l
 int lowbit_linear(const void *x, const void *w, const void *bias, void *y, int qtype, int layout, int dtype, int64_t M,
                   int64_t N, int64_t K, void *workspace, size_t workspace_bytes, void *stream);
 size_t lowbit_linear_workspace_bytes(int qtype, int layout, int dtype, int64_t M, int64_t N, int64_t K, size_t max_bytes);
+/* Which kernel lowbit_linear runs with workspace_bytes of workspace (0: none) and y and bias 8-byte aligned, LOWBIT_PLAN_*; for
+ * LOWBIT_PLAN_ONE_PASS plan3 (may be null) = {16-row tiles of the weight per workgroup, waves at most, 16-row blocks of x per workgroup}.  Of
+ * float32 rows that take several launches: the first one's.  Negative for an unknown qtype or an empty product.  Host arithmetic only. */
+int lowbit_linear_plan(int qtype, int layout, int dtype, int64_t M, int64_t N, int64_t K, size_t workspace_bytes, int *plan3);
 /* What the call then uses of it: less where the one-pass kernel takes sizes that it takes by estimate (17 rows and more, small weights)
  * and needs none, whatever it is given. */
 size_t lowbit_linear_scratch_bytes(int qtype, int layout, int dtype, int64_t M, int64_t N, int64_t K, size_t max_bytes);

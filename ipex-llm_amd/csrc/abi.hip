@@ -1,6 +1,7 @@
 // extern "C" surface of liblowbit_hip.so (declared in include/lowbit_abi.h).
 #include "../../include/lowbit_abi.h"
 #include "lowbit_formats.h"
+#include "lowbit_wide_plan.h"
 
 #include <stdarg.h>
 #include <stdio.h>
@@ -29,7 +30,8 @@ int launch_dequantize(const void *w, void *out, int qtype, int64_t N, int64_t K,
 int launch_gemv(const void *x, const void *w, const void *bias, void *y, int qtype, int layout, int act_dtype, int M, int N, int K,
                 int waves, hipStream_t st);
 int launch_gemv_wide(const void *x, const void *w, const void *bias, void *y, int qtype, int layout, int act_dtype, int M, int N, int K,
-                     bool linear, hipStream_t st);
+                     const WideShape &s, hipStream_t st);
+WideShape gemv_wide_shape(int qtype, int layout, int act_dtype, int M, int N, int K, bool linear);
 double gemv_wide_batch_us(int qtype, int layout, int M, int N, int K);
 double gemm_rows_us(int qtype, int act_dtype, int M, int N, int K);
 bool gemv_wide_applies(int qtype, int layout, int act_dtype, int M, int N, int K);
@@ -271,7 +273,8 @@ static bool ring_range(int qtype, int64_t M) { return M <= (qtype == LOWBIT_QT_N
 //     small weights ([2048 x 2048], [5632 x 2048], [4096 x 4096]) at a hundred to two thousand rows
 //     (narrow_time_us).
 enum { PLAN_GEMV = LOWBIT_PLAN_GEMV, PLAN_RING = LOWBIT_PLAN_RING, PLAN_GEMM = LOWBIT_PLAN_GEMM,
-       PLAN_GEMM_SPLIT = LOWBIT_PLAN_GEMM_SPLIT, PLAN_GEMM_NARROW = LOWBIT_PLAN_GEMM_NARROW };
+       PLAN_GEMM_SPLIT = LOWBIT_PLAN_GEMM_SPLIT, PLAN_GEMM_NARROW = LOWBIT_PLAN_GEMM_NARROW,
+       PLAN_ONE_PASS = LOWBIT_PLAN_ONE_PASS, PLAN_ROWS = LOWBIT_PLAN_ROWS };
 
 static double gemv_time_us(int qtype, int64_t M, int64_t N, int64_t K) {
     const double rate = qtype == LOWBIT_QT_SYM_INT8 || qtype == LOWBIT_QT_FP8_E4M3 ? 5.03e6 : qtype == LOWBIT_QT_NF4 ? 3.31e6 : 3.97e6;
@@ -386,8 +389,22 @@ extern "C" int lowbit_forward_plan(int qtype, int layout, int64_t M, int64_t N, 
     return plan_forward(qtype, layout, M, N, K, have_workspace != 0, have_workspace ? workspace_bytes : 0, true, nullptr);
 }
 
-// linear: lowbit_linear, which is free to take the one-pass kernel (gemv_wide.hip) in place of any planned one; elsewhere it
-// stands in for the streaming kernel's plan only, which is what it is.
+// The kernel that forward_any launches.  linear: lowbit_linear, which is free to take the one-pass kernel (gemv_wide.hip) in place of any
+// planned one; elsewhere it stands in for the streaming kernel's plan only, which is what it is, and a y off the 8-byte boundaries keeps the
+// streaming kernel's passes, and so its bits.
+static int choose_kernel(int qtype, int layout, int act_dtype, int64_t M, int64_t N, int64_t K, bool have_ws, size_t workspace_bytes,
+                         bool y_aligned8, bool bias_aligned8, bool linear, int *splits, WideShape *shape) {
+    const bool one_pass = linear && one_pass_applies(qtype, layout, act_dtype, M, N, K);
+    const int plan = one_pass ? PLAN_GEMV
+        : plan_forward(qtype, layout, M, N, K, have_ws, workspace_bytes, y_aligned8 && bias_aligned8, splits, linear, act_dtype);
+    *shape = {0, 0};
+    if (plan == PLAN_GEMV && (linear || y_aligned8)) {
+        *shape = gemv_wide_shape(qtype, layout, act_dtype, (int)M, (int)N, (int)K, one_pass);
+        if (shape->r) return PLAN_ONE_PASS;
+    }
+    return layout == LOWBIT_LAYOUT_GGML && M > 16 ? PLAN_ROWS : plan;        // (up to 16 rows: one streaming pass)
+}
+
 static int forward_any(const char *what, const void *x, const void *w, const void *bias, void *y, int qtype, int layout,
                        int act_dtype, int64_t M, int64_t N, int64_t K, void *workspace, size_t workspace_bytes, void *stream,
                        bool linear = false) {
@@ -400,17 +417,11 @@ static int forward_any(const char *what, const void *x, const void *w, const voi
     const int m = (int)M, n = (int)N, k = (int)K;
     hipStream_t st = (hipStream_t)stream;
     int splits = 1, rc = 0;
-    const bool one_pass = linear && one_pass_applies(qtype, layout, act_dtype, M, N, K);
-    const int plan = one_pass ? PLAN_GEMV
-        : plan_forward(qtype, layout, M, N, K, workspace != nullptr, workspace_bytes, !(((uintptr_t)y | (uintptr_t)bias) & 7), &splits, linear, act_dtype);
-    // (a y off the 8-byte boundaries keeps the streaming kernel's passes, and so its bits, at the entry points that say so)
-    if (plan == PLAN_GEMV && (linear || !(((uintptr_t)y) & 7))) {
-        rc = launch_gemv_wide(x, w, bias, y, qtype, layout, act_dtype, m, n, k, one_pass, st);
-        if (rc <= 0) return check_launch(rc, what);
-    }
-    if (layout == LOWBIT_LAYOUT_GGML && M > 16)          // (up to 16 rows: one streaming pass)
-        return check_launch(launch_gemm_rows(x, w, bias, y, qtype, act_dtype, m, n, k, workspace, workspace_bytes, st), what);
-    switch (plan) {
+    WideShape shape;
+    switch (choose_kernel(qtype, layout, act_dtype, M, N, K, workspace != nullptr, workspace_bytes, !(((uintptr_t)y) & 7), !(((uintptr_t)bias) & 7),
+                          linear, &splits, &shape)) {
+    case PLAN_ONE_PASS: rc = launch_gemv_wide(x, w, bias, y, qtype, layout, act_dtype, m, n, k, shape, st); break;
+    case PLAN_ROWS: rc = launch_gemm_rows(x, w, bias, y, qtype, act_dtype, m, n, k, workspace, workspace_bytes, st); break;
     case PLAN_GEMV: rc = launch_gemv(x, w, bias, y, qtype, layout, act_dtype, m, n, k, 0, st); break;
     case PLAN_RING: rc = launch_gemm_ring(x, w, bias, y, qtype, act_dtype, m, n, k, workspace, workspace_bytes, 0, st); break;
     case PLAN_GEMM_SPLIT: rc = launch_gemm(x, w, bias, y, qtype, layout, act_dtype, m, n, k, workspace, workspace_bytes, splits, st); break;
@@ -431,6 +442,11 @@ int lowbit_forward_ws(const void *x, const void *w, void *y, int qtype, int layo
 }
 
 // ---- fp32 activations: the one-pass kernel, above 32 rows (64 on small weights) in passes of 32, the streaming kernel for a rest of up to 8
+// (rows in a launch: all, where the weight is small enough)
+static int f32_rows(int qtype, int layout, int64_t M, int64_t N, int64_t K) {
+    return M > 32 && M <= 64 && gemv_wide_shape(qtype, layout, LOWBIT_DT_F32, (int)M, (int)N, (int)K, true).r ? (int)M : 32;
+}
+
 static int forward_f32(const char *what, const float *x, const void *w, const float *bias, float *y, int qtype, int layout,
                        int64_t M, int64_t N, int64_t K, void *stream) {
     if (int rc = check_weight_shape(what, qtype, N, K, layout)) return rc;
@@ -439,16 +455,14 @@ static int forward_f32(const char *what, const float *x, const void *w, const fl
     if (!x || !w || !y || !aligned16(x) || !aligned16(w) || (((uintptr_t)y | (uintptr_t)bias) & 3))
         return fail(LOWBIT_EARG, "%s: null or misaligned pointer (x, w: 16 bytes)", what);
     if (K % 8) return fail(LOWBIT_ESHAPE, "%s: K must be a multiple of 8", what);
-    if (M > 32 && M <= 64) {                             // in one launch, where the weight is small enough
-        const int rc = launch_gemv_wide(x, w, bias, y, qtype, layout, LOWBIT_DT_F32, (int)M, (int)N, (int)K, true, (hipStream_t)stream);
-        if (rc <= 0) return check_launch(rc, what);
-    }
-    for (int64_t m0 = 0; m0 < M; m0 += 32) {
-        const int m = (int)(M - m0 < 32 ? M - m0 : 32), n = (int)N, k = (int)K;
+    const int64_t step = f32_rows(qtype, layout, M, N, K);
+    for (int64_t m0 = 0; m0 < M; m0 += step) {
+        const int m = (int)(M - m0 < step ? M - m0 : step), n = (int)N, k = (int)K;
         const float *xp = x + m0 * K;
         float *yp = y + m0 * N;
-        int rc = launch_gemv_wide(xp, w, bias, yp, qtype, layout, LOWBIT_DT_F32, m, n, k, true, (hipStream_t)stream);
-        if (rc > 0) rc = launch_gemv(xp, w, bias, yp, qtype, layout, LOWBIT_DT_F32, m, n, k, 0, (hipStream_t)stream);
+        const WideShape shape = gemv_wide_shape(qtype, layout, LOWBIT_DT_F32, m, n, k, true);
+        const int rc = shape.r ? launch_gemv_wide(xp, w, bias, yp, qtype, layout, LOWBIT_DT_F32, m, n, k, shape, (hipStream_t)stream)
+                               : launch_gemv(xp, w, bias, yp, qtype, layout, LOWBIT_DT_F32, m, n, k, 0, (hipStream_t)stream);
         if (rc) return check_launch(rc, what);
     }
     return check_launch(0, what);
@@ -466,6 +480,26 @@ size_t lowbit_linear_scratch_bytes(int qtype, int layout, int dtype, int64_t M, 
     const bool sizes_ok = qk_size(qtype) && M > 16 && N > 0 && K > 0 && M <= 0x7fffffff && N <= 0x7fffffff && K <= 0x7fffffff;
     if (dtype != LOWBIT_DT_F32 && sizes_ok && one_pass_applies(qtype, layout, dtype, M, N, K)) return 0;
     return lowbit_linear_workspace_bytes(qtype, layout, dtype, M, N, K, max_bytes);
+}
+
+int lowbit_linear_plan(int qtype, int layout, int dtype, int64_t M, int64_t N, int64_t K, size_t workspace_bytes, int *plan3) {
+    if (!qk_size(qtype) || M <= 0 || N <= 0 || K <= 0 || M > 0x7fffffff || N > 0x7fffffff || K > 0x7fffffff) return -1;
+    WideShape s = {0, 0};
+    int plan = PLAN_ONE_PASS, splits = 1, rows = (int)M;
+    if (dtype == LOWBIT_DT_F32) {
+        const int step = f32_rows(qtype, layout, M, N, K);
+        rows = rows < step ? rows : step;
+        s = gemv_wide_shape(qtype, layout, dtype, rows, (int)N, (int)K, true);
+        if (!s.r) plan = PLAN_GEMV;
+    } else {
+        plan = choose_kernel(qtype, layout, dtype, M, N, K, workspace_bytes != 0, workspace_bytes, true, true, true, &splits, &s);
+    }
+    if (plan3) {
+        plan3[0] = s.r;
+        plan3[1] = s.r ? s.waves : 0;
+        plan3[2] = s.mb ? s.mb : s.r ? (rows + 15) / 16 : 0;
+    }
+    return plan;
 }
 
 int lowbit_linear(const void *x, const void *w, const void *bias, void *y, int qtype, int layout, int dtype, int64_t M,

@@ -140,8 +140,8 @@ double gemv_wide_batch_us(int qtype, int layout, int M, int N, int K) {
     return wide_batch_shape(qtype, layout, M, N, K, &us).r ? us : 0.0;
 }
 
-// linear: also the sizes that wide_shape leaves to other kernels
-static WideShape wide_shape_for(int qtype, int layout, int dt, int M, int N, int K, bool linear) {
+// linear: also the sizes that wide_shape leaves to other kernels; r = 0: not a size for this kernel
+WideShape gemv_wide_shape(int qtype, int layout, int dt, int M, int N, int K, bool linear) {
     const WideShape s = wide_shape(qtype, layout, dt, M, N, K, linear);
     const int T = (N + TILE_ROWS - 1) / TILE_ROWS, MB = (M + 15) / 16;
     if (dt == DT_F32) {
@@ -208,11 +208,9 @@ bool gemv_wide_applies(int qtype, int layout, int act_dtype, int M, int N, int K
     return wide_shape(qtype, layout, act_dtype, M, N, K, true).r != 0;
 }
 
-// 1: not a shape for this kernel; linear: see wide_shape and wide_shape_for
+// s: from gemv_wide_shape
 int launch_gemv_wide(const void *x, const void *w, const void *bias, void *y, int qtype, int layout, int act_dtype, int M, int N, int K,
-                     bool linear, hipStream_t st) {
-    const WideShape s = wide_shape_for(qtype, layout, act_dtype, M, N, K, linear);
-    if (!s.r) return 1;
+                     const WideShape &s, hipStream_t st) {
     switch (qtype) {
     case QT_SYM_INT4: return launch_wide_q<QT_SYM_INT4>(x, w, bias, y, layout, act_dtype, M, N, K, s, st);
     case QT_ASYM_INT4: return launch_wide_q<QT_ASYM_INT4>(x, w, bias, y, layout, act_dtype, M, N, K, s, st);

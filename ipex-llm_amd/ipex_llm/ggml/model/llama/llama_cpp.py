@@ -249,7 +249,7 @@ def lowbit_backward_ws_applies(qtype, layout, act_dtype, m, n, k, workspace_byte
 
 _lib.lowbit_forward_plan.argtypes = [c_int, c_int, c_int64, c_int64, c_int64, c_int, c_size_t]
 _lib.lowbit_forward_plan.restype = c_int
-PLAN_GEMV, PLAN_RING, PLAN_GEMM, PLAN_GEMM_SPLIT, PLAN_GEMM_NARROW = 0, 1, 2, 3, 4
+PLAN_GEMV, PLAN_RING, PLAN_GEMM, PLAN_GEMM_SPLIT, PLAN_GEMM_NARROW, PLAN_ONE_PASS, PLAN_ROWS = 0, 1, 2, 3, 4, 5, 6
 
 
 _lib.lowbit_workspace_bytes_for.argtypes = [c_int, c_int, c_int64, c_int64, c_int64, c_size_t]
@@ -319,6 +319,16 @@ _lib.lowbit_linear_scratch_bytes.restype = c_size_t
 
 def lowbit_linear_scratch_bytes(qtype, layout, dtype, m, n, k, max_bytes) -> int:
     return int(_lib.lowbit_linear_scratch_bytes(qtype, layout, dtype, m, n, k, max_bytes))
+
+
+_lib.lowbit_linear_plan.argtypes = [c_int, c_int, c_int, c_int64, c_int64, c_int64, c_size_t, ctypes.POINTER(c_int)]
+_lib.lowbit_linear_plan.restype = c_int
+
+
+def lowbit_linear_plan(qtype, layout, dtype, m, n, k, workspace_bytes=0):
+    """(PLAN_* code of the kernel lowbit_linear would run, (tile rows, waves at most, blocks of x) per workgroup of the one-pass kernel)."""
+    plan3 = (c_int * 3)()
+    return _lib.lowbit_linear_plan(qtype, layout, dtype, m, n, k, workspace_bytes, plan3), tuple(plan3)
 
 
 _lib.lowbit_linear.argtypes = [c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int64, c_int64, c_int64,

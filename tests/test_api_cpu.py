@@ -487,6 +487,34 @@ def test_linear_asks_for_a_workspace_only_where_its_kernel_uses_one():
     assert need(tiled, 1 << 40, 4096, 4096) == 0 and need(tiled, 40, 4096, 4096, qtype=99) == 0
 
 
+def test_linear_plan_names_the_kernel():
+    """By size; and the workspace that the call asks for is that of the kernel it names.  Host arithmetic only."""
+    def plan(layout, m, n, k, dtype=ggml.DT_F16, qtype=Q["sym_int4"]):
+        need = ggml.lowbit_linear_scratch_bytes(qtype, layout, dtype, m, n, k, 256 << 20)
+        return ggml.lowbit_linear_plan(qtype, layout, dtype, m, n, k, need)
+    tiled, rows = ggml.LAYOUT_TILED, ggml.LAYOUT_GGML
+    none = (0, 0, 0)
+    assert plan(tiled, 1, 4096, 4096) == plan(rows, 4, 4001, 2112) == (ggml.PLAN_GEMV, none)
+    assert plan(tiled, 12, 4096, 4096) == (ggml.PLAN_ONE_PASS, (1, 12, 1)) and plan(tiled, 128, 2048, 2048)[0] == ggml.PLAN_ONE_PASS
+    assert plan(tiled, 48, 4096, 11008) == plan(tiled, 96, 272, 16512) == (ggml.PLAN_RING, none)
+    assert plan(tiled, 100, 11008, 4096) == plan(tiled, 65, 1040, 16512) == (ggml.PLAN_GEMM_SPLIT, none)
+    assert plan(tiled, 65, 6160, 1152) == (ggml.PLAN_GEMM_NARROW, none) and plan(tiled, 512, 16384, 4096) == (ggml.PLAN_GEMM, none)
+    assert plan(rows, 333, 3200, 8640) == plan(rows, 1025, 31, 64) == (ggml.PLAN_ROWS, none) and plan(rows, 64, 1023, 1216)[0] == ggml.PLAN_ONE_PASS
+    assert plan(tiled, 3, 4096, 4096, ggml.DT_F32) == (ggml.PLAN_GEMV, none) and plan(tiled, 40, 11008, 4096, ggml.DT_F32)[0] == ggml.PLAN_ONE_PASS
+    for args in ((99, 1, 0, 12, 4096, 4096), (2, 1, 0, 0, 4096, 4096), (2, 1, 0, 12, 4096, 0), (2, 1, 0, 1 << 40, 4096, 4096)):
+        assert ggml.lowbit_linear_plan(*args)[0] < 0
+    rng = np.random.default_rng(8)
+    for _ in range(4000):
+        qtype, layout, dtype = int(rng.choice([2, 3, 8, 10, 15])), int(rng.integers(2)), int(rng.integers(3))
+        m, n, k = int(2 ** rng.uniform(0, 11)), 16 * int(2 ** rng.uniform(0, 11)) - 3 * (1 - layout), 128 * int(2 ** rng.uniform(0, 7))
+        need = ggml.lowbit_linear_scratch_bytes(qtype, layout, dtype, m, n, k, 256 << 20)
+        kind, shape = ggml.lowbit_linear_plan(qtype, layout, dtype, m, n, k, need)
+        assert (kind in (ggml.PLAN_RING, ggml.PLAN_GEMM_SPLIT)) == (need > 0) or kind == ggml.PLAN_ROWS, (qtype, layout, dtype, m, n, k)
+        assert (kind == ggml.PLAN_ONE_PASS) == (shape != none) and (layout == tiled or kind in (ggml.PLAN_GEMV, ggml.PLAN_ONE_PASS, ggml.PLAN_ROWS))
+        if kind == ggml.PLAN_ONE_PASS:
+            assert 1 <= shape[0] <= 4 and shape[1] in (4, 8, 12) and 1 <= shape[2] <= 4
+
+
 def test_two_groups_of_waves_are_not_estimated_longer_than_one():
     """lowbit_linear's estimate of narrow tiles: at wide weights of few steps, [26304 x 2432] at 88 rows, the fit of the form with two
     groups alone is above the form with one, which it never exceeds, and loses to slower kernels."""

@@ -43,6 +43,23 @@ def test_mlp_forward_matches_the_exact_gated_product(qtype, dtype, m, act):
     assert np.abs(y - want).max() <= tol * np.abs(want).max()
 
 
+# more workgroups than CUs in every shape of the one-pass kernel, and more than 1024 rows: the fused form of the tiled GEMM
+@pytest.mark.parametrize("qtype", ALL)
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("m,n,act", [(130, 2064, SILU), (300, 2064, GELU), (1030, 304, GELU)])
+def test_mlp_forward_of_sizes_beyond_the_one_pass_kernel(qtype, dtype, m, n, act):
+    k = 640
+    wg, wu = weights(9400 + qtype, (n, k)), weights(9500 + qtype, (n, k))
+    x = acts(9600 + m, m, k, dtype)
+    bg, bu = dev_quantize(wg, qtype, ggml.LAYOUT_TILED), dev_quantize(wu, qtype, ggml.LAYOUT_TILED)
+    y = mlp_forward_xpu(x.cuda(), bg, bu, m, k, n, act, qtype).float().cpu().numpy()
+    xf = x.float().numpy()
+    g = orc.mul_mat_exact(orc.quantize(wg, qtype), xf, (n, k), qtype)
+    u = orc.mul_mat_exact(orc.quantize(wu, qtype), xf, (n, k), qtype)
+    want = (_silu(g) if act == SILU else _gelu_tanh(g)) * u
+    assert np.abs(y - want).max() <= (2e-3 if dtype == torch.float16 else 8e-3) * np.abs(want).max()
+
+
 def test_mlp_forward_whose_row_tiles_are_a_single_round():
     # nine row tiles of 256 rows by three column tiles: few enough for one round of workgroups, where a row tile's
     # column tiles stay on one XCD (the other tile order of the fused launch); the last row tile holds 37 rows

@@ -95,3 +95,45 @@ def test_short_last_splits(qtype, dtype, m, n, k, splits):
     assert ggml.lowbit_linear_workspace_bytes(qtype, GGML, DT[dtype], m, n, k, 256 << 20) == splits * tiles * 64 * 128 * 4
     assert splits * steps > k // 128
     _check(qtype, dtype, GGML, m, n, k, False, m + n)
+
+
+# sizes that the one-pass kernel leaves to this one: more than 1024 rows, more than 16384 columns; short K at the edges of 32 and 128 weight rows
+@pytest.mark.parametrize("qtype", ALL)
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("m,n,k", [(1025, 31, 64), (1057, 33, 192), (1089, 127, 320), (1120, 128, 128), (1151, 129, 448), (1153, 257, 576),
+                                   (20, 40, 16448), (40, 70, 16704), (66, 9001, 320)])
+def test_edges_beyond_the_one_pass_kernel(qtype, dtype, m, n, k):
+    if qtype not in (FP8, 10) and m % 2:
+        k -= 32                                             # an odd number of blocks
+    if qtype == FP8:
+        k = (k + 127) // 128 * 128
+    need = ggml.lowbit_linear_scratch_bytes(qtype, GGML, DT[dtype], m, n, k, 64 << 20)
+    assert ggml.lowbit_linear_plan(qtype, GGML, DT[dtype], m, n, k, need)[0] == ggml.PLAN_ROWS
+    _check(qtype, dtype, GGML, m, n, k, m % 2 == 0, 1500 * m + n)
+
+
+# lowbit_forward keeps this kernel above 64 rows, whatever the weight: last blocks of 1 to 32 rows of every height of a tile
+@pytest.mark.parametrize("qtype", ALL)
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("m,n,k", [(65, 31, 64), (66, 33, 192), (70, 37, 448), (96, 37, 576), (97, 127, 320), (128, 129, 448), (129, 257, 576),
+                                   (129, 37, 4160), (159, 37, 4288), (180, 37, 704), (300, 145, 4288)])
+def test_small_weights_through_lowbit_forward(qtype, dtype, m, n, k):
+    """Sums, and infinities and a nan in the first and the last block of rows, at the last column and at ones that are read past the end."""
+    if qtype in (FP8, 10):
+        k = (k + 127) // 128 * 128 if qtype == FP8 else (k + 63) // 64 * 64
+    blob, x = dev_quantize(weights(m, (n, k)), qtype, GGML), acts(m, m, k, dtype).cuda()
+    w = dev_dequantize(blob, qtype, n, k, GGML, torch.float32).double()
+    for odd in (False, True):
+        if odd:
+            x[3, k - k % 128 if k % 128 else k - 128], x[5, k - 1], x[m - 1, 5], x[m - 2, 3] = float("inf"), -float("inf"), float("nan"), -float("inf")
+        want = x.double() @ w.t()
+        size = x.double().nan_to_num(posinf=0.0, neginf=0.0).abs() @ w.t().abs()
+        # fp32 sums of at most k / 32 scaled partial sums, themselves fp32; one rounding
+        bound = size * (k // 32 + 8) * 2.0 ** -24 + want.abs() * torch.finfo(dtype).eps / 2 * (1 + 2.0 ** -10) + torch.finfo(dtype).smallest_normal
+        y = torch.full((m + 2, n), float("nan"), dtype=dtype, device="cuda")
+        ggml.lowbit_forward(x.data_ptr(), blob.data_ptr(), y[1].data_ptr(), qtype, GGML, DT[dtype], m, n, k, stream())
+        assert torch.isnan(y[0]).all() and torch.isnan(y[m + 1]).all()
+        got, finite = y[1:m + 1].double(), want.isfinite()
+        assert ((got - want).abs() <= bound)[finite].all()
+        assert (got.isnan() == want.isnan()).all() and (got == want)[want.isinf()].all()
+        assert finite.all() != odd

@@ -182,3 +182,29 @@ def test_sums_of_splits(dtype, splits):
     ggml.lowbit_gemm_ws(x.data_ptr(), blob.data_ptr(), y.data_ptr(), qtype, TILED, DT[dtype], m, n, k, ws.data_ptr(), ws.numel(), splits, stream())
     want = x.double() @ dev_dequantize(blob, qtype, n, k, TILED, torch.float32).double().t()
     assert ((y.double() - want).abs().max() <= TOL[dtype] * want.abs().max())
+
+
+# sizes that the one-pass kernel leaves to the kernels that deal tiles or K, with the kernel asserted; row counts around three 32-row blocks
+SPLIT, RING, NARROW, GEMM = ggml.PLAN_GEMM_SPLIT, ggml.PLAN_RING, ggml.PLAN_GEMM_NARROW, ggml.PLAN_GEMM
+THREE_BLOCKS = [65, 96, 97, 129, 161, 192, 193, 224, 225, 257, 288, 289, 352, 480]
+KERNELS = ([(SPLIT, q, m, 1040, 16512) for q in ALL if q != NF4 for m in THREE_BLOCKS] + [(SPLIT, NF4, 129, 4112, 8192), (SPLIT, NF4, 161, 4112, 8192)]
+           + [(SPLIT, NF4, m, 2064, 16512) for m in (129, 257, 288, 289, 480)] + [(RING, NF4, m, 1040, 16512) for m in THREE_BLOCKS]
+           + [(RING, q, m, 272, 16512) for q in ALL for m in (96, 97, 192, 193, 224, 225)] + [(RING, q, 40, 1040, 16512) for q in ALL]
+           + [(RING, q, 128, 528, 20480) for q in ALL] + [(NARROW, q, m, 6160, 1152) for q in ALL for m in THREE_BLOCKS if m < 300]
+           + [(NARROW, q, m, 8208, 384) for q in ALL for m in THREE_BLOCKS] + [(GEMM, q, 480, 8208, 2048) for q in ALL if q != NF4])
+
+
+@pytest.mark.parametrize("plan,qtype,m,n,k", KERNELS)
+def test_bias_of_every_kernel_that_deals_tiles(plan, qtype, m, n, k):
+    dtype = torch.bfloat16 if (m + n + qtype) % 2 else torch.float16
+    need = ggml.lowbit_linear_scratch_bytes(qtype, TILED, DT[dtype], m, n, k, 64 << 20)
+    assert ggml.lowbit_linear_plan(qtype, TILED, DT[dtype], m, n, k, need)[0] == plan
+    blob = dev_quantize((np.random.default_rng(m + n).standard_normal((n, k), dtype=np.float32) * 0.02), qtype, TILED)
+    x, bias = acts(m, m, k, dtype).cuda(), torch.randn(n, generator=torch.Generator().manual_seed(m)).to(dtype).cuda()
+    ws = torch.full((need + 64,), 255, dtype=torch.uint8, device="cuda")
+    y = torch.full((m + 2, n), float("nan"), dtype=dtype, device="cuda")
+    ggml.lowbit_linear(x.data_ptr(), blob.data_ptr(), bias.data_ptr(), y[1].data_ptr(), qtype, TILED, DT[dtype], m, n, k,
+                       ws.data_ptr() if need else None, need, stream())
+    want = x.double() @ dev_dequantize(blob, qtype, n, k, TILED, torch.float32).double().t() + bias.double()
+    assert torch.isnan(y[0]).all() and torch.isnan(y[m + 1]).all() and (ws[need:] == 255).all()
+    assert (y[1:m + 1].double() - want).abs().max() <= TOL[dtype] * want.abs().max()
