@@ -318,10 +318,14 @@ static int plan_forward(int qtype, int layout, int64_t M, int64_t N, int64_t K, 
 }
 
 // Whether lowbit_linear takes the one-pass kernel, 16-bit activations: what gemv_wide.hip names up to 64 rows, and otherwise where its
-// estimate is 5 % below that of the kernel that else takes the size.  Those of the tiled kernels are 0.82 to 0.91 of what they take at 65
-// rows and more on weights so small: fitted to 700 random sizes (M = 65 .. 900, N to 16384, K to 14000), 5 to 10 % rms.  Of these and of
-// 250 row-major ones 533 and 150 change kernel, 0.68 and 0.65 of the time, three of them more than 3 % longer, 1.10 at worst.  Does not depend
-// on the workspace that a call brings: the other kernel's is taken to be there.
+// estimate is 5 % below that of the kernel that else takes the size, 20 % where x is more than an XCD's L2 of 4 MB holds: each XCD's
+// workgroups read all of x, and of 190 such sizes 88 estimated 5 to 20 % shorter took 0.92 of the time on average and up to 1.13 (818 rows
+// on [352 x 5504] in fp8_e4m3 19.5 -> 22.1 us, 407 on [304 x 10368] in sym_int8 19.9 -> 22.1), the other 102 took 0.78 and 1.01 at worst.
+// Smaller x: 321 random sizes that change kernel took 0.71 of the time, 1.01 at worst (M = 17 .. 1024, N to 16384, K to 16384; all of
+// these sizes are others than those that the estimates were fitted to).
+// The estimates of the tiled kernels are 0.82 to 0.91 of what they take at 65 rows and more on weights so small; the lines below
+// were fitted to 700 random sizes (M = 65 .. 900, N to 16384, K to 14000), 5 to 10 % rms, and again if narrow_time_us, gemm_time_us or
+// ring_time_us change.  Does not depend on the workspace that a call brings: the other kernel's is taken to be there.
 static bool one_pass_applies(int qtype, int layout, int act_dtype, int64_t M, int64_t N, int64_t K) {
     const int m = (int)M, n = (int)N, k = (int)K;
     if (gemv_wide_applies(qtype, layout, act_dtype, m, n, k)) return true;
@@ -340,7 +344,7 @@ static bool one_pass_applies(int qtype, int layout, int act_dtype, int64_t M, in
         default: other = 2.24 + 0.877 * other; break;
         }
     }
-    return us < 0.95 * other;
+    return us < (M * K <= (2 << 20) ? 0.95 : 0.80) * other;
 }
 
 static size_t plan_workspace(int plan, int splits, int64_t M, int64_t N, int64_t K) {

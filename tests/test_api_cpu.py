@@ -515,6 +515,19 @@ def test_linear_plan_names_the_kernel():
             assert 1 <= shape[0] <= 4 and shape[1] in (4, 8, 12) and 1 <= shape[2] <= 4
 
 
+def test_rows_of_more_than_an_l2_go_to_the_one_pass_kernel_only_where_that_is_much_shorter():
+    """Sizes that took 4 to 13 % longer there than in K splits, the ring kernel and row-major tiles; beside them ones that took 0.7 to 0.9."""
+    def one_pass(qtype, layout, m, n, k):
+        return ggml.lowbit_linear_plan(qtype, layout, ggml.DT_F16, m, n, k, 256 << 20)[0] == ggml.PLAN_ONE_PASS
+    tiled, rows = ggml.LAYOUT_TILED, ggml.LAYOUT_GGML
+    for args in [(15, tiled, 818, 352, 5504), (8, tiled, 407, 304, 10368), (15, tiled, 829, 560, 5632), (10, tiled, 771, 304, 15360),
+                 (3, tiled, 368, 336, 14080), (3, tiled, 440, 288, 15360), (8, tiled, 428, 176, 8064), (8, rows, 842, 437, 5120),
+                 (2, rows, 1007, 287, 4352), (15, tiled, 433, 528, 7040), (15, rows, 588, 465, 3968), (15, rows, 631, 257, 5376)]:
+        assert not one_pass(*args), args
+    for args in [(2, tiled, 128, 2048, 2048), (15, tiled, 217, 1024, 1408), (8, rows, 217, 1001, 1024), (10, tiled, 1000, 512, 2048), (3, rows, 66, 1001, 1088)]:
+        assert one_pass(*args), args
+
+
 def test_two_groups_of_waves_are_not_estimated_longer_than_one():
     """lowbit_linear's estimate of narrow tiles: at wide weights of few steps, [26304 x 2432] at 88 rows, the fit of the form with two
     groups alone is above the form with one, which it never exceeds, and loses to slower kernels."""
