@@ -152,13 +152,15 @@ WideShape gemv_wide_shape(int qtype, int layout, int dt, int M, int N, int K, bo
         return s;
     }
     if (M <= 16 || (M > 64 && !linear) || (s.r && T > 1024)) return s;
-    // 17 .. 64 rows, where the estimate is 5 % shorter: 122 of 250 random sizes 0.81 of the time, 74 of 200 row-major ones 0.79; beyond 64
-    // groups 12 % (18 rows on [5104 x 9728] in asym_int4, estimated 8 % shorter, took 1.06 of the time)
+    // 17 .. 64 rows, where the estimate is 5 % shorter; beyond 32 groups 8 % where a workgroup then has two tile rows more (35 rows on
+    // [3584 x 6784] in nf4, three in place of one, estimated 7.8 % shorter, took 1.06 of the time), beyond 64 groups 12 % (18 rows on [5104 x
+    // 9728] in asym_int4, estimated 8 % shorter, took 1.06).  453 of 698 random sizes, other ones than those of the fit, in 0.83 of the
+    // time, 1.01 at worst
     const int G = (K + TILE_COLS - 1) / TILE_COLS;
     double us = 0.0;
     const WideShape dealt = wide_batch_shape(qtype, layout, M, N, K, &us);
     if (!s.r) return linear ? dealt : s;
-    return dealt.r && us < (G <= 64 ? 0.95 : 0.88) * wide_us(qtype, layout, s.r, MB, M, T, G) ? dealt : s;
+    return dealt.r && us < (G > 64 ? 0.88 : G > 32 && dealt.r > s.r + 1 ? 0.92 : 0.95) * wide_us(qtype, layout, s.r, MB, M, T, G) ? dealt : s;
 }
 
 // The fused gate/up form: R of either weight, so at most 2.  Against two launches' worth of streaming passes and the fused

@@ -528,6 +528,12 @@ def test_rows_of_more_than_an_l2_go_to_the_one_pass_kernel_only_where_that_is_mu
         assert one_pass(*args), args
 
 
+def test_rows_are_dealt_on_long_walks_only_where_that_is_clearly_shorter():
+    """35 rows on [3584 x 6784] in nf4, 1.06 of the time with 16 rows to a workgroup, and beside it a size of 32 groups, 0.93."""
+    assert ggml.lowbit_linear_plan(10, ggml.LAYOUT_TILED, ggml.DT_F16, 35, 3584, 6784) == (ggml.PLAN_ONE_PASS, (1, 8, 3))
+    assert ggml.lowbit_linear_plan(10, ggml.LAYOUT_TILED, ggml.DT_F16, 35, 3584, 4096) == (ggml.PLAN_ONE_PASS, (3, 8, 1))
+
+
 def test_two_groups_of_waves_are_not_estimated_longer_than_one():
     """lowbit_linear's estimate of narrow tiles: at wide weights of few steps, [26304 x 2432] at 88 rows, the fit of the form with two
     groups alone is above the form with one, which it never exceeds, and loses to slower kernels."""

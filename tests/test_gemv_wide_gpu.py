@@ -54,6 +54,37 @@ def test_rows_dealt_to_several_workgroups(qtype, dtype, layout, m, n, k):
     _check(qtype, dtype, layout, m, n, k, m % 2 == 0, 720 * m + n)
 
 
+def dealt_sizes(qtype, layout, dtype):
+    """(tile rows, blocks of rows) per workgroup -> a size of it, of 17 to 1024 rows on up to 4 million weights."""
+    rng, sizes = np.random.default_rng(11), {}
+    for lm, ln, lk in rng.random((6000, 3)):
+        m, n, k = int(17 * 60.3 ** lm), int(20 * 300 ** ln), int(64 * 40 ** lk) // 32 * 32
+        n = (n + 15) // 16 * 16 if layout == TILED else n
+        k = (k + 127) // 128 * 128 if layout == TILED or qtype == FP8 else (k + 63) // 64 * 64 if qtype == NF4 else k
+        plan, shape = ggml.lowbit_linear_plan(qtype, layout, dtype, m, n, k, 64 << 20)
+        if plan == ggml.PLAN_ONE_PASS and n * k <= 4e6 and m * n <= 2e6 and m > 16 * shape[2]:
+            sizes.setdefault((shape[0], shape[2]), (m, n, k))
+    return sizes
+
+
+@pytest.mark.parametrize("qtype", ALL)
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("layout", [TILED, GGML])
+def test_every_shape_of_rows_dealt_to_several_workgroups(qtype, dtype, layout):
+    sizes = dealt_sizes(qtype, layout, DT[dtype])
+    assert len(sizes) >= 8
+    for m, n, k in sizes.values():
+        blob, x = dev_quantize(weights(n, (n, k)), qtype, layout), acts(m, m, k, dtype).cuda()
+        dense = dev_dequantize(blob, qtype, n, k, layout, torch.float32).double()
+        y = torch.full((m + 1, n), float("nan"), dtype=dtype, device="cuda")
+        ggml.lowbit_linear(x.data_ptr(), blob.data_ptr(), None, y.data_ptr(), qtype, layout, DT[dtype], m, n, k, None, 0, stream())
+        want, eps = x.double() @ dense.t(), torch.finfo(dtype).eps
+        # as in test_few_rows_of_many_tile_rows
+        err = 2.0 ** -24 * 2 * 17 * (k / 32 + 33) + (eps / 2 if qtype == NF4 else 0.0)
+        bound = want.abs() * eps / 2 + x.double().abs().sum(1, keepdim=True) * dense.abs().amax(1) * err + torch.finfo(dtype).smallest_normal
+        assert ((y[:m].double() - want).abs() <= bound).all() and torch.isnan(y[m]).all(), (m, n, k)
+
+
 @pytest.mark.parametrize("qtype", ALL)
 @pytest.mark.parametrize("layout,m,n,k", [(TILED, 17, 1024, 1408), (TILED, 32, 6160, 256), (TILED, 33, 5440, 256), (TILED, 48, 1040, 1152),
                                           (TILED, 64, 48, 128), (GGML, 20, 3001, 320), (GGML, 40, 1001, 1088), (GGML, 63, 2003, 192)])
