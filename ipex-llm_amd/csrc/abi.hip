@@ -32,7 +32,7 @@ int launch_gemv(const void *x, const void *w, const void *bias, void *y, int qty
 int launch_gemv_wide(const void *x, const void *w, const void *bias, void *y, int qtype, int layout, int act_dtype, int M, int N, int K,
                      const WideShape &s, hipStream_t st);
 WideShape gemv_wide_shape(int qtype, int layout, int act_dtype, int M, int N, int K, bool linear);
-double gemv_wide_batch_us(int qtype, int layout, int M, int N, int K);
+double gemv_wide_batch_us(int qtype, int layout, int act_dtype, int M, int N, int K);
 double gemm_rows_us(int qtype, int act_dtype, int M, int N, int K);
 bool gemv_wide_applies(int qtype, int layout, int act_dtype, int M, int N, int K);
 int launch_mlp_wide(const void *x, const void *wg, const void *wu, void *y, int qtype, int act_dtype, int M, int N, int K, int act,
@@ -329,7 +329,7 @@ static int plan_forward(int qtype, int layout, int64_t M, int64_t N, int64_t K, 
 static bool one_pass_applies(int qtype, int layout, int act_dtype, int64_t M, int64_t N, int64_t K) {
     const int m = (int)M, n = (int)N, k = (int)K;
     if (gemv_wide_applies(qtype, layout, act_dtype, m, n, k)) return true;
-    const double us = gemv_wide_batch_us(qtype, layout, m, n, k);
+    const double us = gemv_wide_batch_us(qtype, layout, act_dtype, m, n, k);
     if (us <= 0.0) return false;
     double other = 0.0;
     if (layout == LOWBIT_LAYOUT_GGML) {

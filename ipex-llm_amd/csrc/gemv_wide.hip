@@ -114,14 +114,18 @@ static double wide_us(int qtype, int layout, int r, int mb, int M, int T, int G)
 }
 
 // Rows of x dealt to several workgroups: so many rows and tile rows to each that the workgroups are one per CU at most and the estimate is
-// the shortest; r = 0: there is no such shape.  (r * mb: more than nine products of 16 x 16, six in asym_int4, spill.)
-static WideShape wide_batch_shape(int qtype, int layout, int M, int N, int K, double *us) {
+// the shortest; r = 0: there is no such shape.  r * mb products of 16 x 16: up to nine, six in asym_int4, is what the estimates were fitted to.
+// (No form of these spills, from twelve on all but fp8_e4m3 do, but for four tile rows and two blocks of row-major nf4 in bfloat16, whose weights are
+// three operands: six registers, in the loop.  146 to 160 rows on 3100 .. 3250 weight rows, that form against the row-major GEMM: 0.66 .. 0.88 of
+// its time up to 1344 columns, 0.98 .. 1.03 at 1600 .. 1920, 0.92 .. 0.96 at 2112 .. 2432, 1.01 .. 1.07 at 2816 .. 3904: up to 20 groups.)
+static WideShape wide_batch_shape(int qtype, int layout, int dt, int M, int N, int K, double *us) {
     WideShape best = {0, 0};
     if (M <= 16 || M > 1024 || K > 16384) return best;
     const int T = (N + TILE_ROWS - 1) / TILE_ROWS, G = (K + TILE_COLS - 1) / TILE_COLS;
     for (int r = 1; r <= 4; r++)
         for (int mb = 1; mb <= 4 && r * mb <= (qtype == QT_ASYM_INT4 ? 6 : 9); mb++) {
             if ((int64_t)((T + r - 1) / r) * ((M + 16 * mb - 1) / (16 * mb)) > 256) continue;
+            if (r == 4 && mb == 2 && layout == LAYOUT_GGML && qtype == QT_NF4 && dt == DT_BF16 && G > 20) continue;
             const double t = wide_us(qtype, layout, r, mb, M, T, G);
             if (!best.r || t < *us) {
                 best = {r, 8, mb};
@@ -135,9 +139,9 @@ static WideShape wide_batch_shape(int qtype, int layout, int M, int N, int K, do
 // the place of there: the K splits, half tiles and narrow tiles of the GEMMs, whose few tiles leave CUs idle or walk K at the latency of a
 // step, and their sums.  128 rows on [2048 x 2048] 15.2 -> 7.0 us, 72 on [4096 x 4096] 19.3 -> 12.4, 217 on [1001 x 1024] row-major
 // 11.3 -> 6.2, averages of the formats.)
-double gemv_wide_batch_us(int qtype, int layout, int M, int N, int K) {
+double gemv_wide_batch_us(int qtype, int layout, int dt, int M, int N, int K) {
     double us = 0.0;
-    return wide_batch_shape(qtype, layout, M, N, K, &us).r ? us : 0.0;
+    return wide_batch_shape(qtype, layout, dt, M, N, K, &us).r ? us : 0.0;
 }
 
 // linear: also the sizes that wide_shape leaves to other kernels; r = 0: not a size for this kernel
@@ -158,7 +162,7 @@ WideShape gemv_wide_shape(int qtype, int layout, int dt, int M, int N, int K, bo
     // time, 1.01 at worst
     const int G = (K + TILE_COLS - 1) / TILE_COLS;
     double us = 0.0;
-    const WideShape dealt = wide_batch_shape(qtype, layout, M, N, K, &us);
+    const WideShape dealt = wide_batch_shape(qtype, layout, dt, M, N, K, &us);
     if (!s.r) return linear ? dealt : s;
     return dealt.r && us < (G > 64 ? 0.88 : G > 32 && dealt.r > s.r + 1 ? 0.92 : 0.95) * wide_us(qtype, layout, s.r, MB, M, T, G) ? dealt : s;
 }

@@ -534,6 +534,19 @@ def test_rows_are_dealt_on_long_walks_only_where_that_is_clearly_shorter():
     assert ggml.lowbit_linear_plan(10, ggml.LAYOUT_TILED, ggml.DT_F16, 35, 3584, 4096) == (ggml.PLAN_ONE_PASS, (3, 8, 1))
 
 
+def test_row_major_nf4_in_bfloat16_leaves_the_shape_that_spills_on_long_walks():
+    """Four tile rows and two blocks of x: 1.01 to 1.07 of the row-major GEMM's time beyond 20 groups, in fp16, which spills nothing, 0.95 to 1.01."""
+    rows, four = ggml.LAYOUT_GGML, (ggml.PLAN_ONE_PASS, (4, 8, 2))
+    for m, n, k in [(147, 3131, 2816), (151, 3213, 3072), (160, 3105, 3904)]:
+        assert ggml.lowbit_linear_plan(10, rows, ggml.DT_BF16, m, n, k)[0] == ggml.PLAN_ROWS
+        assert ggml.lowbit_linear_plan(10, rows, ggml.DT_F16, m, n, k) == four
+    assert ggml.lowbit_linear_plan(10, rows, ggml.DT_BF16, 146, 3206, 1152) == four
+    rng = np.random.default_rng(9)
+    for lm, ln, lk in rng.random((20000, 3)):               # (up to 32 rows it is also what covers 769 .. 1024 tile rows in one round)
+        m, n, k = int(33 * 31 ** lm), int(200 * 80 ** ln), 64 * int(41 * 6 ** lk)
+        assert ggml.lowbit_linear_plan(10, rows, ggml.DT_BF16, m, n, k) != four, (m, n, k)
+
+
 def test_two_groups_of_waves_are_not_estimated_longer_than_one():
     """lowbit_linear's estimate of narrow tiles: at wide weights of few steps, [26304 x 2432] at 88 rows, the fit of the form with two
     groups alone is above the form with one, which it never exceeds, and loses to slower kernels."""
