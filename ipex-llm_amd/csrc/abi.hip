@@ -36,7 +36,8 @@ double gemv_wide_batch_us(int qtype, int layout, int act_dtype, int M, int N, in
 double gemm_rows_us(int qtype, int act_dtype, int M, int N, int K);
 bool gemv_wide_applies(int qtype, int layout, int act_dtype, int M, int N, int K);
 int launch_mlp_wide(const void *x, const void *wg, const void *wu, void *y, int qtype, int act_dtype, int M, int N, int K, int act,
-                    bool batch, hipStream_t st);
+                    const WideShape &s, hipStream_t st);
+WideShape mlp_wide_shape(int qtype, int act_dtype, int M, int N, int K, bool linear);
 size_t ring_workspace_bytes(int M, int N, int K, int wgs);
 double ring_time_us(int M, int N, int K, int qtype, bool have_ws);
 int launch_gemm_ring(const void *x, const void *w, const void *bias, void *y, int qtype, int act_dtype, int M, int N, int K,
@@ -639,10 +640,11 @@ static int mlp_any(const char *who, const void *x, const void *w_gate, const voi
     // up to 64 rows (decode, serving batches), more on small weights: one pass over both weights, by the streaming kernel up to 8 rows
     // and the kernel that gemv_wide.hip describes above that; else the fused gate/up form of the tiled MFMA GEMM
     if (M > 64 && (((uintptr_t)y) & 7)) return fail(LOWBIT_EARG, "%s: y must be 8-byte aligned", who);
-    int rc = launch_mlp_wide(x, w_gate, w_up, y, qtype, act_dtype, (int)M, (int)N, (int)K, act, linear, (hipStream_t)stream);
-    if (rc > 0 && M <= 8)
-        rc = launch_mlp_gemv(x, w_gate, w_up, y, qtype, act_dtype, (int)M, (int)N, (int)K, act, (hipStream_t)stream);
-    if (rc <= 0) return check_launch(rc, who);
+    const WideShape shape = mlp_wide_shape(qtype, act_dtype, (int)M, (int)N, (int)K, linear);
+    if (shape.r)
+        return check_launch(launch_mlp_wide(x, w_gate, w_up, y, qtype, act_dtype, (int)M, (int)N, (int)K, act, shape, (hipStream_t)stream), who);
+    if (M <= 8)
+        return check_launch(launch_mlp_gemv(x, w_gate, w_up, y, qtype, act_dtype, (int)M, (int)N, (int)K, act, (hipStream_t)stream), who);
     if (((uintptr_t)y) & 7) return fail(LOWBIT_EARG, "%s: y must be 8-byte aligned", who);
     return check_launch(launch_mlp_gemm(x, w_gate, w_up, y, qtype, act_dtype, (int)M, (int)N, (int)K, act,
                                         (hipStream_t)stream), who);

@@ -184,10 +184,11 @@ static WideShape wide_mlp_shape(int qtype, int act_dtype, int M, int N, int K) {
 }
 
 // The fused form with rows of x dealt to several workgroups, as wide_batch_shape, r of either weight; r = 0: no such shape, or the fused
-// form of the tiled GEMM is the faster one.  Fitted to 920 launches (M = 17 .. 600, N to 16384, K to 14000), 7 to 8 % rms.  17 .. 64 rows: ahead of
-// the shapes with all rows to a workgroup (172 of 183 random sizes 0.87 of the time, one 3 % longer).  More: against narrow tiles, which
+// form of the tiled GEMM is the faster one.  Fitted to 920 launches (M = 17 .. 600, N to 16384, K to 14000), 7 to 8 % rms.  17 .. 64 rows: ahead
+// of the shape with all rows to a workgroup where the estimate is shorter, beyond 8 groups 3 % shorter (34 rows on [2368 x 2048] in fp8_e4m3, estimated 2 % shorter,
+// took 1.10).  216 of 330 random sizes, other ones than those of the fit, in 0.83 of the time.  More: against narrow tiles, which
 // while they are one per CU take 4 to 5 us and 0.54 to 0.65 per 128 columns (118 of 147 random sizes 0.61 of the time, none longer).
-static WideShape wide_mlp_batch_shape(int qtype, int M, int N, int K) {
+static WideShape wide_mlp_batch_shape(int qtype, int act_dtype, int M, int N, int K) {
     static const double fit[5][7] = {{3.495, 0.036, 0.213, 0.220, 0.080, 0.044, 0.030}, {3.097, 0.004, 0.097, 0.235, 0.141, 0.139, 0.041},
                                      {3.434, 0.091, 0.134, 0.416, 0.039, 0.063, 0.043}, {3.493, 0.000, 0.116, 0.322, 0.085, 0.088, 0.031},
                                      {3.293, 0.115, 0.195, 0.351, 0.018, 0.054, 0.043}};
@@ -196,18 +197,24 @@ static WideShape wide_mlp_batch_shape(int qtype, int M, int N, int K) {
     if (M <= 16 || M > 1024 || K > 16384) return best;
     const int T = N / TILE_ROWS, G = K / TILE_COLS, q = format_index(qtype);
     const double(&f)[7] = fit[q];
+    auto workgroups = [&](int r, int mb) { return (int64_t)((T + r - 1) / r) * ((M + 16 * mb - 1) / (16 * mb)); };
+    auto estimate = [&](int r, int mb) {
+        return f[0] + (G + 7) / 8 * (f[1] + f[2] * mb + f[3] * 2 * r + f[4] * 2 * r * mb) + f[5] * 2 * r * mb
+            + f[6] * (double)workgroups(r, mb) / 256 * G * mb;
+    };
     double us = M <= 64 ? 1e30 : 0.95 * (tiled[q][0] + tiled[q][1] * G);
     for (int r = 1; r <= 2; r++)
         for (int mb = 1; r * mb <= 4; mb++) {
-            const int64_t wgs = (int64_t)((T + r - 1) / r) * ((M + 16 * mb - 1) / (16 * mb));
-            if (wgs > 256) continue;
-            const double t = f[0] + (G + 7) / 8 * (f[1] + f[2] * mb + f[3] * 2 * r + f[4] * 2 * r * mb) + f[5] * 2 * r * mb + f[6] * (double)wgs / 256 * G * mb;
+            if (workgroups(r, mb) > 256) continue;
+            const double t = estimate(r, mb);
             if (t < us) {
                 best = {r, 8, mb};
                 us = t;
             }
         }
-    return best;
+    const WideShape all = wide_mlp_shape(qtype, act_dtype, M, N, K);
+    const int MB = (M + 15) / 16;
+    return best.r && all.r && workgroups(all.r, MB) <= 256 && us >= (G > 8 ? 0.97 : 1.0) * estimate(all.r, MB) ? all : best;
 }
 
 bool gemv_wide_applies(int qtype, int layout, int act_dtype, int M, int N, int K) {
@@ -227,12 +234,16 @@ int launch_gemv_wide(const void *x, const void *w, const void *bias, void *y, in
     }
 }
 
-int launch_mlp_wide(const void *x, const void *wg, const void *wu, void *y, int qtype, int act_dtype, int M, int N, int K, int act,
-                    bool batch, hipStream_t st) {
+// linear: also above 64 rows, on small weights; r = 0: not a size for this kernel
+WideShape mlp_wide_shape(int qtype, int act_dtype, int M, int N, int K, bool linear) {
     WideShape s = {0, 0};
-    if (M <= 64 || batch) s = wide_mlp_batch_shape(qtype, M, N, K);
-    if (!s.r) s = wide_mlp_shape(qtype, act_dtype, M, N, K);
-    if (!s.r) return 1;
+    if (M <= 64 || linear) s = wide_mlp_batch_shape(qtype, act_dtype, M, N, K);
+    return s.r ? s : wide_mlp_shape(qtype, act_dtype, M, N, K);
+}
+
+// s: from mlp_wide_shape
+int launch_mlp_wide(const void *x, const void *wg, const void *wu, void *y, int qtype, int act_dtype, int M, int N, int K, int act,
+                    const WideShape &s, hipStream_t st) {
     switch (qtype) {
     case QT_SYM_INT4: return launch_wide_mlp_q<QT_SYM_INT4>(x, wg, wu, y, act_dtype, M, N, K, act, s, st);
     case QT_ASYM_INT4: return launch_wide_mlp_q<QT_ASYM_INT4>(x, wg, wu, y, act_dtype, M, N, K, act, s, st);
