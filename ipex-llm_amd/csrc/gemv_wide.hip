@@ -40,12 +40,20 @@ static WideShape wide_shape(int qtype, int layout, int dt, int M, int N, int K, 
         // / 30.4 -> 17.7 us, on [9600 x 8192] 31.7 -> 19.6 / 55.3 -> 29.6.  Four tile rows have the registers for 16 rows
         // of x only, and row-major weights need more instructions per tile: [14336 x 4096], 9 rows, four / two tile rows 15.2 / 17.2
         // us.  Beyond 1024 tile rows three with four waves, several workgroups per CU ([18000 x 1024], 9 / 24 rows: 10.3 -> 8.2 / 15.1 ->
-        // 11.8; eight waves 9.9 / 13.9).  12 waves up to 12 rows and one tile row, where the walk's latency counts ([4096 x 4096]
-        // in sym_int4, 9 / 12 / 16 rows, 8 waves / 12: 9.3 / 8.4, 9.4 / 8.9, 9.4 / 9.1 us; [2048 x 3072] at 16 rows 7.6 / 8.2;
-        // fp8_e4m3 on [4096 x 6144] at 12 rows 11.7 / 12.7).
+        // 11.8; eight waves 9.9 / 13.9).  12 waves with one tile row and 16 rows of x in the formats of four bits, where the walk's latency counts
+        // more than what each wave adds of the sums and of x, of which there is less with fewer rows (rows past M are read as the last one).
+        // 12 against 8 at 9 / 11 / 13 / 16 rows, averages over 19 weights of 512 to 4096 rows: row-major sym_int4 0.97 / 0.97 / 0.98 /
+        // 0.99, asym_int4 0.94 / 0.95 / 0.95 / 0.97; tiled, 13 to 29 groups, 0.98 / 1.00 / 1.02 / 1.03 and 0.98 / 0.99 / 1.00 / 1.02; 12
+        // groups, one round of waves, 1.01 / 0.98 / 0.98 / 0.97 and 1.01 / 0.99 / 1.00 / 1.00; 30 and more 0.94 / 0.97 / 0.99 / 1.01 and 0.96 /
+        // 0.97 / 0.98 / 1.00, 1.03 at worst from 13 rows on.  nf4, tiled, 0.97 / 0.98 / 0.98 / 0.99 over all of them (row-major 0.99 / 0.99 / 1.00 /
+        // 1.00); sym_int8 0.98 at 9 rows and up to 1.06 at 16, fp8_e4m3 0.98 and up to 1.08 from 12 on.
         if (M > 32 || (M <= 8 && !shared_by_three)) return none;
-        const bool int4 = qtype == QT_SYM_INT4 || qtype == QT_ASYM_INT4;
-        if (rounds <= 3) return {rounds, rounds == 1 && M <= 12 && int4 ? 12 : 8};
+        if (rounds == 1 && MB == 1) {
+            const bool int4 = qtype == QT_SYM_INT4 || qtype == QT_ASYM_INT4, tiled = layout == LAYOUT_TILED;
+            const int most = int4 ? (tiled && G > 12 && G < 30 ? 10 : 13) : qtype == QT_NF4 && tiled ? 16 : 0;      // rows of x
+            return {1, M <= most ? 12 : 8};
+        }
+        if (rounds <= 3) return {rounds, 8};
         if (rounds == 4) return layout == LAYOUT_TILED && MB == 1 ? WideShape{4, 8} : WideShape{2, 4};
         return {3, 4};
     }

@@ -564,6 +564,20 @@ def test_gated_mlp_rows_are_dealt_only_where_that_is_clearly_shorter():
     assert of(2, 130, 1024, 2048)[2] > 0 and of(2, 130, 1024, 2048, False) == (0, 0, 0)
 
 
+def test_waves_of_float32_rows_go_by_format_and_walk():
+    """One tile row and up to 16 rows of x: what 12 waves gain over 8 depends on the format, the groups of columns and the rows."""
+    def most(qtype, layout, n, k):
+        waves = [ggml.lowbit_linear_plan(qtype, layout, ggml.DT_F32, m, n, k)[1][1] for m in range(9, 17)]
+        assert waves == sorted(waves, reverse=True) and set(waves) <= {8, 12}
+        return 8 + waves.count(12)
+    tiled, rows = ggml.LAYOUT_TILED, ggml.LAYOUT_GGML
+    assert [most(q, tiled, 2048, 1536) for q in (2, 3, 8, 10, 15)] == [13, 13, 8, 16, 8]
+    assert [most(q, tiled, 4096, 3072) for q in (2, 3, 8, 10, 15)] == [10, 10, 8, 16, 8]
+    for n, k in ((4096, 4096), (512, 4096), (2048, 14336)):
+        assert [most(q, tiled, n, k) for q in (2, 3, 8, 10, 15)] == [13, 13, 8, 16, 8]
+    assert [most(q, rows, 2001, 4608) for q in (2, 3, 8, 10, 15)] == [13, 13, 8, 8, 8]
+
+
 def test_two_groups_of_waves_are_not_estimated_longer_than_one():
     """lowbit_linear's estimate of narrow tiles: at wide weights of few steps, [26304 x 2432] at 88 rows, the fit of the form with two
     groups alone is above the form with one, which it never exceeds, and loses to slower kernels."""

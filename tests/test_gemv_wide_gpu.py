@@ -167,6 +167,16 @@ def test_float32_activations_shared_by_tile_rows(qtype, layout, m, n, k):
     _check(qtype, torch.float32, layout, m, n, k, m % 2 == 0, 950 * m + n)
 
 
+# 12 waves and 8 beside them: fewer groups than waves, one more, a whole second round, and long walks
+@pytest.mark.parametrize("qtype,layout,m,n,k,waves", [(q, TILED, m, 48, k, 12) for q in (2, 3, NF4) for m, k in ((9, 1152), (13, 1536), (10, 1664), (13, 3968))]
+                         + [(q, GGML, m, 33, k, 12) for q in (2, 3) for m, k in ((9, 1600), (13, 3904))] + [(NF4, TILED, 16, 48, k, 12) for k in (1664, 3968)]
+                         + [(q, TILED, 16, 48, k, 8) for q in (2, 3) for k in (1536, 1664, 3968)]
+                         + [(q, TILED, 9, 48, 1664, 8) for q in (8, FP8)] + [(q, GGML, 9, 33, 1664, 8) for q in (8, NF4, FP8)])
+def test_float32_activations_in_8_and_12_waves(qtype, layout, m, n, k, waves):
+    assert ggml.lowbit_linear_plan(qtype, layout, ggml.DT_F32, m, n, k) == (ggml.PLAN_ONE_PASS, (1, waves, 1))
+    _check(qtype, torch.float32, layout, m, n, k, m % 2 == 0, 960 * m + n)
+
+
 @pytest.mark.parametrize("qtype", ALL)
 @pytest.mark.parametrize("layout,m,n,k", [(TILED, 9, 48, 256), (TILED, 20, 8224, 128), (TILED, 16, 12336, 128), (GGML, 17, 8215, 128)])
 def test_float32_activations_beyond_bfloat16(qtype, layout, m, n, k):
