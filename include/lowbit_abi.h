@@ -186,8 +186,8 @@ int lowbit_dequantize_rows(const void *w, const int64_t *rows, int64_t n_rows, v
  * gate/up form of the tiled GEMM (y 8-byte aligned, M < 2^24, K < 2^23). */
 int lowbit_mlp_forward(const void *x, const void *w_gate, const void *w_up, void *y, int qtype, int act_dtype,
                        int64_t M, int64_t N, int64_t K, int act, void *stream);
-/* The same, what a converted model's MLP calls: on small weights the one-pass kernel, whose weights are not rounded to 16 bits, takes up to
- * 1024 rows where it is estimated to be the faster one. */
+/* The same, what a converted model's MLP calls: on small weights the one-pass kernel takes up to 1024 rows where it is estimated to be the
+ * faster one.  Its weights are exact codes (nf4: levels rounded to act_dtype) times a scale in fp32, not products rounded to act_dtype. */
 int lowbit_gated_mlp(const void *x, const void *w_gate, const void *w_up, void *y, int qtype, int act_dtype,
                      int64_t M, int64_t N, int64_t K, int act, void *stream);
 
@@ -229,8 +229,8 @@ int lowbit_gemm_ws(const void *x, const void *w, void *y, int qtype, int layout,
  * hands them a float x (python/llm/src/ipex_llm/transformers/low_bit_linear.py:657-668: only M > 1 with
  * conver_to_half casts to half first) and what the CPU branch's ggml_compute_forward_mul_mat_q_fp32 returns.
  * x is split into two bf16 planes (16 mantissa bits, fp32's exponent range), the product of the 2M rows is
- * accumulated and stored in fp32 and the halves are added.  Every M runs in passes over the weights of up to
- * 32 rows: meant for decode and small batches.  workspace: caller-owned device
+ * accumulated and stored in fp32 and the halves are added.  Up to 64 rows on small weights run in one pass over them, any
+ * other M in passes of up to 32 rows: meant for decode and small batches.  workspace: caller-owned device
  * memory of lowbit_forward_f32_workspace_bytes(M, N, K) bytes, 16-byte aligned. */
 size_t lowbit_forward_f32_workspace_bytes(int64_t M, int64_t N, int64_t K);
 int lowbit_forward_f32(const float *x, const void *w, float *y, int qtype, int layout, int64_t M, int64_t N, int64_t K,
@@ -241,8 +241,8 @@ int lowbit_forward_f32(const float *x, const void *w, float *y, int qtype, int l
  * (lowbit_linear_workspace_bytes says what to pass within a budget; null is valid), but for three choices that the other entry
  * points, whose kernel a caller may rely on, do not make: the one-pass kernel at 17 .. 64 rows of x, and up to 1024 on small weights, in
  * place of the ring kernel, a K split, row-major tiles or several streaming passes, and up to 16 rows on more weights than they take
- * it on (where lowbit_forward(_ws) plans one streaming pass and y is 8-byte aligned, it takes the one-pass kernel in its place at 9 .. 16
- * rows of x on tiled and 5 .. 16 on row-major weights, up to 16384 weight rows; row-major ones up to 64); narrow tiles more often (two groups of waves share such a tile's K where CUs
+ * it on (with y 8-byte aligned lowbit_forward(_ws) takes the one-pass kernel in place of one streaming pass at 9 .. 16 rows of x on tiled
+ * and 5 .. 16 on row-major weights of up to 16384 rows, and on most row-major ones up to 64 rows of x); narrow tiles more often (two groups of waves share such a tile's K where CUs
  * would idle); and tiles of 256 rows ahead of all estimates where they fill the GPU's rounds well (the rounds depend on the
  * activation type).  The bias is added to the fp32 sums before the one rounding (a bias that is not 8-byte aligned is valid and
  * slower above 16 rows).  What LowBitLinear.forward computes

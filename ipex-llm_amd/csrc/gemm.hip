@@ -71,6 +71,7 @@ static bool half_tiles(int M, int64_t tiles, int n_cus) { return M > GM / 2 && t
 //     tile to 0.043 us to write and sum (a quarter of it fixed, the rest by the rows it holds);
 //   - the formats with more work per weight take longer per step: sym_int8 1.30, fp8_e4m3 1.15, nf4 1.30 - 2.48 in
 //     the register-staged form it uses up to one workgroup per CU; half tiles take 0.88 (0.83) of a tile's step.
+// (abi.hip's one_pass_applies has a fit of its own on top of this, to be made again when this changes.)
 double gemm_time_us(int M, int N, int K, int splits, int qtype) {
     const int tiles_m = (M + GM - 1) / GM;
     const double tiles = (double)tiles_m * (double)((N + GN - 1) / GN);
@@ -283,6 +284,7 @@ static bool narrow_two_groups(int M, int N, int K) { return narrow_workgroups(M,
 // random points: the fit is too long for wide weights of few steps ([26304 x 2432] at 88 rows in sym_int4 26.1 us; where it
 // passed them over, 37.6).  Against the choice with one group the one made with this is 6.2 % faster on average over 2164
 // of them; 20 are slower by 3 to 11 % (a larger scale loses as much elsewhere).
+// (abi.hip's one_pass_applies has a fit of its own on top of this, to be made again when this changes.)
 double narrow_time_us(int M, int N, int K, int qtype, bool linear) {
     const int tiles_m = (M + GM - 1) / GM;
     const bool halves = narrow_halves(M, N);

@@ -497,6 +497,7 @@ static RingPlan ring_plan(int M, int N, int K, int rnb, int wgs, bool have_ws) {
 // the steps of the longest run; 8-bit codes and nf4 take 15 - 30 % longer per step, and steps are shorter on a
 // machine that is not full.  The whole is scaled by 0.95: against the estimates of the other kernels that picks
 // the fastest one most often.
+// (abi.hip's one_pass_applies has a fit of its own on top of this, to be made again when this changes.)
 double ring_time_us(int M, int N, int K, int qtype, bool have_ws) {
     const int mb = M <= 32 ? 1 : M <= 64 ? 2 : 4;
     const RingPlan p = ring_plan(M, N, K, ring_rnb_of(qtype, mb), 0, have_ws);

@@ -403,7 +403,7 @@ struct RowsPlan {
 };
 // With row tiles of 32 * mb rows.  K splits: until the workgroups are about two per CU (the kernel's occupancy), of at least four
 // steps each.  cost: a step reckons its weights as two row blocks, a workgroup that has a CU to itself takes 0.7 of the time, a split
-// costs 2 and 5 per round of fp32 tiles.
+// costs 2 and 5 per round of fp32 tiles.  (gemm_rows_us is a fit on top of it, to be made again when this changes.)
 static RowsPlan rows_plan_of(int mb, int M, int N, int K, size_t ws_bytes) {
     RowsPlan p;
     p.mb = mb;

@@ -418,7 +418,7 @@ static int launch_wide_mlp_mb(const void *x, const void *wg, const void *wu, voi
     return -7;
 }
 
-// y = act(x wg^T) * (x wu^T) for up to 64 rows
+// y = act(x wg^T) * (x wu^T), s.mb 16-row blocks of x to a workgroup (0: all of up to 64 rows)
 template <int QT, typename AT>
 static int launch_wide_mlp_t(const void *x, const void *wg, const void *wu, void *y, int M, int N, int K, int act, const WideShape &s,
                              hipStream_t st) {

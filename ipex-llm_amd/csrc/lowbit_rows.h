@@ -1,5 +1,5 @@
 // Weights in the row-major (ggml) layout as operands of v_mfma_f32_16x16x32: what the streaming kernel and the one-pass
-// kernel for up to 64 rows share (more rows: gemm_rows.hip, in 32 x 32 tiles).
+// kernel share (larger products: gemm_rows.hip, in 32 x 32 tiles).
 //
 // Both take 16 weight rows by 128 columns at a time, lane l = 16*c + r standing for row r.  A lane loads 16 bytes of
 // codes per load (8-bit formats: twice) at the 2-byte alignment that the blocks have, and the header in front:
