@@ -107,7 +107,9 @@ static int format_index(int qtype) {
 
 // What a launch takes whose workgroups are one per CU at most, 8 waves each, with r tile rows and 16 * mb rows of x to a workgroup:
 // microseconds, fitted to 1250 sizes (M = 17 .. 900, N to 16384, K to 14000) in up to three shapes each, 6 to 10 % rms.  A launch; per
-// 1024 columns what goes with the groups, with x, with the weights and with their products; the sums; x out of L2.
+// 1024 columns what goes with the groups, with x, with the weights and with their products; the sums; x out of L2.  x's type counts in row-major
+// nf4 only, three operands in bfloat16 and two in fp16, and is left out: 1.02 .. 1.08 of the fp16 time with up to six products (1.15 with eight and
+// nine) where the row-major GEMM, which it is compared with, takes 1.11.
 static double wide_us(int qtype, int layout, int r, int mb, int M, int T, int G) {
     static const double fit[2][5][7] = {                    // row-major, tiled; sym_int4, asym_int4, sym_int8, nf4, fp8_e4m3
         {{2.680, 0.076, 0.200, 0.466, 0.032, 0.249, 0.020}, {2.423, 0.326, 0.100, 0.390, 0.114, 0.296, 0.042},

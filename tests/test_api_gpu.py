@@ -304,6 +304,33 @@ def test_lowbit_linears_replay_correctly_from_a_hip_graph():
             assert torch.equal(static_y, want), (rows, step)
 
 
+@pytest.mark.parametrize("plan,m,n,k", [(ggml.PLAN_GEMM_SPLIT, 65, 1040, 16512), (ggml.PLAN_RING, 96, 272, 16512), (ggml.PLAN_ROWS, 20, 40, 16448),
+                                        (ggml.PLAN_ONE_PASS, 130, 1024, 512), (ggml.PLAN_ONE_PASS, 70, 301, 320)])
+def test_layers_with_partial_sums_and_dealt_rows_replay_from_a_hip_graph(plan, m, n, k):
+    """Layers whose kernel leaves partial sums in a workspace, and ones whose rows are dealt to several workgroups: captured once, each
+    replay with other inputs and eager work in between."""
+    layout = ggml.LAYOUT_TILED if n % 16 == 0 and k % 128 == 0 else ggml.LAYOUT_GGML
+    need = ggml.lowbit_linear_scratch_bytes(2, layout, ggml.DT_F16, m, n, k, 256 << 20)
+    assert ggml.lowbit_linear_plan(2, layout, ggml.DT_F16, m, n, k, need)[0] == plan and (need > 0) == (plan != ggml.PLAN_ONE_PASS)
+    layer = _layer(np.random.default_rng(n).standard_normal((n, k), dtype=np.float32) * 0.02, 2).to("cuda")
+    static_x, side, graph = torch.zeros(m, k, dtype=torch.float16, device="cuda"), torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        layer(static_x)
+    torch.cuda.current_stream().wait_stream(side)
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graph):
+        static_y = layer(static_x)
+    for _ in range(4):
+        x = torch.randn(m, k, device="cuda").half()
+        want = layer(x)
+        torch.cuda.synchronize()
+        static_x.copy_(x)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(static_y, want)
+
+
 @pytest.mark.parametrize("qname", ["sym_int4", "nf4"])
 def test_module_cuda_and_cpu_keep_the_residency_rule(qname):
     """model.cuda() calls Tensor.cuda on every parameter, not .to(): the blob must still arrive tiled, and
