@@ -319,10 +319,13 @@ static int plan_forward(int qtype, int layout, int64_t M, int64_t N, int64_t K, 
 }
 
 // Whether lowbit_linear takes the one-pass kernel, 16-bit activations: what gemv_wide.hip names up to 64 rows, and otherwise where its
-// estimate is 5 % below that of the kernel that else takes the size, 20 % where x is more than an XCD's L2 of 4 MB holds: each XCD's
-// workgroups read all of x, and of 190 such sizes 88 estimated 5 to 20 % shorter took 0.92 of the time on average and up to 1.13 (818 rows
-// on [352 x 5504] in fp8_e4m3 19.5 -> 22.1 us, 407 on [304 x 10368] in sym_int8 19.9 -> 22.1), the other 102 took 0.78 and 1.01 at worst.
-// Smaller x: 321 random sizes that change kernel took 0.71 of the time, 1.01 at worst (M = 17 .. 1024, N to 16384, K to 16384; all of
+// estimate is 5 % below that of the kernel that else takes the size.  Where x is more than an XCD's L2 of 4 MB holds, each of which serves all
+// of x, the estimate is less certain, and the more so the more rows there are: above 320 rows 10 % with tiled weights of four bits, 15 % with
+// row-major ones and those of eight bits, whose lines take more of it.  Of 291 random sizes with so much x 47 stay with the other kernel, of
+// whose time this one took 0.99 on average and up to 1.13 (818 rows on [352 x 5504] in fp8_e4m3 19.5 -> 22.1 us, 829 on [560 x 5632]
+// 22.2 -> 24.2); the 244 others took 0.80, seven of them 1.02 to 1.09 (627 on [352 x 7936] in asym_int4 19.6 -> 21.4, whose estimate is 13 %
+// shorter).  Up to 320 rows: 55 sizes, 0.80, one of them 1.05.
+// Smaller x: 267 sizes of 65 rows and more that change kernel took 0.70 of the time, 1.01 at worst (N to 16384, K to 16384; all of
 // these sizes are others than those that the estimates were fitted to).
 // The estimates of the tiled kernels are 0.82 to 0.91 of what they take at 65 rows and more on weights so small; the lines below
 // were fitted to 700 random sizes (M = 65 .. 900, N to 16384, K to 14000), 5 to 10 % rms, and again if narrow_time_us, gemm_time_us or
@@ -345,7 +348,8 @@ static bool one_pass_applies(int qtype, int layout, int act_dtype, int64_t M, in
         default: other = 2.24 + 0.877 * other; break;
         }
     }
-    return us < (M * K <= (2 << 20) ? 0.95 : 0.80) * other;
+    const bool bits8 = qtype == LOWBIT_QT_SYM_INT8 || qtype == LOWBIT_QT_FP8_E4M3;
+    return us < (M <= 320 || M * K <= (2 << 20) ? 0.95 : bits8 || layout == LOWBIT_LAYOUT_GGML ? 0.85 : 0.90) * other;
 }
 
 static size_t plan_workspace(int plan, int splits, int64_t M, int64_t N, int64_t K) {
